@@ -3,9 +3,9 @@
  * vocabulary matrix, and the device half of greedy sampling (argmax, and the softmax probability of the maximum).
  *
  * Replaces `xabe_cuda::kernels::lm_head::{LmHeadKernels, LmHeadGeometry, HeadFormat, HeadTensor, LmHeadError}`
- * ("L" = crates/xabe-cuda/src/kernels/lm_head.rs).  The same streaming machinery as the decode kernels of
+ * ("L" = crates/xabe-cuda/src/kernels/lm_head.rs).  The same contraction as the decode kernels of
  * xabe_hip.h: every 16-byte piece of the matrix is requested once, coalesced, and the fields are unpacked
- * from a wavefront-private staging slot; a pass over the weights serves up to
+ * from a wavefront-private staging slot; a pass over the weights serves at least
  * XABE_LM_HEAD_MAX_BATCH_TILE tokens.  Statuses are the `xabe_status` values of xabe_hip.h.
  */
 #ifndef XABE_LM_HEAD_H
@@ -20,8 +20,9 @@
 extern "C" {
 #endif
 
-/* Tokens one pass over the weights serves (L:125 has 8: here a lane keeps the tile's activations in
- * registers, 32 per token, which fits four). */
+/* Tokens one pass over the weights serves in every format (L:125 has 8): a 16-bit matrix keeps the tile's activations
+ * in a lane's registers, which fits four; a quantized one takes up to eight per pass, so the pass and byte counts
+ * below, which use this number, are upper bounds for it. */
 #define XABE_LM_HEAD_MAX_BATCH_TILE 4
 /* Length of the partial-winner buffers xabe_lm_head_argmax takes (L:169). */
 #define XABE_LM_HEAD_ARGMAX_BLOCKS 512

@@ -1,24 +1,18 @@
 // LM head: logits[t][v] = sum_h W[v][h] * x[t][h] for a [vocab][hidden] matrix in Q8_0, Q6_K, bf16 or f16,
 // and the device half of greedy sampling.  Takes the place of crates/xabe-cuda/src/kernels/lm_head.rs.
 //
-// The matrix is read once per pass and a pass serves up to four tokens: the lane's activations of the tile
-// (32 per token for a 2048-wide row) stay in registers for the whole launch, so the only stream is the
-// weights.  A wavefront owns R adjacent rows at a time, requests the next R rows before it accumulates the
-// current ones, and walks the vocabulary with all other wavefronts in row order, so the launch reads the
-// tensor front to back.  Quantized rows go through the coalesced loader of decode_kernels.h (each 16-byte
-// piece requested once, fields unpacked from a wavefront-private LDS slot); 16-bit rows are read as
-// 16-byte pieces directly.
-//
-// Numerics: fp32, no contraction.  A lane sums its products in element order (the accumulation of the decode
-// kernels), the 64 lane sums are combined by the fixed DPP tree, and nothing depends on the batch: a token's
-// logits are the same bits at every batch width and position.
+// Quantized matrices go through the digit contraction (digits.h), up to eight tokens per pass over the weights; 16-bit
+// ones through the vector ALU, up to four.  Nothing depends on the batch: a token's logits are the same bits at every
+// batch width and position.
 #include <string.h>
 
 #include <algorithm>
+#include <utility>
 
 #include "../../include/xabe_gguf.h"
 #include "../../include/xabe_lm_head.h"
 #include "decode_kernels.h"
+#include "digits.h"
 #include "host_common.h"
 
 namespace xabe {
@@ -29,110 +23,128 @@ struct LmHeadArgs {
   float* out;       // [*][vocab]
   int K, vocab;
   int t0, nt;       // tokens [t0, t0 + nt) are served by this launch, 1 <= nt <= TOK
-  int row_lo, row_hi;    // quantized kernels: rows [row_lo, row_hi) are served by this launch
-  const uint8_t* w_end;  // TAIL launches: one past the tensor's last byte
+  size_t w_bytes;   // quantized kernels: the tensor's length
+  int seg_sb;       // quantized kernels: superblocks whose activations LDS holds at a time
 };
 
-// Q8_0 / Q6_K rows.  ONE: the row is a single wavefront step (K <= 2048) and the activations are hoisted out
-// of the row loop; otherwise the contraction is walked step by step with the activations re-read per step.
-// TAIL: the launch that serves the last row of a tensor whose length is not a multiple of 16 bytes; the one
-// piece that would reach past the tensor is put together from 2-byte loads.
-template <int QUANT, int R, int TOK, bool ONE, bool TAIL = false>
-__global__ void __launch_bounds__(256) k_lm_head_quant(LmHeadArgs a) {
-  using F = Fmt<QUANT>;
-  using Raw = typename F::Raw;
-  constexpr int kSlot = StageFmt<QUANT>::kSlotBytes;
-  __shared__ __attribute__((aligned(16))) uint8_t s_slots[kWavesPerWg * R * kSlot];
-  const LaneGeom g = lane_geom<QUANT>();
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const size_t row_bytes = (size_t)(a.K / F::kBlockElems) * F::kBlockBytes;
-  const int steps = (a.K + kStepElems - 1) / kStepElems;
-  const int groups = (a.row_hi - a.row_lo + R - 1) / R;
-  const int stride = (int)gridDim.x * kWavesPerWg;
-  uint8_t* slots = s_slots + (size_t)wave * R * kSlot;
+// Q8_0 / Q6_K rows, NT tokens.  The launch is one workgroup per CU; every wavefront owns a contiguous range of the
+// vocabulary and takes it 32 rows and one superblock at a time through its own LDS slot (SliceDma), against the tokens'
+// digits, which the workgroup makes once and keeps in LDS.  A wavefront's ranges are equal to within a row, so the last
+// round of tiles is as long for everyone: 7760 tiles of 32 rows do not divide over 2048 wavefronts, rows do.
+// Per row and token: superblock sums in order, each half of the wavefront its own, then half 0 + half 1.
+// Bound by bytes up to four tokens (Q8_0: 96 us for one, 102 for three = 5.3-5.6 TB/s, the rate a plain read loop
+// reaches), by the vector ALU beyond (eight: 120 us).  Eight wavefronts per CU: twelve and sixteen measured slower.
+// SEG: rows whose digits do not fit in LDS are staged seg_sb superblocks at a time, again for every tile.
+constexpr size_t kHeadLdsMax = 160 * 1024;
+constexpr size_t kHeadZeros = 1024;
+constexpr size_t kHeadQuantTokens = 8;  // tokens per pass over a quantized matrix
 
-  auto issue_w = [&](int rg, int k, Staged<QUANT> (&pend)[R]) __attribute__((always_inline)) {
-    const uint32_t nbytes = (uint32_t)(min(kStepElems, a.K - k * kStepElems) / F::kBlockElems) * F::kBlockBytes;
+template <int QUANT, int NT, bool SEG>
+__global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
+  using Dma = SliceDma<QUANT>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_head[];
+  const int lane = (int)__lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int waves = (int)(blockDim.x >> 6);
+  const int nsb = a.K / kSbElems, seg_sb = SEG ? a.seg_sb : nsb;
+  uint8_t* const s_zero = s_head;
+  uint8_t* const s_x = s_zero + kHeadZeros;                             // [superblock][token][kSbLdsBytes]
+  uint8_t* const slot = s_x + (size_t)seg_sb * NT * kSbLdsBytes + (size_t)wave * Dma::kSlotBytes;
+  const uint32_t slot_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot;
+  const uint32_t row_bytes = (uint32_t)nsb * SbRaw<QUANT>::kBytes;
+  const int index = (int)blockIdx.x * waves + wave, n_waves = (int)gridDim.x * waves;
+  const int row_lo = (int)((long long)a.vocab * index / n_waves), row_hi = (int)((long long)a.vocab * (index + 1) / n_waves);
+  const int tiles = SEG ? (int)((a.vocab / n_waves + 1 + 31) / 32) : (row_hi - row_lo + 31) / 32;  // (SEG: barriers inside, so the same for all)
+
+  auto stage = [&](int sb0) __attribute__((always_inline)) {
+    const int n = min(seg_sb, nsb - sb0) * 16;  // groups of 16 per token
+    for (int i = threadIdx.x; i < NT * n; i += (int)blockDim.x) {
+      const int t = i / n, gi = i % n, sb = gi >> 4, pos = gi & 15;
+      const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.t0 + min(t, a.nt - 1)) * a.K + (size_t)sb0 * kSbElems + gi * 16);
+      float x[16];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int row = min(a.row_lo + rg * R + r, a.row_hi - 1);  // a group past the last row repeats it and stores nothing
-      const uint8_t* chunk = a.w + (size_t)row * row_bytes + (size_t)k * F::kChunkBytes;
-      if constexpr (TAIL) stage_load_bounded<QUANT>(chunk, nbytes, a.w_end, pend[r]);
-      else stage_load<QUANT>(chunk, nbytes, pend[r]);
-    }
-    issue_fence();
-  };
-  auto load_x = [&](int k, float (&xl)[TOK][32], float (&xs)[TOK][4]) __attribute__((always_inline)) {
-    const int koff = min(lane_koff<QUANT, 1>(g, k), a.K - F::kBlockElems);
-    const bool act = lane_koff<QUANT, 1>(g, k) < a.K;
-#pragma unroll
-    for (int t = 0; t < TOK; ++t) {
-      float v[32];
-      lane_x_load<QUANT>(a.x + (size_t)(a.t0 + min(t, a.nt - 1)) * a.K, koff, g, v);
-#pragma unroll
-      for (int i = 0; i < 32; ++i) xl[t][i] = act ? v[i] : 0.0f;
-      lane_x_offsets<QUANT>(xl[t], xs[t]);
-    }
-  };
-  auto store = [&](int rg, const float (&acc)[R][TOK]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int t = 0; t < TOK; ++t) {
-      if (t >= a.nt) break;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float tot = group_sum<64>(acc[r][t]);
-        const int row = a.row_lo + rg * R + r;
-        if (g.lane == 0 && row < a.row_hi) a.out[(size_t)(a.t0 + t) * a.vocab + row] = 1.0f * tot;
+      for (int j = 0; j < 4; ++j) {
+        const float4 f = src[j];
+        x[4 * j] = f.x, x[4 * j + 1] = f.y, x[4 * j + 2] = f.z, x[4 * j + 3] = f.w;
       }
+      v4u_t plane[4];
+      float scale;
+      digitize16(x, plane, scale);
+      uint8_t* base = s_x + (size_t)(sb * NT + t) * kSbLdsBytes;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) *reinterpret_cast<v4u_t*>(base + digit_group_offset(pos) + 16 * p) = plane[p];
+      reinterpret_cast<float*>(base + kSbDigitBytes)[scale_group_index(pos)] = scale;
     }
   };
 
-  int rg = (int)blockIdx.x * kWavesPerWg + wave;
-  if (rg >= groups) return;
-  if constexpr (ONE) {
-    float xl[TOK][32], xs[TOK][4];
-    load_x(0, xl, xs);
-    const bool act = lane_koff<QUANT, 1>(g, 0) < a.K;
-    Staged<QUANT> pend[R];
-    issue_w(rg, 0, pend);
-#pragma unroll 1
-    for (; rg < groups; rg += stride) {
-      Raw raw[R];
+  Dma dma[2];
+  int row0 = 0;
+  auto take_tile = [&](int i) __attribute__((always_inline)) {
+    row0 = min(row_lo + 32 * i, a.vocab - 1);
+    const int live = max(1, row_hi - row0);
+    if (i == 0 || live < 32) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) stage_pick<QUANT>(pend[r], slots + (size_t)r * kSlot, act, g, raw[r]);
-      if (rg + stride < groups) issue_w(rg + stride, 0, pend);
-      float acc[R][TOK];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) acc[r][t] = 0.0f;
-        accum<QUANT, TOK>(raw[r], g, xl, xs, acc[r]);
-      }
-      store(rg, acc);
+      for (int u = 0; u < 2; ++u) dma[u].init(row_bytes, min(max(live - 16 * u, 1), 16));
     }
-  } else {
+  };
+  auto run_off = [&](int u) __attribute__((always_inline)) { return (size_t)min(row0 + 16 * u, a.vocab - 1) * row_bytes; };
+  auto request = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) dma[u].request(a.w, a.w_bytes, run_off(u), sb, slot_lds + u * Dma::kRunBytes);
+  };
+  if (tiles > 0) {
+    take_tile(0);
+    request(0);
+  }
+  for (int i = threadIdx.x; i < (int)kHeadZeros / 16; i += (int)blockDim.x) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
+  if constexpr (!SEG) {
+    stage(0);
+    __syncthreads();
+  }
+  const int u = (lane >> 4) & 1, r = lane & 15, h = lane >> 5;
+  for (int i = 0; i < tiles; ++i) {
+    float acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
+    const int my_row = row0 + (lane & 31);
 #pragma unroll 1
-    for (; rg < groups; rg += stride) {
-      float acc[R][TOK];
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int t = 0; t < TOK; ++t) acc[r][t] = 0.0f;
-      Staged<QUANT> pend[R];
-      issue_w(rg, 0, pend);
-#pragma unroll 1
-      for (int k = 0; k < steps; ++k) {
-        float xl[TOK][32], xs[TOK][4];
-        load_x(k, xl, xs);
-        const bool act = lane_koff<QUANT, 1>(g, k) < a.K;
-        Raw raw[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) stage_pick<QUANT>(pend[r], slots + (size_t)r * kSlot, act, g, raw[r]);
-        if (k + 1 < steps) issue_w(rg, k + 1, pend);
-#pragma unroll
-        for (int r = 0; r < R; ++r) accum<QUANT, TOK>(raw[r], g, xl, xs, acc[r]);
+    for (int sb = 0; sb < nsb; ++sb) {
+      if constexpr (SEG) {
+        if (sb % seg_sb == 0) {
+          __syncthreads();
+          stage(sb);
+          __syncthreads();
+        }
       }
-      store(rg, acc);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if ((a.w_bytes & 15) != 0 && sb == nsb - 1 && row0 + 32 >= a.vocab) {
+        // the tensor ends inside a 16-byte piece: its last bytes, which no whole piece holds, two by two
+        const int last_u = (a.vocab - 1 - row0) >> 4, last_r = (a.vocab - 1 - row0) & 15;
+        const size_t tail = a.w_bytes & ~(size_t)15, start = (size_t)(a.vocab - 1) * row_bytes + (size_t)sb * SbRaw<QUANT>::kBytes;
+        uint8_t* p = slot + last_u * Dma::kRunBytes + last_r * (Dma::kP * 16) + (start & 15);
+        if (2 * lane < (int)(a.w_bytes & 15))
+          *reinterpret_cast<uint16_t*>(p + (tail - start) + 2 * lane) = *reinterpret_cast<const uint16_t*>(a.w + tail + 2 * lane);
+        __builtin_amdgcn_wave_barrier();
+      }
+      SbRaw<QUANT> raw;
+      sb_read(dma[0].row_at(slot + u * Dma::kRunBytes, run_off(u), r, sb), h, raw);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (sb + 1 < nsb) {
+        request(sb + 1);
+      } else if (i + 1 < tiles) {
+        take_tile(i + 1);
+        request(0);
+      }
+      LdsDigits x;
+      x.point<NT>(s_x + (size_t)(SEG ? sb % seg_sb : sb) * NT * kSbLdsBytes, s_zero);
+      float v[NT];
+      sb_dot<QUANT, NT>(raw, [&](int s, int l, int tg) { return x.digits(s, l, tg); }, [&](int t, int l) { return x.scales(t, l); }, v);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] += v[t];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float total = acc[t] + __shfl_xor(acc[t], 32, 64);
+      if (h == 0 && my_row < row_hi && t < a.nt) a.out[(size_t)(a.t0 + t) * a.vocab + my_row] = total;
     }
   }
 }
@@ -320,6 +332,24 @@ static size_t format_elements(int format, size_t bytes, size_t* block_bytes) {
   }
 }
 
+template <int QUANT, int NT, bool SEG>
+static int head_raise_lds() {
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_lm_head_quant<QUANT, NT, SEG>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kHeadLdsMax));
+  return XABE_OK;
+}
+template <int QUANT, int... NT>
+static int head_raise_all(std::integer_sequence<int, NT...>) {
+  int st = head_raise_lds<QUANT, 1, true>();
+  ((st = st == XABE_OK ? head_raise_lds<QUANT, NT + 1, false>() : st), ...);
+  return st;
+}
+// at handle creation, not on the launch path (launches are captured into graphs)
+static int head_configure() {
+  XABE_TRY((head_raise_all<kQ8_0>(std::make_integer_sequence<int, (int)kHeadQuantTokens>())));
+  return head_raise_all<kQ6K>(std::make_integer_sequence<int, (int)kHeadQuantTokens>());
+}
+
 }  // namespace xabe
 
 using xabe::set_error;
@@ -393,6 +423,7 @@ int xabe_lm_head_new(const xabe_lm_head_geometry* geometry, xabe_lm_head** out) 
   int dev = 0, cus = 256;
   XABE_HIP_TRY(hipGetDevice(&dev));
   XABE_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  XABE_TRY(xabe::head_configure());
   xabe_lm_head* h = new xabe_lm_head();
   h->g = g;
   h->num_cus = cus;
@@ -412,35 +443,58 @@ int xabe_lm_head_geometry_of(const xabe_lm_head* h, xabe_lm_head_geometry* out) 
 
 namespace xabe {
 
+template <int QUANT, int NT, bool SEG>
+static int launch_quant(unsigned grid, unsigned waves, size_t smem, hipStream_t s, const LmHeadArgs& a) {
+  hipLaunchKernelGGL((k_lm_head_quant<QUANT, NT, SEG>), dim3(grid), dim3(64 * waves), smem, s, a);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
+// One pass of a.nt <= 8 tokens: as many wavefronts per workgroup, up to eight, as the digits leave LDS for.
+template <int QUANT>
+static int launch_quant_pass(const xabe_lm_head* h, hipStream_t s, LmHeadArgs a) {
+  constexpr size_t kSlot = SliceDma<QUANT>::kSlotBytes;
+  const size_t nsb = (size_t)a.K / kSbElems;
+  const size_t digits = nsb * a.nt * kSbLdsBytes;
+  const size_t room = kHeadLdsMax - kHeadZeros;
+  const bool seg = digits + kSlot > room;
+  a.seg_sb = seg ? (int)((room - kSlot) / kSbLdsBytes) : (int)nsb;
+  const size_t waves = seg ? 1 : std::min<size_t>(8, (room - digits) / kSlot);
+  const size_t smem = kHeadZeros + (seg ? (size_t)a.seg_sb * kSbLdsBytes : digits) + waves * kSlot;
+  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(h->num_cus, ((size_t)a.vocab + 32 * waves - 1) / (32 * waves)));
+  if (seg) {  // rows of more than 35 000 elements: one token at a time
+    const int n = a.nt, t0 = a.t0;
+    for (int t = 0; t < n; ++t) {
+      a.t0 = t0 + t;
+      a.nt = 1;
+      XABE_TRY((launch_quant<QUANT, 1, true>(grid, 1, smem, s, a)));
+    }
+    return XABE_OK;
+  }
+  switch (a.nt) {
+    case 1: return launch_quant<QUANT, 1, false>(grid, (unsigned)waves, smem, s, a);
+    case 2: return launch_quant<QUANT, 2, false>(grid, (unsigned)waves, smem, s, a);
+    case 3: return launch_quant<QUANT, 3, false>(grid, (unsigned)waves, smem, s, a);
+    case 4: return launch_quant<QUANT, 4, false>(grid, (unsigned)waves, smem, s, a);
+    case 5: return launch_quant<QUANT, 5, false>(grid, (unsigned)waves, smem, s, a);
+    case 6: return launch_quant<QUANT, 6, false>(grid, (unsigned)waves, smem, s, a);
+    case 7: return launch_quant<QUANT, 7, false>(grid, (unsigned)waves, smem, s, a);
+    default: return launch_quant<QUANT, 8, false>(grid, (unsigned)waves, smem, s, a);
+  }
+}
+
 template <int TOK>
-static void launch_pass(const xabe_lm_head* h, hipStream_t s, int format, const LmHeadArgs& a) {
+static void launch_half_pass(const xabe_lm_head* h, hipStream_t s, bool f16, const LmHeadArgs& a) {
   // rows per wavefront iteration: four for one token, two once the tile's activations take the registers
   constexpr int R = TOK == 1 ? 4 : 2;
-  const int groups = (a.row_hi - a.row_lo + R - 1) / R;
+  const int groups = (a.vocab + R - 1) / R;
   const unsigned grid = (unsigned)std::max(1, std::min((groups + kWavesPerWg - 1) / kWavesPerWg, h->num_cus * 4));
-  const bool one = a.K <= kStepElems;
-  if (a.w_end) {  // the last row of a tensor that ends inside a 16-byte piece: one wavefront, bounded loads
-    if (format == XABE_HEAD_Q8_0) hipLaunchKernelGGL((k_lm_head_quant<kQ8_0, R, TOK, false, true>), dim3(1), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_lm_head_quant<kQ6K, R, TOK, false, true>), dim3(1), dim3(256), 0, s, a);
-    return;
-  }
-  switch (format) {
-    case XABE_HEAD_Q8_0:
-      if (one) hipLaunchKernelGGL((k_lm_head_quant<kQ8_0, R, TOK, true>), dim3(grid), dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((k_lm_head_quant<kQ8_0, R, TOK, false>), dim3(grid), dim3(256), 0, s, a);
-      break;
-    case XABE_HEAD_Q6K:
-      if (one) hipLaunchKernelGGL((k_lm_head_quant<kQ6K, R, TOK, true>), dim3(grid), dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((k_lm_head_quant<kQ6K, R, TOK, false>), dim3(grid), dim3(256), 0, s, a);
-      break;
-    case XABE_HEAD_BF16:
-      if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
-      break;
-    default:
-      if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
-      else hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
-      break;
+  if (f16) {
+    if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
+  } else {
+    if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
   }
 }
 
@@ -473,11 +527,6 @@ int xabe_lm_head_forward(const xabe_lm_head* h, void* stream, int format, const 
   XABE_TRY(check_len("logits", g.max_tokens * g.vocab, logits_len));
   if ((reinterpret_cast<uintptr_t>(weight) & 15u) != 0 || (reinterpret_cast<uintptr_t>(hidden_states) & 15u) != 0)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "LM head: the weight tensor and the hidden states must start on 16-byte boundaries");
-  // the coalesced loader reads whole 16-byte pieces.  A quantized tensor that ends inside one has its last row
-  // served by a launch of its own, whose loads stop at the tensor's end; the 16-byte windows of every earlier
-  // row end inside the last row.
-  const bool quant = format == XABE_HEAD_Q8_0 || format == XABE_HEAD_Q6K;
-  const bool ragged_end = quant && weight_len % 16 != 0;
   hipStream_t s = xabe::as_stream(stream);
   xabe::LmHeadArgs a;
   a.w = static_cast<const uint8_t*>(weight);
@@ -485,23 +534,32 @@ int xabe_lm_head_forward(const xabe_lm_head* h, void* stream, int format, const 
   a.out = logits;
   a.K = (int)g.hidden;
   a.vocab = (int)g.vocab;
-  for (size_t base = 0; base < tokens; base += XABE_LM_HEAD_MAX_BATCH_TILE) {
-    const int tile = (int)std::min<size_t>(XABE_LM_HEAD_MAX_BATCH_TILE, tokens - base);
+  a.w_bytes = weight_len;
+  a.seg_sb = 0;
+  const bool quant = format == XABE_HEAD_Q8_0 || format == XABE_HEAD_Q6K;
+  // passes of equal width: nine tokens as five and four, not as eight and one
+  const size_t most = quant ? xabe::kHeadQuantTokens : XABE_LM_HEAD_MAX_BATCH_TILE;
+  const size_t passes = (tokens + most - 1) / most, width = (tokens + passes - 1) / passes;
+  for (size_t base = 0; base < tokens; base += width) {
+    const int tile = (int)std::min<size_t>(width, tokens - base);
     a.t0 = (int)base;
     a.nt = tile;
-    for (int part = 0; part < (ragged_end ? 2 : 1); ++part) {
-      a.row_lo = part == 0 ? 0 : a.vocab - 1;
-      a.row_hi = ragged_end && part == 0 ? a.vocab - 1 : a.vocab;
-      a.w_end = part == 0 ? nullptr : a.w + weight_len;
-      if (a.row_lo >= a.row_hi) continue;  // a one-row tensor has only the bounded part
-      switch (tile) {
-        case 1: xabe::launch_pass<1>(h, s, format, a); break;
-        case 2: xabe::launch_pass<2>(h, s, format, a); break;
-        case 3: xabe::launch_pass<3>(h, s, format, a); break;
-        default: xabe::launch_pass<4>(h, s, format, a); break;
-      }
-      XABE_HIP_TRY(hipGetLastError());
+    if (format == XABE_HEAD_Q8_0) {
+      XABE_TRY(xabe::launch_quant_pass<xabe::kQ8_0>(h, s, a));
+      continue;
     }
+    if (format == XABE_HEAD_Q6K) {
+      XABE_TRY(xabe::launch_quant_pass<xabe::kQ6K>(h, s, a));
+      continue;
+    }
+    const bool f16 = format == XABE_HEAD_F16;
+    switch (tile) {
+      case 1: xabe::launch_half_pass<1>(h, s, f16, a); break;
+      case 2: xabe::launch_half_pass<2>(h, s, f16, a); break;
+      case 3: xabe::launch_half_pass<3>(h, s, f16, a); break;
+      default: xabe::launch_half_pass<4>(h, s, f16, a); break;
+    }
+    XABE_HIP_TRY(hipGetLastError());
   }
   return XABE_OK;
 }

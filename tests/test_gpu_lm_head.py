@@ -111,6 +111,29 @@ def test_formats_and_shapes(oracle, X, fmt, vocab, hidden, max_tokens, tokens):
     assert np.array_equal(alone[0].view(np.uint32), got[0].view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q6K"])
+@pytest.mark.parametrize("vocab,hidden,tokens", [
+    (33, 512, 8), (2049, 2048, 9), (95, 2048, 6),     # a row past a tile; two passes; ranges shorter than a tile
+    (31, 12288, 7), (70, 36864, 2)])                  # fewer wavefronts for the digits' sake; digits staged in segments
+def test_quantized_passes_at_their_edges(oracle, X, fmt, vocab, hidden, tokens):
+    import torch
+
+    fmt = getattr(X.HeadFormat, fmt)
+    w, host = _weights(X, oracle, fmt, vocab, hidden, 33000 + vocab)
+    k = X.LmHeadKernels(X.LmHeadGeometry(hidden, vocab, tokens))
+    x = X.synth_normal_f32(33001, tokens * hidden, 1.0).view(tokens, hidden)
+    x[0, 5] = 3e4                       # an outlier beside ordinary values in one group of sixteen
+    x[1, 16:32] = 0.0                   # a group of zeros
+    x[1, 32:48] *= 1e-25
+    got = _run(X, k, w, fmt, x, tokens)
+    xs = x.cpu().numpy()
+    for t in range(tokens):
+        ref = host.astype(np.float64) @ xs[t].astype(np.float64)
+        assert np.abs(got[t] - ref).max() <= 1e-6 * np.abs(ref).max(), (str(fmt), t)
+    alone = _run(X, k, w, fmt, x, 1)
+    assert np.array_equal(alone[0].view(np.uint32), got[0].view(np.uint32))
+
+
 def test_forward_error_paths(oracle, X):
     import torch
 
