@@ -261,15 +261,22 @@ __device__ __forceinline__ Cand better(Cand a, Cand b) {
   const bool take_b = b.i >= 0 && (a.i < 0 || b.v > a.v || (b.v == a.v && b.i < a.i));
   return take_b ? b : a;
 }
+template <int CTRL>
+__device__ __forceinline__ Cand dpp_best(Cand c) {
+  const Cand o{dpp_f<CTRL>(c.v), dpp_i<CTRL>(c.i)};
+  return better(c, o);
+}
+__device__ __forceinline__ Cand lane_cand(Cand c, int lane) {
+  return Cand{lane_bcast(c.v, lane), __builtin_amdgcn_readlane(c.i, lane)};
+}
+// The order of the comparisons does not matter (equal values keep the lower index), so the wavefront goes by data
+// parallel moves inside its 16-lane rows and scalar reads across them, without a trip through LDS.
 __device__ __forceinline__ Cand block_best(Cand c, Cand* s) {
-  // wavefront: butterfly through LDS-free lane permutes, then one slot per wavefront
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    Cand o;
-    o.v = __shfl_xor(c.v, d, 64);
-    o.i = __shfl_xor(c.i, d, 64);
-    c = better(c, o);
-  }
+  c = dpp_best<0xB1>(c);
+  c = dpp_best<0x4E>(c);
+  c = dpp_best<0x141>(c);
+  c = dpp_best<0x140>(c);
+  c = better(better(lane_cand(c, 0), lane_cand(c, 16)), better(lane_cand(c, 32), lane_cand(c, 48)));
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) s[wave] = c;
   __syncthreads();
@@ -278,13 +285,29 @@ __device__ __forceinline__ Cand block_best(Cand c, Cand* s) {
   return r;
 }
 
+// Bound by latency (a megabyte of logits over the whole chip): one 16-byte load per thread covers the vocabulary of
+// the shipped model in one round, where a strided scalar loop made two.
 __global__ void __launch_bounds__(256) k_argmax_partial(const float* __restrict__ v, int n, float* __restrict__ pv,
                                                          int* __restrict__ pi) {
   __shared__ Cand s[4];
   Cand c{0.0f, -1};
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const float x = v[i];
+  auto take = [&](float x, int i) __attribute__((always_inline)) {
     if (x == x) c = better(c, Cand{x, i});
+  };
+  const int head = min(n, (int)((16 - (reinterpret_cast<uintptr_t>(v) & 15)) & 15) / 4);  // values before the first 16-byte boundary
+  const int quads = (n - head) / 4;
+  for (int q = blockIdx.x * 256 + threadIdx.x; q < quads; q += gridDim.x * 256) {
+    const float4 x = reinterpret_cast<const float4*>(v + head)[q];
+    const int i = head + 4 * q;
+    take(x.x, i);
+    take(x.y, i + 1);
+    take(x.z, i + 2);
+    take(x.w, i + 3);
+  }
+  if (blockIdx.x == gridDim.x - 1) {
+    if ((int)threadIdx.x < head) take(v[threadIdx.x], threadIdx.x);
+    const int rest = head + 4 * quads + (int)threadIdx.x;
+    if (rest < n) take(v[rest], rest);
   }
   c = block_best(c, s);
   if (threadIdx.x == 0) {
@@ -296,13 +319,11 @@ __global__ void __launch_bounds__(256) k_argmax_partial(const float* __restrict_
 __global__ void __launch_bounds__(256) k_argmax_final(const float* __restrict__ pv, const int* __restrict__ pi, int blocks,
                                                        const float* __restrict__ v, int* __restrict__ out) {
   __shared__ Cand s[4];
-  Cand c{0.0f, -1};
-  for (int b = threadIdx.x; b < blocks; b += 256) c = better(c, Cand{pv[b], pi[b]});
+  const float first = v[0];
+  const int b0 = min((int)threadIdx.x, blocks - 1), b1 = min((int)threadIdx.x + 256, blocks - 1);  // (at most 512)
+  Cand c = better(Cand{pv[b0], pi[b0]}, Cand{pv[b1], pi[b1]});
   c = block_best(c, s);
-  if (threadIdx.x == 0) {
-    const float first = v[0];
-    out[0] = (first != first || c.i < 0) ? 0 : c.i;
-  }
+  if (threadIdx.x == 0) out[0] = (first != first || c.i < 0) ? 0 : c.i;
 }
 
 // 1 / sum(exp(x - max)): one workgroup, a maximum pass and a sum pass, both in a fixed order.
@@ -573,7 +594,7 @@ int xabe_lm_head_argmax(const xabe_lm_head* h, void* stream, const float* values
   XABE_TRY(check_len("argmax partial values", XABE_LM_HEAD_ARGMAX_BLOCKS, partial_values_len));
   XABE_TRY(check_len("argmax partial indices", XABE_LM_HEAD_ARGMAX_BLOCKS, partial_indices_len));
   XABE_TRY(check_len("argmax output", 1, out_len));
-  const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, XABE_LM_HEAD_ARGMAX_BLOCKS);
+  const unsigned blocks = (unsigned)std::min<size_t>((n + 1023) / 1024, XABE_LM_HEAD_ARGMAX_BLOCKS);
   hipStream_t s = xabe::as_stream(stream);
   hipLaunchKernelGGL(xabe::k_argmax_partial, dim3(blocks), dim3(256), 0, s, values, (int)n, partial_values, partial_indices);
   XABE_HIP_TRY(hipGetLastError());
