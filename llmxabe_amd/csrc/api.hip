@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "decode_kernels.h"
+#include "digit_rows.h"
 #include "host_common.h"
 #include "small_kernels.h"
 
@@ -148,142 +149,6 @@ static bool launch_block_resident(Shape shape, const ExpertArgs& a, size_t units
   return true;
 }
 
-constexpr size_t kLongRowsLdsMax = 159 * 1024;  // what a workgroup of the LDS-activation form may ask for
-template <int Q, int NM, int R, int TOK, bool RESID>
-static bool launch_long_rows_lds(const LongRowArgs& la, dim3 grid, dim3 block, size_t smem, hipStream_t s) {
-  hipLaunchKernelGGL((k_shared_long_rows<Q, NM, R, TOK, RESID, true>), grid, block, smem, s, la);
-  return true;
-}
-int long_rows_configure() {
-  static bool done = false;  // (one device per process)
-  if (done) return XABE_OK;
-  const void* fns[2] = {reinterpret_cast<const void*>(k_shared_long_rows<kQ6K, 2, 2, 4, false, true>),
-                        reinterpret_cast<const void*>(k_shared_long_rows<kQ8_0, 2, 2, 4, false, true>)};
-  for (const void* f : fns)
-    XABE_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLongRowsLdsMax));
-  const void* staged[8] = {reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 2, 2, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 2, 2, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 2, 1, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 2, 1, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 1, 4, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 1, 4, false>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 1, 4, true>),
-                           reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 1, 4, true>)};
-  const void* staged10[4] = {reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 1, 2, false, 10>),
-                             reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 1, 2, false, 10>),
-                             reinterpret_cast<const void*>(k_long_rows_staged<kQ6K, 1, 2, true, 10>),
-                             reinterpret_cast<const void*>(k_long_rows_staged<kQ8_0, 1, 2, true, 10>)};
-  for (const void* f : staged10)
-    XABE_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStagedLdsBytes));
-  for (const void* f : staged)
-    XABE_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStagedLdsBytes));
-  done = true;
-  return XABE_OK;
-}
-
-// Rows longer than one step, no expert indirection (dense sibling, wide shared experts): the step-outer
-// kernel, R rows per wavefront (2 for a gate/up pair, 4 for one matrix).  `la.l_out` set: add the residual
-// in the epilogue.
-bool launch_long_rows(const xabe_moe_kernels* k, int quant, int nm, const LongRowArgs& la, hipStream_t s) {
-  const ExpertArgs& a = la.m;
-  if (k->force_community || a.K <= 2048 || !(quant == XABE_QUANT_Q6K || quant == XABE_QUANT_Q8_0)) return false;
-  // rows per wavefront: 2 gate/up pairs or 4 single rows (the step's activations are read once for all of
-  // them).  Wavefronts are independent, so a matrix with few row groups is launched as one-wavefront
-  // workgroups, which spread evenly over the CUs.
-  const int tok = k->g.max_tokens == 1 ? 1 : 2;  // tokens per pass over the weights
-  const int r = nm == 2 ? 2 : 4;
-  if (a.n_rows % (kWavesPerWg * r) != 0) return false;
-  const unsigned passes = (unsigned)((k->g.max_tokens + tok - 1) / tok);
-  const int groups = a.n_rows / r;
-  const unsigned waves = (size_t)groups / kWavesPerWg * passes < (size_t)4 * k->num_cus ? 1 : kWavesPerWg;
-  if (groups / waves > 0x7fffffffu / 64) return false;
-  dim3 grid((unsigned)groups / waves, passes), block(64 * waves);
-  const bool resid = la.l_out != nullptr;
-  // the coalesced loader reads whole 16-byte pieces: the tensors must start and end on 16-byte boundaries
-  const size_t row_bytes = (size_t)a.K / xabe_expert_quant_block_elements(quant) * xabe_expert_quant_block_bytes(quant);
-  auto on16 = [&](const uint8_t* w) { return !w || (reinterpret_cast<uintptr_t>(w) % 16 == 0 && ((size_t)a.n_rows * row_bytes) % 16 == 0); };
-  if (!(on16(a.w0) && on16(a.w1))) return false;
-  // Five tokens or more: eight tokens per pass, the step's activations staged in LDS for the whole workgroup
-  // (k_long_rows_staged); one workgroup of eight wavefronts per CU, persistent over groups of 8 r rows.
-  if (k->g.max_tokens >= 5 && a.n_rows % (8 * r) == 0 && a.K % 256 == 0 &&
-      (size_t)k->g.max_tokens * (size_t)a.K * sizeof(float) < ((size_t)1 << 32) && reinterpret_cast<uintptr_t>(a.x) % 16 == 0) {
-    const unsigned pass8 = (unsigned)((k->g.max_tokens + kStagedTok - 1) / kStagedTok);
-    const unsigned groups8 = (unsigned)(a.n_rows / (8 * r));
-    dim3 grid8(std::min<unsigned>(groups8, (unsigned)k->num_cus), pass8), block8(512);
-    // a single matrix whose groups of 32 rows leave CUs idle while groups of 20 fill them (the dense sibling's down
-    // projection: 5120 rows, 160 against 256 groups): ten wavefronts of two rows
-    const bool ten = nm == 1 && a.n_rows % 20 == 0 && groups8 < (unsigned)k->num_cus && (unsigned)(a.n_rows / 20) >= groups8 * 3 / 2;
-    const dim3 grid10(std::min<unsigned>((unsigned)(a.n_rows / 20), (unsigned)k->num_cus), pass8), block10(640);
-    // gate/up whose groups do not divide evenly over the CUs (17408 row pairs: 1088 groups of 16 on 256 CUs, a fifth
-    // round for a quarter of them): whole rounds in the main launch, the left-over rows as half-size groups (one row
-    // pair per wavefront) spread over twice as many CUs in a second launch
-    LongRowArgs la_main = la, la_rest = la;
-    unsigned rest_groups = 0;
-    if (nm == 2 && groups8 > (unsigned)k->num_cus && groups8 % (unsigned)k->num_cus != 0 &&
-        2 * (groups8 % (unsigned)k->num_cus) <= (unsigned)k->num_cus) {
-      const unsigned whole = groups8 / (unsigned)k->num_cus * (unsigned)k->num_cus;
-      la_main.row_begin = 0;
-      la_main.row_end = (int)(whole * 8 * r);
-      la_rest.row_begin = la_main.row_end;
-      la_rest.row_end = a.n_rows;
-      rest_groups = (groups8 - whole) * 2;
-    }
-#define XABE_STAGED(Q)                                                                                                          \
-  do {                                                                                                                          \
-    if (nm == 2) {                                                                                                              \
-      hipLaunchKernelGGL((k_long_rows_staged<Q, 2, 2, false>), grid8, block8, kStagedLdsBytes, s, la_main);                     \
-      if (rest_groups)                                                                                                          \
-        hipLaunchKernelGGL((k_long_rows_staged<Q, 2, 1, false>), dim3(rest_groups, pass8), block8, kStagedLdsBytes, s, la_rest); \
-    }                                                                                                                           \
-    else if (ten && resid) hipLaunchKernelGGL((k_long_rows_staged<Q, 1, 2, true, 10>), grid10, block10, kStagedLdsBytes, s, la); \
-    else if (ten) hipLaunchKernelGGL((k_long_rows_staged<Q, 1, 2, false, 10>), grid10, block10, kStagedLdsBytes, s, la);        \
-    else if (resid) hipLaunchKernelGGL((k_long_rows_staged<Q, 1, 4, true>), grid8, block8, kStagedLdsBytes, s, la);             \
-    else hipLaunchKernelGGL((k_long_rows_staged<Q, 1, 4, false>), grid8, block8, kStagedLdsBytes, s, la);                       \
-  } while (0)
-    if (quant == XABE_QUANT_Q6K) XABE_STAGED(kQ6K);
-    else XABE_STAGED(kQ8_0);
-#undef XABE_STAGED
-    return true;
-  }
-  // Three tokens or more, gate/up: four tokens per pass with the activation rows in LDS (the kernel's XLDS form),
-  // where four rows and eight wavefronts' staging slots fit; eight wavefronts per workgroup, one workgroup per
-  // CU and pass, persistent over the row groups.  (Down's rows are too long for four of them to fit.)
-  if (nm == 2 && k->g.max_tokens >= 3 && a.K % 4 == 0) {
-    const int tokx = 4;
-    const unsigned wv = 8;
-    const size_t slot = (size_t)r * nm * (quant == XABE_QUANT_Q6K ? StageFmt<kQ6K>::kSlotBytes : StageFmt<kQ8_0>::kSlotBytes);
-    const size_t smem = (size_t)tokx * a.K * sizeof(float) + wv * slot;
-    if (smem <= kLongRowsLdsMax) {
-      const unsigned passx = (unsigned)((k->g.max_tokens + tokx - 1) / tokx);
-      dim3 gridx((unsigned)std::min<size_t>(((size_t)groups + wv - 1) / wv, (size_t)k->num_cus), passx), blockx(64 * wv);
-      if (quant == XABE_QUANT_Q6K) return launch_long_rows_lds<kQ6K, 2, 2, 4, false>(la, gridx, blockx, smem, s);
-      return launch_long_rows_lds<kQ8_0, 2, 2, 4, false>(la, gridx, blockx, smem, s);
-    }
-  }
-#define XABE_LONG4(Q, TOK, R)                                                                                    \
-  do {                                                                                                            \
-    if (nm == 2) hipLaunchKernelGGL((k_shared_long_rows<Q, 2, R, TOK, false>), grid, block, 0, s, la);            \
-    else if (resid) hipLaunchKernelGGL((k_shared_long_rows<Q, 1, R, TOK, true>), grid, block, 0, s, la);          \
-    else hipLaunchKernelGGL((k_shared_long_rows<Q, 1, R, TOK, false>), grid, block, 0, s, la);                    \
-  } while (0)
-#define XABE_LONG3(Q, TOK)                              \
-  do {                                                  \
-    if (nm == 2) XABE_LONG4(Q, TOK, 2);                 \
-    else XABE_LONG4(Q, TOK, 4);                         \
-  } while (0)
-#define XABE_LONG(Q)                  \
-  do {                                \
-    if (tok == 1) XABE_LONG3(Q, 1);   \
-    else XABE_LONG3(Q, 2);            \
-  } while (0)
-  if (quant == XABE_QUANT_Q6K) XABE_LONG(kQ6K);
-  else XABE_LONG(kQ8_0);
-#undef XABE_LONG4
-#undef XABE_LONG3
-#undef XABE_LONG
-  return true;
-}
-
 int pick_tile_rows(const xabe_moe_kernels* k, size_t live_units, int n_rows, int rps) {
   // aim for ~12 wavefronts per CU across the launch
   const size_t items = std::max<size_t>(1, live_units) * (size_t)n_rows / rps;
@@ -305,15 +170,6 @@ static int launch_expert(const xabe_moe_kernels* k, Mode mode, int quant, int nm
     if (quant == XABE_QUANT_Q6K) done = nm == 2 ? launch_block_resident<kQ6K, 2>(shape, a, units, s) : launch_block_resident<kQ6K, 1>(shape, a, units, s);
     else if (quant == XABE_QUANT_Q8_0) done = nm == 2 ? launch_block_resident<kQ8_0, 2>(shape, a, units, s) : launch_block_resident<kQ8_0, 1>(shape, a, units, s);
     if (done) {
-      XABE_HIP_TRY(hipGetLastError());
-      return XABE_OK;
-    }
-  }
-  if (mode == kShared && a.expert_bytes == 0) {
-    LongRowArgs la;
-    memset(&la, 0, sizeof(la));
-    la.m = a;
-    if (launch_long_rows(k, quant, nm, la, s)) {
       XABE_HIP_TRY(hipGetLastError());
       return XABE_OK;
     }
@@ -471,7 +327,7 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
                      prop.gcnArchName);
   // a code object that does not load shows up here rather than at the first launch
   hipFuncAttributes attr;
-  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows));
+  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows<false>));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return set_error(XABE_ERR_COMPILE, "kernel load failed: %s", hipGetErrorString(e));
@@ -485,7 +341,7 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
   k->num_cus = prop.multiProcessorCount;
   // everything one-time happens here, none of it on the launch path (launches are captured into graphs)
   int st = mfma_configure();
-  if (st == XABE_OK) st = long_rows_configure();
+  if (st == XABE_OK) st = digit_rows_configure();
   if (st != XABE_OK) {
     delete k;
     return st;
@@ -574,6 +430,13 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->inter, b->n_inter);
   A(&b->partial, b->n_partial);
   A(&b->shared_inter, b->n_shared_inter);
+  const size_t nsb_h = digit_superblocks(g.hidden), nsb_i = digit_superblocks(g.intermediate);
+  A(&b->x_d, g.max_tokens * nsb_h * kSbDigitBytes);
+  A(&b->x_e, g.max_tokens * nsb_h * 16);
+  A(&b->inter_d, (routed ? sorted : 0) * nsb_i * kSbDigitBytes);
+  A(&b->inter_e, (routed ? sorted : 0) * nsb_i * 16);
+  A(&b->shared_inter_d, g.max_tokens * nsb_i * kSbDigitBytes);
+  A(&b->shared_inter_e, g.max_tokens * nsb_i * 16);
   // matrix-core staging: only passes wide enough to take that regime pay for it
   A(&b->x_h, (wide && mma) ? g.max_tokens * g.hidden : 0);
   A(&b->inter_h, (wide && mma && routed) ? sorted * g.intermediate : 0);
@@ -607,7 +470,8 @@ void xabe_moe_buffers_free(xabe_moe_buffers* b) {
   if (!b) return;
   void* ptrs[] = {b->topk_ids, b->topk_weights, b->sorted_token_ids, b->expert_ids, b->bucket_live, b->expert_counts,
                   b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->inter, b->partial, b->shared_inter, b->x_h, b->inter_h,
-                  b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals};
+                  b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals,
+                  b->x_d, b->x_e, b->inter_d, b->inter_e, b->shared_inter_d, b->shared_inter_e};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete b;
@@ -864,9 +728,56 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
   return XABE_OK;
 }
 
+static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
+  RowsArgs a;
+  memset(&a, 0, sizeof(a));
+  a.valid_tokens = b->valid_tokens;
+  a.topk_ids = b->topk_ids;
+  a.topk_weights = b->topk_weights;
+  a.sorted_token_ids = b->sorted_token_ids;
+  a.expert_ids = b->expert_ids;
+  a.top_k = (int)k->g.experts_per_token;
+  a.block_size = (int)k->g.block_size;
+  return a;
+}
+
+// gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->x_d
+static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
+                         xabe_quant_tensor up, xabe_quant_tensor down, float* out, const float* residual = nullptr,
+                         float* l_out = nullptr) {
+  const xabe_moe_geometry& g = k->g;
+  RowsArgs a = rows_args(k, b);
+  a.w0 = static_cast<const uint8_t*>(gate.bytes);
+  a.w1 = static_cast<const uint8_t*>(up.bytes);
+  a.w_bytes = gate.len;
+  a.xd = b->x_d;
+  a.xe = b->x_e;
+  a.out = b->shared_inter;
+  a.out_d = b->shared_inter_d;
+  a.out_e = b->shared_inter_e;
+  a.K = (int)g.hidden;
+  a.n_rows = (int)g.intermediate;
+  XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, 0, s));
+  a.w0 = static_cast<const uint8_t*>(down.bytes);
+  a.w1 = nullptr;
+  a.w_bytes = down.len;
+  a.xd = b->shared_inter_d;
+  a.xe = b->shared_inter_e;
+  a.out = out;
+  a.residual = residual;
+  a.l_out = l_out;
+  a.K = (int)g.intermediate;
+  a.n_rows = (int)g.hidden;
+  return launch_digit_rows(k, kRowsShared, down.quant, 1, a, 0, s);
+}
+
 static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
   const xabe_moe_geometry& g = k->g;
+  if (g.hidden > 2048) {
+    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->x_d, b->x_e));
+    return shared_digits(k, s, b, gate, up, down, out);
+  }
   const size_t units = (g.max_tokens + 1) / 2;
   ExpertArgs a = base_args(k, b);
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
@@ -887,49 +798,20 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   return XABE_OK;
 }
 
-// The dense block's fp32 path on the long-row kernel, the residual folded into down: three launches.
-// Returns false (nothing launched) where the long-row kernel does not apply.
-static int check_shared_stacks(const xabe_moe_kernels* k, xabe_quant_tensor gate, xabe_quant_tensor up,
-                               xabe_quant_tensor down);
-
+// The dense block's fp32 path: the norm launch writes the digits, down adds the residual; three launches.
 int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                            xabe_quant_tensor up, xabe_quant_tensor down, const float* post_norm, float eps,
                            const float* residual, float* normed, float* ffn_out, float* l_out, bool* launched) {
   const xabe_moe_geometry& g = k->g;
   *launched = false;
   XABE_TRY(check_shared_stacks(k, gate, up, down));  // the checks xabe_moe_shared_expert makes
-  LongRowArgs la;
-  memset(&la, 0, sizeof(la));
-  la.m = base_args(k, b);
-  la.m.w0 = static_cast<const uint8_t*>(gate.bytes);
-  la.m.w1 = static_cast<const uint8_t*>(up.bytes);
-  // (normalising on load was tried: with thousands of wavefronts each re-deriving the RMS scale of every
-  // token it costs more than the stand-alone RMSNorm launch it saves)
-  XABE_TRY(xabe_rms_norm(s, residual, g.max_tokens * g.hidden, post_norm, g.hidden, normed, g.max_tokens * g.hidden,
-                         g.max_tokens, g.hidden, eps));
-  la.m.x = normed;
-  la.m.out = b->shared_inter;
-  la.m.K = (int)g.hidden;
-  la.m.n_rows = (int)g.intermediate;
-  LongRowArgs ld;
-  memset(&ld, 0, sizeof(ld));
-  ld.m = base_args(k, b);
-  ld.m.w0 = static_cast<const uint8_t*>(down.bytes);
-  ld.m.x = b->shared_inter;
-  ld.m.out = ffn_out;
-  ld.m.K = (int)g.intermediate;
-  ld.m.n_rows = (int)g.hidden;
-  ld.residual = residual;
-  ld.l_out = l_out;
-  // both or neither: check the second shape before launching the first
-  const int r_up = 2, r_down = 4;
-  if (k->force_community || g.hidden <= 2048 || g.intermediate <= 2048) return XABE_OK;
-  if (g.intermediate % (kWavesPerWg * r_up) != 0 || g.hidden % (kWavesPerWg * r_down) != 0) return XABE_OK;
-  auto ok = [](int q) { return q == XABE_QUANT_Q6K || q == XABE_QUANT_Q8_0; };
-  if (!ok(gate.quant) || !ok(down.quant)) return XABE_OK;
-  if (!launch_long_rows(k, gate.quant, 2, la, s) || !launch_long_rows(k, down.quant, 1, ld, s))
-    return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "dense block: the long-row kernel refused a shape it was checked for");
+  if (g.hidden <= 2048) return XABE_OK;
+  if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(post_norm)) % 16 != 0)
+    return set_error(XABE_ERR_INVALID_ARGUMENT, "rms_norm: x, weight and out must be 16-byte aligned");
+  hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)g.max_tokens), dim3(256), 0, s, residual, post_norm, normed, (int)g.hidden,
+                     eps, b->x_d, b->x_e);
   XABE_HIP_TRY(hipGetLastError());
+  XABE_TRY(shared_digits(k, s, b, gate, up, down, ffn_out, residual, l_out));
   *launched = true;
   return XABE_OK;
 }
@@ -1028,7 +910,8 @@ int xabe_rms_norm(void* stream, const float* x, size_t x_len, const float* weigh
     hipLaunchKernelGGL(k_rms_norm_short_rows<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream), x, weight, out,
                        static_cast<_Float16*>(nullptr), (int)rows, (int)width, eps);
   else
-    hipLaunchKernelGGL(k_rms_norm_rows, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out, (int)width, eps);
+    hipLaunchKernelGGL(k_rms_norm_rows<false>, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out, (int)width, eps,
+                       static_cast<uint8_t*>(nullptr), static_cast<float*>(nullptr));
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }

@@ -1,0 +1,85 @@
+// Interface of the digit row contractions (digit_rows.hip) and the device helpers that write digits.
+#pragma once
+
+#include "digits.h"
+
+struct xabe_moe_kernels;
+
+namespace xabe {
+
+constexpr int kRowsFlat = 0;    // one (token, k) pair per unit, straight from topk_ids
+constexpr int kRowsBlock = 1;   // one dispatch block per unit: one expert, its run of tokens
+constexpr int kRowsShared = 2;  // every live token, one matrix
+constexpr int kRowsMaxTiles = 5;  // tiles of one wavefront's share whose sums it keeps in registers
+
+inline __host__ __device__ size_t digit_superblocks(size_t K) { return (K + kSbElems - 1) / kSbElems; }
+
+struct RowsArgs {
+  const uint8_t* w0;         // gate stack (nm = 2) or the one matrix
+  const uint8_t* w1;         // up stack (nm = 2)
+  size_t w_bytes;            // length of each stack
+  size_t expert_bytes;       // bytes of one expert in a stack (0: a single matrix)
+  const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes]
+  const float* xe;           // their group scales, [row][superblock][16]
+  float* out;                // [row][n_rows]; nm = 2: may be null
+  uint8_t* out_d;            // nm = 2: digits of the output rows
+  float* out_e;
+  const float* residual;     // with l_out: l_out = out + residual
+  float* l_out;
+  const int* valid_tokens;
+  const int* topk_ids;
+  const float* topk_weights;
+  const int* sorted_token_ids;
+  const int* expert_ids;
+  int K, n_rows, top_k, block_size;
+  // filled in by launch_digit_rows
+  int nsb, out_nsb, classes, tile_rows, n_tiles;
+  uint32_t row_bytes;
+};
+
+__device__ __forceinline__ void dma_16b(const uint8_t* base, uint32_t voff, uint32_t dst) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+// Group `gi` of a row, its sixteen values in `v`, into the row's digit planes and scales (zeros where the group lies
+// past the row's end).
+__device__ __forceinline__ void store_digits16(float (&v)[16], int gi, bool in, uint8_t* xd, float* xe) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = in ? v[i] : 0.0f;
+  v4u_t plane[4];
+  float scale;
+  digitize16(v, plane, scale);
+  uint8_t* d = xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) reinterpret_cast<v4u_t*>(d)[p] = plane[p];
+  xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = in ? scale : 0.0f;
+}
+
+// The same for a group that sixteen consecutive lanes (a DPP row) hold one element each: lane's value `v` is element
+// `row` of the output row whose digits start at xd and scales at xe.
+__device__ __forceinline__ void store_digit_group(float v, int row, int nsb, uint8_t* xd, float* xe, bool live) {
+  int mag = (int)(__builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+  mag = max(mag, dpp_i<0xB1>(mag));
+  mag = max(mag, dpp_i<0x4E>(mag));
+  mag = max(mag, dpp_i<0x141>(mag));
+  mag = max(mag, dpp_i<0x140>(mag));
+  const int e = mag >> 23, s = min(156 - e, 126);
+  const uint32_t y = ((uint32_t)(int)__builtin_rintf(__builtin_ldexpf(v, s)) + 0x00808080u) ^ 0x00808080u;
+  if (!live) return;
+  const int gi = row >> 4, j = row & 15;
+  uint8_t* d = xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15) + j;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) d[16 * p] = (uint8_t)(y >> (24 - 8 * p));
+  if (j == 0) xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = e == 255 ? __builtin_nanf("") : __builtin_ldexpf(1.0f, 16 - s);
+}
+
+// host side
+int digit_rows_configure();
+int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
+// `units`: pairs (flat) or dispatch blocks (block); token chunks are counted here
+int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s);
+
+}  // namespace xabe

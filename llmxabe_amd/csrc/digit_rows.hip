@@ -1,0 +1,366 @@
+// The fp32 regimes' row contractions on the digit core (digits.h): quantized rows of one matrix, or of a gate/up pair
+// with SwiGLU between them, against the tokens of a work unit.  Replaces the reference's gemv / flat / tiled fp32
+// families (crates/xabe-cuda/src/kernels/moe.rs:2403-3124, :3425-3725, :4082-4227).
+//
+// A workgroup is eight wavefronts over the row tiles of its share (32 rows, or 16 gate and the 16 matching up rows).
+// The contraction is split between the wavefronts by superblock class (superblock mod 8; rows of fewer than eight
+// superblocks leave several wavefronts per class, which take the tiles in turn), so that a wavefront meets few
+// superblocks of activations and reuses their digits, held in registers, for every tile of its share.
+//
+// Order of operations per (row, token), whatever the launch shape: a class sums its superblocks in order, each half of
+// the wavefront its own groups; the classes are added in order, then half 0 + half 1.  A token's row is therefore the
+// same bits alone, in a batch, in any mode.
+#include <string.h>
+
+#include <algorithm>
+
+#include "digit_rows.h"
+#include "host_common.h"
+
+namespace xabe {
+
+// Digits of fp32 rows: one thread per group of sixteen; groups past the end of the row are zeros with scale zero.
+__global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__ x, int K, int nsb, int rows, uint8_t* __restrict__ xd,
+                                                       float* __restrict__ xe) {
+  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (i >= rows * nsb * 16) return;
+  const int row = i / (nsb * 16), gi = i % (nsb * 16);
+  float v[16];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(4 * gi + j, K / 4 - 1)];
+    v[4 * j] = f.x, v[4 * j + 1] = f.y, v[4 * j + 2] = f.z, v[4 * j + 3] = f.w;
+  }
+  store_digits16(v, gi, gi * 16 < K, xd + (size_t)row * nsb * kSbDigitBytes, xe + (size_t)row * nsb * 16);
+}
+
+constexpr int kRowsZeros = 1024;
+
+template <int QUANT, int NT, bool TAIL>
+struct RowsLds {
+  using Dma = SliceDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
+  static constexpr int kDigits = NT * kSbDigitBytes, kScales = NT * kSbScaleBytes;
+  static constexpr int kPerWave = Dma::kSlotBytes + kDigits + 2 * kScales;
+};
+
+template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+__global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
+  using L = RowsLds<QUANT, NT, TAIL>;
+  using Dma = typename L::Dma;
+  constexpr int TG = (NT + 3) / 4;
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
+  const int lane = (int)__lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int valid = *a.valid_tokens;
+  // ---- the unit's weights and token rows
+  size_t e_off = 0;
+  int n_tok, pair = 0;
+  const int* slots = nullptr;
+  size_t slot0 = 0;
+  if constexpr (MODE == kRowsFlat) {
+    pair = (int)blockIdx.y;
+    if (pair >= valid * a.top_k) return;
+    e_off = (size_t)a.topk_ids[pair] * a.expert_bytes;
+    n_tok = 1;
+  } else if constexpr (MODE == kRowsBlock) {
+    const int e = a.expert_ids[blockIdx.y];
+    if (e < 0) return;
+    e_off = (size_t)e * a.expert_bytes;
+    slot0 = (size_t)blockIdx.y * a.block_size;
+    slots = a.sorted_token_ids + slot0;
+    n_tok = a.block_size;
+  } else {
+    slot0 = (size_t)blockIdx.y * NT;
+    if ((int)slot0 >= valid) return;
+    n_tok = min(NT, valid - (int)slot0);
+  }
+  const int sentinel = valid * a.top_k;
+
+  // ---- this wavefront's class and tiles
+  const int classes = a.classes, per_class = 8 / classes;
+  const int cls = wave % classes, sub = wave / classes;
+  const int tile_lo = (int)((long long)a.n_tiles * (int)blockIdx.x / (int)gridDim.x);
+  const int n_wg = (int)((long long)a.n_tiles * ((int)blockIdx.x + 1) / (int)gridDim.x) - tile_lo;  // <= MT * per_class
+  const int n_mine = (n_wg - sub + per_class - 1) / per_class;
+  const int nsb = a.nsb;
+  const uint32_t row_bytes = a.row_bytes;
+  uint8_t* const s_zero = s_rows;
+  uint8_t* const w_slot = s_rows + kRowsZeros + (size_t)wave * L::kPerWave;
+  uint8_t* const d_slot = w_slot + Dma::kSlotBytes;
+  uint8_t* const e_slot = d_slot + L::kDigits;
+  auto lds_addr = [](uint8_t* p) __attribute__((always_inline)) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p);
+  };
+  const uint32_t w_lds = lds_addr(w_slot), d_lds = lds_addr(d_slot), e_lds = lds_addr(e_slot);
+  for (int i = threadIdx.x; i < kRowsZeros / 16; i += 512) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
+
+  // rows of tile i of this wavefront: run 0 and run 1 (NM == 2: gate and up, the same 16 rows of each)
+  const int tile_rows = NM == 2 ? 16 : a.tile_rows;
+  auto tile_of = [&](int i) __attribute__((always_inline)) { return tile_lo + sub + per_class * i; };
+  auto run_row = [&](int i, int u) __attribute__((always_inline)) {
+    const int row = tile_of(i) * tile_rows + (NM == 2 ? 0 : 16 * u);
+    return min(row, a.n_rows - 1);
+  };
+  Dma dma[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) dma[u].init(row_bytes, NM == 2 ? 16 : min(max(tile_rows - 16 * u, 1), 16));
+  auto request_w = [&](int i, int sb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      dma[u].request(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, e_off + (size_t)run_row(i, u) * row_bytes, sb, w_lds + u * Dma::kRunBytes);
+  };
+  const int u_lane = (lane >> 4) & 1, r_lane = lane & 15, half = lane >> 5;
+
+  for (int first = 0; first < n_tok; first += NT) {
+    // the chunk's tokens: activation rows (tokens past the live ones repeat one of them and are never stored)
+    int x_row[NT], n_live = 0;
+    if constexpr (MODE == kRowsFlat) {
+      x_row[0] = NM == 2 ? pair / a.top_k : pair;
+      n_live = 1;
+    } else if constexpr (MODE == kRowsBlock) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int f = first + t < n_tok ? slots[first + t] : sentinel;
+        const bool live = f < sentinel && n_live == t;
+        if (live) ++n_live;
+        x_row[t] = NM == 2 ? (live ? f : slots[first]) / a.top_k : (int)slot0 + first + (live ? t : 0);
+      }
+      if (n_live == 0) break;
+    } else {
+      n_live = n_tok;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x_row[t] = (int)slot0 + min(t, n_live - 1);
+    }
+    int x_row_l = x_row[NT - 1];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if ((lane >> 2) == t) x_row_l = x_row[t];
+    auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        dma_16b(a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
+      if (lane < 4 * NT)  // (64 bytes per token)
+        dma_16b(reinterpret_cast<const uint8_t*>(a.xe), ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16,
+                e_lds + buf * L::kScales);
+    };
+
+    float acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[i][t] = 0.0f;
+    if (first == 0) __syncthreads();  // the zeros are there
+    if (cls < nsb && n_mine > 0) {
+      request_w(0, cls);
+      request_x(cls, 0);
+    }
+    int buf = 0;
+    if (n_mine > 0) {
+#pragma unroll 1
+      for (int sb = cls; sb < nsb; sb += classes, buf ^= 1) {
+        v4i_t ax[8][TG];
+        LdsDigits<NT, kSbDigitBytes> x;
+#pragma unroll 1
+        for (int i = 0; i < n_mine; ++i) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          if (i == 0) {
+            x.point(d_slot, e_slot + buf * L::kScales, s_zero);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+              for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.digit(j & 3, j >> 2, tg);
+          }
+          if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const size_t off = e_off + (size_t)run_row(i, u) * row_bytes;
+              const int live = min(min(tile_rows - (NM == 2 ? 0 : 16 * u), 16), a.n_rows - (tile_of(i) * tile_rows + (NM == 2 ? 0 : 16 * u)));
+              if (live >= 1 && off + (size_t)live * row_bytes == a.w_bytes) dma[u].patch_tail(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, off, live, sb, w_slot + u * Dma::kRunBytes);
+            }
+          }
+          SbRaw<QUANT> raw;
+          sb_read(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          if (i + 1 < n_mine) {
+            request_w(i + 1, sb);
+          } else if (sb + classes < nsb) {
+            request_w(0, sb + classes);
+            request_x(sb + classes, buf ^ 1);
+          }
+          float v[NT];
+          sb_dot<QUANT, NT, TAIL>(raw, [&](int s, int l, int tg) { return ax[4 * l + s][tg]; },
+                                  [&](int t, int l) { return x.template scale<kSbScaleBytes>(t, l); }, v,
+                                  TAIL && half == 1 && (sb * kSbElems + 128) >= a.K);
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {  // (the sums stay in registers: the tile's own by a uniform branch, not by an index)
+            if (MT > 1 && m != i) continue;
+            if (MT > 1) asm volatile("");
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[m][t] += v[t];
+          }
+        }
+      }
+    }
+
+    // ---- classes meet in LDS (over the slots, which everyone is done with)
+    __syncthreads();
+    float* const red = reinterpret_cast<float*>(s_rows + kRowsZeros);  // [class][tile of the workgroup][token][64]
+    const int span = MT * per_class;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if (i >= n_mine) continue;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) red[(((size_t)cls * span + sub + per_class * i) * NT + t) * 64 + lane] = acc[i][t];
+    }
+    __syncthreads();
+    const int live_classes = min(classes, nsb);
+    auto total = [&](int tl, int t, int col) __attribute__((always_inline)) {
+      float h[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float* p = red + ((size_t)tl * NT + t) * 64 + 32 * q + col;
+        float v = p[0];
+        for (int c = 1; c < live_classes; ++c) v += p[(size_t)c * span * NT * 64];
+        h[q] = v;
+      }
+      return h[0] + h[1];
+    };
+    constexpr int kCols = NM == 2 ? 16 : 32;
+    for (int i = threadIdx.x; i < n_wg * NT * kCols; i += 512) {
+      const int col = i % kCols, t = i / kCols % NT, tl = i / (kCols * NT);
+      const int row = (tile_lo + tl) * tile_rows + col;
+      const bool live = t < n_live && col < tile_rows && row < a.n_rows;
+      size_t o_row = 0;
+      float scale = 1.0f;
+      if constexpr (MODE == kRowsFlat) {
+        o_row = pair;
+        if (NM == 1) scale = a.topk_weights[pair];
+      } else if constexpr (MODE == kRowsBlock) {
+        if (NM == 2) {
+          o_row = slot0 + first + t;
+        } else {
+          const int f = slots[min(first + t, n_tok - 1)];
+          o_row = live ? (size_t)f : 0;
+          if (live) scale = a.topk_weights[f];
+        }
+      } else {
+        o_row = slot0 + t;
+      }
+      if constexpr (NM == 2) {
+        const float v = silu_f(total(tl, t, col)) * total(tl, t, col + 16);
+        if (live && a.out) a.out[o_row * a.n_rows + row] = v;
+        // sixteen consecutive threads hold one group of the next contraction's activations
+        store_digit_group(v, row, a.out_nsb, a.out_d + o_row * a.out_nsb * kSbDigitBytes, a.out_e + o_row * a.out_nsb * 16, live);
+      } else {
+        const float v = scale * total(tl, t, col);
+        if (live) {
+          a.out[o_row * a.n_rows + row] = v;
+          if (a.l_out) a.l_out[o_row * a.n_rows + row] = v + a.residual[o_row * a.n_rows + row];
+        }
+      }
+    }
+    if (first + NT < n_tok) __syncthreads();  // (before the next chunk's requests land in the slots)
+  }
+}
+
+// ------------------------------------------------------------------ host side
+template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+static size_t rows_lds() {
+  const size_t slots = (size_t)8 * RowsLds<QUANT, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * 64 * sizeof(float);
+  return kRowsZeros + std::max(slots, red);
+}
+
+template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+static int rows_go(dim3 grid, hipStream_t s, const RowsArgs* a) {
+  const size_t smem = rows_lds<MODE, QUANT, NM, NT, MT, TAIL>();
+  if (!a) {  // (at handle creation: the LDS limit)
+    XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_rows<MODE, QUANT, NM, NT, MT, TAIL>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    return XABE_OK;
+  }
+  hipLaunchKernelGGL((k_digit_rows<MODE, QUANT, NM, NT, MT, TAIL>), grid, dim3(512), smem, s, *a);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
+template <int MODE, int NM, int NT, int MT>
+static int rows_quant(int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
+  if (quant == XABE_QUANT_Q6K) return rows_go<MODE, kQ6K, NM, NT, MT, false>(grid, s, a);
+  return tail ? rows_go<MODE, kQ8_0, NM, NT, MT, true>(grid, s, a) : rows_go<MODE, kQ8_0, NM, NT, MT, false>(grid, s, a);
+}
+
+template <int NM, int MT>
+static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
+  switch (nt) {
+    case 1: return rows_quant<kRowsShared, NM, 1, MT>(quant, tail, grid, s, a);
+    case 2: return rows_quant<kRowsShared, NM, 2, MT>(quant, tail, grid, s, a);
+    case 4: return rows_quant<kRowsShared, NM, 4, MT>(quant, tail, grid, s, a);
+    default: return rows_quant<kRowsShared, NM, 8, MT>(quant, tail, grid, s, a);
+  }
+}
+
+template <int NM>
+static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
+  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, 1>(quant, tail, grid, s, a);
+  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, 4, 1>(quant, tail, grid, s, a);
+  return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
+}
+
+int digit_rows_configure() {
+  static bool done = false;  // (one device per process)
+  if (done) return XABE_OK;
+  for (int q : {XABE_QUANT_Q6K, XABE_QUANT_Q8_0})
+    for (bool tail : {false, true})
+      for (int mode : {kRowsFlat, kRowsBlock, kRowsShared})
+        for (int nt : {1, 2, 4, 8})
+          for (int mt : {1, kRowsMaxTiles}) {
+            XABE_TRY(rows_mode<1>(mode, nt, mt, q, tail, dim3(1), nullptr, nullptr));
+            XABE_TRY(rows_mode<2>(mode, nt, mt, q, tail, dim3(1), nullptr, nullptr));
+          }
+  done = true;
+  return XABE_OK;
+}
+
+int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe) {
+  const size_t nsb = digit_superblocks(K), n = rows * nsb * 16;
+  hipLaunchKernelGGL(k_digitize_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
+int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s) {
+  const size_t be = xabe_expert_quant_block_elements(quant), bb = xabe_expert_quant_block_bytes(quant);
+  a.nsb = (int)digit_superblocks((size_t)a.K);
+  a.row_bytes = (uint32_t)((size_t)a.K / be * bb);
+  a.out_nsb = (int)digit_superblocks((size_t)a.n_rows);
+  a.classes = a.nsb >= 8 ? 8 : a.nsb > 4 ? 8 : a.nsb > 2 ? 4 : a.nsb;
+  const int per_class = 8 / a.classes;
+  int nt = 1;
+  if (mode == kRowsShared) {
+    // tokens per pass over the weights: all of them up to eight, equal passes beyond
+    const size_t t = k->g.max_tokens, passes = (t + 7) / 8, each = (t + passes - 1) / passes;
+    nt = each == 1 ? 1 : each == 2 ? 2 : each <= 4 ? 4 : 8;
+    units = (t + nt - 1) / nt;
+  }
+  a.tile_rows = nm == 2 ? 16 : 32;
+  int mt = 1;
+  const int tiles16 = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
+  a.n_tiles = tiles16;
+  unsigned grid_x = (unsigned)((tiles16 + per_class - 1) / per_class);
+  if (mode == kRowsShared && per_class == 1 && tiles16 > k->num_cus) {
+    // many tiles: one workgroup per CU with an even share of them, so that a superblock's digits serve the whole share
+    mt = kRowsMaxTiles;
+    const unsigned rounds = (unsigned)((tiles16 + (size_t)k->num_cus * mt - 1) / ((size_t)k->num_cus * mt));
+    grid_x = rounds * (unsigned)k->num_cus;
+  } else if (mode == kRowsShared && nm == 1 && per_class == 1 && tiles16 * 2 > k->num_cus && a.n_rows > k->num_cus) {
+    // fewer tiles than CUs, but not by half: narrower tiles, one for every CU (5120 rows: 256 of 20, not 160 of 32)
+    a.tile_rows = std::max(1, (a.n_rows + k->num_cus - 1) / k->num_cus);
+    a.n_tiles = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
+    grid_x = (unsigned)a.n_tiles;
+  }
+  if (units > 65535) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "%zu work units exceed the 65535 grid.y limit of the fp32 regime", units);
+  const bool tail = a.K % kSbElems != 0;
+  const dim3 grid(grid_x, (unsigned)units);
+  return nm == 2 ? rows_mode<2>(mode, nt, mt, quant, tail, grid, s, &a) : rows_mode<1>(mode, nt, mt, quant, tail, grid, s, &a);
+}
+
+}  // namespace xabe

@@ -98,7 +98,7 @@ template <>
 struct SbRaw<kQ8_0> {
   uint32_t v[34];  // blocks 4 h .. 4 h + 3, 34 bytes each
   static constexpr int kBytes = 8 * kQ8Bytes;
-  static constexpr int kPieces = 17;  // 272 bytes, 16-byte aligned
+  static constexpr int kPieces = 17;  // 272 bytes, 16-byte aligned where rows are whole superblocks (18 otherwise)
 };
 
 // `p`: the row's superblock (any even address, global or LDS)
@@ -147,36 +147,39 @@ __device__ __forceinline__ void sb_group(const SbRaw<kQ8_0>& r, int s, int l, v4
 // The lane's eight group sums of one superblock for NT tokens: out[t] = the half's sum, from zero.
 //   a_of(s, l, tg): operand A of group (s, l) for tokens 4 tg .. 4 tg + 3 (zeros for tokens past NT)
 //   e_of(t, l):     the four group scales (s = 0..3) of token t in half `lane >> 5`
-// Group j + 1's matrix instructions are issued before group j's sums are taken up, so that their latency is covered.
-template <int QUANT, int NT, typename AOf, typename EOf>
-__device__ __forceinline__ void sb_dot(const SbRaw<QUANT>& r, AOf a_of, EOf e_of, float (&out)[NT]) {
-  constexpr int TG = (NT + 3) / 4;
+//   dead:           this half of the superblock lies past the end of the row (its codes are other data's bytes)
+// The work goes by units of (group, four tokens): a unit's matrix instruction is issued before the sums of the unit
+// before it are taken up, which covers its latency with two result registers in rotation.
+template <int QUANT, int NT, bool TAIL = false, typename AOf, typename EOf>
+__device__ __forceinline__ void sb_dot(const SbRaw<QUANT>& r, AOf a_of, EOf e_of, float (&out)[NT], bool dead = false) {
+  constexpr int TG = (NT + 3) / 4, kUnits = 8 * TG;
 #pragma unroll
   for (int t = 0; t < NT; ++t) out[t] = 0.0f;
-  v16i_t d[2][TG];
+  v16i_t d[2];
+  v4i_t c;
   float ws[2];
   float4 xe[NT];
-  auto issue = [&](int j) __attribute__((always_inline)) {
-    v4i_t c;
-    sb_group(r, j & 3, j >> 2, c, ws[j & 1]);
-#pragma unroll
-    for (int tg = 0; tg < TG; ++tg) {
-      const v16i_t zero = {0};
-      d[j & 1][tg] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_of(j & 3, j >> 2, tg), c, zero, 0, 0, 0);
+  auto issue = [&](int u) __attribute__((always_inline)) {
+    const int j = u / TG, tg = u % TG;
+    if (tg == 0) {
+      sb_group(r, j & 3, j >> 2, c, ws[j & 1]);
+      if (TAIL && dead) ws[j & 1] = 0.0f;
     }
+    const v16i_t zero = {0};
+    d[u & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_of(j & 3, j >> 2, tg), c, zero, 0, 0, 0);
   };
   issue(0);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int s = j & 3, l = j >> 2;
-    if (j < 7) issue(j + 1);
-    if (s == 0) {
+  for (int u = 0; u < kUnits; ++u) {
+    const int j = u / TG, tg = u % TG, s = j & 3, l = j >> 2;
+    if (u + 1 < kUnits) issue(u + 1);
+    if (s == 0 && tg == 0) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) xe[t] = e_of(t, l);
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const v16i_t& dd = d[j & 1][t >> 2];
+    for (int t = 4 * tg; t < 4 * tg + 4 && t < NT; ++t) {
+      const v16i_t& dd = d[u & 1];
       const int k = 4 * (t & 3);
       const int hi = (dd[k] << 8) + dd[k + 1], lo = (dd[k + 2] << 8) + dd[k + 3];
       const float f = __builtin_fmaf((float)lo, 0x1p-16f, (float)hi);
@@ -189,22 +192,25 @@ __device__ __forceinline__ void sb_dot(const SbRaw<QUANT>& r, AOf a_of, EOf e_of
 // Operand A and the group scales out of LDS, tokens of a superblock kSbBytes apart (digits, then scales); `zeros`: a
 // kilobyte of zero bytes that the lanes without a digit read.
 constexpr int kSbLdsBytes = kSbDigitBytes + kSbScaleBytes;  // 272 words: four tokens' rows start 16 banks apart
+template <int NT, int STRIDE>
 struct LdsDigits {
-  const uint8_t* a[2];
+  static constexpr int kQuads = (NT + 3) / 4;
+  const uint8_t* a[kQuads];
   const uint8_t* e;
-  template <int NT>
-  __device__ __forceinline__ void point(const uint8_t* sb_base, const uint8_t* zeros) {
+  // `digits`, `scales`: token 0's, the other tokens' STRIDE and E_STRIDE bytes apart
+  __device__ __forceinline__ void point(const uint8_t* digits, const uint8_t* scales, const uint8_t* zeros) {
     const int lane = (int)__lane_id(), h = lane >> 5, m = lane & 31;
     const bool mine = ((m >> 2) & 1) == h;
 #pragma unroll
-    for (int tg = 0; tg < (NT + 3) / 4; ++tg) {
+    for (int tg = 0; tg < kQuads; ++tg) {
       const int t = 4 * tg + (m >> 3);
-      a[tg] = mine && t < NT ? sb_base + t * kSbLdsBytes + h * 128 + (m & 3) * 16 : zeros;
+      a[tg] = mine && t < NT ? digits + t * STRIDE + h * 128 + (m & 3) * 16 : zeros;
     }
-    e = sb_base + kSbDigitBytes + h * 32;
+    e = scales + h * 32;
   }
-  __device__ __forceinline__ v4i_t digits(int s, int l, int tg) const { return *reinterpret_cast<const v4i_t*>(a[tg] + s * 256 + l * 64); }
-  __device__ __forceinline__ float4 scales(int t, int l) const { return *reinterpret_cast<const float4*>(e + t * kSbLdsBytes + l * 16); }
+  __device__ __forceinline__ v4i_t digit(int s, int l, int tg) const { return *reinterpret_cast<const v4i_t*>(a[tg] + s * 256 + l * 64); }
+  template <int E_STRIDE>
+  __device__ __forceinline__ float4 scale(int t, int l) const { return *reinterpret_cast<const float4*>(e + t * E_STRIDE + l * 16); }
 };
 
 // ---------------------------------------------------------------------------------
@@ -215,9 +221,9 @@ struct LdsDigits {
 // One slot is enough: it is free again as soon as its bytes are in registers, so the next request is in flight
 // while this superblock is multiplied.
 // ---------------------------------------------------------------------------------
-template <int QUANT>
+template <int QUANT, int PIECES = SbRaw<QUANT>::kPieces>
 struct SliceDma {
-  static constexpr int kP = SbRaw<QUANT>::kPieces;
+  static constexpr int kP = PIECES;
   static constexpr int kInstr = (16 * kP + 63) / 64;     // DMA instructions per run
   static constexpr int kRunBytes = kInstr * 1024;        // (a run's last instruction pads)
   static constexpr int kSlotBytes = 2 * kRunBytes;
@@ -251,6 +257,17 @@ struct SliceDma {
       asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(to) : "memory", "m0");
 #pragma clang diagnostic pop
     }
+  }
+  // A tensor that ends inside a 16-byte piece: its last bytes, which no whole piece holds, go to the slot two by two
+  // (the run's `live` rows end the tensor, and `sb` is the rows' last superblock).
+  __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t w_bytes, size_t run_off, int live, int sb, uint8_t* run_slot) const {
+    const int lane = (int)__lane_id();
+    const size_t tail = w_bytes & ~(size_t)15, start = run_off + (size_t)(live - 1) * row_bytes + (size_t)sb * SbRaw<QUANT>::kBytes;
+    uint8_t* p = run_slot + (live - 1) * (kP * 16) + (start & 15) + (tail - start);
+    if (2 * lane < (int)(w_bytes & 15)) *reinterpret_cast<uint16_t*>(p + 2 * lane) = *reinterpret_cast<const uint16_t*>(w + tail + 2 * lane);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   // the address of the lane's row inside the run's slot
   __device__ __forceinline__ const uint8_t* row_at(const uint8_t* run_slot, size_t run_off, int row, int sb) const {

@@ -125,9 +125,8 @@ int route_planes_and_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_
 // elements, at least 64 of them); returns false in *done when the shape is not served.
 int rms_norm_rows_with_f16(void* stream, const float* x, const float* weight, float* out, void* out_h, size_t rows,
                            size_t width, float eps, bool* done);
-// one-time, at handle creation: LDS limits of the kernels that ask for more than the static 64 KB (mfma.hip, api.hip)
+// one-time, at handle creation: LDS limits of the kernels that ask for more than the static 64 KB (mfma.hip)
 int mfma_configure();
-int long_rows_configure();
 bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int gate_q, int up_q, int down_q, bool routed);
 // token-tile heights of the routed down and gate/up launches of the pass as published, and the entries one of the two
 // lists in `tile_list` holds; false when these buffers carry no lists
@@ -171,6 +170,10 @@ struct xabe_moe_buffers {
   int32_t valid_published;  // what `valid_tokens` holds (0 after allocation)
   int32_t valid_host;       // source of the host-to-device copy that publishes a new count
   float* inter;         // [slot][intermediate] fp32 (decode regimes)
+  // digits and group scales (digits.h) of what the fp32 row contractions read: the pass's activation rows, the routed
+  // intermediate rows (one per slot), the shared ones (one per token)
+  uint8_t *x_d, *inter_d, *shared_inter_d;
+  float *x_e, *inter_e, *shared_inter_e;
   float* partial;       // [flat][hidden]
   float* shared_inter;  // [token][intermediate]
   // matrix-core regime staging

@@ -116,14 +116,12 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
         }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if ((a.w_bytes & 15) != 0 && sb == nsb - 1 && row0 + 32 >= a.vocab) {
-        // the tensor ends inside a 16-byte piece: its last bytes, which no whole piece holds, two by two
-        const int last_u = (a.vocab - 1 - row0) >> 4, last_r = (a.vocab - 1 - row0) & 15;
-        const size_t tail = a.w_bytes & ~(size_t)15, start = (size_t)(a.vocab - 1) * row_bytes + (size_t)sb * SbRaw<QUANT>::kBytes;
-        uint8_t* p = slot + last_u * Dma::kRunBytes + last_r * (Dma::kP * 16) + (start & 15);
-        if (2 * lane < (int)(a.w_bytes & 15))
-          *reinterpret_cast<uint16_t*>(p + (tail - start) + 2 * lane) = *reinterpret_cast<const uint16_t*>(a.w + tail + 2 * lane);
-        __builtin_amdgcn_wave_barrier();
+      if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          const int live = a.vocab - (row0 + 16 * v);
+          if (live >= 1 && live <= 16 && row_hi == a.vocab) dma[v].patch_tail(a.w, a.w_bytes, run_off(v), live, sb, slot + v * Dma::kRunBytes);
+        }
       }
       SbRaw<QUANT> raw;
       sb_read(dma[0].row_at(slot + u * Dma::kRunBytes, run_off(u), r, sb), h, raw);
@@ -134,10 +132,12 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
         take_tile(i + 1);
         request(0);
       }
-      LdsDigits x;
-      x.point<NT>(s_x + (size_t)(SEG ? sb % seg_sb : sb) * NT * kSbLdsBytes, s_zero);
+      LdsDigits<NT, kSbLdsBytes> x;
+      const uint8_t* sb_x = s_x + (size_t)(SEG ? sb % seg_sb : sb) * NT * kSbLdsBytes;
+      x.point(sb_x, sb_x + kSbDigitBytes, s_zero);
       float v[NT];
-      sb_dot<QUANT, NT>(raw, [&](int s, int l, int tg) { return x.digits(s, l, tg); }, [&](int t, int l) { return x.scales(t, l); }, v);
+      sb_dot<QUANT, NT>(raw, [&](int s, int l, int tg) { return x.digit(s, l, tg); },
+                        [&](int t, int l) { return x.template scale<kSbLdsBytes>(t, l); }, v);
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[t] += v[t];
     }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "device_common.h"
+#include "digit_rows.h"
 #include "route_device.h"
 
 namespace xabe {
@@ -23,8 +24,11 @@ __device__ __forceinline__ float block_sum_256(float v, float* scratch) {
 // rms_norm_rows (crates/xabe-cuda/src/kernels/layer_ops.rs:129-151): every row of the
 // buffer, y = x * (1/sqrtf(mean(x^2) + eps)) * w.  grid = rows, 256 threads.
 // ---------------------------------------------------------------------------------
+// DIGITS: the row also goes out as the digits and group scales the fp32 row contractions read (digits.h).
+template <bool DIGITS>
 __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__ x, const float* __restrict__ w,
-                                                        float* __restrict__ out, int width, float eps) {
+                                                        float* __restrict__ out, int width, float eps,
+                                                        uint8_t* __restrict__ xd, float* __restrict__ xe) {
   const float* xr = x + (size_t)blockIdx.x * width;
   float* o = out + (size_t)blockIdx.x * width;
   // width is a multiple of 4; up to eight float4 columns per thread (rows up to 8192 wide) are requested
@@ -52,6 +56,21 @@ __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__
   for (int j = threadIdx.x + 2048; j < n4; j += 256) {
     const float4 a = x4[j], b = w4[j];
     o4[j] = make_float4(a.x * inv * b.x, a.y * inv * b.y, a.z * inv * b.z, a.w * inv * b.w);
+  }
+  if constexpr (DIGITS) {  // (the same products from the row's cached pieces, sixteen consecutive elements per thread)
+    const int nsb = (width + kSbElems - 1) / kSbElems;
+    uint8_t* d = xd + (size_t)blockIdx.x * nsb * kSbDigitBytes;
+    float* e = xe + (size_t)blockIdx.x * nsb * 16;
+    for (int gi = threadIdx.x; gi < nsb * 16; gi += 256) {
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = min(4 * gi + i, n4 - 1);
+        const float4 a = x4[j], b = w4[j];
+        v[4 * i] = a.x * inv * b.x, v[4 * i + 1] = a.y * inv * b.y, v[4 * i + 2] = a.z * inv * b.z, v[4 * i + 3] = a.w * inv * b.w;
+      }
+      store_digits16(v, gi, 16 * gi < width, d, e);
+    }
   }
 }
 
