@@ -308,7 +308,7 @@ int xabe_moe_gate_and_combine_seam(const xabe_moe_kernels* k, void* stream, cons
                                    const float* next_norm_weight, float next_eps, float* next_normed, void* next_normed_h);
 int xabe_moe_block_disable_tensor_cores(xabe_moe_block* blk);            /* B:987-989 */
 int xabe_moe_block_set_exact_decode_regime(xabe_moe_block* blk, int on); /* B:1003-1005 */
-/* At max_tokens <= 32 and the model shapes (hidden 2048 / intermediate 512, and the 512 / 256 test shape) the
+/* At max_tokens < 64 and the model shapes (hidden 2048 / intermediate 512, and the 512 / 256 test shape) the
  * block's eight steps are regrouped into three launches (logits + shared gate/up; route + gate/up; down +
  * combine) that compute the same values bit for bit.  `on` = 0 keeps one launch per step as the reference
  * has them (B:1091-1329); the switch exists for tests and measurement. */
@@ -326,7 +326,7 @@ int xabe_moe_block_tensor_cores_enabled(const xabe_moe_block* blk);      /* B:10
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code that builds its launches
  * under hipGraph capture without handles, tight serving loops, harnesses that forbid hipMalloc): xabe_moe_block_forward
  * at decode widths with the block's working set (normalised rows, logits, selections, intermediates, the live-token
- * count) in a device array the library holds statically (1.4 MB per GPU, until the process ends) instead of in buffers
+ * count) in a device array the library holds statically (1.8 MB per GPU, until the process ends) instead of in buffers
  * that xabe_moe_block_new allocates.  No handle, no hipMalloc/hipFree, the same three launches and the same bits.
  * Serves max_tokens <= 32, hidden <= 2048, intermediate <= 512, <= 512 experts, top-k <= 8, in the shapes and
  * formats of the three-launch decode block; anything larger is XABE_ERR_UNSUPPORTED_GEOMETRY.  The live-token count

@@ -101,52 +101,16 @@ static Shape shape_for(size_t K) {
 }
 static int rows_per_step(Shape s) { return s == kRps8 ? 8 : s == kRps4 ? 4 : s == kRps2 ? 2 : 1; }
 
-enum Mode { kFlat, kBlock, kShared };
-
-template <int QUANT, int KS, int RPS, int NM>
-static void launch_mode(Mode mode, dim3 grid, hipStream_t s, const ExpertArgs& a) {
-  if (mode == kFlat) hipLaunchKernelGGL((k_expert_flat<QUANT, KS, RPS, NM>), grid, dim3(256), 0, s, a);
-  else if (mode == kBlock) hipLaunchKernelGGL((k_expert_block<QUANT, KS, RPS, NM>), grid, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((k_expert_shared<QUANT, KS, RPS, NM>), grid, dim3(256), 0, s, a);
-}
-
 template <int QUANT, int NM>
-static void launch_shape(Shape shape, Mode mode, dim3 grid, hipStream_t s, const ExpertArgs& a) {
+static void launch_shape(Shape shape, dim3 grid, hipStream_t s, const ExpertArgs& a) {
   switch (shape) {
-    case kRps8: launch_mode<QUANT, 1, 8, NM>(mode, grid, s, a); break;
-    case kRps4: launch_mode<QUANT, 1, 4, NM>(mode, grid, s, a); break;
-    case kRps2: launch_mode<QUANT, 1, 2, NM>(mode, grid, s, a); break;
-    case kKs1: launch_mode<QUANT, 1, 1, NM>(mode, grid, s, a); break;
-    case kKs2: launch_mode<QUANT, 2, 1, NM>(mode, grid, s, a); break;
-    default: launch_mode<QUANT, 0, 1, NM>(mode, grid, s, a); break;
+    case kRps8: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 8, NM>), grid, dim3(256), 0, s, a); break;
+    case kRps4: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 4, NM>), grid, dim3(256), 0, s, a); break;
+    case kRps2: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 2, NM>), grid, dim3(256), 0, s, a); break;
+    case kKs1: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 1, NM>), grid, dim3(256), 0, s, a); break;
+    case kKs2: hipLaunchKernelGGL((k_expert_shared<QUANT, 2, 1, NM>), grid, dim3(256), 0, s, a); break;
+    default: hipLaunchKernelGGL((k_expert_shared<QUANT, 0, 1, NM>), grid, dim3(256), 0, s, a); break;
   }
-}
-
-// Dispatch-table regime, rows of one step: the weights-resident kernel where its tile divides the rows.
-template <int QUANT, int NM>
-static bool launch_block_resident(Shape shape, const ExpertArgs& a, size_t units, hipStream_t s) {
-  if (shape == kKs2 || shape == kStream || a.K * rows_per_step(shape) != 2048) return false;
-  const int rps = rows_per_step(shape);
-  // steps per wavefront: as many as keep the raw bytes of a tile within ~36 registers per lane
-  const int want = NM == 2 ? 2 : 4;
-  const int depth = a.n_rows % (kWavesPerWg * want * rps) == 0 ? want : a.n_rows % (kWavesPerWg * 2 * rps) == 0 ? 2 : 0;
-  if (!depth) return false;
-  const unsigned tiles = (unsigned)(a.n_rows / (kWavesPerWg * depth * rps));
-  if (tiles > 65535u || units > 65535u) return false;
-  dim3 grid(tiles, (unsigned)units);
-#define XABE_RESIDENT(RPS)                                                                                         \
-  do {                                                                                                             \
-    if (depth == 4) hipLaunchKernelGGL((k_expert_block_resident<QUANT, RPS, NM, 4>), grid, dim3(256), 0, s, a);    \
-    else hipLaunchKernelGGL((k_expert_block_resident<QUANT, RPS, NM, 2>), grid, dim3(256), 0, s, a);               \
-  } while (0)
-  switch (shape) {
-    case kRps8: XABE_RESIDENT(8); break;
-    case kRps4: XABE_RESIDENT(4); break;
-    case kRps2: XABE_RESIDENT(2); break;
-    default: XABE_RESIDENT(1); break;
-  }
-#undef XABE_RESIDENT
-  return true;
 }
 
 int pick_tile_rows(const xabe_moe_kernels* k, size_t live_units, int n_rows, int rps) {
@@ -159,22 +123,11 @@ int pick_tile_rows(const xabe_moe_kernels* k, size_t live_units, int n_rows, int
   return (int)(pw * kWavesPerWg * rps);
 }
 
-// `units`: grid.y work units (pairs, dispatch blocks, token chunks); `live_units`: how many
-// of them a typical step actually uses, for sizing the row tile.
-static int launch_expert(const xabe_moe_kernels* k, Mode mode, int quant, int nm, ExpertArgs a, size_t units,
-                         size_t live_units, hipStream_t s) {
+// `units`: grid.y work units (chunks of two tokens)
+static int launch_expert(const xabe_moe_kernels* k, int quant, int nm, ExpertArgs a, size_t units, hipStream_t s) {
   const Shape shape = shape_for((size_t)a.K);
   const int rps = rows_per_step(shape);
-  if (mode == kBlock && !k->force_community) {
-    bool done = false;
-    if (quant == XABE_QUANT_Q6K) done = nm == 2 ? launch_block_resident<kQ6K, 2>(shape, a, units, s) : launch_block_resident<kQ6K, 1>(shape, a, units, s);
-    else if (quant == XABE_QUANT_Q8_0) done = nm == 2 ? launch_block_resident<kQ8_0, 2>(shape, a, units, s) : launch_block_resident<kQ8_0, 1>(shape, a, units, s);
-    if (done) {
-      XABE_HIP_TRY(hipGetLastError());
-      return XABE_OK;
-    }
-  }
-  a.tile_rows = pick_tile_rows(k, live_units, a.n_rows, rps);
+  a.tile_rows = pick_tile_rows(k, units, a.n_rows, rps);
   const unsigned tiles = (unsigned)((a.n_rows + a.tile_rows - 1) / a.tile_rows);
   if (tiles > 65535) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "row-tile count %u exceeds the grid.y limit", tiles);
   dim3 grid(tiles, (unsigned)units);  // x = row tile (fast), y = unit
@@ -182,13 +135,13 @@ static int launch_expert(const xabe_moe_kernels* k, Mode mode, int quant, int nm
     return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "%zu work units exceed the 65535 grid.y limit of the fp32 regime", units);
   }
   if (quant == XABE_QUANT_Q6K) {
-    if (nm == 2) launch_shape<kQ6K, 2>(shape, mode, grid, s, a);
-    else launch_shape<kQ6K, 1>(shape, mode, grid, s, a);
+    if (nm == 2) launch_shape<kQ6K, 2>(shape, grid, s, a);
+    else launch_shape<kQ6K, 1>(shape, grid, s, a);
   } else if (quant == XABE_QUANT_Q8_0) {
-    if (nm == 2) launch_shape<kQ8_0, 2>(shape, mode, grid, s, a);
-    else launch_shape<kQ8_0, 1>(shape, mode, grid, s, a);
-  } else if (quant < 0 && nm == 1 && mode == kShared) {  // plain fp32 rows
-    launch_shape<kF32, 1>(shape, mode, grid, s, a);
+    if (nm == 2) launch_shape<kQ8_0, 2>(shape, grid, s, a);
+    else launch_shape<kQ8_0, 1>(shape, grid, s, a);
+  } else if (quant < 0 && nm == 1) {  // plain fp32 rows
+    launch_shape<kF32, 1>(shape, grid, s, a);
   } else {
     return set_error(XABE_ERR_UNSUPPORTED_QUANT, "no kernel for quantization code %d", quant);
   }
@@ -342,6 +295,7 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
   // everything one-time happens here, none of it on the launch path (launches are captured into graphs)
   int st = mfma_configure();
   if (st == XABE_OK) st = digit_rows_configure();
+  if (st == XABE_OK) st = decode_block_configure();
   if (st != XABE_OK) {
     delete k;
     return st;
@@ -407,7 +361,6 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   b->n_topk = routed ? flat : 0;
   b->n_sorted = routed ? sorted : 0;
   b->n_expert_blocks = routed ? eb : 0;
-  b->n_inter = routed ? sorted * g.intermediate : 0;
   b->n_partial = routed ? flat * g.hidden : 0;
   b->n_shared_inter = g.max_tokens * g.intermediate;
   const bool wide = g.max_tokens >= kMfmaMinTokens;
@@ -427,7 +380,6 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->align_hist, b->n_align_chunks * g.num_experts);
   A(&b->num_tokens_post_pad, routed ? 1 : 0);
   A(&b->valid_tokens, 1);
-  A(&b->inter, b->n_inter);
   A(&b->partial, b->n_partial);
   A(&b->shared_inter, b->n_shared_inter);
   const size_t nsb_h = digit_superblocks(g.hidden), nsb_i = digit_superblocks(g.intermediate);
@@ -448,7 +400,7 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
                             : 0;
   A(&b->router_partial, b->n_router_partial);
   // decode widths: one arrival counter per token for the seam's tail in the third launch (decode_block.hip)
-  b->n_seam_arrivals = (routed && g.max_tokens <= 32) ? g.max_tokens * seam_counter_ints_per_token() : 0;
+  b->n_seam_arrivals = (routed && g.max_tokens < kMfmaMinTokens) ? g.max_tokens * seam_counter_ints_per_token() : 0;
   A(&b->seam_arrivals, b->n_seam_arrivals);
   b->bytes = total;
   b->valid_published = 0;
@@ -469,7 +421,7 @@ int xabe_moe_shared_only_buffers_new(const xabe_moe_kernels* k, void* stream, in
 void xabe_moe_buffers_free(xabe_moe_buffers* b) {
   if (!b) return;
   void* ptrs[] = {b->topk_ids, b->topk_weights, b->sorted_token_ids, b->expert_ids, b->bucket_live, b->expert_counts,
-                  b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->inter, b->partial, b->shared_inter, b->x_h, b->inter_h,
+                  b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->partial, b->shared_inter, b->x_h, b->inter_h,
                   b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals,
                   b->x_d, b->x_e, b->inter_d, b->inter_e, b->shared_inter_d, b->shared_inter_e};
   for (void* p : ptrs)
@@ -650,33 +602,52 @@ static int check_routed_stacks(const xabe_moe_kernels* k, xabe_quant_tensor gate
   return XABE_OK;
 }
 
-// stages: bit 0 = gate/up + SwiGLU, bit 1 = down
+static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
+  RowsArgs a;
+  memset(&a, 0, sizeof(a));
+  a.valid_tokens = b->valid_tokens;
+  a.topk_ids = b->topk_ids;
+  a.topk_weights = b->topk_weights;
+  a.sorted_token_ids = b->sorted_token_ids;
+  a.expert_ids = b->expert_ids;
+  a.top_k = (int)k->g.experts_per_token;
+  a.block_size = (int)k->g.block_size;
+  return a;
+}
+
+// stages: bit 0 = gate/up + SwiGLU (from the digits of x), bit 1 = down
 static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, int stages = 3) {
   const xabe_moe_geometry& g = k->g;
-  const bool flat = flat_regime(k);
-  const size_t units = flat ? xabe_moe_geometry_max_flat_pairs(&g) : b->n_expert_blocks;
-  const size_t live = std::min(units, std::min(g.num_experts, xabe_moe_geometry_max_flat_pairs(&g)));
+  const int mode = flat_regime(k) ? kRowsFlat : kRowsBlock;
+  const size_t units = mode == kRowsFlat ? xabe_moe_geometry_max_flat_pairs(&g) : b->n_expert_blocks;
   const size_t expert_elems = g.intermediate * g.hidden;
-  ExpertArgs a = base_args(k, b);
-  a.w0 = static_cast<const uint8_t*>(gate.bytes);
-  a.w1 = static_cast<const uint8_t*>(up.bytes);
-  a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
-  a.x = x;
-  a.out = b->inter;
-  a.K = (int)g.hidden;
-  a.n_rows = (int)g.intermediate;
-  if (stages & 1) XABE_TRY(launch_expert(k, flat ? kFlat : kBlock, gate.quant, 2, a, units, flat ? units : live, s));
+  RowsArgs a = rows_args(k, b);
+  if (stages & 1) {
+    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->x_d, b->x_e));
+    a.w0 = static_cast<const uint8_t*>(gate.bytes);
+    a.w1 = static_cast<const uint8_t*>(up.bytes);
+    a.w_bytes = gate.len;
+    a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
+    a.xd = b->x_d;
+    a.xe = b->x_e;
+    a.out_d = b->inter_d;
+    a.out_e = b->inter_e;
+    a.K = (int)g.hidden;
+    a.n_rows = (int)g.intermediate;
+    XABE_TRY(launch_digit_rows(k, mode, gate.quant, 2, a, units, s));
+  }
   if (!(stages & 2)) return XABE_OK;
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
+  a.w_bytes = down.len;
   a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(down.quant) * xabe_expert_quant_block_bytes(down.quant);
-  a.x = b->inter;
+  a.xd = b->inter_d;
+  a.xe = b->inter_e;
   a.out = b->partial;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  XABE_TRY(launch_expert(k, flat ? kFlat : kBlock, down.quant, 1, a, units, flat ? units : live, s));
-  return XABE_OK;
+  return launch_digit_rows(k, mode, down.quant, 1, a, units, s);
 }
 
 int xabe_moe_grouped_forward_partial(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, xabe_quant_tensor gate,
@@ -728,19 +699,6 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
   return XABE_OK;
 }
 
-static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
-  RowsArgs a;
-  memset(&a, 0, sizeof(a));
-  a.valid_tokens = b->valid_tokens;
-  a.topk_ids = b->topk_ids;
-  a.topk_weights = b->topk_weights;
-  a.sorted_token_ids = b->sorted_token_ids;
-  a.expert_ids = b->expert_ids;
-  a.top_k = (int)k->g.experts_per_token;
-  a.block_size = (int)k->g.block_size;
-  return a;
-}
-
 // gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->x_d
 static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                          xabe_quant_tensor up, xabe_quant_tensor down, float* out, const float* residual = nullptr,
@@ -787,14 +745,14 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   a.out = b->shared_inter;
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
-  XABE_TRY(launch_expert(k, kShared, gate.quant, 2, a, units, units, s));
+  XABE_TRY(launch_expert(k, gate.quant, 2, a, units, s));
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.x = b->shared_inter;
   a.out = out;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  XABE_TRY(launch_expert(k, kShared, down.quant, 1, a, units, units, s));
+  XABE_TRY(launch_expert(k, down.quant, 1, a, units, s));
   return XABE_OK;
 }
 
@@ -862,20 +820,8 @@ int xabe_moe_grouped_forward_partial_with_shared(const xabe_moe_kernels* k, void
   XABE_TRY(check_shared_stacks(k, shared_gate, shared_up, shared_down));
   XABE_TRY(check_len("hidden_states", g.max_tokens * g.hidden, hidden_states_len));
   XABE_TRY(check_len("out", g.max_tokens * g.hidden, out_len));
-  // The shared expert's units ride the routed grid: two launches instead of four.  Same bodies as the
-  // separate entry points, so the outputs are bit-identical to them.
-  {
-    const size_t expert_elems = g.intermediate * g.hidden;
-    hipStream_t s = as_stream(stream);
-    const size_t gate_eb = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
-    const size_t down_eb = expert_elems / xabe_expert_quant_block_elements(down.quant) * xabe_expert_quant_block_bytes(down.quant);
-    XABE_TRY(launch_flat_with_shared(k, s, b, 2, gate.quant, shared_gate.quant, gate.bytes, up.bytes, gate_eb, hidden_states,
-                                     b->inter, shared_gate.bytes, shared_up.bytes, hidden_states, b->shared_inter,
-                                     (int)g.hidden, (int)g.intermediate));
-    XABE_TRY(launch_flat_with_shared(k, s, b, 1, down.quant, shared_down.quant, down.bytes, nullptr, down_eb, b->inter,
-                                     b->partial, shared_down.bytes, nullptr, b->shared_inter, out, (int)g.intermediate,
-                                     (int)g.hidden));
-  }
+  XABE_TRY(routed_fp32(k, as_stream(stream), b, gate, up, down, hidden_states));
+  XABE_TRY(shared_fp32(k, as_stream(stream), b, shared_gate, shared_up, shared_down, hidden_states, out));
   *fused = 1;
   return XABE_OK;
 }
@@ -968,7 +914,7 @@ int xabe::router_logits_biased(const xabe_moe_kernels* k, void* stream, const xa
   a.K = (int)g.hidden;
   a.n_rows = (int)g.num_experts;
   const size_t units = (g.max_tokens + 1) / 2;
-  return launch_expert(k, kShared, fmt, 1, a, units, units, as_stream(stream));
+  return launch_expert(k, fmt, 1, a, units, as_stream(stream));
 }
 
 int xabe_moe_gate_and_combine(const xabe_moe_kernels* k, void* stream, const xabe_moe_buffers* b,

@@ -1,67 +1,64 @@
-// The decode-width MoE block (max_tokens <= 32) as three launches with no intermediate passes.
+// The MoE block below the matrix-core widths (max_tokens < 64) as three launches with no intermediate passes.
 //
 // At a few tokens the block moves ~20 MB per token and every dependent memory access costs 1-2 us, so what
-// decides the time is the number of dependent round trips and launch boundaries on the critical path, not
-// bytes.  The eight steps of the block (norm, router, bias, route, gate/up, down, shared expert, combine)
-// are regrouped so that each launch issues everything it needs in one or two rounds of loads:
+// decides the time is the number of dependent round trips and launch boundaries on the critical path; at a few
+// dozen it is vector instructions per weight and token, and bytes.  The eight steps of the block (norm, router, bias,
+// route, gate/up, down, shared expert, combine) are regrouped so that each launch issues everything it needs in one or
+// two rounds of loads:
 //
 //   A  k_decode_logits:  router logits (+ bias) and the shared expert's gate/up, both normalising the
-//                        residual rows on load; one workgroup per token writes the normalised row and
-//                        the sigmoid gate scalar.
-//   B  k_decode_up:      one (token, k) pair x row tile per workgroup.  One wavefront routes the token from
-//                        its logits (every workgroup of a token repeats this: a few microseconds of one
-//                        wavefront is cheaper than one more launch or a device-wide handshake), then the
-//                        four wavefronts stream the selected expert's gate/up rows, all loads in flight
-//                        at once.
-//   C  k_decode_down:    one (token, row tile) per workgroup: the eight routed down projections and the
-//                        shared one for those rows, summed in registers in k order, gated, combined with
+//                        residual rows on load; two workgroups per token write the normalised row with its digits
+//                        (digits.h) and the sigmoid gate scalar.
+//   B  k_decode_up:      one (token, k) pair x share of its row tiles per workgroup.  One wavefront routes the token
+//                        from its logits (every workgroup of a token repeats this: a few microseconds of one
+//                        wavefront is cheaper than one more launch or a device-wide handshake), then the wavefronts
+//                        stream the selected expert's gate/up rows through the digit contraction and write the
+//                        intermediate row as digits.
+//   C  k_decode_down:    one token x share of its row tiles per workgroup, a wavefront per selection: the routed down
+//                        projections (and, at few tokens, the shared one), summed in k order, gated, combined with
 //                        the residual.  No partial buffer, no reduction pass.
 //
-// Every value is produced by the same per-row device functions (load_raw, accum, group_sum, rms_fold,
-// route_one_token) and the same sequence of fp32 operations as the multi-launch path, so the outputs are
-// bit-identical to it and to the wider regimes: the batch-invariance contract is unchanged.
+// The routed contractions are pair_dot's (digits.h), whose values are k_digit_rows' bit for bit; routing, norm, router
+// and shared expert are the per-row device functions of the multi-launch path.  So the outputs are bit-identical to that
+// path: the batch-invariance contract.  One multiply-add and one conversion per weight on the vector ALU, which this
+// replaces, made B 95 and C 52 us at 32 tokens; the digit form takes 71 and 39 (us per block, same box: 13 tokens
+// 96 -> 79, 32: 162 -> 131; 45 tokens, then ten launches, 252 -> 173; three tokens 31.6 both; one token 21.2 -> 21.8,
+// whose routed contractions wait for one more hop through LDS).  What bounds B and C now at 32 tokens: ~330 vector
+// instructions per (token, row tile, pair of superblocks), about half of the launch, and one expert read once per
+// selection and XCD rather than once.
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "decode_kernels.h"
+#include "digit_rows.h"
 #include "host_common.h"
 #include "route_device.h"
 
 namespace xabe {
 
-constexpr size_t kDecodeBlockMaxTokens = 32;  // widest batch served by the three launches (at 32 tokens 198 against the dispatch-table regime's 203 us; it wins beyond)
+constexpr size_t kDecodeBlockMaxTokens = kMfmaMinTokens - 1;  // every width below the matrix-core regime
 // From this width on the routing is a launch of its own between the first two (one wavefront per token) and the second
 // launch reads the selections: inside the second launch every workgroup of a token repeats the token's routing, and
-// past a few tokens its grid runs in several rounds per CU, each paying for it again.  Same-box, us per block, routing
-// inside / routing launch: 4 tokens 38.6 / 40.5, 6: 49.8 / 51.2, 8: 61.5 / 61.1, 12: 83.3 / 79.4, 16: 101.7 / 94.9,
+// past a few tokens its grid runs in several rounds per CU, each paying for it again.  Measured before the routed
+// contractions took their present form, us per block, routing inside / routing launch: 4 tokens 38.6 / 40.5, 6: 49.8 / 51.2, 8: 61.5 / 61.1, 12: 83.3 / 79.4, 16: 101.7 / 94.9,
 // 32: 181.3 / 161.5.
 constexpr int kPreRouteMinTokens = 8;
 // From this width on the second and third launches deal their workgroups so that the ones that read the same row
 // tile (of whichever experts their pairs or tokens selected) run next to each other on one XCD: workgroup ids go
 // round-robin to the eight XCDs, each with its own L2, and at these widths several pairs select the same expert
 // (32 tokens: 256 pairs over ~163 experts), whose rows then come out of HBM once per XCD instead of once per pair.
-// Fetched per launch at 32 tokens (FETCH_SIZE): gate/up 415 -> 342 MB, down 204 -> 151 MB.  The launches take the
-// same time either way (they are bound by vector instructions at these widths, not by bytes): at 16 tokens and
-// below, where fewer pairs coincide, the plain order measured 0.1-0.5 us faster and is kept.
-// (Grouping the second launch by expert instead, one workgroup per (expert, row tile) running its pairs against
-// one copy of the rows in registers, reads every expert exactly once and was measured slower: 109 us against 95 at
-// 32 tokens with one pair at a time, 135 us two at a time (sharing the dequantisation takes ~230 registers); the
-// pairs of an expert run one after the other there, and a third of the workgroups find no pair at all.)
+// At 16 tokens and below, where fewer pairs coincide, the plain order measured 0.1-0.5 us faster and is kept.
 constexpr int kXcdGroupMinTokens = 24;
 // the seam's arrival counters: per token one counter and one per group of kSeamGroup workgroups, 128 bytes apart
 constexpr int kSeamGroup = 16, kSeamMaxGroups = 64, kSeamCountersPerToken = 1 + kSeamMaxGroups, kSeamCounterStride = 32;
+constexpr int kMaxShare = 4;      // consecutive tiles a workgroup of the second or third launch takes at most
 constexpr int kMaxTopK = 8;       // contributions held in registers by k_decode_down
-constexpr int kMaxInter = 512;    // intermediate width staged in LDS by k_decode_down
 // Steps per wavefront of the first launch: a wavefront reads 24 KB of activation rows and norm weights for the 2-4 KB
 // of weights of one step, so more steps against the same registers cut what the launch pulls out of L2, at the
 // price of fewer workgroups.  Measured per width (launch A, us, depth 1 / 2 / 4): one token 5.2 / 5.3 / 6.6, three
 // 7.7 / 6.5 / 8.4, eight 14.2 / 9.4 / 8.4, sixteen - / 15.7 / 11.7.
-// Row steps per workgroup of the third launch (two wavefronts each): two, i.e. eight rows of the 2048-wide block.
-// Four (half as many workgroups, each staging the token's nine activation rows for twice as many rows) measured
-// slower or equal at every width: one token 22.3 against 20.9 us per block, three 32.6 / 31.2, eight 63.8 / 61.8,
-// thirty-two 195.7 / 185.6.
-constexpr int kDownSteps = 2;
 static int logits_depth(int max_tokens) { return max_tokens <= 1 ? 1 : max_tokens <= 6 ? 2 : 4; }
 
 
@@ -78,7 +75,8 @@ struct DecodeArgs {
   float* logits;
   int* topk_ids;
   float* topk_weights;
-  float* inter;
+  uint8_t *x_d, *inter_d;  // digits of the normalised rows and of the routed intermediate rows (digits.h)
+  float *x_e, *inter_e;    // their group scales
   float* shared_inter;
   float* shexp;
   float* gate_out;
@@ -94,9 +92,12 @@ struct DecodeArgs {
   float next_eps;
   size_t expert_bytes;  // bytes of one expert's gate (= up) matrix
   size_t down_bytes;    // bytes of one expert's down matrix (its format may differ)
+  size_t up_len;        // bytes of a whole gate (= up) stack
   float eps;
   int H, I, E, top_k, max_tokens;
   int tiles_r, tiles_s, tiles_g, tiles_d;  // row tiles: router, shared gate/up (launch A), gate/up (B), down (C)
+  int shared_from;                         // first workgroup of the shared down projection in B (wider batches)
+  int share_g, share_d;                    // consecutive tiles of a workgroup (B, C): divide tiles_g and tiles_d
 };
 
 // Row tiles of the first launch: D steps (RPS rows of K = 2048 / RPS elements each) per wavefront of a matrix, or of
@@ -216,7 +217,7 @@ __device__ __forceinline__ void tile_normed(const uint8_t* __restrict__ w0, cons
 }
 
 // ------------------------------------------------------------------------------------------------
-// A: grid = max_tokens (norm + gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
+// A: grid = 2 max_tokens (norm and digits, gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
 // A chunk is two tokens sharing one pass over the weights.
 // ------------------------------------------------------------------------------------------------
 template <int SQ, int RF, int RPS, int kLogitsDepth, bool PRE = false>
@@ -226,8 +227,8 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
   const int chunks = (a.max_tokens + 1) / 2;
   const int n_r = chunks * a.tiles_r;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if ((int)blockIdx.x >= a.max_tokens) {
-    int item = blockIdx.x - a.max_tokens;
+  if ((int)blockIdx.x >= 2 * a.max_tokens) {
+    int item = blockIdx.x - 2 * a.max_tokens;
     const bool router = item < n_r;
     if (!router) item -= n_r;
     const int tiles = router ? a.tiles_r : a.tiles_s;
@@ -257,7 +258,9 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
   }
   // the normalised row (callers read it back) and g = sigmoid(shared_gate_inp . normed): the order of
   // operations of the stand-alone RMSNorm and gate kernels
-  const int t = blockIdx.x;
+  // (two workgroups per token: the row and its digits, and the scalar; in one they were the launch's last to end)
+  const bool writes_row = (int)blockIdx.x < a.max_tokens;
+  const int t = writes_row ? (int)blockIdx.x : (int)blockIdx.x - a.max_tokens;
   const int valid = *a.valid_tokens;
   const float* xr = (PRE ? a.normed : a.residual) + (size_t)t * a.H;
   // hidden <= 2048: eight columns per thread, every load issued before the first use
@@ -268,24 +271,27 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
     const bool in = j < a.H;
     xv[i] = in ? xr[j] : 0.0f;
     nv[i] = in && !PRE ? a.post_norm[j] : 0.0f;
-    gv[i] = in ? a.shared_gate_inp[j] : 0.0f;
+    gv[i] = in && !writes_row ? a.shared_gate_inp[j] : 0.0f;
   }
   float inv = 1.0f;
   if constexpr (!PRE) inv = row_inv_rms(xr, a.H, a.eps);
   if (t >= valid) return;
   float s = 0.0f;
+  const int nsb = a.H / kSbElems;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int j = threadIdx.x + 256 * i;
-    if (j < a.H) {
+    if (256 * i < a.H) {  // (the served widths are multiples of 256)
       float v = xv[i];  // (PRE: the row is there already, written by the previous block's tail)
       if constexpr (!PRE) {
         v = xv[i] * inv * nv[i];
-        a.normed[(size_t)t * a.H + j] = v;
+        if (writes_row) a.normed[(size_t)t * a.H + j] = v;
       }
-      s = __builtin_fmaf(gv[i], v, s);
+      if (writes_row) store_digit_group(v, j, nsb, a.x_d + (size_t)t * nsb * kSbDigitBytes, a.x_e + (size_t)t * nsb * 16, true);
+      else s = __builtin_fmaf(gv[i], v, s);
     }
   }
+  if (writes_row) return;
   s = group_sum<64>(s);
   if ((threadIdx.x & 63) == 0) s_red[wave] = s;
   __syncthreads();
@@ -311,22 +317,78 @@ __global__ void __launch_bounds__(64) k_decode_route(DecodeArgs a) {
   }
 }
 
+// Shared expert's down projection: unit = (chunk of two tokens, WAVES * 4 steps of RPS rows).
+template <int SQ, int RPS, int WAVES>
+__device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) {
+  using RawS = typename Fmt<SQ>::Raw;
+  constexpr int G = 64 / RPS;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)__lane_id();
+  const int units_per_chunk = a.H / (WAVES * 4 * RPS);
+  const int t0 = 2 * (unit / units_per_chunk), row0 = ((unit % units_per_chunk) * WAVES + wave) * 4 * RPS;
+  const int t1 = min(t0 + 1, a.max_tokens - 1);
+  const int valid = *a.valid_tokens;
+  const LaneGeom g = lane_geom<SQ>();
+  const int koff = lane_koff<SQ, RPS>(g, 0);
+  const size_t row_bytes = (size_t)(a.I / Fmt<SQ>::kBlockElems) * Fmt<SQ>::kBlockBytes;
+  float x[2][32], xs[2][4];
+  lane_x_load<SQ>(a.shared_inter + (size_t)t0 * a.I, koff, g, x[0]);
+  lane_x_load<SQ>(a.shared_inter + (size_t)t1 * a.I, koff, g, x[1]);
+  lane_x_offsets<SQ>(x[0], xs[0]);
+  lane_x_offsets<SQ>(x[1], xs[1]);
+#pragma unroll 1
+  for (int d0 = 0; d0 < 4; d0 += 2) {  // (two steps in flight: four do not fit the registers of two workgroups per CU)
+    RawS raw[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) load_raw<SQ, true>(a.sdown + (size_t)(row0 + (d0 + d) * RPS) * row_bytes, true, g, raw[d]);
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      float tot[2] = {0.0f, 0.0f};
+      accum<SQ, 2>(raw[d], g, x, xs, tot);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const float sh = 1.0f * group_sum<G>(tot[t]);
+        if ((lane % G) == 0 && t0 + t < valid) a.shexp[(size_t)(t0 + t) * a.H + row0 + (d0 + d) * RPS + lane / G] = sh;
+      }
+    }
+  }
+}
+
 // ROUTED: the token's selection was made by a routing launch between A and this one (wider batches: there a token's
 // routing would otherwise be repeated by every one of its workgroups, several rounds of them per CU); the pair's
 // expert then comes out of topk_ids through the scalar cache and nothing else of the routing runs here.
-template <int RQ, int RPS, int DEPTH, bool ROUTED = false>
-__global__ void __launch_bounds__(256) k_decode_up(DecodeArgs a) {
-  using F = Fmt<RQ>;
-  using Raw = typename F::Raw;
-  constexpr int G = 64 / RPS;
-  extern __shared__ float s_route[];  // num_experts floats for the routing wavefront
-  __shared__ int s_expert, s_final;  // the candidate expert of this pair; the one routing settles on
-  int p = blockIdx.x / a.tiles_g, tile = blockIdx.x % a.tiles_g;
-  if (ROUTED && a.max_tokens >= kXcdGroupMinTokens && (a.tiles_g & 7) == 0) {
-    // wide batches (see kXcdGroupMinTokens): all pairs of one row tile next to each other on one XCD
-    const int n_pairs = a.max_tokens * a.top_k, xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    tile = xcd + 8 * (j / n_pairs);
+// A tile is sixteen gate rows and the sixteen matching up rows; wavefront w takes pair w >> 1 of the rows' superblocks
+// (NP pairs: hidden / 512) of matrix w & 1.  A workgroup runs `share_g` consecutive tiles of its pair against one copy of
+// the activation digits in registers: a wavefront's slot is free once the tile's bytes are in registers, so the next
+// tile's rows are on their way while this one is multiplied.  The tiles' sums wait in LDS for one barrier at the end, so
+// that no wavefront of the loop waits for another (with a barrier and one wavefront's SwiGLU per tile a tile took 9 us).
+// ROUTED: the workgroups past the pairs' are the shared expert's down projection (its intermediate is launch A's), 8 NP
+// steps of RPSI rows each, two tokens per pass, on the lanes' fp32 sums of the separate kernels.  (At fewer tokens a
+// wavefront of the third launch does it: here, on a few CUs only, its uncoalesced loads were the launch's last to end,
+// 13.5 against 9.3 us for one token.)
+template <int RQ, int SQ, int NP, int RPSI, bool ROUTED>
+__global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
+  using Dma = typename PairDma<RQ>::Dma;
+  constexpr int kWaves = 2 * NP;
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_up[];  // a weight slot per wavefront, then the routing's num_experts floats
+  __shared__ int s_expert, s_final;      // the candidate expert of this pair; the one routing settles on
+  __shared__ float s_red[kMaxShare][2 * NP][64];  // [tile][superblock][half, matrix, row]
+  float* const s_route = reinterpret_cast<float*>(s_up + kWaves * PairDma<RQ>::kSlotBytes);
+  if constexpr (ROUTED) {
+    if ((int)blockIdx.x >= a.shared_from) {
+      shared_down_rows<SQ, RPSI, 2 * NP>(a, (int)blockIdx.x - a.shared_from);
+      return;
+    }
+  }
+  const int block = (int)blockIdx.x;
+  const int shares = a.tiles_g / a.share_g;
+  int p = block / shares, share = block % shares;
+  if (ROUTED && a.max_tokens >= kXcdGroupMinTokens) {
+    // wide batches (see kXcdGroupMinTokens): all pairs of one share next to each other on one XCD (the grid is padded
+    // to whole rounds of eight shares)
+    const int n_pairs = a.max_tokens * a.top_k, xcd = block & 7, j = block >> 3;
+    share = xcd + 8 * (j / n_pairs);
     p = j % n_pairs;
+    if (share >= shares) return;
   }
   const int t = p / a.top_k, k = p % a.top_k;
   [[maybe_unused]] int pre_e = 0;
@@ -334,22 +396,26 @@ __global__ void __launch_bounds__(256) k_decode_up(DecodeArgs a) {
   // everything read before the live-token count is known is sized for max_tokens rows
   const int valid = *a.valid_tokens;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const LaneGeom g = lane_geom<RQ>();
-  const int koff = lane_koff<RQ, RPS>(g, 0);
+  const int lane = (int)__lane_id(), quarter = lane >> 4;
+  const int mat = wave & 1, sb0 = 2 * (wave >> 1), sb = sb0 + (quarter >> 1);
   // one wavefront routes the token (a different one in neighbouring workgroups, which share a CU); its
-  // logits and every wavefront's copy of the normalised row are requested together
-  const bool routes = !ROUTED && wave == (int)((blockIdx.x >> 8) & 3);
+  // logits and every wavefront's activation digits are requested together
+  const bool routes = !ROUTED && wave == (int)((block >> 8) % kWaves);
   const bool few = a.E <= 256;
   float lg[kRouteMaxPerLane];
   if (routes) {
     if (few) route_load<4>(a.logits + (size_t)t * a.E, a.E, nullptr, nullptr, *reinterpret_cast<float(*)[4]>(lg));
     else route_load<kRouteMaxPerLane>(a.logits + (size_t)t * a.E, a.E, nullptr, nullptr, lg);
   }
-  float x[1][32], xs[1][4];
-  lane_x_load<RQ>(a.normed + (size_t)t * a.H, koff, g, x[0]);
+  const uint32_t row_bytes = (uint32_t)(2 * NP * SbRaw<RQ>::kBytes);
+  Dma dma;  // (its lane offsets are ready before the expert is known)
+  dma.init(row_bytes, 16);
+  const size_t x_sb = (size_t)t * (2 * NP) + sb;
+  PairDigits x;
+  x.load(a.x_d + x_sb * kSbDigitBytes, a.x_e + x_sb * 16);
   if (t >= valid) return;
   // Routing in two halves (route_device.h).  The first orders the experts by logit: its k-th candidate is
-  // the pair's expert unless probabilities tie, and it is known ~2 us before the softmax is, so the four
+  // the pair's expert unless probabilities tie, and it is known ~2 us before the softmax is, so the
   // wavefronts request the candidate's rows right away.  The routing wavefront then finishes the softmax
   // under its own loads' latency; in the rare pass where the probabilities reorder the candidates, the rows
   // are streamed again for the expert the reference's rule selects.
@@ -366,33 +432,18 @@ __global__ void __launch_bounds__(256) k_decode_up(DecodeArgs a) {
       route_keys<kRouteMaxPerLane>(lg, a.E, key);
       route_rounds<kRouteMaxPerLane>(key, 0, k + 1, cand_i);
     }
-    if (g.lane == k) s_expert = cand_i;
+    if (lane == k) s_expert = cand_i;
   }
-  lane_x_offsets<RQ>(x[0], xs[0]);
   if constexpr (!ROUTED) __syncthreads();
-  const size_t row_bytes = (size_t)(a.H / F::kBlockElems) * F::kBlockBytes;
-  const int wave_row0 = (tile * kWavesPerWg + wave) * DEPTH * RPS;
-  float* out = a.inter + (size_t)p * a.I;
-  // the pair's rows of expert e: all loads, (the routing wavefront: the rest of the routing,) accumulation
+  uint8_t* const slot = s_up + wave * PairDma<RQ>::kSlotBytes;
+  const uint32_t slot_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot);
+  // the pair's rows of expert e: the request, (the routing wavefront: the rest of the routing,) the contraction
   auto stream_rows = [&](int e, auto finish_c) __attribute__((always_inline)) {
-    constexpr bool kFinish = decltype(finish_c)::value;
-    const uint8_t* wg = a.gate + (size_t)e * a.expert_bytes;
-    const uint8_t* wu = a.up + (size_t)e * a.expert_bytes;
-    Raw r[DEPTH][2];
-    auto request = [&](int d0, int d1) __attribute__((always_inline)) {
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        if (d < d0 || d >= d1) continue;
-        const int row0 = wave_row0 + d * RPS;  // the tiles divide the rows exactly (checked by the host)
-        load_raw<RQ, true>(wg + (size_t)row0 * row_bytes, true, g, r[d][0]);
-        load_raw<RQ, true>(wu + (size_t)row0 * row_bytes, true, g, r[d][1]);
-      }
-    };
-    // The routing wavefront finishes the softmax before it requests its own rows: its neighbours' requests
-    // fill the CU's memory pipeline at this point, and a load issued now would hold the wavefront (and the
-    // routing) until they drain; raised priority keeps it ahead of their arithmetic.
-    if constexpr (kFinish) {
-      if (routes) {
+    const size_t e_off = (size_t)e * a.expert_bytes;
+    auto run_off = [&](int i) __attribute__((always_inline)) { return e_off + (size_t)(16 * (share * a.share_g + i)) * row_bytes; };
+    dma.request(mat ? a.up : a.gate, a.up_len, run_off(0), sb0, slot_lds);
+    if constexpr (decltype(finish_c)::value) {
+      if (routes) {  // (raised priority keeps it ahead of its neighbours' arithmetic)
         __builtin_amdgcn_s_setprio(3);
         int sel_i;
         float sel_w;
@@ -401,206 +452,184 @@ __global__ void __launch_bounds__(256) k_decode_up(DecodeArgs a) {
         else route_rounds<kRouteMaxPerLane>(key, k + 1, n_cand, cand_i);
         if (few) route_finish<4>(*reinterpret_cast<float(*)[4]>(lg), a.E, a.top_k, n_cand, cand_i, s_route, sel_i, sel_w, exact);
         else route_finish<kRouteMaxPerLane>(lg, a.E, a.top_k, n_cand, cand_i, s_route, sel_i, sel_w, exact);
-        if (g.lane == k) s_final = sel_i;
-        if (k == 0 && tile == 0 && g.lane < a.top_k) {
-          a.topk_ids[(size_t)t * a.top_k + g.lane] = sel_i;
-          a.topk_weights[(size_t)t * a.top_k + g.lane] = sel_w;
+        if (lane == k) s_final = sel_i;
+        if (k == 0 && share == 0 && lane < a.top_k) {
+          a.topk_ids[(size_t)t * a.top_k + lane] = sel_i;
+          a.topk_weights[(size_t)t * a.top_k + lane] = sel_w;
         }
         __builtin_amdgcn_s_setprio(0);
       }
     }
-    request(0, DEPTH);  // (the other wavefronts come straight here)
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      float tg[1] = {0.0f}, tu[1] = {0.0f};
-      accum<RQ, 1>(r[d][0], g, x, xs, tg);
-      accum<RQ, 1>(r[d][1], g, x, xs, tu);
-      const float sg = group_sum<G>(tg[0]), su = group_sum<G>(tu[0]);
-      const int row = wave_row0 + d * RPS + g.lane / G;
-      if ((g.lane % G) == 0 && row < a.I) out[row] = silu_f(sg) * su;
+#pragma unroll 1
+    for (int i = 0; i < a.share_g; ++i) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      SbRaw<RQ> raw;
+      sb_read(dma.row_at(slot, run_off(i), lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), sb0, slot_lds);
+      s_red[i][sb][(quarter & 1) * 32 + mat * 16 + (lane & 15)] = pair_dot<RQ>(raw, x);
     }
+    __syncthreads();  // (s_final is there, too)
   };
   if constexpr (ROUTED) {
-    stream_rows(min(max(pre_e, 0), a.E - 1), std::false_type{});
+    stream_rows(__builtin_amdgcn_readfirstlane(min(max(pre_e, 0), a.E - 1)), std::false_type{});
   } else {
-    const int e = s_expert;
+    const int e = __builtin_amdgcn_readfirstlane(s_expert);
     stream_rows(e, std::true_type{});
-    __syncthreads();  // s_final is there
-    const int e_final = s_final;
-    if (e_final != e) stream_rows(e_final, std::false_type{});  // (same rows of `inter`, written again)
+    const int e_final = __builtin_amdgcn_readfirstlane(s_final);
+    if (e_final != e) stream_rows(e_final, std::false_type{});  // (the sums, written again)
+  }
+  for (int i = wave; i < a.share_g; i += kWaves) {
+    // superblocks in order, then half 0 + half 1; lanes 0..15 hold the gate sums, 16..31 the up sums
+    const float (&red)[2 * NP][64] = s_red[i];
+    float h0 = red[0][lane & 31], h1 = red[0][32 + (lane & 31)];
+#pragma unroll
+    for (int c = 1; c < 2 * NP; ++c) {
+      h0 += red[c][lane & 31];
+      h1 += red[c][32 + (lane & 31)];
+    }
+    const float total = h0 + h1, up = __shfl_xor(total, 16);
+    const int nsb_i = a.I / kSbElems;
+    store_digit_group(silu_f(total) * up, 16 * (share * a.share_g + i) + (lane & 15), nsb_i,
+                      a.inter_d + (size_t)p * nsb_i * kSbDigitBytes, a.inter_e + (size_t)p * nsb_i * 16, lane < 16);
   }
 }
 
 // ------------------------------------------------------------------------------------------------
-// C: grid = max_tokens * tiles_d.  A workgroup is RS row steps (RPS rows each; K = intermediate = 2048 / RPS)
-// x two wavefronts per step: the first takes the first half of the token's selections and the shared expert,
-// the second the other half, so that a token's nine contractions per row step spread over twice as many
-// wavefronts and every SIMD of the chip gets the same number of them (max_tokens x hidden / RPS x 2
-// wavefronts: 12 per CU at three tokens).  The second wavefront hands its weighted row sums to the first
-// through LDS, which adds all of them in selection order: the same operations as one wavefront would do.
+// C: grid = max_tokens * shares of the row tiles.  A tile is sixteen output rows of 512 elements (or 32 of 256: pairs of
+// superblocks either way) of one token; a wavefront takes one selection for the `share_d` consecutive tiles of its
+// workgroup against one copy of the token's intermediate digits in registers, the next tile's rows on their way while
+// this one is multiplied.  The weighted row sums meet in LDS once, at the end, and are added in selection order.
 // ------------------------------------------------------------------------------------------------
-template <int RQ, int SQ, int RPS, int RS>
-__global__ void __launch_bounds__(128 * RS) k_decode_down(DecodeArgs a) {
-  using RawR = typename Fmt<RQ>::Raw;
-  using RawS = typename Fmt<SQ>::Raw;
-  constexpr int G = 64 / RPS;
-  constexpr int kThreads = 128 * RS;
-  constexpr int kHalf = kMaxTopK / 2;  // selections per wavefront
-  __shared__ __attribute__((aligned(16))) float s_x[(kMaxTopK + 1) * kMaxInter];
-  __shared__ float s_xs[(kMaxTopK + 1) * kMaxInter / 8];  // -32 * (sum of each run of eight), Q6_K's code offset
-  __shared__ float s_part[RS][kHalf][RPS];               // the second wavefront's weighted row sums
-  __shared__ int s_arrived;                              // the seam's tail: storing wavefronts of this workgroup that are done
-  if (threadIdx.x == 0) s_arrived = 0;                   // (two barriers before anyone counts)
-  int t = blockIdx.x / a.tiles_d, tile = blockIdx.x % a.tiles_d;
-  if (a.max_tokens >= kXcdGroupMinTokens && (a.tiles_d & 7) == 0) {
-    // wide batches (see kXcdGroupMinTokens): all tokens of one row tile next to each other on one XCD
+// SHARED (the widths whose second launch leaves it out): one more wavefront takes the shared expert's rows (four, with a
+// step of each tile apiece, were slower: 7.0 against 6.8 us for one token).
+template <int RQ, int SQ, int kPairRows, bool SHARED>  // kPairRows: rows a pair of superblocks covers
+__global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_decode_down(DecodeArgs a) {
+  using Dma = PairRunDma<RQ>;
+  constexpr int kRows = 16 * kPairRows;  // rows per tile
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_down[];  // a weight slot per selection
+  __shared__ float s_part[kMaxShare][kMaxTopK + SHARED][kRows];  // [tile][selection]: the weighted row sums
+  const int shares = a.tiles_d / a.share_d;
+  int t = blockIdx.x / shares, share = blockIdx.x % shares;
+  if (a.max_tokens >= kXcdGroupMinTokens) {
+    // wide batches (see kXcdGroupMinTokens): all tokens of one share next to each other on one XCD (the grid is padded
+    // to whole rounds of eight shares)
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    tile = xcd + 8 * (j / a.max_tokens);
+    share = xcd + 8 * (j / a.max_tokens);
     t = j % a.max_tokens;
+    if (share >= shares) return;
   }
   // every buffer read below is sized for max_tokens rows, so round one is issued before the live-token
   // count is known; rows past it hold an earlier pass's values or zeros, and nothing is stored for them
   const int valid = *a.valid_tokens;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int rs = wave >> 1, second = wave & 1;
-  const int lane = __lane_id();
-  const int row0 = (tile * RS + rs) * RPS;  // hidden is a multiple of RS * RPS
-  // this wavefront's selections: [k0, k1)
-  const int split = (a.top_k + 1) / 2;
-  const int k0 = second ? split : 0, k1 = second ? a.top_k : split;
-  // round one: selections (addressed uniformly, so they come through the scalar cache and arrive in the registers
-  // the row addresses are formed from), gate scalar, the nine activation rows, the shared expert's rows
-  int sel_e[kHalf];
-  float sel_w[kHalf];
-#pragma unroll
-  for (int j = 0; j < kHalf; ++j) {
-    const int kk = min(k0 + j, a.top_k - 1);
-    sel_e[j] = a.topk_ids[(size_t)t * a.top_k + kk];
-    sel_w[j] = a.topk_weights[(size_t)t * a.top_k + kk];
-  }
+  const int lane = (int)__lane_id(), quarter = lane >> 4;
+  const int tile0 = share * a.share_d;  // hidden is a multiple of kRows * share_d
   const float gate = a.gate_out[t];
-  // a thread stages whole runs of eight consecutive activations (two 16-byte pieces): the run's sum is then
-  // formed once per workgroup, in element order, instead of once per lane and selection
-  constexpr int kRunsMax = (kMaxTopK + 1) * kMaxInter / 8;
-  constexpr int kStage = (kRunsMax + kThreads - 1) / kThreads;
-  float4 stage[kStage][2];
-  const int runs_per_row = a.I / 8, n_runs = (a.top_k + 1) * runs_per_row;
-  {
-    const float4* src_r = reinterpret_cast<const float4*>(a.inter + (size_t)t * a.top_k * a.I);
-    const float4* src_s = reinterpret_cast<const float4*>(a.shared_inter + (size_t)t * a.I);
+  // what the thread's output row needs besides the sums, requested with round one
+  const int n_out = a.share_d * kRows, n0 = min((int)threadIdx.x, n_out - 1);
+  const size_t o0 = (size_t)t * a.H + (size_t)tile0 * kRows;  // (a share's rows are consecutive)
+  float sh = SHARED ? 0.0f : a.shexp[o0 + n0], res = a.residual[o0 + n0];
+  if (SHARED && wave >= a.top_k) {
+    constexpr int RPS = kRows / 4, G = 64 / RPS;
+    const LaneGeom gs = lane_geom<SQ>();
+    const int koff = lane_koff<SQ, RPS>(gs, 0);
+    const size_t rb_s = (size_t)(a.I / Fmt<SQ>::kBlockElems) * Fmt<SQ>::kBlockBytes;
+    float x[1][32], xs[1][4];
+    lane_x_load<SQ>(a.shared_inter + (size_t)t * a.I, koff, gs, x[0]);
+    typename Fmt<SQ>::Raw raw[4];
+    auto request = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kStage; ++j) {
-      const int i = threadIdx.x + kThreads * j;
-      stage[j][0] = stage[j][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (i < n_runs) {
-        const float4* p = i < a.top_k * runs_per_row ? src_r + 2 * i : src_s + 2 * (i - a.top_k * runs_per_row);
-        stage[j][0] = p[0];
-        stage[j][1] = p[1];
+      for (int d = 0; d < 4; ++d) load_raw<SQ, true>(a.sdown + (size_t)((tile0 + i) * kRows + d * RPS) * rb_s, true, gs, raw[d]);
+    };
+    request(0);
+    if (t >= valid) return;
+    lane_x_offsets<SQ>(x[0], xs[0]);
+#pragma unroll 1
+    for (int i = 0; i < a.share_d; ++i) {
+      float tot[4][1];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        tot[d][0] = 0.0f;
+        accum<SQ, 1>(raw[d], gs, x, xs, tot[d]);
+      }
+      if (i + 1 < a.share_d) request(i + 1);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const float v = 1.0f * group_sum<G>(tot[d][0]);
+        if ((lane % G) == 0) s_part[i][kMaxTopK][d * RPS + lane / G] = v;
+      }
+    }
+  } else {
+    const int p = t * a.top_k + wave;
+    const int e = __builtin_amdgcn_readfirstlane(min(max(a.topk_ids[p], 0), a.E - 1));
+    const float sel_w = a.topk_weights[p];
+    constexpr int nsb = kPairRows == 1 ? 2 : 1;
+    const size_t x_sb = (size_t)p * nsb + (kPairRows == 1 ? quarter >> 1 : 0);
+    const uint32_t pair_bytes = 2 * SbRaw<RQ>::kBytes;
+    uint8_t* const slot = s_down + wave * Dma::kSlotBytes;
+    const uint32_t slot_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot);
+    auto run = [&](int i) __attribute__((always_inline)) { return a.down + (size_t)e * a.down_bytes + (size_t)(tile0 + i) * 16 * pair_bytes; };
+    if (t >= valid) return;
+    Dma::request(run(0), slot_lds);
+    PairDigits x;
+    x.load(a.inter_d + x_sb * kSbDigitBytes, a.inter_e + x_sb * 16);
+#pragma unroll 1
+    for (int i = 0; i < a.share_d; ++i) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      SbRaw<RQ> raw;
+      sb_read(slot + (lane & 15) * Dma::kRowStride + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (i + 1 < a.share_d) Dma::request(run(i + 1), slot_lds);
+      float v = pair_dot<RQ>(raw, x);
+      // superblock 0 + superblock 1 of each half, then half 0 + half 1
+      if constexpr (kPairRows == 1) v += __shfl_xor(v, 32);
+      v += __shfl_xor(v, 16);
+      if constexpr (kPairRows == 1) {
+        if (lane < 16) s_part[i][wave][lane] = sel_w * v;
+      } else {
+        if ((quarter & 1) == 0) s_part[i][wave][2 * (lane & 15) + (quarter >> 1)] = sel_w * v;
       }
     }
   }
-  const LaneGeom gs = lane_geom<SQ>();
-  const LaneGeom gr = lane_geom<RQ>();
-  const size_t rb_s = (size_t)(a.I / Fmt<SQ>::kBlockElems) * Fmt<SQ>::kBlockBytes;
-  const size_t rb_r = (size_t)(a.I / Fmt<RQ>::kBlockElems) * Fmt<RQ>::kBlockBytes;
-  RawS raw_s;
-  if (!second) load_raw<SQ, true>(a.sdown + (size_t)row0 * rb_s, true, gs, raw_s);
-  if (t >= valid) return;
-  // round two: the selected experts' rows
-  RawR rr[kHalf];
-#pragma unroll
-  for (int j = 0; j < kHalf; ++j) {
-    const int e = min(max(sel_e[j], 0), a.E - 1);
-    // j past this wavefront's share reads a selected expert's rows again and never uses them: an unconditional
-    // load keeps all of round two in one basic block, so every load is issued before the first wait
-    load_raw<RQ, true>(a.down + (size_t)e * a.down_bytes + (size_t)row0 * rb_r, true, gr, rr[j]);
-  }
-  // the activation rows arrived before the weights (loads return in order); publish them and their run sums
-#pragma unroll
-  for (int j = 0; j < kStage; ++j) {
-    const int i = threadIdx.x + kThreads * j;
-    if (i < n_runs) {
-      reinterpret_cast<float4*>(s_x)[2 * i] = stage[j][0];
-      reinterpret_cast<float4*>(s_x)[2 * i + 1] = stage[j][1];
-      float sum = 0.0f;  // (the order of lane_x_offsets)
-      sum += stage[j][0].x; sum += stage[j][0].y; sum += stage[j][0].z; sum += stage[j][0].w;
-      sum += stage[j][1].x; sum += stage[j][1].y; sum += stage[j][1].z; sum += stage[j][1].w;
-      s_xs[i] = -32.0f * sum;
-    }
-  }
   __syncthreads();
-  // x[32] of one staged row for this lane, and (Q6_K) the four run sums that go with them
-  auto lane_x = [&](auto quant_c, int slot, const LaneGeom& g, float (&x)[1][32], float (&xs)[1][4]) __attribute__((always_inline)) {
-    constexpr int Q = decltype(quant_c)::value;
-    const int koff = lane_koff<Q, RPS>(g, 0);
-    lane_x_load<Q>(s_x + slot * a.I, koff, g, x[0]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      xs[0][j] = Q == kQ6K ? s_xs[slot * runs_per_row + (koff + g.half * 128 + j * 32 + g.l8 * 8) / 8] : 0.0f;
-  };
-  float part[kHalf];
-#pragma unroll
-  for (int j = 0; j < kHalf; ++j) {
-    part[j] = 0.0f;
-    if (k0 + j < k1) {
-      float x[1][32], xs[1][4], tot[1] = {0.0f};
-      lane_x(std::integral_constant<int, RQ>{}, k0 + j, gr, x, xs);
-      accum<RQ, 1>(rr[j], gr, x, xs, tot);
-      part[j] = sel_w[j] * group_sum<G>(tot[0]);
-    }
-  }
-  const bool writes = (lane % G) == 0;
-  if (second) {
-    if (writes) {
-#pragma unroll
-      for (int j = 0; j < kHalf; ++j) s_part[rs][j][lane / G] = part[j];
-    }
-  }
-  float sh = 0.0f;
-  if (!second) {
-    float x[1][32], xs[1][4], tot[1] = {0.0f};
-    lane_x(std::integral_constant<int, SQ>{}, a.top_k, gs, x, xs);
-    accum<SQ, 1>(raw_s, gs, x, xs, tot);
-    sh = 1.0f * group_sum<G>(tot[0]);
-  }
-  __syncthreads();
-  const int row = row0 + lane / G;
-  if (!second && writes && row < a.H) {
-    // the routed sum in selection order: this wavefront's share, then the other's
+  // rows kRows * i + r of the share: the routed sum in selection order, shared expert, gate, residual
+  for (int n = (int)threadIdx.x; n < n_out; n += (int)blockDim.x) {
+    const int i = n / kRows, row = n % kRows;
+    const size_t o = o0 + n;
+    if (n >= (int)blockDim.x) res = a.residual[o];
+    if constexpr (SHARED) sh = s_part[i][kMaxTopK + SHARED - 1][row], a.shexp[o] = sh;
+    else if (n >= (int)blockDim.x) sh = a.shexp[o];
     float r = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kHalf; ++j)
-      if (j < k1) r += part[j];
-#pragma unroll
-    for (int j = 0; j < kHalf; ++j)
-      if (split + j < a.top_k) r += s_part[rs][j][lane / G];
-    const size_t i = (size_t)t * a.H + row;
+    for (int j = 0; j < kMaxTopK; ++j)
+      if (j < a.top_k) r += s_part[i][j][row];
     const float v = r + sh * gate;
-    a.routed[i] = r;
-    a.shexp[i] = sh;
-    if (a.ffn_out) a.ffn_out[i] = v;
-    const float lo = v + a.residual[i];
+    a.routed[o] = r;
+    if (a.ffn_out) a.ffn_out[o] = v;
+    const float lo = v + res;
     // (with the seam on, another workgroup of this launch reads the row back: the store goes through to memory)
-    if (a.next_normed) __hip_atomic_store(a.l_out + i, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else a.l_out[i] = lo;
+    if (a.next_normed) __hip_atomic_store(a.l_out + o, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else a.l_out[o] = lo;
   }
   if (!a.next_normed) return;
+  if (a.share_d * kRows > 64) {  // (several wavefronts have stored: all of them acknowledged before one counts the workgroup in)
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  }
+  if (wave != 0) return;
   // The seam (docs/BENCHMARKS.md:1376 of the reference: the next layer's RMSNorm in the combine's tail).  A token's
-  // row is finished by tiles_d workgroups, and the wavefront that finishes it last applies the norm.  Arrivals are
-  // counted in three levels so that no counter sees more than a few dozen of them (atomics on one address are served
-  // one after the other, ~70 ns each: 256 arrivals on one counter cost 18 us per pass at 32 tokens): the storing
-  // wavefronts of a workgroup in LDS, 16 workgroups on a group counter, the groups on the token's counter, every
-  // counter on a 128-byte line of its own.  A wavefront counts itself once its own stores are acknowledged (they go
-  // through to memory: no fence, whose L2 write-back costs microseconds here), so whoever sees a count complete knows
-  // all stores below it have landed.  No workgroup barrier: the other wavefronts are done.
-  if (second) return;
+  // row is finished by several workgroups, and the wavefront that finishes it last applies the norm.  Arrivals are
+  // counted in two levels so that no counter sees more than a few dozen of them (atomics on one address are served
+  // one after the other, ~70 ns each: 256 arrivals on one counter cost 18 us per pass at 32 tokens): 16 workgroups on
+  // a group counter, the groups on the token's counter, every counter on a 128-byte line of its own.  A wavefront
+  // counts itself once its own stores are acknowledged (they go through to memory: no fence, whose L2 write-back costs
+  // microseconds here), so whoever sees a count complete knows all stores below it have landed.
   __builtin_amdgcn_s_waitcnt(0);
   int prev = 0;
-  if (lane == 0) prev = __hip_atomic_fetch_add(&s_arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  if (__builtin_amdgcn_readfirstlane(prev) != RS - 1) return;
   int* const token_ctr = a.arrivals + (size_t)t * kSeamCountersPerToken * kSeamCounterStride;
-  const int groups = (a.tiles_d + kSeamGroup - 1) / kSeamGroup, grp = tile / kSeamGroup;
-  const int in_group = min(kSeamGroup, a.tiles_d - grp * kSeamGroup);
+  const int groups = (shares + kSeamGroup - 1) / kSeamGroup, grp = share / kSeamGroup;
+  const int in_group = min(kSeamGroup, shares - grp * kSeamGroup);
   int* const group_ctr = token_ctr + (1 + grp) * kSeamCounterStride;
   if (lane == 0) prev = __hip_atomic_fetch_add(group_ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(prev) != in_group - 1) return;
@@ -610,9 +639,9 @@ __global__ void __launch_bounds__(128 * RS) k_decode_down(DecodeArgs a) {
   }
   if (__builtin_amdgcn_readfirstlane(prev) != groups - 1) return;
   if (lane == 0) __hip_atomic_store(token_ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // the row comes in coalesced (element 64 j + lane per load) and changes hands through LDS (s_x is free now), padded
-  // by four floats per 32 as the first launch pads its rows
-  float* s_l = s_x;  // (free since the last barrier; one wavefront per workgroup at most gets here: a workgroup serves one token)
+  // the row comes in coalesced (element 64 j + lane per load) and changes hands through LDS (the weight slots are free
+  // now), padded by four floats per 32 as the first launch pads its rows
+  float* s_l = reinterpret_cast<float*>(s_down);  // (kXnPad floats; one wavefront per workgroup gets here)
   const float* lrow = a.l_out + (size_t)t * a.H;
   float in[32];
 #pragma unroll
@@ -642,20 +671,37 @@ __global__ void __launch_bounds__(128 * RS) k_decode_down(DecodeArgs a) {
 }
 
 // ------------------------------------------------------------------ host side
+// Tiles per workgroup of the second and third launch: the largest power of two up to kMaxShare that divides the tiles and
+// leaves 192 workgroups.  Same box, us per block, tiles of (second, third) launch: one token (1, 1) 24.1, (2, 1) 24.3,
+// (1, 2) 25.6; three (1, 1) 37.4, (2, 2) 31.8, (4, 2) 31.4, (4, 4) 34.5; thirteen (1, 1) 91.1, (2, 2) 80.9, (4, 4) 79.9;
+// thirty-two (1, 1) 172, (2, 2) 146, (4, 4) 132.
+static int decode_share(size_t units, int tiles) {
+  int share = 1;
+  while (share < kMaxShare && tiles % (2 * share) == 0 && units * tiles >= (size_t)384 * share) share *= 2;
+  return share;
+}
+
 struct Launch {
   const DecodeArgs& a;
   hipStream_t s;
   unsigned grid_a, grid_b, grid_c;
   bool pre_routed;  // a routing launch between A and B instead of routing inside B
   bool pre_normed;  // `normed` holds this pass's rows already (the previous block's tail): A neither normalises nor writes them
-  size_t route_lds;
   unsigned launches;  // bit i: issue launch i (A, B, C); all three outside measurements
 };
 
 // Each launch is chosen by the formats it reads: A by the shared gate/up and router formats, B by the routed
 // gate/up format, C by the routed and shared down formats (the shipped layers mix them: gate/up Q6_K with
 // down Q8_0).
-template <int RPSH, int DEPTH, int RPSI>
+template <int NP>
+static size_t up_lds(int gq, int num_experts) {
+  return 2 * NP * (size_t)(gq == XABE_QUANT_Q6K ? PairDma<kQ6K>::kSlotBytes : PairDma<kQ8_0>::kSlotBytes) + num_experts * sizeof(float);
+}
+static size_t down_lds(int dq, int top_k) {  // (the seam's tail stages a row in it)
+  return std::max((size_t)top_k * (dq == XABE_QUANT_Q6K ? PairRunDma<kQ6K>::kSlotBytes : PairRunDma<kQ8_0>::kSlotBytes), (size_t)kXnPad * sizeof(float));
+}
+
+template <int RPSH, int NP, int RPSI>
 static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int router_quant) {
   const bool g6 = gq == XABE_QUANT_Q6K, d6 = dq == XABE_QUANT_Q6K, sg6 = sgq == XABE_QUANT_Q6K, sd6 = sdq == XABE_QUANT_Q6K;
   const bool rf32 = router_quant < 0;
@@ -681,25 +727,63 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
 #undef XABE_A1
   }
   if (l.launches & 2u) {
+    const size_t lds = up_lds<NP>(gq, l.a.E);
+    const dim3 grid(l.grid_b), block(128 * NP);
     if (l.pre_routed) {
-      hipLaunchKernelGGL(k_decode_route, dim3((unsigned)l.a.max_tokens), dim3(64), l.route_lds, l.s, l.a);
-      if (g6) hipLaunchKernelGGL((k_decode_up<kQ6K, RPSH, DEPTH, true>), dim3(l.grid_b), dim3(256), 0, l.s, l.a);
-      else hipLaunchKernelGGL((k_decode_up<kQ8_0, RPSH, DEPTH, true>), dim3(l.grid_b), dim3(256), 0, l.s, l.a);
-    } else if (g6) hipLaunchKernelGGL((k_decode_up<kQ6K, RPSH, DEPTH>), dim3(l.grid_b), dim3(256), l.route_lds, l.s, l.a);
-    else hipLaunchKernelGGL((k_decode_up<kQ8_0, RPSH, DEPTH>), dim3(l.grid_b), dim3(256), l.route_lds, l.s, l.a);
+      hipLaunchKernelGGL(k_decode_route, dim3((unsigned)l.a.max_tokens), dim3(64), l.a.E * sizeof(float), l.s, l.a);
+    }
+#define XABE_B(RQ, SQ)                                                                                            \
+  do {                                                                                                            \
+    if (l.pre_routed) hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, true>), grid, block, lds, l.s, l.a);       \
+    else hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, false>), grid, block, lds, l.s, l.a);                   \
+  } while (0)
+    if (g6 && sd6) XABE_B(kQ6K, kQ6K);
+    else if (g6) XABE_B(kQ6K, kQ8_0);
+    else if (sd6) XABE_B(kQ8_0, kQ6K);
+    else XABE_B(kQ8_0, kQ8_0);
+#undef XABE_B
   }
   if (l.launches & 4u) {
-#define XABE_C(RQ, SQ)                                                                                            \
-  do {                                                                                                          \
-    hipLaunchKernelGGL((k_decode_down<RQ, SQ, RPSI, kDownSteps>), dim3(l.grid_c), dim3(128 * kDownSteps), 0, l.s, l.a); \
-  } while (0)
-    if (d6 && sd6) XABE_C(kQ6K, kQ6K);
-    else if (d6) XABE_C(kQ6K, kQ8_0);
-    else if (sd6) XABE_C(kQ8_0, kQ6K);
-    else XABE_C(kQ8_0, kQ8_0);
-#undef XABE_C
+    const size_t lds = down_lds(dq, l.a.top_k);
+    const dim3 grid(l.grid_c), block(64 * (l.a.top_k + (l.pre_routed ? 0 : 1)));
+    if (l.pre_routed) {
+      if (d6) hipLaunchKernelGGL((k_decode_down<kQ6K, kQ8_0, RPSI / 4, false>), grid, block, lds, l.s, l.a);
+      else hipLaunchKernelGGL((k_decode_down<kQ8_0, kQ8_0, RPSI / 4, false>), grid, block, lds, l.s, l.a);
+    } else if (d6 && sd6) hipLaunchKernelGGL((k_decode_down<kQ6K, kQ6K, RPSI / 4, true>), grid, block, lds, l.s, l.a);
+    else if (d6) hipLaunchKernelGGL((k_decode_down<kQ6K, kQ8_0, RPSI / 4, true>), grid, block, lds, l.s, l.a);
+    else if (sd6) hipLaunchKernelGGL((k_decode_down<kQ8_0, kQ6K, RPSI / 4, true>), grid, block, lds, l.s, l.a);
+    else hipLaunchKernelGGL((k_decode_down<kQ8_0, kQ8_0, RPSI / 4, true>), grid, block, lds, l.s, l.a);
   }
   return true;
+}
+
+// LDS limits of the launches that ask for more than the static 64 KB; at handle creation (or a first call without one)
+int decode_block_configure() {
+  static bool done = false;  // (one device per process)
+  if (done) return XABE_OK;
+#define XABE_LDS(kernel, bytes) \
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes)))
+#define XABE_UP(Q, code, SQ, NP, RPSI)                                                       \
+  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, false>), up_lds<NP>(code, (int)kRouteMaxExperts)); \
+  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, true>), up_lds<NP>(code, (int)kRouteMaxExperts))
+#define XABE_DOWN(Q, code)                                          \
+  XABE_LDS((k_decode_down<Q, kQ8_0, 1, false>), down_lds(code, kMaxTopK));  \
+  XABE_LDS((k_decode_down<Q, kQ8_0, 2, false>), down_lds(code, kMaxTopK));  \
+  XABE_LDS((k_decode_down<Q, kQ6K, 1, true>), down_lds(code, kMaxTopK));    \
+  XABE_LDS((k_decode_down<Q, kQ6K, 2, true>), down_lds(code, kMaxTopK));    \
+  XABE_LDS((k_decode_down<Q, kQ8_0, 1, true>), down_lds(code, kMaxTopK));   \
+  XABE_LDS((k_decode_down<Q, kQ8_0, 2, true>), down_lds(code, kMaxTopK));   \
+  XABE_UP(Q, code, kQ6K, 4, 4);                                     \
+  XABE_UP(Q, code, kQ8_0, 4, 4);                                    \
+  XABE_UP(Q, code, kQ6K, 1, 8);                                     \
+  XABE_UP(Q, code, kQ8_0, 1, 8)
+  XABE_DOWN(kQ6K, XABE_QUANT_Q6K);
+  XABE_DOWN(kQ8_0, XABE_QUANT_Q8_0);
+#undef XABE_DOWN
+#undef XABE_UP
+#undef XABE_LDS
+  done = true;
+  return XABE_OK;
 }
 
 static bool launch_shape(const Launch& l, int gq, int dq, int sgq, int sdq, int router_quant) {
@@ -754,7 +838,11 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   a.logits = logits;
   a.topk_ids = b->topk_ids;
   a.topk_weights = b->topk_weights;
-  a.inter = b->inter;
+  a.x_d = b->x_d;
+  a.x_e = b->x_e;
+  a.inter_d = b->inter_d;
+  a.inter_e = b->inter_e;
+  a.up_len = w->gate_exps.len;
   a.shared_inter = b->shared_inter;
   a.shexp = shexp;
   a.gate_out = gate_out;
@@ -774,19 +862,21 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   const int da = logits_depth(a.max_tokens);
   a.tiles_r = (a.E + kWavesPerWg * rps_h * da - 1) / (kWavesPerWg * rps_h * da);
   a.tiles_s = (a.I + kWavesPerWg * rps_h * da - 1) / (kWavesPerWg * rps_h * da);
-  const int depth = a.H == 2048 ? 4 : 1;  // steps per wavefront of the gate/up launch (launch_shape)
-  a.tiles_g = (a.I + kWavesPerWg * depth * rps_h - 1) / (kWavesPerWg * depth * rps_h);
-  const int down_steps = kDownSteps;
-  a.tiles_d = (a.H + down_steps * rps_i - 1) / (down_steps * rps_i);
-  if (a.E % rps_h != 0 || a.I % (kWavesPerWg * depth * rps_h) != 0 || a.H % (down_steps * rps_i) != 0)
-    return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "decode block: %d experts / %d intermediate rows do not fill whole steps of %d rows",
-                     a.E, a.I, rps_h);
+  a.tiles_g = a.I / 16;
+  a.tiles_d = a.H / (4 * rps_i);
+  if (a.E % rps_h != 0)
+    return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "decode block: %d experts do not fill whole steps of %d rows", a.E, rps_h);
+  a.share_g = decode_share((size_t)a.max_tokens * a.top_k, a.tiles_g);
+  a.share_d = decode_share((size_t)a.max_tokens, a.tiles_d);
   const int chunks = (a.max_tokens + 1) / 2;
   const bool pre_routed = a.max_tokens >= kPreRouteMinTokens;
-  Launch l{a, s, 0, 0, 0, pre_routed, seam && seam->input_normed, g.num_experts * sizeof(float), launches};
-  l.grid_a = (unsigned)(chunks * (a.tiles_r + a.tiles_s) + a.max_tokens);
-  l.grid_b = (unsigned)(a.max_tokens * a.top_k * a.tiles_g);
-  l.grid_c = (unsigned)(a.max_tokens * a.tiles_d);
+  Launch l{a, s, 0, 0, 0, pre_routed, seam && seam->input_normed, launches};
+  l.grid_a = (unsigned)(chunks * (a.tiles_r + a.tiles_s) + 2 * a.max_tokens);
+  // wide batches pad the shares of a pair (token) to whole rounds of eight, one per XCD
+  auto grid_of = [&](size_t units, int shares) { return (unsigned)(units * (a.max_tokens >= kXcdGroupMinTokens ? (shares + 7) / 8 * 8 : shares)); };
+  a.shared_from = (int)grid_of((size_t)a.max_tokens * a.top_k, a.tiles_g / a.share_g);
+  l.grid_b = (unsigned)(a.shared_from + (pre_routed ? chunks * (a.H / (4 * rps_i * (a.H / 512) * 2)) : 0));
+  l.grid_c = grid_of((size_t)a.max_tokens, a.tiles_d / a.share_d);
   const bool ok = launch_shape(l, w->gate_exps.quant, w->down_exps.quant, w->shared_gate.quant, w->shared_down.quant, w->router_quant);
   if (!ok) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "decode block: no kernels for this shape or format");
   XABE_HIP_TRY(hipGetLastError());

@@ -1,7 +1,7 @@
-// Decode-regime expert kernels: fp32 accumulation, weights streamed once from HBM
-// in their file layout (210-byte Q6_K superblocks / 34-byte Q8_0 blocks), dequantised
-// in registers.  Replaces the reference's gemv / flat / tiled fp32 families
-// (crates/xabe-cuda/src/kernels/moe.rs:2403-3124, :3425-3725, :4082-4227).
+// The lanes' fp32 row contractions: router logits and the shared expert below the matrix-core widths; weights streamed
+// once from HBM in their file layout (210-byte Q6_K superblocks / 34-byte Q8_0 blocks), dequantised in registers.  (The
+// routed experts and longer rows go through the digit contraction, digits.h.)  Replaces the reference's shared-expert
+// gemv / tiled fp32 families (crates/xabe-cuda/src/kernels/moe.rs:3425-3725, :4082-4227).
 //
 // One wavefront "step" covers 2048 contraction elements of a row: 8 Q6_K superblocks
 // (1680 B) or 64 Q8_0 blocks (2176 B), 32 elements per lane.  Rows shorter than 2048
@@ -188,71 +188,6 @@ __device__ __forceinline__ void accum(const typename Fmt<QUANT>::Raw& r, const L
 }
 
 // ---------------------------------------------------------------------------------
-// Coalesced form of load_raw.  A lane picking its own fields out of global memory touches every cache
-// line of the step with every one of its seven to ten load instructions, and the vector L1 serves a
-// line that is still pending by stalling; measured on this part, that halves the streaming rate
-// (2.7 against 5.5 TB/s).  Instead the wavefront requests the step as consecutive 16-byte pieces (each
-// line touched once), parks them in a wavefront-private LDS slot and picks the fields up from there with
-// the same funnel loads, so the Raw it produces is bit for bit the one load_raw produces.
-//   stage_load:  issue the global loads of one step (`nbytes` live bytes starting at `chunk`, any 2-byte
-//                alignment).  The 16-byte window around them must lie inside the tensor: the host checks
-//                that the tensor starts and ends on 16-byte boundaries.
-//   stage_pick:  pieces -> LDS slot -> Raw.  Slots are private to a wavefront, whose LDS operations
-//                complete in program order; the fences only keep the compiler from reordering them.
-// ---------------------------------------------------------------------------------
-template <int QUANT>
-struct StageFmt;
-template <>
-struct StageFmt<kQ6K> {
-  static constexpr int kPieces = 2;        // 1680 (+14) bytes: up to 106 pieces
-  static constexpr int kSlotBytes = 1696;
-};
-template <>
-struct StageFmt<kQ8_0> {
-  static constexpr int kPieces = 3;        // 2176 (+14) bytes: up to 137 pieces
-  static constexpr int kSlotBytes = 2192;
-};
-
-typedef uint32_t stage_piece __attribute__((ext_vector_type(4)));  // a first-class vector: stays in registers
-
-template <int QUANT>
-struct Staged {
-  stage_piece p[StageFmt<QUANT>::kPieces];
-  uint32_t mis;  // bytes from the 16-byte boundary below `chunk` to `chunk`
-  int last;      // index of the last live piece
-};
-
-template <int QUANT>
-__device__ __forceinline__ void stage_load(const uint8_t* chunk, uint32_t nbytes, Staged<QUANT>& s) {
-  s.mis = (uint32_t)(reinterpret_cast<uintptr_t>(chunk) & 15u);
-  s.last = (int)((s.mis + nbytes + 15u) >> 4) - 1;
-  const stage_piece* base = reinterpret_cast<const stage_piece*>(chunk - s.mis);
-  const int lane = (int)__lane_id();
-#pragma unroll
-  for (int i = 0; i < StageFmt<QUANT>::kPieces; ++i) s.p[i] = base[min(lane + 64 * i, s.last)];
-}
-
-template <int QUANT>
-__device__ __forceinline__ void stage_pick(const Staged<QUANT>& s, uint8_t* slot, bool active, const LaneGeom& g,
-                                           typename Fmt<QUANT>::Raw& r) {
-  const int lane = (int)__lane_id();
-#pragma unroll
-  for (int i = 0; i < StageFmt<QUANT>::kPieces; ++i)  // lanes past the last piece repeat its store
-    reinterpret_cast<stage_piece*>(slot)[min(lane + 64 * i, s.last)] = s.p[i];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (active) {
-    if constexpr (QUANT == kQ6K) q6_load(slot, g.lane_off + s.mis, g.half, g.l8, r);
-    else q8_load(slot, g.lane_off + s.mis, r);
-  } else {
-    raw_zero<QUANT>(r);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// ---------------------------------------------------------------------------------
 // matvec_rows: the body every decode kernel shares.
 //   NM = 2: out[t][row] = silu(gate_row . x_t) * (up_row . x_t)      (gate/up + SwiGLU)
 //   NM = 1: out[t][row] = scale[t] * (w_row . x_t)                    (down / plain GEMV)
@@ -399,154 +334,6 @@ struct ExpertArgs {
   int tile_rows;             // rows per workgroup
 };
 
-// Flat regime (max_tokens <= 4, or the exact decode regime): one work unit per live
-// (token, k) pair read straight from topk_ids; no dispatch table
-// (crates/xabe-cuda/src/kernels/moe.rs:2525-2634, :3066-3124).
-template <int QUANT, int KS, int RPS, int NM>
-__device__ __forceinline__ void flat_body(const ExpertArgs& a, int p, int tile) {
-  const int valid = *a.valid_tokens;
-  if (p >= valid * a.top_k) return;
-  const int e = a.topk_ids[p];
-  const uint8_t* w0 = a.w0 + (size_t)e * a.expert_bytes;
-  const uint8_t* w1 = NM == 2 ? a.w1 + (size_t)e * a.expert_bytes : nullptr;
-  // gate/up reads the token's activation row; down reads the pair's own inter row
-  const float* const xr[1] = {a.x + (size_t)(NM == 2 ? p / a.top_k : p) * a.K};
-  float* const o[1] = {a.out + (size_t)p * a.n_rows};
-  const float sc[1] = {NM == 2 ? 1.0f : a.topk_weights[p]};
-  matvec_rows<QUANT, KS, RPS, 1, NM>(w0, w1, a.K, a.n_rows, tile * a.tile_rows, a.tile_rows, xr, o, sc);
-}
-
-template <int QUANT, int KS, int RPS, int NM>
-__global__ void __launch_bounds__(256) k_expert_flat(ExpertArgs a) {
-  flat_body<QUANT, KS, RPS, NM>(a, blockIdx.y, blockIdx.x);
-}
-
-// Dispatch-table regime: one work unit per dispatch block; the block's live slots all
-// belong to one expert, whose rows are streamed once per chunk of two tokens
-// (chunks after the first hit in L2).  gate/up writes inter[slot]; down reads
-// inter[slot] and writes partial[flat].
-template <int QUANT, int KS, int RPS, int NM>
-__global__ void __launch_bounds__(256) k_expert_block(ExpertArgs a) {
-  const int b = blockIdx.y;
-  const int e = a.expert_ids[b];
-  if (e < 0) return;
-  const int valid = *a.valid_tokens;
-  const int sentinel = valid * a.top_k;
-  const uint8_t* w0 = a.w0 + (size_t)e * a.expert_bytes;
-  const uint8_t* w1 = NM == 2 ? a.w1 + (size_t)e * a.expert_bytes : nullptr;
-  const int* slots = a.sorted_token_ids + (size_t)b * a.block_size;
-  for (int i = 0; i < a.block_size; i += 2) {
-    const int f0 = slots[i];
-    if (f0 >= sentinel) break;
-    const int f1 = (i + 1 < a.block_size) ? slots[i + 1] : sentinel;
-    const size_t s0 = (size_t)b * a.block_size + i;
-    if (f1 < sentinel) {
-      const float* const xr[2] = {a.x + (NM == 2 ? (size_t)(f0 / a.top_k) : s0) * a.K,
-                                  a.x + (NM == 2 ? (size_t)(f1 / a.top_k) : s0 + 1) * a.K};
-      float* const o[2] = {a.out + (NM == 2 ? s0 : (size_t)f0) * a.n_rows,
-                           a.out + (NM == 2 ? s0 + 1 : (size_t)f1) * a.n_rows};
-      const float sc[2] = {NM == 2 ? 1.0f : a.topk_weights[f0], NM == 2 ? 1.0f : a.topk_weights[f1]};
-      matvec_rows<QUANT, KS, RPS, 2, NM>(w0, w1, a.K, a.n_rows, blockIdx.x * a.tile_rows, a.tile_rows, xr, o, sc);
-    } else {
-      const float* const xr[1] = {a.x + (NM == 2 ? (size_t)(f0 / a.top_k) : s0) * a.K};
-      float* const o[1] = {a.out + (NM == 2 ? s0 : (size_t)f0) * a.n_rows};
-      const float sc[1] = {NM == 2 ? 1.0f : a.topk_weights[f0]};
-      matvec_rows<QUANT, KS, RPS, 1, NM>(w0, w1, a.K, a.n_rows, blockIdx.x * a.tile_rows, a.tile_rows, xr, o, sc);
-    }
-  }
-}
-
-// The same dispatch-table work unit with the weights resident: a workgroup's tile is exactly what its four
-// wavefronts can hold in registers (DEPTH steps each), every weight byte is requested before the first wait,
-// and the block's token chunks then run against those registers -- the weights are read once per block
-// instead of once per chunk, and a wavefront's loads are all in flight together instead of one step at a
-// time.  Rows of at most 2048 elements (one step); n_rows must be a multiple of 4 * DEPTH * RPS.
-// The per-row arithmetic is matvec_rows', so the outputs are bit-identical to k_expert_block's.
-template <int N>
-struct TcC {
-  static constexpr int value = N;
-};
-
-template <int QUANT, int RPS, int NM, int DEPTH>
-__global__ void __launch_bounds__(256) k_expert_block_resident(ExpertArgs a) {
-  using F = Fmt<QUANT>;
-  using Raw = typename F::Raw;
-  constexpr int G = 64 / RPS;
-  const int b = blockIdx.y;
-  const int* slots = a.sorted_token_ids + (size_t)b * a.block_size;
-  const int e = a.expert_ids[b];
-  int f0 = slots[0], f1 = a.block_size > 1 ? slots[1] : 0x7fffffff;
-  const int valid = *a.valid_tokens;
-  if (e < 0) return;
-  const int sentinel = valid * a.top_k;
-  if (f0 >= sentinel) return;
-  const LaneGeom g = lane_geom<QUANT>();
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int koff = lane_koff<QUANT, RPS>(g, 0);
-  const size_t row_bytes = (size_t)(a.K / F::kBlockElems) * F::kBlockBytes;
-  const uint8_t* w0 = a.w0 + (size_t)e * a.expert_bytes;
-  const uint8_t* w1 = NM == 2 ? a.w1 + (size_t)e * a.expert_bytes : nullptr;
-  const int wave_row0 = ((int)blockIdx.x * kWavesPerWg + wave) * DEPTH * RPS;
-  // a chunk's activation rows (the second repeats the first in a one-token chunk: loaded, never used)
-  float x[2][32], xs[2][4];
-  bool two;
-  auto load_chunk = [&](int i) {
-    two = f1 < sentinel;
-    const size_t s0 = (size_t)b * a.block_size + i;
-    load_x<QUANT>(a.x + (NM == 2 ? (size_t)(f0 / a.top_k) : s0) * a.K, koff, true, g, x[0], xs[0]);
-    load_x<QUANT>(a.x + (NM == 2 ? (size_t)((two ? f1 : f0) / a.top_k) : (two ? s0 + 1 : s0)) * a.K, koff, true, g, x[1], xs[1]);
-  };
-  load_chunk(0);  // requested ahead of the weights, so it is there when they arrive
-  Raw r[DEPTH][NM];
-#pragma unroll
-  for (int d = 0; d < DEPTH; ++d) {
-    const size_t off = (size_t)(wave_row0 + d * RPS) * row_bytes;
-    load_raw<QUANT>(w0 + off, true, g, r[d][0]);
-    if constexpr (NM == 2) load_raw<QUANT>(w1 + off, true, g, r[d][NM - 1]);
-  }
-  for (int i = 0;;) {
-    const size_t s0 = (size_t)b * a.block_size + i;
-    auto chunk = [&](auto tc_c) {
-      constexpr int TC = decltype(tc_c)::value;
-      const int f[2] = {f0, f1};
-      const float (&xt)[TC][32] = *reinterpret_cast<const float (*)[TC][32]>(&x);
-      const float (&xst)[TC][4] = *reinterpret_cast<const float (*)[TC][4]>(&xs);
-      float* o[TC];
-      float sc[TC];
-#pragma unroll
-      for (int t = 0; t < TC; ++t) {
-        o[t] = a.out + (NM == 2 ? s0 + t : (size_t)f[t]) * a.n_rows;
-        sc[t] = NM == 2 ? 1.0f : a.topk_weights[f[t]];
-      }
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        float tot[NM][TC];
-#pragma unroll
-        for (int m = 0; m < NM; ++m) {
-#pragma unroll
-          for (int t = 0; t < TC; ++t) tot[m][t] = 0.0f;
-          accum<QUANT, TC>(r[d][m], g, xt, xst, tot[m]);
-#pragma unroll
-          for (int t = 0; t < TC; ++t) tot[m][t] = group_sum<G>(tot[m][t]);
-        }
-        const int row = wave_row0 + d * RPS + g.lane / G;
-        if ((g.lane % G) == 0) {
-#pragma unroll
-          for (int t = 0; t < TC; ++t) o[t][row] = NM == 2 ? silu_f(tot[0][t]) * tot[NM - 1][t] : sc[t] * tot[0][t];
-        }
-      }
-    };
-    if (two) chunk(TcC<2>{});
-    else chunk(TcC<1>{});
-    i += 2;
-    if (i >= a.block_size) break;
-    f0 = slots[i];
-    f1 = (i + 1 < a.block_size) ? slots[i + 1] : sentinel;
-    if (f0 >= sentinel) break;
-    load_chunk(i);
-  }
-}
-
 // Shared expert / dense MLP: every live token, no indirection, no routing weight
 // (crates/xabe-cuda/src/kernels/moe.rs:3425-3725, :4082-4227).  One work unit per chunk of two tokens.
 template <int QUANT, int KS, int RPS, int NM>
@@ -603,22 +390,6 @@ __device__ __forceinline__ void issue_fence() {
 template <int QUANT, int KS, int RPS, int NM>
 __global__ void __launch_bounds__(256) k_expert_shared(ExpertArgs a) {
   shared_body<QUANT, KS, RPS, NM>(a, blockIdx.y, blockIdx.x);
-}
-
-// The shared expert's work units appended to the routed grid (blockIdx.y >= routed_units), each
-// unit running the body its separate launch runs, so every output is bit-identical to the
-// four-launch form (crates/xabe-cuda/src/kernels/moe.rs:3727-4032).
-struct FusedArgs {
-  ExpertArgs routed;
-  ExpertArgs shared;
-  int routed_units;
-};
-
-template <int RQ, int SQ, int KS, int RPS, int NM>
-__global__ void __launch_bounds__(256) k_expert_flat_with_shared(FusedArgs a) {
-  const int unit = blockIdx.y;
-  if (unit < a.routed_units) flat_body<RQ, KS, RPS, NM>(a.routed, unit, blockIdx.x);
-  else shared_body<SQ, KS, RPS, NM>(a.shared, unit - a.routed_units, blockIdx.x);
 }
 
 }  // namespace xabe

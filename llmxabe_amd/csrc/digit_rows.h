@@ -68,11 +68,13 @@ __device__ __forceinline__ void store_digit_group(float v, int row, int nsb, uin
   mag = max(mag, dpp_i<0x140>(mag));
   const int e = mag >> 23, s = min(156 - e, 126);
   const uint32_t y = ((uint32_t)(int)__builtin_rintf(__builtin_ldexpf(v, s)) + 0x00808080u) ^ 0x00808080u;
+  // four lanes transpose their four digits: lane q of a quad stores digit q of the quad's elements as one word
+  const uint32_t y0 = dpp_i<0x00>((int)y), y1 = dpp_i<0x55>((int)y), y2 = dpp_i<0xAA>((int)y), y3 = dpp_i<0xFF>((int)y);
+  const int gi = row >> 4, j = row & 15, q = row & 3;
+  const uint32_t sel = (uint32_t)((7 - q) << 8 | (3 - q));
+  const uint32_t w = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y3, y2, sel), __builtin_amdgcn_perm(y1, y0, sel), 0x05040100u);
   if (!live) return;
-  const int gi = row >> 4, j = row & 15;
-  uint8_t* d = xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15) + j;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) d[16 * p] = (uint8_t)(y >> (24 - 8 * p));
+  *reinterpret_cast<uint32_t*>(xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15) + 16 * q + (j & ~3)) = w;
   if (j == 0) xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = e == 255 ? __builtin_nanf("") : __builtin_ldexpf(1.0f, 16 - s);
 }
 

@@ -35,17 +35,22 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
 }
 
 constexpr int kRowsZeros = 1024;
+// Tiles per wavefront of a routed unit, the next one's rows in flight while one is multiplied.  (Routed units serve the
+// step-by-step entry points; the block goes through decode_block.hip.)
+constexpr int kRowsRoutedTiles = 4;
+constexpr int kRowsBlockTokens = 2;  // tokens per chunk of a dispatch block (most hold one or two)
 
-template <int QUANT, int NT, bool TAIL>
+
+template <int MODE, int QUANT, int NT, bool TAIL>
 struct RowsLds {
   using Dma = SliceDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
-  static constexpr int kDigits = NT * kSbDigitBytes, kScales = NT * kSbScaleBytes;
+  static constexpr int kDigits = MODE == kRowsShared ? NT * kSbDigitBytes : 0, kScales = NT * kSbScaleBytes;
   static constexpr int kPerWave = Dma::kSlotBytes + kDigits + 2 * kScales;
 };
 
 template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
 __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
-  using L = RowsLds<QUANT, NT, TAIL>;
+  using L = RowsLds<MODE, QUANT, NT, TAIL>;
   using Dma = typename L::Dma;
   constexpr int TG = (NT + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
@@ -135,8 +140,10 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     for (int t = 0; t < NT; ++t)
       if ((lane >> 2) == t) x_row_l = x_row[t];
     auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
+      // (routed units keep a superblock's digits for a whole share and their tokens are few: they come straight into
+      // registers below, and the LDS they would take makes room for a second workgroup on the CU)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < NT && MODE == kRowsShared; ++t)
         dma_16b(a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
       if (lane < 4 * NT)  // (64 bytes per token)
         dma_16b(reinterpret_cast<const uint8_t*>(a.xe), ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16,
@@ -164,10 +171,26 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           if (i == 0) {
             x.point(d_slot, e_slot + buf * L::kScales, s_zero);
+            if constexpr (MODE == kRowsShared) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
+              for (int j = 0; j < 8; ++j)
 #pragma unroll
-              for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.digit(j & 3, j >> 2, tg);
+                for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.digit(j & 3, j >> 2, tg);
+            } else {
+              static_assert(MODE == kRowsShared || TG == 1, "routed units hold at most four tokens");
+              const int m = lane & 31;
+              int row = x_row[0];
+#pragma unroll
+              for (int t = 1; t < NT; ++t)
+                if ((m >> 3) == t) row = x_row[t];
+              const bool mine = ((m >> 2) & 1) == half && (m >> 3) < NT;
+              const uint8_t* d = a.xd + ((size_t)row * nsb + sb) * kSbDigitBytes + half * 128 + (m & 3) * 16;
+#pragma unroll
+              for (int j = 0; j < 8; ++j) {
+                ax[j][0] = v4i_t{0, 0, 0, 0};
+                if (mine) ax[j][0] = *reinterpret_cast<const v4i_t*>(d + (j & 3) * 256 + (j >> 2) * 64);
+              }
+            }
           }
           if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
 #pragma unroll
@@ -265,7 +288,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
 // ------------------------------------------------------------------ host side
 template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
 static size_t rows_lds() {
-  const size_t slots = (size_t)8 * RowsLds<QUANT, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * 64 * sizeof(float);
+  const size_t slots = (size_t)8 * RowsLds<MODE, QUANT, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * 64 * sizeof(float);
   return kRowsZeros + std::max(slots, red);
 }
 
@@ -300,8 +323,8 @@ static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, c
 
 template <int NM>
 static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
-  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, 1>(quant, tail, grid, s, a);
-  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, 4, 1>(quant, tail, grid, s, a);
+  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
+  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, kRowsBlockTokens, kRowsRoutedTiles>(quant, tail, grid, s, a);
   return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
 }
 
@@ -346,12 +369,14 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
   const int tiles16 = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
   a.n_tiles = tiles16;
   unsigned grid_x = (unsigned)((tiles16 + per_class - 1) / per_class);
-  if (mode == kRowsShared && per_class == 1 && tiles16 > k->num_cus) {
+  if (mode != kRowsShared) {
+    grid_x = (unsigned)((tiles16 + per_class * kRowsRoutedTiles - 1) / (per_class * kRowsRoutedTiles));
+  } else if (per_class == 1 && tiles16 > k->num_cus) {
     // many tiles: one workgroup per CU with an even share of them, so that a superblock's digits serve the whole share
     mt = kRowsMaxTiles;
     const unsigned rounds = (unsigned)((tiles16 + (size_t)k->num_cus * mt - 1) / ((size_t)k->num_cus * mt));
     grid_x = rounds * (unsigned)k->num_cus;
-  } else if (mode == kRowsShared && nm == 1 && per_class == 1 && tiles16 * 2 > k->num_cus && a.n_rows > k->num_cus) {
+  } else if (nm == 1 && per_class == 1 && tiles16 * 2 > k->num_cus && a.n_rows > k->num_cus) {
     // fewer tiles than CUs, but not by half: narrower tiles, one for every CU (5120 rows: 256 of 20, not 160 of 32)
     a.tile_rows = std::max(1, (a.n_rows + k->num_cus - 1) / k->num_cus);
     a.n_tiles = (a.n_rows + a.tile_rows - 1) / a.tile_rows;

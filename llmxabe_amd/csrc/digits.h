@@ -276,4 +276,83 @@ struct SliceDma {
   }
 };
 
+// ---------------------------------------------------------------------------------
+// Sixteen rows of two superblocks, one token: the one-token form of the core, on v_mfma_i32_16x16x64_i8.  Lane 16 q + r
+// holds row r and half q & 1 of superblock q >> 1 of the pair; operand A's row m is digit m & 3 in quarter m >> 2 of K
+// and zero elsewhere, so that the four result registers of a lane are the digit sums of the sixteen elements the lane
+// itself unpacked.  The same exact sums and the same fp32 operations per half superblock as sb_dot's, with no operand
+// rows spent on other tokens: for a single token 32 rows x 1 superblock and this shape carry the same bytes, and this
+// one needs no kilobyte of zeros in LDS and fits rows of one or two superblocks (a pair is then one row or two).
+// ---------------------------------------------------------------------------------
+template <int QUANT>
+struct PairDma {  // 29 pieces: 420 bytes at any even offset, rows four words apart modulo the banks; 35 likewise
+  using Dma = SliceDma<QUANT, QUANT == kQ6K ? 29 : 35>;
+  static constexpr int kSlotBytes = Dma::kRunBytes;
+};
+
+// The same slot where the sixteen pairs follow one another in memory (rows of one or two superblocks) from a 16-byte
+// boundary: 6720 or 8704 bytes, whole pieces, requested as they lie.  Q6_K pairs keep their 420-byte stride (105 words:
+// no two rows on one bank); Q8_0 pairs of 544 bytes get a piece between them.
+template <int QUANT>
+struct PairRunDma {
+  static constexpr int kPairPieces = 2 * SbRaw<QUANT>::kBytes / 16;  // (Q8_0: 34; Q6_K pairs are not whole pieces)
+  static constexpr int kRowStride = QUANT == kQ6K ? 2 * kQ6KBytes : (kPairPieces + 1) * 16;
+  static constexpr int kPieces = 16 * kRowStride / 16;
+  static constexpr int kInstr = (kPieces + 63) / 64, kSlotBytes = kInstr * 1024;
+  static __device__ __forceinline__ void request(const uint8_t* run, uint32_t dst) {
+    const uint32_t lane = __lane_id();
+#pragma unroll
+    for (int i = 0; i < kInstr; ++i) {
+      const uint32_t pc = min((uint32_t)(64 * i) + lane, (uint32_t)kPieces - 1);  // (a slot's padding repeats its last piece)
+      const uint32_t voff = QUANT == kQ6K ? pc * 16 : (pc / (kPairPieces + 1) * kPairPieces + min(pc % (kPairPieces + 1), (uint32_t)kPairPieces - 1)) * 16;
+      const uint32_t to = __builtin_amdgcn_readfirstlane(dst + i * 1024);
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(run), "s"(to) : "memory", "m0");
+#pragma clang diagnostic pop
+    }
+  }
+};
+
+// Operand A and the group scales of the lane's half superblock, straight from memory.
+struct PairDigits {
+  v4i_t a[8];   // [4 l + s]
+  float4 e[2];  // [l], s = 0..3
+  // `xd`, `xe`: digits and scales of the activation superblock the lane's weights lie in
+  __device__ __forceinline__ void load(const uint8_t* xd, const float* xe) {
+    const int lane = (int)__lane_id(), q = lane >> 4, m = lane & 15, h = q & 1;
+    const bool mine = (m >> 2) == q;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      a[j] = v4i_t{0, 0, 0, 0};
+      if (mine) a[j] = *reinterpret_cast<const v4i_t*>(xd + (j & 3) * 256 + (2 * h + (j >> 2)) * 64 + (m & 3) * 16);
+    }
+#pragma unroll
+    for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
+  }
+};
+
+template <int QUANT>
+__device__ __forceinline__ float pair_dot(const SbRaw<QUANT>& r, const PairDigits& x) {
+  float out = 0.0f, ws[2];
+  v4i_t d[2];
+  auto issue = [&](int j) __attribute__((always_inline)) {
+    v4i_t c;
+    sb_group(r, j & 3, j >> 2, c, ws[j & 1]);
+    const v4i_t zero = {0, 0, 0, 0};
+    d[j & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.a[j], c, zero, 0, 0, 0);
+  };
+  issue(0);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (j + 1 < 8) issue(j + 1);
+    const v4i_t& dd = d[j & 1];
+    const int hi = (dd[0] << 8) + dd[1], lo = (dd[2] << 8) + dd[3], s = j & 3;
+    const float f = __builtin_fmaf((float)lo, 0x1p-16f, (float)hi);
+    const float4& e = x.e[j >> 2];
+    out = __builtin_fmaf(f, ws[j & 1] * (s == 0 ? e.x : s == 1 ? e.y : s == 2 ? e.z : e.w), out);
+  }
+  return out;
+}
+
 }  // namespace xabe

@@ -13,11 +13,11 @@
 namespace xabe {
 
 // Widths at which the regimes change hands.
-//   <= kFlatMaxTokens: flat per-pair kernels, no dispatch table
+//   <= kFlatMaxTokens: one work unit per (token, k) pair, no dispatch table
 //      (MOE_NARROW_DECODE_MAX, crates/xabe-cuda/src/kernels/moe.rs:213-229).
 //   >= kMfmaMinTokens: matrix-core grouped GEMM.  The reference switches its int8 path in at 8
 //      tokens (MMA_MIN_TOKENS); here the fp32 regime is kept through 63 so that every decode
-//      batch up to 32 sequences stays bit-identical to single-stream decode.
+//      batch up to that width stays bit-identical to single-stream decode.
 constexpr size_t kFlatMaxTokens = 4;
 constexpr size_t kMfmaMinTokens = 64;
 constexpr size_t kRouteMaxExperts = 512;  // the routing wavefront holds 8 experts per lane
@@ -61,15 +61,11 @@ struct xabe_moe_kernels;
 struct xabe_moe_buffers;
 
 namespace xabe {
-// decode-width fusions (fused.hip).  `quant` < 0 means plain fp32 rows.
-int launch_flat_with_shared(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, int nm, int routed_quant,
-                            int shared_quant, const void* rw0, const void* rw1, size_t expert_bytes, const float* rx,
-                            float* rout, const void* sw0, const void* sw1, const float* sx, float* sout, int K,
-                            int n_rows);
 // rows per workgroup for a launch with `live_units` busy work units
 int pick_tile_rows(const xabe_moe_kernels* k, size_t live_units, int n_rows, int rows_per_step);
 
 // the decode-width block in three launches (decode_block.hip)
+int decode_block_configure();
 bool decode_block_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, const xabe_moe_layer_weights* w);
 // the checks the step-by-step entry points make on a layer's six stacks (whole blocks, element counts, formats,
 // 16-byte-aligned device pointers), for the block-level paths that launch without passing through them (api.hip)
@@ -156,7 +152,7 @@ struct xabe_moe_buffers {
   bool mma;
   xabe_moe_geometry g;
   // lengths in elements
-  size_t n_topk, n_sorted, n_expert_blocks, n_inter, n_partial, n_shared_inter;
+  size_t n_topk, n_sorted, n_expert_blocks, n_partial, n_shared_inter;
   int32_t* topk_ids;
   float* topk_weights;
   int32_t* sorted_token_ids;
@@ -169,7 +165,6 @@ struct xabe_moe_buffers {
   int32_t* valid_tokens;
   int32_t valid_published;  // what `valid_tokens` holds (0 after allocation)
   int32_t valid_host;       // source of the host-to-device copy that publishes a new count
-  float* inter;         // [slot][intermediate] fp32 (decode regimes)
   // digits and group scales (digits.h) of what the fp32 row contractions read: the pass's activation rows, the routed
   // intermediate rows (one per slot), the shared ones (one per token)
   uint8_t *x_d, *inter_d, *shared_inter_d;

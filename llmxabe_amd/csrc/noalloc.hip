@@ -16,6 +16,7 @@
 
 #include <mutex>
 
+#include "digit_rows.h"
 #include "host_common.h"
 
 namespace xabe {
@@ -31,11 +32,16 @@ constexpr size_t kNaTopkIds = kNaGate + na_align(kNaMaxTokens);                 
 constexpr size_t kNaTopkW = kNaTopkIds + na_align(kNaMaxTokens * kNaMaxTopK);         // [tokens][top_k]
 constexpr size_t kNaLogits = kNaTopkW + na_align(kNaMaxTokens * kNaMaxTopK);          // [tokens][experts]
 constexpr size_t kNaSharedInter = kNaLogits + na_align(kNaMaxTokens * kNaMaxExperts); // [tokens][intermediate]
-constexpr size_t kNaInter = kNaSharedInter + na_align(kNaMaxTokens * kNaMaxInter);    // [tokens * top_k][intermediate]
-constexpr size_t kNaNormed = kNaInter + na_align(kNaMaxTokens * kNaMaxTopK * kNaMaxInter);  // [tokens][hidden]
+// digits and group scales (digits.h) of the intermediate rows [tokens * top_k] and of the normalised rows [tokens]
+constexpr size_t kNaInterSb = kNaMaxTokens * kNaMaxTopK * (kNaMaxInter / kSbElems), kNaXSb = kNaMaxTokens * (kNaMaxHidden / kSbElems);
+constexpr size_t kNaInterD = kNaSharedInter + na_align(kNaMaxTokens * kNaMaxInter);
+constexpr size_t kNaInterE = kNaInterD + na_align(kNaInterSb * kSbDigitBytes / 4);
+constexpr size_t kNaXD = kNaInterE + na_align(kNaInterSb * kSbScaleBytes / 4);
+constexpr size_t kNaXE = kNaXD + na_align(kNaXSb * kSbDigitBytes / 4);
+constexpr size_t kNaNormed = kNaXE + na_align(kNaXSb * kSbScaleBytes / 4);             // [tokens][hidden]
 constexpr size_t kNaRouted = kNaNormed + na_align(kNaMaxTokens * kNaMaxHidden);
 constexpr size_t kNaShexp = kNaRouted + na_align(kNaMaxTokens * kNaMaxHidden);
-constexpr size_t kNaFloats = kNaShexp + na_align(kNaMaxTokens * kNaMaxHidden);        // 1 458 432 B in all
+constexpr size_t kNaFloats = kNaShexp + na_align(kNaMaxTokens * kNaMaxHidden);
 
 static __device__ __align__(256) float scratch[kNaFloats];
 
@@ -59,6 +65,7 @@ static int na_scratch(hipStream_t s, float** out) {
                        "block_forward_noalloc: the first call on device %d arrived while the stream is capturing; make one "
                        "call on the device before the capture begins", dev);
     float* p = nullptr;
+    XABE_TRY(decode_block_configure());
     XABE_HIP_TRY(hipGetSymbolAddress(reinterpret_cast<void**>(&p), HIP_SYMBOL(scratch)));
     if (!p) return set_error(XABE_ERR_DRIVER, "block_forward_noalloc: the scratch array has no address on device %d", dev);
     g_na_ptr[dev] = p;
@@ -113,10 +120,12 @@ int xabe_moe_block_forward_noalloc(const xabe_moe_geometry* geometry, float eps,
   b.valid_tokens = reinterpret_cast<int32_t*>(base + kNaValid);
   b.topk_ids = reinterpret_cast<int32_t*>(base + kNaTopkIds);
   b.topk_weights = base + kNaTopkW;
-  b.inter = base + kNaInter;
+  b.inter_d = reinterpret_cast<uint8_t*>(base + kNaInterD);
+  b.inter_e = base + kNaInterE;
+  b.x_d = reinterpret_cast<uint8_t*>(base + kNaXD);
+  b.x_e = base + kNaXE;
   b.shared_inter = base + kNaSharedInter;
   b.n_topk = g.max_tokens * g.experts_per_token;
-  b.n_inter = b.n_topk * g.intermediate;
   b.n_shared_inter = g.max_tokens * g.intermediate;
   if (!decode_block_supported(&k, &b, w))
     return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY,

@@ -149,3 +149,22 @@ def test_many_replays_keep_the_bits(oracle, X):
         blk.forward(layer.dev, x, 3, ffn, lout)
     torch.cuda.synchronize()
     assert torch.equal(first.view(torch.int32), lout.view(torch.int32))
+
+
+@pytest.mark.parametrize("max_tokens,tokens_seq", [(33, (33, 7)), (45, (45, 44)), (63, (63, 1, 0, 63))])
+def test_model_geometry_up_to_the_matrix_core_regime(oracle, X, max_tokens, tokens_seq):
+    # (the per-step path is the dispatch-table regime: blocks of several tokens against one token per work unit here)
+    g = X.MoeGeometry.qwen3_6(X.moe_block_size(max_tokens), max_tokens)
+    _compare(X, oracle, g, tokens_seq, seed=4700 + max_tokens, bias=(max_tokens == 45))
+
+
+@pytest.mark.parametrize("max_tokens", [6, 9, 47])
+@pytest.mark.parametrize("eq,dq,sq,sdq", [("Q6K", "Q8_0", "Q8_0", "Q6K"), ("Q8_0", "Q6K", "Q6K", "Q8_0"),
+                                          ("Q8_0", "Q8_0", "Q6K", "Q6K")])
+def test_formats_with_the_routing_inside_and_apart(oracle, X, max_tokens, eq, dq, sq, sdq):
+    # one, three and eight selections; the shared expert's down projection in the third launch (6 tokens) and in the second
+    q = lambda n: getattr(X.ExpertQuant, n)
+    for top_k in (1, 3, 8):
+        g = X.MoeGeometry(16, top_k, 512, 256, 32, max_tokens)
+        _compare(X, oracle, g, (max_tokens, max_tokens - 1), seed=4800 + max_tokens + top_k, expert_quant=q(eq),
+                 shared_quant=q(sq), down_quant=q(dq), shared_down_quant=q(sdq))
