@@ -408,11 +408,11 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
     else route_load<kRouteMaxPerLane>(a.logits + (size_t)t * a.E, a.E, nullptr, nullptr, lg);
   }
   const uint32_t row_bytes = (uint32_t)(2 * NP * SbRaw<RQ>::kBytes);
-  Dma dma;  // (its lane offsets are ready before the expert is known)
-  dma.init(row_bytes, 16);
   const size_t x_sb = (size_t)t * (2 * NP) + sb;
   PairDigits x;
   x.load(a.x_d + x_sb * kSbDigitBytes, a.x_e + x_sb * 16);
+  Dma dma;  // (its lane offsets are ready before the expert is known)
+  dma.init(row_bytes, 16);
   if (t >= valid) return;
   // Routing in two halves (route_device.h).  The first orders the experts by logit: its k-th candidate is
   // the pair's expert unless probabilities tie, and it is known ~2 us before the softmax is, so the

@@ -126,10 +126,12 @@ __device__ __forceinline__ void sb_group(const SbRaw<kQ6K>& r, int s, int l, v4i
   const v4u_t a = r.ql[(s & 1) * 2 + l], q = r.qh[l];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t lo = (s < 2 ? a[i] << 2 : a[i] >> 2) & 0x3c3c3c3cu;
-    const uint32_t f = q[i] ^ 0xaaaaaaaau;
-    const uint32_t hi = (s == 0 ? f << 6 : s == 1 ? f << 4 : s == 2 ? f << 2 : f) & 0xc0c0c0c0u;
-    c[i] = (int)(lo | hi);
+    // two shifts, one select of the two high bits from qh and the rest from ql, one mask and flip: four instructions per
+    // four codes, spelled out because the compiler makes five of the plain expression
+    const uint32_t lo = s < 2 ? a[i] << 2 : a[i] >> 2;
+    const uint32_t hi = s == 0 ? q[i] << 6 : s == 1 ? q[i] << 4 : s == 2 ? q[i] << 2 : q[i];
+    const uint32_t t = __builtin_amdgcn_bitop3_b32(hi, lo, 0xc0c0c0c0u, 0xE4);   // (hi & m) | (lo & ~m)
+    c[i] = (int)__builtin_amdgcn_bitop3_b32(t, 0xfcfcfcfcu, 0x80808080u, 0x6A);  // (t & b) ^ c
   }
   const uint32_t sw = s < 2 ? r.sc.x : r.sc.y;
   ws = (f16_bits_to_f32(r.d) * 0.25f) * (float)(int8_t)(sw >> (16 * (s & 1) + 8 * l));
@@ -323,9 +325,11 @@ struct PairDigits {
     const int lane = (int)__lane_id(), q = lane >> 4, m = lane & 15, h = q & 1;
     const bool mine = (m >> 2) == q;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      a[j] = v4i_t{0, 0, 0, 0};
-      if (mine) a[j] = *reinterpret_cast<const v4i_t*>(xd + (j & 3) * 256 + (2 * h + (j >> 2)) * 64 + (m & 3) * 16);
+    for (int j = 0; j < 8; ++j) a[j] = v4i_t{0, 0, 0, 0};
+    if (mine) {  // (one region for all eight loads)
+      const uint8_t* p = xd + h * 128 + (m & 3) * 16;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] = *reinterpret_cast<const v4i_t*>(p + (j & 3) * 256 + (j >> 2) * 64);
     }
 #pragma unroll
     for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
