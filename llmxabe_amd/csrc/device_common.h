@@ -136,6 +136,20 @@ __device__ __forceinline__ float row_inv_rms(const float* __restrict__ x, int wi
   return rms_finish(s, width, eps);
 }
 
+// One 16-byte piece per lane from `base` + the lane's byte offset `voff` straight into LDS, lane i's at byte address
+// `dst` + 16 i (`dst` the same in every lane; an inactive lane's sixteen bytes are left alone).  The DMA takes its LDS
+// address from m0 and may not be the instruction right after the write of m0: the hardware does not interlock that pair,
+// the compiler separates it by a wait state in code of its own and leaves inline assembly as it is, so the wait state is
+// spelled out.  m0 is named as clobbered so that the compiler sets it again before any use of its own; it warns that it
+// does not preserve the register across the statement, which is what is wanted here.
+__device__ __forceinline__ void lds_dma_16(const void* base, uint32_t voff, uint32_t dst) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base),
+               "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 // ---------------------------------------------------------------------------------
 // Streaming loads.  Blocks are 210 or 34 bytes, so block fields sit at 2-byte
 // alignment.  Unaligned dword loads cost about 15 % of achieved bandwidth on this

@@ -37,13 +37,6 @@ struct RowsArgs {
   uint32_t row_bytes;
 };
 
-__device__ __forceinline__ void dma_16b(const uint8_t* base, uint32_t voff, uint32_t dst) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
-#pragma clang diagnostic pop
-}
-
 // Group `gi` of a row, its sixteen values in `v`, into the row's digit planes and scales (zeros where the group lies
 // past the row's end).
 __device__ __forceinline__ void store_digits16(float (&v)[16], int gi, bool in, uint8_t* xd, float* xe) {

@@ -144,9 +144,9 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       // registers below, and the LDS they would take makes room for a second workgroup on the CU)
 #pragma unroll
       for (int t = 0; t < NT && MODE == kRowsShared; ++t)
-        dma_16b(a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
+        lds_dma_16(a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
       if (lane < 4 * NT)  // (64 bytes per token)
-        dma_16b(reinterpret_cast<const uint8_t*>(a.xe), ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16,
+        lds_dma_16(a.xe, ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16,
                 e_lds + buf * L::kScales);
     };
 

@@ -253,11 +253,7 @@ struct SliceDma {
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) {
       const uint32_t voff = min(((mis + row_off[i] + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & ~15u) + col[i], last);
-      const uint32_t to = __builtin_amdgcn_readfirstlane(dst + i * 1024);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(to) : "memory", "m0");
-#pragma clang diagnostic pop
+      lds_dma_16(base, voff, dst + i * 1024);
     }
   }
   // A tensor that ends inside a 16-byte piece: its last bytes, which no whole piece holds, go to the slot two by two
@@ -307,11 +303,7 @@ struct PairRunDma {
     for (int i = 0; i < kInstr; ++i) {
       const uint32_t pc = min((uint32_t)(64 * i) + lane, (uint32_t)kPieces - 1);  // (a slot's padding repeats its last piece)
       const uint32_t voff = QUANT == kQ6K ? pc * 16 : (pc / (kPairPieces + 1) * kPairPieces + min(pc % (kPairPieces + 1), (uint32_t)kPairPieces - 1)) * 16;
-      const uint32_t to = __builtin_amdgcn_readfirstlane(dst + i * 1024);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(run), "s"(to) : "memory", "m0");
-#pragma clang diagnostic pop
+      lds_dma_16(run, voff, dst + i * 1024);
     }
   }
 };

@@ -363,12 +363,7 @@ __global__ void __launch_bounds__(TBM == 384 ? 512 : 256, TBM == 64 ? 3 : 2) k_m
       // (the tile's base in scalar registers plus a 32-bit byte offset per lane: one address register instead of two)
       const uint32_t voff = (arow_off[i] + (uint32_t)ks * (uint32_t)kBK) * 2u;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_a + (uint32_t)(kThreads * 16) * i);  // + 16 * lane, by the hardware
-      // (m0 is named as clobbered so that the compiler sets it again before any use of its own; it warns that it
-      // does not preserve the register across the statement, which is what is wanted here)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(a.a), "s"(dst) : "memory", "m0");
-#pragma clang diagnostic pop
+      lds_dma_16(a.a, voff, dst);
     }
   };
 
@@ -872,10 +867,7 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
       const int q = i * kPCWaves + wave;
       const uint32_t voff = (off[i] + (uint32_t)ks * (uint32_t)kPK) * 2u;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_a + (uint32_t)(slot * kPM * kPK * 2) + (uint32_t)q * 1024u);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(a.a), "s"(dst) : "memory", "m0");
-#pragma clang diagnostic pop
+      lds_dma_16(a.a, voff, dst);
     }
   };
 
