@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "decode_kernels.h"
+#include "device_once.h"
 #include "digit_rows.h"
 #include "host_common.h"
 #include "route_device.h"
@@ -757,10 +758,8 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
   return true;
 }
 
-// LDS limits of the launches that ask for more than the static 64 KB; at handle creation (or a first call without one)
-int decode_block_configure() {
-  static bool done = false;  // (one device per process)
-  if (done) return XABE_OK;
+// LDS limits of the launches that ask for more than the static 64 KB
+static int decode_block_set_limits() {
 #define XABE_LDS(kernel, bytes) \
   XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes)))
 #define XABE_UP(Q, code, SQ, NP, RPSI)                                                       \
@@ -782,8 +781,15 @@ int decode_block_configure() {
 #undef XABE_DOWN
 #undef XABE_UP
 #undef XABE_LDS
-  done = true;
   return XABE_OK;
+}
+
+// at handle creation (or a first call without one), for the current device
+int decode_block_configure() {
+  static DeviceOnce once;
+  int dev = 0;
+  XABE_HIP_TRY(hipGetDevice(&dev));
+  return once.run(dev, decode_block_set_limits);
 }
 
 static bool launch_shape(const Launch& l, int gq, int dq, int sgq, int sdq, int router_quant) {

@@ -14,6 +14,7 @@
 
 #include <algorithm>
 
+#include "device_once.h"
 #include "digit_rows.h"
 #include "host_common.h"
 
@@ -328,9 +329,7 @@ static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, 
   return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
 }
 
-int digit_rows_configure() {
-  static bool done = false;  // (one device per process)
-  if (done) return XABE_OK;
+static int digit_rows_set_limits() {
   for (int q : {XABE_QUANT_Q6K, XABE_QUANT_Q8_0})
     for (bool tail : {false, true})
       for (int mode : {kRowsFlat, kRowsBlock, kRowsShared})
@@ -339,8 +338,15 @@ int digit_rows_configure() {
             XABE_TRY(rows_mode<1>(mode, nt, mt, q, tail, dim3(1), nullptr, nullptr));
             XABE_TRY(rows_mode<2>(mode, nt, mt, q, tail, dim3(1), nullptr, nullptr));
           }
-  done = true;
   return XABE_OK;
+}
+
+// at handle creation, for the current device
+int digit_rows_configure() {
+  static DeviceOnce once;
+  int dev = 0;
+  XABE_HIP_TRY(hipGetDevice(&dev));
+  return once.run(dev, digit_rows_set_limits);
 }
 
 int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe) {

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "device_once.h"
 #include "host_common.h"
 
 namespace xabe {
@@ -1169,9 +1170,7 @@ static int launch_pc(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, si
   return XABE_OK;
 }
 
-int mfma_configure() {
-  static bool done = false;  // (one device per process)
-  if (done) return XABE_OK;
+static int mfma_set_limits() {
   XABE_TRY((configure_pc<2>()));
   XABE_TRY((configure_pc<1>()));
   XABE_TRY((configure_one<1, false, 64>()));
@@ -1183,8 +1182,15 @@ int mfma_configure() {
   XABE_TRY((configure_one<2, true, 64>()));
   XABE_TRY((configure_one<2, true, 128>()));
   XABE_TRY((configure_one<2, true, 384>()));
-  done = true;
   return XABE_OK;
+}
+
+// at handle creation, for the current device
+int mfma_configure() {
+  static DeviceOnce once;
+  int dev = 0;
+  XABE_HIP_TRY(hipGetDevice(&dev));
+  return once.run(dev, mfma_set_limits);
 }
 
 template <int NM, bool ROUTED, int TBM>

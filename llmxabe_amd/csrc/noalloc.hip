@@ -16,6 +16,7 @@
 
 #include <mutex>
 
+#include "device_once.h"
 #include "digit_rows.h"
 #include "host_common.h"
 
@@ -45,9 +46,8 @@ constexpr size_t kNaFloats = kNaShexp + na_align(kNaMaxTokens * kNaMaxHidden);
 
 static __device__ __align__(256) float scratch[kNaFloats];
 
-constexpr int kNaMaxDevices = 64;
 static std::mutex g_na_mutex;
-static float* g_na_ptr[kNaMaxDevices];  // the array's address on each device, resolved on first use there
+static float* g_na_ptr[kMaxDevices];  // the array's address on each device, resolved on first use there
 
 // The calling thread's current device and the address of that device's copy of the array.  The address is resolved
 // on the first call on a device, and that call must not arrive while `s` is capturing: resolving the symbol may load
@@ -55,9 +55,9 @@ static float* g_na_ptr[kNaMaxDevices];  // the array's address on each device, r
 static int na_scratch(hipStream_t s, float** out) {
   int dev = 0;
   XABE_HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kNaMaxDevices)
+  if (dev < 0 || dev >= kMaxDevices)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "block_forward_noalloc: device ordinal %d is beyond the %d this entry point tracks",
-                     dev, kNaMaxDevices);
+                     dev, kMaxDevices);
   std::lock_guard<std::mutex> lock(g_na_mutex);
   if (!g_na_ptr[dev]) {
     if (stream_capture_id(s) != 0)
