@@ -383,10 +383,13 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->partial, b->n_partial);
   A(&b->shared_inter, b->n_shared_inter);
   const size_t nsb_h = digit_superblocks(g.hidden), nsb_i = digit_superblocks(g.intermediate);
-  A(&b->x_d, g.max_tokens * nsb_h * kSbDigitBytes);
-  A(&b->x_e, g.max_tokens * nsb_h * 16);
+  A(&b->x_d, routed ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
+  A(&b->x_e, routed ? g.max_tokens * nsb_h * 16 : 0);
   A(&b->inter_d, (routed ? sorted : 0) * nsb_i * kSbDigitBytes);
   A(&b->inter_e, (routed ? sorted : 0) * nsb_i * 16);
+  const bool shared_long = g.hidden > 2048;  // (shorter rows: the lanes' sums, shared_fp32)
+  A(&b->shared_x_d, shared_long ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
+  A(&b->shared_x_e, shared_long ? g.max_tokens * nsb_h * 16 : 0);
   A(&b->shared_inter_d, g.max_tokens * nsb_i * kSbDigitBytes);
   A(&b->shared_inter_e, g.max_tokens * nsb_i * 16);
   // matrix-core staging: only passes wide enough to take that regime pay for it
@@ -423,7 +426,8 @@ void xabe_moe_buffers_free(xabe_moe_buffers* b) {
   void* ptrs[] = {b->topk_ids, b->topk_weights, b->sorted_token_ids, b->expert_ids, b->bucket_live, b->expert_counts,
                   b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->partial, b->shared_inter, b->x_h, b->inter_h,
                   b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals,
-                  b->x_d, b->x_e, b->inter_d, b->inter_e, b->shared_inter_d, b->shared_inter_e};
+                  b->x_d, b->x_e, b->inter_d, b->inter_e, b->shared_x_d, b->shared_x_e,
+                  b->shared_inter_d, b->shared_inter_e};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete b;
@@ -699,7 +703,7 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
   return XABE_OK;
 }
 
-// gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->x_d
+// gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->shared_x_d
 static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                          xabe_quant_tensor up, xabe_quant_tensor down, float* out, const float* residual = nullptr,
                          float* l_out = nullptr) {
@@ -708,8 +712,8 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
   a.w1 = static_cast<const uint8_t*>(up.bytes);
   a.w_bytes = gate.len;
-  a.xd = b->x_d;
-  a.xe = b->x_e;
+  a.xd = b->shared_x_d;
+  a.xe = b->shared_x_e;
   a.out = b->shared_inter;
   a.out_d = b->shared_inter_d;
   a.out_e = b->shared_inter_e;
@@ -733,7 +737,7 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
   const xabe_moe_geometry& g = k->g;
   if (g.hidden > 2048) {
-    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->x_d, b->x_e));
+    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->shared_x_d, b->shared_x_e));
     return shared_digits(k, s, b, gate, up, down, out);
   }
   const size_t units = (g.max_tokens + 1) / 2;
@@ -767,7 +771,7 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
   if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(post_norm)) % 16 != 0)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "rms_norm: x, weight and out must be 16-byte aligned");
   hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)g.max_tokens), dim3(256), 0, s, residual, post_norm, normed, (int)g.hidden,
-                     eps, b->x_d, b->x_e);
+                     eps, b->shared_x_d, b->shared_x_e);
   XABE_HIP_TRY(hipGetLastError());
   XABE_TRY(shared_digits(k, s, b, gate, up, down, ffn_out, residual, l_out));
   *launched = true;
