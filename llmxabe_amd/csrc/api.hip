@@ -384,12 +384,13 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->shared_inter, b->n_shared_inter);
   const size_t nsb_h = digit_superblocks(g.hidden), nsb_i = digit_superblocks(g.intermediate);
   A(&b->x_d, routed ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
-  A(&b->x_e, routed ? g.max_tokens * nsb_h * 16 : 0);
+  A(&b->x_e, routed ? g.max_tokens * nsb_h : 0);
+  A(&b->inter, routed ? sorted * g.intermediate : 0);
   A(&b->inter_d, (routed ? sorted : 0) * nsb_i * kSbDigitBytes);
   A(&b->inter_e, (routed ? sorted : 0) * nsb_i * 16);
   const bool shared_long = g.hidden > 2048;  // (shorter rows: the lanes' sums, shared_fp32)
   A(&b->shared_x_d, shared_long ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
-  A(&b->shared_x_e, shared_long ? g.max_tokens * nsb_h * 16 : 0);
+  A(&b->shared_x_e, shared_long ? g.max_tokens * nsb_h : 0);
   A(&b->shared_inter_d, g.max_tokens * nsb_i * kSbDigitBytes);
   A(&b->shared_inter_e, g.max_tokens * nsb_i * 16);
   // matrix-core staging: only passes wide enough to take that regime pay for it
@@ -426,7 +427,7 @@ void xabe_moe_buffers_free(xabe_moe_buffers* b) {
   void* ptrs[] = {b->topk_ids, b->topk_weights, b->sorted_token_ids, b->expert_ids, b->bucket_live, b->expert_counts,
                   b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->partial, b->shared_inter, b->x_h, b->inter_h,
                   b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals,
-                  b->x_d, b->x_e, b->inter_d, b->inter_e, b->shared_x_d, b->shared_x_e,
+                  b->x_d, b->x_e, b->inter, b->inter_d, b->inter_e, b->shared_x_d, b->shared_x_e,
                   b->shared_inter_d, b->shared_inter_e};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -633,8 +634,10 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
     a.w1 = static_cast<const uint8_t*>(up.bytes);
     a.w_bytes = gate.len;
     a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
+    a.x = x;
     a.xd = b->x_d;
     a.xe = b->x_e;
+    a.out = b->inter;
     a.out_d = b->inter_d;
     a.out_e = b->inter_e;
     a.K = (int)g.hidden;
@@ -646,6 +649,7 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   a.w1 = nullptr;
   a.w_bytes = down.len;
   a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(down.quant) * xabe_expert_quant_block_bytes(down.quant);
+  a.x = b->inter;
   a.xd = b->inter_d;
   a.xe = b->inter_e;
   a.out = b->partial;
@@ -704,14 +708,16 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
 }
 
 // gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->shared_x_d
+// (x: the rows themselves)
 static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                         xabe_quant_tensor up, xabe_quant_tensor down, float* out, const float* residual = nullptr,
-                         float* l_out = nullptr) {
+                         xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out,
+                         const float* residual = nullptr, float* l_out = nullptr) {
   const xabe_moe_geometry& g = k->g;
   RowsArgs a = rows_args(k, b);
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
   a.w1 = static_cast<const uint8_t*>(up.bytes);
   a.w_bytes = gate.len;
+  a.x = x;
   a.xd = b->shared_x_d;
   a.xe = b->shared_x_e;
   a.out = b->shared_inter;
@@ -723,6 +729,7 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.w_bytes = down.len;
+  a.x = b->shared_inter;
   a.xd = b->shared_inter_d;
   a.xe = b->shared_inter_e;
   a.out = out;
@@ -738,7 +745,7 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   const xabe_moe_geometry& g = k->g;
   if (g.hidden > 2048) {
     XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->shared_x_d, b->shared_x_e));
-    return shared_digits(k, s, b, gate, up, down, out);
+    return shared_digits(k, s, b, gate, up, down, x, out);
   }
   const size_t units = (g.max_tokens + 1) / 2;
   ExpertArgs a = base_args(k, b);
@@ -773,7 +780,7 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
   hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)g.max_tokens), dim3(256), 0, s, residual, post_norm, normed, (int)g.hidden,
                      eps, b->shared_x_d, b->shared_x_e);
   XABE_HIP_TRY(hipGetLastError());
-  XABE_TRY(shared_digits(k, s, b, gate, up, down, ffn_out, residual, l_out));
+  XABE_TRY(shared_digits(k, s, b, gate, up, down, normed, ffn_out, residual, l_out));
   *launched = true;
   return XABE_OK;
 }

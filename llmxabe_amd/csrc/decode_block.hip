@@ -7,8 +7,8 @@
 // two rounds of loads:
 //
 //   A  k_decode_logits:  router logits (+ bias) and the shared expert's gate/up, both normalising the
-//                        residual rows on load; two workgroups per token write the normalised row with its digits
-//                        (digits.h) and the sigmoid gate scalar.
+//                        residual rows on load; a workgroup per superblock of a token writes the normalised row with
+//                        its digits (digits.h), one more per token the sigmoid gate scalar.
 //   B  k_decode_up:      one (token, k) pair x share of its row tiles per workgroup.  One wavefront routes the token
 //                        from its logits (every workgroup of a token repeats this: a few microseconds of one
 //                        wavefront is cheaper than one more launch or a device-wide handshake), then the wavefronts
@@ -77,7 +77,8 @@ struct DecodeArgs {
   int* topk_ids;
   float* topk_weights;
   uint8_t *x_d, *inter_d;  // digits of the normalised rows and of the routed intermediate rows (digits.h)
-  float *x_e, *inter_e;    // their group scales
+  float *x_e, *inter_e;    // their scales: of whole superblocks, of groups of 16
+  float* inter;            // the routed intermediate rows themselves
   float* shared_inter;
   float* shexp;
   float* gate_out;
@@ -218,18 +219,20 @@ __device__ __forceinline__ void tile_normed(const uint8_t* __restrict__ w0, cons
 }
 
 // ------------------------------------------------------------------------------------------------
-// A: grid = 2 max_tokens (norm and digits, gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
+// A: grid = max_tokens * superblocks (norm and digits) + max_tokens (gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
 // A chunk is two tokens sharing one pass over the weights.
 // ------------------------------------------------------------------------------------------------
 template <int SQ, int RF, int RPS, int kLogitsDepth, bool PRE = false>
 __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
   __shared__ float s_red[4];
+  __shared__ uint32_t s_mag[4];  // the row writers': a wavefront's largest magnitude
   __shared__ __attribute__((aligned(16))) float s_xn[3 * kXnPad];  // the chunk's rows and the norm weight
   const int chunks = (a.max_tokens + 1) / 2;
   const int n_r = chunks * a.tiles_r;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if ((int)blockIdx.x >= 2 * a.max_tokens) {
-    int item = blockIdx.x - 2 * a.max_tokens;
+  const int first_item = a.max_tokens * (a.H / kSbElems + 1);
+  if ((int)blockIdx.x >= first_item) {
+    int item = (int)blockIdx.x - first_item;
     const bool router = item < n_r;
     if (!router) item -= n_r;
     const int tiles = router ? a.tiles_r : a.tiles_s;
@@ -257,12 +260,32 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
     }
     return;
   }
-  // the normalised row (callers read it back) and g = sigmoid(shared_gate_inp . normed): the order of
-  // operations of the stand-alone RMSNorm and gate kernels
-  // (two workgroups per token: the row and its digits, and the scalar; in one they were the launch's last to end)
-  const bool writes_row = (int)blockIdx.x < a.max_tokens;
-  const int t = writes_row ? (int)blockIdx.x : (int)blockIdx.x - a.max_tokens;
+  const int nsb = a.H / kSbElems;  // (the served widths are multiples of 256)
   const int valid = *a.valid_tokens;
+  if ((int)blockIdx.x < a.max_tokens * nsb) {
+    // a superblock of the normalised row (callers read it back) and its digits, an element per thread: the order of
+    // operations of the stand-alone RMSNorm kernel
+    const int t = (int)blockIdx.x / nsb, sb = (int)blockIdx.x % nsb, j = sb * kSbElems + (int)threadIdx.x;
+    const float* xr = (PRE ? a.normed : a.residual) + (size_t)t * a.H;
+    float v = xr[j];  // (PRE: the row is there already, written by the previous block's tail)
+    if constexpr (!PRE) {
+      const float nw = a.post_norm[j], inv = row_inv_rms(xr, a.H, a.eps);
+      v = v * inv * nw;
+    }
+    if (t >= valid) return;
+    if constexpr (!PRE) a.normed[(size_t)t * a.H + j] = v;
+    uint32_t mag = (uint32_t)wave_max_i((int)(__builtin_bit_cast(uint32_t, v) & 0x7fffffffu));
+    if ((threadIdx.x & 63) == 0) s_mag[wave] = mag;
+    __syncthreads();
+    mag = max(max(s_mag[0], s_mag[1]), max(s_mag[2], s_mag[3]));
+    const int e = digit_exponent(mag);
+    const bool inexact = store_digit_lane(v, digit_shift(e), j, a.x_d + (size_t)t * nsb * kSbDigitBytes, true);
+    const float scale = digit_scale(mag, e, __syncthreads_or(inexact));
+    if (threadIdx.x == 0) a.x_e[(size_t)t * nsb + sb] = scale;
+    return;
+  }
+  // g = sigmoid(shared_gate_inp . normed): the order of operations of the stand-alone gate kernel
+  const int t = (int)blockIdx.x - a.max_tokens * nsb;
   const float* xr = (PRE ? a.normed : a.residual) + (size_t)t * a.H;
   // hidden <= 2048: eight columns per thread, every load issued before the first use
   float xv[8], nv[8], gv[8];
@@ -272,27 +295,15 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
     const bool in = j < a.H;
     xv[i] = in ? xr[j] : 0.0f;
     nv[i] = in && !PRE ? a.post_norm[j] : 0.0f;
-    gv[i] = in && !writes_row ? a.shared_gate_inp[j] : 0.0f;
+    gv[i] = in ? a.shared_gate_inp[j] : 0.0f;
   }
   float inv = 1.0f;
   if constexpr (!PRE) inv = row_inv_rms(xr, a.H, a.eps);
   if (t >= valid) return;
   float s = 0.0f;
-  const int nsb = a.H / kSbElems;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int j = threadIdx.x + 256 * i;
-    if (256 * i < a.H) {  // (the served widths are multiples of 256)
-      float v = xv[i];  // (PRE: the row is there already, written by the previous block's tail)
-      if constexpr (!PRE) {
-        v = xv[i] * inv * nv[i];
-        if (writes_row) a.normed[(size_t)t * a.H + j] = v;
-      }
-      if (writes_row) store_digit_group(v, j, nsb, a.x_d + (size_t)t * nsb * kSbDigitBytes, a.x_e + (size_t)t * nsb * 16, true);
-      else s = __builtin_fmaf(gv[i], v, s);
-    }
-  }
-  if (writes_row) return;
+  for (int i = 0; i < 8; ++i)
+    if (256 * i < a.H) s = __builtin_fmaf(gv[i], PRE ? xv[i] : xv[i] * inv * nv[i], s);
   s = group_sum<64>(s);
   if ((threadIdx.x & 63) == 0) s_red[wave] = s;
   __syncthreads();
@@ -368,7 +379,7 @@ __device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) 
 // 13.5 against 9.3 us for one token.)
 template <int RQ, int SQ, int NP, int RPSI, bool ROUTED>
 __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
-  using Dma = typename PairDma<RQ>::Dma;
+  using Dma = PairDma<RQ>;
   constexpr int kWaves = 2 * NP;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_up[];  // a weight slot per wavefront, then the routing's num_experts floats
   __shared__ int s_expert, s_final;      // the candidate expert of this pair; the one routing settles on
@@ -410,10 +421,10 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
   }
   const uint32_t row_bytes = (uint32_t)(2 * NP * SbRaw<RQ>::kBytes);
   const size_t x_sb = (size_t)t * (2 * NP) + sb;
-  PairDigits x;
-  x.load(a.x_d + x_sb * kSbDigitBytes, a.x_e + x_sb * 16);
+  PairDigits<kWhole> x;
+  x.load(a.x_d + x_sb * kSbDigitBytes, a.x_e + x_sb);
   Dma dma;  // (its lane offsets are ready before the expert is known)
-  dma.init(row_bytes, 16);
+  dma.init(row_bytes, sb0);
   if (t >= valid) return;
   // Routing in two halves (route_device.h).  The first orders the experts by logit: its k-th candidate is
   // the pair's expert unless probabilities tie, and it is known ~2 us before the softmax is, so the
@@ -442,7 +453,7 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
   auto stream_rows = [&](int e, auto finish_c) __attribute__((always_inline)) {
     const size_t e_off = (size_t)e * a.expert_bytes;
     auto run_off = [&](int i) __attribute__((always_inline)) { return e_off + (size_t)(16 * (share * a.share_g + i)) * row_bytes; };
-    dma.request(mat ? a.up : a.gate, a.up_len, run_off(0), sb0, slot_lds);
+    dma.request(mat ? a.up : a.gate, a.up_len, run_off(0), slot_lds);
     if constexpr (decltype(finish_c)::value) {
       if (routes) {  // (raised priority keeps it ahead of its neighbours' arithmetic)
         __builtin_amdgcn_s_setprio(3);
@@ -463,12 +474,13 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
     }
 #pragma unroll 1
     for (int i = 0; i < a.share_g; ++i) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      wait_loads();
       SbRaw<RQ> raw;
-      sb_read(dma.row_at(slot, run_off(i), lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+      sb_read(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), sb0, slot_lds);
-      s_red[i][sb][(quarter & 1) * 32 + mat * 16 + (lane & 15)] = pair_dot<RQ>(raw, x);
+      if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), slot_lds);
+      s_red[i][sb][(quarter & 1) * 32 + mat * 16 + (lane & 15)] = pair_dot<RQ>(
+          raw, x, [&](int q) __attribute__((always_inline)) { return a.normed + (size_t)t * a.H + (sb0 + (q >> 1)) * kSbElems; });
     }
     __syncthreads();  // (s_final is there, too)
   };
@@ -491,8 +503,10 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
     }
     const float total = h0 + h1, up = __shfl_xor(total, 16);
     const int nsb_i = a.I / kSbElems;
-    store_digit_group(silu_f(total) * up, 16 * (share * a.share_g + i) + (lane & 15), nsb_i,
-                      a.inter_d + (size_t)p * nsb_i * kSbDigitBytes, a.inter_e + (size_t)p * nsb_i * 16, lane < 16);
+    const float v = silu_f(total) * up;
+    const int row = 16 * (share * a.share_g + i) + (lane & 15);
+    if (lane < 16) a.inter[(size_t)p * a.I + row] = v;
+    store_digit_group(v, row, a.inter_d + (size_t)p * nsb_i * kSbDigitBytes, a.inter_e + (size_t)p * nsb_i * 16, lane < 16);
   }
 }
 
@@ -566,23 +580,26 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
     const int e = __builtin_amdgcn_readfirstlane(min(max(a.topk_ids[p], 0), a.E - 1));
     const float sel_w = a.topk_weights[p];
     constexpr int nsb = kPairRows == 1 ? 2 : 1;
-    const size_t x_sb = (size_t)p * nsb + (kPairRows == 1 ? quarter >> 1 : 0);
     const uint32_t pair_bytes = 2 * SbRaw<RQ>::kBytes;
     uint8_t* const slot = s_down + wave * Dma::kSlotBytes;
     const uint32_t slot_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot);
     auto run = [&](int i) __attribute__((always_inline)) { return a.down + (size_t)e * a.down_bytes + (size_t)(tile0 + i) * 16 * pair_bytes; };
     if (t >= valid) return;
-    Dma::request(run(0), slot_lds);
-    PairDigits x;
+    Dma dma;
+    dma.init();
+    dma.request(run(0), slot_lds);
+    const size_t x_sb = (size_t)p * nsb + (kPairRows == 1 ? quarter >> 1 : 0);
+    PairDigits<kGroups> x;
     x.load(a.inter_d + x_sb * kSbDigitBytes, a.inter_e + x_sb * 16);
 #pragma unroll 1
     for (int i = 0; i < a.share_d; ++i) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      wait_loads();
       SbRaw<RQ> raw;
       sb_read(slot + (lane & 15) * Dma::kRowStride + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (i + 1 < a.share_d) Dma::request(run(i + 1), slot_lds);
-      float v = pair_dot<RQ>(raw, x);
+      if (i + 1 < a.share_d) dma.request(run(i + 1), slot_lds);
+      float v = pair_dot<RQ>(
+          raw, x, [&](int q) __attribute__((always_inline)) { return a.inter + ((size_t)p * nsb + (kPairRows == 1 ? q >> 1 : 0)) * kSbElems; });
       // superblock 0 + superblock 1 of each half, then half 0 + half 1
       if constexpr (kPairRows == 1) v += __shfl_xor(v, 32);
       v += __shfl_xor(v, 16);
@@ -848,6 +865,7 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   a.x_e = b->x_e;
   a.inter_d = b->inter_d;
   a.inter_e = b->inter_e;
+  a.inter = b->inter;
   a.up_len = w->gate_exps.len;
   a.shared_inter = b->shared_inter;
   a.shexp = shexp;
@@ -877,7 +895,7 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   const int chunks = (a.max_tokens + 1) / 2;
   const bool pre_routed = a.max_tokens >= kPreRouteMinTokens;
   Launch l{a, s, 0, 0, 0, pre_routed, seam && seam->input_normed, launches};
-  l.grid_a = (unsigned)(chunks * (a.tiles_r + a.tiles_s) + 2 * a.max_tokens);
+  l.grid_a = (unsigned)(chunks * (a.tiles_r + a.tiles_s) + a.max_tokens * (a.H / kSbElems + 1));
   // wide batches pad the shares of a pair (token) to whole rounds of eight, one per XCD
   auto grid_of = [&](size_t units, int shares) { return (unsigned)(units * (a.max_tokens >= kXcdGroupMinTokens ? (shares + 7) / 8 * 8 : shares)); };
   a.shared_from = (int)grid_of((size_t)a.max_tokens * a.top_k, a.tiles_g / a.share_g);

@@ -150,6 +150,15 @@ __device__ __forceinline__ void lds_dma_16(const void* base, uint32_t voff, uint
 #pragma clang diagnostic pop
 }
 
+// Everything this wavefront has requested from memory is there, the DMA's bytes in LDS among it.  Said twice: the compiler
+// counts its own loads and takes note of the builtin (a wait of its own for a register loaded before a loop would
+// otherwise stand at its use inside, and wait there for the DMA requested since); it does not count the DMA, whose wait
+// the statement is.
+__device__ __forceinline__ void wait_loads() {
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------------
 // Streaming loads.  Blocks are 210 or 34 bytes, so block fields sit at 2-byte
 // alignment.  Unaligned dword loads cost about 15 % of achieved bandwidth on this

@@ -19,9 +19,10 @@ struct RowsArgs {
   const uint8_t* w1;         // up stack (nm = 2)
   size_t w_bytes;            // length of each stack
   size_t expert_bytes;       // bytes of one expert in a stack (0: a single matrix)
+  const float* x;            // the activation rows, [row][K] (what a marked group goes back to)
   const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes]
-  const float* xe;           // their group scales, [row][superblock][16]
-  float* out;                // [row][n_rows]; nm = 2: may be null
+  const float* xe;           // their scales: gate/up [row][superblock], down [row][superblock][16] (by group)
+  float* out;                // [row][n_rows]
   uint8_t* out_d;            // nm = 2: digits of the output rows
   float* out_e;
   const float* residual;     // with l_out: l_out = out + residual
@@ -37,38 +38,42 @@ struct RowsArgs {
   uint32_t row_bytes;
 };
 
-// Group `gi` of a row, its sixteen values in `v`, into the row's digit planes and scales (zeros where the group lies
-// past the row's end).
+// Group `gi` of a row, its sixteen values in `v` (sixteen consecutive lanes hold a superblock's), into the row's digits and
+// superblock scales (zeros where the group lies past the row's end).
 __device__ __forceinline__ void store_digits16(float (&v)[16], int gi, bool in, uint8_t* xd, float* xe) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) v[i] = in ? v[i] : 0.0f;
-  v4u_t plane[4];
-  float scale;
-  digitize16(v, plane, scale);
-  uint8_t* d = xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15);
-#pragma unroll
-  for (int p = 0; p < 4; ++p) reinterpret_cast<v4u_t*>(d)[p] = plane[p];
-  xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = in ? scale : 0.0f;
+  const float scale = digitize_superblock(v, gi & 15, xd + (size_t)(gi >> 4) * kSbDigitBytes);
+  if ((gi & 15) == 0) xe[gi >> 4] = scale;
 }
 
-// The same for a group that sixteen consecutive lanes (a DPP row) hold one element each: lane's value `v` is element
-// `row` of the output row whose digits start at xd and scales at xe.
-__device__ __forceinline__ void store_digit_group(float v, int row, int nsb, uint8_t* xd, float* xe, bool live) {
-  int mag = (int)(__builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
-  mag = max(mag, dpp_i<0xB1>(mag));
-  mag = max(mag, dpp_i<0x4E>(mag));
-  mag = max(mag, dpp_i<0x141>(mag));
-  mag = max(mag, dpp_i<0x140>(mag));
-  const int e = mag >> 23, s = min(156 - e, 126);
-  const uint32_t y = ((uint32_t)(int)__builtin_rintf(__builtin_ldexpf(v, s)) + 0x00808080u) ^ 0x00808080u;
-  // four lanes transpose their four digits: lane q of a quad stores digit q of the quad's elements as one word
+// The digits of a group that sixteen consecutive lanes (a DPP row) hold one element each: lane's value `v` is element
+// `row` of the row whose digits start at xd.  Returns whether this lane's element is not held exactly.
+__device__ __forceinline__ bool store_digit_lane(float v, int shift, int row, uint8_t* xd, bool live) {
+  uint32_t y, z;
+  bool inexact = false;
+  digits_of(v, shift, y, z, inexact);
+  // four lanes transpose their digits: lane q of a quad stores digit q of the quad's elements as one word, lanes 0 and 1
+  // digits 4 and 5 as well
   const uint32_t y0 = dpp_i<0x00>((int)y), y1 = dpp_i<0x55>((int)y), y2 = dpp_i<0xAA>((int)y), y3 = dpp_i<0xFF>((int)y);
+  const uint32_t z0 = dpp_i<0x00>((int)z), z1 = dpp_i<0x55>((int)z), z2 = dpp_i<0xAA>((int)z), z3 = dpp_i<0xFF>((int)z);
   const int gi = row >> 4, j = row & 15, q = row & 3;
-  const uint32_t sel = (uint32_t)((7 - q) << 8 | (3 - q));
+  const uint32_t sel = (uint32_t)((7 - q) << 8 | (3 - q)), sel_z = (uint32_t)((5 - (q & 1)) << 8 | (1 - (q & 1)));
   const uint32_t w = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y3, y2, sel), __builtin_amdgcn_perm(y1, y0, sel), 0x05040100u);
-  if (!live) return;
-  *reinterpret_cast<uint32_t*>(xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15) + 16 * q + (j & ~3)) = w;
-  if (j == 0) xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = e == 255 ? __builtin_nanf("") : __builtin_ldexpf(1.0f, 16 - s);
+  const uint32_t wz = __builtin_amdgcn_perm(__builtin_amdgcn_perm(z3, z2, sel_z), __builtin_amdgcn_perm(z1, z0, sel_z), 0x05040100u);
+  if (!live) return inexact;
+  uint8_t* d = xd + (size_t)(gi >> 4) * kSbDigitBytes + digit_group_offset(gi & 15) + 16 * q + (j & ~3);
+  *reinterpret_cast<uint32_t*>(d) = w;
+  if (q < 2) *reinterpret_cast<uint32_t*>(d + 64) = wz;
+  return inexact;
+}
+
+// The same with the scale of the group, [superblock][16] at xe.
+__device__ __forceinline__ void store_digit_group(float v, int row, uint8_t* xd, float* xe, bool live) {
+  const uint32_t mag = row16_max(__builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
+  const int e = digit_exponent(mag), gi = row >> 4;
+  const bool inexact = row16_any(store_digit_lane(v, digit_shift(e), row, xd, live));
+  if (live && (row & 15) == 0) xe[(gi >> 4) * 16 + scale_group_index(gi & 15)] = digit_scale(mag, e, inexact);
 }
 
 // host side

@@ -20,7 +20,7 @@
 
 namespace xabe {
 
-// Digits of fp32 rows: one thread per group of sixteen; groups past the end of the row are zeros with scale zero.
+// Digits of fp32 rows, scaled by superblocks: one thread per group of sixteen; groups past the end of the row are zeros.
 __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__ x, int K, int nsb, int rows, uint8_t* __restrict__ xd,
                                                        float* __restrict__ xe) {
   const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -32,26 +32,30 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
     const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(4 * gi + j, K / 4 - 1)];
     v[4 * j] = f.x, v[4 * j + 1] = f.y, v[4 * j + 2] = f.z, v[4 * j + 3] = f.w;
   }
-  store_digits16(v, gi, gi * 16 < K, xd + (size_t)row * nsb * kSbDigitBytes, xe + (size_t)row * nsb * 16);
+  store_digits16(v, gi, gi * 16 < K, xd + (size_t)row * nsb * kSbDigitBytes, xe + (size_t)row * nsb);
 }
 
-constexpr int kRowsZeros = 1024;
 // Tiles per wavefront of a routed unit, the next one's rows in flight while one is multiplied.  (Routed units serve the
 // step-by-step entry points; the block goes through decode_block.hip.)
 constexpr int kRowsRoutedTiles = 4;
 constexpr int kRowsBlockTokens = 2;  // tokens per chunk of a dispatch block (most hold one or two)
 
-
-template <int MODE, int QUANT, int NT, bool TAIL>
+template <int MODE, int QUANT, int NM, int NT, bool TAIL>
 struct RowsLds {
   using Dma = SliceDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
-  static constexpr int kDigits = MODE == kRowsShared ? NT * kSbDigitBytes : 0, kScales = NT * kSbScaleBytes;
+  static constexpr int kDigits = MODE == kRowsShared ? NT * kSbDigitBytes : 0, kScales = NM == 1 ? NT * kSbScaleBytes : 0;
   static constexpr int kPerWave = Dma::kSlotBytes + kDigits + 2 * kScales;
 };
 
-template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+// TEAMS: one team of eight wavefronts for up to four tokens, or two teams of four, each with four tokens of its own and
+// twice the classes: the digits and sums of eight tokens take more registers than a wavefront has and more LDS than
+// eight wavefronts have.  Both teams request every row (the second time out of L2) and wait for nobody.
+template <int MODE, int QUANT, int NM, int NT, int TEAMS, int MT, bool TAIL>
 __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
-  using L = RowsLds<MODE, QUANT, NT, TAIL>;
+  constexpr int kTeam = 8 / TEAMS, kRounds = TEAMS, kTokens = NT * TEAMS;
+  using L = RowsLds<MODE, QUANT, NM, NT, TAIL>;
+  // gate and up read rows whose scales are whole superblocks', down the intermediate rows, scaled by groups
+  constexpr bool kScale = NM == 2 ? kWhole : kGroups, kSwapped = kAddsGroups<QUANT, kScale> && !digits_in_one(NT);
   using Dma = typename L::Dma;
   constexpr int TG = (NT + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
@@ -75,29 +79,30 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     slots = a.sorted_token_ids + slot0;
     n_tok = a.block_size;
   } else {
-    slot0 = (size_t)blockIdx.y * NT;
+    slot0 = (size_t)blockIdx.y * kTokens;
     if ((int)slot0 >= valid) return;
-    n_tok = min(NT, valid - (int)slot0);
+    n_tok = min(kTokens, valid - (int)slot0);
   }
   const int sentinel = valid * a.top_k;
 
   // ---- this wavefront's class and tiles
-  const int classes = a.classes, per_class = 8 / classes;
-  const int cls = wave % classes, sub = wave / classes;
+  const int team = wave / kTeam, member = wave % kTeam, t0 = team * NT;             // (the team's tokens: t0 ..)
+  const int classes = a.classes, side = min(classes, kTeam), per_class = kTeam / side;  // `side` classes at a time
+  const int cls = member % side, sub = member / side, rounds = classes / side;        // (at most kRounds)
   const int tile_lo = (int)((long long)a.n_tiles * (int)blockIdx.x / (int)gridDim.x);
   const int n_wg = (int)((long long)a.n_tiles * ((int)blockIdx.x + 1) / (int)gridDim.x) - tile_lo;  // <= MT * per_class
   const int n_mine = (n_wg - sub + per_class - 1) / per_class;
   const int nsb = a.nsb;
   const uint32_t row_bytes = a.row_bytes;
   uint8_t* const s_zero = s_rows;
-  uint8_t* const w_slot = s_rows + kRowsZeros + (size_t)wave * L::kPerWave;
+  uint8_t* const w_slot = s_rows + kZeroBytes + (size_t)wave * L::kPerWave;
   uint8_t* const d_slot = w_slot + Dma::kSlotBytes;
   uint8_t* const e_slot = d_slot + L::kDigits;
   auto lds_addr = [](uint8_t* p) __attribute__((always_inline)) {
     return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)p);
   };
   const uint32_t w_lds = lds_addr(w_slot), d_lds = lds_addr(d_slot), e_lds = lds_addr(e_slot);
-  for (int i = threadIdx.x; i < kRowsZeros / 16; i += 512) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
+  for (int i = threadIdx.x; i < kZeroBytes / 16; i += 512) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
 
   // rows of tile i of this wavefront: run 0 and run 1 (NM == 2: gate and up, the same 16 rows of each)
   const int tile_rows = NM == 2 ? 16 : a.tile_rows;
@@ -109,14 +114,25 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   Dma dma[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) dma[u].init(row_bytes, NM == 2 ? 16 : min(max(tile_rows - 16 * u, 1), 16));
+  const uint64_t live_lanes = __builtin_amdgcn_ballot_w64((lane & 31) < (NM == 2 ? 32 : tile_rows));
   auto request_w = [&](int i, int sb) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 2; ++u)
       dma[u].request(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, e_off + (size_t)run_row(i, u) * row_bytes, sb, w_lds + u * Dma::kRunBytes);
   };
+  // A wavefront's steps: for every superblock of its classes in order, every one of its tiles.
+  struct Step {
+    int sb, i, round;
+  };
+  auto advance = [&](Step& p) __attribute__((always_inline)) {
+    if (++p.i < n_mine) return;
+    p.i = 0;
+    p.sb += classes;
+    if (kRounds > 1 && p.sb >= nsb && ++p.round < rounds) p.sb = cls + p.round * side;
+  };
   const int u_lane = (lane >> 4) & 1, r_lane = lane & 15, half = lane >> 5;
 
-  for (int first = 0; first < n_tok; first += NT) {
+  for (int first = 0; first < n_tok; first += kTokens) {
     // the chunk's tokens: activation rows (tokens past the live ones repeat one of them and are never stored)
     int x_row[NT], n_live = 0;
     if constexpr (MODE == kRowsFlat) {
@@ -134,106 +150,136 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     } else {
       n_live = n_tok;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) x_row[t] = (int)slot0 + min(t, n_live - 1);
+      for (int t = 0; t < NT; ++t) x_row[t] = (int)slot0 + min(t0 + t, n_live - 1);
     }
     int x_row_l = x_row[NT - 1];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       if ((lane >> 2) == t) x_row_l = x_row[t];
+    float e_now[NT], e_next[NT];  // (whole superblocks' scales)
     auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
       // (routed units keep a superblock's digits for a whole share and their tokens are few: they come straight into
       // registers below, and the LDS they would take makes room for a second workgroup on the CU)
 #pragma unroll
-      for (int t = 0; t < NT && MODE == kRowsShared; ++t)
-        lds_dma_16(a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
-      if (lane < 4 * NT)  // (64 bytes per token)
-        lds_dma_16(a.xe, ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16,
-                e_lds + buf * L::kScales);
+      for (int t = 0; t < NT && MODE == kRowsShared; ++t) {
+        const uint8_t* from = a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes;
+        lds_dma_16(from, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
+        if (lane < 32) lds_dma_16(from + 1024, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes + 1024);
+      }
+      if constexpr (kScale == kGroups) {
+        if (lane < 4 * NT)  // (64 bytes per token)
+          lds_dma_16(a.xe, ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16, e_lds + buf * L::kScales);
+      } else {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) e_next[t] = a.xe[(size_t)x_row[t] * nsb + sb];
+      }
     };
 
-    float acc[MT][NT];
+    float acc[kRounds][MT][NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int r = 0; r < kRounds; ++r)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[i][t] = 0.0f;
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[r][i][t] = 0.0f;
     if (first == 0) __syncthreads();  // the zeros are there
-    if (cls < nsb && n_mine > 0) {
+    // Requests run one step ahead, rows and digits: both leave LDS for registers before the next ones are requested.
+    Step now = {cls, 0, 0};
+    const bool any = cls < nsb && n_mine > 0 && t0 < n_live;
+    if (any) {
       request_w(0, cls);
       request_x(cls, 0);
     }
     int buf = 0;
-    if (n_mine > 0) {
+    if (any) {
+      v4i_t ax[8][TG], az[kSwapped ? 8 : 4][TG];
+      LdsDigits<NT, kSbDigitBytes, kSwapped> x;
 #pragma unroll 1
-      for (int sb = cls; sb < nsb; sb += classes, buf ^= 1) {
-        v4i_t ax[8][TG];
-        LdsDigits<NT, kSbDigitBytes> x;
-#pragma unroll 1
-        for (int i = 0; i < n_mine; ++i) {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          if (i == 0) {
-            x.point(d_slot, e_slot + buf * L::kScales, s_zero);
-            if constexpr (MODE == kRowsShared) {
+      while (now.sb < nsb) {
+        const int sb = now.sb, i = now.i;
+        Step next = now;
+        advance(next);
+        wait_loads();
+        if (i == 0) {
+          if constexpr (kScale == kWhole) {
 #pragma unroll
-              for (int j = 0; j < 8; ++j)
+            for (int t = 0; t < NT; ++t) e_now[t] = e_next[t];
+          }
+          x.point(d_slot, e_slot + buf * L::kScales, s_zero);
+          if constexpr (MODE == kRowsShared) {
 #pragma unroll
-                for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.digit(j & 3, j >> 2, tg);
-            } else {
-              static_assert(MODE == kRowsShared || TG == 1, "routed units hold at most four tokens");
-              const int m = lane & 31;
-              int row = x_row[0];
+            for (int j = 0; j < 8; ++j)
 #pragma unroll
-              for (int t = 1; t < NT; ++t)
-                if ((m >> 3) == t) row = x_row[t];
-              const bool mine = ((m >> 2) & 1) == half && (m >> 3) < NT;
-              const uint8_t* d = a.xd + ((size_t)row * nsb + sb) * kSbDigitBytes + half * 128 + (m & 3) * 16;
+              for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.high(j & 3, j >> 2, tg);
 #pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                ax[j][0] = v4i_t{0, 0, 0, 0};
-                if (mine) ax[j][0] = *reinterpret_cast<const v4i_t*>(d + (j & 3) * 256 + (j >> 2) * 64);
-              }
+            for (int j = 0; j < (kSwapped ? 8 : 4) && !digits_in_one(NT); ++j)
+#pragma unroll
+              for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
+          } else {
+            static_assert(MODE == kRowsShared || digits_in_one(NT), "routed units hold one or two tokens");
+            const int at = high_digit_at<NT>(lane, 0, 0);
+            const int row = NT > 1 && (lane & 16) ? x_row[NT - 1] : x_row[0];
+            const uint8_t* d = a.xd + ((size_t)row * nsb + sb) * kSbDigitBytes + max(at, 0);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              ax[j][0] = v4i_t{0, 0, 0, 0};
+              if (at >= 0) ax[j][0] = *reinterpret_cast<const v4i_t*>(d + (4 * (j & 3) + (j >> 2)) * kGroupBytes);
             }
-          }
-          if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              const size_t off = e_off + (size_t)run_row(i, u) * row_bytes;
-              const int live = min(min(tile_rows - (NM == 2 ? 0 : 16 * u), 16), a.n_rows - (tile_of(i) * tile_rows + (NM == 2 ? 0 : 16 * u)));
-              if (live >= 1 && off + (size_t)live * row_bytes == a.w_bytes) dma[u].patch_tail(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, off, live, sb, w_slot + u * Dma::kRunBytes);
-            }
-          }
-          SbRaw<QUANT> raw;
-          sb_read(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-          if (i + 1 < n_mine) {
-            request_w(i + 1, sb);
-          } else if (sb + classes < nsb) {
-            request_w(0, sb + classes);
-            request_x(sb + classes, buf ^ 1);
-          }
-          float v[NT];
-          sb_dot<QUANT, NT, TAIL>(raw, [&](int s, int l, int tg) { return ax[4 * l + s][tg]; },
-                                  [&](int t, int l) { return x.template scale<kSbScaleBytes>(t, l); }, v,
-                                  TAIL && half == 1 && (sb * kSbElems + 128) >= a.K);
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {  // (the sums stay in registers: the tile's own by a uniform branch, not by an index)
-            if (MT > 1 && m != i) continue;
-            if (MT > 1) asm volatile("");
-#pragma unroll
-            for (int t = 0; t < NT; ++t) acc[m][t] += v[t];
           }
         }
+        if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const size_t off = e_off + (size_t)run_row(i, u) * row_bytes;
+            const int live = min(min(tile_rows - (NM == 2 ? 0 : 16 * u), 16), a.n_rows - (tile_of(i) * tile_rows + (NM == 2 ? 0 : 16 * u)));
+            if (live >= 1 && off + (size_t)live * row_bytes == a.w_bytes) dma[u].patch_tail(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, off, live, sb, w_slot + u * Dma::kRunBytes);
+          }
+        }
+        SbRaw<QUANT> raw;
+        sb_read(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (next.sb < nsb) request_w(next.i, next.sb);
+        if (next.sb < nsb && next.i == 0) request_x(next.sb, buf ^ 1);
+        float v[NT];
+        auto x_of = [&](int t) __attribute__((always_inline)) {
+          int row = x_row[0];
+          if constexpr (MODE == kRowsShared) row = (int)slot0 + min(t0 + t, n_live - 1);
+          else if constexpr (NT > 1) row = t ? x_row[NT - 1] : row;
+          return a.x + (size_t)row * a.K + sb * kSbElems;
+        };
+        auto e_of = [&](int t, int l) __attribute__((always_inline)) {
+          if constexpr (kScale == kWhole) return e_now[t];
+          else return x.template scale<kSbScaleBytes>(t, l);
+        };
+        sb_dot<QUANT, kScale, NT, TAIL>(
+            raw, [&](int s, int l, int tg) { return ax[4 * l + s][tg]; },
+            [&](int s, int l, int tg) { return az[kSwapped ? 4 * l + s : s][tg]; }, e_of, x_of, v, live_lanes,
+            TAIL && half == 1 && (sb * kSbElems + 128) >= a.K);
+#pragma unroll
+        for (int m = 0; m < kRounds * MT; ++m) {  // (the sums stay in registers: the tile's own by a uniform branch, not by an index)
+          if (kRounds * MT > 1 && m != now.round * MT + i) continue;
+          if (kRounds * MT > 1) asm volatile("");
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[m / MT][m % MT][t] += v[t];
+        }
+        if (next.i == 0) buf ^= 1;
+        now = next;
       }
     }
 
     // ---- classes meet in LDS (over the slots, which everyone is done with)
     __syncthreads();
-    float* const red = reinterpret_cast<float*>(s_rows + kRowsZeros);  // [class][tile of the workgroup][token][64]
+    float* const red = reinterpret_cast<float*>(s_rows + kZeroBytes);  // [class][tile of the workgroup][token][64]
     const int span = MT * per_class;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      if (i >= n_mine) continue;
+    for (int r = 0; r < kRounds; ++r) {
+      if (r >= rounds) continue;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) red[(((size_t)cls * span + sub + per_class * i) * NT + t) * 64 + lane] = acc[i][t];
+      for (int i = 0; i < MT; ++i) {
+        if (i >= n_mine) continue;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) red[(((size_t)(cls + r * side) * span + sub + per_class * i) * kTokens + t0 + t) * 64 + lane] = acc[r][i][t];
+      }
     }
     __syncthreads();
     const int live_classes = min(classes, nsb);
@@ -241,16 +287,16 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       float h[2];
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const float* p = red + ((size_t)tl * NT + t) * 64 + 32 * q + col;
+        const float* p = red + ((size_t)tl * kTokens + t) * 64 + 32 * q + col;
         float v = p[0];
-        for (int c = 1; c < live_classes; ++c) v += p[(size_t)c * span * NT * 64];
+        for (int c = 1; c < live_classes; ++c) v += p[(size_t)c * span * kTokens * 64];
         h[q] = v;
       }
       return h[0] + h[1];
     };
     constexpr int kCols = NM == 2 ? 16 : 32;
-    for (int i = threadIdx.x; i < n_wg * NT * kCols; i += 512) {
-      const int col = i % kCols, t = i / kCols % NT, tl = i / (kCols * NT);
+    for (int i = threadIdx.x; i < n_wg * kTokens * kCols; i += 512) {
+      const int col = i % kCols, t = i / kCols % kTokens, tl = i / (kCols * kTokens);
       const int row = (tile_lo + tl) * tile_rows + col;
       const bool live = t < n_live && col < tile_rows && row < a.n_rows;
       size_t o_row = 0;
@@ -271,9 +317,9 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       }
       if constexpr (NM == 2) {
         const float v = silu_f(total(tl, t, col)) * total(tl, t, col + 16);
-        if (live && a.out) a.out[o_row * a.n_rows + row] = v;
+        if (live) a.out[o_row * a.n_rows + row] = v;
         // sixteen consecutive threads hold one group of the next contraction's activations
-        store_digit_group(v, row, a.out_nsb, a.out_d + o_row * a.out_nsb * kSbDigitBytes, a.out_e + o_row * a.out_nsb * 16, live);
+        store_digit_group(v, row, a.out_d + o_row * a.out_nsb * kSbDigitBytes, a.out_e + o_row * a.out_nsb * 16, live);
       } else {
         const float v = scale * total(tl, t, col);
         if (live) {
@@ -282,50 +328,50 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
         }
       }
     }
-    if (first + NT < n_tok) __syncthreads();  // (before the next chunk's requests land in the slots)
+    if (first + kTokens < n_tok) __syncthreads();  // (before the next chunk's requests land in the slots)
   }
 }
 
 // ------------------------------------------------------------------ host side
-template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+template <int MODE, int QUANT, int NM, int NT, int TEAMS, int MT, bool TAIL>
 static size_t rows_lds() {
-  const size_t slots = (size_t)8 * RowsLds<MODE, QUANT, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * 64 * sizeof(float);
-  return kRowsZeros + std::max(slots, red);
+  const size_t slots = (size_t)8 * RowsLds<MODE, QUANT, NM, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * TEAMS * 64 * sizeof(float);
+  return kZeroBytes + std::max(slots, red);
 }
 
-template <int MODE, int QUANT, int NM, int NT, int MT, bool TAIL>
+template <int MODE, int QUANT, int NM, int NT, int TEAMS, int MT, bool TAIL>
 static int rows_go(dim3 grid, hipStream_t s, const RowsArgs* a) {
-  const size_t smem = rows_lds<MODE, QUANT, NM, NT, MT, TAIL>();
+  const size_t smem = rows_lds<MODE, QUANT, NM, NT, TEAMS, MT, TAIL>();
   if (!a) {  // (at handle creation: the LDS limit)
-    XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_rows<MODE, QUANT, NM, NT, MT, TAIL>),
+    XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_rows<MODE, QUANT, NM, NT, TEAMS, MT, TAIL>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     return XABE_OK;
   }
-  hipLaunchKernelGGL((k_digit_rows<MODE, QUANT, NM, NT, MT, TAIL>), grid, dim3(512), smem, s, *a);
+  hipLaunchKernelGGL((k_digit_rows<MODE, QUANT, NM, NT, TEAMS, MT, TAIL>), grid, dim3(512), smem, s, *a);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
 
-template <int MODE, int NM, int NT, int MT>
+template <int MODE, int NM, int NT, int TEAMS, int MT>
 static int rows_quant(int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
-  if (quant == XABE_QUANT_Q6K) return rows_go<MODE, kQ6K, NM, NT, MT, false>(grid, s, a);
-  return tail ? rows_go<MODE, kQ8_0, NM, NT, MT, true>(grid, s, a) : rows_go<MODE, kQ8_0, NM, NT, MT, false>(grid, s, a);
+  if (quant == XABE_QUANT_Q6K) return rows_go<MODE, kQ6K, NM, NT, TEAMS, MT, false>(grid, s, a);
+  return tail ? rows_go<MODE, kQ8_0, NM, NT, TEAMS, MT, true>(grid, s, a) : rows_go<MODE, kQ8_0, NM, NT, TEAMS, MT, false>(grid, s, a);
 }
 
 template <int NM, int MT>
 static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
   switch (nt) {
-    case 1: return rows_quant<kRowsShared, NM, 1, MT>(quant, tail, grid, s, a);
-    case 2: return rows_quant<kRowsShared, NM, 2, MT>(quant, tail, grid, s, a);
-    case 4: return rows_quant<kRowsShared, NM, 4, MT>(quant, tail, grid, s, a);
-    default: return rows_quant<kRowsShared, NM, 8, MT>(quant, tail, grid, s, a);
+    case 1: return rows_quant<kRowsShared, NM, 1, 1, MT>(quant, tail, grid, s, a);
+    case 2: return rows_quant<kRowsShared, NM, 2, 1, MT>(quant, tail, grid, s, a);
+    case 4: return rows_quant<kRowsShared, NM, 4, 1, MT>(quant, tail, grid, s, a);
+    default: return rows_quant<kRowsShared, NM, 4, 2, MT>(quant, tail, grid, s, a);
   }
 }
 
 template <int NM>
 static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
-  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
-  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, kRowsBlockTokens, kRowsRoutedTiles>(quant, tail, grid, s, a);
+  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
+  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, kRowsBlockTokens, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
   return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
 }
 
@@ -362,7 +408,6 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
   a.row_bytes = (uint32_t)((size_t)a.K / be * bb);
   a.out_nsb = (int)digit_superblocks((size_t)a.n_rows);
   a.classes = a.nsb >= 8 ? 8 : a.nsb > 4 ? 8 : a.nsb > 2 ? 4 : a.nsb;
-  const int per_class = 8 / a.classes;
   int nt = 1;
   if (mode == kRowsShared) {
     // tokens per pass over the weights: all of them up to eight, equal passes beyond
@@ -370,6 +415,7 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
     nt = each == 1 ? 1 : each == 2 ? 2 : each <= 4 ? 4 : 8;
     units = (t + nt - 1) / nt;
   }
+  const int per_class = std::max(1, (nt > 4 ? 4 : 8) / a.classes);  // (as the kernel has it: nt > 4 is two teams)
   a.tile_rows = nm == 2 ? 16 : 32;
   int mt = 1;
   const int tiles16 = (a.n_rows + a.tile_rows - 1) / a.tile_rows;

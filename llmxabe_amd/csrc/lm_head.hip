@@ -36,7 +36,6 @@ struct LmHeadArgs {
 // reaches), by the vector ALU beyond (eight: 120 us).  Eight wavefronts per CU: twelve and sixteen measured slower.
 // SEG: rows whose digits do not fit in LDS are staged seg_sb superblocks at a time, again for every tile.
 constexpr size_t kHeadLdsMax = 160 * 1024;
-constexpr size_t kHeadZeros = 1024;
 constexpr size_t kHeadQuantTokens = 8;  // tokens per pass over a quantized matrix
 
 template <int QUANT, int NT, bool SEG>
@@ -47,7 +46,7 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
   const int waves = (int)(blockDim.x >> 6);
   const int nsb = a.K / kSbElems, seg_sb = SEG ? a.seg_sb : nsb;
   uint8_t* const s_zero = s_head;
-  uint8_t* const s_x = s_zero + kHeadZeros;                             // [superblock][token][kSbLdsBytes]
+  uint8_t* const s_x = s_zero + kZeroBytes;                             // [superblock][token][kSbLdsBytes]
   uint8_t* const slot = s_x + (size_t)seg_sb * NT * kSbLdsBytes + (size_t)wave * Dma::kSlotBytes;
   const uint32_t slot_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot;
   const uint32_t row_bytes = (uint32_t)nsb * SbRaw<QUANT>::kBytes;
@@ -66,13 +65,9 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
         const float4 f = src[j];
         x[4 * j] = f.x, x[4 * j + 1] = f.y, x[4 * j + 2] = f.z, x[4 * j + 3] = f.w;
       }
-      v4u_t plane[4];
-      float scale;
-      digitize16(x, plane, scale);
       uint8_t* base = s_x + (size_t)(sb * NT + t) * kSbLdsBytes;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) *reinterpret_cast<v4u_t*>(base + digit_group_offset(pos) + 16 * p) = plane[p];
-      reinterpret_cast<float*>(base + kSbDigitBytes)[scale_group_index(pos)] = scale;
+      const float scale = digitize_superblock(x, pos, base);  // (a superblock's groups: sixteen consecutive threads)
+      if (pos == 0) *reinterpret_cast<float*>(base + kSbDigitBytes) = scale;
     }
   };
 
@@ -95,7 +90,7 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
     take_tile(0);
     request(0);
   }
-  for (int i = threadIdx.x; i < (int)kHeadZeros / 16; i += (int)blockDim.x) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
+  for (int i = threadIdx.x; i < kZeroBytes / 16; i += (int)blockDim.x) reinterpret_cast<v4u_t*>(s_zero)[i] = v4u_t{0, 0, 0, 0};
   if constexpr (!SEG) {
     stage(0);
     __syncthreads();
@@ -132,12 +127,15 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
         take_tile(i + 1);
         request(0);
       }
-      LdsDigits<NT, kSbLdsBytes> x;
+      LdsDigits<NT, kSbLdsBytes, QUANT == kQ8_0> x;
       const uint8_t* sb_x = s_x + (size_t)(SEG ? sb % seg_sb : sb) * NT * kSbLdsBytes;
       x.point(sb_x, sb_x + kSbDigitBytes, s_zero);
       float v[NT];
-      sb_dot<QUANT, NT>(raw, [&](int s, int l, int tg) { return x.digit(s, l, tg); },
-                        [&](int t, int l) { return x.template scale<kSbLdsBytes>(t, l); }, v);
+      sb_dot<QUANT, kWhole, NT>(
+          raw, [&](int s, int l, int tg) { return x.high(s, l, tg); }, [&](int s, int l, int tg) { return x.low(s, l, tg); },
+          [&](int t, int) { return *reinterpret_cast<const float*>(sb_x + t * kSbLdsBytes + kSbDigitBytes); },
+          [&](int t) { return a.x + (size_t)(a.t0 + min(t, a.nt - 1)) * a.K + sb * kSbElems; }, v,
+          __builtin_amdgcn_ballot_w64(my_row < row_hi));
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[t] += v[t];
     }
@@ -471,36 +469,38 @@ static int launch_quant(unsigned grid, unsigned waves, size_t smem, hipStream_t 
   return XABE_OK;
 }
 
-// One pass of a.nt <= 8 tokens: as many wavefronts per workgroup, up to eight, as the digits leave LDS for.
+// Wavefronts of a workgroup in a pass of nt tokens: as many, up to eight, as the digits leave LDS for (0: not even one).
+template <int QUANT>
+static size_t head_waves(size_t K, size_t nt) {
+  const size_t room = kHeadLdsMax - kZeroBytes, digits = K / kSbElems * nt * kSbLdsBytes;
+  return digits > room ? 0 : std::min<size_t>(8, (room - digits) / SliceDma<QUANT>::kSlotBytes);
+}
+// Tokens of one pass over the matrix: as many as leave room for four wavefronts, or one.
+template <int QUANT>
+static size_t head_tokens(size_t K) {
+  size_t nt = kHeadQuantTokens;
+  while (nt > 1 && head_waves<QUANT>(K, nt) < 4) --nt;
+  return nt;
+}
+
 template <int QUANT>
 static int launch_quant_pass(const xabe_lm_head* h, hipStream_t s, LmHeadArgs a) {
   constexpr size_t kSlot = SliceDma<QUANT>::kSlotBytes;
-  const size_t nsb = (size_t)a.K / kSbElems;
-  const size_t digits = nsb * a.nt * kSbLdsBytes;
-  const size_t room = kHeadLdsMax - kHeadZeros;
-  const bool seg = digits + kSlot > room;
-  a.seg_sb = seg ? (int)((room - kSlot) / kSbLdsBytes) : (int)nsb;
-  const size_t waves = seg ? 1 : std::min<size_t>(8, (room - digits) / kSlot);
-  const size_t smem = kHeadZeros + (seg ? (size_t)a.seg_sb * kSbLdsBytes : digits) + waves * kSlot;
-  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(h->num_cus, ((size_t)a.vocab + 32 * waves - 1) / (32 * waves)));
-  if (seg) {  // rows of more than 35 000 elements: one token at a time
-    const int n = a.nt, t0 = a.t0;
-    for (int t = 0; t < n; ++t) {
-      a.t0 = t0 + t;
-      a.nt = 1;
-      XABE_TRY((launch_quant<QUANT, 1, true>(grid, 1, smem, s, a)));
-    }
-    return XABE_OK;
-  }
+  const size_t fit = head_waves<QUANT>(a.K, a.nt), waves = std::max<size_t>(1, fit);
+  // one workgroup per CU, and no more than there are tiles for
+  const unsigned w = (unsigned)waves, grid = (unsigned)std::max<size_t>(1, std::min<size_t>(h->num_cus, ((size_t)a.vocab + 32 * waves - 1) / (32 * waves)));
+  a.seg_sb = fit ? a.K / kSbElems : (int)((kHeadLdsMax - kZeroBytes - kSlot) / kSbLdsBytes);
+  const size_t smem = kZeroBytes + (size_t)a.seg_sb * a.nt * kSbLdsBytes + waves * kSlot;
+  if (!fit) return launch_quant<QUANT, 1, true>(grid, 1, smem, s, a);  // (rows of more than 24 000 elements, one token)
   switch (a.nt) {
-    case 1: return launch_quant<QUANT, 1, false>(grid, (unsigned)waves, smem, s, a);
-    case 2: return launch_quant<QUANT, 2, false>(grid, (unsigned)waves, smem, s, a);
-    case 3: return launch_quant<QUANT, 3, false>(grid, (unsigned)waves, smem, s, a);
-    case 4: return launch_quant<QUANT, 4, false>(grid, (unsigned)waves, smem, s, a);
-    case 5: return launch_quant<QUANT, 5, false>(grid, (unsigned)waves, smem, s, a);
-    case 6: return launch_quant<QUANT, 6, false>(grid, (unsigned)waves, smem, s, a);
-    case 7: return launch_quant<QUANT, 7, false>(grid, (unsigned)waves, smem, s, a);
-    default: return launch_quant<QUANT, 8, false>(grid, (unsigned)waves, smem, s, a);
+    case 1: return launch_quant<QUANT, 1, false>(grid, w, smem, s, a);
+    case 2: return launch_quant<QUANT, 2, false>(grid, w, smem, s, a);
+    case 3: return launch_quant<QUANT, 3, false>(grid, w, smem, s, a);
+    case 4: return launch_quant<QUANT, 4, false>(grid, w, smem, s, a);
+    case 5: return launch_quant<QUANT, 5, false>(grid, w, smem, s, a);
+    case 6: return launch_quant<QUANT, 6, false>(grid, w, smem, s, a);
+    case 7: return launch_quant<QUANT, 7, false>(grid, w, smem, s, a);
+    default: return launch_quant<QUANT, 8, false>(grid, w, smem, s, a);
   }
 }
 
@@ -559,7 +559,8 @@ int xabe_lm_head_forward(const xabe_lm_head* h, void* stream, int format, const 
   a.seg_sb = 0;
   const bool quant = format == XABE_HEAD_Q8_0 || format == XABE_HEAD_Q6K;
   // passes of equal width: nine tokens as five and four, not as eight and one
-  const size_t most = quant ? xabe::kHeadQuantTokens : XABE_LM_HEAD_MAX_BATCH_TILE;
+  const size_t most = !quant ? XABE_LM_HEAD_MAX_BATCH_TILE
+                    : format == XABE_HEAD_Q8_0 ? xabe::head_tokens<xabe::kQ8_0>(g.hidden) : xabe::head_tokens<xabe::kQ6K>(g.hidden);
   const size_t passes = (tokens + most - 1) / most, width = (tokens + passes - 1) / passes;
   for (size_t base = 0; base < tokens; base += width) {
     const int tile = (int)std::min<size_t>(width, tokens - base);

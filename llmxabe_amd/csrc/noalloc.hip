@@ -37,7 +37,8 @@ constexpr size_t kNaSharedInter = kNaLogits + na_align(kNaMaxTokens * kNaMaxExpe
 constexpr size_t kNaInterSb = kNaMaxTokens * kNaMaxTopK * (kNaMaxInter / kSbElems), kNaXSb = kNaMaxTokens * (kNaMaxHidden / kSbElems);
 constexpr size_t kNaInterD = kNaSharedInter + na_align(kNaMaxTokens * kNaMaxInter);
 constexpr size_t kNaInterE = kNaInterD + na_align(kNaInterSb * kSbDigitBytes / 4);
-constexpr size_t kNaXD = kNaInterE + na_align(kNaInterSb * kSbScaleBytes / 4);
+constexpr size_t kNaInter = kNaInterE + na_align(kNaInterSb * kSbScaleBytes / 4);       // [tokens * top_k][intermediate]
+constexpr size_t kNaXD = kNaInter + na_align(kNaInterSb * kSbElems);
 constexpr size_t kNaXE = kNaXD + na_align(kNaXSb * kSbDigitBytes / 4);
 constexpr size_t kNaNormed = kNaXE + na_align(kNaXSb * kSbScaleBytes / 4);             // [tokens][hidden]
 constexpr size_t kNaRouted = kNaNormed + na_align(kNaMaxTokens * kNaMaxHidden);
@@ -122,6 +123,7 @@ int xabe_moe_block_forward_noalloc(const xabe_moe_geometry* geometry, float eps,
   b.topk_weights = base + kNaTopkW;
   b.inter_d = reinterpret_cast<uint8_t*>(base + kNaInterD);
   b.inter_e = base + kNaInterE;
+  b.inter = base + kNaInter;
   b.x_d = reinterpret_cast<uint8_t*>(base + kNaXD);
   b.x_e = base + kNaXE;
   b.shared_inter = base + kNaSharedInter;

@@ -24,7 +24,7 @@ __device__ __forceinline__ float block_sum_256(float v, float* scratch) {
 // rms_norm_rows (crates/xabe-cuda/src/kernels/layer_ops.rs:129-151): every row of the
 // buffer, y = x * (1/sqrtf(mean(x^2) + eps)) * w.  grid = rows, 256 threads.
 // ---------------------------------------------------------------------------------
-// DIGITS: the row also goes out as the digits and group scales the fp32 row contractions read (digits.h).
+// DIGITS: the row also goes out as the digits and superblock scales the fp32 row contractions read (digits.h).
 template <bool DIGITS>
 __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__ x, const float* __restrict__ w,
                                                         float* __restrict__ out, int width, float eps,
@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__
   if constexpr (DIGITS) {  // (the same products from the row's cached pieces, sixteen consecutive elements per thread)
     const int nsb = (width + kSbElems - 1) / kSbElems;
     uint8_t* d = xd + (size_t)blockIdx.x * nsb * kSbDigitBytes;
-    float* e = xe + (size_t)blockIdx.x * nsb * 16;
+    float* e = xe + (size_t)blockIdx.x * nsb;
     for (int gi = threadIdx.x; gi < nsb * 16; gi += 256) {
       float v[16];
 #pragma unroll
