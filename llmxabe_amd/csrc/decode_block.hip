@@ -377,8 +377,10 @@ __device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) 
 // steps of RPSI rows each, two tokens per pass, on the lanes' fp32 sums of the separate kernels.  (At fewer tokens a
 // wavefront of the third launch does it: here, on a few CUs only, its uncoalesced loads were the launch's last to end,
 // 13.5 against 9.3 us for one token.)
-template <int RQ, int SQ, int NP, int RPSI, bool ROUTED>
-__global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
+// DIRECT (one tile per workgroup, one workgroup per CU): the rows go straight into registers; there is no next tile whose
+// bytes the slot would receive meanwhile, and the way through LDS is a trip that everything after it waits for.
+template <int RQ, int SQ, int NP, int RPSI, bool ROUTED, bool DIRECT>
+__global__ void __launch_bounds__(128 * NP, DIRECT ? 2 : 4) k_decode_up(DecodeArgs a) {
   using Dma = PairDma<RQ>;
   constexpr int kWaves = 2 * NP;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_up[];  // a weight slot per wavefront, then the routing's num_experts floats
@@ -424,7 +426,7 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
   PairDigits<kWhole> x;
   x.load(a.x_d + x_sb * kSbDigitBytes, a.x_e + x_sb);
   Dma dma;  // (its lane offsets are ready before the expert is known)
-  dma.init(row_bytes, sb0);
+  if constexpr (!DIRECT) dma.init(row_bytes, sb0);
   if (t >= valid) return;
   // Routing in two halves (route_device.h).  The first orders the experts by logit: its k-th candidate is
   // the pair's expert unless probabilities tie, and it is known ~2 us before the softmax is, so the
@@ -453,7 +455,11 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
   auto stream_rows = [&](int e, auto finish_c) __attribute__((always_inline)) {
     const size_t e_off = (size_t)e * a.expert_bytes;
     auto run_off = [&](int i) __attribute__((always_inline)) { return e_off + (size_t)(16 * (share * a.share_g + i)) * row_bytes; };
-    dma.request(mat ? a.up : a.gate, a.up_len, run_off(0), slot_lds);
+    SbRaw<RQ> raw;
+    if constexpr (DIRECT)
+      sb_read((mat ? a.up : a.gate) + run_off(0) + (size_t)(lane & 15) * row_bytes + sb * SbRaw<RQ>::kBytes, quarter & 1, raw);
+    else
+      dma.request(mat ? a.up : a.gate, a.up_len, run_off(0), slot_lds);
     if constexpr (decltype(finish_c)::value) {
       if (routes) {  // (raised priority keeps it ahead of its neighbours' arithmetic)
         __builtin_amdgcn_s_setprio(3);
@@ -473,12 +479,13 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up(DecodeArgs a) {
       }
     }
 #pragma unroll 1
-    for (int i = 0; i < a.share_g; ++i) {
-      wait_loads();
-      SbRaw<RQ> raw;
-      sb_read(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), slot_lds);
+    for (int i = 0; i < (DIRECT ? 1 : a.share_g); ++i) {
+      if constexpr (!DIRECT) {
+        wait_loads();
+        sb_read(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), slot_lds);
+      }
       s_red[i][sb][(quarter & 1) * 32 + mat * 16 + (lane & 15)] = pair_dot<RQ>(
           raw, x, [&](int q) __attribute__((always_inline)) { return a.normed + (size_t)t * a.H + (sb0 + (q >> 1)) * kSbElems; });
     }
@@ -577,9 +584,13 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
     }
   } else {
     const int p = t * a.top_k + wave;
-    const int e = __builtin_amdgcn_readfirstlane(min(max(a.topk_ids[p], 0), a.E - 1));
+    const int id = a.topk_ids[p];
     const float sel_w = a.topk_weights[p];
     constexpr int nsb = kPairRows == 1 ? 2 : 1;
+    const size_t x_sb = (size_t)p * nsb + (kPairRows == 1 ? quarter >> 1 : 0);
+    PairDigits<kGroups> x;  // (requested with the expert's index, not after it)
+    x.load(a.inter_d + x_sb * kSbDigitBytes, a.inter_e + x_sb * 16);
+    const int e = __builtin_amdgcn_readfirstlane(min(max(id, 0), a.E - 1));
     const uint32_t pair_bytes = 2 * SbRaw<RQ>::kBytes;
     uint8_t* const slot = s_down + wave * Dma::kSlotBytes;
     const uint32_t slot_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)slot);
@@ -588,9 +599,6 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
     Dma dma;
     dma.init();
     dma.request(run(0), slot_lds);
-    const size_t x_sb = (size_t)p * nsb + (kPairRows == 1 ? quarter >> 1 : 0);
-    PairDigits<kGroups> x;
-    x.load(a.inter_d + x_sb * kSbDigitBytes, a.inter_e + x_sb * 16);
 #pragma unroll 1
     for (int i = 0; i < a.share_d; ++i) {
       wait_loads();
@@ -752,8 +760,9 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
     }
 #define XABE_B(RQ, SQ)                                                                                            \
   do {                                                                                                            \
-    if (l.pre_routed) hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, true>), grid, block, lds, l.s, l.a);       \
-    else hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, false>), grid, block, lds, l.s, l.a);                   \
+    if (l.pre_routed) hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, true, false>), grid, block, lds, l.s, l.a); \
+    else if (l.a.share_g == 1) hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, false, true>), grid, block, lds, l.s, l.a); \
+    else hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, false, false>), grid, block, lds, l.s, l.a);            \
   } while (0)
     if (g6 && sd6) XABE_B(kQ6K, kQ6K);
     else if (g6) XABE_B(kQ6K, kQ8_0);
@@ -779,9 +788,10 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
 static int decode_block_set_limits() {
 #define XABE_LDS(kernel, bytes) \
   XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes)))
-#define XABE_UP(Q, code, SQ, NP, RPSI)                                                       \
-  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, false>), up_lds<NP>(code, (int)kRouteMaxExperts)); \
-  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, true>), up_lds<NP>(code, (int)kRouteMaxExperts))
+#define XABE_UP(Q, code, SQ, NP, RPSI)                                                              \
+  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, false, false>), up_lds<NP>(code, (int)kRouteMaxExperts)); \
+  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, false, true>), up_lds<NP>(code, (int)kRouteMaxExperts));  \
+  XABE_LDS((k_decode_up<Q, SQ, NP, RPSI, true, false>), up_lds<NP>(code, (int)kRouteMaxExperts))
 #define XABE_DOWN(Q, code)                                          \
   XABE_LDS((k_decode_down<Q, kQ8_0, 1, false>), down_lds(code, kMaxTopK));  \
   XABE_LDS((k_decode_down<Q, kQ8_0, 2, false>), down_lds(code, kMaxTopK));  \
@@ -789,9 +799,9 @@ static int decode_block_set_limits() {
   XABE_LDS((k_decode_down<Q, kQ6K, 2, true>), down_lds(code, kMaxTopK));    \
   XABE_LDS((k_decode_down<Q, kQ8_0, 1, true>), down_lds(code, kMaxTopK));   \
   XABE_LDS((k_decode_down<Q, kQ8_0, 2, true>), down_lds(code, kMaxTopK));   \
-  XABE_UP(Q, code, kQ6K, 4, 4);                                     \
-  XABE_UP(Q, code, kQ8_0, 4, 4);                                    \
-  XABE_UP(Q, code, kQ6K, 1, 8);                                     \
+  XABE_UP(Q, code, kQ6K, 4, 4);                                              \
+  XABE_UP(Q, code, kQ8_0, 4, 4);                                             \
+  XABE_UP(Q, code, kQ6K, 1, 8);                                              \
   XABE_UP(Q, code, kQ8_0, 1, 8)
   XABE_DOWN(kQ6K, XABE_QUANT_Q6K);
   XABE_DOWN(kQ8_0, XABE_QUANT_Q8_0);
