@@ -607,6 +607,25 @@ static int check_routed_stacks(const xabe_moe_kernels* k, xabe_quant_tensor gate
   return XABE_OK;
 }
 
+// The shared expert's two contractions on the lanes' fp32 sums.
+static void shared_up_args(ExpertArgs& a, const xabe_moe_kernels* k, const xabe_moe_buffers* b, xabe_quant_tensor gate,
+                           xabe_quant_tensor up, const float* x) {
+  a.w0 = static_cast<const uint8_t*>(gate.bytes);
+  a.w1 = static_cast<const uint8_t*>(up.bytes);
+  a.x = x;
+  a.out = b->shared_inter;
+  a.K = (int)k->g.hidden;
+  a.n_rows = (int)k->g.intermediate;
+}
+static void shared_down_args(ExpertArgs& a, const xabe_moe_kernels* k, const xabe_moe_buffers* b, xabe_quant_tensor down, float* out) {
+  a.w0 = static_cast<const uint8_t*>(down.bytes);
+  a.w1 = nullptr;
+  a.x = b->shared_inter;
+  a.out = out;
+  a.K = (int)k->g.intermediate;
+  a.n_rows = (int)k->g.hidden;
+}
+
 static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
   RowsArgs a;
   memset(&a, 0, sizeof(a));
@@ -620,42 +639,74 @@ static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) 
   return a;
 }
 
-// stages: bit 0 = gate/up + SwiGLU (from the digits of x), bit 1 = down
+// One (token, k) pair per unit below the matrix-core widths (most dispatch blocks hold one or two tokens there, and the
+// pair kernel runs twice as many workgroups) and in the exact regime; dispatch blocks at wider passes.  Microseconds of
+// the routed experts of the model (256 experts, top 8), pairs / blocks: 5 tokens 38 / 51, 13: 71 / 84, 32: 130 / 160, 45:
+// 171 / 213, 63: 224 / 268; 64 experts, top 4, hidden 1024: 13 tokens 26 / 56, 45: 51 / 80.  force_community keeps the
+// blocks, where there are any, for comparison: same bits.
+static bool routed_by_pairs(const xabe_moe_kernels* k) {
+  return flat_regime(k) || (k->g.max_tokens < kMfmaMinTokens && !k->force_community);
+}
+
+// The shared expert's tensors and rows, for launches that take its row tiles along (x: the routed experts' own rows).
+struct SharedRide {
+  xabe_quant_tensor gate, up, down;
+  float* out;
+};
+
+// stages: bit 0 = gate/up + SwiGLU, bit 1 = down
 static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, int stages = 3) {
+                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, int stages = 3,
+                       const SharedRide* ride = nullptr) {
   const xabe_moe_geometry& g = k->g;
-  const int mode = flat_regime(k) ? kRowsFlat : kRowsBlock;
-  const size_t units = mode == kRowsFlat ? xabe_moe_geometry_max_flat_pairs(&g) : b->n_expert_blocks;
+  const bool pairs = routed_by_pairs(k);
+  const size_t units = pairs ? xabe_moe_geometry_max_flat_pairs(&g) : b->n_expert_blocks;
+  if (units > 65535) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "%zu work units exceed the 65535 grid.y limit of the fp32 regime", units);
   const size_t expert_elems = g.intermediate * g.hidden;
-  RowsArgs a = rows_args(k, b);
+  RowsArgs up_a = rows_args(k, b);
+  up_a.w0 = static_cast<const uint8_t*>(gate.bytes);
+  up_a.w1 = static_cast<const uint8_t*>(up.bytes);
+  up_a.w_bytes = gate.len;
+  up_a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
+  up_a.x = x;
+  up_a.xd = b->x_d;
+  up_a.xe = b->x_e;
+  up_a.out = b->inter;
+  up_a.out_d = b->inter_d;
+  up_a.out_e = b->inter_e;
+  up_a.K = (int)g.hidden;
+  up_a.n_rows = (int)g.intermediate;
+  RowsArgs down_a = rows_args(k, b);
+  down_a.w0 = static_cast<const uint8_t*>(down.bytes);
+  down_a.w_bytes = down.len;
+  down_a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(down.quant) * xabe_expert_quant_block_bytes(down.quant);
+  down_a.x = b->inter;
+  down_a.xd = b->inter_d;
+  down_a.xe = b->inter_e;
+  down_a.out = b->partial;
+  down_a.K = (int)g.intermediate;
+  down_a.n_rows = (int)g.hidden;
+  if (pairs) {
+    ExpertArgs sh_up = base_args(k, b), sh_down = sh_up;
+    if (ride) {
+      shared_up_args(sh_up, k, b, ride->gate, ride->up, x);
+      shared_down_args(sh_down, k, b, ride->down, ride->out);
+    }
+    // (4096 pairs a launch: at the widths of the exact regime a grid may not hold more)
+    constexpr size_t kPairsPerLaunch = 4096;
+    for (size_t first = 0; first < units; first += kPairsPerLaunch) {
+      const size_t n = std::min(kPairsPerLaunch, units - first);
+      up_a.unit0 = down_a.unit0 = (int)first;
+      if (stages & 1) XABE_TRY(launch_digit_pairs(k, gate.quant, 2, up_a, n, s, ride ? &sh_up : nullptr, ride ? ride->gate.quant : -1));
+      if (stages & 2) XABE_TRY(launch_digit_pairs(k, down.quant, 1, down_a, n, s, ride ? &sh_down : nullptr, ride ? ride->down.quant : -1));
+    }
+    return XABE_OK;
+  }
   if (stages & 1) {
     XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->x_d, b->x_e));
-    a.w0 = static_cast<const uint8_t*>(gate.bytes);
-    a.w1 = static_cast<const uint8_t*>(up.bytes);
-    a.w_bytes = gate.len;
-    a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
-    a.x = x;
-    a.xd = b->x_d;
-    a.xe = b->x_e;
-    a.out = b->inter;
-    a.out_d = b->inter_d;
-    a.out_e = b->inter_e;
-    a.K = (int)g.hidden;
-    a.n_rows = (int)g.intermediate;
-    XABE_TRY(launch_digit_rows(k, mode, gate.quant, 2, a, units, s));
+    XABE_TRY(launch_digit_rows(k, kRowsBlock, gate.quant, 2, up_a, units, s));
   }
-  if (!(stages & 2)) return XABE_OK;
-  a.w0 = static_cast<const uint8_t*>(down.bytes);
-  a.w1 = nullptr;
-  a.w_bytes = down.len;
-  a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(down.quant) * xabe_expert_quant_block_bytes(down.quant);
-  a.x = b->inter;
-  a.xd = b->inter_d;
-  a.xe = b->inter_e;
-  a.out = b->partial;
-  a.K = (int)g.intermediate;
-  a.n_rows = (int)g.hidden;
-  return launch_digit_rows(k, mode, down.quant, 1, a, units, s);
+  return stages & 2 ? launch_digit_rows(k, kRowsBlock, down.quant, 1, down_a, units, s) : XABE_OK;
 }
 
 int xabe_moe_grouped_forward_partial(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, xabe_quant_tensor gate,
@@ -749,22 +800,10 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   }
   const size_t units = (g.max_tokens + 1) / 2;
   ExpertArgs a = base_args(k, b);
-  a.w0 = static_cast<const uint8_t*>(gate.bytes);
-  a.w1 = static_cast<const uint8_t*>(up.bytes);
-  a.expert_bytes = 0;
-  a.x = x;
-  a.out = b->shared_inter;
-  a.K = (int)g.hidden;
-  a.n_rows = (int)g.intermediate;
+  shared_up_args(a, k, b, gate, up, x);
   XABE_TRY(launch_expert(k, gate.quant, 2, a, units, s));
-  a.w0 = static_cast<const uint8_t*>(down.bytes);
-  a.w1 = nullptr;
-  a.x = b->shared_inter;
-  a.out = out;
-  a.K = (int)g.intermediate;
-  a.n_rows = (int)g.hidden;
-  XABE_TRY(launch_expert(k, down.quant, 1, a, units, s));
-  return XABE_OK;
+  shared_down_args(a, k, b, down, out);
+  return launch_expert(k, down.quant, 1, a, units, s);
 }
 
 // The dense block's fp32 path: the norm launch writes the digits, down adds the residual; three launches.
@@ -831,8 +870,14 @@ int xabe_moe_grouped_forward_partial_with_shared(const xabe_moe_kernels* k, void
   XABE_TRY(check_shared_stacks(k, shared_gate, shared_up, shared_down));
   XABE_TRY(check_len("hidden_states", g.max_tokens * g.hidden, hidden_states_len));
   XABE_TRY(check_len("out", g.max_tokens * g.hidden, out_len));
-  XABE_TRY(routed_fp32(k, as_stream(stream), b, gate, up, down, hidden_states));
-  XABE_TRY(shared_fp32(k, as_stream(stream), b, shared_gate, shared_up, shared_down, hidden_states, out));
+  // rows the lanes' sums take in one step, in the launches of the routed experts; others in launches of their own
+  if (g.hidden <= 2048 && g.hidden % 256 == 0 && g.intermediate <= 2048 && g.intermediate % 256 == 0) {
+    const SharedRide ride = {shared_gate, shared_up, shared_down, out};
+    XABE_TRY(routed_fp32(k, as_stream(stream), b, gate, up, down, hidden_states, 3, &ride));
+  } else {
+    XABE_TRY(routed_fp32(k, as_stream(stream), b, gate, up, down, hidden_states));
+    XABE_TRY(shared_fp32(k, as_stream(stream), b, shared_gate, shared_up, shared_down, hidden_states, out));
+  }
   *fused = 1;
   return XABE_OK;
 }

@@ -205,7 +205,7 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
   constexpr int G = 64 / RPS;
   static_assert(RPS == 1 || KS == 1, "short rows take exactly one step");
   const LaneGeom g = lane_geom<QUANT>();
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % kWavesPerWg;  // (four take a tile, however many there are)
   const size_t row_bytes = (size_t)(K / F::kBlockElems) * F::kBlockBytes;
   const int tile_end = min(tile0 + tile_rows, n_rows);
 

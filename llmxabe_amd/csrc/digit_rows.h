@@ -7,7 +7,8 @@ struct xabe_moe_kernels;
 
 namespace xabe {
 
-constexpr int kRowsFlat = 0;    // one (token, k) pair per unit, straight from topk_ids
+struct ExpertArgs;
+
 constexpr int kRowsBlock = 1;   // one dispatch block per unit: one expert, its run of tokens
 constexpr int kRowsShared = 2;  // every live token, one matrix
 constexpr int kRowsMaxTiles = 5;  // tiles of one wavefront's share whose sums it keeps in registers
@@ -20,7 +21,7 @@ struct RowsArgs {
   size_t w_bytes;            // length of each stack
   size_t expert_bytes;       // bytes of one expert in a stack (0: a single matrix)
   const float* x;            // the activation rows, [row][K] (what a marked group goes back to)
-  const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes]
+  const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes] (pairs' gate/up makes its own)
   const float* xe;           // their scales: gate/up [row][superblock], down [row][superblock][16] (by group)
   float* out;                // [row][n_rows]
   uint8_t* out_d;            // nm = 2: digits of the output rows
@@ -33,8 +34,11 @@ struct RowsArgs {
   const int* sorted_token_ids;
   const int* expert_ids;
   int K, n_rows, top_k, block_size;
+  int unit0;  // pairs: the first of this launch
   // filled in by launch_digit_rows
   int nsb, out_nsb, classes, tile_rows, n_tiles;
+  int units, shares, xcd_units;  // pairs (xcd_units: units of one share side by side, one per XCD; 0: plain order)
+  int shared_wgs, shared_rps;      // pairs with the shared expert: its workgroups per chunk of two tokens, rows per step
   uint32_t row_bytes;
 };
 
@@ -79,7 +83,11 @@ __device__ __forceinline__ void store_digit_group(float v, int row, uint8_t* xd,
 // host side
 int digit_rows_configure();
 int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
-// `units`: pairs (flat) or dispatch blocks (block); token chunks are counted here
+// `units`: dispatch blocks (block); token chunks are counted here
 int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s);
+// One (token, k) pair per unit, straight from topk_ids: pairs a.unit0 .. a.unit0 + units - 1.  `shared`: the shared
+// expert's rows of the same shape (whole superblocks, at most 2048 elements) ride along.
+int launch_digit_pairs(const xabe_moe_kernels* k, int quant, int nm, RowsArgs a, size_t units, hipStream_t s,
+                       const ExpertArgs* shared = nullptr, int shared_quant = -1);
 
 }  // namespace xabe

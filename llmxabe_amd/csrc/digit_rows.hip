@@ -14,6 +14,7 @@
 
 #include <algorithm>
 
+#include "decode_kernels.h"
 #include "device_once.h"
 #include "digit_rows.h"
 #include "host_common.h"
@@ -35,8 +36,7 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
   store_digits16(v, gi, gi * 16 < K, xd + (size_t)row * nsb * kSbDigitBytes, xe + (size_t)row * nsb);
 }
 
-// Tiles per wavefront of a routed unit, the next one's rows in flight while one is multiplied.  (Routed units serve the
-// step-by-step entry points; the block goes through decode_block.hip.)
+// Tiles per wavefront of a dispatch block, the next one's rows in flight while one is multiplied.
 constexpr int kRowsRoutedTiles = 4;
 constexpr int kRowsBlockTokens = 2;  // tokens per chunk of a dispatch block (most hold one or two)
 
@@ -63,15 +63,10 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   const int valid = *a.valid_tokens;
   // ---- the unit's weights and token rows
   size_t e_off = 0;
-  int n_tok, pair = 0;
+  int n_tok;
   const int* slots = nullptr;
   size_t slot0 = 0;
-  if constexpr (MODE == kRowsFlat) {
-    pair = (int)blockIdx.y;
-    if (pair >= valid * a.top_k) return;
-    e_off = (size_t)a.topk_ids[pair] * a.expert_bytes;
-    n_tok = 1;
-  } else if constexpr (MODE == kRowsBlock) {
+  if constexpr (MODE == kRowsBlock) {
     const int e = a.expert_ids[blockIdx.y];
     if (e < 0) return;
     e_off = (size_t)e * a.expert_bytes;
@@ -135,10 +130,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   for (int first = 0; first < n_tok; first += kTokens) {
     // the chunk's tokens: activation rows (tokens past the live ones repeat one of them and are never stored)
     int x_row[NT], n_live = 0;
-    if constexpr (MODE == kRowsFlat) {
-      x_row[0] = NM == 2 ? pair / a.top_k : pair;
-      n_live = 1;
-    } else if constexpr (MODE == kRowsBlock) {
+    if constexpr (MODE == kRowsBlock) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int f = first + t < n_tok ? slots[first + t] : sentinel;
@@ -158,8 +150,8 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       if ((lane >> 2) == t) x_row_l = x_row[t];
     float e_now[NT], e_next[NT];  // (whole superblocks' scales)
     auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
-      // (routed units keep a superblock's digits for a whole share and their tokens are few: they come straight into
-      // registers below, and the LDS they would take makes room for a second workgroup on the CU)
+      // (dispatch blocks keep a superblock's digits for a whole share and their chunks are small: they come straight into
+      // registers below)
 #pragma unroll
       for (int t = 0; t < NT && MODE == kRowsShared; ++t) {
         const uint8_t* from = a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes;
@@ -216,7 +208,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
 #pragma unroll
               for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
           } else {
-            static_assert(MODE == kRowsShared || digits_in_one(NT), "routed units hold one or two tokens");
+            static_assert(MODE == kRowsShared || digits_in_one(NT), "chunks of a dispatch block are one or two tokens");
             const int at = high_digit_at<NT>(lane, 0, 0);
             const int row = NT > 1 && (lane & 16) ? x_row[NT - 1] : x_row[0];
             const uint8_t* d = a.xd + ((size_t)row * nsb + sb) * kSbDigitBytes + max(at, 0);
@@ -301,10 +293,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       const bool live = t < n_live && col < tile_rows && row < a.n_rows;
       size_t o_row = 0;
       float scale = 1.0f;
-      if constexpr (MODE == kRowsFlat) {
-        o_row = pair;
-        if (NM == 1) scale = a.topk_weights[pair];
-      } else if constexpr (MODE == kRowsBlock) {
+      if constexpr (MODE == kRowsBlock) {
         if (NM == 2) {
           o_row = slot0 + first + t;
         } else {
@@ -332,7 +321,240 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// Routed experts, one (token, k) pair per unit: what the step-by-step entry points run below the matrix-core widths (the
+// block as a whole goes through decode_block.hip, whose second and third launch have the same core) and the exact regime
+// at any width.
+//
+// Same classes, tiles and order of operations as above on the one-token core (pair_dot: four result registers where
+// sb_dot has sixteen, two workgroups on a CU), quarters 0, 1 of the wavefront on a tile's first sixteen rows and 2, 3 on
+// the others.  gate/up makes the digits of its activation superblocks itself, four elements per lane, in the weight slot
+// between a tile's bytes and the next one's: a launch of its own for them cost 4.7 us and its boundary.  Sums wait in LDS.
+// What bounds it: at a few tokens the chain of round trips of two launches; from 13 tokens on the vector instructions of
+// one unpacking per pair, and one expert read once per pair and XCD.  (k_digit_rows unpacks once per two tokens of a
+// dispatch block, but most blocks hold one, and its 170 registers leave one workgroup per CU.)
+// Routed experts of the model geometry, us: one token 31 -> 16, three 33 -> 26, 45 213 -> 171 (k_digit_rows -> this).
+// ------------------------------------------------------------------------------------------------
+constexpr int kPairTiles = 4;  // tiles a wavefront takes at most
+// From this width on the workgroups that read the same rows run side by side on one XCD (kXcdGroupMinTokens in
+// decode_block.hip says why).  Shares that do not divide evenly over the eight XCDs keep the plain order: padded to eight
+// they left half of the chip idle (four shares: 126 against 84 us for the down launch of 64 tokens).
+constexpr size_t kPairsXcdMinTokens = 24;
+
+// SliceDma's slot for tiles that start on 16-byte boundaries (sixteen rows of an expert are whole pieces, and so are the
+// rows before them): the lane's offsets are the same for every tile of a superblock and kept in units of pieces, two to a
+// register (rows of more than 64 KB: worked out again for every tile).
+template <int QUANT, int PIECES>
+struct TileDma {
+  static constexpr int kP = PIECES, kInstr = (16 * kP + 63) / 64, kLast = 16 * kP - 64 * (kInstr - 1);
+  static constexpr int kRunBytes = 16 * kP * 16, kSlotBytes = 2 * kRunBytes;
+  PackedOffsets<kInstr> off;
+  static __device__ __forceinline__ uint32_t piece(int i, uint32_t row_bytes, int sb) {
+    const uint32_t pc = min((uint32_t)(64 * i) + __lane_id(), 16u * kP - 1);
+    return ((pc / kP * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) >> 4) + pc % kP;
+  }
+  __device__ __forceinline__ void init(uint32_t row_bytes, int sb) {
+#pragma unroll
+    for (int i = 0; i < kInstr; ++i) off.set(i, piece(i, row_bytes, sb) & 0xffffu);
+  }
+  // pieces past the tensor's end (padding of the last rows' windows) repeat its last one
+  __device__ __forceinline__ void request(const uint8_t* w, size_t w_bytes, size_t tile, uint32_t row_bytes, int sb, uint32_t dst) {
+    const uint32_t last = (uint32_t)min(w_bytes - 16 - tile, (size_t)0xfffffff0u);
+    const bool fits = row_bytes <= 65535 - kP;  // (16 rows and a window are at most 65535 pieces)
+    off.opaque();
+#pragma unroll
+    for (int i = 0; i < kInstr; ++i) {
+      uint32_t o = off.get(i);
+      if (__builtin_expect(!fits, 0)) o = piece(i, row_bytes, sb);
+      if (i + 1 < kInstr || kLast == 64 || (int)__lane_id() < kLast) lds_dma_16(w + tile, min(o * 16, last), dst + i * 1024);
+    }
+  }
+  static __device__ __forceinline__ const uint8_t* row_at(const uint8_t* run_slot, uint32_t row_bytes, int row, int sb) {
+    return run_slot + row * (kP * 16) + (((uint32_t)row * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & 15u);
+  }
+};
+
+template <int QUANT, bool TAIL, bool DIRECT>
+struct PairRowsLds {
+  using Dma = TileDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
+  static constexpr int kTiles = DIRECT ? 1 : kPairTiles, kSlot = DIRECT ? kSbDigitBytes : Dma::kSlotBytes;
+  static constexpr size_t kSlots = 8 * (size_t)kSlot, kBytes = kSlots + (size_t)8 * kTiles * 64 * sizeof(float);
+};
+
+// DIRECT (one tile and one superblock per wavefront): its rows go straight into registers; there is no next tile whose
+// bytes a slot would receive meanwhile, and the digits of gate/up are made while they are on their way.
+// SQ >= 0: the workgroups past the pairs' are the shared expert's row tiles on the lanes' fp32 sums, two tiles of
+// k_expert_shared each (`sh`): at a few tokens a launch of their own is mostly its boundary.
+template <int QUANT, int NM, bool TAIL, bool DIRECT, int SQ>
+__global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a, ExpertArgs sh) {
+  using L = PairRowsLds<QUANT, TAIL, DIRECT>;
+  using Dma = typename L::Dma;
+  constexpr int kTiles = L::kTiles;
+  constexpr bool kScale = NM == 2 ? kWhole : kGroups;
+  constexpr int tile_rows = NM == 2 ? 16 : 32;
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_pair[];
+  const int lane = (int)__lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if constexpr (SQ >= 0) {
+    const int pair_wgs = a.units * a.shares;
+    if ((int)blockIdx.x >= pair_wgs) {
+      const int n = (int)blockIdx.x - pair_wgs, chunk = n / a.shared_wgs, tile = 2 * (n % a.shared_wgs) + (wave >> 2);
+      switch (a.shared_rps) {
+        case 8: shared_body<SQ, 1, 8, NM>(sh, chunk, tile); break;
+        case 4: shared_body<SQ, 1, 4, NM>(sh, chunk, tile); break;
+        case 2: shared_body<SQ, 1, 2, NM>(sh, chunk, tile); break;
+        default: shared_body<SQ, 1, 1, NM>(sh, chunk, tile); break;
+      }
+      return;
+    }
+  }
+  int u = (int)blockIdx.x / a.shares, share = (int)blockIdx.x % a.shares;
+  if (a.xcd_units) {  // one XCD's workgroups: one share at a time, all its units next to each other
+    const int xcd = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+    if (a.xcd_units == 1) {
+      share = xcd + 8 * (j / a.units);
+      u = j % a.units;
+    } else {
+      share = xcd % a.shares;
+      u = j * a.xcd_units + xcd / a.shares;
+      if (u >= a.units) return;
+    }
+  }
+  const int pair = a.unit0 + u;
+  const int id = a.topk_ids[pair];
+  const float weight = NM == 1 ? a.topk_weights[pair] : 1.0f;
+  const int classes = a.classes, per_class = 8 / classes;
+  const int cls = wave % classes, sub = wave / classes;
+  const int tile_lo = (int)((long long)a.n_tiles * share / a.shares);
+  const int n_wg = (int)((long long)a.n_tiles * (share + 1) / a.shares) - tile_lo;  // <= kTiles * per_class
+  const int n_mine = (n_wg - sub + per_class - 1) / per_class;
+  const int nsb = a.nsb;
+  const uint32_t row_bytes = a.row_bytes;
+  const bool any = cls < nsb && n_mine > 0;
+  uint8_t* const w_slot = s_pair + (size_t)wave * L::kSlot;
+  const uint32_t w_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)w_slot);
+  float* const red = reinterpret_cast<float*>(s_pair + L::kSlots);  // [class][tile of the workgroup][half, row]
+  const int run = lane >> 5, half = (lane >> 4) & 1;
+
+  // the pair's activations, requested before its expert is known
+  const size_t x_row = NM == 2 ? (size_t)(pair / a.top_k) : (size_t)pair;
+  const float* const x_f = a.x + x_row * a.K;
+  PairDigits<kScale> x;
+  float4 quad = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto load_x = [&](int sb) __attribute__((always_inline)) {
+    if constexpr (NM == 2) quad = reinterpret_cast<const float4*>(x_f)[min(sb * 64 + lane, a.K / 4 - 1)];
+    else x.load(a.xd + (x_row * nsb + sb) * kSbDigitBytes, a.xe + (x_row * nsb + sb) * 16);
+  };
+  Dma dma;  // (its lane offsets are ready before the expert is known)
+  if (any) {
+    load_x(cls);
+    if constexpr (!DIRECT) dma.init(row_bytes, cls);
+  }
+  if (pair >= *a.valid_tokens * a.top_k) return;
+  const size_t e_off = (size_t)__builtin_amdgcn_readfirstlane(id) * a.expert_bytes;
+  auto request_w = [&](int i, int sb) __attribute__((always_inline)) {
+    const size_t tile = e_off + (size_t)(tile_lo + sub + per_class * i) * tile_rows * row_bytes;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      dma.request(NM == 2 && r ? a.w1 : a.w0, a.w_bytes, NM == 2 ? tile : tile + (size_t)(16 * r) * row_bytes, row_bytes, sb,
+                  w_lds + r * Dma::kRunBytes);
+  };
+  SbRaw<QUANT> raw;
+  if constexpr (DIRECT) {
+    const bool dead = TAIL && half == 1 && cls * kSbElems + 128 >= a.K;  // (a half past the row's end: its bytes are never looked at)
+    const size_t row = (size_t)(tile_lo + sub) * tile_rows + (NM == 2 ? 0 : 16 * run) + (lane & 15);
+    if (any) sb_read((NM == 2 && run ? a.w1 : a.w0) + e_off + row * row_bytes + (size_t)cls * SbRaw<QUANT>::kBytes, dead ? 0 : half, raw);
+  } else {
+    if (any) request_w(0, cls);
+  }
+  int sb = any ? cls : nsb, i = 0;
+#pragma unroll 1
+  while (sb < nsb) {
+    const bool last = i + 1 >= n_mine;
+    const int next_i = last ? 0 : i + 1, next_sb = last ? sb + classes : sb;
+    if constexpr (!DIRECT) {
+      wait_loads();
+      sb_read(Dma::row_at(w_slot + run * Dma::kRunBytes, row_bytes, lane & 15, sb), half, raw);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if constexpr (NM == 2) {
+      if (i == 0) {
+        const bool in = !TAIL || sb * kSbElems + 4 * lane < a.K;
+        const float q[4] = {in ? quad.x : 0.0f, in ? quad.y : 0.0f, in ? quad.z : 0.0f, in ? quad.w : 0.0f};
+        x.e[0].x = digitize_quads(q, w_slot);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        x.load_digits(w_slot);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    }
+    if (!DIRECT && next_sb < nsb) {
+      if (next_sb != sb) dma.init(row_bytes, next_sb);
+      request_w(next_i, next_sb);
+    }
+    const float v = pair_dot<QUANT, kScale, TAIL>(
+        raw, x, [&](int) __attribute__((always_inline)) { return x_f + sb * kSbElems; }, TAIL && half == 1 && sb * kSbElems + 128 >= a.K);
+    float* const r = red + (((size_t)cls * (kTiles * per_class) + sub + per_class * i) * 64 + half * 32 + run * 16 + (lane & 15));
+    *r = (sb == cls ? 0.0f : *r) + v;
+    if (DIRECT) break;
+    if (last && next_sb < nsb) load_x(next_sb);
+    sb = next_sb;
+    i = next_i;
+  }
+  __syncthreads();
+  const int live_classes = min(classes, nsb), class_stride = kTiles * per_class * 64;
+  auto total = [&](int tl, int col) __attribute__((always_inline)) {
+    float h[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const float* p = red + (size_t)tl * 64 + 32 * q + col;
+      float v = p[0];
+      for (int c = 1; c < live_classes; ++c) v += p[(size_t)c * class_stride];
+      h[q] = v;
+    }
+    return h[0] + h[1];
+  };
+  for (int n = threadIdx.x; n < n_wg * tile_rows; n += 512) {
+    const int col = n % tile_rows, tl = n / tile_rows, row = (tile_lo + tl) * tile_rows + col;
+    if constexpr (NM == 2) {
+      const float v = silu_f(total(tl, col)) * total(tl, col + 16);
+      a.out[(size_t)pair * a.n_rows + row] = v;
+      // sixteen consecutive threads hold one group of the next contraction's activations
+      store_digit_group(v, row, a.out_d + (size_t)pair * a.out_nsb * kSbDigitBytes, a.out_e + (size_t)pair * a.out_nsb * 16, true);
+    } else {
+      a.out[(size_t)pair * a.n_rows + row] = weight * total(tl, col);
+    }
+  }
+}
+
 // ------------------------------------------------------------------ host side
+template <int QUANT, int NM, bool TAIL, bool DIRECT, int SQ>
+static int pairs_go(dim3 grid, hipStream_t s, const RowsArgs* a, const ExpertArgs& sh) {
+  constexpr size_t smem = PairRowsLds<QUANT, TAIL, DIRECT>::kBytes;
+  if (!a) {
+    XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_pairs<QUANT, NM, TAIL, DIRECT, SQ>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    return XABE_OK;
+  }
+  hipLaunchKernelGGL((k_digit_pairs<QUANT, NM, TAIL, DIRECT, SQ>), grid, dim3(512), smem, s, *a, sh);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+// `sq`: the format of the shared expert's rows (negative: not in this launch)
+template <int QUANT, int NM, bool TAIL>
+static int pairs_form(bool direct, int sq, dim3 grid, hipStream_t s, const RowsArgs* a, const ExpertArgs& sh) {
+  if constexpr (!TAIL) {
+    if (sq == XABE_QUANT_Q6K) return pairs_go<QUANT, NM, false, true, kQ6K>(grid, s, a, sh);
+    if (sq == XABE_QUANT_Q8_0) return pairs_go<QUANT, NM, false, true, kQ8_0>(grid, s, a, sh);
+  }
+  return direct ? pairs_go<QUANT, NM, TAIL, true, -1>(grid, s, a, sh) : pairs_go<QUANT, NM, TAIL, false, -1>(grid, s, a, sh);
+}
+template <int NM>
+static int pairs_quant(int quant, bool tail, bool direct, int sq, dim3 grid, hipStream_t s, const RowsArgs* a, const ExpertArgs& sh) {
+  if (quant == XABE_QUANT_Q6K) return pairs_form<kQ6K, NM, false>(direct, sq, grid, s, a, sh);
+  return tail ? pairs_form<kQ8_0, NM, true>(direct, sq, grid, s, a, sh) : pairs_form<kQ8_0, NM, false>(direct, sq, grid, s, a, sh);
+}
+
 template <int MODE, int QUANT, int NM, int NT, int TEAMS, int MT, bool TAIL>
 static size_t rows_lds() {
   const size_t slots = (size_t)8 * RowsLds<MODE, QUANT, NM, NT, TAIL>::kPerWave, red = (size_t)8 * MT * NT * TEAMS * 64 * sizeof(float);
@@ -370,7 +592,6 @@ static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, c
 
 template <int NM>
 static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
-  if (mode == kRowsFlat) return rows_quant<kRowsFlat, NM, 1, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
   if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, kRowsBlockTokens, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
   return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
 }
@@ -378,7 +599,14 @@ static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, 
 static int digit_rows_set_limits() {
   for (int q : {XABE_QUANT_Q6K, XABE_QUANT_Q8_0})
     for (bool tail : {false, true})
-      for (int mode : {kRowsFlat, kRowsBlock, kRowsShared})
+      for (bool direct : {false, true})
+        for (int sq : {-1, (int)XABE_QUANT_Q6K, (int)XABE_QUANT_Q8_0}) {
+          XABE_TRY(pairs_quant<1>(q, tail, direct, sq, dim3(1), nullptr, nullptr, ExpertArgs{}));
+          XABE_TRY(pairs_quant<2>(q, tail, direct, sq, dim3(1), nullptr, nullptr, ExpertArgs{}));
+        }
+  for (int q : {XABE_QUANT_Q6K, XABE_QUANT_Q8_0})
+    for (bool tail : {false, true})
+      for (int mode : {kRowsBlock, kRowsShared})
         for (int nt : {1, 2, 4, 8})
           for (int mt : {1, kRowsMaxTiles}) {
             XABE_TRY(rows_mode<1>(mode, nt, mt, q, tail, dim3(1), nullptr, nullptr));
@@ -402,12 +630,46 @@ int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, u
   return XABE_OK;
 }
 
-int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s) {
+static void rows_shape(RowsArgs& a, int quant, int nm) {
   const size_t be = xabe_expert_quant_block_elements(quant), bb = xabe_expert_quant_block_bytes(quant);
   a.nsb = (int)digit_superblocks((size_t)a.K);
   a.row_bytes = (uint32_t)((size_t)a.K / be * bb);
   a.out_nsb = (int)digit_superblocks((size_t)a.n_rows);
-  a.classes = a.nsb >= 8 ? 8 : a.nsb > 4 ? 8 : a.nsb > 2 ? 4 : a.nsb;
+  a.classes = a.nsb > 4 ? 8 : a.nsb > 2 ? 4 : a.nsb;
+  a.tile_rows = nm == 2 ? 16 : 32;
+  a.n_tiles = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
+}
+
+
+int launch_digit_pairs(const xabe_moe_kernels* k, int quant, int nm, RowsArgs a, size_t units, hipStream_t s, const ExpertArgs* shared, int shared_quant) {
+  rows_shape(a, quant, nm);
+  const int per_class = 8 / a.classes, wg_tiles = (a.n_tiles + per_class - 1) / per_class;
+  // tiles per wavefront: as many as leave 384 workgroups (one with the shared expert: those launches have at most 32
+  // pairs; us with it, one / two tiles: three tokens 28.1 / 29, four 36.1 / 37)
+  int each = 1;
+  while (!shared && each < kPairTiles && units * (size_t)wg_tiles >= (size_t)768 * each) each *= 2;
+  a.shares = (wg_tiles + each - 1) / each;
+  a.units = (int)units;
+  const bool direct = each == 1 && a.nsb <= a.classes, tail = a.K % kSbElems != 0;
+  // (shares that divide evenly over the XCDs, or the XCDs over them)
+  a.xcd_units = k->g.max_tokens < kPairsXcdMinTokens ? 0 : a.shares % 8 == 0 ? 1 : 8 % a.shares == 0 ? 8 / a.shares : 0;
+  size_t wgs = a.xcd_units > 1 ? (units + a.xcd_units - 1) / a.xcd_units * 8 : units * a.shares;
+  ExpertArgs sh;
+  memset(&sh, 0, sizeof(sh));
+  if (shared) {
+    sh = *shared;
+    a.shared_rps = a.K == 256 ? 8 : a.K == 512 ? 4 : a.K == 1024 ? 2 : 1;
+    sh.tile_rows = kWavesPerWg * a.shared_rps;
+    a.shared_wgs = (a.n_rows / sh.tile_rows + 1) / 2;
+    wgs += (k->g.max_tokens + 1) / 2 * a.shared_wgs;
+  }
+  const dim3 grid((unsigned)wgs);
+  const int sq = shared ? shared_quant : -1;
+  return nm == 2 ? pairs_quant<2>(quant, tail, direct, sq, grid, s, &a, sh) : pairs_quant<1>(quant, tail, direct, sq, grid, s, &a, sh);
+}
+
+int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s) {
+  rows_shape(a, quant, nm);
   int nt = 1;
   if (mode == kRowsShared) {
     // tokens per pass over the weights: all of them up to eight, equal passes beyond
@@ -416,12 +678,10 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
     units = (t + nt - 1) / nt;
   }
   const int per_class = std::max(1, (nt > 4 ? 4 : 8) / a.classes);  // (as the kernel has it: nt > 4 is two teams)
-  a.tile_rows = nm == 2 ? 16 : 32;
   int mt = 1;
-  const int tiles16 = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
-  a.n_tiles = tiles16;
+  const int tiles16 = a.n_tiles;
   unsigned grid_x = (unsigned)((tiles16 + per_class - 1) / per_class);
-  if (mode != kRowsShared) {
+  if (mode == kRowsBlock) {
     grid_x = (unsigned)((tiles16 + per_class * kRowsRoutedTiles - 1) / (per_class * kRowsRoutedTiles));
   } else if (per_class == 1 && tiles16 > k->num_cus) {
     // many tiles: one workgroup per CU with an even share of them, so that a superblock's digits serve the whole share

@@ -95,22 +95,30 @@ __device__ __forceinline__ uint32_t magnitude16(const float (&x)[16]) {
   for (int i = 0; i < 16; ++i) mag = max(mag, __builtin_bit_cast(uint32_t, x[i]) & 0x7fffffffu);
   return mag;
 }
-// The digits of one group of 16 activations; `inexact` is set where they do not hold one.
+// The digits of four and of sixteen activations, a word (a 16-byte piece) per digit; `inexact` is set where they do not
+// hold one.
+__device__ __forceinline__ void digitize4(const float (&x)[4], int shift, uint32_t (&plane)[6], bool& inexact) {
+  uint32_t y[4], z[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) digits_of(x[i], shift, y[i], z[i], inexact);
+  const uint32_t ab_hi = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u), cd_hi = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+  const uint32_t ab_lo = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), cd_lo = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
+  const uint32_t ab_z = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), cd_z = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
+  plane[0] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x07060302u);
+  plane[1] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x05040100u);
+  plane[2] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x07060302u);
+  plane[3] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x05040100u);
+  plane[4] = __builtin_amdgcn_perm(cd_z, ab_z, 0x07060302u);
+  plane[5] = __builtin_amdgcn_perm(cd_z, ab_z, 0x05040100u);
+}
 __device__ __forceinline__ void digitize16(const float (&x)[16], int shift, v4u_t (&plane)[6], bool& inexact) {
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    uint32_t y[4], z[4];
+    const float q[4] = {x[4 * w], x[4 * w + 1], x[4 * w + 2], x[4 * w + 3]};
+    uint32_t word[6];
+    digitize4(q, shift, word, inexact);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) digits_of(x[4 * w + i], shift, y[i], z[i], inexact);
-    const uint32_t ab_hi = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u), cd_hi = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
-    const uint32_t ab_lo = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), cd_lo = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
-    const uint32_t ab_z = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), cd_z = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
-    plane[0][w] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x07060302u);
-    plane[1][w] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x05040100u);
-    plane[2][w] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x07060302u);
-    plane[3][w] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x05040100u);
-    plane[4][w] = __builtin_amdgcn_perm(cd_z, ab_z, 0x07060302u);
-    plane[5][w] = __builtin_amdgcn_perm(cd_z, ab_z, 0x05040100u);
+    for (int p = 0; p < 6; ++p) plane[p][w] = word[p];
   }
 }
 // The largest of sixteen consecutive lanes' values (a DPP row), and whether any of them says yes.
@@ -136,6 +144,23 @@ __device__ __forceinline__ float digitize_superblock(const float (&x)[16], int p
 #pragma unroll
   for (int p = 0; p < 6; ++p) reinterpret_cast<v4u_t*>(d)[p] = plane[p];
   return digit_scale(mag, e, row16_any(inexact));
+}
+
+// A superblock whose sixty-four quads of elements the wavefront's lanes hold: digits to `base`; returns its scale.
+__device__ __forceinline__ float digitize_quads(const float (&x)[4], uint8_t* base) {
+  const int lane = (int)__lane_id();
+  uint32_t mag = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) mag = max(mag, __builtin_bit_cast(uint32_t, x[i]) & 0x7fffffffu);
+  mag = (uint32_t)wave_max_i((int)mag);
+  const int e = digit_exponent(mag), shift = digit_shift(e);
+  uint32_t plane[6];
+  bool inexact = false;
+  digitize4(x, shift, plane, inexact);
+  uint8_t* d = base + digit_group_offset(lane >> 2) + 4 * (lane & 3);
+#pragma unroll
+  for (int p = 0; p < 6; ++p) *reinterpret_cast<uint32_t*>(d + 16 * p) = plane[p];
+  return digit_scale(mag, e, __builtin_amdgcn_ballot_w64(inexact) != 0);
 }
 
 // Where group `pos` (elements 16 pos .. 16 pos + 15 of its superblock) lies among the digits and the scales.
@@ -509,7 +534,8 @@ struct SliceDma {
 // and zero elsewhere, so that the four result registers of a lane are the digit sums of the sixteen elements the lane
 // itself unpacked.  The same exact sums and the same fp32 operations per half superblock as sb_dot's, with no operand
 // rows spent on other tokens: for a single token 32 rows x 1 superblock and this shape carry the same bytes, and this
-// one needs no zeros in LDS and fits rows of one or two superblocks (a pair is then one row or two).
+// one needs no zeros in LDS, four result registers instead of sixteen, and fits rows of one or two superblocks (a pair
+// is then one row or two).  A caller may as well give quarters 2 and 3 sixteen other rows of the same superblock.
 // ---------------------------------------------------------------------------------
 // N byte offsets below 65536, two to a register: what a lane adds per DMA instruction, unpacked where it is used.
 template <int N>
@@ -584,6 +610,16 @@ struct PairDigits {
   float4 e[WHOLE ? 1 : 2];   // the superblock's in .x, or [l], s = 0..3
   // `xd`, `xe`: digits and scales of the activation superblock the lane's weights lie in
   __device__ __forceinline__ void load(const uint8_t* xd, const float* xe) {
+    load_digits(xd);
+    if constexpr (WHOLE) {
+      e[0].x = *xe;
+    } else {
+      const int h = ((int)__lane_id() >> 4) & 1;
+#pragma unroll
+      for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
+    }
+  }
+  __device__ __forceinline__ void load_digits(const uint8_t* xd) {
     const int lane = (int)__lane_id(), q = lane >> 4, m = lane & 15, h = q & 1;
     const bool mine = (m >> 2) == q;
 #pragma unroll
@@ -598,19 +634,13 @@ struct PairDigits {
 #pragma unroll
       for (int s = 0; s < 4; ++s) z[s] = *reinterpret_cast<const v4i_t*>(pz + 4 * s * kGroupBytes);
     }
-    if constexpr (WHOLE) {
-      e[0].x = *xe;
-    } else {
-#pragma unroll
-      for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
-    }
   }
 };
 
 // `x_of(quarter)`: the 256 fp32 activations of the superblock that quarter `lane >> 4` of the wavefront holds, read where
-// a scale is a mark.
-template <int QUANT, bool WHOLE, typename XOf>
-__device__ __forceinline__ float pair_dot(SbRaw<QUANT>& r, const PairDigits<WHOLE>& x, XOf x_of) {
+// a scale is a mark.  `dead`: the lane's half lies past the end of the row (its codes are other data's bytes).
+template <int QUANT, bool WHOLE, bool TAIL = false, typename XOf>
+__device__ __forceinline__ float pair_dot(SbRaw<QUANT>& r, const PairDigits<WHOLE>& x, XOf x_of, bool dead = false) {
   constexpr bool kPairs = kAddsGroups<QUANT, WHOLE>, kInts = WHOLE && QUANT == kQ6K;
   constexpr int kUnits = kPairs ? 4 : 8;
   float out = 0.0f, ws[2];
@@ -654,10 +684,11 @@ __device__ __forceinline__ float pair_dot(SbRaw<QUANT>& r, const PairDigits<WHOL
   }
   if constexpr (kInts) out = join_sums(sum) * (sb_quarter(r) * x.e[0].x);
   else if constexpr (WHOLE) out *= x.e[0].x;
+  if (TAIL && dead) out = 0.0f;
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(out != out) != 0, 0)) {
     int quarter = (int)__lane_id() >> 4;
     asm volatile("" : "+v"(quarter));  // (keeps the address out of the registers of the loop around)
-    const float plain = half_fp32(r, x_of(quarter) + 128 * (quarter & 1));
+    const float plain = half_fp32(r, x_of(quarter) + (TAIL && dead ? 0 : 128 * (quarter & 1)));
     if (out != out) out = plain;
   }
   return out;

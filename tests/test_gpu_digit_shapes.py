@@ -1,0 +1,89 @@
+"""The digit row contractions over the row lengths where their forms differ: rows that end in half a superblock (Q8_0 rows of
+128 elements modulo 256: a wider window, a half that is not there), one to ten superblocks (the split between the
+wavefronts changes at 3, 5 and 9), both formats, every pass width of a single matrix, pairs against dispatch blocks.
+
+Tolerance: three contractions in a row, each held to 5e-7 of the peak (tests/test_gpu_digit_precision.py derives it)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 3 * 5e-7
+
+
+def _stacks(X, q, E, H, I, seed):
+    import torch
+
+    out = [X.QuantTensor(X.synth_quant(q, seed + i, E * H * I, 0.02), q) for i in range(3)]
+    host = [X.dequantize(q, t.bytes).double().cpu().numpy() for t in out]
+    torch.cuda.synchronize()
+    return out, (host[0].reshape(E, I, H), host[1].reshape(E, I, H), host[2].reshape(E, H, I))
+
+
+def _ffn64(host, e, x):
+    g, u = host[0][e] @ x, host[1][e] @ x
+    return host[2][e] @ (g / (1 + np.exp(-g)) * u)
+
+
+ROUTED = [("q8", 128, 128), ("q8", 384, 128), ("q8", 640, 384), ("q8", 1152, 896), ("q8", 2176, 1280), ("q8", 512, 2176),
+          ("q6", 256, 256), ("q6", 768, 1280), ("q6", 1792, 768), ("q6", 2304, 2560)]
+
+
+@pytest.mark.parametrize("fmt,hidden,inter", ROUTED)
+def test_routed_experts(fmt, hidden, inter):
+    import torch
+    import llmxabe_amd as X
+
+    E, K = 5, 2
+    q = X.ExpertQuant.Q8_0 if fmt == "q8" else X.ExpertQuant.Q6K
+    st, host = _stacks(X, q, E, hidden, inter, 9000)
+    for tokens, live in ((1, 1), (4, 3), (5, 5), (25, 23), (63, 63)):
+        x = X.synth_normal_f32(9010 + tokens, tokens * hidden, 1.0)
+        logits = X.synth_normal_f32(9011 + tokens, tokens * E, 1.0)
+        got = []
+        for blocks in (False, True) if tokens > 4 else (False,):
+            k = X.MoeKernels(X.MoeGeometry(E, K, hidden, inter, 32, tokens))
+            k.force_community(blocks)
+            b = k.buffers()
+            k.set_valid_tokens(b, live)
+            k.route_and_dispatch(b, logits)
+            k.grouped_forward_partial(b, *st, x)
+            got.append(b.partial().cpu().numpy().reshape(tokens, K, hidden)[:live].copy())
+        ids = b.topk_ids().cpu().numpy().reshape(tokens, K)
+        wts = b.topk_weights().cpu().numpy().reshape(tokens, K)
+        xs = x.double().cpu().numpy().reshape(tokens, hidden)
+        ref = np.array([[wts[t, j] * _ffn64(host, ids[t, j], xs[t]) for j in range(K)] for t in range(live)])
+        err = np.abs(got[0] - ref).max() / np.abs(ref).max()
+        print(fmt, hidden, inter, tokens, f"{err:.2e}", flush=True)
+        assert err <= TOL, (tokens, err)
+        assert len(got) == 1 or np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), tokens
+
+
+SHARED = [("q8", 2176, 128), ("q8", 2432, 384), ("q8", 2304, 1152), ("q8", 4096, 1664), ("q6", 2304, 768), ("q6", 2560, 1280),
+          ("q6", 4096, 1792), ("q6", 5120, 2304)]
+
+
+@pytest.mark.parametrize("fmt,hidden,inter", SHARED)
+def test_single_matrix_rows(fmt, hidden, inter):
+    # hidden above 2048: the shared expert's (the dense block's) rows on the digits, one to eight tokens per pass
+    import torch
+    import llmxabe_amd as X
+
+    q = X.ExpertQuant.Q8_0 if fmt == "q8" else X.ExpertQuant.Q6K
+    st, host = _stacks(X, q, 1, hidden, inter, 9100)
+    x = X.synth_normal_f32(9110, 17 * hidden, 1.0).view(17, hidden)
+    ref = np.array([_ffn64(host, 0, v) for v in x.double().cpu().numpy()])
+    alone = None
+    for tokens, live in ((1, 1), (2, 2), (3, 3), (4, 4), (7, 6), (8, 8), (17, 17)):
+        k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, tokens))
+        b = k.shared_only_buffers(False)
+        k.set_valid_tokens(b, live)
+        out = torch.full((tokens, hidden), 7.0, device="cuda")
+        k.shared_expert(b, *st, x[:tokens].reshape(-1).contiguous(), out.view(-1))
+        got = out.cpu().numpy()
+        err = np.abs(got[:live] - ref[:live]).max() / np.abs(ref).max()
+        print(fmt, hidden, inter, tokens, f"{err:.2e}", flush=True)
+        assert err <= TOL, (tokens, err)
+        assert (got[live:] == 7.0).all(), tokens     # rows past the live ones are not written
+        alone = got if tokens == 1 else alone
+        assert np.array_equal(got[0].view(np.uint32), alone[0].view(np.uint32)), tokens
