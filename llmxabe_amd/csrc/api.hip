@@ -101,6 +101,7 @@ static Shape shape_for(size_t K) {
 }
 static int rows_per_step(Shape s) { return s == kRps8 ? 8 : s == kRps4 ? 4 : s == kRps2 ? 2 : 1; }
 
+// (gate/up rows longer than one step go through the digit contraction)
 template <int QUANT, int NM>
 static void launch_shape(Shape shape, dim3 grid, hipStream_t s, const ExpertArgs& a) {
   switch (shape) {
@@ -108,8 +109,12 @@ static void launch_shape(Shape shape, dim3 grid, hipStream_t s, const ExpertArgs
     case kRps4: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 4, NM>), grid, dim3(256), 0, s, a); break;
     case kRps2: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 2, NM>), grid, dim3(256), 0, s, a); break;
     case kKs1: hipLaunchKernelGGL((k_expert_shared<QUANT, 1, 1, NM>), grid, dim3(256), 0, s, a); break;
-    case kKs2: hipLaunchKernelGGL((k_expert_shared<QUANT, 2, 1, NM>), grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_expert_shared<QUANT, 0, 1, NM>), grid, dim3(256), 0, s, a); break;
+    case kKs2:
+      if constexpr (NM == 1) hipLaunchKernelGGL((k_expert_shared<QUANT, 2, 1, NM>), grid, dim3(256), 0, s, a);
+      break;
+    default:
+      if constexpr (NM == 1) hipLaunchKernelGGL((k_expert_shared<QUANT, 0, 1, NM>), grid, dim3(256), 0, s, a);
+      break;
   }
 }
 
@@ -126,6 +131,8 @@ int pick_tile_rows(const xabe_moe_kernels* k, size_t live_units, int n_rows, int
 // `units`: grid.y work units (chunks of two tokens)
 static int launch_expert(const xabe_moe_kernels* k, int quant, int nm, ExpertArgs a, size_t units, hipStream_t s) {
   const Shape shape = shape_for((size_t)a.K);
+  if (nm == 2 && (shape == kKs2 || shape == kStream))
+    return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "gate/up rows of %d elements take more than one step", a.K);
   const int rps = rows_per_step(shape);
   a.tile_rows = pick_tile_rows(k, units, a.n_rows, rps);
   const unsigned tiles = (unsigned)((a.n_rows + a.tile_rows - 1) / a.tile_rows);
@@ -335,6 +342,15 @@ int xabe_moe_kernels_set_exact_decode_regime(xabe_moe_kernels* k, int on) {
 }
 
 // ------------------------------------------------------------------ MoeBuffers
+// Single-expert stacks whose rows take more than one step of the lanes' sums: the digit contraction, except for small
+// matrices whose gate/up rows do fit a step, where the lanes' shorter chain wins at decode widths.  By the geometry alone,
+// so that a token's row is the same bits at every width.  Dense block, Q6_K, us, lanes / digits: hidden 1024, intermediate
+// 4352: one token 15 / 21, eight 30 / 36, thirty-two 87 / 63; 2048, 6144: 20 / 26, 50 / 45, 157 / 87; Q8_0, 2048, 8192:
+// 29 / 29, seven 105 / 48.
+static bool shared_on_digits(const xabe_moe_geometry& g) {
+  return g.hidden > 2048 || (g.intermediate > 2048 && g.hidden * g.intermediate >= ((size_t)10 << 20));
+}
+
 template <typename T>
 static int alloc_zeros(T** p, size_t n, hipStream_t s, size_t* total) {
   *p = nullptr;
@@ -388,7 +404,7 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->inter, routed ? sorted * g.intermediate : 0);
   A(&b->inter_d, (routed ? sorted : 0) * nsb_i * kSbDigitBytes);
   A(&b->inter_e, (routed ? sorted : 0) * nsb_i * 16);
-  const bool shared_long = g.hidden > 2048;  // (shorter rows: the lanes' sums, shared_fp32)
+  const bool shared_long = shared_on_digits(g);
   A(&b->shared_x_d, shared_long ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
   A(&b->shared_x_e, shared_long ? g.max_tokens * nsb_h : 0);
   A(&b->shared_inter_d, g.max_tokens * nsb_i * kSbDigitBytes);
@@ -791,10 +807,45 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   return launch_digit_rows(k, kRowsShared, down.quant, 1, a, 0, s);
 }
 
+// The same on the pair kernel: a token is a unit of expert 0.  Up to four tokens it saves the launch that makes the digits
+// (hidden 4096, intermediate 1024, Q6_K: one token 18.7 -> 17.9 us, three 22.5 -> 17.9); beyond, and for matrices that do
+// not stay in the caches, rows read and unpacked once per token cost more.
+static bool shared_by_pairs(const xabe_moe_kernels* k) {
+  return k->g.max_tokens <= 4 && k->g.hidden * k->g.intermediate <= ((size_t)8 << 20) && !k->force_community;
+}
+static int shared_pairs(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
+                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
+  const xabe_moe_geometry& g = k->g;
+  RowsArgs a = rows_args(k, b);
+  a.topk_ids = nullptr;
+  a.top_k = 1;
+  a.w0 = static_cast<const uint8_t*>(gate.bytes);
+  a.w1 = static_cast<const uint8_t*>(up.bytes);
+  a.w_bytes = gate.len;
+  a.x = x;
+  a.out = b->shared_inter;
+  a.out_d = b->shared_inter_d;
+  a.out_e = b->shared_inter_e;
+  a.K = (int)g.hidden;
+  a.n_rows = (int)g.intermediate;
+  XABE_TRY(launch_digit_pairs(k, gate.quant, 2, a, g.max_tokens, s));
+  a.w0 = static_cast<const uint8_t*>(down.bytes);
+  a.w1 = nullptr;
+  a.w_bytes = down.len;
+  a.x = b->shared_inter;
+  a.xd = b->shared_inter_d;
+  a.xe = b->shared_inter_e;
+  a.out = out;
+  a.K = (int)g.intermediate;
+  a.n_rows = (int)g.hidden;
+  return launch_digit_pairs(k, down.quant, 1, a, g.max_tokens, s);
+}
+
 static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
   const xabe_moe_geometry& g = k->g;
-  if (g.hidden > 2048) {
+  if (shared_on_digits(g)) {
+    if (shared_by_pairs(k)) return shared_pairs(k, s, b, gate, up, down, x, out);
     XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->shared_x_d, b->shared_x_e));
     return shared_digits(k, s, b, gate, up, down, x, out);
   }
@@ -813,7 +864,7 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
   const xabe_moe_geometry& g = k->g;
   *launched = false;
   XABE_TRY(check_shared_stacks(k, gate, up, down));  // the checks xabe_moe_shared_expert makes
-  if (g.hidden <= 2048) return XABE_OK;
+  if (!shared_on_digits(g)) return XABE_OK;
   if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(post_norm)) % 16 != 0)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "rms_norm: x, weight and out must be 16-byte aligned");
   hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)g.max_tokens), dim3(256), 0, s, residual, post_norm, normed, (int)g.hidden,

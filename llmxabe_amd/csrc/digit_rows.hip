@@ -21,19 +21,18 @@
 
 namespace xabe {
 
-// Digits of fp32 rows, scaled by superblocks: one thread per group of sixteen; groups past the end of the row are zeros.
+// Digits of fp32 rows, scaled by superblocks: a wavefront per superblock; elements past the end of the row are zeros.
+// (A thread per group of sixteen took 4.7 us for a single row, this 2.)
 __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__ x, int K, int nsb, int rows, uint8_t* __restrict__ xd,
                                                        float* __restrict__ xe) {
-  const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
-  if (i >= rows * nsb * 16) return;
-  const int row = i / (nsb * 16), gi = i % (nsb * 16);
-  float v[16];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(4 * gi + j, K / 4 - 1)];
-    v[4 * j] = f.x, v[4 * j + 1] = f.y, v[4 * j + 2] = f.z, v[4 * j + 3] = f.w;
-  }
-  store_digits16(v, gi, gi * 16 < K, xd + (size_t)row * nsb * kSbDigitBytes, xe + (size_t)row * nsb);
+  const int i = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)__lane_id();
+  if (i >= rows * nsb) return;
+  const int row = i / nsb, sb = i % nsb, at = sb * 64 + lane;
+  const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(at, K / 4 - 1)];
+  const bool in = 4 * at < K;
+  const float v[4] = {in ? f.x : 0.0f, in ? f.y : 0.0f, in ? f.z : 0.0f, in ? f.w : 0.0f};
+  const float scale = digitize_quads(v, xd + (size_t)i * kSbDigitBytes);
+  if (lane == 0) xe[i] = scale;
 }
 
 // Tiles per wavefront of a dispatch block, the next one's rows in flight while one is multiplied.
@@ -420,8 +419,8 @@ __global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a,
     }
   }
   const int pair = a.unit0 + u;
-  const int id = a.topk_ids[pair];
-  const float weight = NM == 1 ? a.topk_weights[pair] : 1.0f;
+  const int id = a.topk_ids ? a.topk_ids[pair] : 0;  // (none: a single expert, a token per unit)
+  const float weight = NM == 1 && a.topk_ids ? a.topk_weights[pair] : 1.0f;
   const int classes = a.classes, per_class = 8 / classes;
   const int cls = wave % classes, sub = wave / classes;
   const int tile_lo = (int)((long long)a.n_tiles * share / a.shares);
@@ -624,8 +623,8 @@ int digit_rows_configure() {
 }
 
 int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe) {
-  const size_t nsb = digit_superblocks(K), n = rows * nsb * 16;
-  hipLaunchKernelGGL(k_digitize_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
+  const size_t nsb = digit_superblocks(K), n = rows * nsb;
+  hipLaunchKernelGGL(k_digitize_rows, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
@@ -673,7 +672,8 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
   int nt = 1;
   if (mode == kRowsShared) {
     // tokens per pass over the weights: all of them up to eight, equal passes beyond
-    const size_t t = k->g.max_tokens, passes = (t + 7) / 8, each = (t + passes - 1) / passes;
+    // (force_community: one, for comparison: the same bits)
+    const size_t t = k->g.max_tokens, passes = k->force_community ? t : (t + 7) / 8, each = (t + passes - 1) / passes;
     nt = each == 1 ? 1 : each == 2 ? 2 : each <= 4 ? 4 : 8;
     units = (t + nt - 1) / nt;
   }

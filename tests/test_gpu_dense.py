@@ -88,9 +88,9 @@ def test_dense_prefill_2048_matches_oracle_on_sampled_rows(oracle, dense):
 
 
 @pytest.mark.parametrize("max_tokens,tokens", [(1, 1), (8, 8), (16, 13)])
-def test_long_row_kernel_equals_the_plain_one(dense, max_tokens, tokens):
-    # rows longer than one 2048-element step take the step-outer kernel (weights read once per eight tokens);
-    # force_community keeps the row-outer streaming kernel: same operation order per (row, token), same bits
+def test_passes_of_several_tokens_equal_passes_of_one(dense, max_tokens, tokens):
+    # up to eight tokens share a pass over the weights, in other kernels than a single token's; force_community makes a
+    # pass per token (and keeps a single token off the pair kernel): same operation order per (row, token), same bits
     import torch
 
     X, w, host, H, I = dense

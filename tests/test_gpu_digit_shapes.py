@@ -60,12 +60,13 @@ def test_routed_experts(fmt, hidden, inter):
 
 
 SHARED = [("q8", 2176, 128), ("q8", 2432, 384), ("q8", 2304, 1152), ("q8", 4096, 1664), ("q6", 2304, 768), ("q6", 2560, 1280),
-          ("q6", 4096, 1792), ("q6", 5120, 2304)]
+          ("q6", 4096, 1792), ("q6", 5120, 2304), ("q8", 1152, 9472), ("q6", 2048, 5120)]
 
 
 @pytest.mark.parametrize("fmt,hidden,inter", SHARED)
 def test_single_matrix_rows(fmt, hidden, inter):
-    # hidden above 2048: the shared expert's (the dense block's) rows on the digits, one to eight tokens per pass
+    # hidden above 2048, or a long intermediate row: the shared expert's (the dense block's) rows on the digits, one to
+    # eight tokens per pass
     import torch
     import llmxabe_amd as X
 
@@ -85,5 +86,9 @@ def test_single_matrix_rows(fmt, hidden, inter):
         print(fmt, hidden, inter, tokens, f"{err:.2e}", flush=True)
         assert err <= TOL, (tokens, err)
         assert (got[live:] == 7.0).all(), tokens     # rows past the live ones are not written
+        one = torch.zeros_like(out)
+        k.force_community(True)                      # a pass per token, in the kernel of a single matrix
+        k.shared_expert(b, *st, x[:tokens].reshape(-1).contiguous(), one.view(-1))
+        assert np.array_equal(got[:live].view(np.uint32), one.cpu().numpy()[:live].view(np.uint32)), tokens
         alone = got if tokens == 1 else alone
         assert np.array_equal(got[0].view(np.uint32), alone[0].view(np.uint32)), tokens
