@@ -655,13 +655,15 @@ static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) 
   return a;
 }
 
-// One (token, k) pair per unit below the matrix-core widths (most dispatch blocks hold one or two tokens there, and the
-// pair kernel runs twice as many workgroups) and in the exact regime; dispatch blocks at wider passes.  Microseconds of
-// the routed experts of the model (256 experts, top 8), pairs / blocks: 5 tokens 38 / 51, 13: 71 / 84, 32: 130 / 160, 45:
-// 171 / 213, 63: 224 / 268; 64 experts, top 4, hidden 1024: 13 tokens 26 / 56, 45: 51 / 80.  force_community keeps the
-// blocks, where there are any, for comparison: same bits.
+// One (token, k) pair per unit while fewer than four select an expert on average, and in the exact regime; dispatch blocks
+// beyond, which read and unpack an expert's rows once per four or eight tokens.  Routed experts, us, pairs / blocks: the
+// model's 256 experts, top 8, 32 tokens 130 / 165, 45: 171 / 198, 63: 224 / 237, 64: 236 / 244, 256: 792 / 549, 1024:
+// 3049 / 1612; 64 experts, top 4, hidden 1024: 45 tokens 51 / 70, 256: 199 / 150.
+// force_community keeps the blocks, where there are any, for comparison: same bits.
+constexpr size_t kPairsPerExpert = 4;
 static bool routed_by_pairs(const xabe_moe_kernels* k) {
-  return flat_regime(k) || (k->g.max_tokens < kMfmaMinTokens && !k->force_community);
+  const xabe_moe_geometry& g = k->g;
+  return flat_regime(k) || (!k->force_community && g.max_tokens * g.experts_per_token < kPairsPerExpert * g.num_experts);
 }
 
 // The shared expert's tensors and rows, for launches that take its row tiles along (x: the routed experts' own rows).
@@ -677,7 +679,8 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   const xabe_moe_geometry& g = k->g;
   const bool pairs = routed_by_pairs(k);
   const size_t units = pairs ? xabe_moe_geometry_max_flat_pairs(&g) : b->n_expert_blocks;
-  if (units > 65535) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "%zu work units exceed the 65535 grid.y limit of the fp32 regime", units);
+  if (flat_regime(k) && units > 65535)
+    return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "%zu work units exceed the 65535 grid.y limit of the fp32 regime", units);
   const size_t expert_elems = g.intermediate * g.hidden;
   RowsArgs up_a = rows_args(k, b);
   up_a.w0 = static_cast<const uint8_t*>(gate.bytes);

@@ -37,12 +37,11 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
 
 // Tiles per wavefront of a dispatch block, the next one's rows in flight while one is multiplied.
 constexpr int kRowsRoutedTiles = 4;
-constexpr int kRowsBlockTokens = 2;  // tokens per chunk of a dispatch block (most hold one or two)
 
 template <int MODE, int QUANT, int NM, int NT, bool TAIL>
 struct RowsLds {
   using Dma = SliceDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
-  static constexpr int kDigits = MODE == kRowsShared ? NT * kSbDigitBytes : 0, kScales = NM == 1 ? NT * kSbScaleBytes : 0;
+  static constexpr int kDigits = NT * kSbDigitBytes, kScales = NM == 1 ? NT * kSbScaleBytes : 0;
   static constexpr int kPerWave = Dma::kSlotBytes + kDigits + 2 * kScales;
 };
 
@@ -127,17 +126,17 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   const int u_lane = (lane >> 4) & 1, r_lane = lane & 15, half = lane >> 5;
 
   for (int first = 0; first < n_tok; first += kTokens) {
-    // the chunk's tokens: activation rows (tokens past the live ones repeat one of them and are never stored)
+    // the chunk's tokens: activation rows (tokens past the live ones repeat the last of them and are never stored)
     int x_row[NT], n_live = 0;
     if constexpr (MODE == kRowsBlock) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int f = first + t < n_tok ? slots[first + t] : sentinel;
-        const bool live = f < sentinel && n_live == t;
-        if (live) ++n_live;
-        x_row[t] = NM == 2 ? (live ? f : slots[first]) / a.top_k : (int)slot0 + first + (live ? t : 0);
-      }
+      for (int t = 0; t < kTokens; ++t) n_live += n_live == t && first + t < n_tok && slots[first + t] < sentinel;
       if (n_live == 0) break;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int at = first + min(t0 + t, n_live - 1);
+        x_row[t] = NM == 2 ? slots[at] / a.top_k : (int)slot0 + at;
+      }
     } else {
       n_live = n_tok;
 #pragma unroll
@@ -149,10 +148,8 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
       if ((lane >> 2) == t) x_row_l = x_row[t];
     float e_now[NT], e_next[NT];  // (whole superblocks' scales)
     auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
-      // (dispatch blocks keep a superblock's digits for a whole share and their chunks are small: they come straight into
-      // registers below)
 #pragma unroll
-      for (int t = 0; t < NT && MODE == kRowsShared; ++t) {
+      for (int t = 0; t < NT; ++t) {
         const uint8_t* from = a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes;
         lds_dma_16(from, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
         if (lane < 32) lds_dma_16(from + 1024, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes + 1024);
@@ -197,26 +194,14 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
             for (int t = 0; t < NT; ++t) e_now[t] = e_next[t];
           }
           x.point(d_slot, e_slot + buf * L::kScales, s_zero);
-          if constexpr (MODE == kRowsShared) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
+          for (int j = 0; j < 8; ++j)
 #pragma unroll
-              for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.high(j & 3, j >> 2, tg);
+            for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.high(j & 3, j >> 2, tg);
 #pragma unroll
-            for (int j = 0; j < (kSwapped ? 8 : 4) && !digits_in_one(NT); ++j)
+          for (int j = 0; j < (kSwapped ? 8 : 4) && !digits_in_one(NT); ++j)
 #pragma unroll
-              for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
-          } else {
-            static_assert(MODE == kRowsShared || digits_in_one(NT), "chunks of a dispatch block are one or two tokens");
-            const int at = high_digit_at<NT>(lane, 0, 0);
-            const int row = NT > 1 && (lane & 16) ? x_row[NT - 1] : x_row[0];
-            const uint8_t* d = a.xd + ((size_t)row * nsb + sb) * kSbDigitBytes + max(at, 0);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              ax[j][0] = v4i_t{0, 0, 0, 0};
-              if (at >= 0) ax[j][0] = *reinterpret_cast<const v4i_t*>(d + (4 * (j & 3) + (j >> 2)) * kGroupBytes);
-            }
-          }
+            for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
         }
         if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
 #pragma unroll
@@ -234,8 +219,8 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
         float v[NT];
         auto x_of = [&](int t) __attribute__((always_inline)) {
           int row = x_row[0];
-          if constexpr (MODE == kRowsShared) row = (int)slot0 + min(t0 + t, n_live - 1);
-          else if constexpr (NT > 1) row = t ? x_row[NT - 1] : row;
+#pragma unroll
+          for (int j = 1; j < NT; ++j) row = t == j ? x_row[j] : row;
           return a.x + (size_t)row * a.K + sb * kSbElems;
         };
         auto e_of = [&](int t, int l) __attribute__((always_inline)) {
@@ -330,8 +315,9 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
 // the others.  gate/up makes the digits of its activation superblocks itself, four elements per lane, in the weight slot
 // between a tile's bytes and the next one's: a launch of its own for them cost 4.7 us and its boundary.  Sums wait in LDS.
 // What bounds it: at a few tokens the chain of round trips of two launches; from 13 tokens on the vector instructions of
-// one unpacking per pair, and one expert read once per pair and XCD.  (k_digit_rows unpacks once per two tokens of a
-// dispatch block, but most blocks hold one, and its 170 registers leave one workgroup per CU.)
+// one unpacking per pair, and one expert read once per pair and XCD.  (k_digit_rows unpacks once per four or eight tokens
+// of a dispatch block, but below the matrix-core widths most blocks hold one or two, and its registers leave one
+// workgroup per CU.)
 // Routed experts of the model geometry, us: one token 31 -> 16, three 33 -> 26, 45 213 -> 171 (k_digit_rows -> this).
 // ------------------------------------------------------------------------------------------------
 constexpr int kPairTiles = 4;  // tiles a wavefront takes at most
@@ -591,7 +577,9 @@ static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, c
 
 template <int NM>
 static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
-  if (mode == kRowsBlock) return rows_quant<kRowsBlock, NM, kRowsBlockTokens, 1, kRowsRoutedTiles>(quant, tail, grid, s, a);
+  if (mode == kRowsBlock)
+    return nt == 4 ? rows_quant<kRowsBlock, NM, 4, 1, kRowsRoutedTiles>(quant, tail, grid, s, a)
+                   : rows_quant<kRowsBlock, NM, 4, 2, kRowsRoutedTiles>(quant, tail, grid, s, a);
   return mt == 1 ? rows_shared<NM, 1>(nt, quant, tail, grid, s, a) : rows_shared<NM, kRowsMaxTiles>(nt, quant, tail, grid, s, a);
 }
 
@@ -676,6 +664,10 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
     const size_t t = k->g.max_tokens, passes = k->force_community ? t : (t + 7) / 8, each = (t + passes - 1) / passes;
     nt = each == 1 ? 1 : each == 2 ? 2 : each <= 4 ? 4 : 8;
     units = (t + nt - 1) / nt;
+  } else {
+    // tokens of a block per pass over an expert's rows: four, or eight where an expert has six on average (a pass for two,
+    // as it was: 256 tokens 797 us, now 549; 1024 tokens 2724, now 1612)
+    nt = k->g.max_tokens * k->g.experts_per_token >= 6 * k->g.num_experts ? 8 : 4;
   }
   const int per_class = std::max(1, (nt > 4 ? 4 : 8) / a.classes);  // (as the kernel has it: nt > 4 is two teams)
   int mt = 1;

@@ -287,10 +287,10 @@ def test_fused_shared_is_bit_identical_to_separate_launches(oracle, X, max_token
     assert torch.all(sh8 == 0)
 
 
-@pytest.mark.parametrize("geom,max_tokens,tokens", [("model", 8, 8), ("model", 32, 29), ("model", 40, 37), ("small", 40, 40), ("small", 5, 5)])
+@pytest.mark.parametrize("geom,max_tokens,tokens", [("model", 8, 8), ("model", 32, 29), ("model", 40, 37), ("small", 40, 40), ("small", 5, 5), ("small", 63, 61)])
 def test_pair_kernel_equals_the_dispatch_block_kernel(oracle, X, geom, max_tokens, tokens):
-    # below the matrix-core widths a unit is one (token, k) pair; force_community takes the dispatch blocks, two tokens
-    # per pass over an expert's rows: same bits, both stages
+    # a unit is one (token, k) pair in the exact regime, and wherever few tokens select an expert; force_community takes the
+    # dispatch blocks, four or eight tokens per pass over an expert's rows: same bits, both stages
     import torch
 
     if geom == "model":
@@ -305,6 +305,7 @@ def test_pair_kernel_equals_the_dispatch_block_kernel(oracle, X, geom, max_token
     for plain in (False, True):
         k = X.MoeKernels(g)
         k.force_community(plain)
+        k.set_exact_decode_regime(not plain)
         b = k.buffers()
         k.set_valid_tokens(b, tokens)
         lg = torch.zeros(max_tokens, g.num_experts, device="cuda")

@@ -44,6 +44,7 @@ def test_routed_experts(fmt, hidden, inter):
         for blocks in (False, True) if tokens > 4 else (False,):
             k = X.MoeKernels(X.MoeGeometry(E, K, hidden, inter, 32, tokens))
             k.force_community(blocks)
+            k.set_exact_decode_regime(not blocks)    # (pairs whatever the width)
             b = k.buffers()
             k.set_valid_tokens(b, live)
             k.route_and_dispatch(b, logits)
