@@ -351,6 +351,9 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
   return g.hidden > 2048 || (g.intermediate > 2048 && g.hidden * g.intermediate >= ((size_t)10 << 20));
 }
 
+constexpr size_t kDigitScratchRows = 8192;  // intermediate rows of the routed experts whose digits the scratch holds
+constexpr size_t kSharedDigitTokens = 64;   // the same of a single matrix, and its activation rows
+
 template <typename T>
 static int alloc_zeros(T** p, size_t n, hipStream_t s, size_t* total) {
   *p = nullptr;
@@ -399,16 +402,23 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->partial, b->n_partial);
   A(&b->shared_inter, b->n_shared_inter);
   const size_t nsb_h = digit_superblocks(g.hidden), nsb_i = digit_superblocks(g.intermediate);
-  A(&b->x_d, routed ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
-  A(&b->x_e, routed ? g.max_tokens * nsb_h : 0);
   A(&b->inter, routed ? sorted * g.intermediate : 0);
-  A(&b->inter_d, (routed ? sorted : 0) * nsb_i * kSbDigitBytes);
-  A(&b->inter_e, (routed ? sorted : 0) * nsb_i * 16);
-  const bool shared_long = shared_on_digits(g);
-  A(&b->shared_x_d, shared_long ? g.max_tokens * nsb_h * kSbDigitBytes : 0);
-  A(&b->shared_x_e, shared_long ? g.max_tokens * nsb_h : 0);
-  A(&b->shared_inter_d, g.max_tokens * nsb_i * kSbDigitBytes);
-  A(&b->shared_inter_e, g.max_tokens * nsb_i * 16);
+  // Digits: scratch of a bounded number of rows, which wide passes of the fp32 regimes go through in parts (an 8192-token
+  // handle of the model, or a 2048-token one of the dense sibling, serves its passes on the matrix cores and would
+  // carry 360 and 230 MB that nobody reads).
+  b->n_digit_rows = routed ? std::min(sorted, kDigitScratchRows) : 0;
+  A(&b->inter_d, b->n_digit_rows * nsb_i * kSbDigitBytes);
+  A(&b->inter_e, b->n_digit_rows * nsb_i * 16);
+  // (at the matrix-core widths the activations' lie in `partial` until the down launch writes it, where they fit)
+  const size_t x_digits = routed ? g.max_tokens * nsb_h * kSbDigitBytes : 0, x_scales = routed ? g.max_tokens * nsb_h : 0;
+  const bool x_apart = !wide || x_digits + x_scales * sizeof(float) > b->n_partial * sizeof(float);
+  A(&b->x_d, x_apart ? x_digits : 0);
+  A(&b->x_e, x_apart ? x_scales : 0);
+  const size_t shared_rows = shared_on_digits(g) ? std::min(g.max_tokens, kSharedDigitTokens) : 0;
+  A(&b->shared_x_d, shared_rows * nsb_h * kSbDigitBytes);
+  A(&b->shared_x_e, shared_rows * nsb_h);
+  A(&b->shared_inter_d, shared_rows * nsb_i * kSbDigitBytes);
+  A(&b->shared_inter_e, shared_rows * nsb_i * 16);
   // matrix-core staging: only passes wide enough to take that regime pay for it
   A(&b->x_h, (wide && mma) ? g.max_tokens * g.hidden : 0);
   A(&b->inter_h, (wide && mma && routed) ? sorted * g.intermediate : 0);
@@ -657,8 +667,8 @@ static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) 
 
 // One (token, k) pair per unit while fewer than four select an expert on average, and in the exact regime; dispatch blocks
 // beyond, which read and unpack an expert's rows once per four or eight tokens.  Routed experts, us, pairs / blocks: the
-// model's 256 experts, top 8, 32 tokens 130 / 165, 45: 171 / 198, 63: 224 / 237, 64: 236 / 244, 256: 792 / 549, 1024:
-// 3049 / 1612; 64 experts, top 4, hidden 1024: 45 tokens 51 / 70, 256: 199 / 150.
+// model's 256 experts, top 8, 32 tokens 130 / 165, 45: 171 / 198, 63: 224 / 237, 64: 236 / 244, 256: 792 / 565, 1024:
+// 3091 / 1638; 64 experts, top 4, hidden 1024: 45 tokens 51 / 70, 256: 199 / 150.
 // force_community keeps the blocks, where there are any, for comparison: same bits.
 constexpr size_t kPairsPerExpert = 4;
 static bool routed_by_pairs(const xabe_moe_kernels* k) {
@@ -688,11 +698,7 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   up_a.w_bytes = gate.len;
   up_a.expert_bytes = expert_elems / xabe_expert_quant_block_elements(gate.quant) * xabe_expert_quant_block_bytes(gate.quant);
   up_a.x = x;
-  up_a.xd = b->x_d;
-  up_a.xe = b->x_e;
   up_a.out = b->inter;
-  up_a.out_d = b->inter_d;
-  up_a.out_e = b->inter_e;
   up_a.K = (int)g.hidden;
   up_a.n_rows = (int)g.intermediate;
   RowsArgs down_a = rows_args(k, b);
@@ -705,27 +711,44 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   down_a.out = b->partial;
   down_a.K = (int)g.intermediate;
   down_a.n_rows = (int)g.hidden;
-  if (pairs) {
-    ExpertArgs sh_up = base_args(k, b), sh_down = sh_up;
-    if (ride) {
-      shared_up_args(sh_up, k, b, ride->gate, ride->up, x);
-      shared_down_args(sh_down, k, b, ride->down, ride->out);
-    }
-    // (4096 pairs a launch: at the widths of the exact regime a grid may not hold more)
-    constexpr size_t kPairsPerLaunch = 4096;
-    for (size_t first = 0; first < units; first += kPairsPerLaunch) {
-      const size_t n = std::min(kPairsPerLaunch, units - first);
-      up_a.unit0 = down_a.unit0 = (int)first;
-      if (stages & 1) XABE_TRY(launch_digit_pairs(k, gate.quant, 2, up_a, n, s, ride ? &sh_up : nullptr, ride ? ride->gate.quant : -1));
-      if (stages & 2) XABE_TRY(launch_digit_pairs(k, down.quant, 1, down_a, n, s, ride ? &sh_down : nullptr, ride ? ride->down.quant : -1));
-    }
-    return XABE_OK;
+  // the intermediate rows' digits: written by gate/up where the scratch holds all of them, else made part by part
+  const size_t unit_rows = pairs ? 1 : g.block_size, per_part = std::max<size_t>(1, b->n_digit_rows / unit_rows);
+  const bool whole = units <= per_part;
+  if (whole) {
+    up_a.out_d = b->inter_d;
+    up_a.out_e = b->inter_e;
+  }
+  ExpertArgs sh_up = base_args(k, b), sh_down = sh_up;
+  if (ride) {
+    shared_up_args(sh_up, k, b, ride->gate, ride->up, x);
+    shared_down_args(sh_down, k, b, ride->down, ride->out);
   }
   if (stages & 1) {
-    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->x_d, b->x_e));
-    XABE_TRY(launch_digit_rows(k, kRowsBlock, gate.quant, 2, up_a, units, s));
+    if (pairs) {
+      for (size_t first = 0; first < units; first += per_part) {  // (a grid of all units might not be a valid one)
+        up_a.unit0 = (int)first;
+        XABE_TRY(launch_digit_pairs(k, gate.quant, 2, up_a, std::min(per_part, units - first), s, ride ? &sh_up : nullptr, ride ? ride->gate.quant : -1));
+      }
+    } else {
+      const size_t nsb = digit_superblocks(g.hidden);
+      uint8_t* xd = b->x_d ? b->x_d : reinterpret_cast<uint8_t*>(b->partial);
+      float* xe = b->x_d ? b->x_e : reinterpret_cast<float*>(xd + g.max_tokens * nsb * kSbDigitBytes);
+      XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, xd, xe));
+      up_a.xd = xd;
+      up_a.xe = xe;
+      XABE_TRY(launch_digit_rows(k, kRowsBlock, gate.quant, 2, up_a, units, s));
+    }
   }
-  return stages & 2 ? launch_digit_rows(k, kRowsBlock, down.quant, 1, down_a, units, s) : XABE_OK;
+  if (!(stages & 2)) return XABE_OK;
+  for (size_t first = 0; first < units; first += per_part) {
+    const size_t n = std::min(per_part, units - first);
+    down_a.unit0 = (int)first;
+    if (!whole)
+      XABE_TRY(launch_digitize_groups(s, b->inter + first * unit_rows * g.intermediate, g.intermediate, n * unit_rows, b->inter_d, b->inter_e));
+    if (pairs) XABE_TRY(launch_digit_pairs(k, down.quant, 1, down_a, n, s, ride ? &sh_down : nullptr, ride ? ride->down.quant : -1));
+    else XABE_TRY(launch_digit_rows(k, kRowsBlock, down.quant, 1, down_a, n, s));
+  }
+  return XABE_OK;
 }
 
 int xabe_moe_grouped_forward_partial(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, xabe_quant_tensor gate,
@@ -777,37 +800,38 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
   return XABE_OK;
 }
 
-// gate/up and down of a single-expert stack on the digit contraction, from the activation digits in b->shared_x_d
-// (x: the rows themselves)
+// gate/up and down of a single-expert stack on the digit contraction, for tokens first .. first + n - 1, whose activation
+// digits are in b->shared_x_d (x: the rows of all tokens)
 static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                         xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out,
+                         xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out, size_t first, size_t n,
                          const float* residual = nullptr, float* l_out = nullptr) {
   const xabe_moe_geometry& g = k->g;
   RowsArgs a = rows_args(k, b);
+  a.unit0 = (int)first;
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
   a.w1 = static_cast<const uint8_t*>(up.bytes);
   a.w_bytes = gate.len;
-  a.x = x;
+  a.x = x + first * g.hidden;
   a.xd = b->shared_x_d;
   a.xe = b->shared_x_e;
-  a.out = b->shared_inter;
+  a.out = b->shared_inter + first * g.intermediate;
   a.out_d = b->shared_inter_d;
   a.out_e = b->shared_inter_e;
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
-  XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, 0, s));
+  XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, n, s));
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.w_bytes = down.len;
-  a.x = b->shared_inter;
+  a.x = b->shared_inter + first * g.intermediate;
   a.xd = b->shared_inter_d;
   a.xe = b->shared_inter_e;
-  a.out = out;
-  a.residual = residual;
-  a.l_out = l_out;
+  a.out = out + first * g.hidden;
+  a.residual = residual ? residual + first * g.hidden : nullptr;
+  a.l_out = l_out ? l_out + first * g.hidden : nullptr;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  return launch_digit_rows(k, kRowsShared, down.quant, 1, a, 0, s);
+  return launch_digit_rows(k, kRowsShared, down.quant, 1, a, n, s);
 }
 
 // The same on the pair kernel: a token is a unit of expert 0.  Up to four tokens it saves the launch that makes the digits
@@ -849,8 +873,12 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   const xabe_moe_geometry& g = k->g;
   if (shared_on_digits(g)) {
     if (shared_by_pairs(k)) return shared_pairs(k, s, b, gate, up, down, x, out);
-    XABE_TRY(launch_digitize_rows(s, x, g.hidden, g.max_tokens, b->shared_x_d, b->shared_x_e));
-    return shared_digits(k, s, b, gate, up, down, x, out);
+    for (size_t first = 0; first < g.max_tokens; first += kSharedDigitTokens) {
+      const size_t n = std::min(kSharedDigitTokens, g.max_tokens - first);
+      XABE_TRY(launch_digitize_rows(s, x + first * g.hidden, g.hidden, n, b->shared_x_d, b->shared_x_e));
+      XABE_TRY(shared_digits(k, s, b, gate, up, down, x, out, first, n));
+    }
+    return XABE_OK;
   }
   const size_t units = (g.max_tokens + 1) / 2;
   ExpertArgs a = base_args(k, b);
@@ -860,7 +888,7 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   return launch_expert(k, down.quant, 1, a, units, s);
 }
 
-// The dense block's fp32 path: the norm launch writes the digits, down adds the residual; three launches.
+// The dense block's fp32 path: the norm launch writes the digits, down adds the residual; three launches (per 64 tokens).
 int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                            xabe_quant_tensor up, xabe_quant_tensor down, const float* post_norm, float eps,
                            const float* residual, float* normed, float* ffn_out, float* l_out, bool* launched) {
@@ -870,10 +898,13 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
   if (!shared_on_digits(g)) return XABE_OK;
   if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(post_norm)) % 16 != 0)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "rms_norm: x, weight and out must be 16-byte aligned");
-  hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)g.max_tokens), dim3(256), 0, s, residual, post_norm, normed, (int)g.hidden,
-                     eps, b->shared_x_d, b->shared_x_e);
-  XABE_HIP_TRY(hipGetLastError());
-  XABE_TRY(shared_digits(k, s, b, gate, up, down, normed, ffn_out, residual, l_out));
+  for (size_t first = 0; first < g.max_tokens; first += kSharedDigitTokens) {
+    const size_t n = std::min(kSharedDigitTokens, g.max_tokens - first), at = first * g.hidden;
+    hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)n), dim3(256), 0, s, residual + at, post_norm, normed + at, (int)g.hidden,
+                       eps, b->shared_x_d, b->shared_x_e);
+    XABE_HIP_TRY(hipGetLastError());
+    XABE_TRY(shared_digits(k, s, b, gate, up, down, normed, ffn_out, first, n, residual, l_out));
+  }
   *launched = true;
   return XABE_OK;
 }

@@ -24,7 +24,7 @@ struct RowsArgs {
   const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes] (pairs' gate/up makes its own)
   const float* xe;           // their scales: gate/up [row][superblock], down [row][superblock][16] (by group)
   float* out;                // [row][n_rows]
-  uint8_t* out_d;            // nm = 2: digits of the output rows
+  uint8_t* out_d;            // nm = 2: digits of the output rows (null: not written)
   float* out_e;
   const float* residual;     // with l_out: l_out = out + residual
   float* l_out;
@@ -34,7 +34,8 @@ struct RowsArgs {
   const int* sorted_token_ids;
   const int* expert_ids;
   int K, n_rows, top_k, block_size;
-  int unit0;  // pairs: the first of this launch
+  int unit0;  // the first pair, block or (a single matrix, whose pointers are that token's) token of this launch; digits of
+              // intermediate rows are counted from its rows
   // filled in by launch_digit_rows
   int nsb, out_nsb, classes, tile_rows, n_tiles;
   int units, shares, xcd_units;  // pairs (xcd_units: units of one share side by side, one per XCD; 0: plain order)
@@ -83,7 +84,8 @@ __device__ __forceinline__ void store_digit_group(float v, int row, uint8_t* xd,
 // host side
 int digit_rows_configure();
 int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
-// `units`: dispatch blocks (block); token chunks are counted here
+int launch_digitize_groups(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
+// `units`: dispatch blocks, or the tokens of a single matrix
 int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s);
 // One (token, k) pair per unit, straight from topk_ids: pairs a.unit0 .. a.unit0 + units - 1.  `shared`: the shared
 // expert's rows of the same shape (whole superblocks, at most 2048 elements) ride along.

@@ -35,6 +35,18 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
   if (lane == 0) xe[i] = scale;
 }
 
+// Digits of fp32 rows, scaled by groups of sixteen (what a gate/up launch writes where the scratch holds all of its rows).
+__global__ void __launch_bounds__(256) k_digitize_groups(const float* __restrict__ x, int K, int nsb, int rows, uint8_t* __restrict__ xd,
+                                                         float* __restrict__ xe) {
+  const int i = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)__lane_id();
+  if (i >= rows * nsb) return;
+  const int row = i / nsb, sb = i % nsb, at = sb * 64 + lane;
+  const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(at, K / 4 - 1)];
+  const bool in = 4 * at < K;
+  const float v[4] = {in ? f.x : 0.0f, in ? f.y : 0.0f, in ? f.z : 0.0f, in ? f.w : 0.0f};
+  digitize_quads_by_group(v, xd + (size_t)i * kSbDigitBytes, xe + (size_t)i * 16);
+}
+
 // Tiles per wavefront of a dispatch block, the next one's rows in flight while one is multiplied.
 constexpr int kRowsRoutedTiles = 4;
 
@@ -58,17 +70,17 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
   constexpr int TG = (NT + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
   const int lane = (int)__lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int valid = *a.valid_tokens;
+  const int valid = *a.valid_tokens - (MODE == kRowsShared ? a.unit0 : 0);
   // ---- the unit's weights and token rows
   size_t e_off = 0;
   int n_tok;
   const int* slots = nullptr;
   size_t slot0 = 0;
   if constexpr (MODE == kRowsBlock) {
-    const int e = a.expert_ids[blockIdx.y];
+    const int block = a.unit0 + (int)blockIdx.y, e = a.expert_ids[block];
     if (e < 0) return;
     e_off = (size_t)e * a.expert_bytes;
-    slot0 = (size_t)blockIdx.y * a.block_size;
+    slot0 = (size_t)block * a.block_size;
     slots = a.sorted_token_ids + slot0;
     n_tok = a.block_size;
   } else {
@@ -77,6 +89,8 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     n_tok = min(kTokens, valid - (int)slot0);
   }
   const int sentinel = valid * a.top_k;
+  // rows are counted from here among the digits
+  const int d_row0 = MODE == kRowsBlock && NM == 1 ? a.unit0 * a.block_size : 0;
 
   // ---- this wavefront's class and tiles
   const int team = wave / kTeam, member = wave % kTeam, t0 = team * NT;             // (the team's tokens: t0 ..)
@@ -150,13 +164,13 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     auto request_x = [&](int sb, int buf) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const uint8_t* from = a.xd + ((size_t)x_row[t] * nsb + sb) * kSbDigitBytes;
+        const uint8_t* from = a.xd + ((size_t)(x_row[t] - d_row0) * nsb + sb) * kSbDigitBytes;
         lds_dma_16(from, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes);
         if (lane < 32) lds_dma_16(from + 1024, (uint32_t)lane * 16, d_lds + t * kSbDigitBytes + 1024);
       }
       if constexpr (kScale == kGroups) {
         if (lane < 4 * NT)  // (64 bytes per token)
-          lds_dma_16(a.xe, ((uint32_t)x_row_l * nsb + sb) * kSbScaleBytes + (lane & 3) * 16, e_lds + buf * L::kScales);
+          lds_dma_16(a.xe, ((uint32_t)(x_row_l - d_row0) * nsb + sb) * kSbScaleBytes + (lane & 3) * 16, e_lds + buf * L::kScales);
       } else {
 #pragma unroll
         for (int t = 0; t < NT; ++t) e_next[t] = a.xe[(size_t)x_row[t] * nsb + sb];
@@ -292,7 +306,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
         const float v = silu_f(total(tl, t, col)) * total(tl, t, col + 16);
         if (live) a.out[o_row * a.n_rows + row] = v;
         // sixteen consecutive threads hold one group of the next contraction's activations
-        store_digit_group(v, row, a.out_d + o_row * a.out_nsb * kSbDigitBytes, a.out_e + o_row * a.out_nsb * 16, live);
+        if (a.out_d) store_digit_group(v, row, a.out_d + o_row * a.out_nsb * kSbDigitBytes, a.out_e + o_row * a.out_nsb * 16, live);
       } else {
         const float v = scale * total(tl, t, col);
         if (live) {
@@ -427,7 +441,7 @@ __global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a,
   float4 quad = {0.0f, 0.0f, 0.0f, 0.0f};
   auto load_x = [&](int sb) __attribute__((always_inline)) {
     if constexpr (NM == 2) quad = reinterpret_cast<const float4*>(x_f)[min(sb * 64 + lane, a.K / 4 - 1)];
-    else x.load(a.xd + (x_row * nsb + sb) * kSbDigitBytes, a.xe + (x_row * nsb + sb) * 16);
+    else x.load(a.xd + ((size_t)u * nsb + sb) * kSbDigitBytes, a.xe + ((size_t)u * nsb + sb) * 16);
   };
   Dma dma;  // (its lane offsets are ready before the expert is known)
   if (any) {
@@ -505,7 +519,7 @@ __global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a,
       const float v = silu_f(total(tl, col)) * total(tl, col + 16);
       a.out[(size_t)pair * a.n_rows + row] = v;
       // sixteen consecutive threads hold one group of the next contraction's activations
-      store_digit_group(v, row, a.out_d + (size_t)pair * a.out_nsb * kSbDigitBytes, a.out_e + (size_t)pair * a.out_nsb * 16, true);
+      if (a.out_d) store_digit_group(v, row, a.out_d + (size_t)u * a.out_nsb * kSbDigitBytes, a.out_e + (size_t)u * a.out_nsb * 16, true);
     } else {
       a.out[(size_t)pair * a.n_rows + row] = weight * total(tl, col);
     }
@@ -617,6 +631,13 @@ int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, u
   return XABE_OK;
 }
 
+int launch_digitize_groups(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe) {
+  const size_t nsb = digit_superblocks(K), n = rows * nsb;
+  hipLaunchKernelGGL(k_digitize_groups, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
 static void rows_shape(RowsArgs& a, int quant, int nm) {
   const size_t be = xabe_expert_quant_block_elements(quant), bb = xabe_expert_quant_block_bytes(quant);
   a.nsb = (int)digit_superblocks((size_t)a.K);
@@ -661,12 +682,12 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
   if (mode == kRowsShared) {
     // tokens per pass over the weights: all of them up to eight, equal passes beyond
     // (force_community: one, for comparison: the same bits)
-    const size_t t = k->g.max_tokens, passes = k->force_community ? t : (t + 7) / 8, each = (t + passes - 1) / passes;
+    const size_t t = units, passes = k->force_community ? t : (t + 7) / 8, each = (t + passes - 1) / passes;
     nt = each == 1 ? 1 : each == 2 ? 2 : each <= 4 ? 4 : 8;
     units = (t + nt - 1) / nt;
   } else {
     // tokens of a block per pass over an expert's rows: four, or eight where an expert has six on average (a pass for two,
-    // as it was: 256 tokens 797 us, now 549; 1024 tokens 2724, now 1612)
+    // as it was: 256 tokens 797 us, now 565; 1024 tokens 2724, now 1638)
     nt = k->g.max_tokens * k->g.experts_per_token >= 6 * k->g.num_experts ? 8 : 4;
   }
   const int per_class = std::max(1, (nt > 4 ? 4 : 8) / a.classes);  // (as the kernel has it: nt > 4 is two teams)

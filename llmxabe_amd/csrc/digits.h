@@ -163,6 +163,26 @@ __device__ __forceinline__ float digitize_quads(const float (&x)[4], uint8_t* ba
   return digit_scale(mag, e, __builtin_amdgcn_ballot_w64(inexact) != 0);
 }
 
+// The same with the scale of every group, sixteen at `scales`.
+__device__ __forceinline__ int scale_group_index(int pos);
+__device__ __forceinline__ void digitize_quads_by_group(const float (&x)[4], uint8_t* base, float* scales) {
+  const int lane = (int)__lane_id();
+  int m = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m = max(m, (int)(__builtin_bit_cast(uint32_t, x[i]) & 0x7fffffffu));
+  m = max(m, dpp_i<0xB1>(m));  // (four lanes hold a group)
+  m = max(m, dpp_i<0x4E>(m));
+  const int e = digit_exponent((uint32_t)m);
+  uint32_t plane[6];
+  bool inexact = false;
+  digitize4(x, digit_shift(e), plane, inexact);
+  uint8_t* d = base + digit_group_offset(lane >> 2) + 4 * (lane & 3);
+#pragma unroll
+  for (int p = 0; p < 6; ++p) *reinterpret_cast<uint32_t*>(d + 16 * p) = plane[p];
+  const bool any = (__builtin_amdgcn_ballot_w64(inexact) >> (lane & 60) & 15) != 0;
+  if ((lane & 3) == 0) scales[scale_group_index(lane >> 2)] = digit_scale((uint32_t)m, e, any);
+}
+
 // Where group `pos` (elements 16 pos .. 16 pos + 15 of its superblock) lies among the digits and the scales.
 __device__ __forceinline__ int digit_group_offset(int pos) {
   const int h = pos >> 3, s = (pos >> 1) & 3, l = pos & 1;

@@ -165,9 +165,11 @@ struct xabe_moe_buffers {
   int32_t* valid_tokens;
   int32_t valid_published;  // what `valid_tokens` holds (0 after allocation)
   int32_t valid_host;       // source of the host-to-device copy that publishes a new count
-  // digits and scales (digits.h) of what the fp32 row contractions read.  Routed experts: the activation rows and
-  // the intermediate rows (one per slot); shared expert: the same of its own (one per token), so that the two may run
-  // on two streams, with rows of their own.
+  // digits and scales (digits.h) of what the fp32 row contractions read.  Routed experts: the activation rows (null at
+  // matrix-core widths where `partial` has room for them) and up to n_digit_rows intermediate rows; shared expert, where
+  // its rows go through digits: the same of its own, up to 64 tokens, so that the two may run on two streams, with rows of
+  // their own.
+  size_t n_digit_rows;
   uint8_t *x_d, *inter_d, *shared_x_d, *shared_inter_d;
   float *x_e, *inter_e, *shared_x_e, *shared_inter_e;
   float* inter;         // [slot][intermediate]: the routed intermediate rows
