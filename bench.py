@@ -50,7 +50,7 @@ def source_digest():
     import hashlib
 
     h = hashlib.sha256()
-    for name in ("decode_block.hip", "decode_kernels.h", "device_common.h", "route_device.h"):
+    for name in ("decode_block.hip", "decode_kernels.h", "device_common.h", "digit_rows.h", "digits.h", "route_device.h"):
         with open(os.path.join(ROOT, "llmxabe_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]

@@ -577,7 +577,7 @@ int xabe_moe_route_and_dispatch(const xabe_moe_kernels* k, void* stream, xabe_mo
   if (!k || !b) return set_error(XABE_ERR_INVALID_ARGUMENT, "route_and_dispatch: null handle");
   XABE_TRY(require_routed(b, "route_and_dispatch"));
   XABE_TRY(xabe_moe_route(k, stream, b, logits, logits_len));
-  if (flat_regime(k)) return XABE_OK;  // the flat kernels read topk_ids directly
+  if (flat_regime(k)) return XABE_OK;  // units of one pair read topk_ids directly
   return xabe_moe_build_dispatch(k, stream, b);
 }
 
@@ -604,16 +604,10 @@ int xabe::route_planes_and_dispatch(const xabe_moe_kernels* k, void* stream, xab
 }
 
 // ------------------------------------------------------------------ expert contractions
-static ExpertArgs base_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
+static ExpertArgs base_args(const xabe_moe_buffers* b) {
   ExpertArgs a;
   memset(&a, 0, sizeof(a));
   a.valid_tokens = b->valid_tokens;
-  a.topk_ids = b->topk_ids;
-  a.topk_weights = b->topk_weights;
-  a.sorted_token_ids = b->sorted_token_ids;
-  a.expert_ids = b->expert_ids;
-  a.top_k = (int)k->g.experts_per_token;
-  a.block_size = (int)k->g.block_size;
   return a;
 }
 
@@ -718,7 +712,7 @@ static int routed_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
     up_a.out_d = b->inter_d;
     up_a.out_e = b->inter_e;
   }
-  ExpertArgs sh_up = base_args(k, b), sh_down = sh_up;
+  ExpertArgs sh_up = base_args(b), sh_down = sh_up;
   if (ride) {
     shared_up_args(sh_up, k, b, ride->gate, ride->up, x);
     shared_down_args(sh_down, k, b, ride->down, ride->out);
@@ -881,7 +875,7 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
     return XABE_OK;
   }
   const size_t units = (g.max_tokens + 1) / 2;
-  ExpertArgs a = base_args(k, b);
+  ExpertArgs a = base_args(b);
   shared_up_args(a, k, b, gate, up, x);
   XABE_TRY(launch_expert(k, gate.quant, 2, a, units, s));
   shared_down_args(a, k, b, down, out);
@@ -1048,7 +1042,7 @@ int xabe::router_logits_biased(const xabe_moe_kernels* k, void* stream, const xa
   XABE_TRY(check_len("logits", g.max_tokens * g.num_experts, logits_len));
   if (router_gemm_supported(k, b, fmt))
     return launch_router_gemm(k, as_stream(stream), b, router, fmt, normed, logits, bias, bias_added, sum_deferred);
-  ExpertArgs a = base_args(k, b);
+  ExpertArgs a = base_args(b);
   a.w0 = static_cast<const uint8_t*>(router);
   a.x = normed;
   a.out = logits;

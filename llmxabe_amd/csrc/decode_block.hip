@@ -18,12 +18,12 @@
 //                        projections (and, at few tokens, the shared one), summed in k order, gated, combined with
 //                        the residual.  No partial buffer, no reduction pass.
 //
-// The routed contractions are pair_dot's (digits.h), whose values are k_digit_rows' bit for bit; routing, norm, router
+// The routed contractions are pair_dot's (digits.h), as are k_digit_pairs', and sb_dot's in k_digit_rows bit for bit; routing, norm, router
 // and shared expert are the per-row device functions of the multi-launch path.  So the outputs are bit-identical to that
 // path: the batch-invariance contract.  One multiply-add and one conversion per weight on the vector ALU, which this
-// replaces, made B 95 and C 52 us at 32 tokens; the digit form takes 71 and 39 (us per block, same box: 13 tokens
-// 96 -> 79, 32: 162 -> 131; 45 tokens, then ten launches, 252 -> 173; three tokens 31.6 both; one token 21.2 -> 21.8,
-// whose routed contractions wait for one more hop through LDS).  What bounds B and C now at 32 tokens: ~330 vector
+// replaces, made B 95 and C 52 us at 32 tokens; the digit form takes 77 and 42 (us per block, same box: 13 tokens
+// 96 -> 85, 32: 162 -> 138; 45 tokens, then ten launches, 252 -> 178; three tokens 31.6 -> 32.1; one token 21.2 -> 21.0,
+// with its rows straight into registers; four digits instead of six, which lose bits beside outliers, took 71 and 39).  What bounds B and C now at 32 tokens: ~330 vector
 // instructions per (token, row tile, pair of superblocks), about half of the launch, and one expert read once per
 // selection and XCD rather than once.
 #include <string.h>
@@ -312,7 +312,8 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// B: grid = max_tokens * top_k * tiles_g.  A tile is 4 wavefronts x DEPTH steps x RPS rows.
+// B: grid = max_tokens * top_k * shares of the row tiles (in wide batches padded to whole rounds of the XCDs, and the
+// shared expert's down projection behind them).
 // ------------------------------------------------------------------------------------------------
 // The routing launch of wider batches: one wavefront per token (route_one_token, the stand-alone routing kernel's
 // body), one token per workgroup so that the tokens spread over the chip.
@@ -547,11 +548,12 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = (int)__lane_id(), quarter = lane >> 4;
   const int tile0 = share * a.share_d;  // hidden is a multiple of kRows * share_d
-  const float gate = a.gate_out[t];
-  // what the thread's output row needs besides the sums, requested with round one
+  // what the thread's output row needs besides the sums: requested with round one where the launch is a single round of
+  // workgroups, at the end where others are at work meanwhile (held all along they spill; 13 tokens 504 -> 499 us)
+  float gate = SHARED ? a.gate_out[t] : 0.0f;
   const int n_out = a.share_d * kRows, n0 = min((int)threadIdx.x, n_out - 1);
   const size_t o0 = (size_t)t * a.H + (size_t)tile0 * kRows;  // (a share's rows are consecutive)
-  float sh = SHARED ? 0.0f : a.shexp[o0 + n0], res = a.residual[o0 + n0];
+  float sh = 0.0f, res = SHARED ? a.residual[o0 + n0] : 0.0f;
   if (SHARED && wave >= a.top_k) {
     constexpr int RPS = kRows / 4, G = 64 / RPS;
     const LaneGeom gs = lane_geom<SQ>();
@@ -619,13 +621,14 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
     }
   }
   __syncthreads();
+  if constexpr (!SHARED) gate = a.gate_out[t];
   // rows kRows * i + r of the share: the routed sum in selection order, shared expert, gate, residual
   for (int n = (int)threadIdx.x; n < n_out; n += (int)blockDim.x) {
     const int i = n / kRows, row = n % kRows;
     const size_t o = o0 + n;
-    if (n >= (int)blockDim.x) res = a.residual[o];
+    if (!SHARED || n >= (int)blockDim.x) res = a.residual[o];
     if constexpr (SHARED) sh = s_part[i][kMaxTopK + SHARED - 1][row], a.shexp[o] = sh;
-    else if (n >= (int)blockDim.x) sh = a.shexp[o];
+    else sh = a.shexp[o];
     float r = 0.0f;
 #pragma unroll
     for (int j = 0; j < kMaxTopK; ++j)

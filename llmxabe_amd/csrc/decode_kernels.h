@@ -73,64 +73,23 @@ __device__ __forceinline__ int lane_koff(const LaneGeom& g, int k) {
   return ((g.lane % (64 / RPS)) + k * 64) * 32;
 }
 
-// How a kernel obtains its activations and publishes its outputs.
-//   kXPlain: read fp32 rows as they are.
-//   kXNorm:  RMS-normalise on load, (x * inv_rms) * norm_weight -- the same two products, in the same
-//            order, as the stand-alone RMSNorm kernel, so the values are bit-identical to its output.
-//   kXCoherent: the rows were written earlier in the SAME launch by other workgroups; read them with
-//            agent-scope loads (sc1) so another XCD's writes are visible without a cache flush.
-constexpr int kXPlain = 0, kXNorm = 1, kXCoherent = 2;
-// kOPlain: ordinary stores.  kOCoherent: agent-scope stores (written through to the coherence point).
-constexpr int kOPlain = 0, kOCoherent = 1;
-
-struct XNorm {
-  float inv;              // 1 / sqrt(mean(x^2) + eps) of this token
-  const float* weight;    // norm weight, indexed like the row
-};
-
-__device__ __forceinline__ float2 load2_coherent(const float* p) {
-  const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-  return make_float2(__builtin_bit_cast(float, (uint32_t)v), __builtin_bit_cast(float, (uint32_t)(v >> 32)));
-}
-__device__ __forceinline__ void store_coherent(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Eight consecutive activations starting at xrow + off (off a multiple of 4).
-template <int XMODE>
-__device__ __forceinline__ void load8(const float* __restrict__ xrow, int off, const XNorm& nm, float (&v)[8]) {
-  if constexpr (XMODE == kXCoherent) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float2 a = load2_coherent(xrow + off + 2 * i);
-      v[2 * i] = a.x;
-      v[2 * i + 1] = a.y;
-    }
-  } else {
-    const float4 a = reinterpret_cast<const float4*>(xrow + off)[0];
-    const float4 b = reinterpret_cast<const float4*>(xrow + off)[1];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    if constexpr (XMODE == kXNorm) {
-      const float4 wa = reinterpret_cast<const float4*>(nm.weight + off)[0];
-      const float4 wb = reinterpret_cast<const float4*>(nm.weight + off)[1];
-      const float w[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = v[i] * nm.inv * w[i];
-    }
-  }
+__device__ __forceinline__ void load8(const float* __restrict__ xrow, int off, float (&v)[8]) {
+  const float4 a = reinterpret_cast<const float4*>(xrow + off)[0];
+  const float4 b = reinterpret_cast<const float4*>(xrow + off)[1];
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-template <int QUANT, int XMODE = kXPlain>
+template <int QUANT>
 __device__ __forceinline__ void load_x(const float* __restrict__ xrow, int koff, bool active, const LaneGeom& g,
-                                       float (&x)[32], float (&xs)[4], const XNorm& nm = XNorm{1.0f, nullptr}) {
+                                       float (&x)[32], float (&xs)[4]) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // Q6_K: run j of the lane's superblock unit; Q8_0 / fp32: the j-th eight of 32 consecutive elements
     const int off = QUANT == kQ6K ? koff + g.half * 128 + j * 32 + g.l8 * 8 : koff + j * 8;
-    if (active) load8<XMODE>(xrow, off, nm, v);
+    if (active) load8(xrow, off, v);
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[j * 8 + i] = v[i];
     if (QUANT == kQ6K) {
@@ -195,11 +154,11 @@ __device__ __forceinline__ void accum(const typename Fmt<QUANT>::Raw& r, const L
 // are split over the workgroup's four wavefronts.  KS > 0: steps per row, activations
 // in registers.  KS == 0: steps from K at run time, activations re-read per step.
 // ---------------------------------------------------------------------------------
-template <int QUANT, int KS, int RPS, int TC, int NM, int XMODE = kXPlain, int OMODE = kOPlain>
+template <int QUANT, int KS, int RPS, int TC, int NM>
 __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, int K,
                                             int n_rows, int tile0, int tile_rows,
                                             const float* const (&xrow)[TC], float* const (&out)[TC],
-                                            const float (&scale)[TC], const XNorm* norm = nullptr) {
+                                            const float (&scale)[TC]) {
   using F = Fmt<QUANT>;
   using Raw = typename F::Raw;
   constexpr int G = 64 / RPS;
@@ -219,7 +178,7 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
       active[k] = koff < K;
 #pragma unroll
       for (int t = 0; t < TC; ++t)
-        load_x<QUANT, XMODE>(xrow[t], koff, active[k], g, x[k][t], xs[k][t], XMODE == kXNorm ? norm[t] : XNorm{1.0f, nullptr});
+        load_x<QUANT>(xrow[t], koff, active[k], g, x[k][t], xs[k][t]);
     }
     auto load_item = [&](int row0, Raw (&r)[NM][KS]) {
 #pragma unroll
@@ -245,8 +204,7 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
 #pragma unroll
         for (int t = 0; t < TC; ++t) {
           const float v = NM == 2 ? silu_f(tot[0][t]) * tot[NM - 1][t] : scale[t] * tot[0][t];
-          if constexpr (OMODE == kOCoherent) store_coherent(&out[t][row], v);
-          else out[t][row] = v;
+          out[t][row] = v;
         }
       }
     };
@@ -285,7 +243,7 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
         float xs[TC][4];
 #pragma unroll
         for (int t = 0; t < TC; ++t)
-          load_x<QUANT, XMODE>(xrow[t], koff, act, g, x[t], xs[t], XMODE == kXNorm ? norm[t] : XNorm{1.0f, nullptr});
+          load_x<QUANT>(xrow[t], koff, act, g, x[t], xs[t]);
         const size_t off = (size_t)row0 * row_bytes + (size_t)k * F::kChunkBytes;
         Raw r0;
         load_raw<QUANT>(w0 + off, act, g, r0);
@@ -304,8 +262,7 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
 #pragma unroll
         for (int t = 0; t < TC; ++t) {
           const float v = NM == 2 ? silu_f(tot[0][t]) * tot[NM - 1][t] : scale[t] * tot[0][t];
-          if constexpr (OMODE == kOCoherent) store_coherent(&out[t][row0], v);
-          else out[t][row0] = v;
+          out[t][row0] = v;
         }
       }
     }
@@ -317,21 +274,14 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* __restrict__ w0, cons
 // a function of the geometry, the live token count is read from `valid_tokens`.
 // ---------------------------------------------------------------------------------
 struct ExpertArgs {
-  const uint8_t* w0;         // gate stack (NM=2) or down stack (NM=1)
-  const uint8_t* w1;         // up stack (NM=2) or unused
-  size_t expert_bytes;       // bytes of one expert in a stack (0 for a single-expert stack)
-  const float* x;            // activations: [token][K] (gate/up: normed; down: inter rows)
-  float* out;                // gate/up: inter [unit][n_rows]; down: partial/out [unit][n_rows]
-  const int* valid_tokens;   // device scalar
-  const int* topk_ids;       // [T][top_k]
-  const float* topk_weights; // [T][top_k]
-  const int* sorted_token_ids;
-  const int* expert_ids;
-  int K;                     // contraction length
-  int n_rows;                // output rows per expert
-  int top_k;
-  int block_size;
-  int tile_rows;             // rows per workgroup
+  const uint8_t* w0;       // gate (NM = 2) or the one matrix
+  const uint8_t* w1;       // up (NM = 2)
+  const float* x;          // activations: [token][K]
+  float* out;              // [token][n_rows]
+  const int* valid_tokens; // device scalar
+  int K;                   // contraction length
+  int n_rows;
+  int tile_rows;           // rows per workgroup
 };
 
 // Shared expert / dense MLP: every live token, no indirection, no routing weight

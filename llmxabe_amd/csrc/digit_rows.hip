@@ -1,5 +1,5 @@
 // The fp32 regimes' row contractions on the digit core (digits.h): quantized rows of one matrix, or of a gate/up pair
-// with SwiGLU between them, against the tokens of a work unit.  Replaces the reference's gemv / flat / tiled fp32
+// with SwiGLU between them, against the tokens of a work unit.  Replaces the reference's flat and tiled fp32
 // families (crates/xabe-cuda/src/kernels/moe.rs:2403-3124, :3425-3725, :4082-4227).
 //
 // A workgroup is eight wavefronts over the row tiles of its share (32 rows, or 16 gate and the 16 matching up rows).
@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a,
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        x.load_digits(w_slot);
+        x.template load<false>(w_slot, nullptr);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       }
     }

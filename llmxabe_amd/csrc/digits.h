@@ -628,18 +628,11 @@ struct PairDigits {
   v4i_t a[8];                // [4 l + s]: digits 0..3
   v4i_t z[4];                // [s]: digits 4 and 5 of l = 0, then of l = 1
   float4 e[WHOLE ? 1 : 2];   // the superblock's in .x, or [l], s = 0..3
-  // `xd`, `xe`: digits and scales of the activation superblock the lane's weights lie in
+  // `xd`, `xe`: digits and scales of the activation superblock the lane's weights lie in (SCALES false: the digits
+  // only; one function, because with the scales' loads in another the block's down launch spilled 9 more registers and 13
+  // tokens took 3 % longer)
+  template <bool SCALES = true>
   __device__ __forceinline__ void load(const uint8_t* xd, const float* xe) {
-    load_digits(xd);
-    if constexpr (WHOLE) {
-      e[0].x = *xe;
-    } else {
-      const int h = ((int)__lane_id() >> 4) & 1;
-#pragma unroll
-      for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
-    }
-  }
-  __device__ __forceinline__ void load_digits(const uint8_t* xd) {
     const int lane = (int)__lane_id(), q = lane >> 4, m = lane & 15, h = q & 1;
     const bool mine = (m >> 2) == q;
 #pragma unroll
@@ -653,6 +646,12 @@ struct PairDigits {
       for (int j = 0; j < 8; ++j) a[j] = *reinterpret_cast<const v4i_t*>(pa + (4 * (j & 3) + (j >> 2)) * kGroupBytes);
 #pragma unroll
       for (int s = 0; s < 4; ++s) z[s] = *reinterpret_cast<const v4i_t*>(pz + 4 * s * kGroupBytes);
+    }
+    if constexpr (SCALES && WHOLE) {
+      e[0].x = *xe;
+    } else if constexpr (SCALES) {
+#pragma unroll
+      for (int l = 0; l < 2; ++l) e[l] = reinterpret_cast<const float4*>(xe)[2 * h + l];
     }
   }
 };

@@ -1,5 +1,5 @@
-"""The decode-width block (max_tokens <= 32) regrouped into three launches against the same block with one
-launch per step (flat per-pair kernels up to 4 tokens, the dispatch-table regime above): every observable
+"""The block below the matrix-core widths (max_tokens < 64) regrouped into three launches (from eight tokens on the routing
+is a fourth) against the same block step by step, one pair or one dispatch block per unit: every observable
 tensor bit for bit, over repeated calls, with fewer live tokens than
 the buffer holds, with and without a logit bias, and for each format pairing.  The per-step launches are
 the ones the oracle comparisons of test_gpu_decode.py cover; test_block_matches_oracle runs the regrouped
