@@ -287,7 +287,7 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
                      prop.gcnArchName);
   // a code object that does not load shows up here rather than at the first launch
   hipFuncAttributes attr;
-  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows<false>));
+  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return set_error(XABE_ERR_COMPILE, "kernel load failed: %s", hipGetErrorString(e));
@@ -894,8 +894,9 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
     return set_error(XABE_ERR_INVALID_ARGUMENT, "rms_norm: x, weight and out must be 16-byte aligned");
   for (size_t first = 0; first < g.max_tokens; first += kSharedDigitTokens) {
     const size_t n = std::min(kSharedDigitTokens, g.max_tokens - first), at = first * g.hidden;
-    hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)n), dim3(256), 0, s, residual + at, post_norm, normed + at, (int)g.hidden,
-                       eps, b->shared_x_d, b->shared_x_e);
+    const int nsb = (int)digit_superblocks(g.hidden);
+    hipLaunchKernelGGL(k_rms_norm_digits, dim3((unsigned)n, (unsigned)((nsb + 3) / 4)), dim3(256), 0, s, residual + at, post_norm,
+                       normed + at, (int)g.hidden, eps, nsb, b->shared_x_d, b->shared_x_e);
     XABE_HIP_TRY(hipGetLastError());
     XABE_TRY(shared_digits(k, s, b, gate, up, down, normed, ffn_out, first, n, residual, l_out));
   }
@@ -991,8 +992,7 @@ int xabe_rms_norm(void* stream, const float* x, size_t x_len, const float* weigh
     hipLaunchKernelGGL(k_rms_norm_short_rows<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream), x, weight, out,
                        static_cast<_Float16*>(nullptr), (int)rows, (int)width, eps);
   else
-    hipLaunchKernelGGL(k_rms_norm_rows<false>, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out, (int)width, eps,
-                       static_cast<uint8_t*>(nullptr), static_cast<float*>(nullptr));
+    hipLaunchKernelGGL(k_rms_norm_rows, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out, (int)width, eps);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }

@@ -43,15 +43,6 @@ struct RowsArgs {
   uint32_t row_bytes;
 };
 
-// Group `gi` of a row, its sixteen values in `v` (sixteen consecutive lanes hold a superblock's), into the row's digits and
-// superblock scales (zeros where the group lies past the row's end).
-__device__ __forceinline__ void store_digits16(float (&v)[16], int gi, bool in, uint8_t* xd, float* xe) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) v[i] = in ? v[i] : 0.0f;
-  const float scale = digitize_superblock(v, gi & 15, xd + (size_t)(gi >> 4) * kSbDigitBytes);
-  if ((gi & 15) == 0) xe[gi >> 4] = scale;
-}
-
 // The digits of a group that sixteen consecutive lanes (a DPP row) hold one element each: lane's value `v` is element
 // `row` of the row whose digits start at xd.  Returns whether this lane's element is not held exactly.
 __device__ __forceinline__ bool store_digit_lane(float v, int shift, int row, uint8_t* xd, bool live) {

@@ -24,11 +24,8 @@ __device__ __forceinline__ float block_sum_256(float v, float* scratch) {
 // rms_norm_rows (crates/xabe-cuda/src/kernels/layer_ops.rs:129-151): every row of the
 // buffer, y = x * (1/sqrtf(mean(x^2) + eps)) * w.  grid = rows, 256 threads.
 // ---------------------------------------------------------------------------------
-// DIGITS: the row also goes out as the digits and superblock scales the fp32 row contractions read (digits.h).
-template <bool DIGITS>
 __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__ x, const float* __restrict__ w,
-                                                        float* __restrict__ out, int width, float eps,
-                                                        uint8_t* __restrict__ xd, float* __restrict__ xe) {
+                                                        float* __restrict__ out, int width, float eps) {
   const float* xr = x + (size_t)blockIdx.x * width;
   float* o = out + (size_t)blockIdx.x * width;
   // width is a multiple of 4; up to eight float4 columns per thread (rows up to 8192 wide) are requested
@@ -57,21 +54,26 @@ __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__
     const float4 a = x4[j], b = w4[j];
     o4[j] = make_float4(a.x * inv * b.x, a.y * inv * b.y, a.z * inv * b.z, a.w * inv * b.w);
   }
-  if constexpr (DIGITS) {  // (the same products from the row's cached pieces, sixteen consecutive elements per thread)
-    const int nsb = (width + kSbElems - 1) / kSbElems;
-    uint8_t* d = xd + (size_t)blockIdx.x * nsb * kSbDigitBytes;
-    float* e = xe + (size_t)blockIdx.x * nsb;
-    for (int gi = threadIdx.x; gi < nsb * 16; gi += 256) {
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = min(4 * gi + i, n4 - 1);
-        const float4 a = x4[j], b = w4[j];
-        v[4 * i] = a.x * inv * b.x, v[4 * i + 1] = a.y * inv * b.y, v[4 * i + 2] = a.z * inv * b.z, v[4 * i + 3] = a.w * inv * b.w;
-      }
-      store_digits16(v, gi, 16 * gi < width, d, e);
-    }
-  }
+}
+
+// The same with the row's digits and superblock scales (digits.h), which the fp32 row contractions read.  grid = (rows, a
+// workgroup per four superblocks): every wavefront folds the row for its scale, as above, and writes one superblock, whose
+// digits are a chain of ~150 instructions.  One row of 5120 elements, us: a workgroup per row, sixteen elements per thread
+// 8.0, a quad per thread 7.9 (of 1024 threads 13.6); this 5.0.
+__global__ void __launch_bounds__(256) k_rms_norm_digits(const float* __restrict__ x, const float* __restrict__ w,
+                                                         float* __restrict__ out, int width, float eps, int nsb,
+                                                         uint8_t* __restrict__ xd, float* __restrict__ xe) {
+  const float* xr = x + (size_t)blockIdx.x * width;
+  const int n4 = width / 4, j = (int)blockIdx.y * 256 + (int)threadIdx.x, jc = min(j, n4 - 1);
+  const float4 a = reinterpret_cast<const float4*>(xr)[jc], b = reinterpret_cast<const float4*>(w)[jc];
+  const float inv = row_inv_rms(xr, width, eps);
+  const bool in = j < n4;
+  const float v[4] = {in ? a.x * inv * b.x : 0.0f, in ? a.y * inv * b.y : 0.0f, in ? a.z * inv * b.z : 0.0f, in ? a.w * inv * b.w : 0.0f};
+  if (in) reinterpret_cast<float4*>(out + (size_t)blockIdx.x * width)[j] = make_float4(v[0], v[1], v[2], v[3]);
+  const int sb = __builtin_amdgcn_readfirstlane(j >> 6);
+  if (sb >= nsb) return;
+  const float scale = digitize_quads(v, xd + ((size_t)blockIdx.x * nsb + sb) * kSbDigitBytes);
+  if ((threadIdx.x & 63) == 0) xe[(size_t)blockIdx.x * nsb + sb] = scale;
 }
 
 // Rows of at most 2048 elements: one wavefront per row, four rows per workgroup.  The lane's 32 elements are the ones
