@@ -17,6 +17,8 @@
  *     live token count from the device scalar `valid_tokens` (M:34-41): the sequence can be
  *     captured into a hipGraph.  No entry point allocates except the `_new` / `_upload` ones.
  *   - One kernels+buffers pair per pass shape per thread; calls on one buffer set must not overlap.
+ *   - Below 64 tokens, in the exact regime and with the matrix cores disabled every contraction keeps all bits of its
+ *     fp32 activations, whatever their range; infinities and NaN reach the outputs as fp32 multiply-adds take them there.
  */
 #ifndef XABE_HIP_H
 #define XABE_HIP_H
@@ -135,15 +137,16 @@ int xabe_moe_kernels_geometry(const xabe_moe_kernels* k, xabe_moe_geometry* out)
 /* M:5416-5418: force the matrix-core (MFMA) regime off; prefill widths then take the fp32 kernels. */
 int xabe_moe_kernels_disable_tensor_cores(xabe_moe_kernels* k);
 int xabe_moe_kernels_tensor_cores_enabled(const xabe_moe_kernels* k);             /* M:5456-5458 */
-/* M:5432-5434: no community-format kernels exist here; `on != 0` is accepted and recorded only. */
+/* M:5432-5434: no community-format kernels exist here; `on != 0` selects the other of two kernels wherever there are two
+ * with the same results (a comparison switch). */
 int xabe_moe_kernels_force_community(xabe_moe_kernels* k, int on);
-/* M:5450-5452: pin the fp32 decode kernels at any width so rows equal plain decode bit for bit. */
 /* No counterpart in the reference (a test and comparison switch like force_community): which of the two
  * matrix-core grouped-GEMM kernels the routed launches of a wide pass take.  0 (default) and 1: the kernel whose
  * wavefronts all load, dequantise and multiply in turn; 2: the kernel whose wavefronts are specialised (half of them
  * multiply, half dequantise) wherever the shape allows: same bits, measured slower at every width, kept as the
  * reproducible record of that comparison. */
 int xabe_moe_kernels_set_mfma_form(xabe_moe_kernels* k, int form);
+/* M:5450-5452: pin the fp32 decode kernels at any width so rows equal plain decode bit for bit. */
 int xabe_moe_kernels_set_exact_decode_regime(xabe_moe_kernels* k, int on);
 
 /* MoeKernels::buffers (M:5338-5340) / shared_only_buffers (M:5354-5360) */
