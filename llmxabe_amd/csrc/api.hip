@@ -661,8 +661,8 @@ static RowsArgs rows_args(const xabe_moe_kernels* k, const xabe_moe_buffers* b) 
 
 // One (token, k) pair per unit while fewer than four select an expert on average, and in the exact regime; dispatch blocks
 // beyond, which read and unpack an expert's rows once per four or eight tokens.  Routed experts, us, pairs / blocks: the
-// model's 256 experts, top 8, 32 tokens 130 / 165, 45: 171 / 198, 63: 224 / 237, 64: 236 / 244, 256: 792 / 565, 1024:
-// 3091 / 1638; 64 experts, top 4, hidden 1024: 45 tokens 51 / 70, 256: 199 / 150.
+// model's 256 experts, top 8, 32 tokens 130 / 165, 45: 171 / 198, 63: 224 / 237, 64: 236 / 244, 256: 792 / 530, 1024:
+// 3091 / 1553; 64 experts, top 4, hidden 1024: 45 tokens 51 / 70, 256: 199 / 161.
 // force_community keeps the blocks, where there are any, for comparison: same bits.
 constexpr size_t kPairsPerExpert = 4;
 static bool routed_by_pairs(const xabe_moe_kernels* k) {

@@ -5,7 +5,7 @@
 // A workgroup is eight wavefronts over the row tiles of its share (32 rows, or 16 gate and the 16 matching up rows).
 // The contraction is split between the wavefronts by superblock class (superblock mod 8; rows of fewer than eight
 // superblocks leave several wavefronts per class, which take the tiles in turn), so that a wavefront meets few
-// superblocks of activations and reuses their digits, held in registers, for every tile of its share.
+// superblocks of activations and reuses their digits for every tile of its share.
 //
 // Order of operations per (row, token), whatever the launch shape: a class sums its superblocks in order, each half of
 // the wavefront its own groups; the classes are added in order, then half 0 + half 1.  A token's row is therefore the
@@ -52,16 +52,22 @@ constexpr int kRowsRoutedTiles = 4;
 
 template <int MODE, int QUANT, int NM, int NT, bool TAIL>
 struct RowsLds {
-  using Dma = SliceDma<QUANT, TAIL ? 18 : SbRaw<QUANT>::kPieces>;
+  static constexpr bool kFromLds = NT > 4;  // a superblock's digits are read from LDS as they are used
+  // (14 pieces are enough for 210 bytes at any even offset)
+  using Dma = SliceDma<QUANT, TAIL ? 18 : kFromLds && NM == 1 ? 14 : SbRaw<QUANT>::kPieces>;
   static constexpr int kDigits = NT * kSbDigitBytes, kScales = NM == 1 ? NT * kSbScaleBytes : 0;
-  static constexpr int kPerWave = Dma::kSlotBytes + kDigits + 2 * kScales;
+  static constexpr int kPerWave = Dma::kSlotBytes + kDigits + (kFromLds ? 1 : 2) * kScales;
 };
 
-// TEAMS: one team of eight wavefronts for up to four tokens, or two teams of four, each with four tokens of its own and
-// twice the classes: the digits and sums of eight tokens take more registers than a wavefront has and more LDS than
-// eight wavefronts have.  Both teams request every row (the second time out of L2) and wait for nobody.
+// Up to four tokens hold a superblock's digits in registers for every tile of the share.  Eight do not fit there: Q6_K
+// passes of eight read them from LDS as the matrix instructions take them (the slot is busy until the last tile is done, so
+// the next superblock's digits are requested only then; down's weight windows give up the piece that spreads rows over
+// the banks, and scales their second buffer, to make room).  Q8_0's weight slots leave no such room: two TEAMS of four
+// wavefronts, each with four tokens of its own and twice the classes; both request and unpack every row.  Dense sibling,
+// eight tokens, us, two teams / one: gate/up 69.5 / 64.5, down 61 / 49.5; 32 tokens 475 / 417.
 template <int MODE, int QUANT, int NM, int NT, int TEAMS, int MT, bool TAIL>
 __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
+  constexpr bool kFromLds = RowsLds<MODE, QUANT, NM, NT, TAIL>::kFromLds;
   constexpr int kTeam = 8 / TEAMS, kRounds = TEAMS, kTokens = NT * TEAMS;
   using L = RowsLds<MODE, QUANT, NM, NT, TAIL>;
   // gate and up read rows whose scales are whole superblocks', down the intermediate rows, scaled by groups
@@ -194,7 +200,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
     }
     int buf = 0;
     if (any) {
-      v4i_t ax[8][TG], az[kSwapped ? 8 : 4][TG];
+      v4i_t ax[kFromLds ? 1 : 8][TG], az[kFromLds ? 1 : kSwapped ? 8 : 4][TG];
       LdsDigits<NT, kSbDigitBytes, kSwapped> x;
 #pragma unroll 1
       while (now.sb < nsb) {
@@ -208,14 +214,16 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
             for (int t = 0; t < NT; ++t) e_now[t] = e_next[t];
           }
           x.point(d_slot, e_slot + buf * L::kScales, s_zero);
+          if constexpr (!kFromLds) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
+            for (int j = 0; j < 8; ++j)
 #pragma unroll
-            for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.high(j & 3, j >> 2, tg);
+              for (int tg = 0; tg < TG; ++tg) ax[j][tg] = x.high(j & 3, j >> 2, tg);
 #pragma unroll
-          for (int j = 0; j < (kSwapped ? 8 : 4) && !digits_in_one(NT); ++j)
+            for (int j = 0; j < (kSwapped ? 8 : 4) && !digits_in_one(NT); ++j)
 #pragma unroll
-            for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
+              for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
+          }
         }
         if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
 #pragma unroll
@@ -229,7 +237,7 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
         sb_read(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (next.sb < nsb) request_w(next.i, next.sb);
-        if (next.sb < nsb && next.i == 0) request_x(next.sb, buf ^ 1);
+        if (!kFromLds && next.sb < nsb && next.i == 0) request_x(next.sb, buf ^ 1);
         float v[NT];
         auto x_of = [&](int t) __attribute__((always_inline)) {
           int row = x_row[0];
@@ -242,8 +250,16 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
           else return x.template scale<kSbScaleBytes>(t, l);
         };
         sb_dot<QUANT, kScale, NT, TAIL>(
-            raw, [&](int s, int l, int tg) { return ax[4 * l + s][tg]; },
-            [&](int s, int l, int tg) { return az[kSwapped ? 4 * l + s : s][tg]; }, e_of, x_of, v, live_lanes,
+            raw,
+            [&](int s, int l, int tg) __attribute__((always_inline)) {
+              if constexpr (kFromLds) return x.high(s, l, tg);
+              else return ax[4 * l + s][tg];
+            },
+            [&](int s, int l, int tg) __attribute__((always_inline)) {
+              if constexpr (kFromLds) return x.low(s, l, tg);
+              else return az[kSwapped ? 4 * l + s : s][tg];
+            },
+            e_of, x_of, v, live_lanes,
             TAIL && half == 1 && (sb * kSbElems + 128) >= a.K);
 #pragma unroll
         for (int m = 0; m < kRounds * MT; ++m) {  // (the sums stay in registers: the tile's own by a uniform branch, not by an index)
@@ -252,7 +268,11 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
 #pragma unroll
           for (int t = 0; t < NT; ++t) acc[m / MT][m % MT][t] += v[t];
         }
-        if (next.i == 0) buf ^= 1;
+        if (next.i == 0 && !kFromLds) buf ^= 1;
+        if (kFromLds && next.sb < nsb && next.i == 0) {  // (the last tile is done with the slot)
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          request_x(next.sb, buf);
+        }
         now = next;
       }
     }
@@ -579,18 +599,24 @@ static int rows_quant(int quant, bool tail, dim3 grid, hipStream_t s, const Rows
   return tail ? rows_go<MODE, kQ8_0, NM, NT, TEAMS, MT, true>(grid, s, a) : rows_go<MODE, kQ8_0, NM, NT, TEAMS, MT, false>(grid, s, a);
 }
 
+// (see k_digit_rows)
+static bool one_team(int quant) { return quant == XABE_QUANT_Q6K; }
+
 template <int NM, int MT>
 static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
   switch (nt) {
     case 1: return rows_quant<kRowsShared, NM, 1, 1, MT>(quant, tail, grid, s, a);
     case 2: return rows_quant<kRowsShared, NM, 2, 1, MT>(quant, tail, grid, s, a);
     case 4: return rows_quant<kRowsShared, NM, 4, 1, MT>(quant, tail, grid, s, a);
-    default: return rows_quant<kRowsShared, NM, 4, 2, MT>(quant, tail, grid, s, a);
+    default:
+      if (one_team(quant)) return rows_go<kRowsShared, kQ6K, NM, 8, 1, MT, false>(grid, s, a);
+      return rows_quant<kRowsShared, NM, 4, 2, MT>(quant, tail, grid, s, a);
   }
 }
 
 template <int NM>
 static int rows_mode(int mode, int nt, int mt, int quant, bool tail, dim3 grid, hipStream_t s, const RowsArgs* a) {
+  if (mode == kRowsBlock && nt > 4 && one_team(quant)) return rows_go<kRowsBlock, kQ6K, NM, 8, 1, kRowsRoutedTiles, false>(grid, s, a);
   if (mode == kRowsBlock)
     return nt == 4 ? rows_quant<kRowsBlock, NM, 4, 1, kRowsRoutedTiles>(quant, tail, grid, s, a)
                    : rows_quant<kRowsBlock, NM, 4, 2, kRowsRoutedTiles>(quant, tail, grid, s, a);
@@ -687,15 +713,20 @@ int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, Ro
     units = (t + nt - 1) / nt;
   } else {
     // tokens of a block per pass over an expert's rows: four, or eight where an expert has six on average (a pass for two,
-    // as it was: 256 tokens 797 us, now 565; 1024 tokens 2724, now 1638)
+    // as it was: 256 tokens 797 us, now 530; 1024 tokens 2724, now 1553)
     nt = k->g.max_tokens * k->g.experts_per_token >= 6 * k->g.num_experts ? 8 : 4;
   }
-  const int per_class = std::max(1, (nt > 4 ? 4 : 8) / a.classes);  // (as the kernel has it: nt > 4 is two teams)
+  const bool teams = nt > 4 && !one_team(quant);
+  const int per_class = std::max(1, (teams ? 4 : 8) / a.classes);  // (as the kernel has it)
   int mt = 1;
   const int tiles16 = a.n_tiles;
   unsigned grid_x = (unsigned)((tiles16 + per_class - 1) / per_class);
   if (mode == kRowsBlock) {
-    grid_x = (unsigned)((tiles16 + per_class * kRowsRoutedTiles - 1) / (per_class * kRowsRoutedTiles));
+    // tiles per wavefront: as many as leave two workgroups per CU for the blocks a pass is likely to have
+    const size_t pairs = k->g.max_tokens * k->g.experts_per_token, live = std::max(std::min(k->g.num_experts, pairs), pairs / k->g.block_size);
+    int each = kRowsRoutedTiles;
+    while (each > 1 && live * ((tiles16 + per_class * each - 1) / (per_class * each)) < (size_t)2 * k->num_cus) each /= 2;
+    grid_x = (unsigned)((tiles16 + per_class * each - 1) / (per_class * each));
   } else if (per_class == 1 && tiles16 > k->num_cus) {
     // many tiles: one workgroup per CU with an even share of them, so that a superblock's digits serve the whole share
     mt = kRowsMaxTiles;
