@@ -275,3 +275,44 @@ def test_infinities_and_nan_reach_the_outputs_as_in_plain_fp32(quant):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
     assert np.isinf(ref[0]).sum() > 50 and np.isinf(ref[1]).sum() > 20 and np.isnan(ref[2]).all()
+
+
+@pytest.mark.parametrize("quant", ["Q8_0", "Q6_K"])
+@pytest.mark.parametrize("tokens", [1, 3, 8])
+def test_infinities_reach_the_gate_and_up_products(quant, tokens):
+    # one activation of one token is infinite; gate's weight there is positive, so silu(g) is +infinity and the product has
+    # the sign of up's weight (a NaN where that is zero); the other tokens' products are what they are without it
+    import torch
+    import llmxabe_amd as X
+
+    H, I, col = 2560, 512, 1234
+    rng = np.random.default_rng(17)
+    make = _q8_0 if quant == "Q8_0" else _q6_k
+    hi = 127 if quant == "Q8_0" else 31
+    d = np.full(I, 2e-4 if quant == "Q8_0" else 6e-5)
+    codes = [rng.integers(-hi, hi + 1, (I, H)).astype(np.int8) for _ in range(2)]
+    codes[0][:, col] = 5
+    codes[1][::7, col] = 0
+    q = X.ExpertQuant.Q8_0 if quant == "Q8_0" else X.ExpertQuant.Q6K
+    st = [X.QuantTensor(torch.from_numpy(make(c, d)[0]).cuda(), q) for c in codes]
+    st.append(X.QuantTensor(torch.from_numpy(_matrix(rng, quant, H, I)[0]).cuda(), q))
+    x = rng.standard_normal((tokens, H)).astype(np.float32)
+
+    def products(rows, plain):
+        k = X.MoeKernels(X.MoeGeometry(1, 1, H, I, 32, tokens))
+        k.force_community(plain)
+        b = k.shared_only_buffers(False)
+        k.set_valid_tokens(b, tokens)
+        out = torch.zeros(tokens * H, device="cuda")
+        k.shared_expert(b, *st, torch.from_numpy(rows).cuda().view(-1), out)
+        torch.cuda.synchronize()
+        return b.shared_inter().cpu().numpy().reshape(tokens, I).copy()
+
+    for plain in (False, True):
+        finite = products(x, plain)
+        y = x.copy()
+        y[tokens - 1, col] = np.inf
+        got, sign = products(y, plain), np.sign(codes[1][:, col].astype(int))
+        assert np.array_equal(np.isposinf(got[-1]), sign > 0) and np.array_equal(np.isneginf(got[-1]), sign < 0)
+        assert np.array_equal(np.isnan(got[-1]), sign == 0)
+        assert np.array_equal(got[:-1].view(np.uint32), finite[:-1].view(np.uint32))
