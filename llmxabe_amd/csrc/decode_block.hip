@@ -483,7 +483,8 @@ __global__ void __launch_bounds__(128 * NP, DIRECT ? 2 : 4) k_decode_up(DecodeAr
     for (int i = 0; i < (DIRECT ? 1 : a.share_g); ++i) {
       if constexpr (!DIRECT) {
         wait_loads();
-        sb_read(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+        if (RQ == kQ6K && sb0 + 2 == 2 * NP && run_off(i) + (size_t)16 * row_bytes == a.up_len) Dma::patch_tail(mat ? a.up : a.gate, a.up_len, slot);
+        sb_read_slot(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (i + 1 < a.share_g) dma.request(mat ? a.up : a.gate, a.up_len, run_off(i + 1), slot_lds);
       }
@@ -605,7 +606,7 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
     for (int i = 0; i < a.share_d; ++i) {
       wait_loads();
       SbRaw<RQ> raw;
-      sb_read(slot + (lane & 15) * Dma::kRowStride + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
+      sb_read_words(slot + (lane & 15) * Dma::kRowStride + (quarter >> 1) * SbRaw<RQ>::kBytes, quarter & 1, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (i + 1 < a.share_d) dma.request(run(i + 1), slot_lds);
       float v = pair_dot<RQ>(

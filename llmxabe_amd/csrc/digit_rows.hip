@@ -53,7 +53,7 @@ constexpr int kRowsRoutedTiles = 4;
 template <int MODE, int QUANT, int NM, int NT, bool TAIL>
 struct RowsLds {
   static constexpr bool kFromLds = NT > 4;  // a superblock's digits are read from LDS as they are used
-  // (14 pieces are enough for 210 bytes at any even offset)
+  // (14 pieces are enough for 210 bytes from the word boundary below)
   using Dma = SliceDma<QUANT, TAIL ? 18 : kFromLds && NM == 1 ? 14 : SbRaw<QUANT>::kPieces>;
   static constexpr int kDigits = NT * kSbDigitBytes, kScales = NM == 1 ? NT * kSbScaleBytes : 0;
   static constexpr int kPerWave = Dma::kSlotBytes + kDigits + (kFromLds ? 1 : 2) * kScales;
@@ -225,16 +225,16 @@ __global__ void __launch_bounds__(512, 2) k_digit_rows(RowsArgs a) {
               for (int tg = 0; tg < TG; ++tg) az[j][tg] = x.low(j & 3, j >> 2, tg);
           }
         }
-        if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
+        if (sb == nsb - 1 && dma[0].ends_apart(a.w_bytes)) {
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             const size_t off = e_off + (size_t)run_row(i, u) * row_bytes;
             const int live = min(min(tile_rows - (NM == 2 ? 0 : 16 * u), 16), a.n_rows - (tile_of(i) * tile_rows + (NM == 2 ? 0 : 16 * u)));
-            if (live >= 1 && off + (size_t)live * row_bytes == a.w_bytes) dma[u].patch_tail(NM == 2 && u ? a.w1 : a.w0, a.w_bytes, off, live, sb, w_slot + u * Dma::kRunBytes);
+            if (live >= 1 && off + (size_t)live * row_bytes == a.w_bytes) dma[u].patch_tail(NM == 2 && u ? a.w1 : a.w0, off, live, sb, w_slot + u * Dma::kRunBytes);
           }
         }
         SbRaw<QUANT> raw;
-        sb_read(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
+        sb_read_slot(dma[0].row_at(w_slot + u_lane * Dma::kRunBytes, e_off + (size_t)run_row(i, u_lane) * row_bytes, r_lane, sb), half, raw);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (next.sb < nsb) request_w(next.i, next.sb);
         if (!kFromLds && next.sb < nsb && next.i == 0) request_x(next.sb, buf ^ 1);
@@ -361,35 +361,40 @@ constexpr int kPairTiles = 4;  // tiles a wavefront takes at most
 constexpr size_t kPairsXcdMinTokens = 24;
 
 // SliceDma's slot for tiles that start on 16-byte boundaries (sixteen rows of an expert are whole pieces, and so are the
-// rows before them): the lane's offsets are the same for every tile of a superblock and kept in units of pieces, two to a
-// register (rows of more than 64 KB: worked out again for every tile).
+// rows before them): the lane's offsets are the same for every tile of a superblock and kept in units of what windows start
+// on, two to a register (longer rows, Q6_K's of 16 KB: worked out again for every tile).
 template <int QUANT, int PIECES>
 struct TileDma {
   static constexpr int kP = PIECES, kInstr = (16 * kP + 63) / 64, kLast = 16 * kP - 64 * (kInstr - 1);
   static constexpr int kRunBytes = 16 * kP * 16, kSlotBytes = 2 * kRunBytes;
+  static constexpr uint32_t kStart = SbRaw<QUANT>::kStart, kUnit = kStart + 1;
   PackedOffsets<kInstr> off;
   static __device__ __forceinline__ uint32_t piece(int i, uint32_t row_bytes, int sb) {
     const uint32_t pc = min((uint32_t)(64 * i) + __lane_id(), 16u * kP - 1);
-    return ((pc / kP * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) >> 4) + pc % kP;
+    return (pc / kP * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) / kUnit + pc % kP * (16 / kUnit);
   }
   __device__ __forceinline__ void init(uint32_t row_bytes, int sb) {
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) off.set(i, piece(i, row_bytes, sb) & 0xffffu);
   }
-  // pieces past the tensor's end (padding of the last rows' windows) repeat its last one
+  // pieces that would reach past the tensor repeat its end (Q6_K: see patch_tail; otherwise they are padding)
   __device__ __forceinline__ void request(const uint8_t* w, size_t w_bytes, size_t tile, uint32_t row_bytes, int sb, uint32_t dst) {
     const uint32_t last = (uint32_t)min(w_bytes - 16 - tile, (size_t)0xfffffff0u);
-    const bool fits = row_bytes <= 65535 - kP;  // (16 rows and a window are at most 65535 pieces)
+    const bool fits = row_bytes <= 65536 / 16 * kUnit - kP;  // (16 rows and a window are at most 65535 units)
     off.opaque();
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) {
       uint32_t o = off.get(i);
       if (__builtin_expect(!fits, 0)) o = piece(i, row_bytes, sb);
-      if (i + 1 < kInstr || kLast == 64 || (int)__lane_id() < kLast) lds_dma_16(w + tile, min(o * 16, last), dst + i * 1024);
+      if (i + 1 < kInstr || kLast == 64 || (int)__lane_id() < kLast) lds_dma_16(w + tile, min(o * kUnit, last), dst + i * 1024);
     }
   }
+  // (the run's last row ends the tensor, and this is its last superblock; Q6_K)
+  static __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t w_bytes, uint8_t* run_slot) {
+    patch_window<QUANT>(w, w_bytes - SbRaw<QUANT>::kBytes, run_slot + 15 * (kP * 16));
+  }
   static __device__ __forceinline__ const uint8_t* row_at(const uint8_t* run_slot, uint32_t row_bytes, int row, int sb) {
-    return run_slot + row * (kP * 16) + (((uint32_t)row * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & 15u);
+    return run_slot + row * (kP * 16) + (((uint32_t)row * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & kStart);
   }
 };
 
@@ -492,7 +497,14 @@ __global__ void __launch_bounds__(512, DIRECT ? 2 : 4) k_digit_pairs(RowsArgs a,
     const int next_i = last ? 0 : i + 1, next_sb = last ? sb + classes : sb;
     if constexpr (!DIRECT) {
       wait_loads();
-      sb_read(Dma::row_at(w_slot + run * Dma::kRunBytes, row_bytes, lane & 15, sb), half, raw);
+      if (QUANT == kQ6K && sb == nsb - 1) {
+        const size_t end = e_off + ((size_t)(tile_lo + sub + per_class * i) * tile_rows + tile_rows) * row_bytes;
+        if (end == a.w_bytes) {  // (NM == 2: both matrices end here)
+          if constexpr (NM == 2) Dma::patch_tail(a.w0, a.w_bytes, w_slot);
+          Dma::patch_tail(NM == 2 ? a.w1 : a.w0, a.w_bytes, w_slot + Dma::kRunBytes);
+        }
+      }
+      sb_read_slot(Dma::row_at(w_slot + run * Dma::kRunBytes, row_bytes, lane & 15, sb), half, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     if constexpr (NM == 2) {
@@ -609,7 +621,9 @@ static int rows_shared(int nt, int quant, bool tail, dim3 grid, hipStream_t s, c
     case 2: return rows_quant<kRowsShared, NM, 2, 1, MT>(quant, tail, grid, s, a);
     case 4: return rows_quant<kRowsShared, NM, 4, 1, MT>(quant, tail, grid, s, a);
     default:
-      if (one_team(quant)) return rows_go<kRowsShared, kQ6K, NM, 8, 1, MT, false>(grid, s, a);
+      // (down: the form for several tiles also where there is one: the other's compiled loop spills registers, and waits for
+      // them together with the rows it has just requested)
+      if (one_team(quant)) return rows_go<kRowsShared, kQ6K, NM, 8, 1, NM == 1 ? kRowsMaxTiles : MT, false>(grid, s, a);
       return rows_quant<kRowsShared, NM, 4, 2, MT>(quant, tail, grid, s, a);
   }
 }

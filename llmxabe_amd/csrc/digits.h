@@ -204,14 +204,17 @@ struct SbRaw<kQ6K> {
   uint2 sc;            // scales 8 h .. 8 h + 7
   uint32_t d;
   static constexpr int kBytes = kQ6KBytes;
-  static constexpr int kPieces = 15;  // 16-byte pieces of a row's window: 210 bytes at any even offset, and one more
-                                      // that spreads the rows of a tile over the LDS banks
+  static constexpr int kPieces = 15;  // 16-byte pieces of a row's window: 210 bytes from the word boundary below, and one
+                                      // more that spreads the rows of a tile over the LDS banks
+  static constexpr uint32_t kStart = 3;  // windows start on words (so that they lie on 16 bytes in LDS, see sb_read_slot)
+  static constexpr int kWhole16 = kBytes / 16 * 16;  // a window's bytes in whole pieces
 };
 template <>
 struct SbRaw<kQ8_0> {
   uint32_t v[34];  // blocks 4 h .. 4 h + 3, 34 bytes each
   static constexpr int kBytes = 8 * kQ8Bytes;
   static constexpr int kPieces = 17;  // 272 bytes, 16-byte aligned where rows are whole superblocks (18 otherwise)
+  static constexpr uint32_t kStart = 15;
 };
 
 // `p`: the row's superblock (any even address, global or LDS)
@@ -223,6 +226,75 @@ __device__ __forceinline__ void sb_read(const uint8_t* p, int h, SbRaw<kQ6K>& r)
   __builtin_memcpy(&r.sc, __builtin_assume_aligned(p + 192 + 8 * h, 2), 8);
   r.d = *reinterpret_cast<const uint16_t*>(p + 208);
 }
+// The raw words as registers nothing is known about.
+__device__ __forceinline__ void opaque(SbRaw<kQ6K>& r) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(r.ql[i]));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(r.qh[i]));
+  asm volatile("" : "+v"(r.sc.x), "+v"(r.sc.y), "+v"(r.d));
+}
+// A word of LDS by itself: the compiler would merge neighbours into a read wider than their alignment.
+__device__ __forceinline__ uint32_t lds_word(const uint8_t* p) {
+  return *reinterpret_cast<const volatile __attribute__((address_space(3))) uint32_t*>(
+      (const volatile __attribute__((address_space(3))) uint8_t*)p);
+}
+// The same out of LDS, where a read that does not start on a multiple of its own width takes 64 cycles of the unit, one lane
+// after the other (on such a multiple 4.4 for sixteen bytes per lane): superblocks lie at even offsets, so the words are
+// read where words are and shifted by the half word that is left.  `p`: at most two bytes past a 16-byte boundary.
+// (Seven reads at any even address held the unit 448 cycles per superblock of a tile, two thirds of the block's second
+// launch at 45 tokens; these ten 60, and 26 shifts.)
+__device__ __forceinline__ void sb_read_slot(const uint8_t* p, int h, SbRaw<kQ6K>& r) {
+  const uint32_t at = (uint32_t)(uintptr_t)p, shift = (at & 2u) << 3;
+  const uint8_t* const b = static_cast<const uint8_t*>(__builtin_assume_aligned(p - (at & 2u), 16));
+  // (in place, run by run: the shifted words of all three runs beside the unshifted ones are registers the widest passes
+  // do not have)
+  auto shift_down = [&](uint32_t (&w)[4], uint32_t next) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) w[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], shift);
+    w[3] = __builtin_amdgcn_alignbit(next, w[3], shift);
+  };
+  uint32_t w[6][4];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    const v4u_t v = *reinterpret_cast<const v4u_t*>(i < 4 ? b + 64 * h + 16 * i : b + 64 + 32 * h + 16 * i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[i][j] = v[j];
+  }
+  const uint32_t ql_end = lds_word(b + 64 * h + 64), qh_end = lds_word(b + 160 + 32 * h);
+  const uint2 sc = *reinterpret_cast<const uint2*>(b + 192 + 8 * h);
+  const uint32_t sc_end = lds_word(b + 200 + 8 * h);
+  r.d = *reinterpret_cast<const uint16_t*>(p + 208);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) shift_down(w[i], i == 3 ? ql_end : i == 5 ? qh_end : w[i + 1][0]);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.ql[i][j] = w[i][j];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) r.qh[i][j] = w[4 + i][j];
+  }
+  r.sc = make_uint2(__builtin_amdgcn_alignbit(sc.y, sc.x, shift), __builtin_amdgcn_alignbit(sc_end, sc.y, shift));
+  opaque(r);  // (shifted here: put off until they are used, the words take more registers)
+}
+// (any even address, rows an odd number of words apart: word by word)
+__device__ __forceinline__ void sb_read_words(const uint8_t* p, int h, SbRaw<kQ6K>& r) {
+  const uint32_t at = (uint32_t)(uintptr_t)p, shift = (at & 2u) << 3;
+  const uint8_t* const b = p - (at & 2u);
+  uint32_t ql[17], qh[9], sc[3];
+#pragma unroll
+  for (int i = 0; i < 17; ++i) ql[i] = lds_word(b + 64 * h + 4 * i);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) qh[i] = lds_word(b + 128 + 32 * h + 4 * i);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) sc[i] = lds_word(b + 192 + 8 * h + 4 * i);
+  r.d = *reinterpret_cast<const uint16_t*>(p + 208);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r.ql[i / 4][i % 4] = __builtin_amdgcn_alignbit(ql[i + 1], ql[i], shift);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r.qh[i / 4][i % 4] = __builtin_amdgcn_alignbit(qh[i + 1], qh[i], shift);
+  r.sc = make_uint2(__builtin_amdgcn_alignbit(sc[1], sc[0], shift), __builtin_amdgcn_alignbit(sc[2], sc[1], shift));
+}
 __device__ __forceinline__ void sb_read(const uint8_t* p, int h, SbRaw<kQ8_0>& r) {  // (`p` on an 8-byte boundary)
 #pragma unroll
   for (int i = 0; i < 17; ++i) {
@@ -231,6 +303,9 @@ __device__ __forceinline__ void sb_read(const uint8_t* p, int h, SbRaw<kQ8_0>& r
     r.v[2 * i + 1] = t.y;
   }
 }
+
+__device__ __forceinline__ void sb_read_slot(const uint8_t* p, int h, SbRaw<kQ8_0>& r) { sb_read(p, h, r); }
+__device__ __forceinline__ void sb_read_words(const uint8_t* p, int h, SbRaw<kQ8_0>& r) { sb_read(p, h, r); }
 
 // Codes of group (s, l) as int8.  Q6_K codes come out times four, as signed bytes: the six bits sit at the byte's top with
 // the code's top bit flipped (c - 32 in two's complement), which costs no more than unpacking them in place; the quarter
@@ -294,13 +369,6 @@ __device__ __forceinline__ float join_sums(const int (&d)[6]) {
 // each of its sixteen lanes loads eight of them (one trip to memory) and the others take them from there.
 // (The registers go through an empty statement first and the groups are kept apart: the compiler would otherwise keep the
 // codes it unpacked for the matrix instruction for this branch, or unpack all of them at once.)
-__device__ __forceinline__ void opaque(SbRaw<kQ6K>& r) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(r.ql[i]));
-#pragma unroll
-  for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(r.qh[i]));
-  asm volatile("" : "+v"(r.sc.x), "+v"(r.sc.y), "+v"(r.d));
-}
 __device__ __forceinline__ void opaque(SbRaw<kQ8_0>& r) {
 #pragma unroll
   for (int i = 0; i < 34; ++i) asm volatile("" : "+v"(r.v[i]));
@@ -488,6 +556,20 @@ struct LdsDigits {
   __device__ __forceinline__ float4 scale(int t, int l) const { return *reinterpret_cast<const float4*>(e + t * E_STRIDE + l * 16); }
 };
 
+// What the pieces of the window that starts at byte `start` of a tensor and ends with it could not hold, two bytes at a time,
+// to the window at `slot`.  SPAN: the bytes wanted from `start` on.
+template <int QUANT, int SPAN = SbRaw<QUANT>::kBytes>
+__device__ __forceinline__ void patch_window(const uint8_t* w, size_t start, uint8_t* slot) {
+  int lane = (int)__lane_id();
+  asm volatile("" : "+v"(lane));  // (once per launch: its arithmetic stays here, out of the registers of the loop around)
+  const size_t from = start & ~(size_t)SbRaw<QUANT>::kStart, whole = (start + SPAN - from) & ~(size_t)15;
+  if (2 * lane < (int)(start + SPAN - from - whole))
+    *reinterpret_cast<uint16_t*>(slot + whole + 2 * lane) = *reinterpret_cast<const uint16_t*>(w + from + whole + 2 * lane);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------------
 // A wavefront's private LDS slot for one superblock of 32 rows (two runs of 16 rows each, from one matrix or from
 // two), filled by global -> LDS DMA.  Each row's window is requested as whole 16-byte pieces: a lane that reads its
@@ -518,32 +600,29 @@ struct SliceDma {
     }
   }
   // Requests superblock `sb` of the run whose first row starts `run_off` bytes into the tensor at `w` (16-byte aligned,
-  // `w_bytes` long) into LDS at `dst` (byte address).  Pieces past the tensor's last whole one repeat it.
+  // `w_bytes` long) into LDS at `dst` (byte address).  Pieces that would reach past the tensor repeat its end.
   __device__ __forceinline__ void request(const uint8_t* w, size_t w_bytes, size_t run_off, int sb, uint32_t dst) const {
+    constexpr uint32_t kStart = SbRaw<QUANT>::kStart;
     const uint8_t* base = w + (run_off & ~(size_t)15);
     const uint32_t mis = (uint32_t)run_off & 15u;
     const size_t left = w_bytes - (run_off & ~(size_t)15);
-    const uint32_t last = (uint32_t)min(left >= 16 ? (left & ~(size_t)15) - 16 : (size_t)0, (size_t)0xfffffff0u);
+    const uint32_t last = (uint32_t)min(left >= 16 ? (left - 16) & ~(size_t)kStart : (size_t)0, (size_t)0xfffffff0u);
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) {
-      const uint32_t voff = min(((mis + row_off[i] + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & ~15u) + col[i], last);
+      const uint32_t voff = min(((mis + row_off[i] + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & ~kStart) + col[i], last);
       if (i + 1 < kInstr || kLast == 64 || (int)__lane_id() < kLast) lds_dma_16(base, voff, dst + i * 1024);
     }
   }
-  // A tensor that ends inside a 16-byte piece: its last bytes, which no whole piece holds, go to the slot two by two
-  // (the run's `live` rows end the tensor, and `sb` is the rows' last superblock).
-  __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t w_bytes, size_t run_off, int live, int sb, uint8_t* run_slot) const {
-    const int lane = (int)__lane_id();
-    const size_t tail = w_bytes & ~(size_t)15, start = run_off + (size_t)(live - 1) * row_bytes + (size_t)sb * SbRaw<QUANT>::kBytes;
-    uint8_t* p = run_slot + (live - 1) * (kP * 16) + (start & 15) + (tail - start);
-    if (2 * lane < (int)(w_bytes & 15)) *reinterpret_cast<uint16_t*>(p + 2 * lane) = *reinterpret_cast<const uint16_t*>(w + tail + 2 * lane);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // The run's `live` rows end the tensor, and `sb` is their last superblock: the bytes that no piece inside the tensor
+  // held go to the slot two by two.
+  __device__ __forceinline__ bool ends_apart(size_t w_bytes) const { return QUANT == kQ6K || (w_bytes & 15) != 0; }
+  __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t run_off, int live, int sb, uint8_t* run_slot) const {
+    const size_t start = run_off + (size_t)(live - 1) * row_bytes + (size_t)sb * SbRaw<QUANT>::kBytes;
+    patch_window<QUANT>(w, start, run_slot + (live - 1) * (kP * 16));
   }
   // the address of the lane's row inside the run's slot
   __device__ __forceinline__ const uint8_t* row_at(const uint8_t* run_slot, size_t run_off, int row, int sb) const {
-    const uint32_t mis = ((uint32_t)run_off + (uint32_t)row * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & 15u;
+    const uint32_t mis = ((uint32_t)run_off + (uint32_t)row * row_bytes + (uint32_t)(sb * SbRaw<QUANT>::kBytes)) & SbRaw<QUANT>::kStart;
     return run_slot + row * (kP * 16) + mis;
   }
 };
@@ -572,7 +651,7 @@ struct PackedOffsets {
 
 template <int QUANT>
 struct PairDma {
-  static constexpr int kP = QUANT == kQ6K ? 29 : 35;  // 420 bytes at any even offset, rows four words apart modulo the banks; 35 likewise
+  static constexpr int kP = QUANT == kQ6K ? 29 : 35;  // 420 bytes from a word boundary, rows four words apart modulo the banks; 35 likewise
   static constexpr int kInstr = (16 * kP + 63) / 64, kSlotBytes = kInstr * 1024;  // (a slot's last instruction pads)
   PackedOffsets<kInstr> off;  // the lane's piece of each instruction, relative to the tile's first row
   // sixteen rows of `row_bytes` (16 row_bytes are whole pieces, and fewer than 65536), superblocks sb0 and sb0 + 1
@@ -581,19 +660,23 @@ struct PairDma {
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) {
       const int pc = min(64 * i + lane, 16 * kP - 1);
-      off.set(i, (((uint32_t)(pc / kP) * row_bytes + (uint32_t)(sb0 * SbRaw<QUANT>::kBytes)) & ~15u) + (uint32_t)(pc % kP) * 16);
+      off.set(i, (((uint32_t)(pc / kP) * row_bytes + (uint32_t)(sb0 * SbRaw<QUANT>::kBytes)) & ~SbRaw<QUANT>::kStart) + (uint32_t)(pc % kP) * 16);
     }
   }
   // `tile`: offset of the tile's first row in the tensor at `w` (16-byte aligned, `w_bytes` long, like the tile); pieces
-  // past the tensor's last whole one repeat it (they are padding: a pair's own bytes lie in whole pieces)
+  // that would reach past the tensor repeat its end (Q6_K: see patch_tail; otherwise they are padding)
   __device__ __forceinline__ void request(const uint8_t* w, size_t w_bytes, size_t tile, uint32_t dst) {
     const uint32_t last = (uint32_t)min((w_bytes & ~(size_t)15) - 16 - tile, (size_t)0xfffffff0u);
     off.opaque();
 #pragma unroll
     for (int i = 0; i < kInstr; ++i) lds_dma_16(w + tile, min(off.get(i), last), dst + i * 1024);
   }
+  // (the tile's last row, this pair its last one, ends the tensor; Q6_K)
+  static __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t w_bytes, uint8_t* slot) {
+    patch_window<QUANT, 2 * SbRaw<QUANT>::kBytes>(w, w_bytes - 2 * SbRaw<QUANT>::kBytes, slot + 15 * (kP * 16));
+  }
   static __device__ __forceinline__ const uint8_t* row_at(const uint8_t* slot, uint32_t row_bytes, int row, int sb0) {
-    return slot + row * (kP * 16) + (((uint32_t)row * row_bytes + (uint32_t)(sb0 * SbRaw<QUANT>::kBytes)) & 15u);
+    return slot + row * (kP * 16) + (((uint32_t)row * row_bytes + (uint32_t)(sb0 * SbRaw<QUANT>::kBytes)) & SbRaw<QUANT>::kStart);
   }
 };
 

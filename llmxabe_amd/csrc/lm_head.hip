@@ -111,15 +111,15 @@ __global__ void __launch_bounds__(512, 2) k_lm_head_quant(LmHeadArgs a) {
         }
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if ((a.w_bytes & 15) != 0 && sb == nsb - 1) {
+      if (sb == nsb - 1 && dma[0].ends_apart(a.w_bytes)) {
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
           const int live = a.vocab - (row0 + 16 * v);
-          if (live >= 1 && live <= 16 && row_hi == a.vocab) dma[v].patch_tail(a.w, a.w_bytes, run_off(v), live, sb, slot + v * Dma::kRunBytes);
+          if (live >= 1 && live <= 16 && row_hi == a.vocab) dma[v].patch_tail(a.w, run_off(v), live, sb, slot + v * Dma::kRunBytes);
         }
       }
       SbRaw<QUANT> raw;
-      sb_read(dma[0].row_at(slot + u * Dma::kRunBytes, run_off(u), r, sb), h, raw);
+      sb_read_slot(dma[0].row_at(slot + u * Dma::kRunBytes, run_off(u), r, sb), h, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (sb + 1 < nsb) {
         request(sb + 1);
