@@ -423,7 +423,7 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->x_h, (wide && mma) ? g.max_tokens * g.hidden : 0);
   A(&b->inter_h, (wide && mma && routed) ? sorted * g.intermediate : 0);
   A(&b->shared_inter_h, (wide && mma) ? g.max_tokens * g.intermediate : 0);
-  b->n_tile_list = (wide && mma && routed) ? 2 * (4 * (eb + 1) + 4) : 0;  // two lists (mfma_grouped_forward_partial)
+  b->n_tile_list = (wide && mma && routed) ? 4 * (eb + 1) + 4 : 0;
   A(&b->tile_list, b->n_tile_list);
   b->n_router_partial = (mma && routed && g.max_tokens >= kRouterGemmMinTokens && router_gemm_splits(g) > 1)
                             ? (size_t)router_gemm_splits(g) * g.max_tokens * g.num_experts
@@ -522,21 +522,19 @@ int xabe_moe_build_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_bu
   XABE_TRY(require_routed(b, "build_dispatch"));
   const xabe_moe_geometry& g = k->g;
   hipStream_t s = as_stream(stream);
-  // the matrix-core grouped GEMM's token-tile lists come out of the same launch where one workgroup holds every
-  // expert's count and first slot; the heights they were cut for are noted for the launch that reads them
+  // the matrix-core grouped GEMM's token-tile list comes out of the same launch where one workgroup holds every
+  // expert's count and first slot; the height it was cut for is noted for the launch that reads it
   TileListArgs tl;
   memset(&tl, 0, sizeof(tl));
-  b->tiles_bm = b->tiles_bm_up = 0;
+  b->tiles_bm = 0;
   b->tiles_capture = stream_capture_id(s);
   if (b->tiles_capture != 0) b->tiles_graph_owned = true;
-  int bm = 0, bm_up = 0, cap = 0;
-  const bool lists = mfma_tile_plan(k, b, &bm, &bm_up, &cap) && g.num_experts <= 512;
-  if (lists) {
+  int bm = 0, cap = 0;
+  const bool list = mfma_tile_plan(k, b, &bm, &cap) && g.num_experts <= 512;
+  if (list) {
     tl.capacity = cap;
     tl.bm = bm;
     tl.list = b->tile_list;
-    tl.bm_b = bm_up != bm ? bm_up : 0;
-    tl.list_b = b->tile_list + b->n_tile_list / 2;
   }
   if (b->n_align_chunks) {
     const unsigned chunks = (unsigned)b->n_align_chunks;
@@ -549,7 +547,7 @@ int xabe_moe_build_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_bu
     hipLaunchKernelGGL(k_align_place, dim3(chunks), dim3(256), 0, s, b->topk_ids, b->valid_tokens, (int)g.experts_per_token,
                        (int)g.num_experts, (int)b->n_sorted, b->align_hist, b->sorted_token_ids);
     XABE_HIP_TRY(hipGetLastError());
-    if (lists) b->tiles_bm = bm, b->tiles_bm_up = bm_up;
+    if (list) b->tiles_bm = bm;
     return XABE_OK;
   }
   if (g.max_tokens * g.experts_per_token <= (size_t)kAlignFusedMaxSelections && g.num_experts <= 512) {
@@ -557,7 +555,7 @@ int xabe_moe_build_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_bu
                        (int)g.num_experts, (int)g.block_size, (int)b->n_sorted, (int)b->n_expert_blocks, b->sorted_token_ids,
                        b->expert_ids, b->bucket_live, b->expert_counts, b->num_tokens_post_pad, tl);
     XABE_HIP_TRY(hipGetLastError());
-    if (lists) b->tiles_bm = bm, b->tiles_bm_up = bm_up;
+    if (list) b->tiles_bm = bm;
     return XABE_OK;
   }
   hipLaunchKernelGGL(k_align_count, dim3((unsigned)g.num_experts), dim3(256), 0, s, b->topk_ids, b->valid_tokens,

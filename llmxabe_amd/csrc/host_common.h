@@ -124,9 +124,9 @@ int rms_norm_rows_with_f16(void* stream, const float* x, const float* weight, fl
 // one-time, at handle creation: LDS limits of the kernels that ask for more than the static 64 KB (mfma.hip)
 int mfma_configure();
 bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int gate_q, int up_q, int down_q, bool routed);
-// token-tile heights of the routed down and gate/up launches of the pass as published, and the entries one of the two
-// lists in `tile_list` holds; false when these buffers carry no lists
-bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* bm_up, int* capacity);
+// token-tile height of the routed launches of the pass as published, and the entries `tile_list` holds; false when
+// these buffers carry no list
+bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* capacity);
 int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                                  xabe_quant_tensor up, xabe_quant_tensor down, const float* x);
 int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
@@ -142,7 +142,7 @@ struct xabe_moe_kernels {
   bool tensor_cores;
   bool exact_regime;
   bool force_community;
-  int mfma_form;  // matrix-core regime, routed launches: 0 chosen by width, 1 k_mfma_expert, 2 k_mfma_pc (mfma.hip)
+  int mfma_form;  // matrix-core regime, routed launches: 0 and 1 k_mfma_rows, 2 k_mfma_pc (mfma.hip)
   int device;
   int num_cus;
 };
@@ -182,13 +182,13 @@ struct xabe_moe_buffers {
   uint16_t* shared_inter_h;
   int32_t* tile_list;   // device-built tile schedule
   size_t n_tile_list;
-  // tile heights the lists were cut for by the last dispatch build (0: not built there), and the capture that
-  // build was recorded into (0: launched eagerly): a forward trusts the lists only inside the same capture, or
-  // eagerly after an eager build, so that a captured forward never depends on lists made outside its graph
-  int tiles_bm, tiles_bm_up;
+  // tile height the list was cut for by the last dispatch build (0: not built there), and the capture that
+  // build was recorded into (0: launched eagerly): a forward trusts the list only inside the same capture, or
+  // eagerly after an eager build, so that a captured forward never depends on a list made outside its graph
+  int tiles_bm;
   unsigned long long tiles_capture;
   // set for good once a dispatch build on these buffers has been recorded into a capture: a replay of that graph
-  // rewrites the device lists without touching the fields above, so from then on only a forward inside a capture
+  // rewrites the device list without touching the fields above, so from then on only a forward inside a capture
   // that holds its own build trusts them; eager forwards always make their own
   bool tiles_graph_owned;
   int32_t* seam_arrivals;  // decode widths: arrival counters of the seam's tail (zero between passes)

@@ -1,18 +1,14 @@
 // Matrix-core regime for prefill widths: a grouped GEMM over expert-sorted tokens that
-// dequantises Q6_K / Q8_0 weight tiles into LDS as fp16 and feeds v_mfma_f32_32x32x16_f16.
+// dequantises Q6_K / Q8_0 weights to fp16 and feeds v_mfma_f32_32x32x16_f16.
 // Takes the place of the reference's int8 tensor-core family
 // (crates/xabe-cuda/src/kernels/moe.rs:1316-1819, :2901-2943, :3152-3373) and of its
-// int8 shared-expert path (moe.rs:6389-6476); one prologue per format feeds the same
+// int8 shared-expert path (moe.rs:6389-6476); one reader per format feeds the same
 // MFMA body for gate, up and down, so there is no per-format asymmetry.
 //
-// Work decomposition.  A workgroup (4 wavefronts, 2x2) owns a 128-token x 128-weight-row
-// tile and walks the contraction in steps of 128.  For gate/up the 128 weight rows are 64
-// gate rows and the matching 64 up rows, so SwiGLU happens in registers.  Token tiles come
-// from a device-built list with one entry per 128-slot chunk of every *active* expert's
-// run of the dispatch table: experts with no tokens cost nothing, whatever the skew.
-// Workgroups are persistent and stride over (token tile, row tile) items.  (Token tiles are 64 rows while an
-// expert's share of a pass is small, and 384 rows on eight wavefronts for the routed gate/up launch of wide passes:
-// see k_mfma_expert's TBM.)
+// Two kernels: k_mfma_rows, and k_mfma_pc, an alternative form of the routed launches (same bits) kept for comparison.
+// Token tiles of the routed launches come from a device-built list with entries for the run of every *active* expert in
+// the dispatch table: experts with no tokens cost nothing, whatever the skew.  Workgroups are persistent and stride over
+// (token tile, row tile) items.
 //
 // Numerics.  Operands are fp16: activations rounded once; weights are (code - offset) exactly,
 // times fp16(d * sc * 256) -- the 2^8 keeps small scales out of the fp16 subnormal range and
@@ -26,7 +22,9 @@
 
 #include "device_common.h"
 #include "device_once.h"
+#include "digits.h"
 #include "host_common.h"
+#include "tile_list.h"
 
 namespace xabe {
 
@@ -35,21 +33,6 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 128;          // token rows per tile (64 in the narrow form: see k_mfma_expert's TBM)
-constexpr int kBR = 128;          // weight rows per tile
-constexpr int kBK = 128;          // contraction elements per step
-// The weight tile's rows are unpadded too, its 16-byte chunks XOR-swizzled by w_swizzle(row): any eight
-// consecutive rows spread one chunk over the eight 16-byte slots of a 128-byte bank line (the fragment reads:
-// lanes = rows), and two neighbouring rows put chunks 4j .. 4j + 3 into disjoint halves of it (the
-// dequantised stores: eight lanes = two rows x four units).  With padded rows (272 B) the reads were
-// conflict-free and the stores two-way conflicted: a fifth of the LDS cycles the counters showed; the bank
-// conflict counter now reads zero (the launches take the same time: LDS was not what held them).
-constexpr int kLd = kBK;
-// The activation tile goes from global memory straight into LDS (global_load_lds_dwordx4: no registers, no
-// store instructions), which writes a wavefront's 64 pieces contiguously, so its rows are unpadded (256 B)
-// and the 16-byte chunks of a row are stored XOR-swizzled by the row number instead: chunk c of row r sits at
-// position c ^ (r & 15), and 16 consecutive rows reading the same chunk hit 16 different bank groups.
-constexpr int kLdA = kBK;
 constexpr float kWScale = 256.0f;
 constexpr float kWScaleInv = 1.0f / 256.0f;
 
@@ -57,6 +40,7 @@ struct MfmaArgs {
   const uint8_t* w0;            // gate (NM=2) or down (NM=1) stack
   const uint8_t* w1;            // up stack (NM=2)
   size_t expert_bytes;          // bytes of one expert in a stack
+  size_t w_bytes;               // bytes of a whole stack
   const _Float16* a;            // activations, row-major [*][K]
   void* out;                    // NM=2: fp16 [*][n_rows]; NM=1: fp32 [*][n_rows]
   const int* valid_tokens;
@@ -66,6 +50,7 @@ struct MfmaArgs {
   int K;                        // contraction length
   int n_rows;                   // output columns per token (rows of one weight matrix)
   int top_k;
+  int tile_rows;                // unrouted: token rows of a tile
 };
 
 // SwiGLU's gate in the matrix-core regime: x / (1 + e^-x) from the hardware's exp2 and reciprocal (a few ulp of
@@ -74,11 +59,6 @@ __device__ __forceinline__ float silu_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896340736f * x));
 }
 
-__device__ __forceinline__ int w_swizzle(int row) {
-  return (row & 8) | ((row & 1) << 2) | ((row >> 1) & 3);
-}
-
-// ---- prologues: one 32-element unit of one weight row -> 32 halfs in LDS -----------------
 __device__ __forceinline__ u32x4 pack8(uint32_t c0, uint32_t c1, half2v off, half2v s) {
   // c0, c1: eight byte codes; returns eight halfs (code + 1024 - off) * s
   uint32_t p[4];
@@ -95,41 +75,6 @@ __device__ __forceinline__ u32x4 pack8(uint32_t c0, uint32_t c1, half2v off, hal
   }
   u32x4 r = {o[0], o[1], o[2], o[3]};
   return r;
-}
-
-// Q6_K unit (half h of a superblock, l8): codes at j*32 + l8*8 + i of that half.
-__device__ __forceinline__ void q6_unit_to_lds(const Q6Raw& r, int l8, _Float16* brow, int swz) {
-  const int is8 = (l8 >> 1) * 8;
-  const uint32_t slo = r.sc0 >> is8, shi = r.sc1 >> is8;
-  const float d = f16_bits_to_f32(r.dh) * kWScale;
-  const float ds[4] = {d * (float)(int8_t)(slo & 0xff), d * (float)(int8_t)((slo >> 16) & 0xff),
-                       d * (float)(int8_t)(shi & 0xff), d * (float)(int8_t)((shi >> 16) & 0xff)};
-  uint32_t c[2][4];
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    const uint32_t a = w ? r.qa1 : r.qa0, b = w ? r.qb1 : r.qb0, h = w ? r.qh1 : r.qh0;
-    c[w][0] = (a & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u);
-    c[w][1] = (b & 0x0F0F0F0Fu) | ((h << 2) & 0x30303030u);
-    c[w][2] = ((a >> 4) & 0x0F0F0F0Fu) | (h & 0x30303030u);
-    c[w][3] = ((b >> 4) & 0x0F0F0F0Fu) | ((h >> 2) & 0x30303030u);
-  }
-  const half2v off = {(_Float16)-1056.0f, (_Float16)-1056.0f};  // 1024 (perm bias) + 32 (code centre)
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const _Float16 sh = (_Float16)ds[j];
-    const half2v s = {sh, sh};
-    *reinterpret_cast<u32x4*>(brow + ((j * 4 + l8) ^ swz) * 8) = pack8(c[0][j], c[1][j], off, s);
-  }
-}
-
-// Q8_0 unit: one 34-byte block -> the row's chunks 4 du .. 4 du + 3.
-__device__ __forceinline__ void q8_unit_to_lds(const Q8Raw& r, int du, _Float16* brow, int swz) {
-  const _Float16 sh = (_Float16)(f16_bits_to_f32(r.dh) * kWScale);  // exact: d is fp16, scaled by 2^8
-  const half2v s = {sh, sh};
-  const half2v off = {(_Float16)-1152.0f, (_Float16)-1152.0f};      // 1024 (perm bias) + 128 (sign flip)
-#pragma unroll
-  for (int w = 0; w < 4; ++w)
-    *reinterpret_cast<u32x4*>(brow + ((du * 4 + w) ^ swz) * 8) = pack8(r.q[2 * w] ^ 0x80808080u, r.q[2 * w + 1] ^ 0x80808080u, off, s);
 }
 
 // Nothing moves across this point, in either direction, when the compiler schedules.
@@ -166,456 +111,18 @@ __device__ __forceinline__ void q6_issue(const uint8_t* blk, int half, int l8, Q
   r.sc = load_any<uint2>(blk + 192 + half * 8);
   r.dh = load_any<uint16_t>(blk + 208);
 }
-__device__ __forceinline__ void q6_finish(const Q6Pend& p, Q6Raw& r) {
-  r.qa0 = p.qa.x, r.qa1 = p.qa.y;
-  r.qb0 = p.qb.x, r.qb1 = p.qb.y;
-  r.qh0 = p.qh.x, r.qh1 = p.qh.y;
-  r.sc0 = p.sc.x, r.sc1 = p.sc.y;
-  r.dh = p.dh;
-}
 __device__ __forceinline__ void q8_issue(const uint8_t* blk, Q8Pend& r) {
   r.dh = load_any<uint16_t>(blk);
   r.lo = load_any<u32x4>(blk + 2);
   r.hi = load_any<u32x4>(blk + 18);
 }
-__device__ __forceinline__ void q8_finish(const Q8Pend& p, Q8Raw& r) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r.q[i] = p.lo[i], r.q[4 + i] = p.hi[i];
-  r.dh = p.dh;
-}
-
-template <int QUANT, int UNITS>
-struct WRaw {
-  typename std::conditional<QUANT == kQ6K, Q6Pend, Q8Pend>::type u[UNITS];
-};
-
-// Global loads of one contraction step into registers: the raw blocks of this thread's weight-row units.
-template <int QUANT, int UNITS>
-__device__ __forceinline__ void load_unit_w(int ks, int i, const uint8_t* const (&wrow)[UNITS], int du, WRaw<QUANT, UNITS>& wreg) {
-  {
-    if constexpr (QUANT == kQ6K) {
-      // step ks covers half (ks & 1) of superblock ks >> 1
-      q6_issue(wrow[i] + (size_t)(ks >> 1) * kQ6KBytes, ks & 1, du, wreg.u[i]);
-    } else {
-      q8_issue(wrow[i] + (size_t)(ks * 4 + du) * kQ8Bytes, wreg.u[i]);
-    }
-  }
-}
-template <int QUANT, int UNITS>
-__device__ __forceinline__ void load_step_w(int ks, const uint8_t* const (&wrow)[UNITS], int du, WRaw<QUANT, UNITS>& wreg) {
-#pragma unroll
-  for (int i = 0; i < UNITS; ++i) load_unit_w<QUANT, UNITS>(ks, i, wrow, du, wreg);
-}
-
-
-// TBM: token rows per tile, 384, 128 or 64.  The narrow form serves geometries whose experts see at most ~64 tokens
-// each (up to ~2000 tokens per pass): half the matrix instructions, activation bytes and output stores per
-// item, the same weight work.  A wavefront then owns 32 x 64 of the tile instead of 64 x 64; every output
-// element sees the same operands in the same order, so the forms give the same bits.
-// The tall form (384 token rows) is a workgroup of eight wavefronts, 4 x 2, each owning 96 x 64.  The vector
-// instructions of the dequantisation cost a SIMD more time than the matrix instructions they feed (39 % against 32 %
-// of the launch at 128 rows) and the two do not overlap, so what pays is dequantising a weight tile less often: at
-// ~256 rows per expert one tall tile holds all of an expert's rows, one dequantisation per expert and row tile
-// instead of two or three, one unit per thread and step instead of two.  A wavefront multiplies only the 32-row
-// blocks that hold live rows, and only live rows' activation pieces are requested.
-template <int QUANT, int NM, bool ROUTED, int TBM = 128>
-__global__ void __launch_bounds__(TBM == 384 ? 512 : 256, TBM == 64 ? 3 : 2) k_mfma_expert(MfmaArgs a) {
-  static_assert(TBM == 384 || TBM == 128 || TBM == 64, "token tile");
-  constexpr bool kTall = TBM == 384;
-  // Routed tiles are rarely full (an expert's run ends inside its last tile, and below ~1000 tokens most experts hold
-  // a handful of rows): a wavefront multiplies only its 32-row blocks that hold live rows, and only live rows'
-  // activation pieces are requested.  Same-box, per block: 512 tokens 304 -> 289 us, 2048: 482 -> 442, 4096: 716 -> 693.
-  constexpr bool kSkip = kTall || ROUTED;
-  constexpr int kThreads = kTall ? 512 : 256;
-  constexpr int kUnits = 512 / kThreads;          // weight-row units (32 elements of a row) per thread and step
-  constexpr int MI = kTall ? 3 : TBM / 64;        // 32-row blocks of the tile per wavefront
-  // first tile row of block mi of wavefront row wm: consecutive blocks in the short forms; in the tall form block b of
-  // the tile belongs to wavefront row b % 4, so that the live rows (the first `rows` of the tile) spread evenly
-  constexpr int kBlockStride = kTall ? 128 : 32;  // rows between a wavefront's consecutive blocks
-  constexpr int kWaveStride = kTall ? 32 : 32 * MI;  // rows between consecutive wavefront rows' first blocks
-  constexpr int kAPieces = TBM * 16 / kThreads;   // 16-byte activation pieces per thread and step
-  // 67.5 KB of LDS per workgroup at 128 token rows (two per CU), 137 KB at 384: dynamic, since the static limit is 64 KB
-  extern __shared__ __attribute__((aligned(16))) uint8_t mfma_smem[];
-  _Float16* sA = reinterpret_cast<_Float16*>(mfma_smem);
-  _Float16* sB = sA + TBM * kLdA;
-  // row tables, two sets (this item's and the next one's), each kTable = 3 * TBM words apart
-  constexpr int kTable = 3 * TBM;
-  int* sArow = reinterpret_cast<int*>(sB + kBR * kLd);  // activation row index of each tile row
-  int* sOrow = sArow + TBM;                             // output row index, or -1 for a dead row
-  float* sScale = reinterpret_cast<float*>(sOrow + TBM);
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  // (uniform, so that the count of live blocks is a scalar and dead ones are branched around)
-  const int wave = kSkip ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int valid = *a.valid_tokens;
-  const int n_ntiles = a.n_rows / (NM == 2 ? 64 : 128);
-  const int n_mtiles = ROUTED ? a.tile_list[0] : (valid + TBM - 1) / TBM;
-  const int total = n_mtiles * n_ntiles;
-  const int nks = a.K / kBK;
-  const size_t row_bytes = QUANT == kQ6K ? (size_t)(a.K / 256) * kQ6KBytes : (size_t)(a.K / 32) * kQ8Bytes;
-
-  // dequant mapping: unit u of LDS weight rows rb0 and rb0 + 64
-  const int du = tid & 3, rb0 = tid >> 2;
-
-  // Which items this workgroup takes.  Workgroup ids are dealt round-robin to the eight XCDs, each with its
-  // own L2: when there is work for every workgroup, XCD x takes a contiguous eighth of the token tiles and its
-  // workgroups walk that range together (token tile major), so an activation tile is fetched into one L2
-  // once instead of into all eight, and the token tiles of one expert reuse its weights from that L2.
-  const bool by_xcd = (gridDim.x & 7u) == 0 && total >= 2 * (int)gridDim.x && n_mtiles >= 8;
-  const int xcd = blockIdx.x & 7;
-  const int m_lo = by_xcd ? (int)((long long)n_mtiles * xcd / 8) : 0;
-  const int m_hi = by_xcd ? (int)((long long)n_mtiles * (xcd + 1) / 8) : n_mtiles;
-  const int first = by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-  const int stride = by_xcd ? (int)(gridDim.x >> 3) : (int)gridDim.x;
-  const int local_total = (m_hi - m_lo) * n_ntiles;
-  if (first >= local_total) return;
-
-  // One item = (token tile, weight-row tile).  Items are pipelined: the row tables, pointers and first loads of
-  // item i + 1 are set up inside the last contraction step of item i, so its epilogue and the latency of the
-  // next item's first loads overlap instead of adding up (the weight loads of a short contraction, 4 steps
-  // for the down projection, otherwise wait ~8 us per item with nothing to hide behind).
-  struct Item { int e, m0, rows, nt; };
-  auto decode = [&](int item) __attribute__((always_inline)) {
-    const int mt = m_lo + item / n_ntiles;
-    Item it{0, mt * TBM, min(TBM, valid - mt * TBM), item % n_ntiles};
-    if (ROUTED) {
-      // The tile's entry through the scalar unit: a vector load here would be waited for with a count of zero,
-      // i.e. together with every store the previous item's epilogue has just issued.
-      typedef int int4v __attribute__((ext_vector_type(4)));
-      int4v ent;
-      const int* p = a.tile_list + 4 + 4 * mt;  // 16-byte aligned: the list starts on an allocation boundary
-      asm volatile("s_load_dwordx4 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(ent) : "s"(p));
-      it.e = ent.x;
-      it.m0 = ent.y;
-      it.rows = ent.z;
-    }
-    return it;
-  };
-  // table entry of tile row `tid` (threads below TBM): activation row, output row (-1: dead), output scale.
-  // In two parts, so that nothing waits for a load it has just issued: the row's flat selection index is
-  // requested when the item is decoded, the entry is derived from it steps later.
-  auto table_flat = [&](const Item& it) __attribute__((always_inline)) {
-    // (an address that is always valid rather than a select on the loaded value, which would wait for it here)
-    return ROUTED ? a.sorted_token_ids[it.m0 + min(tid, it.rows - 1)] : 0;
-  };
-  auto table_scale = [&](const Item& it, int flat) __attribute__((always_inline)) {
-    return ROUTED && NM == 1 ? a.topk_weights[flat] : 1.0f;
-  };
-  auto table_entry = [&](const Item& it, int flat, int& arow, int& orow) __attribute__((always_inline)) {
-    arow = 0, orow = -1;
-    if (tid < it.rows) {
-      if (ROUTED) {
-        const int slot = it.m0 + tid;
-        if (NM == 2) { arow = flat / a.top_k; orow = slot; }
-        else { arow = slot; orow = flat; }
-      } else {
-        arow = orow = it.m0 + tid;
-      }
-    }
-  };
-  const ptrdiff_t up_minus_gate = NM == 2 ? a.w1 - a.w0 : 0;
-  const uint8_t* wrow[kUnits];   // weight rows this thread dequantises
-  uint32_t arow_off[kAPieces];   // activation chunks this thread moves, 16 bytes each per step: element offsets
-  [[maybe_unused]] uint32_t arow_live = ~0u;  // routed forms: bit i set when piece i belongs to a live row
-  auto set_wrow = [&](const Item& it) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kUnits; ++i) {
-      const int rb = rb0 + 64 * i;
-      const uint8_t* base = a.w0;
-      int wr;
-      if (NM == 2) {
-        const int half_n = rb >> 6, which = (rb >> 5) & 1, c = rb & 31;
-        // (arithmetic, not a select of the two pointers: the compiler turns that into a per-lane load from the
-        // kernel arguments, a memory operation in the middle of the steps)
-        base += which ? up_minus_gate : (ptrdiff_t)0;
-        wr = it.nt * 64 + half_n * 32 + c;
-      } else {
-        wr = it.nt * 128 + rb;
-      }
-      wrow[i] = base + (size_t)it.e * a.expert_bytes + (size_t)wr * row_bytes;
-    }
-  };
-  auto set_arow = [&](int buf, [[maybe_unused]] int live_rows) __attribute__((always_inline)) {
-    if constexpr (kSkip) arow_live = 0u;
-#pragma unroll
-    for (int i = 0; i < kAPieces; ++i) {
-      const int c = tid + kThreads * i;
-      // piece c of the tile lands at LDS byte 16 c: row c >> 4, position c & 15, which holds chunk pos ^ (row & 15)
-      const int row = c >> 4, chunk = (c & 15) ^ (row & 15);
-      arow_off[i] = (uint32_t)sArow[buf * kTable + row] * (uint32_t)a.K + (uint32_t)chunk * 8u;
-      if constexpr (kSkip) arow_live |= row < live_rows ? 1u << i : 0u;
-    }
-  };
-
-  // this step's activation tile: 1 KB pieces (eight per wavefront for 128 rows), global memory -> LDS.
-  // Written as assembly on purpose: the compiler's wait bookkeeping treats the instruction as one that may
-  // complete out of order with everything else, and answers any later wait for a weight register with "wait
-  // for all of memory", which stalls every other step on the pieces it has just requested.  Unseen by that
-  // bookkeeping, the pieces are covered by the step's second barrier (written by hand below), and the waits
-  // the compiler computes for the weight registers only ever come out too strict, by the pieces it did not count.
-  const uint32_t lds_a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)sA + (uint32_t)wave * 1024u;
-  auto move_a = [&](int ks) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kAPieces; ++i) {
-      if constexpr (kSkip) {
-        if (!(arow_live & (1u << i))) continue;  // (a dead row's slot in LDS keeps whatever it held: its products are dropped)
-      }
-      // (the tile's base in scalar registers plus a 32-bit byte offset per lane: one address register instead of two)
-      const uint32_t voff = (arow_off[i] + (uint32_t)ks * (uint32_t)kBK) * 2u;
-      const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_a + (uint32_t)(kThreads * 16) * i);  // + 16 * lane, by the hardware
-      lds_dma_16(a.a, voff, dst);
-    }
-  };
-
-  // In flight per step: the raw weight bytes of the next two steps (the HBM-cold ones), in w[ks & 1]; the
-  // activation tile (L2-warm) is moved during the step's own write phase, behind the dequantisation.  The contraction has an even
-  // number of steps (whole superblocks), so the step pairs are unrolled and no register is copied.
-  // (The down launch, NM = 1, has no registers to spare for the second step and keeps one in flight.)
-  // (tall form: one step ahead; its steps are long enough, and a second set of raw registers does not fit)
-  constexpr int kWDepth = kTall ? 1 : 2;
-  // load instructions one step's two units issue at the very least, one per separately addressed piece: Q6_K ql
-  // low, ql high, qh, scales, d; Q8_0 the two 16-byte halves of the codes and d.  (No two pieces of a unit
-  // are adjacent in memory except the scales and d, ten bytes that no single load covers, so the compiler cannot
-  // issue fewer; issuing more only makes the barrier's wait stricter.)
-  constexpr int kWLoadsAtLeast = (QUANT == kQ6K ? 5 : 3) * kUnits;
-  WRaw<QUANT, kUnits> w[kWDepth];
-
-  Item cur = decode(first);
-  {
-    int arow, orow;
-    if (tid < TBM) {
-      const int flat = table_flat(cur);
-      table_entry(cur, flat, arow, orow);
-      sArow[tid] = arow;
-      sOrow[tid] = orow;
-      sScale[tid] = table_scale(cur, flat);
-    }
-    __syncthreads();
-    set_wrow(cur);
-    set_arow(0, cur.rows);
-    // (fenced apart: the waits the compiler places in the steps are the strictest any path into them needs, and
-    // with these two sets of loads interleaved here it would make every step wait for its newest loads)
-    order_fence();
-    load_step_w<QUANT, kUnits>(0, wrow, du, w[0]);
-    order_fence();
-    if constexpr (kWDepth == 2) load_step_w<QUANT, kUnits>(1, wrow, du, w[kWDepth - 1]);
-    order_fence();
-  }
-  int buf = 0;
-  // (routed down launch: the output scales requested during the previous item, stored to this item's table at its
-  // start, by which time the load is many requests old and waiting for it waits for nothing else)
-  float carried_sc = 1.0f;
-  for (int item = first;; item += stride) {
-    if constexpr (ROUTED && NM == 1) {
-      if (item != first && tid < TBM) sScale[buf * kTable + tid] = carried_sc;
-    }
-    const bool has_next = item + stride < local_total;
-    const Item nxt = has_next ? decode(item + stride) : cur;
-    // (materialised here: a load sunk into the steps would put a full wait on one of their paths)
-    asm volatile("" ::"s"(nxt.e), "s"(nxt.m0), "s"(nxt.rows), "s"(nxt.nt));
-    // the next item's table entries: the flat index requested now, the scale two steps before the end, both
-    // stored to the other table in the last step
-    int n_flat = 0;
-    if (has_next && tid < TBM) n_flat = table_flat(nxt);
-
-    float16v acc[MI][2];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    auto step = [&](auto p_c, int ks) __attribute__((always_inline)) {
-      constexpr int P = decltype(p_c)::value % kWDepth;
-      // first barrier of the step: everyone has finished reading the previous step's tiles (LDS reads only: the
-      // weight loads in flight stay in flight)
-      order_fence();
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      order_fence();
-      if constexpr (ROUTED && NM == 1) {
-        // the next item's output scales, two steps before they are stored.  (First thing in the step: the
-        // compiler waits for everything in flight before it uses the flat index, and at this point that is the
-        // previous step's weight loads, a whole step old, and not yet this step's activation pieces.)
-        if (ks + kWDepth == nks && has_next && tid < TBM) {
-          int flat = n_flat;
-          asm volatile("" : "+v"(flat));
-          carried_sc = table_scale(nxt, flat);
-        }
-      }
-      move_a(ks);
-#pragma unroll
-      for (int i = 0; i < kUnits; ++i) {
-        const int rb = rb0 + 64 * i;
-        if constexpr (QUANT == kQ6K) {
-          Q6Raw r;
-          q6_finish(w[P].u[i], r);
-          q6_unit_to_lds(r, du, &sB[rb * kLd], w_swizzle(rb));
-        } else {
-          Q8Raw r;
-          q8_finish(w[P].u[i], r);
-          q8_unit_to_lds(r, du, &sB[rb * kLd], w_swizzle(rb));
-        }
-      }
-      if (ks == nks - 1 && has_next && tid < TBM) {
-        // (the other table's last reader, the previous item's epilogue, finished before this item's first barrier)
-        int n_arow, n_orow, flat = n_flat;
-        asm volatile("" : "+v"(flat));  // (pins the entry's arithmetic here: hoisted to the item's start it would wait for the load there)
-        table_entry(nxt, flat, n_arow, n_orow);
-        sArow[(buf ^ 1) * kTable + tid] = n_arow;
-        sOrow[(buf ^ 1) * kTable + tid] = n_orow;
-        if constexpr (!(ROUTED && NM == 1)) sScale[(buf ^ 1) * kTable + tid] = 1.0f;
-      }
-      // The raw weight bytes of the step after next (past the end of this item: the first steps of the next one),
-      // into the registers the dequantisation above has just released.  Issued after the activation pieces, so
-      // that the wait for those at the barrier leaves these in flight: they have two whole steps to arrive.
-      // (every step issues the same loads, so that the compiler's count of what is in flight is exact on every
-      // path: the last two steps of a workgroup's last item re-read two of its own steps and drop them)
-      const int ks_w = ks + kWDepth < nks ? ks + kWDepth : ks + kWDepth - nks;
-      if (ks + kWDepth == nks && has_next) set_wrow(nxt);
-      load_step_w<QUANT, kUnits>(ks_w, wrow, du, w[P]);
-      // Second barrier of the step, by hand: this wavefront's LDS stores and its activation pieces must have
-      // landed, the weight loads just issued need not.  Memory operations retire in order, so "all but the last
-      // kWLoadsAtLeast" covers the pieces; the count is a lower bound of the load instructions a step issues
-      // (one per field of each unit), so a miscount can only wait for more, never for less.
-      order_fence();
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kWLoadsAtLeast) : "memory");
-      order_fence();
-      if (ks + 1 == nks && has_next) set_arow(buf ^ 1, nxt.rows);
-      const _Float16* pa = &sA[(wm * kWaveStride + (lane & 31)) * kLdA];
-      // 32-row blocks of this wavefront that hold live rows (all of them in the unrouted forms)
-      const int nb = kSkip ? min(max((cur.rows - wm * kWaveStride + kBlockStride - 1) / kBlockStride, 0), MI) : MI;
-      const int swz = lane & 15, khalf = lane >> 5;  // (the row's low four bits are the lane's)
-      const _Float16* pb = &sB[(wn * 64 + (lane & 31)) * kLd];
-      const int wswz = w_swizzle(lane & 15);  // (the rows' low four bits are the lane's)
-      // Operand fragments one sub-step ahead, in two register sets: the four LDS reads of sub-step kk + 1 are
-      // issued before the four matrix instructions of sub-step kk, so their latency hides behind 128 cycles of
-      // matrix work instead of standing between every group of four.
-      // (tall form: one register set for the activation fragments, read at the start of their sub-step: a second set
-      // does not fit beside 96 accumulators, and the SIMD's other wavefront multiplies while this one waits for LDS)
-      constexpr int kASets = kTall ? 1 : 2;
-      half8 fa[kASets][MI], fb[2][2];
-      auto frags_a = [&](int kk, int set) __attribute__((always_inline)) {
-        const int apos = ((kk * 2 + khalf) ^ swz) * 8;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-          if (mi < nb) fa[set][mi] = *reinterpret_cast<const half8*>(pa + mi * kBlockStride * kLdA + apos);
-      };
-      auto frags_b = [&](int kk, int set) __attribute__((always_inline)) {
-        const int bpos = ((kk * 2 + khalf) ^ wswz) * 8;
-        fb[set][0] = *reinterpret_cast<const half8*>(pb + bpos);
-        fb[set][1] = *reinterpret_cast<const half8*>(pb + 32 * kLd + bpos);
-      };
-      if (nb > 0) {
-        frags_a(0, 0);
-        frags_b(0, 0);
-#pragma unroll
-        for (int kk = 0; kk < kBK / 16; ++kk) {
-          const int c = kk & 1;
-          if (kk + 1 < kBK / 16) {
-            if constexpr (kASets == 2) frags_a(kk + 1, c ^ 1);
-            frags_b(kk + 1, c ^ 1);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int mi = 0; mi < MI; ++mi) {
-            if (mi < nb) {
-              acc[mi][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[c % kASets][mi], fb[c][0], acc[mi][0], 0, 0, 0);
-              acc[mi][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[c % kASets][mi], fb[c][1], acc[mi][1], 0, 0, 0);
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (kASets == 1) {
-            if (kk + 1 < kBK / 16) frags_a(kk + 1, 0);
-          }
-        }
-      }
-    };
-    if constexpr (kWDepth == 2) {
-      // (at least one pair of steps, and written so: a path around the loop would count for the compiler's waits
-      // after it, and on that path the loads issued just before the loop are the newest)
-      int ks = 0;
-      do {
-        step(std::integral_constant<int, 0>{}, ks);
-        step(std::integral_constant<int, 1>{}, ks + 1);
-        ks += 2;
-      } while (ks < nks);
-    } else {
-#pragma unroll 1
-      for (int ks = 0; ks < nks; ++ks) step(std::integral_constant<int, 0>{}, ks);
-    }
-
-    // epilogue.  acc[mi][ni][v]: tile row (v/4)*8 + (lane/32)*4 + v%4, tile column lane%32
-    // (transposing the tile through LDS so that every lane stores 16 bytes of a row was measured: two more
-    // barriers per item and the extra registers cost more than the 48 fewer store instructions gave; so was
-    // the transposed product, weights as the first operand, whose lanes hold four consecutive columns of one
-    // token row: a quarter of the store instructions, but each touches 32 rows' cache lines with 32 bytes
-    // instead of two rows' with 128, and the block took 1365 against 1333 us at 8192 tokens)
-    // (the rows' table entries are all read first: one LDS round trip for the item instead of one per row)
-    // (tall form: one 32-row block at a time, skipping blocks without live rows: all three blocks' entries at once
-    // do not fit the registers beside 96 accumulators)
-    auto store_blocks = [&](auto first_c, auto count_c) __attribute__((always_inline)) {
-      constexpr int M0 = decltype(first_c)::value, MN = decltype(count_c)::value;
-      int orows[MN][16];
-      [[maybe_unused]] float scs[MN][16];
-#pragma unroll
-      for (int mi = 0; mi < MN; ++mi) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = wm * kWaveStride + (M0 + mi) * kBlockStride + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-          orows[mi][v] = sOrow[buf * kTable + r];
-          if (NM == 1) scs[mi][v] = sScale[buf * kTable + r];
-        }
-      }
-#pragma unroll
-      for (int mi = 0; mi < MN; ++mi) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int orow = orows[mi][v];
-          if (orow < 0) continue;
-          if (NM == 2) {
-            const int col = cur.nt * 64 + wn * 32 + (lane & 31);
-            const float g = acc[M0 + mi][0][v] * kWScaleInv, u = acc[M0 + mi][1][v] * kWScaleInv;
-            static_cast<_Float16*>(a.out)[(size_t)orow * a.n_rows + col] = (_Float16)(silu_fast(g) * u);
-          } else {
-            const float sc = scs[mi][v];
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni) {
-              const int col = cur.nt * 128 + wn * 64 + ni * 32 + (lane & 31);
-              static_cast<float*>(a.out)[(size_t)orow * a.n_rows + col] = sc * (acc[M0 + mi][ni][v] * kWScaleInv);
-            }
-          }
-        }
-      }
-    };
-    if constexpr (kTall) {
-      const int nb = min(max((cur.rows - wm * kWaveStride + kBlockStride - 1) / kBlockStride, 0), MI);
-      if (nb > 0) store_blocks(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-      if (nb > 1) store_blocks(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
-      if (nb > 2) store_blocks(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
-    } else if constexpr (kSkip) {
-      const int nb = min(max((cur.rows - wm * kWaveStride + kBlockStride - 1) / kBlockStride, 0), MI);
-      if (nb == MI) store_blocks(std::integral_constant<int, 0>{}, std::integral_constant<int, MI>{});
-      else if (MI == 2 && nb == 1) store_blocks(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
-    } else {
-      store_blocks(std::integral_constant<int, 0>{}, std::integral_constant<int, MI>{});
-    }
-    if (!has_next) break;
-    cur = nxt;
-    buf ^= 1;
-  }
-}
 
 // ------------------------------------------------------------------------------------------------------------
 // The same grouped GEMM with the wavefronts of a workgroup specialised: an alternative form of the routed launches,
-// selected with xabe_moe_kernels_set_mfma_form(k, 2).  Same bits as k_mfma_expert; measured within 0-7 % of it and
-// never ahead (8192 tokens: gate/up 461 against 421 us, down 333 against 308), so it is not the default.  It is kept
+// selected with xabe_moe_kernels_set_mfma_form(k, 2).  Same bits as k_mfma_rows, and behind it everywhere (8192 tokens:
+// gate/up 461 against 357 us, down 333 against 287), so it is not the default.  It is kept
 // because it is the measured answer to "would wavefronts that only dequantise beside wavefronts that only multiply
-// overlap the two kinds of work": they do not.  On a SIMD the producers' vector instructions and the consumers'
-// matrix instructions take turns,
-// so what decides the time is the sum of the two per token row, and that sum is smallest for the tallest token tile
-// (one dequantisation per expert), whose accumulators only fit a few fat wavefronts: k_mfma_expert's 384-row form.
+// overlap the two kinds of work": less than one wavefront that does both does, instruction by instruction.
 //
 // A workgroup is sixteen wavefronts with two jobs:
 //   consumers (wavefronts 0-7, 2 row halves x 4 column quarters): request the activation tile three steps ahead
@@ -627,11 +134,10 @@ __global__ void __launch_bounds__(TBM == 384 ? 512 : 256, TBM == 64 ? 3 : 2) k_m
 // consumer's pieces were requested three steps earlier, a producer's raw bytes two to four steps earlier, and each
 // kind of wavefront counts only its own loads (the wait counters are per wavefront).
 //
-// The tile is 128 token rows x 256 weight rows (gate/up: 128 + 128): twice k_mfma_expert's weight rows per
-// activation byte (with 128 weight rows and a one-step-ahead activation tile the consumers waited for L2 every step:
-// 623 us).
-// Per output element the operands and the order of the matrix instructions are k_mfma_expert's (ascending
-// contraction index, 16 elements per instruction), so the bits are the same.
+// The tile is 128 token rows x 256 weight rows (gate/up: 128 + 128; with 128 weight rows and an activation tile one step
+// ahead the consumers waited for L2 every step: 623 us).
+// Per output element the operands and the order of the matrix instructions are k_mfma_rows's (see there which 16 elements
+// an instruction takes), so the bits are the same.
 // A Q6_K unit (32 codes of one row: 8 at each of four places 32 elements apart) spans two steps: its raw registers
 // are loaded once per 128-element block and dequantised a half at a time.
 // LDS: rows of 64 halfs (128 bytes: two rows to a 256-byte line of the 64 banks), 16-byte chunks XOR-swizzled by
@@ -711,7 +217,7 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
   const int nks = a.K / kPK;  // a multiple of four (whole superblocks), at least eight (checked by the host)
   const size_t row_bytes = QUANT == kQ6K ? (size_t)(a.K / 256) * kQ6KBytes : (size_t)(a.K / 32) * kQ8Bytes;
 
-  // which items this workgroup takes: k_mfma_expert's dealing (an XCD walks a contiguous eighth of the token tiles)
+  // which items this workgroup takes (an XCD walks a contiguous eighth of the token tiles)
   const bool by_xcd = (gridDim.x & 7u) == 0 && total >= 2 * (int)gridDim.x && n_mtiles >= 8;
   const int xcd = blockIdx.x & 7;
   const int m_lo = by_xcd ? (int)((long long)n_mtiles * xcd / 8) : 0;
@@ -938,7 +444,7 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
         const int wswz = aswz;
         half8 fa[2][2], fb[2][2];
         auto frags = [&](int kk, int set) __attribute__((always_inline)) {
-          const int apos = ((kk * 2 + khalf) ^ aswz) * 8, bpos = ((kk * 2 + khalf) ^ wswz) * 8;
+          const int piece = (kk >> 1) * 4 + khalf * 2 + (kk & 1), apos = (piece ^ aswz) * 8, bpos = (piece ^ wswz) * 8;
 #pragma unroll
           for (int mi = 0; mi < 2; ++mi)
             if (mi < nb) fa[set][mi] = *reinterpret_cast<const half8*>(pa + mi * 64 * kPK + apos);
@@ -1001,6 +507,612 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// The grouped GEMM.  Each wavefront owns 32 weight rows of the tile (gate/up: 16 gate rows and the matching 16 up rows) for
+// all of the tile's token rows: it brings those rows' raw bytes into an LDS slot of its own, reads its lanes' share into
+// registers, makes halfs of it there, eight at a time as a matrix instruction wants them, and no dequantised weight ever
+// goes through LDS or past a barrier.  The activations are what the wavefronts share: steps of 64 contraction elements go
+// from global memory straight into a ring in LDS, which leaves one barrier per step.
+//
+// What bounds it (gate/up of the dense sibling, 2048 x 5120 -> 2 x 17408, 730 GFLOP): the matrix instructions alone take
+// 450 us at the 1620 TFLOP/s that the chip holds on random data (it lowers its clock: power, not issue slots), the
+// kernel 750 (57 % of its cycles are matrix instructions), the kernel that dequantised 128 x 128 tiles through LDS
+// 969.  Added one by one to the matrix instructions: making halfs 75 us, activation reads 48, raw weight reads 93, the
+// requests 162.  Hence
+//  - vector instructions between the matrix instructions, up to four of which cost one nothing (five parts of a chunk's
+//    weights spread over its NB matrix instructions, w_part);
+//  - tall tiles: a weight is made into a half once per 192 rows.  Eight wavefronts of 192 x 32 accumulators fill the
+//    registers of a CU's SIMDs; 256 rows measured the same on the dense pass (753 us) and behind on the routed (377
+//    against 357 us at 8192 tokens), 128 rows on four wavefronts and two workgroups per CU 652 us;
+//  - requests made long before their use and waited for by count, never by draining ("all but the newest n", Requests);
+//  - the two wavefronts of a SIMD make their requests and read raw weights at different times (`early`): behind a barrier
+//    both would leave the matrix pipe idle together;
+//  - LDS reads on their own width's boundary (any other takes 64 cycles), rows spread over the banks by the windows' odd
+//    count of sixteen bytes, activations by pc_swizzle.
+// A short contraction (down of the routed model: two superblocks) is bound by what an item costs besides: its stores, which
+// the requests' waits count like any memory operation, 287 us at 8192 tokens against 333 before.
+//
+// Which elements a matrix instruction takes: chunk c = 2 j + m of a half superblock is elements 32 j + 16 h + 8 m + [0, 8) for
+// the lanes of half h, since a lane's sixteen consecutive codes then come out of one 16-byte read; the activations'
+// fragments follow (`frag`).  Per output element the order is fixed, whatever the tile.
+//
+// Forms: wide (six blocks of 32 rows, eight wavefronts, a workgroup per CU) and narrow (two blocks, four wavefronts, three
+// workgroups per CU: a tile's start and end are then beside other tiles' steps).  Where the line lies: routed_tile_rows,
+// unrouted_wide.
+constexpr int kSK = 64;                          // contraction elements per activation step
+constexpr int kNarrowRows = 64;                  // token rows of a tile, narrow form
+constexpr int kWideRows = 192;                   // token rows of a tile at most, wide form
+constexpr int kWRows = 32;                       // weight rows of a wavefront
+constexpr int kBlockBytes = 32 * kSK * 2;        // 32 token rows of an activation step in LDS
+
+// A weight row's window in LDS: a superblock of 210 bytes from the word boundary below (Q6_K), four blocks of 34 bytes from a
+// 16-byte boundary (Q8_0, whose superblocks of 272 bytes are taken in two windows: 136 = 8 modulo 16).
+template <int QUANT, int MI>
+struct WWindow {
+  // (Q6_K: fourteen pieces hold it, fifteen spread the rows over the LDS banks; the narrow form has no room for the fifteenth)
+  static constexpr int kPieces = QUANT == kQ6K ? (MI > 2 ? 15 : 14) : 9;
+  static constexpr int kPerSb = QUANT == kQ6K ? 1 : 2, kSpan = QUANT == kQ6K ? kQ6KBytes : 4 * kQ8Bytes;
+  static constexpr uint32_t kStart = QUANT == kQ6K ? 3 : 15;  // what windows start on, less one
+  static constexpr int kRunBytes = 16 * kPieces * 16;         // sixteen rows
+  static constexpr int kRunInstr = (16 * kPieces + 63) / 64;  // DMA instructions of a run
+};
+
+// 128 contraction elements of a weight row as a lane of half h holds them: sixteen of every thirty-two, 32 j + 16 h + [0, 16),
+// which a matrix instruction's chunk c = 2 j + m takes eight at a time: 32 j + 16 h + 8 m + [0, 8).
+template <int QUANT>
+struct WHalf;
+template <>
+struct WHalf<kQ6K> {
+  u32x4 qa, qb, qh;
+  uint2 sc;
+  uint32_t d;
+};
+template <>
+struct WHalf<kQ8_0> {
+  u32x4 q[4];
+  uint32_t d[4];
+};
+// Reads on their own boundaries (see sb_read_slot in digits.h), words shifted by the half word that is left where rows do
+// not start on words.
+__device__ __forceinline__ uint2 lds_pair(const uint8_t* p) { return *static_cast<const uint2*>(__builtin_assume_aligned(p, 8)); }
+__device__ __forceinline__ u32x4 lds_quad(const uint8_t* p) { return *static_cast<const u32x4*>(__builtin_assume_aligned(p, 16)); }
+__device__ __forceinline__ u32x4 words_from(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t w4, uint32_t shift) {
+  const u32x4 r = {__builtin_amdgcn_alignbit(w1, w0, shift), __builtin_amdgcn_alignbit(w2, w1, shift),
+                   __builtin_amdgcn_alignbit(w3, w2, shift), __builtin_amdgcn_alignbit(w4, w3, shift)};
+  return r;
+}
+__device__ __forceinline__ u32x4 lds_quad_shifted(const uint8_t* p, uint32_t shift) {
+  const u32x4 v = lds_quad(p);
+  return words_from(v[0], v[1], v[2], v[3], lds_word(p + 16), shift);
+}
+// half `half` of the superblock whose window lies at `p`, `mis` (0 or 2) bytes in; `even`: 0 in every lane
+__device__ __forceinline__ void w_read(const uint8_t* p, uint32_t mis, bool even, int half, int h, WHalf<kQ6K>& r) {
+  const uint8_t *q = p + 64 * half + 16 * h, *qh = p + 128 + 32 * half + 16 * h, *sc = p + 192 + 8 * half;
+  if (even) {
+    r.qa = lds_quad(q), r.qb = lds_quad(q + 32), r.qh = lds_quad(qh), r.sc = lds_pair(sc);
+  } else {
+    const uint32_t shift = mis << 3;
+    r.qa = lds_quad_shifted(q, shift), r.qb = lds_quad_shifted(q + 32, shift), r.qh = lds_quad_shifted(qh, shift);
+    const uint2 v = lds_pair(sc);
+    r.sc = make_uint2(__builtin_amdgcn_alignbit(v.y, v.x, shift), __builtin_amdgcn_alignbit(lds_word(sc + 8), v.y, shift));
+  }
+  r.d = *reinterpret_cast<const uint16_t*>(p + mis + 208);
+}
+// four blocks from `p` (an 8-byte boundary): their codes start 2, 4, 6 and 0 bytes past one
+__device__ __forceinline__ void w_read(const uint8_t* p, uint32_t, bool, int, int h, WHalf<kQ8_0>& r) {
+  const uint8_t* q = p + 16 * h;
+  const uint2 a = lds_pair(q), b = lds_pair(q + 8), c = lds_pair(q + 40), d = lds_pair(q + 72), e = lds_pair(q + 80);
+  r.q[0] = words_from(a.x, a.y, b.x, b.y, lds_word(q + 16), 16);
+  r.q[1] = u32x4{lds_word(q + 36), c.x, c.y, lds_word(q + 48)};
+  r.q[2] = words_from(lds_word(q + 68), d.x, d.y, e.x, e.y, 16);
+  const uint2 f = lds_pair(q + 104), g = lds_pair(q + 112);
+  r.q[3] = u32x4{f.x, f.y, g.x, g.y};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r.d[j] = *reinterpret_cast<const uint16_t*>(p + 34 * j);
+}
+// fp16(d sc 2^8) of the lane's sixteens 2 p and 2 p + 1.  `pick`: where the lane finds their scales among four bytes
+__device__ __forceinline__ uint32_t w_scale_bytes(int h) { return h ? 0x04030401u : 0x04020400u; }
+__device__ __forceinline__ half2v w_scales(const WHalf<kQ6K>& r, int p, uint32_t pick) {
+  half2v s = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, (p ? r.sc.y : r.sc.x) ^ 0x80808080u, pick));
+  s = s + half2v{(_Float16)-1152.0f, (_Float16)-1152.0f};
+  s = s * half2v{(_Float16)kWScale, (_Float16)kWScale};
+  const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
+  return s * half2v{d, d};
+}
+__device__ __forceinline__ half2v w_scales(const WHalf<kQ8_0>& r, int p, uint32_t) {
+  const half2v d = {__builtin_bit_cast(_Float16, (uint16_t)r.d[2 * p]), __builtin_bit_cast(_Float16, (uint16_t)r.d[2 * p + 1])};
+  return d * half2v{(_Float16)kWScale, (_Float16)kWScale};
+}
+// The lane's eight weights of chunk c in five parts of a few instructions each, for a caller that puts matrix instructions
+// between them: part 0 the scales of four chunks, 1 and 2 four codes each, 3 and 4 those as halfs.
+struct WChunk {
+  half2v scales;
+  uint32_t code[2], out[4];
+};
+constexpr int kWParts = 5;
+template <int C>
+__device__ __forceinline__ uint32_t w_codes(const WHalf<kQ6K>& r, int w) {
+  constexpr int j = C >> 1, m = C & 1;
+  const uint32_t a = r.qa[2 * m + w], b = r.qb[2 * m + w], q = r.qh[2 * m + w];
+  return j == 0   ? (a & 0x0F0F0F0Fu) | ((q << 4) & 0x30303030u)
+         : j == 1 ? (b & 0x0F0F0F0Fu) | ((q << 2) & 0x30303030u)
+         : j == 2 ? ((a >> 4) & 0x0F0F0F0Fu) | (q & 0x30303030u)
+                  : ((b >> 4) & 0x0F0F0F0Fu) | ((q >> 2) & 0x30303030u);
+}
+template <int C>
+__device__ __forceinline__ uint32_t w_codes(const WHalf<kQ8_0>& r, int w) {
+  return r.q[C >> 1][2 * (C & 1) + w] ^ 0x80808080u;
+}
+template <int C, int PART, int QUANT>
+__device__ __forceinline__ void w_part(const WHalf<QUANT>& r, uint32_t pick, WChunk& k) {
+  if constexpr (PART == 0) {
+    if constexpr ((C & 3) == 0) k.scales = w_scales(r, C >> 2, pick);
+  } else if constexpr (PART <= 2) {
+    k.code[PART - 1] = w_codes<C>(r, PART - 1);
+  } else {
+    constexpr int w = PART - 3;
+    const _Float16 off = QUANT == kQ6K ? (_Float16)-1056.0f : (_Float16)-1152.0f;  // (1024 of the byte's placing, and the codes' centre)
+    const _Float16 s = (C >> 1) & 1 ? k.scales.y : k.scales.x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      half2v v = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, k.code[w], i ? 0x04030402u : 0x04010400u));
+      v = (v + half2v{off, off}) * half2v{s, s};
+      k.out[2 * w + i] = __builtin_bit_cast(uint32_t, v);
+    }
+  }
+}
+template <int C, int PART = 0, int QUANT>
+__device__ __forceinline__ void w_parts_from(const WHalf<QUANT>& r, uint32_t pick, WChunk& k) {
+  w_part<C, PART>(r, pick, k);
+  if constexpr (PART + 1 < kWParts) w_parts_from<C, PART + 1>(r, pick, k);
+}
+__device__ __forceinline__ half8 w_halfs(const WChunk& k) {
+  const u32x4 v = {k.out[0], k.out[1], k.out[2], k.out[3]};
+  return __builtin_bit_cast(half8, v);
+}
+
+// All but the newest N memory operations of this wavefront have completed.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// lds_dma_16 for the lanes of `lanes`, which may be none: the instruction is issued and counted all the same, so that the
+// number of memory operations in flight does not depend on the data.  (Every lane of the wavefront is active here.)
+__device__ __forceinline__ void lds_dma_16_lanes(const void* base, uint32_t voff, uint32_t dst, uint32_t lanes_lo, uint32_t lanes_hi) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %4\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(voff),
+               "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)), "s"(__builtin_amdgcn_readfirstlane(lanes_lo)),
+               "s"(__builtin_amdgcn_readfirstlane(lanes_hi)) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+// One dword per lane from `base` + `voff` into LDS at `dst` + 4 * lane (see lds_dma_16).
+__device__ __forceinline__ void lds_dma_4(const void* base, uint32_t voff, uint32_t dst) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base),
+               "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
+}
+
+
+template <int MI>
+constexpr int kRing = MI > 2 ? 4 : 3;  // steps of activations in LDS
+// The requests of a superblock's sixteen chunks, in order.  Activations: after the barrier that frees a place in the ring
+// (chunks 3, 7, 11, 15), the step that goes there, PI instructions.  Weights: behind them from the barrier on that follows the
+// read that empties the slot, two instructions per chunk.  Memory operations complete in order, so a wait for one is
+// "all but those made after it".
+template <int QUANT, int PI>
+struct Requests {
+  static constexpr int a_at(int c) { return (c & 3) == 3 ? PI : 0; }
+  static constexpr int w_at(int c) { return QUANT == kQ6K ? ((c + 1) & 15) < 4 ? 2 : 0 : ((c + 1) & 7) < 3 ? 2 : 0; }
+  // how many are made in chunks [lo, hi)
+  static constexpr int between(int lo, int hi) {
+    int n = 0;
+    for (int c = lo; c < hi; ++c) n += a_at(c + 16) + w_at(c + 16);
+    return n;
+  }
+  // at the start of chunk c: those made after the activations of chunk r, and after the latest weights
+  static constexpr int after_a(int r, int c) { return w_at(r + 16) + between(r + 1, c); }
+  static constexpr int after_w(int c) {
+    int last = c - 1;
+    while (w_at(last + 16) == 0) --last;
+    return between(last + 1, c);
+  }
+};
+template <int QUANT, int MI, int WAVES>
+constexpr size_t mfma_rows_lds() {
+  return (size_t)kRing<MI> * MI * kBlockBytes + (size_t)WAVES * 2 * WWindow<QUANT, MI>::kRunBytes + (size_t)2 * 32 * MI * sizeof(int);
+}
+template <int MI, int WAVES>
+constexpr int kWgsPerCu = MI > 2 ? 1 : 3;
+
+template <int QUANT, int NM, bool ROUTED, int MI, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_rows(MfmaArgs a) {
+  constexpr int kTM = 32 * MI;                    // token rows of a tile at most
+  constexpr int kTR = WAVES * kWRows;             // weight rows of a tile
+  constexpr int kSlot = MI * kBlockBytes;         // an activation step in LDS
+  constexpr int kRing = xabe::kRing<MI>;
+  using Window = WWindow<QUANT, MI>;
+  constexpr int kRun = Window::kRunBytes, kRunInstr = Window::kRunInstr;
+  constexpr bool kScaled = ROUTED && NM == 1;
+  extern __shared__ __attribute__((aligned(16))) uint8_t mfma_smem[];
+  uint8_t* const sA = mfma_smem;
+  uint8_t* const sW = sA + kRing * kSlot;
+  // flat selection indices of an item's rows: gate/up, this item's and the next one's; down, this item's and their weights
+  int* const sId = reinterpret_cast<int*>(sW + WAVES * 2 * kRun);
+  [[maybe_unused]] float* const sScale = reinterpret_cast<float*>(sId + kTM);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, col = lane & 31;
+  const int valid = __builtin_amdgcn_readfirstlane(*a.valid_tokens);
+  const int n_ntiles = a.n_rows / (kTR / NM);
+  const int tile_rows = a.tile_rows;
+  const int n_mtiles = ROUTED ? a.tile_list[0] : (valid + tile_rows - 1) / tile_rows;
+  const int total = n_mtiles * n_ntiles;
+  const int nsteps = a.K / kSK, nsb = a.K / 256;
+  const uint32_t row_bytes = QUANT == kQ6K ? (uint32_t)(a.K / 256) * kQ6KBytes : (uint32_t)(a.K / 32) * kQ8Bytes;
+
+  // Which items this workgroup takes.  Workgroup ids are dealt round-robin to the eight XCDs, each with its own L2: when
+  // there is work for every workgroup, XCD x takes a contiguous eighth of the items (token tile major) and its workgroups
+  // walk that range together, so an activation tile is fetched into one L2 instead of into all eight, and the token tiles
+  // of one expert reuse its weights from that L2.
+  const bool by_xcd = (gridDim.x & 7u) == 0 && total >= 2 * (int)gridDim.x;
+  const int xcd = blockIdx.x & 7;
+  const int lo = by_xcd ? (int)((long long)total * xcd / 8) : 0, hi = by_xcd ? (int)((long long)total * (xcd + 1) / 8) : total;
+  const int first = lo + (by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x);
+  const int stride = by_xcd ? (int)(gridDim.x >> 3) : (int)gridDim.x;
+  if (first >= hi) return;
+
+  struct Item { int e, m0, rows, nt; };
+  auto decode = [&](int item) __attribute__((always_inline)) {
+    const int mt = item / n_ntiles;
+    Item it{0, mt * tile_rows, min(tile_rows, valid - mt * tile_rows), item % n_ntiles};
+    if (ROUTED) {
+      typedef int int4v __attribute__((ext_vector_type(4)));
+      int4v ent;
+      const int* p = a.tile_list + 4 + 4 * mt;
+      asm volatile("s_load_dwordx4 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(ent) : "s"(p));
+      it.e = ent.x;
+      it.m0 = ent.y;
+      it.rows = min(ent.z, kTM);  // (a list is cut for its launch; LDS holds no more)
+    }
+    return it;
+  };
+
+  // ---- weights: the wavefront's slot
+  uint8_t* const slot = sW + wave * 2 * kRun;
+  const uint32_t slot_lds = lds_address(slot);
+  uint32_t w_off[kRunInstr];  // the lane's piece of each instruction of a run
+#pragma unroll
+  for (int i = 0; i < kRunInstr; ++i) {
+    const int pc = min(64 * i + lane, 16 * Window::kPieces - 1);
+    w_off[i] = (uint32_t)(pc / Window::kPieces) * row_bytes + (uint32_t)(pc % Window::kPieces) * 16;
+  }
+  const uint8_t *w_base0, *w_base1;  // the runs' first rows, of the item the weight stream is in
+  uint32_t w_last0, w_last1;         // the last whole piece of the stack from there
+  auto set_w = [&](const Item& it) __attribute__((always_inline)) {
+    const int r0 = it.nt * (kTR / NM) + wave * (kWRows / NM);
+    const size_t off0 = (size_t)it.e * a.expert_bytes + (size_t)r0 * row_bytes;
+    const size_t off1 = NM == 2 ? off0 : off0 + (size_t)16 * row_bytes;
+    w_base0 = a.w0 + off0;
+    w_base1 = (NM == 2 ? a.w1 : a.w0) + off1;
+    w_last0 = (uint32_t)min(a.w_bytes - 16 - off0, (size_t)0x7fffffff);
+    w_last1 = (uint32_t)min(a.w_bytes - 16 - off1, (size_t)0x7fffffff);
+  };
+  uint32_t w_at = 0;  // the requested window's start in its rows
+  auto request_w = [&](auto i_c) __attribute__((always_inline)) {  // instruction i of either run
+    constexpr int i = decltype(i_c)::value, kLastLanes = 16 * Window::kPieces - 64 * (kRunInstr - 1);
+    constexpr uint64_t kLast = kLastLanes == 64 ? ~0ull : (1ull << kLastLanes) - 1;
+    const uint32_t voff = (w_off[i] + w_at) & ~Window::kStart;
+    if (i + 1 < kRunInstr || kLastLanes == 64) {
+      lds_dma_16(w_base0, min(voff, w_last0), slot_lds + i * 1024);
+      lds_dma_16(w_base1, min(voff, w_last1), slot_lds + kRun + i * 1024);
+    } else {
+      lds_dma_16_lanes(w_base0, min(voff, w_last0), slot_lds + i * 1024, (uint32_t)kLast, (uint32_t)(kLast >> 32));
+      lds_dma_16_lanes(w_base1, min(voff, w_last1), slot_lds + kRun + i * 1024, (uint32_t)kLast, (uint32_t)(kLast >> 32));
+    }
+  };
+  auto request_w_all = [&]() __attribute__((always_inline)) {
+    request_w(std::integral_constant<int, 0>{});
+    request_w(std::integral_constant<int, 1>{});
+    request_w(std::integral_constant<int, 2>{});
+    if constexpr (kRunInstr > 3) request_w(std::integral_constant<int, kRunInstr - 1>{});
+  };
+  const uint32_t my_row = (uint32_t)(col & 15) * row_bytes;
+  const bool even_rows = QUANT == kQ6K && (row_bytes & 3) == 0;  // (then a superblock starts on a word in every row or in none)
+  const uint8_t* const my_window = slot + (col >> 4) * kRun + (col & 15) * (Window::kPieces * 16);
+  auto read_w = [&](int u, int half, WHalf<QUANT>& r) __attribute__((always_inline)) {  // half `u` of the contraction out of the slot
+    const uint32_t at = (uint32_t)(QUANT == kQ6K ? u >> 1 : u) * Window::kSpan, mis = (my_row + at) & Window::kStart;
+    if constexpr (QUANT == kQ6K) w_read(my_window, mis, even_rows && (at & 2) == 0, half, h, r);
+    else w_read(my_window + mis, 0, false, half, h, r);
+  };
+  // (Q6_K) the window just landed is the last of its rows: what no piece inside the tensor holds, where a row ends it
+  auto patch_w = [&]() __attribute__((always_inline)) {
+    const size_t run_bytes = (size_t)16 * row_bytes;
+    if (w_base0 + run_bytes == a.w0 + a.w_bytes) patch_window<kQ6K>(a.w0, a.w_bytes - kQ6KBytes, slot + 15 * (Window::kPieces * 16));
+    if (w_base1 + run_bytes == (NM == 2 ? a.w1 : a.w0) + a.w_bytes)
+      patch_window<kQ6K>(NM == 2 ? a.w1 : a.w0, a.w_bytes - kQ6KBytes, slot + kRun + 15 * (Window::kPieces * 16));
+  };
+
+  // ---- activations
+  // piece q = wave + WAVES i of a step: token rows 8 q .. 8 q + 7; lane: row 8 q + (lane >> 3), position lane & 7, which
+  // holds chunk (lane & 7) ^ pc_swizzle(row)
+  constexpr int kPI = 4 * MI / WAVES;
+  uint32_t a_off[kPI], a_lanes[kPI];  // the lane's piece of either instruction; which instructions are for live rows
+  auto set_a = [&](const Item& it, int tb) __attribute__((always_inline)) {
+    const int pieces = (it.rows + 31) / 32 * 4;
+    int lane = (int)__lane_id();
+    asm volatile("" : "+v"(lane));  // (its arithmetic belongs here, once per item, and not in registers all along)
+#pragma unroll
+    for (int i = 0; i < kPI; ++i) {
+      const int row = 8 * (wave + WAVES * i) + (lane >> 3), live = min(row, it.rows - 1);
+      int arow = it.m0 + live;
+      if (ROUTED && NM == 2) arow = sId[tb * kTM + live] / a.top_k;
+      a_lanes[i] = __builtin_amdgcn_readfirstlane(WAVES * i < pieces ? ~0u : 0u);
+      a_off[i] = ((uint32_t)arow * (uint32_t)a.K + (uint32_t)((lane & 7) ^ pc_swizzle(row)) * 8u) * 2u;
+    }
+  };
+  const uint32_t lds_a = lds_address(sA) + (uint32_t)wave * 1024u;
+  int a_ks = 0;       // the activation stream's step
+  uint32_t a_to = 0;  // its place in the ring
+  auto request_a = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kPI; ++i)
+      lds_dma_16_lanes(a.a, a_off[i] + (uint32_t)a_ks * (kSK * 2u), lds_a + a_to + 1024u * WAVES * i, a_lanes[i], a_lanes[i]);
+  };
+  auto request_ids = [&](const Item& it, int tb) __attribute__((always_inline)) {
+    if (64 * wave < kTM)
+      lds_dma_4(a.sorted_token_ids, (uint32_t)(it.m0 + min(64 * wave + lane, it.rows - 1)) * 4u, lds_address(sId + tb * kTM + 64 * wave));
+  };
+  auto request_scales = [&]() __attribute__((always_inline)) {
+    if (64 * wave < kTM) lds_dma_4(a.topk_weights, (uint32_t)sId[64 * wave + lane] * 4u, lds_address(sScale + 64 * wave));
+  };
+  auto all_landed = [&]() __attribute__((always_inline)) {
+    order_fence();
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    order_fence();
+  };
+  // where the lane finds its row's eight elements of chunk kk of a step: piece 4 (kk >> 1) + 2 h + (kk & 1)
+  const uint32_t frag = (uint32_t)col * (kSK * 2) + (uint32_t)(((2 * h) ^ pc_swizzle(col)) * 16);
+  const uint32_t pick = w_scale_bytes(h);
+  // The two wavefronts of a SIMD do what is not matrix instructions at different times (before a chunk's and behind them,
+  // one chunk and the next): behind a barrier both would leave the matrix pipe idle together.
+  const bool early = wave < WAVES / 2;
+
+  Item cur = decode(first), nxt = cur;
+  int tb = 0;              // which of the two tables is this item's
+  WHalf<QUANT> raw[2];     // the raw weights of a superblock's halves, as far as they are at work
+  uint32_t ring = 0;       // this step's place in the ring
+  auto ring_after = [&](uint32_t r) __attribute__((always_inline)) { return r + kSlot == kRing * kSlot ? 0u : r + kSlot; };
+  int w_win = 1;           // the weight stream's next window
+  const int n_win = nsb * Window::kPerSb;
+
+  if (ROUTED && NM == 2) {
+    request_ids(cur, 0);
+    all_landed();
+  }
+  set_w(cur);
+  set_a(cur, 0);
+  request_w_all();
+#pragma unroll
+  for (a_ks = 0; a_ks < kRing; ++a_ks) {  // (a contraction has at least four steps)
+    a_to = (uint32_t)a_ks * kSlot;
+    request_a();
+  }
+  a_ks = kRing - 1;
+  all_landed();
+  if (QUANT == kQ6K && w_win == n_win) patch_w();
+  read_w(0, 0, raw[0]);
+  if constexpr (QUANT == kQ6K) read_w(1, 1, raw[1]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  // (the requests that the chunks before the first would have made: the next window's)
+  if (w_win == n_win) {
+    w_win = 0;
+    if (first + stride < hi) set_w(decode(first + stride));
+  }
+  w_at = (uint32_t)w_win * Window::kSpan;
+  ++w_win;
+  request_w_all();
+  wait_vm<0>();
+
+  for (int item = first;; item += stride) {
+    const bool has_next = item + stride < hi;
+    nxt = has_next ? decode(item + stride) : cur;
+    asm volatile("" ::"s"(nxt.e), "s"(nxt.m0), "s"(nxt.rows), "s"(nxt.nt));
+    if (ROUTED && nsteps < 8) {  // (no step late enough to find the tables by itself)
+      all_landed();                // (the table is free: everyone is past the epilogue that read it)
+      if constexpr (NM == 2) request_ids(nxt, tb ^ 1);
+      else request_ids(cur, 0);
+      all_landed();
+      if constexpr (kScaled) {
+        request_scales();
+        all_landed();
+      }
+    }
+
+    auto run = [&](auto nb_c) __attribute__((always_inline)) {
+      constexpr int NB = decltype(nb_c)::value;
+      float16v acc[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][v] = 0.0f;
+      half8 fa[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) fa[i] = *reinterpret_cast<const half8*>(sA + ring + frag + i * kBlockBytes);
+      WChunk wc;
+      w_parts_from<0>(raw[0], pick, wc);
+      half8 fb = w_halfs(wc);
+#pragma unroll 1
+      for (int sb = 0; sb < nsb; ++sb) {
+        WHalf<QUANT> next[2];
+        auto chunk = [&](auto c_c) __attribute__((always_inline)) {
+          constexpr int C = decltype(c_c)::value, C1 = (C + 1) & 15;
+          using Req = Requests<QUANT, kPI>;
+          // raw weights out of the slot: the next superblock's (Q6_K), the next half's (Q8_0)
+          if constexpr (QUANT == kQ6K) {
+            const int u = sb + 1 == nsb ? 0 : 2 * sb + 2;
+            if constexpr (C == 12 || C == 13) {
+              if (early == (C == 12)) {
+                wait_vm<Req::after_w(C)>();
+                if (w_win == n_win) patch_w();
+                read_w(u, 0, next[0]);
+              }
+            }
+            if constexpr (C == 14) read_w(u + 1, 1, next[1]);
+          } else if constexpr ((C & 7) == 5 || (C & 7) == 6) {
+            if (early == ((C & 7) == 5)) {
+              wait_vm<Req::after_w(C)>();
+              read_w(C < 8 ? 1 : 0, 0, C < 8 ? raw[1] : next[0]);
+            }
+          }
+          if constexpr ((C & 3) == 3) {
+            constexpr int S = C >> 2;
+            // everyone's pieces of the next step have landed, and everyone has read this step's for the last time, and the slot
+            order_fence();
+            wait_vm<Req::after_a(C - 4 * (kRing - 1), C)>();
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            order_fence();
+            if (ROUTED && nsteps >= 8) {
+              if (NM == 2 && S == 0 && sb == 0) request_ids(nxt, tb ^ 1);
+              if (kScaled && S == 0 && sb == 0) request_ids(cur, 0);
+              if (kScaled && S == 0 && sb == 1) request_scales();
+            }
+            if (++a_ks == nsteps) {
+              a_ks = 0;
+              set_a(nxt, tb ^ 1);
+            }
+            a_to = ring;
+            if constexpr (S == 3 || (QUANT == kQ8_0 && S == 1)) {
+              if (w_win == n_win) {
+                w_win = 0;
+                // (windows are requested two ahead: a contraction of one window is past the next item with that)
+                if (QUANT == kQ6K && n_win == 1) {
+                  if (item + 2 * stride < hi) set_w(decode(item + 2 * stride));
+                } else {
+                  set_w(nxt);
+                }
+              }
+              w_at = (uint32_t)w_win * Window::kSpan;
+              ++w_win;
+            }
+            ring = ring_after(ring);
+          }
+          auto requests = [&]() __attribute__((always_inline)) {
+            if constexpr (Req::a_at(C) != 0) request_a();
+            if constexpr (Req::w_at(C) != 0) request_w(std::integral_constant<int, QUANT == kQ6K ? (C + 1) & 15 : (C + 1) & 7>{});
+          };
+          constexpr bool kRequests = Req::a_at(C) != 0 || Req::w_at(C) != 0;
+          if (kRequests && early) requests();
+          order_fence();
+          const WHalf<QUANT>& r1 = C1 == 0 ? next[0] : raw[C1 >> 3];
+          const uint8_t* pa = sA + ((frag ^ (64u * ((C1 >> 1) & 1) + 16u * (C1 & 1))) + ring);
+#pragma unroll
+          for (int i = 0; i < NB; ++i) {
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb, acc[i], 0, 0, 0);
+            fa[i] = *reinterpret_cast<const half8*>(pa + i * kBlockBytes);
+            // the next chunk's weights between the matrix instructions: the two run beside each other (up to four vector
+            // instructions cost a matrix instruction nothing)
+            if (0 * NB / kWParts == i) w_part<C1 & 7, 0>(r1, pick, wc);
+            if (1 * NB / kWParts == i) w_part<C1 & 7, 1>(r1, pick, wc);
+            if (2 * NB / kWParts == i) w_part<C1 & 7, 2>(r1, pick, wc);
+            if (3 * NB / kWParts == i) w_part<C1 & 7, 3>(r1, pick, wc);
+            if (4 * NB / kWParts == i) w_part<C1 & 7, 4>(r1, pick, wc);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (kRequests && !early) requests();
+          fb = w_halfs(wc);
+          if constexpr (C1 == 0) {
+            raw[0] = next[0];
+            if constexpr (QUANT == kQ6K) raw[1] = next[1];
+          }
+        };
+        chunk(std::integral_constant<int, 0>{});
+        chunk(std::integral_constant<int, 1>{});
+        chunk(std::integral_constant<int, 2>{});
+        chunk(std::integral_constant<int, 3>{});
+        chunk(std::integral_constant<int, 4>{});
+        chunk(std::integral_constant<int, 5>{});
+        chunk(std::integral_constant<int, 6>{});
+        chunk(std::integral_constant<int, 7>{});
+        chunk(std::integral_constant<int, 8>{});
+        chunk(std::integral_constant<int, 9>{});
+        chunk(std::integral_constant<int, 10>{});
+        chunk(std::integral_constant<int, 11>{});
+        chunk(std::integral_constant<int, 12>{});
+        chunk(std::integral_constant<int, 13>{});
+        chunk(std::integral_constant<int, 14>{});
+        chunk(std::integral_constant<int, 15>{});
+      }
+
+      // epilogue.  acc[i][v]: tile row 32 i + (v / 4) * 8 + h * 4 + v % 4, column lane % 32 of the wavefront
+      int lane = (int)__lane_id();
+      asm volatile("" : "+v"(lane));
+      const int h = lane >> 5, col = lane & 31;
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int left = cur.rows - 32 * i;  // live rows from this block on
+        if constexpr (NM == 2) {
+          // lanes 0-15 hold a gate column's element, lanes 16-31 the matching up column's: an exchange of two registers'
+          // halves leaves gate and up of one row in lanes 0-15, of the next row in lanes 16-31
+          const int odd = (lane >> 4) & 1, c = cur.nt * (kTR / 2) + 16 * wave + (lane & 15);
+          _Float16* out = static_cast<_Float16*>(a.out) + (size_t)(cur.m0 + 32 * i) * a.n_rows + c;
+#pragma unroll
+          for (int v = 0; v < 16; v += 2) {
+            const float even_row = acc[i][v], odd_row = acc[i][v + 1];
+            const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, even_row), __builtin_bit_cast(uint32_t, odd_row), false, false);
+            const uint32_t gb = sw[0], ub = sw[1];
+            const float g = __builtin_bit_cast(float, gb) * kWScaleInv, up = __builtin_bit_cast(float, ub) * kWScaleInv;
+            const int r = (v >> 2) * 8 + h * 4 + (v & 3) + odd;
+            if (r < left) out[(size_t)r * a.n_rows] = (_Float16)(silu_fast(g) * up);
+          }
+        } else {
+          const int c = cur.nt * kTR + 32 * wave + col;
+          float* out = static_cast<float*>(a.out) + c;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            int orow[4];
+            float s[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const int r = 32 * i + 8 * q + 4 * h + w;
+              orow[w] = ROUTED ? sId[r] : cur.m0 + r;
+              s[w] = ROUTED ? sScale[r] : 1.0f;
+            }
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+              if (8 * q + 4 * h + w < left) out[(size_t)orow[w] * a.n_rows] = s[w] * (acc[i][4 * q + w] * kWScaleInv);
+          }
+        }
+      }
+    };
+    const int nb = (cur.rows + 31) / 32;
+    if constexpr (MI > 2) {
+      switch (nb) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        case 4: run(std::integral_constant<int, 4>{}); break;
+        case 5: run(std::integral_constant<int, 5>{}); break;
+        default: run(std::integral_constant<int, 6>{}); break;
+      }
+    } else {
+      if (nb == 1) run(std::integral_constant<int, 1>{});
+      else run(std::integral_constant<int, 2>{});
+    }
+    if (!has_next) break;
+    cur = nxt;
+    tb ^= 1;
+  }
+  // (nothing may still be on its way into this workgroup's LDS when it ends)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // fp32 -> fp16 activations for live rows; rows past `valid` are left alone.
 __global__ void __launch_bounds__(256) k_to_f16_rows(const float* __restrict__ x, const int* __restrict__ valid_tokens,
                                                       int width, _Float16* __restrict__ out) {
@@ -1015,58 +1127,39 @@ __global__ void __launch_bounds__(256) k_to_f16_rows(const float* __restrict__ x
   }
 }
 
-// Token-tile list: one entry per `bm`-slot chunk of each active expert's run.  One workgroup.  With bm_b > 0 a second
-// list of that tile height goes to tile_list_b in the same launch (the routed gate/up launch's, where it differs).
+// Token-tile list (layout: MfmaArgs), the tiles of each active expert's run at most `bm` rows tall.  One workgroup.
 __global__ void __launch_bounds__(256) k_build_tiles(const int* __restrict__ expert_counts, int num_experts, int block_size,
-                                                      int capacity, int bm, int* __restrict__ tile_list, int bm_b,
-                                                      int* __restrict__ tile_list_b) {
+                                                      int capacity, int bm, int* __restrict__ tile_list) {
   __shared__ int s_base[513], s_tiles[513];
   // exclusive prefixes of the padded run lengths and of the tile counts (num_experts <= 512): every thread
   // takes two experts, the pair sums are scanned across the workgroup in eight doubling steps
   __shared__ int s_scan[2][2][256];
   const int t = threadIdx.x;
-  for (int pass = 0; pass < (bm_b > 0 ? 2 : 1); ++pass) {
-    const int h = pass ? bm_b : bm;
-    int* list = pass ? tile_list_b : tile_list;
-    int pad[2], til[2];
+  int pad[2], til[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int e = 2 * t + j;
-      const int c = e < num_experts ? expert_counts[e] : 0;
-      pad[j] = (c + block_size - 1) / block_size * block_size;
-      til[j] = (c + h - 1) / h;
-    }
-    __syncthreads();  // (the previous pass has read its tables)
-    s_scan[0][0][t] = pad[0] + pad[1];
-    s_scan[0][1][t] = til[0] + til[1];
-    __syncthreads();
-    int cur = 0;
-    for (int d = 1; d < 256; d <<= 1) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][t] = s_scan[cur][a][t] + (t >= d ? s_scan[cur][a][t - d] : 0);
-      cur ^= 1;
-      __syncthreads();
-    }
-    {
-      const int base = s_scan[cur][0][t] - (pad[0] + pad[1]), tiles = s_scan[cur][1][t] - (til[0] + til[1]);
-      if (2 * t < num_experts) s_base[2 * t] = base, s_tiles[2 * t] = tiles;
-      if (2 * t + 1 < num_experts) s_base[2 * t + 1] = base + pad[0], s_tiles[2 * t + 1] = tiles + til[0];
-      if (t == 255) list[0] = min(s_scan[cur][1][t], capacity);
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < num_experts; e += 256) {
-      const int c = expert_counts[e];
-      const int nt = (c + h - 1) / h;
-      for (int i = 0; i < nt; ++i) {
-        const int idx = s_tiles[e] + i;
-        if (idx >= capacity) break;
-        list[4 + 4 * idx + 0] = e;
-        list[4 + 4 * idx + 1] = s_base[e] + i * h;
-        list[4 + 4 * idx + 2] = min(h, c - i * h);
-        list[4 + 4 * idx + 3] = 0;
-      }
-    }
+  for (int j = 0; j < 2; ++j) {
+    const int e = 2 * t + j;
+    const int c = e < num_experts ? expert_counts[e] : 0;
+    pad[j] = (c + block_size - 1) / block_size * block_size;
+    til[j] = (c + bm - 1) / bm;
   }
+  s_scan[0][0][t] = pad[0] + pad[1];
+  s_scan[0][1][t] = til[0] + til[1];
+  __syncthreads();
+  int cur = 0;
+  for (int d = 1; d < 256; d <<= 1) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][t] = s_scan[cur][a][t] + (t >= d ? s_scan[cur][a][t - d] : 0);
+    cur ^= 1;
+    __syncthreads();
+  }
+  const int base = s_scan[cur][0][t] - (pad[0] + pad[1]), tiles = s_scan[cur][1][t] - (til[0] + til[1]);
+  if (2 * t < num_experts) s_base[2 * t] = base, s_tiles[2 * t] = tiles;
+  if (2 * t + 1 < num_experts) s_base[2 * t + 1] = base + pad[0], s_tiles[2 * t + 1] = tiles + til[0];
+  if (t == 255) tile_list[0] = min(s_scan[cur][1][t], capacity);
+  __syncthreads();
+  for (int e = threadIdx.x; e < num_experts; e += 256)
+    write_tile_entries(e, expert_counts[e], s_base[e], s_tiles[e], bm, capacity, tile_list);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1082,7 +1175,7 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
   if (routed && g.num_experts > 512) return false;  // k_build_tiles scans two experts per thread of one 256-thread workgroup
   auto ok = [](int q) { return q == XABE_QUANT_Q6K || q == XABE_QUANT_Q8_0; };
   if (!ok(gate_q) || !ok(down_q) || gate_q != up_q) return false;
-  // contraction in steps of 128 (whole Q6_K superblocks: 256); gate/up tiles 64 columns, down tiles 128
+  // whole superblocks of the contraction; gate/up tiles of 128 columns, down tiles of 256
   if (g.hidden % 256 != 0 || g.intermediate % 256 != 0) return false;
   // an activation piece is addressed by a 32-bit byte offset from its tensor's base (fp16 rows of either width, as
   // many as the sorted table has slots)
@@ -1091,15 +1184,14 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
   return true;
 }
 
-// Token-tile height for a geometry: the narrow tile while an expert's share of a full pass usually fits in it
-// (an average of 48 selections per expert; at 64 every second expert overflows into a second tile, measured
-// 702 against 695 us at 2048 tokens).
-// `tokens`: pass_tokens() below.
+// Token rows of a routed tile: narrow while an expert's share of the pass averages at most 48 rows, so that most experts
+// are one tile either way (1500 tokens of the routed model, 47 a share: 365 us against 388 wide; 2200, 69: 544 against
+// 454).
 static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
-  return tokens * g.experts_per_token <= 48 * g.num_experts ? 64 : kBM;
+  return tokens * g.experts_per_token <= 48 * g.num_experts ? kNarrowRows : kWideRows;
 }
 // The specialised form (k_mfma_pc) serves both routed launches for contractions of whole superblocks and at least
-// eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_expert everywhere; it is the faster at every width
+// eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_rows everywhere; it is the faster at every width
 // measured, see k_mfma_pc).
 static bool pc_shape_ok(const xabe_moe_geometry& g) {
   return g.hidden % 256 == 0 && g.intermediate % 256 == 0 && g.hidden >= 512 && g.intermediate >= 512;
@@ -1112,45 +1204,44 @@ static bool pc_form(const xabe_moe_kernels* k, size_t) { return k->mfma_form == 
 static size_t pass_tokens(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
   return b->valid_published > 0 ? std::min<size_t>((size_t)b->valid_published, k->g.max_tokens) : k->g.max_tokens;
 }
-// Token-tile height of the routed gate/up launch: the tall tile once an expert's share of a full pass fills most of it
-// (an average of 192 selections per expert: 6144 tokens of the model's shape).  Same-box, per block: 8192 tokens 1323
-// -> 1263 us (the launch itself 503 -> ~415), 6144 tokens 1081 -> 1043; at 4096 tokens (128 per expert) the tall tile
-// loses (778 against 767).  The down launch keeps the short tiles at every width: its contraction is four steps, its
-// items are mostly epilogue, and with tall tiles the block measured 1279 us against 1263.
-static int routed_up_tile_rows(const xabe_moe_kernels* k, size_t tokens) {
-  const xabe_moe_geometry& g = k->g;
-  if (pc_form(k, tokens)) return kPM;
-  if (tokens * g.experts_per_token >= 192 * g.num_experts) return 384;
-  return routed_tile_rows(g, tokens);
+// Whether an unrouted pass takes the wide form: when whole tiles of it give every CU one (dense sibling: 300 tokens 432
+// us against 392 narrow, 450 tokens 471 against 518, 2048 1200 against 1750; the shared expert of the routed model stays
+// narrow up to 8192 tokens, where it leaves room beside it for the launches it runs along with: 1965 against 1980 us for
+// two blocks).
+static bool unrouted_wide(const xabe_moe_kernels* k, size_t tokens) {
+  return tokens / kWideRows * (k->g.intermediate / 128) >= (size_t)k->num_cus;
 }
-// The shared expert's launches are short of workgroups below a few thousand tokens: the narrow tile while all
-// of its items still start at once (two workgroups per compute unit), so that twice as many units share the work.
-static int shared_tile_rows(const xabe_moe_kernels* k, size_t tokens, size_t row_tiles) {
-  return (tokens + 63) / 64 * row_tiles <= (size_t)k->num_cus * 2 ? 64 : kBM;
+// Token rows of a wide unrouted tile: the height whose items, dealt in rounds to the CUs, end first, an item's time being
+// that of its 32-row blocks and about 3.6 blocks' more (dense sibling, 2048 tokens: a superblock of the contraction
+// takes 2.3 us and 0.64 us per block; down 385 us at 192 rows, one round, and 616 at 160, two).
+static int unrouted_tile_rows(const xabe_moe_kernels* k, size_t tokens, size_t row_tiles) {
+  int best = 32;
+  double best_cost = 1e30;
+  for (int h = 32; h <= kWideRows; h += 32) {
+    const size_t items = (tokens + h - 1) / h * row_tiles, rounds = (items + k->num_cus - 1) / k->num_cus;
+    const double cost = (double)rounds * (h / 32 + 3.6);
+    if (cost < best_cost) best_cost = cost, best = h;
+  }
+  return best;
 }
 
-bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* bm_up, int* capacity) {
-  if (!b->tile_list || b->n_tile_list < 16 || !k->tensor_cores || k->exact_regime) return false;
+bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* capacity) {
+  if (!b->tile_list || b->n_tile_list < 8 || !k->tensor_cores || k->exact_regime) return false;
   const size_t tokens = pass_tokens(k, b);
   *bm = routed_tile_rows(k->g, tokens);
-  if (pc_form(k, tokens)) *bm = kPM;  // (both specialised launches: 128-row tiles, one list)
-  *bm_up = routed_up_tile_rows(k, tokens);
-  *capacity = (int)((b->n_tile_list / 2 - 4) / 4);
+  if (pc_form(k, tokens)) *bm = kPM;  // (the specialised launches: 128-row tiles)
+  *capacity = (int)((b->n_tile_list - 4) / 4);
   return true;
 }
 
-// LDS a workgroup of the kernel asks for (dynamic: above the static limit).  The limit is raised per function,
-// once, when a kernels handle is created (mfma_configure): nothing on the launch path but the launch.
-template <int TBM>
-constexpr size_t mfma_lds_bytes() {
-  return (size_t)(TBM * kLdA + kBR * kLd) * sizeof(_Float16) + 2 * 3 * TBM * sizeof(int);
-}
-template <int NM, bool ROUTED, int TBM>
+// LDS of the kernels is dynamic, above the static limit, which is raised per function once, when a kernels handle is
+// created (mfma_configure): nothing on the launch path but the launch.
+template <int NM, bool ROUTED, int MI, int WAVES>
 static int configure_one() {
-  const void* fns[2] = {reinterpret_cast<const void*>(k_mfma_expert<kQ6K, NM, ROUTED, TBM>),
-                        reinterpret_cast<const void*>(k_mfma_expert<kQ8_0, NM, ROUTED, TBM>)};
-  for (const void* f : fns)
-    XABE_HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_lds_bytes<TBM>()));
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mfma_rows<kQ6K, NM, ROUTED, MI, WAVES>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_rows_lds<kQ6K, MI, WAVES>()));
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mfma_rows<kQ8_0, NM, ROUTED, MI, WAVES>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_rows_lds<kQ8_0, MI, WAVES>()));
   return XABE_OK;
 }
 template <int NM>
@@ -1173,15 +1264,14 @@ static int launch_pc(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, si
 static int mfma_set_limits() {
   XABE_TRY((configure_pc<2>()));
   XABE_TRY((configure_pc<1>()));
-  XABE_TRY((configure_one<1, false, 64>()));
-  XABE_TRY((configure_one<1, false, 128>()));
-  XABE_TRY((configure_one<1, true, 64>()));
-  XABE_TRY((configure_one<1, true, 128>()));
-  XABE_TRY((configure_one<2, false, 64>()));
-  XABE_TRY((configure_one<2, false, 128>()));
-  XABE_TRY((configure_one<2, true, 64>()));
-  XABE_TRY((configure_one<2, true, 128>()));
-  XABE_TRY((configure_one<2, true, 384>()));
+  XABE_TRY((configure_one<1, false, 6, 8>()));
+  XABE_TRY((configure_one<2, false, 6, 8>()));
+  XABE_TRY((configure_one<1, true, 6, 8>()));
+  XABE_TRY((configure_one<2, true, 6, 8>()));
+  XABE_TRY((configure_one<1, false, 2, 4>()));
+  XABE_TRY((configure_one<2, false, 2, 4>()));
+  XABE_TRY((configure_one<1, true, 2, 4>()));
+  XABE_TRY((configure_one<2, true, 2, 4>()));
   return XABE_OK;
 }
 
@@ -1193,16 +1283,14 @@ int mfma_configure() {
   return once.run(dev, mfma_set_limits);
 }
 
-template <int NM, bool ROUTED, int TBM>
-static int launch_mfma(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, size_t max_items, hipStream_t s) {
-  // workgroups resident per CU: the narrow tile's registers (about 150) and LDS (49.5 KB) leave room for a third
-  // (the tall tile: eight wavefronts and 137 KB of LDS, one workgroup per CU)
-  const size_t per_cu = TBM == 64 ? 3 : TBM == 128 ? 2 : 1;
-  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(max_items, (size_t)k->num_cus * per_cu));
-  constexpr size_t smem = mfma_lds_bytes<TBM>();
-  constexpr unsigned threads = TBM == 384 ? 512 : 256;
-  if (quant == XABE_QUANT_Q6K) hipLaunchKernelGGL((k_mfma_expert<kQ6K, NM, ROUTED, TBM>), dim3(grid), dim3(threads), smem, s, a);
-  else hipLaunchKernelGGL((k_mfma_expert<kQ8_0, NM, ROUTED, TBM>), dim3(grid), dim3(threads), smem, s, a);
+template <int NM, bool ROUTED, int MI, int WAVES>
+static int launch_rows(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, size_t max_mtiles, hipStream_t s) {
+  const size_t max_items = max_mtiles * (size_t)(a.n_rows / (WAVES * kWRows / NM));
+  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(max_items, (size_t)k->num_cus * kWgsPerCu<MI, WAVES>));
+  if (quant == XABE_QUANT_Q6K)
+    hipLaunchKernelGGL((k_mfma_rows<kQ6K, NM, ROUTED, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ6K, MI, WAVES>()), s, a);
+  else
+    hipLaunchKernelGGL((k_mfma_rows<kQ8_0, NM, ROUTED, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ8_0, MI, WAVES>()), s, a);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
@@ -1222,22 +1310,18 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
                                  xabe_quant_tensor up, xabe_quant_tensor down, const float* x) {
   const xabe_moe_geometry& g = k->g;
   if (!b->x_h_ready) XABE_TRY(to_f16(k, s, b, x));
-  // (the allocation holds two lists of the same capacity: the down launch's, and the gate/up launch's where its tile
-  // height differs)
-  const size_t list_ints = b->n_tile_list / 2;
-  int bm = 0, bm_up = 0, cap = 0;
-  if (!mfma_tile_plan(k, b, &bm, &bm_up, &cap))
-    return set_error(XABE_ERR_INVALID_ARGUMENT, "grouped_forward: these buffers hold no token-tile lists");
-  int* list_up = bm_up == bm ? b->tile_list : b->tile_list + list_ints;
-  // (the dispatch build has usually left the lists, cut for these heights)
+  int bm = 0, cap = 0;
+  if (!mfma_tile_plan(k, b, &bm, &cap))
+    return set_error(XABE_ERR_INVALID_ARGUMENT, "grouped_forward: these buffers hold no token-tile list");
+  // the dispatch build has usually left the list, cut for this height:
   // trusted only when nothing can have rewritten them since: inside the capture that holds the build, or eagerly
   // after an eager build on buffers no graph has ever recorded a build on
   const unsigned long long capture = stream_capture_id(s);
-  const bool trusted = b->tiles_bm == bm && b->tiles_bm_up == bm_up && capture != kCaptureUnknown &&
+  const bool trusted = b->tiles_bm == bm && capture != kCaptureUnknown &&
                        b->tiles_capture == capture && (capture != 0 || !b->tiles_graph_owned);
   if (!trusted) {
     hipLaunchKernelGGL(k_build_tiles, dim3(1), dim3(256), 0, s, b->expert_counts, (int)g.num_experts, (int)g.block_size, cap,
-                       bm, b->tile_list, bm_up != bm ? bm_up : 0, list_up);
+                       bm, b->tile_list);
     XABE_HIP_TRY(hipGetLastError());
   }
   MfmaArgs a;
@@ -1245,34 +1329,34 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
   a.valid_tokens = b->valid_tokens;
   a.sorted_token_ids = b->sorted_token_ids;
   a.topk_weights = b->topk_weights;
-  a.tile_list = list_up;
+  a.tile_list = b->tile_list;
   a.top_k = (int)g.experts_per_token;
   const size_t max_mtiles = (size_t)cap;
   // gate/up + SwiGLU -> inter_h[slot][I]
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
   a.w1 = static_cast<const uint8_t*>(up.bytes);
   a.expert_bytes = g.intermediate * stack_row_bytes(gate.quant, g.hidden);
+  a.w_bytes = gate.len;
   a.a = reinterpret_cast<const _Float16*>(b->x_h);
   a.out = b->inter_h;
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
   const bool pc = pc_form(k, pass_tokens(k, b));
-  if (pc && bm_up == kPM) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
-  else if (bm_up == 64) XABE_TRY((launch_mfma<2, true, 64>(k, gate.quant, a, max_mtiles * (g.intermediate / 64), s)));
-  else if (bm_up == 384) XABE_TRY((launch_mfma<2, true, 384>(k, gate.quant, a, max_mtiles * (g.intermediate / 64), s)));
-  else XABE_TRY((launch_mfma<2, true, 128>(k, gate.quant, a, max_mtiles * (g.intermediate / 64), s)));
+  if (pc) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
+  else if (bm == kNarrowRows) XABE_TRY((launch_rows<2, true, 2, 4>(k, gate.quant, a, max_mtiles, s)));
+  else XABE_TRY((launch_rows<2, true, 6, 8>(k, gate.quant, a, max_mtiles, s)));
   // down -> partial[flat][H], scaled by the routing weight
-  a.tile_list = b->tile_list;
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.expert_bytes = g.hidden * stack_row_bytes(down.quant, g.intermediate);
+  a.w_bytes = down.len;
   a.a = reinterpret_cast<const _Float16*>(b->inter_h);
   a.out = b->partial;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  if (pc && bm == kPM) XABE_TRY((launch_pc<1>(k, down.quant, a, max_mtiles * (g.hidden / kPR), s)));
-  else if (bm == 64) XABE_TRY((launch_mfma<1, true, 64>(k, down.quant, a, max_mtiles * (g.hidden / 128), s)));
-  else XABE_TRY((launch_mfma<1, true, 128>(k, down.quant, a, max_mtiles * (g.hidden / 128), s)));
+  if (pc) XABE_TRY((launch_pc<1>(k, down.quant, a, max_mtiles * (g.hidden / kPR), s)));
+  else if (bm == kNarrowRows) XABE_TRY((launch_rows<1, true, 2, 4>(k, down.quant, a, max_mtiles, s)));
+  else XABE_TRY((launch_rows<1, true, 6, 8>(k, down.quant, a, max_mtiles, s)));
   return XABE_OK;
 }
 
@@ -1290,27 +1374,24 @@ int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   a.out = b->shared_inter_h;
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
-  {
-    const size_t row_tiles = g.intermediate / 64;
-    const int bm = shared_tile_rows(k, pass_tokens(k, b), row_tiles);
-    const size_t items = (g.max_tokens + bm - 1) / bm * row_tiles;
-    if (bm == 64) XABE_TRY((launch_mfma<2, false, 64>(k, gate.quant, a, items, s)));
-    else XABE_TRY((launch_mfma<2, false, 128>(k, gate.quant, a, items, s)));
-  }
+  a.w_bytes = gate.len;
+  const size_t tokens = pass_tokens(k, b);
+  const bool wide = unrouted_wide(k, tokens);
+  a.tile_rows = wide ? unrouted_tile_rows(k, tokens, g.intermediate / 128) : kNarrowRows;
+  size_t tiles = (g.max_tokens + a.tile_rows - 1) / a.tile_rows;
+  if (wide) XABE_TRY((launch_rows<2, false, 6, 8>(k, gate.quant, a, tiles, s)));
+  else XABE_TRY((launch_rows<2, false, 2, 4>(k, gate.quant, a, tiles, s)));
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
+  a.w_bytes = down.len;
   a.a = reinterpret_cast<const _Float16*>(b->shared_inter_h);
   a.out = out;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  {
-    const size_t row_tiles = g.hidden / 128;
-    const int bm = shared_tile_rows(k, pass_tokens(k, b), row_tiles);
-    const size_t items = (g.max_tokens + bm - 1) / bm * row_tiles;
-    if (bm == 64) XABE_TRY((launch_mfma<1, false, 64>(k, down.quant, a, items, s)));
-    else XABE_TRY((launch_mfma<1, false, 128>(k, down.quant, a, items, s)));
-  }
-  return XABE_OK;
+  a.tile_rows = wide ? unrouted_tile_rows(k, tokens, g.hidden / 256) : kNarrowRows;
+  tiles = (g.max_tokens + a.tile_rows - 1) / a.tile_rows;
+  if (wide) return launch_rows<1, false, 6, 8>(k, down.quant, a, tiles, s);
+  return launch_rows<1, false, 2, 4>(k, down.quant, a, tiles, s);
 }
 
 }  // namespace xabe

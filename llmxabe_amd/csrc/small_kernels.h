@@ -5,6 +5,7 @@
 #include "device_common.h"
 #include "digit_rows.h"
 #include "route_device.h"
+#include "tile_list.h"
 
 namespace xabe {
 
@@ -315,29 +316,16 @@ __global__ void __launch_bounds__(256) k_align_scatter(const int* __restrict__ t
 }
 
 // ---------------------------------------------------------------------------------
-// Token-tile lists of the matrix-core grouped GEMM, written by the dispatch kernels below that hold every expert's
+// Token-tile list of the matrix-core grouped GEMM, written by the dispatch kernels below that hold every expert's
 // count and first slot in one workgroup (otherwise by k_build_tiles in mfma.hip, which documents the layout): one
-// entry {expert, first slot, live rows, 0} per `bm`-slot piece of each active expert's run, [0] = the entry count.
-// With bm_b > 0 a second list of that tile height goes to list_b.  bm = 0: no lists asked for.
+// entry {expert, first slot, live rows, 0} per tile of at most `bm` rows of each active expert's run, [0] = the entry
+// count.  bm = 0: no list asked for.
 // ---------------------------------------------------------------------------------
 struct TileListArgs {
-  int capacity;  // entries a list holds
-  int bm, bm_b;
+  int capacity;  // entries the list holds
+  int bm;
   int* list;
-  int* list_b;
 };
-// entries of expert e (count selections from slot `base`), the first of them entry `first` of the list
-__device__ __forceinline__ void write_tile_entries(int e, int count, int base, int first, int h, int capacity, int* list) {
-  const int nt = (count + h - 1) / h;
-  for (int i = 0; i < nt; ++i) {
-    const int idx = first + i;
-    if (idx >= capacity) break;
-    list[4 + 4 * idx + 0] = e;
-    list[4 + 4 * idx + 1] = base + i * h;
-    list[4 + 4 * idx + 2] = min(h, count - i * h);
-    list[4 + 4 * idx + 3] = 0;
-  }
-}
 
 // ---------------------------------------------------------------------------------
 // The same tables from ONE launch of one workgroup, for passes of at most 8192 selections (1024 tokens of top-8):
@@ -358,7 +346,7 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
                                                        TileListArgs tl) {
   constexpr int kMaxE = 512, kRounds = kAlignFusedMaxSelections / (kAlignFusedWaves * 64);
   __shared__ int cnt[kAlignFusedWaves][kMaxE];  // per range and expert: count, then next slot
-  __shared__ int s_scan[2][3][kMaxE];           // scanned together: padded counts, tiles of either list
+  __shared__ int s_scan[2][2][kMaxE];           // scanned together: padded counts, tiles
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int numel = min(*valid_tokens * top_k, kAlignFusedMaxSelections);
   // whole-capacity fill first: the barriers below order it before the entries written over it
@@ -380,7 +368,7 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
     if (id[r] >= 0) atomicAdd(&cnt[wave][id[r]], 1);
   }
   __syncthreads();
-  int count = 0, padded = 0, tiles_a = 0, tiles_b = 0;
+  int count = 0, padded = 0, tiles = 0;
   if (tid < kMaxE) {
     if (tid < num_experts) {
 #pragma unroll
@@ -391,18 +379,16 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
       }
       padded = (count + block_size - 1) / block_size * block_size;
     }
-    tiles_a = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
-    tiles_b = tl.bm_b > 0 ? (count + tl.bm_b - 1) / tl.bm_b : 0;
+    tiles = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
     s_scan[0][0][tid] = padded;
-    s_scan[0][1][tid] = tiles_a;
-    s_scan[0][2][tid] = tiles_b;
+    s_scan[0][1][tid] = tiles;
   }
   __syncthreads();
   int cur = 0;
   for (int d = 1; d < kMaxE; d <<= 1) {
     if (tid < kMaxE) {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) s_scan[cur ^ 1][a][tid] = s_scan[cur][a][tid] + (tid >= d ? s_scan[cur][a][tid - d] : 0);
+      for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][tid] = s_scan[cur][a][tid] + (tid >= d ? s_scan[cur][a][tid - d] : 0);
     }
     cur ^= 1;
     __syncthreads();
@@ -412,11 +398,9 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
     if (tid == kMaxE - 1) {
       *num_tokens_post_pad = s_scan[cur][0][tid];
       if (tl.bm > 0) tl.list[0] = min(s_scan[cur][1][tid], tl.capacity);
-      if (tl.bm_b > 0) tl.list_b[0] = min(s_scan[cur][2][tid], tl.capacity);
     }
     if (tid < num_experts) {
-      if (tl.bm > 0) write_tile_entries(tid, count, base, s_scan[cur][1][tid] - tiles_a, tl.bm, tl.capacity, tl.list);
-      if (tl.bm_b > 0) write_tile_entries(tid, count, base, s_scan[cur][2][tid] - tiles_b, tl.bm_b, tl.capacity, tl.list_b);
+      if (tl.bm > 0) write_tile_entries(tid, count, base, s_scan[cur][1][tid] - tiles, tl.bm, tl.capacity, tl.list);
       expert_counts[tid] = count;
 #pragma unroll
       for (int w = 0; w < kAlignFusedWaves; ++w) cnt[w][tid] += base;
@@ -503,7 +487,7 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
                                                         int* __restrict__ expert_ids, int* __restrict__ bucket_live,
                                                         int* __restrict__ num_tokens_post_pad, TileListArgs tl) {
   static_assert(kAlignMaxExperts == 512, "one thread per expert slot of the scan");
-  __shared__ int s_scan[2][3][kAlignMaxExperts];  // scanned together: padded counts, tiles of either list
+  __shared__ int s_scan[2][2][kAlignMaxExperts];  // scanned together: padded counts, tiles
   const int e = threadIdx.x;
   const int numel = *valid_tokens * top_k;
   const int n_chunks = min(n_chunks_max, (numel + kAlignChunk - 1) / kAlignChunk);
@@ -517,17 +501,15 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
   if (live)
     for (int c = kAlignCachedChunks; c < n_chunks; ++c) count += chunk_hist[(size_t)c * num_experts + e];
   const int padded = live ? (count + block_size - 1) / block_size * block_size : 0;
-  const int tiles_a = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
-  const int tiles_b = tl.bm_b > 0 ? (count + tl.bm_b - 1) / tl.bm_b : 0;
+  const int tiles = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
   // inclusive scan of the padded counts and the tile counts (nine doubling steps), then exclusive
   s_scan[0][0][e] = padded;
-  s_scan[0][1][e] = tiles_a;
-  s_scan[0][2][e] = tiles_b;
+  s_scan[0][1][e] = tiles;
   __syncthreads();
   int cur = 0;
   for (int d = 1; d < kAlignMaxExperts; d <<= 1) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) s_scan[cur ^ 1][a][e] = s_scan[cur][a][e] + (e >= d ? s_scan[cur][a][e - d] : 0);
+    for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][e] = s_scan[cur][a][e] + (e >= d ? s_scan[cur][a][e - d] : 0);
     cur ^= 1;
     __syncthreads();
   }
@@ -535,11 +517,9 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
   if (e == kAlignMaxExperts - 1) {
     *num_tokens_post_pad = s_scan[cur][0][e];
     if (tl.bm > 0) tl.list[0] = min(s_scan[cur][1][e], tl.capacity);
-    if (tl.bm_b > 0) tl.list_b[0] = min(s_scan[cur][2][e], tl.capacity);
   }
   if (!live) return;
-  if (tl.bm > 0) write_tile_entries(e, count, base, s_scan[cur][1][e] - tiles_a, tl.bm, tl.capacity, tl.list);
-  if (tl.bm_b > 0) write_tile_entries(e, count, base, s_scan[cur][2][e] - tiles_b, tl.bm_b, tl.capacity, tl.list_b);
+  if (tl.bm > 0) write_tile_entries(e, count, base, s_scan[cur][1][e] - tiles, tl.bm, tl.capacity, tl.list);
   expert_counts[e] = count;
   int run = base;
 #pragma unroll
