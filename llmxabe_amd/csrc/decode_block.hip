@@ -14,6 +14,8 @@
 //                        wavefront is cheaper than one more launch or a device-wide handshake), then the wavefronts
 //                        stream the selected expert's gate/up rows through the digit contraction and write the
 //                        intermediate row as digits.
+//      (From eight tokens on the routing is a launch of its own between A and B, and the shared gate/up runs beside it
+//      instead of in A: k_decode_router, k_decode_route.)
 //   C  k_decode_down:    one token x share of its row tiles per workgroup, a wavefront per selection: the routed down
 //                        projections (and, at few tokens, the shared one), summed in k order, gated, combined with
 //                        the residual.  No partial buffer, no reduction pass.
@@ -44,7 +46,8 @@ constexpr size_t kDecodeBlockMaxTokens = kMfmaMinTokens - 1;  // every width bel
 // launch reads the selections: inside the second launch every workgroup of a token repeats the token's routing, and
 // past a few tokens its grid runs in several rounds per CU, each paying for it again.  Measured before the routed
 // contractions took their present form, us per block, routing inside / routing launch: 4 tokens 38.6 / 40.5, 6: 49.8 / 51.2, 8: 61.5 / 61.1, 12: 83.3 / 79.4, 16: 101.7 / 94.9,
-// 32: 181.3 / 161.5.
+// 32: 181.3 / 161.5.  With the shared gate/up beside the routing launch, 4: 47.8 / 54.3, 6: 64.1 / 67.0, 7: 71.0 / 71.6,
+// 8: 79.4 / 79.3 (one layer by itself, cold).
 constexpr int kPreRouteMinTokens = 8;
 // From this width on the second and third launches deal their workgroups so that the ones that read the same row
 // tile (of whichever experts their pairs or tokens selected) run next to each other on one XCD: workgroup ids go
@@ -59,7 +62,7 @@ constexpr int kMaxTopK = 8;       // contributions held in registers by k_decode
 // Steps per wavefront of the first launch: a wavefront reads 24 KB of activation rows and norm weights for the 2-4 KB
 // of weights of one step, so more steps against the same registers cut what the launch pulls out of L2, at the
 // price of fewer workgroups.  Measured per width (launch A, us, depth 1 / 2 / 4): one token 5.2 / 5.3 / 6.6, three
-// 7.7 / 6.5 / 8.4, eight 14.2 / 9.4 / 8.4, sixteen - / 15.7 / 11.7.
+// 7.7 / 6.5 / 8.4, eight 14.2 / 9.4 / 8.4 (which k_decode_router takes now).
 static int logits_depth(int max_tokens) { return max_tokens <= 1 ? 1 : max_tokens <= 6 ? 2 : 4; }
 
 
@@ -218,48 +221,144 @@ __device__ __forceinline__ void tile_normed(const uint8_t* __restrict__ w0, cons
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// A: grid = max_tokens * superblocks (norm and digits) + max_tokens (gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
-// A chunk is two tokens sharing one pass over the weights.
-// ------------------------------------------------------------------------------------------------
-template <int SQ, int RF, int RPS, int kLogitsDepth, bool PRE = false>
-__global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
-  __shared__ float s_red[4];
-  __shared__ uint32_t s_mag[4];  // the row writers': a wavefront's largest magnitude
-  __shared__ __attribute__((aligned(16))) float s_xn[3 * kXnPad];  // the chunk's rows and the norm weight
-  const int chunks = (a.max_tokens + 1) / 2;
-  const int n_r = chunks * a.tiles_r;
+// group_sum of four values at once, value t in the lanes t and t + 8 of every sixteen: the lanes of a quad add up one value
+// each from the second addition on.  The additions pair the same partial sums in the same order as group_sum's, so the
+// sums are the same bits.
+template <int G>
+__device__ __forceinline__ float group_sum_of_four(const float (&v)[4]) {
+  static_assert(G == 16 || G == 64, "group width");
+  const int lane = __lane_id();
+  const bool b0 = lane & 1, b1 = lane & 2;
+  const float p = (b0 ? v[1] : v[0]) + dpp_f<0xB1>(b0 ? v[0] : v[1]);  // quad_perm [1,0,3,2]
+  const float q = (b0 ? v[3] : v[2]) + dpp_f<0xB1>(b0 ? v[2] : v[3]);
+  float s = (b1 ? q : p) + dpp_f<0x4E>(b1 ? p : q);                    // quad_perm [2,3,0,1]
+  s += dpp_f<0x12C>(s);  // row_ror:12: the next quad's
+  s += dpp_f<0x128>(s);  // row_ror:8: the other eight lanes'
+  if constexpr (G == 64) {
+    const uint32_t a = __builtin_bit_cast(uint32_t, s);
+    const auto r = __builtin_amdgcn_permlane16_swap(a, a, false, false);  // {rows 0 0 2 2, rows 1 1 3 3}
+    const uint32_t r0 = r[0], r1 = r[1];
+    s = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+    const uint32_t c = __builtin_bit_cast(uint32_t, s);
+    const auto h = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+    const uint32_t h0 = h[0], h1 = h[1];
+    s = __builtin_bit_cast(float, h0) + __builtin_bit_cast(float, h1);
+  }
+  return s;
+}
+
+// The same rows for wider batches: four tokens per pass over the rows' weights (tile_normed: two), a token's row normalised
+// once per workgroup instead of once per wavefront, four tokens' sums across the lanes taken together, and one SwiGLU for
+// the four.  What bounds it is the chain (a round trip for the rows, a barrier each for staging and norm) and about 300
+// vector instructions per wavefront; more steps per wavefront save fetched rows and cost workgroups in flight.  Measured,
+// us at 13 / 32 / 45 tokens, steps 1 / 2 / 4 of a wavefront: router 7.0 8.6 11.0 / 6.9 7.6 9.7 / 9.9 8.9 11.2, shared
+// gate/up (with the routing beside it, 6.1 alone) 6.1 8.4 10.4 / 6.1 10.2 11.2 / 10.6 11.6 15.1.  With router, shared
+// gate/up and norm in one launch of two-token chunks and the routing behind it: 20.5 / 22.8 / 26.2 for what now takes
+// 13.0 / 16.0 / 20.1.
+constexpr int kGroupTokens = 4;  // (a wavefront of the workgroup each)
+template <int QUANT, int RPS, int NM, int D, bool PRE>
+__device__ __forceinline__ void tile_group(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, int K, int n_rows,
+                                           int row0, const float* __restrict__ rows, int token0, int max_tokens,
+                                           const float* __restrict__ norm_w, float eps, float* __restrict__ out,
+                                           const float* __restrict__ bias, const int* __restrict__ valid_tokens, float* s_xn) {
+  using F = Fmt<QUANT>;
+  using Raw = typename F::Raw;
+  constexpr int G = 64 / RPS, TC = kGroupTokens;
+  const LaneGeom g = lane_geom<QUANT>();
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int first_item = a.max_tokens * (a.H / kSbElems + 1);
-  if ((int)blockIdx.x >= first_item) {
-    int item = (int)blockIdx.x - first_item;
-    const bool router = item < n_r;
-    if (!router) item -= n_r;
-    const int tiles = router ? a.tiles_r : a.tiles_s;
-    const int c = item / tiles, tile = item % tiles, t0 = 2 * c;
-    const int row0 = (tile * kWavesPerWg + wave) * RPS * kLogitsDepth;
-    const float* x0 = (PRE ? a.normed : a.residual) + (size_t)t0 * a.H;
-    if (t0 + 1 < a.max_tokens) {
-      const float* const xr[2] = {x0, x0 + a.H};
-      if (router) {
-        float* const o[2] = {a.logits + (size_t)t0 * a.E, a.logits + (size_t)(t0 + 1) * a.E};
-        tile_normed<RF, RPS, 2, 1, kLogitsDepth, PRE>(a.router, nullptr, a.H, a.E, row0, xr, a.post_norm, a.eps, o, a.logit_bias, a.valid_tokens, t0, s_xn);
-      } else {
-        float* const o[2] = {a.shared_inter + (size_t)t0 * a.I, a.shared_inter + (size_t)(t0 + 1) * a.I};
-        tile_normed<SQ, RPS, 2, 2, kLogitsDepth, PRE>(a.sgate, a.sup, a.H, a.I, row0, xr, a.post_norm, a.eps, o, nullptr, a.valid_tokens, t0, s_xn);
-      }
-    } else {
-      const float* const xr[1] = {x0};
-      if (router) {
-        float* const o[1] = {a.logits + (size_t)t0 * a.E};
-        tile_normed<RF, RPS, 1, 1, kLogitsDepth, PRE>(a.router, nullptr, a.H, a.E, row0, xr, a.post_norm, a.eps, o, a.logit_bias, a.valid_tokens, t0, s_xn);
-      } else {
-        float* const o[1] = {a.shared_inter + (size_t)t0 * a.I};
-        tile_normed<SQ, RPS, 1, 2, kLogitsDepth, PRE>(a.sgate, a.sup, a.H, a.I, row0, xr, a.post_norm, a.eps, o, nullptr, a.valid_tokens, t0, s_xn);
+  const int koff = lane_koff<QUANT, RPS>(g, 0);
+  const size_t row_bytes = (size_t)(K / F::kBlockElems) * F::kBlockBytes;
+  // (a token past the batch re-reads its last one, a step past the matrix its last one: neither is stored)
+  Raw r[D][NM];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const int rd = min(row0 + d * RPS, n_rows - RPS);
+    load_raw<QUANT, true>(w0 + (size_t)rd * row_bytes, true, g, r[d][0]);
+    if constexpr (NM == 2) load_raw<QUANT, true>(w1 + (size_t)rd * row_bytes, true, g, r[d][NM - 1]);
+  }
+  const int n4 = K / 4;
+  {
+    float4 xq[2][TC];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int t = 0; t < TC; ++t)
+        xq[j][t] = reinterpret_cast<const float4*>(rows + (size_t)min(token0 + t, max_tokens - 1) * K)[min((int)threadIdx.x + 256 * j, n4 - 1)];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = (int)threadIdx.x + 256 * j;
+      if (i < n4) {
+#pragma unroll
+        for (int t = 0; t < TC; ++t) *reinterpret_cast<float4*>(s_xn + t * kXnPad + xn_at(4 * i)) = xq[j][t];
       }
     }
-    return;
   }
+  const int valid = *valid_tokens;
+  __syncthreads();
+  if constexpr (!PRE) {
+    // wavefront t: token t's RMS scale in the canonical order (lane L folds elements 32 L .. 32 L + 31, then the wavefront
+    // tree), and the lane's elements put back as (x * inv) * w
+    float* row = s_xn + wave * kXnPad + xn_at(min(g.lane * 32, K - 32));  // (lanes past the row's end fold zeros)
+    float4 f[8], nw[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) nw[j] = reinterpret_cast<const float4*>(norm_w + min(g.lane * 32, K - 32))[j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = reinterpret_cast<const float4*>(row)[j];
+    float sq = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      sq = __builtin_fmaf(f[j].x, f[j].x, sq);
+      sq = __builtin_fmaf(f[j].y, f[j].y, sq);
+      sq = __builtin_fmaf(f[j].z, f[j].z, sq);
+      sq = __builtin_fmaf(f[j].w, f[j].w, sq);
+    }
+    if (g.lane * 32 >= K) sq = 0.0f;
+    const float inv = rms_finish(sq, K, eps);
+    if (g.lane * 32 < K) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        reinterpret_cast<float4*>(row)[j] = make_float4(f[j].x * inv * nw[j].x, f[j].y * inv * nw[j].y, f[j].z * inv * nw[j].z, f[j].w * inv * nw[j].w);
+    }
+    __syncthreads();
+  }
+  if (row0 >= n_rows) return;
+  float x[TC][32], xs[TC][4];
+#pragma unroll
+  for (int t = 0; t < TC; ++t) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int off = QUANT == kQ6K ? koff + g.half * 128 + j * 32 + g.l8 * 8 : koff + j * 8;
+      const float4* p = reinterpret_cast<const float4*>(s_xn + t * kXnPad + xn_at(off));
+      const float4 lo = p[0], hi = p[1];
+      x[t][j * 8 + 0] = lo.x; x[t][j * 8 + 1] = lo.y; x[t][j * 8 + 2] = lo.z; x[t][j * 8 + 3] = lo.w;
+      x[t][j * 8 + 4] = hi.x; x[t][j * 8 + 5] = hi.y; x[t][j * 8 + 6] = hi.z; x[t][j * 8 + 7] = hi.w;
+    }
+    lane_x_offsets<QUANT>(x[t], xs[t]);
+  }
+  const int t = token0 + (g.lane & 3);
+  const bool stores = (g.lane % G) < TC && t < valid;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    float sum[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      float tot[TC] = {0.0f, 0.0f, 0.0f, 0.0f};
+      accum<QUANT, TC>(r[d][m], g, x, xs, tot);
+      sum[m] = group_sum_of_four<G>(tot);
+    }
+    const int row = row0 + d * RPS + g.lane / G;
+    float v = NM == 2 ? silu_f(sum[0]) * sum[NM - 1] : 1.0f * sum[0];
+    if (stores && row < n_rows) {
+      if (NM == 1 && bias) v += bias[row];
+      out[(size_t)t * n_rows + row] = v;
+    }
+  }
+}
+
+// What the first workgroups of A do: a superblock of a token's normalised row with its digits each, then a token's gate each.
+template <bool PRE>
+__device__ __forceinline__ void token_rows(const DecodeArgs& a, float* s_red, uint32_t* s_mag) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int nsb = a.H / kSbElems;  // (the served widths are multiples of 256)
   const int valid = *a.valid_tokens;
   if ((int)blockIdx.x < a.max_tokens * nsb) {
@@ -312,18 +411,93 @@ __global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// A: grid = max_tokens * superblocks (norm and digits) + max_tokens (gate scalar) + chunks * tiles_r (router) + chunks * tiles_s (shared gate/up).
+// A chunk is two tokens sharing one pass over the weights.
+// ------------------------------------------------------------------------------------------------
+template <int SQ, int RF, int RPS, int kLogitsDepth, bool PRE = false>
+__global__ void __launch_bounds__(256) k_decode_logits(DecodeArgs a) {
+  __shared__ float s_red[4];
+  __shared__ uint32_t s_mag[4];  // the row writers': a wavefront's largest magnitude
+  __shared__ __attribute__((aligned(16))) float s_xn[3 * kXnPad];  // the chunk's rows and the norm weight
+  const int chunks = (a.max_tokens + 1) / 2;
+  const int n_r = chunks * a.tiles_r;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int first_item = a.max_tokens * (a.H / kSbElems + 1);
+  if ((int)blockIdx.x >= first_item) {
+    int item = (int)blockIdx.x - first_item;
+    const bool router = item < n_r;
+    if (!router) item -= n_r;
+    const int tiles = router ? a.tiles_r : a.tiles_s;
+    const int c = item / tiles, tile = item % tiles, t0 = 2 * c;
+    const int row0 = (tile * kWavesPerWg + wave) * RPS * kLogitsDepth;
+    const float* x0 = (PRE ? a.normed : a.residual) + (size_t)t0 * a.H;
+    if (t0 + 1 < a.max_tokens) {
+      const float* const xr[2] = {x0, x0 + a.H};
+      if (router) {
+        float* const o[2] = {a.logits + (size_t)t0 * a.E, a.logits + (size_t)(t0 + 1) * a.E};
+        tile_normed<RF, RPS, 2, 1, kLogitsDepth, PRE>(a.router, nullptr, a.H, a.E, row0, xr, a.post_norm, a.eps, o, a.logit_bias, a.valid_tokens, t0, s_xn);
+      } else {
+        float* const o[2] = {a.shared_inter + (size_t)t0 * a.I, a.shared_inter + (size_t)(t0 + 1) * a.I};
+        tile_normed<SQ, RPS, 2, 2, kLogitsDepth, PRE>(a.sgate, a.sup, a.H, a.I, row0, xr, a.post_norm, a.eps, o, nullptr, a.valid_tokens, t0, s_xn);
+      }
+    } else {
+      const float* const xr[1] = {x0};
+      if (router) {
+        float* const o[1] = {a.logits + (size_t)t0 * a.E};
+        tile_normed<RF, RPS, 1, 1, kLogitsDepth, PRE>(a.router, nullptr, a.H, a.E, row0, xr, a.post_norm, a.eps, o, a.logit_bias, a.valid_tokens, t0, s_xn);
+      } else {
+        float* const o[1] = {a.shared_inter + (size_t)t0 * a.I};
+        tile_normed<SQ, RPS, 1, 2, kLogitsDepth, PRE>(a.sgate, a.sup, a.H, a.I, row0, xr, a.post_norm, a.eps, o, nullptr, a.valid_tokens, t0, s_xn);
+      }
+    }
+    return;
+  }
+  token_rows<PRE>(a, s_red, s_mag);
+}
+
+// ------------------------------------------------------------------------------------------------
 // B: grid = max_tokens * top_k * shares of the row tiles (in wide batches padded to whole rounds of the XCDs, and the
 // shared expert's down projection behind them).
 // ------------------------------------------------------------------------------------------------
-// The routing launch of wider batches: one wavefront per token (route_one_token, the stand-alone routing kernel's
-// body), one token per workgroup so that the tokens spread over the chip.
-__global__ void __launch_bounds__(64) k_decode_route(DecodeArgs a) {
-  extern __shared__ float s_route_one[];  // num_experts floats
+// From kPreRouteMinTokens tokens on: A with the router's rows alone ...
+constexpr int kRouterSteps = 2, kSharedSteps = 1;  // steps per wavefront (tile_group's D)
+template <int RF, int RPS, bool PRE>
+__global__ void __launch_bounds__(256, 2) k_decode_router(DecodeArgs a) {
+  __shared__ float s_red[4];
+  __shared__ uint32_t s_mag[4];
+  __shared__ __attribute__((aligned(16))) float s_xn[kGroupTokens * kXnPad];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int item = (int)blockIdx.x - a.max_tokens * (a.H / kSbElems + 1);
+  if (item < 0) {
+    token_rows<PRE>(a, s_red, s_mag);
+    return;
+  }
+  const int group = item / a.tiles_r, tile = item % a.tiles_r;
+  tile_group<RF, RPS, 1, kRouterSteps, PRE>(a.router, nullptr, a.H, a.E, (tile * kWavesPerWg + wave) * RPS * kRouterSteps,
+                                            PRE ? a.normed : a.residual, group * kGroupTokens, a.max_tokens, a.post_norm, a.eps,
+                                            a.logits, a.logit_bias, a.valid_tokens, s_xn);
+}
+// ... and, once the logits and the normalised rows are there, the routing (one wavefront per token, one token per workgroup
+// so that they spread over the chip: route_one_token, the stand-alone routing kernel's body) beside the shared expert's
+// gate/up, which does not wait for it.
+template <int SQ, int RPS>
+__global__ void __launch_bounds__(256, 2) k_decode_route(DecodeArgs a) {
+  __shared__ __attribute__((aligned(16))) float s_xn[kGroupTokens * kXnPad];
+  static_assert(kGroupTokens * kXnPad >= (int)kRouteMaxExperts, "a token's logits fit");
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int item = (int)blockIdx.x - a.max_tokens;
+  if (item >= 0) {
+    const int group = item / a.tiles_s, tile = item % a.tiles_s;
+    tile_group<SQ, RPS, 2, kSharedSteps, true>(a.sgate, a.sup, a.H, a.I, (tile * kWavesPerWg + wave) * RPS * kSharedSteps, a.normed,
+                                               group * kGroupTokens, a.max_tokens, nullptr, a.eps, a.shared_inter, nullptr,
+                                               a.valid_tokens, s_xn);
+    return;
+  }
   const int t = blockIdx.x;
-  if (t >= *a.valid_tokens) return;
+  if (wave != 0 || t >= *a.valid_tokens) return;
   int sel_i;
   float sel_w;
-  route_one_token(a.logits + (size_t)t * a.E, a.E, a.top_k, s_route_one, sel_i, sel_w);
+  route_one_token(a.logits + (size_t)t * a.E, a.E, a.top_k, s_xn, sel_i, sel_w);
   if ((int)threadIdx.x < a.top_k) {
     a.topk_ids[(size_t)t * a.top_k + threadIdx.x] = sel_i;
     a.topk_weights[(size_t)t * a.top_k + threadIdx.x] = sel_w;
@@ -714,8 +888,8 @@ static int decode_share(size_t units, int tiles) {
 struct Launch {
   const DecodeArgs& a;
   hipStream_t s;
-  unsigned grid_a, grid_b, grid_c;
-  bool pre_routed;  // a routing launch between A and B instead of routing inside B
+  unsigned grid_a, grid_route, grid_b, grid_c;
+  bool pre_routed;  // k_decode_router and k_decode_route instead of k_decode_logits and routing inside B
   bool pre_normed;  // `normed` holds this pass's rows already (the previous block's tail): A neither normalises nor writes them
   unsigned launches;  // bit i: issue launch i (A, B, C); all three outside measurements
 };
@@ -744,23 +918,32 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
     else if (da == 2) hipLaunchKernelGGL((k_decode_logits<SQ, RF, RPSH, 2, PRE>), dim3(l.grid_a), dim3(256), 0, l.s, l.a); \
     else hipLaunchKernelGGL((k_decode_logits<SQ, RF, RPSH, 4, PRE>), dim3(l.grid_a), dim3(256), 0, l.s, l.a);     \
   } while (0)
+#define XABE_AR(RF)                                                                                                      \
+  do {                                                                                                                   \
+    if (l.pre_normed) hipLaunchKernelGGL((k_decode_router<RF, RPSH, true>), dim3(l.grid_a), dim3(256), 0, l.s, l.a);     \
+    else hipLaunchKernelGGL((k_decode_router<RF, RPSH, false>), dim3(l.grid_a), dim3(256), 0, l.s, l.a);                 \
+  } while (0)
 #define XABE_A(SQ, RF)                  \
   do {                                  \
     if (l.pre_normed) XABE_A1(SQ, RF, true); \
     else XABE_A1(SQ, RF, false);        \
   } while (0)
-    if (sg6 && rf32) XABE_A(kQ6K, kF32);
+    if (l.pre_routed && rf32) XABE_AR(kF32);
+    else if (l.pre_routed) XABE_AR(kQ8_0);
+    else if (sg6 && rf32) XABE_A(kQ6K, kF32);
     else if (sg6) XABE_A(kQ6K, kQ8_0);
     else if (rf32) XABE_A(kQ8_0, kF32);
     else XABE_A(kQ8_0, kQ8_0);
 #undef XABE_A
+#undef XABE_AR
 #undef XABE_A1
   }
   if (l.launches & 2u) {
     const size_t lds = up_lds<NP>(gq, l.a.E);
     const dim3 grid(l.grid_b), block(128 * NP);
     if (l.pre_routed) {
-      hipLaunchKernelGGL(k_decode_route, dim3((unsigned)l.a.max_tokens), dim3(64), l.a.E * sizeof(float), l.s, l.a);
+      if (sg6) hipLaunchKernelGGL((k_decode_route<kQ6K, RPSH>), dim3(l.grid_route), dim3(256), 0, l.s, l.a);
+      else hipLaunchKernelGGL((k_decode_route<kQ8_0, RPSH>), dim3(l.grid_route), dim3(256), 0, l.s, l.a);
     }
 #define XABE_B(RQ, SQ)                                                                                            \
   do {                                                                                                            \
@@ -908,8 +1091,18 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   a.share_d = decode_share((size_t)a.max_tokens, a.tiles_d);
   const int chunks = (a.max_tokens + 1) / 2;
   const bool pre_routed = a.max_tokens >= kPreRouteMinTokens;
-  Launch l{a, s, 0, 0, 0, pre_routed, seam && seam->input_normed, launches};
-  l.grid_a = (unsigned)(chunks * (a.tiles_r + a.tiles_s) + a.max_tokens * (a.H / kSbElems + 1));
+  Launch l{a, s, 0, 0, 0, 0, pre_routed, seam && seam->input_normed, launches};
+  const int row_wgs = a.max_tokens * (a.H / kSbElems + 1);
+  if (pre_routed) {
+    const int groups = (a.max_tokens + kGroupTokens - 1) / kGroupTokens;
+    auto tiles_of = [&](int rows, int steps) { return (rows + kWavesPerWg * rps_h * steps - 1) / (kWavesPerWg * rps_h * steps); };
+    a.tiles_r = tiles_of(a.E, kRouterSteps);
+    a.tiles_s = tiles_of(a.I, kSharedSteps);
+    l.grid_a = (unsigned)(row_wgs + groups * a.tiles_r);
+    l.grid_route = (unsigned)(a.max_tokens + groups * a.tiles_s);
+  } else {
+    l.grid_a = (unsigned)(row_wgs + chunks * (a.tiles_r + a.tiles_s));
+  }
   // wide batches pad the shares of a pair (token) to whole rounds of eight, one per XCD
   auto grid_of = [&](size_t units, int shares) { return (unsigned)(units * (a.max_tokens >= kXcdGroupMinTokens ? (shares + 7) / 8 * 8 : shares)); };
   a.shared_from = (int)grid_of((size_t)a.max_tokens * a.top_k, a.tiles_g / a.share_g);

@@ -168,3 +168,13 @@ def test_formats_with_the_routing_inside_and_apart(oracle, X, max_tokens, eq, dq
         g = X.MoeGeometry(16, top_k, 512, 256, 32, max_tokens)
         _compare(X, oracle, g, (max_tokens, max_tokens - 1), seed=4800 + max_tokens + top_k, expert_quant=q(eq),
                  shared_quant=q(sq), down_quant=q(dq), shared_down_quant=q(sdq))
+
+
+@pytest.mark.parametrize("max_tokens", [8, 9, 10, 11, 13, 62])
+@pytest.mark.parametrize("router_q8,shared", [(True, "Q6K"), (False, "Q8_0")])
+@pytest.mark.parametrize("small", [True, False])
+def test_groups_of_four_tokens(oracle, X, max_tokens, router_q8, shared, small):
+    # router and shared gate/up take four tokens per pass over their weights: the last group whole, or short by one to three
+    g = X.MoeGeometry(20, 3, 512, 256, 32, max_tokens) if small else X.MoeGeometry.qwen3_6(X.moe_block_size(max_tokens), max_tokens)
+    _compare(X, oracle, g, (max_tokens, max_tokens - 5), seed=4900 + max_tokens, router_q8=router_q8, bias=router_q8,
+             shared_quant=getattr(X.ExpertQuant, shared))
