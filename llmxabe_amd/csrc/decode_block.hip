@@ -55,6 +55,11 @@ constexpr int kPreRouteMinTokens = 8;
 // (32 tokens: 256 pairs over ~163 experts), whose rows then come out of HBM once per XCD instead of once per pair.
 // At 16 tokens and below, where fewer pairs coincide, the plain order measured 0.1-0.5 us faster and is kept.
 constexpr int kXcdGroupMinTokens = 24;
+// From this width on the second launch of Q6_K gate/up goes by expert, two pairs at a time (k_decode_up_shared): enough pairs
+// coincide to pay for making the units.  us per block of four in one graph, by pair / by expert: uniform routing 20 tokens
+// 365 / 381, 26: 445 / 445, 32: 507 / 497, 40: 601 / 574, 50: 715 / 659, 63: 860 / 753; skewed 20: 285 / 288, 26: 346 / 339,
+// 32: 397 / 377, 63: 687 / 632.  (Q8_0's codes are the matrix operand as they lie: there is no unpacking to share.)
+constexpr int kPairUnitsMinTokens = 28;
 // the seam's arrival counters: per token one counter and one per group of kSeamGroup workgroups, 128 bytes apart
 constexpr int kSeamGroup = 16, kSeamMaxGroups = 64, kSeamCountersPerToken = 1 + kSeamMaxGroups, kSeamCounterStride = 32;
 constexpr int kMaxShare = 4;      // consecutive tiles a workgroup of the second or third launch takes at most
@@ -101,6 +106,7 @@ struct DecodeArgs {
   float eps;
   int H, I, E, top_k, max_tokens;
   int tiles_r, tiles_s, tiles_g, tiles_d;  // row tiles: router, shared gate/up (launch A), gate/up (B), down (C)
+  int shared_units;                        // of the shared down projection in B (k_decode_up_shared)
   int shared_from;                         // first workgroup of the shared down projection in B (wider batches)
   int share_g, share_d;                    // consecutive tiles of a workgroup (B, C): divide tiles_g and tiles_d
 };
@@ -504,14 +510,14 @@ __global__ void __launch_bounds__(256, 2) k_decode_route(DecodeArgs a) {
   }
 }
 
-// Shared expert's down projection: unit = (chunk of two tokens, WAVES * 4 steps of RPS rows).
-template <int SQ, int RPS, int WAVES>
+// Shared expert's down projection, a wavefront's unit: (chunk of two tokens, four steps of RPS rows).
+template <int SQ, int RPS>
 __device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) {
   using RawS = typename Fmt<SQ>::Raw;
   constexpr int G = 64 / RPS;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)__lane_id();
-  const int units_per_chunk = a.H / (WAVES * 4 * RPS);
-  const int t0 = 2 * (unit / units_per_chunk), row0 = ((unit % units_per_chunk) * WAVES + wave) * 4 * RPS;
+  const int lane = (int)__lane_id();
+  const int units_per_chunk = a.H / (4 * RPS);
+  const int t0 = 2 * (unit / units_per_chunk), row0 = (unit % units_per_chunk) * 4 * RPS;
   const int t1 = min(t0 + 1, a.max_tokens - 1);
   const int valid = *a.valid_tokens;
   const LaneGeom g = lane_geom<SQ>();
@@ -564,7 +570,7 @@ __global__ void __launch_bounds__(128 * NP, DIRECT ? 2 : 4) k_decode_up(DecodeAr
   float* const s_route = reinterpret_cast<float*>(s_up + kWaves * PairDma<RQ>::kSlotBytes);
   if constexpr (ROUTED) {
     if ((int)blockIdx.x >= a.shared_from) {
-      shared_down_rows<SQ, RPSI, 2 * NP>(a, (int)blockIdx.x - a.shared_from);
+      shared_down_rows<SQ, RPSI>(a, __builtin_amdgcn_readfirstlane(2 * NP * ((int)blockIdx.x - a.shared_from) + (int)(threadIdx.x >> 6)));
       return;
     }
   }
@@ -691,6 +697,244 @@ __global__ void __launch_bounds__(128 * NP, DIRECT ? 2 : 4) k_decode_up(DecodeAr
     if (lane < 16) a.inter[(size_t)p * a.I + row] = v;
     store_digit_group(v, row, a.inter_d + (size_t)p * nsb_i * kSbDigitBytes, a.inter_e + (size_t)p * nsb_i * 16, lane < 16);
   }
+}
+
+// B for kPairUnitsMinTokens tokens and more, routed gate/up in Q6_K: by expert.  A unit is two (token, k) pairs that selected
+// one expert, or the one left over; their tiles (k_decode_up's, a wavefront's part the same) unpack a weight once for both
+// tokens and fetch it once.  Every workgroup makes the list of units out of topk_ids by itself, alike in all of them (counts by
+// ballots, a scan over the experts): it is resident throughout, two workgroups to a CU, and takes whole units in rounds,
+// then an even share of the tiles of the last, partial round.  An XCD has an eighth of the row tiles, and the units of one
+// expert follow each other, so what more pairs of an expert read again comes out of the L2.  The tokens' digits lie in LDS
+// (24.6 KB: with 16 weight slots of 6.9 KB per CU that leaves room for two workgroups; in registers they would not leave any).
+// Bound by memory: at 45 tokens (360 pairs, 193 experts) 86 us, 382 MB fetched of 332 MB that are distinct; pair by pair
+// 96 us and 590 MB.  Vector instructions 49 % of the cycles.  Measured and not kept: a workgroup per unit, found by a search
+// of its own (88 us; 63 tokens 4 % behind); three pairs with the third's digits in registers (113: spills); the shared
+// expert's rows under the first request instead of at the end (72 against 70 at 32 tokens).
+constexpr int kPairChunks = ((int)kDecodeBlockMaxTokens * kMaxTopK + 63) / 64;
+constexpr int kMaxUnits = 16;  // of a workgroup
+template <int SQ, int NP, int RPSI>
+__global__ void __launch_bounds__(128 * NP, 4) k_decode_up_shared(DecodeArgs a) {
+  using Dma = PairDma<kQ6K, 27, true>;
+  constexpr int kWaves = 2 * NP, kThreads = 64 * kWaves, kDigits = 2 * NP * kSbDigitBytes;  // bytes of a token's row
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_up[];  // two tokens' digits, zeros, a weight slot per wavefront
+  __shared__ int s_first[kMaxUnits], s_second[kMaxUnits];
+  uint8_t* const s_zeros = s_up + 2 * kDigits;
+  uint8_t* const s_slots = s_zeros + kZeroBytes;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = (int)__lane_id(), quarter = lane >> 4;
+  const int valid = *a.valid_tokens, n_live = min(valid, a.max_tokens) * a.top_k;
+
+  // ---- the units: the live pairs by expert, two by two; the same in every workgroup
+  constexpr int kE = (int)kRouteMaxExperts, kPerLane = kE / 64;
+  int* const s_cnt = reinterpret_cast<int*>(s_slots);  // [chunk of 64 pairs][expert]
+  int* const s_pos = s_cnt + kPairChunks * kE;         // [wavefront][expert]: twice the first unit, and the pairs before a chunk's
+  constexpr int kOwn = (kPairChunks + kWaves - 1) / kWaves;  // chunks of a wavefront
+  int id[kOwn], before[kOwn];
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) {
+    const int q = 64 * (wave + kWaves * j) + lane;
+    id[j] = a.topk_ids[min(q, a.max_tokens * a.top_k - 1)];
+    id[j] = q < n_live ? min(max(id[j], 0), a.E - 1) : -1;
+  }
+  typedef int v4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j)
+#pragma unroll
+    for (int i = 0; i < kPerLane / 4; ++i) reinterpret_cast<v4*>(s_cnt + (wave + kWaves * j) * kE)[64 * i + lane] = v4{0, 0, 0, 0};
+  for (int i = (int)threadIdx.x; i < kZeroBytes / 4; i += kThreads) reinterpret_cast<uint32_t*>(s_zeros)[i] = 0;
+  if (threadIdx.x < kMaxUnits) s_second[threadIdx.x] = -1;
+  // (a wavefront's own LDS operations keep their order)
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) {
+    uint64_t same = __builtin_amdgcn_ballot_w64(id[j] >= 0);
+#pragma unroll
+    for (int bit = 0; bit < 9; ++bit) {
+      const uint64_t set = __builtin_amdgcn_ballot_w64((id[j] >> bit) & 1);
+      same &= (id[j] >> bit) & 1 ? set : ~set;
+    }
+    before[j] = __builtin_popcountll(same & ((1ull << lane) - 1));
+    if (id[j] >= 0 && before[j] == 0) s_cnt[(wave + kWaves * j) * kE + id[j]] = __builtin_popcountll(same);
+  }
+  __syncthreads();
+  // every wavefront scans all experts, eight to a lane
+  int n_units;
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) {
+    int count[kPerLane], ahead[kPerLane];
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) count[i] = ahead[i] = 0;
+#pragma unroll
+    for (int c = 0; c < kPairChunks; ++c)
+#pragma unroll
+      for (int q = 0; q < kPerLane / 4; ++q) {
+        const v4 n = reinterpret_cast<const v4*>(s_cnt + c * kE + kPerLane * lane)[q];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (c < wave + kWaves * j) ahead[4 * q + i] += n[i];
+          count[4 * q + i] += n[i];
+        }
+      }
+    int units = 0;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) units += (count[i] + 1) / 2;
+    int scan = units;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(scan, d);
+      if (lane >= d) scan += up;
+    }
+    n_units = __builtin_amdgcn_readlane(scan, 63);
+    int first = scan - units;
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) {
+      s_pos[wave * kE + kPerLane * lane + i] = 2 * first + ahead[i];
+      first += (count[i] + 1) / 2;
+    }
+    if (id[j] >= 0) before[j] += s_pos[wave * kE + id[j]];  // twice the pair's unit, and which of the two it is
+  }
+  // ---- this workgroup's share: an eighth of the row tiles per XCD, the units' tiles dealt evenly and in order
+  const int tiles = a.tiles_g / 8, xcd = (int)blockIdx.x & 7, per_xcd = (int)gridDim.x >> 3, rank = (int)blockIdx.x >> 3;
+  // whole units in rounds (neighbours take units of one expert at the same time: its rows come into the L2 once), the tiles
+  // of the last, partial round dealt evenly
+  const int rounds = n_units / per_xcd, rest = (n_units - rounds * per_xcd) * tiles;
+  const int rest_lo = rest * rank / per_xcd, rest_hi = rest * (rank + 1) / per_xcd;
+  const int rest_unit = rounds * per_xcd + rest_lo / tiles, hi = rounds * tiles + rest_hi - rest_lo;  // (tiles of this workgroup)
+  const uint32_t inverse = ((1u << 20) + per_xcd - 1) / per_xcd;  // (u < 512)
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) {
+    if (id[j] >= 0) {
+      const int u = before[j] >> 1, round = (int)((uint32_t)u * inverse >> 20);
+      const int at = round < rounds ? (u - round * per_xcd == rank ? round : -1) : u >= rest_unit ? rounds + u - rest_unit : -1;
+      const int p = 64 * (wave + kWaves * j) + lane;
+      if (at >= 0 && at < kMaxUnits) {
+        if (before[j] & 1) s_second[at] = p;
+        else s_first[at] = p | id[j] << 9;
+      }
+    }
+  }
+  __syncthreads();
+  // the shared expert's down projection (see k_decode_up): its units dealt over the launch's wavefronts, workgroups first
+  auto shared_down = [&]() __attribute__((always_inline)) {
+    for (int unit = (int)blockIdx.x + wave * (int)gridDim.x; unit < a.shared_units; unit += kWaves * (int)gridDim.x) shared_down_rows<SQ, RPSI>(a, unit);
+  };
+  if (hi > 0) {
+    const int mat = wave & 1, sb0 = 2 * (wave >> 1), sb = sb0 + (quarter >> 1);
+    const uint32_t row_bytes = (uint32_t)(2 * NP * SbRaw<kQ6K>::kBytes);
+    Dma dma;
+    dma.init(row_bytes, sb0);
+    uint8_t* const slot = s_slots + wave * Dma::kSlotBytes;
+    const uint32_t slot_lds = lds_address(slot);
+    const uint8_t* const w = mat ? a.up : a.gate;
+    // the at-th tile of this workgroup: its unit, and its place among the unit's
+    auto tile_of = [&](int at) __attribute__((always_inline)) { return at < rounds * tiles ? at % tiles : (rest_lo + at - rounds * tiles) % tiles; };
+    auto unit_of = [&](int at) __attribute__((always_inline)) {
+      const int i = at < rounds * tiles ? at / tiles : rounds + (rest_lo + at - rounds * tiles) / tiles - rest_lo / tiles;
+      const int f = __builtin_amdgcn_readfirstlane(s_first[i]), g = __builtin_amdgcn_readfirstlane(s_second[i]);
+      return f | (g < 0 ? f & 511 : g) << 18;  // pair, expert, the other pair (or the same)
+    };
+    auto run_off = [&](int unit, int at) __attribute__((always_inline)) {
+      return (size_t)(unit >> 9 & 511) * a.expert_bytes + (size_t)(16 * (xcd * tiles + tile_of(at))) * row_bytes;
+    };
+    const int at_high = pair_high_at(lane), at_low = pair_low_at(lane);
+    const uint8_t *high[2], *low[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint8_t* d = s_up + t * kDigits + sb * kSbDigitBytes;
+      high[t] = at_high >= 0 ? d + at_high : s_zeros;
+      low[t] = at_low >= 0 ? d + at_low : s_zeros;
+    }
+    int unit = unit_of(0);
+    dma.request(w, a.up_len, run_off(unit, 0), slot_lds);
+#pragma unroll 1
+    for (int at = 0; at < hi;) {
+      const int pairs[2] = {unit & 511, unit >> 18}, tok[2] = {pairs[0] / a.top_k, pairs[1] / a.top_k};
+      const bool two = pairs[0] != pairs[1];
+      const int end = min(hi, at + tiles - tile_of(at)), n = end - at;
+      // the tokens' digits: 3 NP pieces of 1 KB each, three per wavefront
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int piece = wave + kWaves * i, t = piece >= 3 * NP, c = piece - 3 * NP * t;
+        lds_dma_16(a.x_d + (size_t)(t ? tok[1] : tok[0]) * kDigits, (uint32_t)(1024 * c + 16 * lane), lds_address(s_up + t * kDigits + 1024 * c));
+      }
+      float xe[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) xe[t] = a.x_e[(size_t)tok[t] * (2 * NP) + sb];
+      wait_loads();
+      __syncthreads();
+      float sums[2][kMaxShare];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < kMaxShare; ++i) sums[t][i] = 0.0f;
+      int next = unit;
+      auto run_tiles = [&](auto nt_c) __attribute__((always_inline)) {
+        constexpr int NT = decltype(nt_c)::value;
+        const uint8_t* hi_at[NT];
+        const uint8_t* lo_at[NT];
+        float es[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) hi_at[t] = high[t], lo_at[t] = low[t], es[t] = xe[t];
+#pragma unroll 1
+        for (int i = 0; i < n; ++i) {
+          wait_loads();
+          if (sb0 + 2 == 2 * NP && run_off(unit, at + i) + (size_t)16 * row_bytes == a.up_len) Dma::patch_tail(w, a.up_len, slot);
+          SbRaw<kQ6K> raw;
+          sb_read_slot(Dma::row_at(slot, row_bytes, lane & 15, sb0) + (quarter >> 1) * SbRaw<kQ6K>::kBytes, quarter & 1, raw);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          if (at + i + 1 < hi) {
+            if (i + 1 == n) next = unit_of(at + i + 1);
+            dma.request(w, a.up_len, run_off(next, at + i + 1), slot_lds);
+          }
+          auto x_of = [&](int t, int q) __attribute__((always_inline)) { return a.normed + (size_t)tok[t] * a.H + (sb0 + (q >> 1)) * kSbElems; };
+          float out[NT];
+          pair_dot_lds<NT>(raw, hi_at, lo_at, es, x_of, out);
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < kMaxShare; ++j)
+              if (j == i) sums[t][j] = out[t];
+        }
+      };
+      if (two) run_tiles(std::integral_constant<int, 2>{});
+      else run_tiles(std::integral_constant<int, 1>{});
+      __syncthreads();  // (everyone has read the digits for the last time: the sums go there)
+      float (*const s_red)[2][2 * NP][64] = reinterpret_cast<float (*)[2][2 * NP][64]>(s_up);  // [tile][token][superblock][half, matrix, row]
+      static_assert(kMaxShare * 2 * 2 * NP * 64 * sizeof(float) <= 2 * kDigits, "the sums fit");
+#pragma unroll
+      for (int i = 0; i < kMaxShare; ++i)
+        if (i < n) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            if (t == 0 || two) s_red[i][t][sb][(quarter & 1) * 32 + mat * 16 + (lane & 15)] = sums[t][i];
+        }
+      __syncthreads();
+      for (int u = wave; u < (two ? 2 : 1) * n; u += kWaves) {
+        const int t = u >= n, i = u - t * n;
+        const float (&red)[2 * NP][64] = s_red[i][t];
+        float h0 = red[0][lane & 31], h1 = red[0][32 + (lane & 31)];
+#pragma unroll
+        for (int c = 1; c < 2 * NP; ++c) {
+          h0 += red[c][lane & 31];
+          h1 += red[c][32 + (lane & 31)];
+        }
+        const float sum = h0 + h1, up = __shfl_xor(sum, 16);
+        const int nsb_i = a.I / kSbElems, pr = t ? pairs[1] : pairs[0];
+        const float v = silu_f(sum) * up;
+        const int row = 16 * (xcd * tiles + tile_of(at) + i) + (lane & 15);
+        if (lane < 16) a.inter[(size_t)pr * a.I + row] = v;
+        store_digit_group(v, row, a.inter_d + (size_t)pr * nsb_i * kSbDigitBytes, a.inter_e + (size_t)pr * nsb_i * 16, lane < 16);
+      }
+      __syncthreads();  // (the sums are read: the next digits go there)
+      at = end;
+      unit = next;
+    }
+  }
+  shared_down();
+}
+template <int NP>
+constexpr size_t up_shared_lds() {
+  return (size_t)2 * 2 * NP * kSbDigitBytes + kZeroBytes +
+         std::max((size_t)2 * NP * PairDma<kQ6K, 27, true>::kSlotBytes, (size_t)(kPairChunks + 2 * NP) * kRouteMaxExperts * sizeof(int));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -888,8 +1132,9 @@ static int decode_share(size_t units, int tiles) {
 struct Launch {
   const DecodeArgs& a;
   hipStream_t s;
-  unsigned grid_a, grid_route, grid_b, grid_c;
+  unsigned grid_a, grid_route, grid_b, grid_shared, grid_c;
   bool pre_routed;  // k_decode_router and k_decode_route instead of k_decode_logits and routing inside B
+  bool pair_units;  // k_decode_up_shared instead of k_decode_up
   bool pre_normed;  // `normed` holds this pass's rows already (the previous block's tail): A neither normalises nor writes them
   unsigned launches;  // bit i: issue launch i (A, B, C); all three outside measurements
 };
@@ -945,6 +1190,10 @@ static bool launch_all(const Launch& l, int gq, int dq, int sgq, int sdq, int ro
       if (sg6) hipLaunchKernelGGL((k_decode_route<kQ6K, RPSH>), dim3(l.grid_route), dim3(256), 0, l.s, l.a);
       else hipLaunchKernelGGL((k_decode_route<kQ8_0, RPSH>), dim3(l.grid_route), dim3(256), 0, l.s, l.a);
     }
+    if (l.pair_units) {
+      if (sd6) hipLaunchKernelGGL((k_decode_up_shared<kQ6K, NP, RPSI>), dim3(l.grid_shared), block, up_shared_lds<NP>(), l.s, l.a);
+      else hipLaunchKernelGGL((k_decode_up_shared<kQ8_0, NP, RPSI>), dim3(l.grid_shared), block, up_shared_lds<NP>(), l.s, l.a);
+    } else
 #define XABE_B(RQ, SQ)                                                                                            \
   do {                                                                                                            \
     if (l.pre_routed) hipLaunchKernelGGL((k_decode_up<RQ, SQ, NP, RPSI, true, false>), grid, block, lds, l.s, l.a); \
@@ -990,6 +1239,8 @@ static int decode_block_set_limits() {
   XABE_UP(Q, code, kQ8_0, 4, 4);                                             \
   XABE_UP(Q, code, kQ6K, 1, 8);                                              \
   XABE_UP(Q, code, kQ8_0, 1, 8)
+  XABE_LDS((k_decode_up_shared<kQ6K, 4, 4>), up_shared_lds<4>());
+  XABE_LDS((k_decode_up_shared<kQ8_0, 4, 4>), up_shared_lds<4>());
   XABE_DOWN(kQ6K, XABE_QUANT_Q6K);
   XABE_DOWN(kQ8_0, XABE_QUANT_Q8_0);
 #undef XABE_DOWN
@@ -1091,7 +1342,8 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   a.share_d = decode_share((size_t)a.max_tokens, a.tiles_d);
   const int chunks = (a.max_tokens + 1) / 2;
   const bool pre_routed = a.max_tokens >= kPreRouteMinTokens;
-  Launch l{a, s, 0, 0, 0, 0, pre_routed, seam && seam->input_normed, launches};
+  const bool pair_units = a.max_tokens >= kPairUnitsMinTokens && rq == XABE_QUANT_Q6K;
+  Launch l{a, s, 0, 0, 0, 0, 0, pre_routed, pair_units, seam && seam->input_normed, launches};
   const int row_wgs = a.max_tokens * (a.H / kSbElems + 1);
   if (pre_routed) {
     const int groups = (a.max_tokens + kGroupTokens - 1) / kGroupTokens;
@@ -1107,6 +1359,8 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   auto grid_of = [&](size_t units, int shares) { return (unsigned)(units * (a.max_tokens >= kXcdGroupMinTokens ? (shares + 7) / 8 * 8 : shares)); };
   a.shared_from = (int)grid_of((size_t)a.max_tokens * a.top_k, a.tiles_g / a.share_g);
   l.grid_b = (unsigned)(a.shared_from + (pre_routed ? chunks * (a.H / (4 * rps_i * (a.H / 512) * 2)) : 0));
+  a.shared_units = chunks * (a.H / (4 * rps_i));
+  l.grid_shared = 8u * (unsigned)std::max<size_t>(k->num_cus / 4, ((size_t)a.max_tokens * a.top_k + kMaxUnits - 3) / (kMaxUnits - 2));
   l.grid_c = grid_of((size_t)a.max_tokens, a.tiles_d / a.share_d);
   const bool ok = launch_shape(l, w->gate_exps.quant, w->down_exps.quant, w->shared_gate.quant, w->shared_down.quant, w->router_quant);
   if (!ok) return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "decode block: no kernels for this shape or format");

@@ -150,6 +150,11 @@ __device__ __forceinline__ void lds_dma_16(const void* base, uint32_t voff, uint
 #pragma clang diagnostic pop
 }
 
+// The byte address in LDS of what every lane of the wavefront has at `p`.
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
+}
+
 // Everything this wavefront has requested from memory is there, the DMA's bytes in LDS among it.  Said twice: the compiler
 // counts its own loads and takes note of the builtin (a wait of its own for a register loaded before a loop would
 // otherwise stand at its use inside, and wait there for the DMA requested since); it does not count the DMA, whose wait

@@ -649,10 +649,11 @@ struct PackedOffsets {
   }
 };
 
-template <int QUANT>
+// PACKED: the last instruction is for the lanes with a piece only, and slots lie without padding between them.
+template <int QUANT, int PIECES = QUANT == kQ6K ? 29 : 35, bool PACKED = false>
 struct PairDma {
-  static constexpr int kP = QUANT == kQ6K ? 29 : 35;  // 420 bytes from a word boundary, rows four words apart modulo the banks; 35 likewise
-  static constexpr int kInstr = (16 * kP + 63) / 64, kSlotBytes = kInstr * 1024;  // (a slot's last instruction pads)
+  static constexpr int kP = PIECES;  // 420 bytes from a word boundary, rows four words apart modulo the banks; 35 likewise
+  static constexpr int kInstr = (16 * kP + 63) / 64, kSlotBytes = PACKED ? 16 * kP * 16 : kInstr * 1024;  // (otherwise the last instruction pads)
   PackedOffsets<kInstr> off;  // the lane's piece of each instruction, relative to the tile's first row
   // sixteen rows of `row_bytes` (16 row_bytes are whole pieces, and fewer than 65536), superblocks sb0 and sb0 + 1
   __device__ __forceinline__ void init(uint32_t row_bytes, int sb0) {
@@ -669,7 +670,8 @@ struct PairDma {
     const uint32_t last = (uint32_t)min((w_bytes & ~(size_t)15) - 16 - tile, (size_t)0xfffffff0u);
     off.opaque();
 #pragma unroll
-    for (int i = 0; i < kInstr; ++i) lds_dma_16(w + tile, min(off.get(i), last), dst + i * 1024);
+    for (int i = 0; i < kInstr; ++i)
+      if (!PACKED || i + 1 < kInstr || (int)__lane_id() < 16 * kP - 64 * (kInstr - 1)) lds_dma_16(w + tile, min(off.get(i), last), dst + i * 1024);
   }
   // (the tile's last row, this pair its last one, ends the tensor; Q6_K)
   static __device__ __forceinline__ void patch_tail(const uint8_t* w, size_t w_bytes, uint8_t* slot) {
@@ -794,6 +796,60 @@ __device__ __forceinline__ float pair_dot(SbRaw<QUANT>& r, const PairDigits<WHOL
     if (out != out) out = plain;
   }
   return out;
+}
+
+// The same for the rows' codes against one or two tokens (whole superblocks, Q6_K), the digits in LDS: the codes are unpacked
+// once, the sums are pair_dot's.  Where a lane finds its rows of the two operands, relative to its superblock's digits
+// (negative: the row is zero, and the lane reads zeros).
+__device__ __forceinline__ int pair_high_at(int lane) {
+  const int q = lane >> 4, m = lane & 15;
+  return (m >> 2) == q ? 2 * (q & 1) * kGroupBytes + (m & 3) * 16 : -1;
+}
+__device__ __forceinline__ int pair_low_at(int lane) {
+  const int q = lane >> 4, m = lane & 15;
+  return (m >> 2) == q ? (2 * (q & 1) + ((m >> 1) & 1)) * kGroupBytes + (4 + (m & 1)) * 16 : -1;
+}
+template <int NT, typename XOf>
+__device__ __forceinline__ void pair_dot_lds(SbRaw<kQ6K>& r, const uint8_t* const (&high)[NT], const uint8_t* const (&low)[NT],
+                                             const float (&e)[NT], XOf x_of, float (&out)[NT]) {
+  int sum[NT][6];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sum[t][k] = 0;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    v4i_t z[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) z[t] = *reinterpret_cast<const v4i_t*>(low[t] + 4 * s * kGroupBytes);
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const v4i_t zero = {0, 0, 0, 0};
+      v4i_t c;
+      sb_codes(r, s, l, c);
+      const int sc = sb_int_scale(r, s, l);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const v4i_t a = *reinterpret_cast<const v4i_t*>(high[t] + (4 * s + l) * kGroupBytes);
+        const v4i_t dd = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, c, zero, 0, 0, 0);
+        const v4i_t zz = __builtin_amdgcn_mfma_i32_16x16x64_i8(z[t], c, zero, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) add_scaled(sum[t][i], sc, dd[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) add_scaled(sum[t][4 + i], sc, zz[2 * l + i]);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    out[t] = join_sums(sum[t]) * (sb_quarter(r) * e[t]);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(out[t] != out[t]) != 0, 0)) {
+      int quarter = (int)__lane_id() >> 4;
+      asm volatile("" : "+v"(quarter));
+      const float plain = half_fp32(r, x_of(t, quarter) + 128 * (quarter & 1));
+      if (out[t] != out[t]) out[t] = plain;
+    }
+  }
 }
 
 }  // namespace xabe

@@ -694,10 +694,6 @@ __device__ __forceinline__ void lds_dma_4(const void* base, uint32_t voff, uint3
                "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
 #pragma clang diagnostic pop
 }
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
-}
-
 
 template <int MI>
 constexpr int kRing = MI > 2 ? 4 : 3;  // steps of activations in LDS

@@ -178,3 +178,23 @@ def test_groups_of_four_tokens(oracle, X, max_tokens, router_q8, shared, small):
     g = X.MoeGeometry(20, 3, 512, 256, 32, max_tokens) if small else X.MoeGeometry.qwen3_6(X.moe_block_size(max_tokens), max_tokens)
     _compare(X, oracle, g, (max_tokens, max_tokens - 5), seed=4900 + max_tokens, router_q8=router_q8, bias=router_q8,
              shared_quant=getattr(X.ExpertQuant, shared))
+
+
+@pytest.mark.parametrize("max_tokens,experts,top_k", [(28, 256, 8), (33, 20, 3), (41, 8, 8), (63, 512, 8), (63, 64, 1), (50, 12, 5)])
+@pytest.mark.parametrize("small", [True, False])
+def test_units_of_two_pairs(oracle, X, max_tokens, experts, top_k, small):
+    # every count of pairs per expert from none to all of them (two to a unit, one left over), and fewer live tokens
+    import torch
+
+    hidden, inter = (512, 256) if small else (2048, 512)
+    g = X.MoeGeometry(experts, top_k, hidden, inter, 32, max_tokens)
+    layer = make_layer(oracle, g, seed=5000 + max_tokens)
+    one, many = X.MoeBlock(g), X.MoeBlock(g)
+    many.set_fused_decode(False)
+    lean = torch.zeros(experts, device="cuda")
+    lean[: max(1, experts // 5)] = 6.0   # half of a skew: some experts take most tokens
+    for i, (tokens, lb) in enumerate(((max_tokens, None), (max_tokens, lean), (max_tokens - 3, lean), (1, None))):
+        x = activations(5100 + i, g.max_tokens, g.hidden, tokens)
+        f1, l1 = run_block(one, layer, x, tokens, logit_bias=lb)
+        f2, l2 = run_block(many, layer, x, tokens, logit_bias=lb)
+        _same_bits(_observe(one, g, f1, l1, tokens), _observe(many, g, f2, l2, tokens), f"call {i} tokens {tokens}")
