@@ -395,7 +395,7 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->bucket_live, b->n_expert_blocks);
   A(&b->expert_counts, routed ? g.num_experts : 0);
   // the counting-sort form of the dispatch tables, from 8192 selections up
-  b->n_align_chunks = (routed && flat >= 8192 && g.num_experts <= 512) ? (flat + 1023) / 1024 : 0;
+  b->n_align_chunks = (routed && flat >= (size_t)kAlignFusedMaxSelections && g.num_experts <= 512) ? (flat + 1023) / 1024 : 0;
   A(&b->align_hist, b->n_align_chunks * g.num_experts);
   A(&b->num_tokens_post_pad, routed ? 1 : 0);
   A(&b->valid_tokens, 1);
@@ -551,9 +551,10 @@ int xabe_moe_build_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_bu
     return XABE_OK;
   }
   if (g.max_tokens * g.experts_per_token <= (size_t)kAlignFusedMaxSelections && g.num_experts <= 512) {
-    hipLaunchKernelGGL(k_align_fused, dim3(1), dim3(1024), 0, s, b->topk_ids, b->valid_tokens, (int)g.experts_per_token,
-                       (int)g.num_experts, (int)g.block_size, (int)b->n_sorted, (int)b->n_expert_blocks, b->sorted_token_ids,
-                       b->expert_ids, b->bucket_live, b->expert_counts, b->num_tokens_post_pad, tl);
+    hipLaunchKernelGGL(k_align_fused, dim3(1), dim3(1024), 0, s, b->topk_ids, b->valid_tokens,
+                       (int)(g.max_tokens * g.experts_per_token), (int)g.experts_per_token, (int)g.num_experts, (int)g.block_size,
+                       (int)b->n_sorted, (int)b->n_expert_blocks, b->sorted_token_ids, b->expert_ids, b->bucket_live,
+                       b->expert_counts, b->num_tokens_post_pad, tl);
     XABE_HIP_TRY(hipGetLastError());
     if (list) b->tiles_bm = bm;
     return XABE_OK;

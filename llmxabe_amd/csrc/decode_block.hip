@@ -746,12 +746,7 @@ __global__ void __launch_bounds__(128 * NP, 4) k_decode_up_shared(DecodeArgs a) 
   // (a wavefront's own LDS operations keep their order)
 #pragma unroll
   for (int j = 0; j < kOwn; ++j) {
-    uint64_t same = __builtin_amdgcn_ballot_w64(id[j] >= 0);
-#pragma unroll
-    for (int bit = 0; bit < 9; ++bit) {
-      const uint64_t set = __builtin_amdgcn_ballot_w64((id[j] >> bit) & 1);
-      same &= (id[j] >> bit) & 1 ? set : ~set;
-    }
+    const uint64_t same = lanes_alike(id[j], id[j] >= 0);
     before[j] = __builtin_popcountll(same & ((1ull << lane) - 1));
     if (id[j] >= 0 && before[j] == 0) s_cnt[(wave + kWaves * j) * kE + id[j]] = __builtin_popcountll(same);
   }

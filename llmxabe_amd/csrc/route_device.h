@@ -35,6 +35,20 @@ __device__ __forceinline__ void route_load(const float* lg, int num_experts, con
   }
 }
 
+// The lanes among those with `in` that hold the same v (0 <= v < 512) as this one, as a mask: a ballot per bit of v.
+__device__ __forceinline__ unsigned long long lanes_alike(int v, bool in) {
+  const unsigned long long all = __builtin_amdgcn_ballot_w64(in);
+  uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
+#pragma unroll
+  for (int bit = 0; bit < 9; ++bit) {
+    const unsigned long long set = __builtin_amdgcn_ballot_w64((v >> bit) & 1);
+    const uint32_t mine = (uint32_t)((v << (31 - bit)) >> 31);  // all ones where this lane's bit is set
+    lo &= ~((uint32_t)set ^ mine);
+    hi &= ~((uint32_t)(set >> 32) ^ mine);
+  }
+  return (unsigned long long)hi << 32 | lo;
+}
+
 // One selection round over per-lane keys (kTaken = out of the running): the largest key, the lowest index
 // among equals; the winner is marked taken.  Returns the winning key and index to every lane.
 // Almost always exactly one (lane, slot) holds the maximum: then its index is read straight off the ballots and

@@ -199,6 +199,8 @@ __global__ void __launch_bounds__(256) k_route_planes(const float* __restrict__ 
                                                        const float* __restrict__ bias, const int* __restrict__ valid_tokens,
                                                        int num_experts, int top_k, float* __restrict__ logits,
                                                        int* __restrict__ topk_ids, float* __restrict__ topk_weights) {
+  // (ahead of the shared expert's launch beside it where the routing is a latency; with many tokens it is work like any other)
+  if (gridDim.x <= 1024) __builtin_amdgcn_s_setprio(3);
   extern __shared__ float route_smem[];  // 4 x num_experts
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + wave;
@@ -315,6 +317,17 @@ __global__ void __launch_bounds__(256) k_align_scatter(const int* __restrict__ t
   }
 }
 
+// The sum of v over the lanes up to and with this one.
+__device__ __forceinline__ int wave_scan(int v) {
+  const int lane = __lane_id();
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(v, d);
+    if (lane >= d) v += up;
+  }
+  return v;
+}
+
 // ---------------------------------------------------------------------------------
 // Token-tile list of the matrix-core grouped GEMM, written by the dispatch kernels below that hold every expert's
 // count and first slot in one workgroup (otherwise by k_build_tiles in mfma.hip, which documents the layout): one
@@ -329,46 +342,53 @@ struct TileListArgs {
 
 // ---------------------------------------------------------------------------------
 // The same tables from ONE launch of one workgroup, for passes of at most 8192 selections (1024 tokens of top-8):
-// the two launches above cost ~15 us at 512 tokens, nearly all of it launch and barrier latency (every expert's
-// workgroup walks all selections, two barriers per 256 of them).  Sixteen wavefronts split the selections into
-// sixteen consecutive ranges.  Each counts its range per expert (LDS atomics: only the totals are used), thread e
-// turns the sixteen counts of expert e into first slots (prefix over the ranges, plus the expert's base from a scan of
-// the padded totals), and each wavefront then ranks its selections among equals in index order, 64 at a time with
+// what the launches above and below cost at these sizes is launch and barrier latency (twice the selections, 1237 tokens:
+// this launch alone 14.6 us against 21.8 for the three below, but beside the shared expert's launch the block took 342 us
+// against 325, since one CU does all of it).  Sixteen wavefronts split the
+// selections into sixteen consecutive ranges.  Each counts its range per expert (LDS atomics: only the totals are used),
+// thread e turns the sixteen counts of expert e into first slots (prefix over the ranges, plus the expert's base from a
+// scan of the padded totals), and each wavefront then ranks its selections among equals in index order, 64 at a time with
 // one ballot per bit of the id, and writes them.  No result depends on the order in which atomics land.
+// A chain of round trips: the ids are requested before the live count is known (ranges cut from the buffers' size), the
+// scan goes through the wavefronts' lanes with two barriers, rounds past the live count are skipped, and the wavefronts
+// run ahead of whatever shares the CU (the shared expert's launch beside: s_setprio; block at 512 tokens 175 -> 171 us, 1237
+// tokens 323 -> 320).  14.6 -> 10.4 us at 512 tokens.
 // ---------------------------------------------------------------------------------
 constexpr int kAlignFusedMaxSelections = 8192;
 constexpr int kAlignFusedWaves = 16;
 __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ topk_ids, const int* __restrict__ valid_tokens,
-                                                       int top_k, int num_experts, int block_size, int sorted_capacity,
+                                                       int capacity, int top_k, int num_experts, int block_size, int sorted_capacity,
                                                        int expert_capacity, int* __restrict__ sorted_token_ids,
                                                        int* __restrict__ expert_ids, int* __restrict__ bucket_live,
                                                        int* __restrict__ expert_counts, int* __restrict__ num_tokens_post_pad,
                                                        TileListArgs tl) {
+  __builtin_amdgcn_s_setprio(3);
   constexpr int kMaxE = 512, kRounds = kAlignFusedMaxSelections / (kAlignFusedWaves * 64);
   __shared__ int cnt[kAlignFusedWaves][kMaxE];  // per range and expert: count, then next slot
-  __shared__ int s_scan[2][2][kMaxE];           // scanned together: padded counts, tiles
+  __shared__ int s_tot[2][kMaxE / 64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int numel = min(*valid_tokens * top_k, kAlignFusedMaxSelections);
-  // whole-capacity fill first: the barriers below order it before the entries written over it
-  for (int i = tid; i < sorted_capacity; i += 1024) sorted_token_ids[i] = numel;
+  const int per_range = ((capacity + kAlignFusedWaves - 1) / kAlignFusedWaves + 63) / 64 * 64;
+  const int r0 = wave * per_range;
+  int id[kRounds];
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) id[r] = 64 * r < per_range ? topk_ids[min(r0 + r * 64 + lane, capacity - 1)] : -1;
+  const int numel = min(*valid_tokens * top_k, capacity), r1 = min(r0 + per_range, numel);
+  // whole-capacity fill: the barriers below order it before the entries written over it
+  for (int i = tid; i < sorted_capacity / 4; i += 1024) reinterpret_cast<int4*>(sorted_token_ids)[i] = make_int4(numel, numel, numel, numel);
+  for (int i = (sorted_capacity & ~3) + tid; i < sorted_capacity; i += 1024) sorted_token_ids[i] = numel;
   for (int i = tid; i < expert_capacity; i += 1024) {
     expert_ids[i] = -1;
     bucket_live[i] = 0;
   }
-  for (int i = tid; i < kAlignFusedWaves * kMaxE; i += 1024) (&cnt[0][0])[i] = 0;
-  __syncthreads();
-  const int per_range = ((numel + kAlignFusedWaves - 1) / kAlignFusedWaves + 63) / 64 * 64;
-  const int r0 = wave * per_range, r1 = min(r0 + per_range, numel);
-  int id[kRounds];
+  // (a wavefront's own LDS operations keep their order)
+  for (int i = lane; i < kMaxE; i += 64) cnt[wave][i] = 0;
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
-    const int i = r0 + r * 64 + lane;
-    id[r] = i < r1 ? topk_ids[i] : -1;
-    if (id[r] >= num_experts) id[r] = -1;  // (an id no expert has matches nothing, as in the two-launch form)
+    if (r0 + r * 64 + lane >= r1 || id[r] >= num_experts) id[r] = -1;  // (an id no expert has matches nothing, as in the two-launch form)
     if (id[r] >= 0) atomicAdd(&cnt[wave][id[r]], 1);
   }
   __syncthreads();
-  int count = 0, padded = 0, tiles = 0;
+  int count = 0, padded = 0, tiles = 0, base = 0, first = 0;
   if (tid < kMaxE) {
     if (tid < num_experts) {
 #pragma unroll
@@ -380,27 +400,20 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
       padded = (count + block_size - 1) / block_size * block_size;
     }
     tiles = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
-    s_scan[0][0][tid] = padded;
-    s_scan[0][1][tid] = tiles;
+    base = wave_scan(padded);
+    first = wave_scan(tiles);
+    if (lane == 63) s_tot[0][wave] = base, s_tot[1][wave] = first;
   }
   __syncthreads();
-  int cur = 0;
-  for (int d = 1; d < kMaxE; d <<= 1) {
-    if (tid < kMaxE) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][tid] = s_scan[cur][a][tid] + (tid >= d ? s_scan[cur][a][tid - d] : 0);
-    }
-    cur ^= 1;
-    __syncthreads();
-  }
   if (tid < kMaxE) {
-    const int base = s_scan[cur][0][tid] - padded;
+    for (int w = 0; w < wave; ++w) base += s_tot[0][w], first += s_tot[1][w];
     if (tid == kMaxE - 1) {
-      *num_tokens_post_pad = s_scan[cur][0][tid];
-      if (tl.bm > 0) tl.list[0] = min(s_scan[cur][1][tid], tl.capacity);
+      *num_tokens_post_pad = base;
+      if (tl.bm > 0) tl.list[0] = min(first, tl.capacity);
     }
+    base -= padded;
     if (tid < num_experts) {
-      if (tl.bm > 0) write_tile_entries(tid, count, base, s_scan[cur][1][tid] - tiles, tl.bm, tl.capacity, tl.list);
+      if (tl.bm > 0) write_tile_entries(tid, count, base, first - tiles, tl.bm, tl.capacity, tl.list);
       expert_counts[tid] = count;
 #pragma unroll
       for (int w = 0; w < kAlignFusedWaves; ++w) cnt[w][tid] += base;
@@ -416,17 +429,12 @@ __global__ void __launch_bounds__(1024) k_align_fused(const int* __restrict__ to
   }
   __syncthreads();
   int* mine = cnt[wave];
-  int id_bits = 1;
-  while ((1 << id_bits) < num_experts) ++id_bits;
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
+    if (r0 + r * 64 >= r1) break;
     const int i = r0 + r * 64 + lane;
     const int v = id[r];
-    unsigned long long same = __ballot(v >= 0);
-    for (int bit = 0; bit < id_bits; ++bit) {
-      const unsigned long long set = __ballot((v >> bit) & 1);
-      same &= ((v >> bit) & 1) ? set : ~set;
-    }
+    const unsigned long long same = lanes_alike(v, v >= 0);
     int pos = -1;
     if (v >= 0) pos = mine[v] + __popcll(same & ((1ull << lane) - 1ull));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -456,6 +464,7 @@ __global__ void __launch_bounds__(256) k_align_hist(const int* __restrict__ topk
                                                      int top_k, int num_experts, int sorted_capacity, int expert_capacity,
                                                      int* __restrict__ chunk_hist, int* __restrict__ sorted_token_ids,
                                                      int* __restrict__ expert_ids, int* __restrict__ bucket_live) {
+  __builtin_amdgcn_s_setprio(3);
   __shared__ int hist[kAlignMaxExperts];
   const int numel = *valid_tokens * top_k;
   for (int e = threadIdx.x; e < num_experts; e += 256) hist[e] = 0;
@@ -486,9 +495,10 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
                                                         int* __restrict__ chunk_hist, int* __restrict__ expert_counts,
                                                         int* __restrict__ expert_ids, int* __restrict__ bucket_live,
                                                         int* __restrict__ num_tokens_post_pad, TileListArgs tl) {
+  __builtin_amdgcn_s_setprio(3);
   static_assert(kAlignMaxExperts == 512, "one thread per expert slot of the scan");
-  __shared__ int s_scan[2][2][kAlignMaxExperts];  // scanned together: padded counts, tiles
-  const int e = threadIdx.x;
+  __shared__ int s_tot[2][kAlignMaxExperts / 64];
+  const int e = threadIdx.x, wave = e >> 6;
   const int numel = *valid_tokens * top_k;
   const int n_chunks = min(n_chunks_max, (numel + kAlignChunk - 1) / kAlignChunk);
   const bool live = e < num_experts;
@@ -502,24 +512,18 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
     for (int c = kAlignCachedChunks; c < n_chunks; ++c) count += chunk_hist[(size_t)c * num_experts + e];
   const int padded = live ? (count + block_size - 1) / block_size * block_size : 0;
   const int tiles = tl.bm > 0 ? (count + tl.bm - 1) / tl.bm : 0;
-  // inclusive scan of the padded counts and the tile counts (nine doubling steps), then exclusive
-  s_scan[0][0][e] = padded;
-  s_scan[0][1][e] = tiles;
+  // inclusive scans of the padded counts and the tile counts, then exclusive
+  int base = wave_scan(padded), first = wave_scan(tiles);
+  if ((e & 63) == 63) s_tot[0][wave] = base, s_tot[1][wave] = first;
   __syncthreads();
-  int cur = 0;
-  for (int d = 1; d < kAlignMaxExperts; d <<= 1) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a) s_scan[cur ^ 1][a][e] = s_scan[cur][a][e] + (e >= d ? s_scan[cur][a][e - d] : 0);
-    cur ^= 1;
-    __syncthreads();
-  }
-  const int base = s_scan[cur][0][e] - padded;
+  for (int w = 0; w < wave; ++w) base += s_tot[0][w], first += s_tot[1][w];
   if (e == kAlignMaxExperts - 1) {
-    *num_tokens_post_pad = s_scan[cur][0][e];
-    if (tl.bm > 0) tl.list[0] = min(s_scan[cur][1][e], tl.capacity);
+    *num_tokens_post_pad = base;
+    if (tl.bm > 0) tl.list[0] = min(first, tl.capacity);
   }
+  base -= padded;
   if (!live) return;
-  if (tl.bm > 0) write_tile_entries(e, count, base, s_scan[cur][1][e] - tiles, tl.bm, tl.capacity, tl.list);
+  if (tl.bm > 0) write_tile_entries(e, count, base, first - tiles, tl.bm, tl.capacity, tl.list);
   expert_counts[e] = count;
   int run = base;
 #pragma unroll
@@ -546,6 +550,7 @@ __global__ void __launch_bounds__(512) k_align_offsets(const int* __restrict__ v
 __global__ void __launch_bounds__(256) k_align_place(const int* __restrict__ topk_ids, const int* __restrict__ valid_tokens,
                                                       int top_k, int num_experts, int sorted_capacity,
                                                       const int* __restrict__ chunk_first, int* __restrict__ sorted_token_ids) {
+  __builtin_amdgcn_s_setprio(3);
   __shared__ int cnt[4][kAlignMaxExperts];  // next slot of expert e for wavefront w
   const int numel = *valid_tokens * top_k;
   const int i0 = blockIdx.x * kAlignChunk;
@@ -578,17 +583,11 @@ __global__ void __launch_bounds__(256) k_align_place(const int* __restrict__ top
   // rounds of ballots and LDS updates per 64 ids: 23 us at 8192 tokens); the lowest lane of each group then moves the
   // expert's next slot on.
   int* mine = cnt[wave];
-  int id_bits = 1;
-  while ((1 << id_bits) < num_experts) ++id_bits;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int i = i0 + wave * 256 + r * 64 + lane;
     const int v = id[r];
-    unsigned long long same = __ballot(v >= 0);
-    for (int bit = 0; bit < id_bits; ++bit) {
-      const unsigned long long set = __ballot((v >> bit) & 1);
-      same &= ((v >> bit) & 1) ? set : ~set;
-    }
+    const unsigned long long same = lanes_alike(v, v >= 0);
     int pos = -1;
     if (v >= 0) {
       const int first = mine[v];

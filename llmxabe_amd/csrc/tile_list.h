@@ -14,10 +14,7 @@ __device__ __forceinline__ void write_tile_entries(int e, int count, int base, i
     const int idx = first + i;
     if (idx >= capacity) break;
     const int lo = blocks * i / nt * 32, hi = min(blocks * (i + 1) / nt * 32, count);
-    list[4 + 4 * idx + 0] = e;
-    list[4 + 4 * idx + 1] = base + lo;
-    list[4 + 4 * idx + 2] = hi - lo;
-    list[4 + 4 * idx + 3] = 0;
+    *reinterpret_cast<int4*>(list + 4 + 4 * idx) = make_int4(e, base + lo, hi - lo, 0);
   }
 }
 
