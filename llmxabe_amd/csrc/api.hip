@@ -287,7 +287,7 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
                      prop.gcnArchName);
   // a code object that does not load shows up here rather than at the first launch
   hipFuncAttributes attr;
-  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows));
+  hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(&k_rms_norm_rows<false>));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return set_error(XABE_ERR_COMPILE, "kernel load failed: %s", hipGetErrorString(e));
@@ -990,8 +990,12 @@ int xabe_rms_norm(void* stream, const float* x, size_t x_len, const float* weigh
   if (width <= 2048 && rows >= 64)  // (a handful of rows: one workgroup per row finishes sooner)
     hipLaunchKernelGGL(k_rms_norm_short_rows<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream), x, weight, out,
                        static_cast<_Float16*>(nullptr), (int)rows, (int)width, eps);
+  else if (width > 2048 && width <= 2048 * kLongRowChunks && rows >= kLongRowsMin)
+    hipLaunchKernelGGL(k_rms_norm_long_rows<false>, dim3((unsigned)rows), dim3(64), 0, as_stream(stream), x, weight, out,
+                       static_cast<_Float16*>(nullptr), (int)width, eps);
   else
-    hipLaunchKernelGGL(k_rms_norm_rows, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out, (int)width, eps);
+    hipLaunchKernelGGL(k_rms_norm_rows<false>, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out,
+                       static_cast<_Float16*>(nullptr), (int)width, eps);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
@@ -999,12 +1003,19 @@ int xabe_rms_norm(void* stream, const float* x, size_t x_len, const float* weigh
 int xabe::rms_norm_rows_with_f16(void* stream, const float* x, const float* weight, float* out, void* out_h, size_t rows,
                                  size_t width, float eps, bool* done) {
   *done = false;
-  if (!out_h || width > 2048 || width % 4 != 0 || rows < 64) return XABE_OK;
+  if (!x || !weight || !out || !out_h || width % 4 != 0 || rows < 64) return XABE_OK;
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out) |
        reinterpret_cast<uintptr_t>(out_h)) % 16 != 0)
     return XABE_OK;
-  hipLaunchKernelGGL(k_rms_norm_short_rows<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream), x, weight, out,
-                     static_cast<_Float16*>(out_h), (int)rows, (int)width, eps);
+  if (width <= 2048)
+    hipLaunchKernelGGL(k_rms_norm_short_rows<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, as_stream(stream), x, weight, out,
+                       static_cast<_Float16*>(out_h), (int)rows, (int)width, eps);
+  else if (width <= 2048 * kLongRowChunks && rows >= kLongRowsMin)
+    hipLaunchKernelGGL(k_rms_norm_long_rows<true>, dim3((unsigned)rows), dim3(64), 0, as_stream(stream), x, weight, out,
+                       static_cast<_Float16*>(out_h), (int)width, eps);
+  else
+    hipLaunchKernelGGL(k_rms_norm_rows<true>, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x, weight, out,
+                       static_cast<_Float16*>(out_h), (int)width, eps);
   XABE_HIP_TRY(hipGetLastError());
   *done = true;
   return XABE_OK;

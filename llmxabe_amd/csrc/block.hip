@@ -358,14 +358,23 @@ int xabe_dense_ffn_block_forward(xabe_dense_ffn_block* blk, void* stream, const 
                               residual, blk->normed, ffn_out, l_out, &launched));
     if (launched) return XABE_OK;
   }
-  XABE_TRY(xabe_rms_norm(stream, residual, blk->n_act, w->post_norm, g.hidden, blk->normed, blk->n_act, g.max_tokens,
-                         g.hidden, blk->eps));
+  bool with_h = false;  // the norm has written the fp16 copy of its rows, too
   if (wide)
-    XABE_TRY(xabe_moe_shared_expert_mma(blk->moe, stream, blk->buffers, w->gate, w->up, w->down, blk->normed, blk->n_act,
-                                        ffn_out, blk->n_act));
-  else
+    XABE_TRY(rms_norm_rows_with_f16(stream, residual, w->post_norm, blk->normed, blk->buffers->x_h, g.max_tokens, g.hidden,
+                                    blk->eps, &with_h));
+  if (!with_h)
+    XABE_TRY(xabe_rms_norm(stream, residual, blk->n_act, w->post_norm, g.hidden, blk->normed, blk->n_act, g.max_tokens,
+                           g.hidden, blk->eps));
+  if (wide) {
+    blk->buffers->x_h_ready = with_h;
+    const int st = xabe_moe_shared_expert_mma(blk->moe, stream, blk->buffers, w->gate, w->up, w->down, blk->normed, blk->n_act,
+                                              ffn_out, blk->n_act);
+    blk->buffers->x_h_ready = false;
+    XABE_TRY(st);
+  } else {
     XABE_TRY(xabe_moe_shared_expert(blk->moe, stream, blk->buffers, w->gate, w->up, w->down, blk->normed, blk->n_act,
                                     ffn_out, blk->n_act));
+  }
   return xabe_dense_ffn_add_residual(blk->moe, stream, blk->buffers, ffn_out, residual, l_out);
 }
 

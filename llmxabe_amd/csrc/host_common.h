@@ -117,8 +117,8 @@ int router_logits_biased(const xabe_moe_kernels* k, void* stream, const xabe_moe
                          size_t logits_len, const float* bias, bool* bias_added, bool* sum_deferred = nullptr);
 int route_planes_and_dispatch(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, float* logits, size_t logits_len,
                               const float* bias);
-// RMSNorm of `rows` rows that also writes the fp16 copy the matrix-core kernels read (rows of at most 2048
-// elements, at least 64 of them); returns false in *done when the shape is not served.
+// RMSNorm of `rows` rows that also writes the fp16 copy the matrix-core kernels read (at least 64
+// rows); returns false in *done when the shape is not served.
 int rms_norm_rows_with_f16(void* stream, const float* x, const float* weight, float* out, void* out_h, size_t rows,
                            size_t width, float eps, bool* done);
 // one-time, at handle creation: LDS limits of the kernels that ask for more than the static 64 KB (mfma.hip)

@@ -25,8 +25,10 @@ __device__ __forceinline__ float block_sum_256(float v, float* scratch) {
 // rms_norm_rows (crates/xabe-cuda/src/kernels/layer_ops.rs:129-151): every row of the
 // buffer, y = x * (1/sqrtf(mean(x^2) + eps)) * w.  grid = rows, 256 threads.
 // ---------------------------------------------------------------------------------
+// WITH_H: the row also goes out as fp16 (see k_rms_norm_short_rows).
+template <bool WITH_H>
 __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__ x, const float* __restrict__ w,
-                                                        float* __restrict__ out, int width, float eps) {
+                                                        float* __restrict__ out, _Float16* __restrict__ out_h, int width, float eps) {
   const float* xr = x + (size_t)blockIdx.x * width;
   float* o = out + (size_t)blockIdx.x * width;
   // width is a multiple of 4; up to eight float4 columns per thread (rows up to 8192 wide) are requested
@@ -45,16 +47,22 @@ __global__ void __launch_bounds__(256) k_rms_norm_rows(const float* __restrict__
     }
   }
   const float inv = row_inv_rms(xr, width, eps);  // each wavefront computes the same scale
+  [[maybe_unused]] uint2* h4 = reinterpret_cast<uint2*>(out_h + (WITH_H ? (size_t)blockIdx.x * width : 0));
+  auto put = [&](int j, const float4& a, const float4& b) __attribute__((always_inline)) {
+    const float4 y = make_float4(a.x * inv * b.x, a.y * inv * b.y, a.z * inv * b.z, a.w * inv * b.w);
+    o4[j] = y;
+    if constexpr (WITH_H) {
+      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+      const h2 lo = {(_Float16)y.x, (_Float16)y.y}, hi = {(_Float16)y.z, (_Float16)y.w};
+      h4[j] = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+    }
+  };
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int j = threadIdx.x + 256 * i;
-    if (j < n4)
-      o4[j] = make_float4(xv[i].x * inv * wv[i].x, xv[i].y * inv * wv[i].y, xv[i].z * inv * wv[i].z, xv[i].w * inv * wv[i].w);
+    if (j < n4) put(j, xv[i], wv[i]);
   }
-  for (int j = threadIdx.x + 2048; j < n4; j += 256) {
-    const float4 a = x4[j], b = w4[j];
-    o4[j] = make_float4(a.x * inv * b.x, a.y * inv * b.y, a.z * inv * b.z, a.w * inv * b.w);
-  }
+  for (int j = threadIdx.x + 2048; j < n4; j += 256) put(j, x4[j], w4[j]);
 }
 
 // The same with the row's digits and superblock scales (digits.h), which the fp32 row contractions read.  grid = (rows, a
@@ -148,6 +156,64 @@ __global__ void __launch_bounds__(256) k_rms_norm_short_rows(const float* __rest
       }
     }
   }
+}
+
+// Rows of 2048 to 6144 elements, many of them: one wavefront per row, which keeps the row's pieces in registers as they
+// come from memory and folds it chunk by chunk through LDS (the transposition of k_rms_norm_short_rows); a workgroup per row
+// (k_rms_norm_rows) reads every row five times, each of its wavefronts for a scale of its own.  Bound by memory: 2048 rows of
+// 5120 with the fp16 copy 26 us, where that kernel and a conversion of its own took 38 and 11.
+constexpr int kLongRowChunks = 3;
+constexpr size_t kLongRowsMin = 1536;  // (1000 rows: no faster, one wavefront per SIMD)
+template <bool WITH_H>
+__global__ void __launch_bounds__(64) k_rms_norm_long_rows(const float* __restrict__ x, const float* __restrict__ w,
+                                                            float* __restrict__ out, _Float16* __restrict__ out_h, int width, float eps) {
+  __shared__ float4 s_chunk[512 + 64];
+  const int lane = (int)__lane_id(), n4 = width / 4;
+  const float4* x4 = reinterpret_cast<const float4*>(x + (size_t)blockIdx.x * width);
+  const float4* w4 = reinterpret_cast<const float4*>(w);
+  auto slot = [](int q) { return q + (q >> 3); };
+  float4 v[kLongRowChunks][8];
+#pragma unroll
+  for (int c = 0; c < kLongRowChunks; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int q = 512 * c + 64 * j + lane;
+      v[c][j] = q < n4 ? x4[q] : make_float4(0.f, 0.f, 0.f, 0.f);  // (zeros past the end: fma(0, 0, s) == s)
+    }
+  float sum = 0.0f;
+#pragma unroll
+  for (int c = 0; c < kLongRowChunks; ++c) {
+    RmsRaw r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s_chunk[slot(64 * j + lane)] = v[c][j];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r.q[i] = s_chunk[slot(8 * lane + i)];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // every lane has read its pieces before the next chunk's overwrite them
+    sum = rms_fold(r, sum);
+  }
+  const float inv = rms_finish(sum, width, eps);
+  float4* o4 = reinterpret_cast<float4*>(out + (size_t)blockIdx.x * width);
+  [[maybe_unused]] uint2* h4 = reinterpret_cast<uint2*>(out_h + (WITH_H ? (size_t)blockIdx.x * width : 0));
+#pragma unroll
+  for (int c = 0; c < kLongRowChunks; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int q = 512 * c + 64 * j + lane;
+      if (q < n4) {
+        const float4 a = v[c][j], b = w4[q];
+        const float4 y = make_float4(a.x * inv * b.x, a.y * inv * b.y, a.z * inv * b.z, a.w * inv * b.w);
+        o4[q] = y;
+        if constexpr (WITH_H) {
+          typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+          const h2 lo = {(_Float16)y.x, (_Float16)y.y}, hi = {(_Float16)y.z, (_Float16)y.w};
+          h4[q] = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+        }
+      }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_route(const float* __restrict__ logits, const int* __restrict__ valid_tokens,
