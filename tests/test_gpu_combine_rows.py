@@ -24,9 +24,11 @@ def test_combine(X, hidden, top_k, tokens):
     k = X.MoeKernels(X.MoeGeometry(16, top_k, hidden, 256, 32, tokens))
     b = k.buffers()
     k.set_valid_tokens(b, live)
-    n = tokens * hidden
+    n, count = tokens * hidden, 16 * hidden * 256
+    stacks = [X.QuantTensor(X.synth_quant(X.ExpertQuant.Q8_0, s, count, 0.05), X.ExpertQuant.Q8_0) for s in (6, 7, 8)]
+    k.route_and_dispatch(b, X.synth_normal_f32(9, tokens * 16, 1.0))
+    k.grouped_forward_partial(b, *stacks, X.synth_normal_f32(10, n, 1.0).view(tokens, hidden))
     part = b.partial()[:tokens * top_k * hidden]
-    part.copy_(X.synth_normal_f32(1, part.numel(), 1.0))
     w = X.synth_normal_f32(2, hidden, 0.05)
     normed, shexp, residual = (X.synth_normal_f32(s, n, 1.0).view(tokens, hidden) for s in (3, 4, 5))
     gate = torch.zeros(tokens, device="cuda")
@@ -35,6 +37,7 @@ def test_combine(X, hidden, top_k, tokens):
     torch.cuda.synchronize()
     p = part.view(tokens, top_k, hidden).double()[:live]
     half = 2.0 ** -24
+    assert bool(p.any())
     r, mag = p.sum(1), p.abs().sum(1)
     assert bool(((routed[:live].double() - r).abs() <= top_k * half * mag).all())
     z = normed[:live].double() @ w.double()
