@@ -1114,7 +1114,7 @@ __global__ void __launch_bounds__(64 * (kMaxTopK + SHARED), SHARED ? 3 : 4) k_de
 }
 
 // ------------------------------------------------------------------ host side
-// Tiles per workgroup of the second and third launch: the largest power of two up to kMaxShare that divides the tiles and
+// Tiles per workgroup of the second launch: the largest power of two up to kMaxShare that divides the tiles and
 // leaves 192 workgroups.  Same box, us per block, tiles of (second, third) launch: one token (1, 1) 24.1, (2, 1) 24.3,
 // (1, 2) 25.6; three (1, 1) 37.4, (2, 2) 31.8, (4, 2) 31.4, (4, 4) 34.5; thirteen (1, 1) 91.1, (2, 2) 80.9, (4, 4) 79.9;
 // thirty-two (1, 1) 172, (2, 2) 146, (4, 4) 132.
@@ -1122,6 +1122,22 @@ static int decode_share(size_t units, int tiles) {
   int share = 1;
   while (share < kMaxShare && tiles % (2 * share) == 0 && units * tiles >= (size_t)384 * share) share *= 2;
   return share;
+}
+
+// Tiles per workgroup of the third launch: the number whose workgroups, dealt in rounds to the CUs, end first, a workgroup's
+// time being that of its tiles and half a tile more; the larger of two alike.  Blocks (of four in one graph, us), two / four
+// tiles: four tokens 132 / 144, five 181 / 171, seven 202 / 192, eight 212 / 210, nine 233 / 242, twelve 264 / 267, fourteen
+// 291 / 286, thirty-two 509 / 498; one / two: two tokens 102 / 108, three 128 / 119.  Past three rounds of the largest the
+// workgroups no longer end together and it is the best (twenty-seven tokens 458 / 448).
+static int down_share(const xabe_moe_kernels* k, size_t tokens, int tiles) {
+  if (tiles % kMaxShare == 0 && tokens * (size_t)(tiles / kMaxShare) > 3 * (size_t)k->num_cus) return kMaxShare;
+  int best = 1;
+  size_t best_cost = ~(size_t)0;
+  for (int share = 1; share <= kMaxShare && tiles % share == 0; share *= 2) {
+    const size_t rounds = (tokens * (size_t)(tiles / share) + k->num_cus - 1) / k->num_cus, cost = rounds * (2 * share + 1);
+    if (cost <= best_cost) best_cost = cost, best = share;
+  }
+  return best;
 }
 
 struct Launch {
@@ -1334,7 +1350,7 @@ int launch_decode_block(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffe
   if (a.E % rps_h != 0)
     return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "decode block: %d experts do not fill whole steps of %d rows", a.E, rps_h);
   a.share_g = decode_share((size_t)a.max_tokens * a.top_k, a.tiles_g);
-  a.share_d = decode_share((size_t)a.max_tokens, a.tiles_d);
+  a.share_d = down_share(k, (size_t)a.max_tokens, a.tiles_d);
   const int chunks = (a.max_tokens + 1) / 2;
   const bool pre_routed = a.max_tokens >= kPreRouteMinTokens;
   const bool pair_units = a.max_tokens >= kPairUnitsMinTokens && rq == XABE_QUANT_Q6K;

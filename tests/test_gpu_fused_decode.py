@@ -198,3 +198,10 @@ def test_units_of_two_pairs(oracle, X, max_tokens, experts, top_k, small):
         f1, l1 = run_block(one, layer, x, tokens, logit_bias=lb)
         f2, l2 = run_block(many, layer, x, tokens, logit_bias=lb)
         _same_bits(_observe(one, g, f1, l1, tokens), _observe(many, g, f2, l2, tokens), f"call {i} tokens {tokens}")
+
+
+@pytest.mark.parametrize("max_tokens", [5, 6, 12, 25])
+def test_tiles_per_workgroup_of_the_down_launch(oracle, X, max_tokens):
+    # one, two and four tiles per workgroup, by how the workgroups fill the compute units
+    for g in (X.MoeGeometry.qwen3_6(X.moe_block_size(max_tokens), max_tokens), X.MoeGeometry(16, 8, 512, 256, 32, max_tokens)):
+        _compare(X, oracle, g, (max_tokens, max_tokens - 1), seed=5200 + max_tokens)
