@@ -23,7 +23,7 @@
 // The routed contractions are pair_dot's (digits.h), as are k_digit_pairs', and sb_dot's in k_digit_rows bit for bit; routing, norm, router
 // and shared expert are the per-row device functions of the multi-launch path.  So the outputs are bit-identical to that
 // path: the batch-invariance contract.  One multiply-add and one conversion per weight on the vector ALU, which this
-// replaces, made B 95 and C 52 us at 32 tokens; the digit form takes 77 and 42 (us per block, same box: 13 tokens
+// replaces, made B 95 and C 52 us at 32 tokens; the digit form took 77 and 42 when it went in, 70 and 39 now (us per block, then, same box: 13 tokens
 // 96 -> 85, 32: 162 -> 138; 45 tokens, then ten launches, 252 -> 178; three tokens 31.6 -> 32.1; one token 21.2 -> 21.0,
 // with its rows straight into registers; four digits instead of six, which lose bits beside outliers, took 71 and 39).  What bounds B and C now at 32 tokens: ~330 vector
 // instructions per (token, row tile, pair of superblocks), about half of the launch, and one expert read once per

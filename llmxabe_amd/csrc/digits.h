@@ -207,7 +207,6 @@ struct SbRaw<kQ6K> {
   static constexpr int kPieces = 15;  // 16-byte pieces of a row's window: 210 bytes from the word boundary below, and one
                                       // more that spreads the rows of a tile over the LDS banks
   static constexpr uint32_t kStart = 3;  // windows start on words (so that they lie on 16 bytes in LDS, see sb_read_slot)
-  static constexpr int kWhole16 = kBytes / 16 * 16;  // a window's bytes in whole pieces
 };
 template <>
 struct SbRaw<kQ8_0> {
