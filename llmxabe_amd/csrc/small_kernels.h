@@ -766,7 +766,11 @@ __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ 
   for (int i = 0; i < 2; ++i) {
     const int q = min((int)threadIdx.x + 256 * i, n4 - 1);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) pv[i][k] = p4[(size_t)min(k, top_k - 1) * n4 + q];
+    for (int k = 0; k < 8; ++k) {
+      typedef float f4 __attribute__((ext_vector_type(4)));
+      const f4 t4 = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p4 + (size_t)min(k, top_k - 1) * n4 + q));
+      pv[i][k] = make_float4(t4.x, t4.y, t4.z, t4.w);
+    }
     sh[i] = reinterpret_cast<const float4*>(shexp + base)[q];
     rs[i] = reinterpret_cast<const float4*>(residual + base)[q];
     if constexpr (NORM) nw[i] = reinterpret_cast<const float4*>(next_w)[q];
