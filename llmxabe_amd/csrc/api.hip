@@ -1123,7 +1123,7 @@ int xabe_dense_ffn_add_residual(const xabe_moe_kernels* k, void* stream, const x
   if (!k || !b || !ffn_out || !residual || !l_out)
     return set_error(XABE_ERR_INVALID_ARGUMENT, "dense_ffn_add_residual: null pointer");
   const xabe_moe_geometry& g = k->g;
-  dim3 grid((unsigned)g.max_tokens, (unsigned)((g.hidden + 255) / 256));
+  dim3 grid((unsigned)g.max_tokens, (unsigned)((g.hidden + 1023) / 1024));
   hipLaunchKernelGGL(k_add_residual, grid, dim3(256), 0, as_stream(stream), ffn_out, residual, b->valid_tokens,
                      (int)g.hidden, l_out);
   XABE_HIP_TRY(hipGetLastError());

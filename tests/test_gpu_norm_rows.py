@@ -49,3 +49,21 @@ def test_the_dense_block_is_its_steps(X, hidden, tokens):
     torch.cuda.synchronize()
     assert torch.equal(ffn.view(torch.int32), want.view(torch.int32))
     assert torch.equal(l_out, want + x)
+
+
+@pytest.mark.parametrize("hidden", [128, 1152, 5120])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_the_residual_is_added_wherever_rows_start(X, hidden, off):
+    import torch
+
+    tokens, live = 5, 4
+    k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, 256, 32, tokens))
+    b = k.shared_only_buffers(False)
+    k.set_valid_tokens(b, live)
+    n = tokens * hidden
+    ffn, res, out = (X.synth_normal_f32(s, n + 4, 1.0)[off * (s == 2) + 2 * (s == 3) * (off > 0):][:n] for s in (1, 2, 3))
+    before = out.clone()
+    k.dense_ffn_add_residual(b, ffn, res, out)
+    torch.cuda.synchronize()
+    m = live * hidden
+    assert torch.equal(out[:m], ffn[:m] + res[:m]) and torch.equal(out[m:], before[m:])
