@@ -524,7 +524,11 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 //  - tall tiles: a weight is made into a half once per 192 rows.  Eight wavefronts of 192 x 32 accumulators fill the
 //    registers of a CU's SIMDs; 256 rows measured the same on the dense pass (753 us) and behind on the routed (377
 //    against 357 us at 8192 tokens), 128 rows on four wavefronts and two workgroups per CU 652 us;
-//  - requests made long before their use and waited for by count, never by draining ("all but the newest n", Requests);
+//  - requests made long before their use and waited for by count, never by draining ("all but the newest n", Requests).  A
+//    spilled vector register would undo that (its reload waits for everything requested before it): there is none
+//    (tests/test_spilled_registers.py).  With up to seven in nine of the sixteen forms the routed down launch drained
+//    its queue once per item, right behind the item's stores.  Scalar registers are kept in lanes of vector ones where there
+//    are too many (up to 119): no memory operation, but lane reads in the loop over the superblocks;
 //  - the two wavefronts of a SIMD make their requests and read raw weights at different times (`early`): behind a barrier
 //    both would leave the matrix pipe idle together;
 //  - LDS reads on their own width's boundary (any other takes 64 cycles), rows spread over the banks by the windows' odd
@@ -764,6 +768,14 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   const int stride = by_xcd ? (int)(gridDim.x >> 3) : (int)gridDim.x;
   if (first >= hi) return;
 
+  // The lane's number for what an item does once: its arithmetic belongs there and not in registers all along, which would
+  // be spilled, and what reloads a spilled register waits for every request in flight.
+  auto item_lane = [&]() __attribute__((always_inline)) {
+    int lane = (int)__lane_id();
+    asm volatile("" : "+v"(lane));
+    return lane;
+  };
+
   struct Item { int e, m0, rows, nt; };
   auto decode = [&](int item) __attribute__((always_inline)) {
     const int mt = item / n_ntiles;
@@ -797,8 +809,12 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
     const size_t off1 = NM == 2 ? off0 : off0 + (size_t)16 * row_bytes;
     w_base0 = a.w0 + off0;
     w_base1 = (NM == 2 ? a.w1 : a.w0) + off1;
-    w_last0 = (uint32_t)min(a.w_bytes - 16 - off0, (size_t)0x7fffffff);
-    w_last1 = (uint32_t)min(a.w_bytes - 16 - off1, (size_t)0x7fffffff);
+    auto to_last = [&](size_t off) __attribute__((always_inline)) {  // (a run's own pieces lie far below 2^31)
+      const size_t n = a.w_bytes - 16 - off;
+      return (n >> 31) != 0 ? 0x7fffffffu : (uint32_t)n;  // (scalar: a 64-bit minimum would hold vector registers)
+    };
+    w_last0 = to_last(off0);
+    w_last1 = to_last(off1);
   };
   uint32_t w_at = 0;  // the requested window's start in its rows
   auto request_w = [&](auto i_c) __attribute__((always_inline)) {  // instruction i of either run
@@ -842,8 +858,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   uint32_t a_off[kPI], a_lanes[kPI];  // the lane's piece of either instruction; which instructions are for live rows
   auto set_a = [&](const Item& it, int tb) __attribute__((always_inline)) {
     const int pieces = (it.rows + 31) / 32 * 4;
-    int lane = (int)__lane_id();
-    asm volatile("" : "+v"(lane));  // (its arithmetic belongs here, once per item, and not in registers all along)
+    const int lane = item_lane();
 #pragma unroll
     for (int i = 0; i < kPI; ++i) {
       const int row = 8 * (wave + WAVES * i) + (lane >> 3), live = min(row, it.rows - 1);
@@ -862,10 +877,12 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
       lds_dma_16_lanes(a.a, a_off[i] + (uint32_t)a_ks * (kSK * 2u), lds_a + a_to + 1024u * WAVES * i, a_lanes[i], a_lanes[i]);
   };
   auto request_ids = [&](const Item& it, int tb) __attribute__((always_inline)) {
+    const int lane = item_lane();
     if (64 * wave < kTM)
       lds_dma_4(a.sorted_token_ids, (uint32_t)(it.m0 + min(64 * wave + lane, it.rows - 1)) * 4u, lds_address(sId + tb * kTM + 64 * wave));
   };
   auto request_scales = [&]() __attribute__((always_inline)) {
+    const int lane = item_lane();
     if (64 * wave < kTM) lds_dma_4(a.topk_weights, (uint32_t)sId[64 * wave + lane] * 4u, lds_address(sScale + 64 * wave));
   };
   auto all_landed = [&]() __attribute__((always_inline)) {
@@ -882,7 +899,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
 
   Item cur = decode(first), nxt = cur;
   int tb = 0;              // which of the two tables is this item's
-  WHalf<QUANT> raw[2];     // the raw weights of a superblock's halves, as far as they are at work
+  WHalf<QUANT> raw[QUANT == kQ6K ? 2 : 1];  // the raw weights that an item starts on: a superblock's halves, or its first
   uint32_t ring = 0;       // this step's place in the ring
   auto ring_after = [&](uint32_t r) __attribute__((always_inline)) { return r + kSlot == kRing * kSlot ? 0u : r + kSlot; };
   int w_win = 1;           // the weight stream's next window
@@ -947,6 +964,16 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
 #pragma unroll 1
       for (int sb = 0; sb < nsb; ++sb) {
         WHalf<QUANT> next[2];
+        // (Q8_0: the second half, read where it is needed.  It lives in here: outside, its last value would be held all round
+        // the loop, since either of two places may write it)
+        [[maybe_unused]] WHalf<QUANT> second;
+        auto half_of = [&](auto c_c) __attribute__((always_inline)) -> const WHalf<QUANT>& {  // what chunk c's weights come from
+          constexpr int c = decltype(c_c)::value;
+          if constexpr (c == 0) return next[0];
+          else if constexpr (c < 8) return raw[0];
+          else if constexpr (QUANT == kQ6K) return raw[1];
+          else return second;
+        };
         auto chunk = [&](auto c_c) __attribute__((always_inline)) {
           constexpr int C = decltype(c_c)::value, C1 = (C + 1) & 15;
           using Req = Requests<QUANT, kPI>;
@@ -964,7 +991,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
           } else if constexpr ((C & 7) == 5 || (C & 7) == 6) {
             if (early == ((C & 7) == 5)) {
               wait_vm<Req::after_w(C)>();
-              read_w(C < 8 ? 1 : 0, 0, C < 8 ? raw[1] : next[0]);
+              read_w(C < 8 ? 1 : 0, 0, C < 8 ? second : next[0]);
             }
           }
           if constexpr ((C & 3) == 3) {
@@ -1006,7 +1033,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
           constexpr bool kRequests = Req::a_at(C) != 0 || Req::w_at(C) != 0;
           if (kRequests && early) requests();
           order_fence();
-          const WHalf<QUANT>& r1 = C1 == 0 ? next[0] : raw[C1 >> 3];
+          const WHalf<QUANT>& r1 = half_of(std::integral_constant<int, C1>{});
           const uint8_t* pa = sA + ((frag ^ (64u * ((C1 >> 1) & 1) + 16u * (C1 & 1))) + ring);
 #pragma unroll
           for (int i = 0; i < NB; ++i) {
@@ -1047,8 +1074,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
       }
 
       // epilogue.  acc[i][v]: tile row 32 i + (v / 4) * 8 + h * 4 + v % 4, column lane % 32 of the wavefront
-      int lane = (int)__lane_id();
-      asm volatile("" : "+v"(lane));
+      const int lane = item_lane();
       const int h = lane >> 5, col = lane & 31;
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
