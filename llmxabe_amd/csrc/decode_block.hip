@@ -515,12 +515,12 @@ template <int SQ, int RPS>
 __device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) {
   using RawS = typename Fmt<SQ>::Raw;
   constexpr int G = 64 / RPS;
-  const int lane = (int)__lane_id();
+  const int lane = fresh_lane();
   const int units_per_chunk = a.H / (4 * RPS);
   const int t0 = 2 * (unit / units_per_chunk), row0 = (unit % units_per_chunk) * 4 * RPS;
   const int t1 = min(t0 + 1, a.max_tokens - 1);
   const int valid = *a.valid_tokens;
-  const LaneGeom g = lane_geom<SQ>();
+  const LaneGeom g = lane_geom<SQ>(lane);
   const int koff = lane_koff<SQ, RPS>(g, 0);
   const size_t row_bytes = (size_t)(a.I / Fmt<SQ>::kBlockElems) * Fmt<SQ>::kBlockBytes;
   float x[2][32], xs[2][4];
@@ -528,13 +528,16 @@ __device__ __forceinline__ void shared_down_rows(const DecodeArgs& a, int unit) 
   lane_x_load<SQ>(a.shared_inter + (size_t)t1 * a.I, koff, g, x[1]);
   lane_x_offsets<SQ>(x[0], xs[0]);
   lane_x_offsets<SQ>(x[1], xs[1]);
+  // steps in flight: more do not fit the registers of two workgroups per CU (Q6_K with two spilled ten to fifteen: four
+  // blocks of 13 / 32 / 45 / 63 tokens 283 / 523 / 642 / 766 us, with one 267 / 470 / 591 / 713)
+  constexpr int kFlight = SQ == kQ6K ? 1 : 2;
 #pragma unroll 1
-  for (int d0 = 0; d0 < 4; d0 += 2) {  // (two steps in flight: four do not fit the registers of two workgroups per CU)
-    RawS raw[2];
+  for (int d0 = 0; d0 < 4; d0 += kFlight) {
+    RawS raw[kFlight];
 #pragma unroll
-    for (int d = 0; d < 2; ++d) load_raw<SQ, true>(a.sdown + (size_t)(row0 + (d0 + d) * RPS) * row_bytes, true, g, raw[d]);
+    for (int d = 0; d < kFlight; ++d) load_raw<SQ, true>(a.sdown + (size_t)(row0 + (d0 + d) * RPS) * row_bytes, true, g, raw[d]);
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
+    for (int d = 0; d < kFlight; ++d) {
       float tot[2] = {0.0f, 0.0f};
       accum<SQ, 2>(raw[d], g, x, xs, tot);
 #pragma unroll

@@ -53,9 +53,9 @@ struct LaneGeom {
 };
 
 template <int QUANT>
-__device__ __forceinline__ LaneGeom lane_geom() {
+__device__ __forceinline__ LaneGeom lane_geom(int lane = (int)__lane_id()) {
   LaneGeom g;
-  g.lane = __lane_id();
+  g.lane = lane;
   g.slot = g.lane >> 3;
   g.half = (g.lane >> 2) & 1;
   g.l8 = g.lane & 3;

@@ -150,6 +150,15 @@ __device__ __forceinline__ void lds_dma_16(const void* base, uint32_t voff, uint
 #pragma clang diagnostic pop
 }
 
+// The lane's number, made where it is asked for (__lane_id() is the same value, but the compiler makes it, and whatever is
+// derived from it, once, outside all loops): for what a loop does rarely, in kernels that fill their registers.  Held all
+// along it would be spilled, and what reloads a spilled register waits for every request in flight.
+__device__ __forceinline__ int fresh_lane() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+  return lane;
+}
+
 // The byte address in LDS of what every lane of the wavefront has at `p`.
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);

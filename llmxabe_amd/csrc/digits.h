@@ -293,6 +293,7 @@ __device__ __forceinline__ void sb_read_words(const uint8_t* p, int h, SbRaw<kQ6
 #pragma unroll
   for (int i = 0; i < 8; ++i) r.qh[i / 4][i % 4] = __builtin_amdgcn_alignbit(qh[i + 1], qh[i], shift);
   r.sc = make_uint2(__builtin_amdgcn_alignbit(sc[1], sc[0], shift), __builtin_amdgcn_alignbit(sc[2], sc[1], shift));
+  opaque(r);
 }
 __device__ __forceinline__ void sb_read(const uint8_t* p, int h, SbRaw<kQ8_0>& r) {  // (`p` on an 8-byte boundary)
 #pragma unroll
@@ -364,8 +365,12 @@ __device__ __forceinline__ float join_sums(const int (&d)[6]) {
 }
 
 // The lane's half superblock by plain fp32 multiply-adds in the order of the groups, weights dequantised exactly: what
-// a half superblock with a mark goes through.  `x`: the 128 activations of the half, the same for the lanes of a DPP row;
-// each of its sixteen lanes loads eight of them (one trip to memory) and the others take them from there.
+// a half superblock with a mark goes through.  `x`: the superblock's activations, of which the half's 128 are taken, the same
+// for the lanes of a DPP row; each of its sixteen lanes loads eight of them (one trip to memory) and the
+// others take them from there.  `lane`: the pair forms pass fresh_lane(), whose registers are full (kept for this branch,
+// which marked superblocks alone take, the lane's offset was spilled by every wavefront of the block's down launch: 13 / 32 /
+// 45 tokens 432 / 488 / 608 us of blocks, 421 / 467 / 586 without); sb_dot, whose registers are not, passes the number it has
+// (made anew 40 tokens of the dense sibling took 431 us instead of 429).
 // (The registers go through an empty statement first and the groups are kept apart: the compiler would otherwise keep the
 // codes it unpacked for the matrix instruction for this branch, or unpack all of them at once.)
 __device__ __forceinline__ void opaque(SbRaw<kQ8_0>& r) {
@@ -391,11 +396,12 @@ __device__ __forceinline__ float half_fp32_all(const SbRaw<QUANT>& r, const floa
   return out;
 }
 template <int QUANT>
-__device__ __forceinline__ float half_fp32(SbRaw<QUANT>& r, const float* __restrict__ x) {
+__device__ __forceinline__ float half_fp32(SbRaw<QUANT>& r, const float* __restrict__ x, int half, int lane) {
   float own[8];
+  const uint8_t* const at = reinterpret_cast<const uint8_t*>(x) + (uint32_t)(half * 512 + (lane & 15) * 32);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const float4 v = reinterpret_cast<const float4*>(x)[2 * ((int)__lane_id() & 15) + i];
+    const float4 v = reinterpret_cast<const float4*>(at)[i];
     own[4 * i] = v.x, own[4 * i + 1] = v.y, own[4 * i + 2] = v.z, own[4 * i + 3] = v.w;
   }
   opaque(r);
@@ -500,7 +506,7 @@ __device__ __forceinline__ void sb_dot(SbRaw<QUANT>& r, HighOf high_of, LowOf lo
 #pragma unroll 1
     for (; marked; marked &= marked - 1) {
       const int m = __builtin_ctz(marked);
-      const float plain = half_fp32(r, x_of(m) + (TAIL && dead ? 0 : 128 * ((int)__lane_id() >> 5)));
+      const float plain = half_fp32(r, x_of(m), TAIL && dead ? 0 : (int)__lane_id() >> 5, (int)__lane_id());
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if (t == m && out[t] != out[t]) out[t] = TAIL && dead ? 0.0f : plain;
@@ -789,9 +795,8 @@ __device__ __forceinline__ float pair_dot(SbRaw<QUANT>& r, const PairDigits<WHOL
   else if constexpr (WHOLE) out *= x.e[0].x;
   if (TAIL && dead) out = 0.0f;
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(out != out) != 0, 0)) {
-    int quarter = (int)__lane_id() >> 4;
-    asm volatile("" : "+v"(quarter));  // (keeps the address out of the registers of the loop around)
-    const float plain = half_fp32(r, x_of(quarter) + (TAIL && dead ? 0 : 128 * (quarter & 1)));
+    const int lane = fresh_lane(), quarter = lane >> 4;
+    const float plain = half_fp32(r, x_of(quarter), TAIL && dead ? 0 : quarter & 1, lane);
     if (out != out) out = plain;
   }
   return out;
@@ -843,9 +848,8 @@ __device__ __forceinline__ void pair_dot_lds(SbRaw<kQ6K>& r, const uint8_t* cons
   for (int t = 0; t < NT; ++t) {
     out[t] = join_sums(sum[t]) * (sb_quarter(r) * e[t]);
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(out[t] != out[t]) != 0, 0)) {
-      int quarter = (int)__lane_id() >> 4;
-      asm volatile("" : "+v"(quarter));
-      const float plain = half_fp32(r, x_of(t, quarter) + 128 * (quarter & 1));
+      const int lane = fresh_lane(), quarter = lane >> 4;
+      const float plain = half_fp32(r, x_of(t, quarter), quarter & 1, lane);
       if (out[t] != out[t]) out[t] = plain;
     }
   }

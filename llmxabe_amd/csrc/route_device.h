@@ -145,10 +145,12 @@ __device__ __forceinline__ void route_finish(const float (&l)[PER], int num_expe
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   // sequential sum in index order on lane 0 alone (a 16-byte LDS read that all 64 lanes aim at one
   // address is serialised lane by lane), 32 values per batch so that the reads are in flight together and
-  // only the additions form the dependent chain
+  // only the additions form the dependent chain (two batches in flight take registers that the caller's operands,
+  // held beside the routing, do not leave)
   float sum = -0.0f;
   if (lane == 0) {
     const int n32 = num_experts & ~31;
+#pragma unroll 1
     for (int i = 0; i < n32; i += 32) {
       float4 v[8];
 #pragma unroll
