@@ -1069,13 +1069,22 @@ int xabe_moe_gate_and_combine(const xabe_moe_kernels* k, void* stream, const xab
     return set_error(XABE_ERR_INVALID_ARGUMENT, "gate_and_combine: null pointer");
   XABE_TRY(require_routed(b, "gate_and_combine"));
   const xabe_moe_geometry& g = k->g;
-  if (g.hidden <= 2048) {
-    // a row's loads all at once (the other form starts on `partial` when the gate is known and takes a selection at a time:
-    // 512 tokens 14.4 us against 11.3, 1237 30.0 against 22.7)
-    hipLaunchKernelGGL((k_combine_rows<false, false>), dim3((unsigned)g.max_tokens), dim3(256), 0, as_stream(stream), shared_gate_inp,
-                       normed, b->partial, shexp, residual, b->valid_tokens, (int)g.experts_per_token, (int)g.hidden, gate, routed,
-                       ffn_out, l_out, static_cast<const float*>(nullptr), 0.0f, static_cast<float*>(nullptr),
-                       static_cast<_Float16*>(nullptr));
+  // Rows of up to 2048 elements: a workgroup per row, a row's loads all at once (k_gate_and_combine starts on `partial` when the
+  // gate is known and takes a selection at a time).  us, this / k_gate_and_combine, hidden 2048: 1 token 3.3 / 3.9, 32: 4.1 / 7.2,
+  // 63: 4.4 / 7.5, 512: 12.1 / 17.2, 1237: 24 / 37, 8192: 165 / 193; hidden 512: 1 token 2.5 / 3.1, 63: 2.9 / 3.7, 1237: 8.8 / 9.0,
+  // 8192: 43 / 49.  Rows of up to 1024 elements take a 16-byte column per thread instead of two, of which one would load nothing
+  // of use (hidden 512, 1237 tokens 9.8 us, 8192: 49).  Many rows of one or two superblocks go the other way: a workgroup then
+  // has as many loads in flight for a row as for a long one, and workgroups are what such a launch is bound by (hidden
+  // 128, 1700 tokens 6.8 / 7.2, 2500: 8.4 / 8.1, 8192: 20 / 15; hidden 256: 1700 7.8 / 8.0, 4096: 14 / 12).
+  if (g.hidden <= 2048 && !(g.hidden <= 256 && g.max_tokens > 2048)) {
+#define XABE_COMBINE(COLS)                                                                                                    \
+  hipLaunchKernelGGL((k_combine_rows<false, false, COLS>), dim3((unsigned)g.max_tokens), dim3(256), 0, as_stream(stream),     \
+                     shared_gate_inp, normed, b->partial, shexp, residual, b->valid_tokens, (int)g.experts_per_token,         \
+                     (int)g.hidden, gate, routed, ffn_out, l_out, static_cast<const float*>(nullptr), 0.0f,                   \
+                     static_cast<float*>(nullptr), static_cast<_Float16*>(nullptr))
+    if (g.hidden <= 1024) XABE_COMBINE(1);
+    else XABE_COMBINE(2);
+#undef XABE_COMBINE
     XABE_HIP_TRY(hipGetLastError());
     return XABE_OK;
   }

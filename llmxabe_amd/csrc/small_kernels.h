@@ -735,7 +735,7 @@ __global__ void __launch_bounds__(256) k_gate_and_combine(const float* __restric
 // hands through LDS for that, padded like k_rms_norm_short_rows'), the normalised elements as (x * inv) * w.
 // `routed` and `ffn_out` may be null (read-back tensors a serving loop does not need: 16 bytes per element less
 // to write); NORM = false leaves the tail out.
-template <bool NORM, bool WITH_H>
+template <bool NORM, bool WITH_H, int COLS = 2>
 __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ w, const float* normed,
                                                        const float* __restrict__ partial, const float* __restrict__ shexp,
                                                        const float* __restrict__ residual, const int* __restrict__ valid_tokens,
@@ -745,6 +745,7 @@ __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ 
                                                        float* next_normed, _Float16* __restrict__ next_normed_h) {
   // (`next_normed` may be `normed` itself, a block that feeds the next pass through its own buffers: the row is read
   // in round one and written after the last barrier, by this workgroup only)
+  static_assert(COLS == 2 || !NORM, "the tail reads a whole row of slots");
   constexpr int kSlots = 512 + 64;  // padded 16-byte slots of one 2048-element row
   __shared__ float scratch[4];
   __shared__ float4 s_row[NORM ? kSlots : 1];
@@ -752,18 +753,18 @@ __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ 
   if (t >= *valid_tokens) return;
   const size_t base = (size_t)t * hidden;
   const int n4 = hidden / 4;
-  // round one: everything the row needs, requested together (two 16-byte columns per thread)
+  // round one: everything the row needs, requested together (COLS 16-byte columns per thread)
   const float4* p4 = reinterpret_cast<const float4*>(partial + (size_t)t * top_k * hidden);
-  float4 pv[2][8], sh[2], rs[2], nw[2];
-  float wv[8], xv[8];
+  float4 pv[COLS][8], sh[COLS], rs[COLS], nw[COLS];
+  float wv[4 * COLS], xv[4 * COLS];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 4 * COLS; ++i) {
     const int j = min((int)threadIdx.x + 256 * i, hidden - 1);
     wv[i] = w[j];
     xv[i] = normed[base + j];
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < COLS; ++i) {
     const int q = min((int)threadIdx.x + 256 * i, n4 - 1);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
@@ -780,14 +781,14 @@ __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ 
   // selections past the eighth (top_k > 8) are added from memory in the loop below
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 4 * COLS; ++i)
     if ((int)threadIdx.x + 256 * i < hidden) s = __builtin_fmaf(wv[i], xv[i], s);
   s = block_sum_256(s, scratch);
   const float g = 1.0f / (1.0f + expf(-s));
   if (threadIdx.x == 0) gate[t] = g;
-  float4 lo[2];
+  float4 lo[COLS];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < COLS; ++i) {
     const int q = (int)threadIdx.x + 256 * i;
     lo[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (q < n4) {
@@ -816,7 +817,7 @@ __global__ void __launch_bounds__(256) k_combine_rows(const float* __restrict__ 
     for (int i = 0; i < 8; ++i) r.q[i] = s_row[8 * lane + i + lane];  // slot(8 * lane + i)
     const float inv = rms_finish(rms_fold(r, 0.0f), hidden, next_eps);  // every wavefront: the same scale
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < COLS; ++i) {
       const int q = (int)threadIdx.x + 256 * i;
       if (q < n4) {
         const float4 v = make_float4(lo[i].x * inv * nw[i].x, lo[i].y * inv * nw[i].y, lo[i].z * inv * nw[i].z,

@@ -50,3 +50,9 @@ def test_combine(X, hidden, top_k, tokens):
     assert bool(((ffn[:live].double() - want).abs() <= bound).all())
     assert bool(((l_out[:live].double() - want - residual[:live].double()).abs() <= bound).all())
     assert not routed[live:].any() and not ffn[live:].any() and not l_out[live:].any()
+
+
+# (one 16-byte column per thread up to 1024 elements; k_gate_and_combine again for more than 2048 rows of at most 256)
+@pytest.mark.parametrize("hidden,tokens", [(256, 2048), (256, 2049), (128, 2049), (384, 2049), (1024, 66), (1024, 2)])
+def test_combine_on_both_sides_of_its_rules(X, hidden, tokens):
+    test_combine(X, hidden, 8, tokens)
