@@ -541,7 +541,7 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 // fragments follow (`frag`).  Per output element the order is fixed, whatever the tile.
 //
 // Forms: wide (six blocks of 32 rows, eight wavefronts, a workgroup per CU) and narrow (two blocks, four wavefronts, three
-// workgroups per CU: a tile's start and end are then beside other tiles' steps).  Where the line lies: routed_tile_rows,
+// workgroups per CU: a tile's start and end are then beside other tiles' steps).  Where the line lies: narrow_tiles,
 // unrouted_wide.
 constexpr int kSK = 64;                          // contraction elements per activation step
 constexpr int kNarrowRows = 64;                  // token rows of a tile, narrow form
@@ -1206,11 +1206,8 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
   return true;
 }
 
-// Token rows of a routed tile: narrow while an expert's share of the pass averages at most 48 rows, so that most experts
-// are one tile either way (1500 tokens of the routed model, 47 a share: 365 us against 388 wide; 2200, 69: 544 against
-// 454).
 static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
-  return tokens * g.experts_per_token <= 48 * g.num_experts ? kNarrowRows : kWideRows;
+  return narrow_tiles(tokens, g.experts_per_token, g.num_experts) ? kNarrowRows : kWideRows;
 }
 // The specialised form (k_mfma_pc) serves both routed launches for contractions of whole superblocks and at least
 // eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_rows everywhere; it is the faster at every width
