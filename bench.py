@@ -5,7 +5,7 @@
 
 A step is one pass of the MoE block over one batch: 3 tokens (three concurrent sequences, one token
 each), 256 experts top-8 + 1 shared, hidden 2048, expert width 512, Q6_K experts, Q8_0 router and
-shared expert -- BASELINE.json configs[1].  Successive steps run on different, independently seeded
+shared expert.  Successive steps run on different, independently seeded
 layers (--layers, default 16, 10.7 GB) so that a step's weights come from HBM and not from the
 256 MB Infinity Cache.  Inputs are resident in HBM before the timed region starts.
 
@@ -120,12 +120,12 @@ def main() -> int:
                     help="--workload prefill_*: which grouped-GEMM kernel the routed launches take (2: the "
                          "specialised-wavefront form, same bits, kept for comparison)")
     ap.add_argument("--no-configs", action="store_true",
-                    help="skip the compact legs of BASELINE's other configurations (decode batch 32, the dense sibling, the 40-layer stack)")
+                    help="skip the compact legs of the other workloads (decode batch 32, the dense sibling, the 40-layer stack)")
     ap.add_argument("--cpu-seconds", type=float, default=12.0)
     ap.add_argument("--workload", default="decode_b3", choices=["decode_b3"] + sorted(OTHER_WORKLOADS),
                     help="decode_b3 is the headline: the batch-3 decode block (value, roofline), followed by the "
                          "8192-token and the skewed 512-token prefill blocks (the `prefill` object); the others are "
-                         "BASELINE's remaining configurations one at a time, for profiles and comparison")
+                         "the remaining workloads one at a time, for profiles and comparison")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)", file=sys.stderr)
@@ -295,7 +295,7 @@ def main() -> int:
     }
     del graph, blk
 
-    # ---- the prefill half of the metric: the 8192-token chunk (MFMA-bound) and configs[2]'s 512-token chunk under a
+    # ---- the prefill half of the metric: the 8192-token chunk (MFMA-bound) and the 512-token chunk under a
     # seeded Zipf(1.1) router bias (HBM-bound), on the first layers of the same weight sets ----
     if not args.no_prefill:
         zipf = torch.from_numpy(X.zipf_logit_bias(256)).cuda()
@@ -307,8 +307,8 @@ def main() -> int:
         out["calibration"] = calibration(X, stream)
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline(layers[0], g, x, T, args.cpu_seconds)
-    # ---- BASELINE's remaining configurations, one compact leg each (the same code `--workload NAME` runs alone):
-    # configs[3] decode batch 32 as a block and through the 40-layer stack, configs[4] the dense sibling ----
+    # ---- the remaining workloads, one compact leg each (the same code `--workload NAME` runs alone):
+    # decode batch 32 as a block and through the 40-layer stack, the dense sibling ----
     if not args.no_configs:
         del layers, x, ffn_out, l_out
         torch.cuda.empty_cache()
@@ -411,7 +411,7 @@ def other_workload(args) -> int:
 
 
 def run_other(args, workload) -> dict:
-    """One of BASELINE's other configurations: the whole block, eager launches, HIP events on the launch
+    """One of the other workloads: the whole block, eager launches, HIP events on the launch
     stream over rotated layers.  One JSON line in the headline's format; the roofline is the block's own
     (algorithmic bytes or flops of a pass over its duration), not one kernel's."""
     import numpy as np

@@ -22,12 +22,11 @@
 //
 // The routed contractions are pair_dot's (digits.h), as are k_digit_pairs', and sb_dot's in k_digit_rows bit for bit; routing, norm, router
 // and shared expert are the per-row device functions of the multi-launch path.  So the outputs are bit-identical to that
-// path: the batch-invariance contract.  One multiply-add and one conversion per weight on the vector ALU, which this
-// replaces, made B 95 and C 52 us at 32 tokens; the digit form took 77 and 42 when it went in, 70 and 39 now (us per block, then, same box: 13 tokens
-// 96 -> 85, 32: 162 -> 138; 45 tokens, then ten launches, 252 -> 178; three tokens 31.6 -> 32.1; one token 21.2 -> 21.0,
-// with its rows straight into registers; four digits instead of six, which lose bits beside outliers, took 71 and 39).  What bounds B and C now at 32 tokens: ~330 vector
-// instructions per (token, row tile, pair of superblocks), about half of the launch, and one expert read once per
-// selection and XCD rather than once.
+// path: the batch-invariance contract.  One multiply-add and one conversion per weight on the vector ALU, which the digit form
+// replaced, made B 95 and C 52 us at 32 tokens; six digits instead of four (71 and 39 then) hold the bits beside outliers.
+// From 28 tokens B goes by expert, two pairs to a unit (k_decode_up_shared), which leaves C alone in going pair by pair.  At 32
+// tokens router and routing take 7 and 8 us, B 69, C 33: B fetches the distinct experts 1.09 times, C 1.15 times (at 45 tokens 1.15
+// and 1.43), vector instructions are 49 and 62 % of the cycles (45: 52 and 66).
 #include <string.h>
 
 #include <algorithm>
@@ -710,7 +709,7 @@ __global__ void __launch_bounds__(128 * NP, DIRECT ? 2 : 4) k_decode_up(DecodeAr
 // expert follow each other, so what more pairs of an expert read again comes out of the L2.  The tokens' digits lie in LDS
 // (24.6 KB: with 16 weight slots of 6.9 KB per CU that leaves room for two workgroups; in registers they would not leave any).
 // Bound by memory: at 45 tokens (360 pairs, 193 experts) 86 us, 382 MB fetched of 332 MB that are distinct; pair by pair
-// 96 us and 590 MB.  Vector instructions 49 % of the cycles.  Measured and not kept: a workgroup per unit, found by a search
+// 96 us and 590 MB.  Vector instructions 52 % of the cycles.  Measured and not kept: a workgroup per unit, found by a search
 // of its own (88 us; 63 tokens 4 % behind); three pairs with the third's digits in registers (113: spills); the shared
 // expert's rows under the first request instead of at the end (72 against 70 at 32 tokens).
 constexpr int kPairChunks = ((int)kDecodeBlockMaxTokens * kMaxTopK + 63) / 64;

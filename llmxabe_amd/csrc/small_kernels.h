@@ -420,9 +420,10 @@ struct TileListArgs {
 // scan of the padded totals), and each wavefront then ranks its selections among equals in index order, 64 at a time with
 // one ballot per bit of the id, and writes them.  No result depends on the order in which atomics land.
 // A chain of round trips: the ids are requested before the live count is known (ranges cut from the buffers' size), the
-// scan goes through the wavefronts' lanes with two barriers, rounds past the live count are skipped, and the wavefronts
-// run ahead of whatever shares the CU (the shared expert's launch beside: s_setprio; block at 512 tokens 175 -> 171 us, 1237
-// tokens 323 -> 320).  14.6 -> 10.4 us at 512 tokens.
+// scan goes through the wavefronts' lanes with two barriers, and rounds past the live count are skipped: 14.6 -> 10.4 us at
+// 512 tokens.  Its wavefronts, like those of the three launches that wider passes take, run ahead of the shared expert's
+// where the two are on one CU (s_setprio: 0.2 to 0.8 % of a block up to 1024 tokens, nothing to see from 2048 on; a workgroup
+// that finds no room on any CU waits for it all the same).
 // ---------------------------------------------------------------------------------
 constexpr int kAlignFusedMaxSelections = 8192;
 constexpr int kAlignFusedWaves = 16;

@@ -1,4 +1,4 @@
-"""Dense-sibling SwiGLU block (BASELINE configs[4]: hidden 5120, intermediate 17408, Q6_K) against the CPU
+"""Dense-sibling SwiGLU block (hidden 5120, intermediate 17408, Q6_K) against the CPU
 oracle: rms_norm -> expert_mlp -> residual add (crates/xabe-engine/src/block/dense_ffn.rs:11-28, tests/
 dense_ffn_differential.rs:110-140).  Rows are independent here (no routing), so at prefill width the oracle
 is evaluated on a sample of rows."""
@@ -115,7 +115,7 @@ CHAIN_LAYERS = 64
 
 @pytest.fixture(scope="module")
 def dense_chain():
-    """configs[4]'s chain: 64 independently seeded layers (14 GB of Q6_K), each block's l_out the next block's input."""
+    """The dense sibling's chain: 64 independently seeded layers (14 GB of Q6_K), each block's l_out the next block's input."""
     import torch
     import llmxabe_amd as X
 

@@ -12,7 +12,7 @@ from util import activations, make_layer, rel_to_peak, run_block
 
 pytestmark = pytest.mark.gpu
 
-MFMA_REL = 1e-3       # max |gpu - oracle| / max |oracle|   (north_star: max-rel <= 1e-3)
+MFMA_REL = 1e-3       # max |gpu - oracle| / max |oracle|   (the workload asks for a relative error of 1e-3 at most)
 MFMA_COS = 1 - 1e-6
 
 
@@ -97,7 +97,7 @@ PREFILL_512_CASES = {"uniform": (710, 32, None), "benched": (10000, 99, 1.0), "s
 
 @pytest.mark.parametrize("case", sorted(PREFILL_512_CASES))
 def test_block_prefill_512_matches_oracle(oracle, X, case):
-    """a 512-token chunk; the skewed cases put a seeded Zipf(1.1) bias on the router logits
+    """A 512-token chunk; the skewed cases put a seeded Zipf(1.1) bias on the router logits
     (`llmxabe_amd.zipf_logit_bias`, the definition bench.py times), so a few experts receive 50+ tokens and many
     receive none."""
     import torch
@@ -471,7 +471,7 @@ def test_router_logits_matrix_core_path(oracle, X, router_q8):
 @pytest.mark.parametrize("tokens,quant", [(8192, "q6k"), (5000, "q6k"), (3072, "q6k"), (1024, "q6k"), (8192, "q8_0"), (640, "q8_0")])
 def test_specialised_wavefronts_give_the_bits_of_the_plain_kernel(oracle, X, tokens, quant):
     """k_mfma_pc (half of a workgroup's wavefronts multiply, half dequantise; 64-element steps; 128-row x 256-weight-row
-    tiles; selected with set_mfma_form(2)) against k_mfma_expert on the same pass: every output element sees the same
+    tiles; selected with set_mfma_form(2)) against k_mfma_rows on the same pass: every output element sees the same
     fp16 operands in the same order of matrix instructions, so `partial` and the reduced rows are the same bits.
     Several widths, a ragged live count, both formats."""
     import torch

@@ -1,4 +1,4 @@
-"""a stack of MoE blocks with independent seeded weights, l_out of one block feeding
+"""A stack of MoE blocks with independent seeded weights, l_out of one block feeding
 the next.  Decode at batch 32 is checked batch-invariant (each token alone through the whole stack equals its
 row in the batch, bit for bit) and each layer is checked against the oracle on the device's own input."""
 import os
