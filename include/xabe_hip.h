@@ -313,7 +313,7 @@ int xabe_moe_block_disable_tensor_cores(xabe_moe_block* blk);            /* B:98
 int xabe_moe_block_set_exact_decode_regime(xabe_moe_block* blk, int on); /* B:1003-1005 */
 /* At max_tokens < 64 and the model shapes (hidden 2048 / intermediate 512, and the 512 / 256 test shape) the
  * block's eight steps are regrouped into three launches (logits + shared gate/up; route + gate/up; down +
- * combine) that compute the same values bit for bit.  `on` = 0 keeps one launch per step as the reference
+ * combine; from eight tokens up the routing is a fourth) that compute the same values bit for bit.  `on` = 0 keeps one launch per step as the reference
  * has them (B:1091-1329); the switch exists for tests and measurement. */
 int xabe_moe_block_set_fused_decode(xabe_moe_block* blk, int on);
 int xabe_moe_block_set_mfma_form(xabe_moe_block* blk, int form); /* xabe_moe_kernels_set_mfma_form on the block's kernels */

@@ -526,7 +526,7 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 //    against 357 us at 8192 tokens), 128 rows on four wavefronts and two workgroups per CU 652 us;
 //  - requests made long before their use and waited for by count, never by draining ("all but the newest n", Requests).  A
 //    spilled vector register would undo that (its reload waits for everything requested before it): there is none
-//    (tests/test_spilled_registers.py).  With up to seven in nine of the sixteen forms the routed down launch drained
+//    (tests/test_spilled_registers.py).  With up to seven in eight of the sixteen forms the routed down launch drained
 //    its queue once per item, right behind the item's stores.  Scalar registers are kept in lanes of vector ones where there
 //    are too many (up to 119): no memory operation, but lane reads in the loop over the superblocks;
 //  - the two wavefronts of a SIMD make their requests and read raw weights at different times (`early`): behind a barrier

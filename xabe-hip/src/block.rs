@@ -2,7 +2,7 @@
 //! (router logits, gate-and-combine: crates/xabe-engine/src/block/moe.rs:200-486); CUDA source strings do not cross
 //! to HIP, so both are library calls here, and `MoeBlock::forward` (block/moe.rs:1091-1329) calls them in place of
 //! its `launch_builder` blocks.  Better: it calls [`MoeBlockHandle::forward`], which runs the same eight steps as
-//! three launches at decode widths (62 -> 31 us per three-token block) and forks the shared expert onto a side
+//! three launches at decode widths, four from eight tokens up (45 -> 29 us per three-token block) and forks the shared expert onto a side
 //! stream at prefill widths, with the same values in `normed()`, `router_logits()`, `routed()`, `shared_ungated()`,
 //! `shared_gate()` and `buffers()` afterwards.
 use std::ffi::c_int;
