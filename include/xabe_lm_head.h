@@ -20,9 +20,9 @@
 extern "C" {
 #endif
 
-/* Tokens one pass over the weights serves in every format (L:125 has 8): a 16-bit matrix keeps the tile's activations
- * in a lane's registers, which fits four; a quantized one takes up to eight per pass, so the pass and byte counts
- * below, which use this number, are upper bounds for it. */
+/* Tokens one pass over the weights serves in every format and at every size (L:125 has 8): f16 and long bf16 rows keep the
+ * tile's activations in a lane's registers, which fits four; quantized ones take up to eight or, with hidden sizes up to
+ * 2048 and like bf16 there, sixteen per pass, so the pass and byte counts below, which use this number, are upper bounds. */
 #define XABE_LM_HEAD_MAX_BATCH_TILE 4
 /* Length of the partial-winner buffers xabe_lm_head_argmax takes (L:169). */
 #define XABE_LM_HEAD_ARGMAX_BLOCKS 512

@@ -1,9 +1,10 @@
 // LM head: logits[t][v] = sum_h W[v][h] * x[t][h] for a [vocab][hidden] matrix in Q8_0, Q6_K, bf16 or f16,
 // and the device half of greedy sampling.  Takes the place of crates/xabe-cuda/src/kernels/lm_head.rs.
 //
-// Quantized matrices go through the digit contraction (digits.h), up to eight tokens per pass over the weights; 16-bit
-// ones through the vector ALU, up to four.  Nothing depends on the batch: a token's logits are the same bits at every
-// batch width and position.
+// Three forms.  Hidden sizes up to 2048 in Q8_0 and bf16, and from five tokens on in Q6_K, take k_head_tiles_*
+// (lm_head_tiles.hip), up to sixteen tokens per pass over the weights; other quantized matrices k_lm_head_quant, on the
+// digit contraction (digits.h), up to eight; f16 and longer bf16 rows k_lm_head_half, on the vector ALU, up to four.
+// Nothing depends on the batch: a token's logits are the same bits at every batch width and position.
 #include <string.h>
 
 #include <algorithm>
@@ -14,26 +15,17 @@
 #include "decode_kernels.h"
 #include "digits.h"
 #include "host_common.h"
+#include "lm_head_tiles.h"
 
 namespace xabe {
-
-struct LmHeadArgs {
-  const uint8_t* w;
-  const float* x;   // [*][K]
-  float* out;       // [*][vocab]
-  int K, vocab;
-  int t0, nt;       // tokens [t0, t0 + nt) are served by this launch, 1 <= nt <= TOK
-  size_t w_bytes;   // quantized kernels: the tensor's length
-  int seg_sb;       // quantized kernels: superblocks whose activations LDS holds at a time
-};
 
 // Q8_0 / Q6_K rows, NT tokens.  The launch is one workgroup per CU; every wavefront owns a contiguous range of the
 // vocabulary and takes it 32 rows and one superblock at a time through its own LDS slot (SliceDma), against the tokens'
 // digits, which the workgroup makes once and keeps in LDS.  A wavefront's ranges are equal to within a row, so the last
 // round of tiles is as long for everyone: 7760 tiles of 32 rows do not divide over 2048 wavefronts, rows do.
 // Per row and token: superblock sums in order, each half of the wavefront its own, then half 0 + half 1.
-// Bound by bytes up to four tokens (Q8_0: 96 us for one, 102 for three = 5.3-5.6 TB/s, the rate a plain read loop
-// reaches), by the vector ALU beyond (eight: 120 us).  Eight wavefronts per CU: twelve and sixteen measured slower.
+// Bound by bytes up to a few tokens (the model's Q6_K matrix: 82 us for one, 93 for three), by the vector ALU beyond.  Eight
+// wavefronts per CU: twelve and sixteen measured slower.
 // SEG: rows whose digits do not fit in LDS are staged seg_sb superblocks at a time, again for every tile.
 constexpr size_t kHeadLdsMax = 160 * 1024;
 constexpr size_t kHeadQuantTokens = 8;  // tokens per pass over a quantized matrix
@@ -365,6 +357,7 @@ static int head_raise_all(std::integer_sequence<int, NT...>) {
 }
 // at handle creation, not on the launch path (launches are captured into graphs)
 static int head_configure() {
+  XABE_TRY(head_tiles_configure());
   XABE_TRY((head_raise_all<kQ8_0>(std::make_integer_sequence<int, (int)kHeadQuantTokens>())));
   return head_raise_all<kQ6K>(std::make_integer_sequence<int, (int)kHeadQuantTokens>());
 }
@@ -510,13 +503,9 @@ static void launch_half_pass(const xabe_lm_head* h, hipStream_t s, bool f16, con
   constexpr int R = TOK == 1 ? 4 : 2;
   const int groups = (a.vocab + R - 1) / R;
   const unsigned grid = (unsigned)std::max(1, std::min((groups + kWavesPerWg - 1) / kWavesPerWg, h->num_cus * 4));
-  if (f16) {
-    if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
-  } else {
-    if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
-  }
+  if (!f16) hipLaunchKernelGGL((k_lm_head_half<false, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);  // (of more than 2048 elements)
+  else if (a.K == 2048) hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 4>), dim3(grid), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((k_lm_head_half<true, R, TOK, 0>), dim3(grid), dim3(256), 0, s, a);
 }
 
 }  // namespace xabe
@@ -558,14 +547,25 @@ int xabe_lm_head_forward(const xabe_lm_head* h, void* stream, int format, const 
   a.w_bytes = weight_len;
   a.seg_sb = 0;
   const bool quant = format == XABE_HEAD_Q8_0 || format == XABE_HEAD_Q6K;
+  // (Q6_K up to four tokens: forward pass over the model's vocabulary, us, k_lm_head_quant / tiles: four 98 / 115, five
+  // 120 / 115, eight 158 / 119, sixteen 309 / 163; the same bits)
+  const bool tiles = xabe::head_tiles_width(g.hidden) &&
+                     (format == XABE_HEAD_Q8_0 || format == XABE_HEAD_BF16 || (format == XABE_HEAD_Q6K && tokens > 4));
   // passes of equal width: nine tokens as five and four, not as eight and one
-  const size_t most = !quant ? XABE_LM_HEAD_MAX_BATCH_TILE
+  const size_t most = tiles ? xabe::kHeadTileTokens
+                    : !quant ? XABE_LM_HEAD_MAX_BATCH_TILE
                     : format == XABE_HEAD_Q8_0 ? xabe::head_tokens<xabe::kQ8_0>(g.hidden) : xabe::head_tokens<xabe::kQ6K>(g.hidden);
   const size_t passes = (tokens + most - 1) / most, width = (tokens + passes - 1) / passes;
   for (size_t base = 0; base < tokens; base += width) {
     const int tile = (int)std::min<size_t>(width, tokens - base);
     a.t0 = (int)base;
     a.nt = tile;
+    if (tiles) {
+      XABE_TRY(format == XABE_HEAD_BF16 ? xabe::launch_head_tiles_bf16(s, h->num_cus, a)
+               : format == XABE_HEAD_Q8_0 ? xabe::launch_head_tiles_q8(s, h->num_cus, a)
+                                          : xabe::launch_head_tiles_q6k(s, h->num_cus, a));
+      continue;
+    }
     if (format == XABE_HEAD_Q8_0) {
       XABE_TRY(xabe::launch_quant_pass<xabe::kQ8_0>(h, s, a));
       continue;

@@ -1,0 +1,672 @@
+// LM head rows of up to 2048 elements against up to sixteen tokens in one pass over the matrix.
+//
+// A workgroup has one wavefront per 256 elements of the contraction and a contiguous share of the vocabulary, which it
+// takes 32 rows at a time: every wavefront multiplies its 256 columns of the tile, the sums meet in LDS and are added in a
+// fixed order.  A wavefront's activations never change, so its operands of the matrix instruction stay in registers for the
+// whole launch (up to sixteen tokens: 96 or 128 registers), and LDS carries nothing but weight bytes (a slot per wavefront,
+// filled by DMA) and the sums.  Wavefronts that own rows instead (k_lm_head_quant) read the digits of every superblock out
+// of LDS for every tile and find room for those of eight tokens at most; lanes that hold activations, for four tokens.
+//
+// A tile is two sets of sixteen rows, each with its half of the slot: once a set's bytes are in registers the same rows of
+// the next tile are requested, so that between one and two halves are on their way at any time.  Waits are by count.  The
+// tile before is added up and stored between the second set's wait and its request: stores count with the loads, and
+// there half a tile's time passes before one is waited for.  Shares are whole tiles, so that a token's 32 logits are one
+// line of memory.
+//
+// Bound by bytes, but for Q6_K's vector instructions at more than eight tokens.  248 320 x 2048, us for a pass over the
+// matrix, before / with these (1 / 3 / 8 / 16 tokens): Q8_0 99 / 107 / 153 / 294, now 97 / 102 / 111 / 128 (5.6 to
+// 4.2 TB/s); bf16 178 / 189 / 389 / 756, now 173 / 180 / 186 / 197 (5.9 to 5.2 TB/s); Q6_K at 8 / 16 tokens 158 / 309, now
+// 119 / 163.  (One request per tile, and shares that do not start on a line: Q8_0 106 / 108 / 119 / 150.)
+//
+// Per (row, token) the order of operations is fixed: a token's logits are the same bits at every batch width.
+#include <algorithm>
+
+#include "digits.h"
+#include "host_common.h"
+#include "lm_head_tiles.h"
+
+namespace xabe {
+
+typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b_t __attribute__((ext_vector_type(8)));
+typedef float v4f_t __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
+typedef uint16_t v2s_t __attribute__((ext_vector_type(2)));
+
+constexpr int kTileRows = 32;
+
+// What every form has in common: the workgroup's rows, the sums' places, the reduction.
+struct HeadShare {
+  int lane, wave, waves, r, g;   // r, g: the lane's weight row of a set of sixteen and its quarter
+  int row_lo, row_hi, tiles;
+  __device__ __forceinline__ HeadShare(int vocab) {
+    lane = (int)__lane_id();
+    wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    waves = (int)(blockDim.x >> 6);
+    r = lane & 15;
+    g = lane >> 4;
+    // whole tiles, so that a token's 32 logits of a tile are a line of memory (shares equal to within a row are as long)
+    const int all = (vocab + kTileRows - 1) / kTileRows, lo = (int)((long long)all * blockIdx.x / gridDim.x);
+    tiles = (int)((long long)all * (blockIdx.x + 1) / gridDim.x) - lo;
+    row_lo = lo * kTileRows;
+    row_hi = min(row_lo + tiles * kTileRows, vocab);
+  }
+};
+
+// All but the last N of this wavefront's requests are there (stores count, too); the last tile waits for everything.
+template <int N>
+__device__ __forceinline__ void wait_but(bool last) {
+  if (last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
+// The sums the wavefronts left at red[wave][half][token][32], added and stored.  HALVES 2: one after the other, each half of
+// the superblocks by itself, then the two (k_lm_head_quant's order); otherwise in pairs.  `plain(v, t, row)`: what the logit v is replaced by.
+template <int HALVES, int TOKENS, typename Plain>
+__device__ __forceinline__ void head_reduce(const float* red, const HeadShare& sh, const LmHeadArgs& a, int row0, Plain plain) {
+  constexpr int kStride = HALVES * TOKENS * kTileRows;
+#pragma unroll 1
+  for (int i = threadIdx.x; i < a.nt * kTileRows; i += (int)blockDim.x) {
+    const int t = i / kTileRows, row = row0 + i % kTileRows;
+    float part[HALVES][8], total[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int w = 0; w < 8; ++w) part[h][w] = red[min(w, sh.waves - 1) * kStride + h * TOKENS * kTileRows + i];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      float (&p)[8] = part[h];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) p[w] = w < sh.waves ? p[w] : 0.0f;
+      if constexpr (HALVES == 2) {
+        total[h] = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) total[h] += p[w];
+      } else {
+        total[h] = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+      }
+    }
+    if (row < sh.row_hi) a.out[(size_t)(a.t0 + t) * a.vocab + row] = plain(HALVES == 2 ? total[0] + total[HALVES - 1] : total[0], t, row);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// bf16.  A fp32 activation is the sum of three bf16 numbers, each the leading eight bits of what is left, so every product
+// is exact in the matrix instruction's fp32.  The first pieces' sums of 32 columns are added in pairs, and so are the
+// wavefronts'; the second and third pieces, 2^-8 of the first, are one chain.  The sums round less often than the lanes'
+// multiplications and additions they replace (against float64, 2048 columns: root mean square of the error over
+// that of the outputs 0.76e-7, the lanes 1.24e-7).
+// A lane's pieces of an activation reach down to bf16's (fp32's) smallest exponent: columns whose largest is below 2^-30
+// are multiplied by 2^90 first, and those with a value that would lose its last piece all the same are marked by a NaN
+// scale.  A logit that is not finite, by a mark, an infinity or a NaN, is summed again by fp32 multiply-adds, so that it is
+// what those make of it.
+// ------------------------------------------------------------------------------------------------
+constexpr int kBf16Slot = kTileRows * 512;
+
+__device__ __forceinline__ float bf16_logit(const LmHeadArgs& a, int t, int row) {
+  const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (size_t)row * a.K;
+  const float* x = a.x + (size_t)(a.t0 + t) * a.K;
+  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 1
+  for (int k = 0; k < a.K; k += 8)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s[j] = __builtin_fmaf(__builtin_bit_cast(float, (uint32_t)w[k + j] << 16), x[k + j], s[j]);
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
+__global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_tiles[];
+  const HeadShare sh(a.vocab);
+  const uint32_t row_bytes = (uint32_t)a.K * 2;
+  uint8_t* const slot = s_tiles + (size_t)sh.wave * kBf16Slot;
+  const uint32_t slot_lds = lds_address(slot);
+  float* const red = reinterpret_cast<float*>(s_tiles + (size_t)sh.waves * kBf16Slot);
+  constexpr int kRed = 16 * kTileRows;
+
+  // Two rows' 512 bytes per DMA instruction.  The 16-byte pieces of a row lie in LDS permuted by the row (piece p at
+  // p ^ (row mod 16)), so that the sixteen rows of a read lie in different banks.
+  auto request = [&](int row0, int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 8 * s; i < 8 * s + 8; ++i) {
+      const int row = 2 * i + (sh.lane >> 5), piece = (sh.lane & 31) ^ (row & 15);
+      const int at = min(row0 + 2 * i, a.vocab - 1);  // (uniform; the row after it only where there is one)
+      const uint32_t next = row0 + 2 * i + 1 < a.vocab ? row_bytes : 0;
+      lds_dma_16(a.w + (size_t)at * row_bytes + sh.wave * 512, (uint32_t)(sh.lane >> 5) * next + piece * 16, slot_lds + i * 1024);
+    }
+  };
+
+  // ---- the pieces of token r's columns 32 j + 8 g .. + 7
+  v8b_t p[3][8];
+  float down;
+  {
+    const bool in = sh.r < a.nt;
+    const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.t0 + min(sh.r, a.nt - 1)) * a.K + sh.wave * 256 + 8 * sh.g);
+    float4 f[8][2];
+    uint32_t mag = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        f[j][i] = src[8 * j + i];
+        const float v[4] = {f[j][i].x, f[j][i].y, f[j][i].z, f[j][i].w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mag = max(mag, __builtin_bit_cast(uint32_t, v[c]) & 0x7fffffffu);
+      }
+    wait_loads();  // (the compiler's loads are done, and the pieces are made while the first tile is on its way)
+    request(sh.row_lo, 0);
+    request(sh.row_lo, 1);
+    mag = max(mag, (uint32_t)__shfl_xor((int)mag, 16, 64));
+    mag = max(mag, (uint32_t)__shfl_xor((int)mag, 32, 64));
+    const bool small = mag < 0x30800000u;  // (2^-30)
+    const float up = small ? 0x1p90f : 1.0f;
+    bool lost = false;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      uint32_t q[3][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 v = f[j][i >> 1];
+        uint32_t b[2][3];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float x = (in ? (i & 1 ? (c ? v.w : v.z) : (c ? v.y : v.x)) : 0.0f) * up;
+          lost = lost || (x != 0.0f && __builtin_fabsf(x) < 0x1p-100f);
+          b[c][0] = __builtin_bit_cast(uint32_t, x);
+          const float rest = x - __builtin_bit_cast(float, b[c][0] & 0xffff0000u);
+          b[c][1] = __builtin_bit_cast(uint32_t, rest);
+          b[c][2] = __builtin_bit_cast(uint32_t, rest - __builtin_bit_cast(float, b[c][1] & 0xffff0000u));
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) q[k][i] = __builtin_amdgcn_perm(b[1][k], b[0][k], 0x07060302u);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) p[k][j] = __builtin_bit_cast(v8b_t, v4u_t{q[k][0], q[k][1], q[k][2], q[k][3]});
+    }
+    lost = (__builtin_amdgcn_ballot_w64(lost) >> sh.r & 0x0001000100010001ull) != 0;
+    down = lost ? __builtin_nanf("") : small ? 0x1p-90f : 1.0f;
+  }
+  float scale[4];  // of tokens 4 g + i, whose sums the lane's result registers are
+#pragma unroll
+  for (int i = 0; i < 4; ++i) scale[i] = __shfl(down, 4 * sh.g + i, 64);
+  auto reduce = [&](int n) __attribute__((always_inline)) {
+    head_reduce<1, 16>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
+                       [&](float v, int t, int row) __attribute__((always_inline)) { return __builtin_isfinite(v) ? v : bf16_logit(a, t, row); });
+  };
+
+#pragma unroll 1
+  for (int n = 0; n < sh.tiles; ++n) {
+    const int row0 = sh.row_lo + kTileRows * n;
+    float* const buf = red + (size_t)(n & 1) * sh.waves * kRed;
+    const bool last = n + 1 == sh.tiles;
+    float* const mine = buf + sh.wave * kRed;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      wait_but<8>(last);
+      v8b_t w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = *reinterpret_cast<const v8b_t*>(slot + (16 * s + sh.r) * 512 + (((4 * j + sh.g) ^ sh.r) * 16));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (s == 1 && n > 0) reduce(n - 1);
+      if (!last) request(row0 + kTileRows, s);
+      const v4f_t zero = {0, 0, 0, 0};
+      v4f_t hi[8], lo = zero;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[2][j], w[j], lo, 0, 0, 0);
+        hi[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[0][j], w[j], zero, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[1][j], w[j], lo, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float sum = ((hi[0][i] + hi[1][i]) + (hi[2][i] + hi[3][i])) + ((hi[4][i] + hi[5][i]) + (hi[6][i] + hi[7][i]));
+        mine[(4 * sh.g + i) * kTileRows + 16 * s + sh.r] = (sum + lo[i]) * scale[i];
+      }
+    }
+    __syncthreads();
+  }
+  reduce(sh.tiles - 1);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Q8_0.  An activation is a 48-bit number relative to the largest of its superblock (digits.h) written as four signed
+// base-4096 digits.  Codes and digits are fp16 integers (digits up to 2048, which fp16 holds), a block's digit sums at most
+// 32 * 128 * 2048 = 2^23: exact in the matrix instruction's fp32.  What is left per (row, block, token) is four fused
+// multiply-adds by the block's scale into sums of their own, joined once per superblock; six base-256 digits on the int8
+// instruction leave nine instructions to join and scale.  The operand's rows are four digits of four tokens.  Against
+// float64, 2048 columns: root mean square of the error over that of the outputs 0.76e-7, six digits 0.79e-7.
+// ------------------------------------------------------------------------------------------------
+using Q8Dma = SliceDma<kQ8_0>;
+constexpr int kQ8Digits = 8192;  // LDS of four tokens' digits of a superblock, as the instruction takes them: [block][lane][16]
+
+// Token t's superblock by multiply-adds, as a lane of quarter g holds it: eight columns of every block; the four quarters'
+// sums are added in pairs.
+__device__ __forceinline__ float q8_plain(const LmHeadArgs& a, int t, int row, int sb, int g) {
+  const uint8_t* w = a.w + (size_t)row * (a.K / 32 * kQ8Bytes) + (size_t)sb * (8 * kQ8Bytes);
+  const float* x = a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems + 8 * g;
+  float v = 0.0f;
+#pragma unroll 2
+  for (int b = 0; b < 8; ++b) {
+    const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(w + kQ8Bytes * b));
+    int8_t c[8];
+    __builtin_memcpy(c, __builtin_assume_aligned(w + kQ8Bytes * b + 2 + 8 * g, 2), 8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v = __builtin_fmaf(x[32 * b + i], d * (float)c[i], v);
+  }
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
+// The lane's activations of tokens t0 + half and t0 + 2 + half: eight columns each.
+__device__ __forceinline__ void q8_load(const LmHeadArgs& a, const HeadShare& sh, int t0, float4 (&f)[2][2]) {
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int t = t0 + 2 * it + (sh.lane >> 5);
+    const float4* src = reinterpret_cast<const float4*>(a.x + (size_t)(a.t0 + min(t, a.nt - 1)) * a.K + sh.wave * kSbElems + 8 * (sh.lane & 31));
+    f[it][0] = src[0];
+    f[it][1] = src[1];
+  }
+}
+// Digits of the four tokens from t0 on: operands to `op`, the scale of token t0 + g returned.
+__device__ __forceinline__ float q8_digits(const LmHeadArgs& a, const HeadShare& sh, int t0, const float4 (&f)[2][2], uint8_t* lds, v8h_t (&op)[8]) {
+  const int octet = sh.lane & 31, b = octet >> 2, q = octet & 3;
+  float own[2];
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int t = 2 * it + (sh.lane >> 5);
+    const bool in = t0 + t < a.nt;
+    const float4 f0 = f[it][0], f1 = f[it][1];
+    float v[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    uint32_t mag = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = in ? v[i] : 0.0f;
+      mag = max(mag, __builtin_bit_cast(uint32_t, v[i]) & 0x7fffffffu);
+    }
+    mag = row16_max(mag);
+    mag = max(mag, (uint32_t)__shfl_xor((int)mag, 16, 64));
+    const int e = digit_exponent(mag), shift = digit_shift(e);
+    bool inexact = false;
+    v4u_t plane[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float d[2][4];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        float rest = __builtin_ldexpf(v[2 * i + c], shift);
+        inexact = inexact || __builtin_rintf(rest) != rest;
+        d[c][0] = __builtin_rintf(rest * 0x1p-36f);
+        rest = __builtin_fmaf(d[c][0], -0x1p36f, rest);
+        d[c][1] = __builtin_rintf(rest * 0x1p-24f);
+        rest = __builtin_fmaf(d[c][1], -0x1p24f, rest);
+        d[c][2] = __builtin_rintf(rest * 0x1p-12f);
+        d[c][3] = __builtin_fmaf(d[c][2], -0x1p12f, rest);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) plane[k][i] = __builtin_bit_cast(uint32_t, v2h_t{(_Float16)d[0][k], (_Float16)d[1][k]});
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) *reinterpret_cast<v4u_t*>(lds + b * 1024 + (q * 16 + 4 * t + k) * 16) = plane[k];
+    const uint64_t any = __builtin_amdgcn_ballot_w64(inexact);
+    own[it] = digit_scale(mag, e, (uint32_t)(sh.lane >> 5 ? any >> 32 : any) != 0);
+  }
+  const float s0 = __shfl(own[0], 32 * (sh.g & 1), 64), s1 = __shfl(own[1], 32 * (sh.g & 1), 64);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int j = 0; j < 8; ++j) op[j] = *reinterpret_cast<const v8h_t*>(lds + j * 1024 + sh.lane * 16);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  return sh.g >> 1 ? s1 : s0;
+}
+
+template <int NQ>
+__global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_tiles[];
+  const HeadShare sh(a.vocab);
+  const int sb = sh.wave;
+  const uint32_t row_bytes = (uint32_t)sh.waves * SbRaw<kQ8_0>::kBytes;
+  uint8_t* const slot = s_tiles + (size_t)sh.wave * Q8Dma::kSlotBytes;
+  const uint32_t slot_lds = lds_address(slot);
+  uint8_t* const rest = s_tiles + (size_t)sh.waves * Q8Dma::kSlotBytes;  // the digits' places at first, then the sums'
+  float* const red = reinterpret_cast<float*>(rest);
+  constexpr int kRed = 4 * NQ * kTileRows;
+
+  Q8Dma dma;
+  dma.init(row_bytes, 16);
+  auto request = [&](int row0, int s) __attribute__((always_inline)) {
+    dma.request(a.w, a.w_bytes, (size_t)min(row0 + 16 * s, a.vocab - 1) * row_bytes, sb, slot_lds + s * Q8Dma::kRunBytes);
+  };
+  v8h_t op[NQ][8];
+  float e[NQ];
+  float4 f[NQ][2][2];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) q8_load(a, sh, 4 * q, f[q]);
+  wait_loads();  // (the compiler's loads are done, and the digits are made while the first tile is on its way)
+  request(sh.row_lo, 0);
+  request(sh.row_lo, 1);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) e[q] = 16.0f * q8_digits(a, sh, 4 * q, f[q], rest + (size_t)sh.wave * kQ8Digits, op[q]);  // (2^36 of the digits, 2^32 of the scale)
+  __syncthreads();
+  auto reduce = [&](int n) __attribute__((always_inline)) {
+    head_reduce<1, 4 * NQ>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
+                        [](float v, int, int) __attribute__((always_inline)) { return v; });
+  };
+
+#pragma unroll 1
+  for (int n = 0; n < sh.tiles; ++n) {
+    const int row0 = sh.row_lo + kTileRows * n;
+    float* const buf = red + (size_t)(n & 1) * sh.waves * kRed;
+    const bool last = n + 1 == sh.tiles;
+    float* const mine = buf + sh.wave * kRed;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      wait_but<Q8Dma::kInstr>(last);
+      // The lane's eight codes of every block: on a word in odd blocks, half a word past one in even ones.
+      uint32_t code[8][2], d[4];  // (two blocks' scales to a register)
+      const uint8_t* p = slot + s * Q8Dma::kRunBytes + sh.r * SbRaw<kQ8_0>::kBytes;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const uint8_t* at = p + kQ8Bytes * b + 8 * sh.g;
+        const uint32_t scale = *reinterpret_cast<const uint16_t*>(p + kQ8Bytes * b);
+        d[b / 2] = b & 1 ? d[b / 2] | scale << 16 : scale;
+        if (b & 1) {
+          code[b][0] = lds_word(at + 2);
+          code[b][1] = lds_word(at + 6);
+        } else {
+          const uint32_t w0 = lds_word(at), w1 = lds_word(at + 4), w2 = lds_word(at + 8);
+          code[b][0] = __builtin_amdgcn_alignbit(w1, w0, 16);
+          code[b][1] = __builtin_amdgcn_alignbit(w2, w1, 16);
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (s == 1 && n > 0) reduce(n - 1);
+      if (!last) request(row0 + kTileRows, s);
+      v4f_t acc[NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[q] = v4f_t{0, 0, 0, 0};
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        // 1024 + 128 + code as halves, less 1152
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const uint32_t u = code[b][i] ^ 0x80808080u;
+          h[2 * i] = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
+          h[2 * i + 1] = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
+        }
+        v8h_t w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const v2h_t v = __builtin_bit_cast(v2h_t, h[i]) - v2h_t{(_Float16)1152.0f, (_Float16)1152.0f};
+          w[2 * i] = v[0];
+          w[2 * i + 1] = v[1];
+        }
+        const float ws = f16_bits_to_f32(d[b / 2] >> (16 * (b & 1)));
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const v4f_t sums = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[q][b], w, v4f_t{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) acc[q][k] = __builtin_fmaf(ws, sums[k], acc[q][k]);
+        }
+      }
+      float out[NQ];
+      bool nan = false;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        out[q] = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(acc[q][3], 0x1p-12f, acc[q][2]), 0x1p-12f, acc[q][1]), 0x1p-12f, acc[q][0]) * e[q];
+        nan |= out[q] != out[q];
+      }
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan && row0 + 16 * s + sh.r < sh.row_hi) != 0, 0)) {
+        const int row = min(row0 + 16 * s + sh.r, a.vocab - 1);
+#pragma unroll 1
+        for (int t = 0; t < a.nt; ++t) {
+          bool mine_too = false;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) mine_too |= t == 4 * q + sh.g && out[q] != out[q];
+          if (!__builtin_amdgcn_ballot_w64(mine_too)) continue;
+          const float plain = q8_plain(a, t, row, sb, sh.g);
+#pragma unroll
+          for (int q = 0; q < NQ; ++q)
+            if (t == 4 * q + sh.g && out[q] != out[q]) out[q] = plain;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) mine[(4 * q + sh.g) * kTileRows + 16 * s + sh.r] = out[q];
+    }
+    __syncthreads();
+  }
+  reduce(sh.tiles - 1);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Q6_K, from five tokens on.  The sums of half a superblock are integers (digits.h): codes times their group's scale times
+// digits.  Here the scale goes to the code first, once for all tokens: the product has fifteen bits and is two int8 planes,
+// high and low, so the matrix instruction carries a digit's sum through the whole half superblock and what is left per
+// (row, half, token) is one shift and addition per digit and the join, where a scale per group left six multiply-adds for
+// every sixteen elements.  That costs ten instructions per four weights to make both planes and twice the matrix
+// instructions, which are full here: the rows of the operand are four digits of four tokens (twice), then the two low
+// digits of all eight.  The same integers, joined the same way: the bits of k_lm_head_quant, which up to four tokens is
+// the faster one.
+// ------------------------------------------------------------------------------------------------
+using Q6Dma = SliceDma<kQ6K>;
+constexpr int kQ6Digits = 8 * kSbDigitBytes;  // LDS of eight tokens' digits of a superblock
+
+// Both planes of the sixteen codes of a lane: ql and qh words, step 0 low nibbles and 1 high ones; `up`, `down`: how far the
+// two high bits of the lane's group are from bits 4 and 5; `scale`: four times the group's scale, twice; `add`: 128 less
+// 32 times that.
+__device__ __forceinline__ void q6_planes(const v4u_t& ql, const v4u_t& qh, int step, uint32_t shift, v2s_t scale, v2s_t add, v4i_t& hi, v4i_t& lo) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t t = step == 0 ? (ql[i] & 0x0f0f0f0fu) | ((qh[i] << shift) & 0x30303030u)
+                                 : ((ql[i] >> 4) & 0x0f0f0f0fu) | ((qh[i] >> shift) & 0x30303030u);
+    const v2s_t even = __builtin_bit_cast(v2s_t, t & 0x00ff00ffu), odd = __builtin_bit_cast(v2s_t, (t >> 8) & 0x00ff00ffu);
+    const uint32_t pe = __builtin_bit_cast(uint32_t, (v2s_t)(even * scale + add)), po = __builtin_bit_cast(uint32_t, (v2s_t)(odd * scale + add));
+    hi[i] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
+    lo[i] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
+  }
+}
+
+template <int NO>
+__global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_tiles[];
+  const HeadShare sh(a.vocab);
+  const int sb = sh.wave, r = sh.r, g = sh.g;
+  const uint32_t row_bytes = (uint32_t)sh.waves * kQ6KBytes;
+  uint8_t* const slot = s_tiles + (size_t)sh.wave * Q6Dma::kSlotBytes;
+  const uint32_t slot_lds = lds_address(slot);
+  uint8_t* const rest = s_tiles + (size_t)sh.waves * Q6Dma::kSlotBytes;  // the digits' places at first, then the sums'
+  float* const red = reinterpret_cast<float*>(rest);
+  constexpr int kRed = 2 * 8 * NO * kTileRows;
+
+  Q6Dma dma;
+  dma.init(row_bytes, 16);
+  auto run_off = [&](int row0, int u) __attribute__((always_inline)) { return (size_t)min(row0 + 16 * u, a.vocab - 1) * row_bytes; };
+  auto request = [&](int row0, int s) __attribute__((always_inline)) {
+    dma.request(a.w, a.w_bytes, run_off(row0, s), sb, slot_lds + s * Q6Dma::kRunBytes);
+  };
+  v4i_t op[NO][4][3];  // [step of 64 elements: half, step][digits 0..3 of tokens 0..3, of tokens 4..7, digits 4 and 5]
+  float e[NO][2];      // scales of tokens g and 4 + g
+  float4 f[8 * NO];
+#pragma unroll
+  for (int t = 0; t < 8 * NO; ++t)
+    f[t] = reinterpret_cast<const float4*>(a.x + (size_t)(a.t0 + min(t, a.nt - 1)) * a.K + sb * kSbElems)[sh.lane];
+  wait_loads();  // (the compiler's loads are done, and the digits are made while the first tile is on its way)
+  request(sh.row_lo, 0);
+  request(sh.row_lo, 1);
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    uint8_t* const lds = rest + (size_t)sh.wave * kQ6Digits;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const bool in = 8 * o + t < a.nt;
+      const float v[4] = {in ? f[8 * o + t].x : 0.0f, in ? f[8 * o + t].y : 0.0f, in ? f[8 * o + t].z : 0.0f, in ? f[8 * o + t].w : 0.0f};
+      const float scale = digitize_quads(v, lds + t * kSbDigitBytes);
+      if ((t & 3) == 0 || g == (t & 3)) e[o][t >> 2] = scale;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint8_t* group = lds + (4 * (2 * (j & 1) + (g >> 1)) + 2 * (j >> 1) + (g & 1)) * kGroupBytes;
+      const int t = r >> 2, i = r & 3;
+      op[o][j][0] = *reinterpret_cast<const v4i_t*>(group + t * kSbDigitBytes + 16 * i);
+      op[o][j][1] = *reinterpret_cast<const v4i_t*>(group + (4 + t) * kSbDigitBytes + 16 * i);
+      op[o][j][2] = *reinterpret_cast<const v4i_t*>(group + (t + 4 * (i >> 1)) * kSbDigitBytes + 16 * (4 + (i & 1)));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  __syncthreads();
+  auto reduce = [&](int n) __attribute__((always_inline)) {
+    head_reduce<2, 8 * NO>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
+                        [](float v, int, int) __attribute__((always_inline)) { return v; });
+  };
+  const uint32_t shift[2] = {4u - 2u * (uint32_t)(g >> 1), 2u * (uint32_t)(g >> 1)};
+
+#pragma unroll 1
+  for (int n = 0; n < sh.tiles; ++n) {
+    const int row0 = sh.row_lo + kTileRows * n;
+    float* const buf = red + (size_t)(n & 1) * sh.waves * kRed;
+    const bool last = n + 1 == sh.tiles;
+    float* const mine = buf + sh.wave * kRed;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      wait_but<Q6Dma::kInstr>(last);
+      if (sb == sh.waves - 1 && row0 + kTileRows >= a.vocab) {  // (the tensor's last bytes, which no whole piece held)
+        const int live = a.vocab - (row0 + 16 * s);
+        if (live >= 1 && live <= 16) dma.patch_tail(a.w, run_off(row0, s), live, sb, slot + s * Q6Dma::kRunBytes);
+      }
+      v4u_t ql[2], qh[2];
+      int sc[4];
+      // (rows are whole words: every window starts at the same half word)
+      const uint8_t* const b = static_cast<const uint8_t*>(__builtin_assume_aligned(slot + s * Q6Dma::kRunBytes + r * (Q6Dma::kP * 16), 16));
+      const uint32_t mis = (uint32_t)(sb & 1) * 2;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const v4u_t l = *reinterpret_cast<const v4u_t*>(b + 64 * h + 16 * g), m = *reinterpret_cast<const v4u_t*>(b + 128 + 32 * h + 16 * (g & 1));
+        const uint32_t l4 = lds_word(b + 64 * h + 16 * g + 16), m4 = lds_word(b + 128 + 32 * h + 16 * (g & 1) + 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ql[h][i] = __builtin_amdgcn_alignbit(i < 3 ? l[i + 1] : l4, l[i], 8 * mis);
+          qh[h][i] = __builtin_amdgcn_alignbit(i < 3 ? m[i + 1] : m4, m[i], 8 * mis);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sc[2 * h + j] = *reinterpret_cast<const int8_t*>(b + mis + 192 + 8 * h + 4 * j + g);
+      }
+      const uint32_t d = *reinterpret_cast<const uint16_t*>(b + mis + 208);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (s == 1 && n > 0) reduce(n - 1);
+      if (!last) request(row0 + kTileRows, s);
+      float out[2][NO][2];
+      bool nan = false;
+      const float quarter = f16_bits_to_f32(d) * 0.25f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        v4i_t hi[2], lo[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint16_t four = (uint16_t)(sc[2 * h + j] << 2);
+          const v2s_t scale = {four, four}, add = (v2s_t){128, 128} - (v2s_t)(scale << 5);
+          q6_planes(ql[h], qh[h], j, shift[j], scale, add, hi[j], lo[j]);
+        }
+#pragma unroll
+        for (int o = 0; o < NO; ++o) {
+          v4i_t H[3], L[3];
+#pragma unroll
+          for (int f = 0; f < 3; ++f) {
+            const v4i_t zero = {0, 0, 0, 0};
+            H[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h][f], hi[0], zero, 0, 0, 0);
+            L[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h][f], lo[0], zero, 0, 0, 0);
+          }
+#pragma unroll
+          for (int f = 0; f < 3; ++f) {
+            H[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h + 1][f], hi[1], H[f], 0, 0, 0);
+            L[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h + 1][f], lo[1], L[f], 0, 0, 0);
+          }
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            int sum[6];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sum[k] = (H[t][k] << 8) + L[t][k];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) sum[4 + k] = (H[2][2 * t + k] << 8) + L[2][2 * t + k];
+            out[h][o][t] = join_sums(sum) * (quarter * e[o][t]);
+            nan |= out[h][o][t] != out[h][o][t];
+          }
+        }
+      }
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan && row0 + 16 * s + r < sh.row_hi) != 0, 0)) {
+        // half_fp32 wants a lane per row and half: lane 32 h + r
+        const int row = min(row0 + 16 * s + r, a.vocab - 1);
+        SbRaw<kQ6K> raw;
+        sb_read(a.w + (size_t)row * row_bytes + (size_t)sb * kQ6KBytes, sh.lane >> 5, raw);
+#pragma unroll 1
+        for (int t = 0; t < a.nt; ++t) {
+          const float plain = half_fp32(raw, a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems, sh.lane >> 5, sh.lane);
+          const float half[2] = {__shfl(plain, r, 64), __shfl(plain, 32 + r, 64)};
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int o = 0; o < NO; ++o)
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                if (t == 8 * o + 4 * u + g && out[h][o][u] != out[h][o][u]) out[h][o][u] = half[h];
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int o = 0; o < NO; ++o)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) mine[(h * 8 * NO + 8 * o + 4 * t + g) * kTileRows + 16 * s + r] = out[h][o][t];
+    }
+    __syncthreads();
+  }
+  reduce(sh.tiles - 1);
+}
+
+// ------------------------------------------------------------------ host side
+typedef void (*HeadKernel)(LmHeadArgs);
+
+static int head_tiles_limit(HeadKernel kernel, size_t smem) {
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  return XABE_OK;
+}
+static size_t head_bf16_lds(size_t waves) { return waves * (kBf16Slot + 2 * 16 * kTileRows * sizeof(float)); }
+static size_t head_q8_lds(size_t waves, size_t nq) {
+  return waves * (Q8Dma::kSlotBytes + std::max<size_t>(kQ8Digits, 2 * 4 * nq * kTileRows * sizeof(float)));
+}
+static size_t head_q6_lds(size_t waves, size_t no) {
+  return waves * (Q6Dma::kSlotBytes + std::max<size_t>(kQ6Digits, 2 * 2 * 8 * no * kTileRows * sizeof(float)));
+}
+static const HeadKernel kHeadQ8[4] = {k_head_tiles_q8<1>, k_head_tiles_q8<2>, k_head_tiles_q8<3>, k_head_tiles_q8<4>};
+static const HeadKernel kHeadQ6[2] = {k_head_tiles_q6<1>, k_head_tiles_q6<2>};
+
+// at handle creation, not on the launch path (launches are captured into graphs)
+int head_tiles_configure() {
+  XABE_TRY(head_tiles_limit(k_head_tiles_bf16, head_bf16_lds(8)));
+  for (size_t i = 0; i < 4; ++i) XABE_TRY(head_tiles_limit(kHeadQ8[i], head_q8_lds(8, i + 1)));
+  for (size_t i = 0; i < 2; ++i) XABE_TRY(head_tiles_limit(kHeadQ6[i], head_q6_lds(8, i + 1)));
+  return XABE_OK;
+}
+
+// As many workgroups as are resident at once (eight wavefronts to a compute unit), and no more than there are tiles.
+static int head_tiles_go(HeadKernel kernel, hipStream_t s, int num_cus, size_t smem, const LmHeadArgs& a) {
+  const int waves = a.K / kSbElems, tiles = (a.vocab + kTileRows - 1) / kTileRows;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(tiles, num_cus * (8 / waves))), dim3((unsigned)(64 * waves)), smem, s, a);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+int launch_head_tiles_bf16(hipStream_t s, int num_cus, const LmHeadArgs& a) {
+  return head_tiles_go(k_head_tiles_bf16, s, num_cus, head_bf16_lds(a.K / kSbElems), a);
+}
+int launch_head_tiles_q8(hipStream_t s, int num_cus, const LmHeadArgs& a) {
+  const size_t nq = ((size_t)a.nt + 3) / 4;
+  return head_tiles_go(kHeadQ8[nq - 1], s, num_cus, head_q8_lds(a.K / kSbElems, nq), a);
+}
+int launch_head_tiles_q6k(hipStream_t s, int num_cus, const LmHeadArgs& a) {
+  const size_t no = ((size_t)a.nt + 7) / 8;
+  return head_tiles_go(kHeadQ6[no - 1], s, num_cus, head_q6_lds(a.K / kSbElems, no), a);
+}
+
+}  // namespace xabe

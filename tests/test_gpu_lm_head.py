@@ -134,6 +134,42 @@ def test_quantized_passes_at_their_edges(oracle, X, fmt, vocab, hidden, tokens):
     assert np.array_equal(alone[0].view(np.uint32), got[0].view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q6K", "Bf16"])
+@pytest.mark.parametrize("vocab,hidden,tokens", [
+    (31, 512, 13), (33, 1024, 16), (1000, 1536, 12),    # two, four and six wavefronts; rows short of a tile and past one
+    (257 * 32 + 5, 2048, 16), (2049, 2048, 19)])        # workgroups with a tile more than others; two passes
+def test_passes_of_up_to_sixteen_tokens(oracle, X, fmt, vocab, hidden, tokens):
+    # float64 within 5e-7 of the peak (tests/test_gpu_digit_precision.py derives it); the same bits alone
+    import torch
+
+    fmt = getattr(X.HeadFormat, fmt)
+    w, host = _weights(X, oracle, fmt, vocab, hidden, 34000 + vocab)
+    k = X.LmHeadKernels(X.LmHeadGeometry(hidden, vocab, tokens))
+    x = X.synth_normal_f32(34001, tokens * hidden, 1.0).view(tokens, hidden)
+    x[1, 5] = 3e4                                       # an outlier beside ordinary values
+    x[2, 256:512] *= 1e-30                              # columns of one wavefront far below the others
+    x[3] *= 2.0 ** -100                                 # a row of tiny values
+    x[4, ::2] *= 2.0 ** -100                            # (tiny values beside ordinary ones lose bits in pieces and digits)
+    x[5, 7] = 2.0 ** -135
+    got = _run(X, k, w, fmt, x, tokens)
+    xs = x.cpu().numpy()
+    for t in range(tokens):
+        ref = host.astype(np.float64) @ xs[t].astype(np.float64)
+        err = np.abs(got[t] - ref).max() / np.abs(ref).max()
+        assert err <= 5e-7, (str(fmt), t, err)
+    for t in (0, tokens - 1):
+        alone = _run(X, X.LmHeadKernels(X.LmHeadGeometry(hidden, vocab, 1)), w, fmt, x[t:t + 1].contiguous(), 1)
+        assert np.array_equal(alone[0].view(np.uint32), got[t].view(np.uint32)), t
+    # an infinity and a NaN reach their own token's logits as in plain fp32, and no other's
+    x[0, 100], x[tokens - 1, 3] = np.inf, np.nan
+    bad = _run(X, k, w, fmt, x, tokens)
+    with np.errstate(invalid="ignore"):
+        ref = (host * x[0].cpu().numpy()).sum(1)
+    assert np.array_equal(np.isnan(bad[0]), np.isnan(ref)) and np.array_equal(np.isposinf(bad[0]), np.isposinf(ref))
+    assert np.isnan(bad[tokens - 1]).all()
+    assert np.array_equal(bad[1:tokens - 1].view(np.uint32), got[1:tokens - 1].view(np.uint32))
+
+
 def test_forward_error_paths(oracle, X):
     import torch
 

@@ -11,8 +11,8 @@ use crate::moe::{check, MoeError};
 
 /// lm_head.rs:169
 pub const ARGMAX_BLOCKS: usize = ffi::XABE_LM_HEAD_ARGMAX_BLOCKS;
-/// Tokens one pass over the weights serves in every format (the reference's tile is 8, which quantized heads reach here, too;
-/// byte accounting goes through [`LmHeadGeometry::weight_passes`], an upper bound for those).
+/// Tokens one pass over the weights serves in every format (the reference's tile is 8; most heads reach 8 or 16 here;
+/// byte accounting goes through [`LmHeadGeometry::weight_passes`], an upper bound).
 pub const MAX_BATCH_TILE: usize = ffi::XABE_LM_HEAD_MAX_BATCH_TILE;
 
 /// lm_head.rs `HeadFormat`; the community formats are recognised and refused (`UnsupportedExpertType`).
