@@ -913,12 +913,12 @@ int xabe_moe_shared_expert(const xabe_moe_kernels* k, void* stream, xabe_moe_buf
   return shared_fp32(k, as_stream(stream), b, gate, up, down, hidden_states, out);
 }
 
-int xabe_moe_shared_expert_mma(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                               xabe_quant_tensor up, xabe_quant_tensor down, const float* hidden_states,
-                               size_t hidden_states_len, float* out, size_t out_len) {
-  if (!k || !b || !hidden_states || !out) return set_error(XABE_ERR_INVALID_ARGUMENT, "shared_expert_mma: null pointer");
+int xabe::shared_expert_mma_residual(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
+                                     xabe_quant_tensor up, xabe_quant_tensor down, const float* x, size_t x_len, float* out,
+                                     size_t out_len, const float* residual, float* l_out, bool* added) {
+  if (!k || !b || !x || !out) return set_error(XABE_ERR_INVALID_ARGUMENT, "shared_expert_mma: null pointer");
   XABE_TRY(check_shared_stacks(k, gate, up, down));
-  XABE_TRY(check_len("hidden_states", k->g.max_tokens * k->g.hidden, hidden_states_len));
+  XABE_TRY(check_len("hidden_states", k->g.max_tokens * k->g.hidden, x_len));
   XABE_TRY(check_len("out", k->g.max_tokens * k->g.hidden, out_len));
   if (!k->tensor_cores)
     return set_error(XABE_ERR_UNSUPPORTED_GEOMETRY, "unsupported MoE geometry %s: the matrix cores are disabled on this instance",
@@ -926,7 +926,15 @@ int xabe_moe_shared_expert_mma(const xabe_moe_kernels* k, void* stream, xabe_moe
   if (!mfma_supported(k, b, gate.quant, up.quant, down.quant, false))
     return set_error(XABE_ERR_MMA, "the matrix-core path needs buffers allocated with mma staging and max_tokens >= %zu",
                      kMfmaMinTokens);
-  return mfma_shared_expert(k, as_stream(stream), b, gate, up, down, hidden_states, out);
+  return mfma_shared_expert(k, s, b, gate, up, down, x, out, residual, l_out, added);
+}
+
+int xabe_moe_shared_expert_mma(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b, xabe_quant_tensor gate,
+                               xabe_quant_tensor up, xabe_quant_tensor down, const float* hidden_states,
+                               size_t hidden_states_len, float* out, size_t out_len) {
+  bool added = false;
+  return xabe::shared_expert_mma_residual(k, as_stream(stream), b, gate, up, down, hidden_states, hidden_states_len, out, out_len,
+                                          nullptr, nullptr, &added);
 }
 
 int xabe_moe_grouped_forward_partial_with_shared(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b,

@@ -367,10 +367,12 @@ int xabe_dense_ffn_block_forward(xabe_dense_ffn_block* blk, void* stream, const 
                            g.hidden, blk->eps));
   if (wide) {
     blk->buffers->x_h_ready = with_h;
-    const int st = xabe_moe_shared_expert_mma(blk->moe, stream, blk->buffers, w->gate, w->up, w->down, blk->normed, blk->n_act,
-                                              ffn_out, blk->n_act);
+    bool added = false;
+    const int st = shared_expert_mma_residual(blk->moe, as_stream(stream), blk->buffers, w->gate, w->up, w->down, blk->normed,
+                                              blk->n_act, ffn_out, blk->n_act, residual, l_out, &added);
     blk->buffers->x_h_ready = false;
     XABE_TRY(st);
+    if (added) return XABE_OK;
   } else {
     XABE_TRY(xabe_moe_shared_expert(blk->moe, stream, blk->buffers, w->gate, w->up, w->down, blk->normed, blk->n_act,
                                     ffn_out, blk->n_act));

@@ -129,8 +129,14 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
 bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* capacity);
 int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                                  xabe_quant_tensor up, xabe_quant_tensor down, const float* x);
+// (`residual`, `l_out`: null, or l_out = out + residual where a launch comes by that can add it: `*added`)
 int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out);
+                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out, const float* residual,
+                       float* l_out, bool* added);
+// xabe_moe_shared_expert_mma with that residual (api.hip)
+int shared_expert_mma_residual(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
+                               xabe_quant_tensor up, xabe_quant_tensor down, const float* x, size_t x_len, float* out,
+                               size_t out_len, const float* residual, float* l_out, bool* added);
 // fp16 copy of the activations both of the above start from; a caller that makes it once sets
 // `x_h_ready` on the buffers for the calls that follow and clears it afterwards
 int mfma_convert_activations(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, const float* x);

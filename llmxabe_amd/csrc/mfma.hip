@@ -51,6 +51,9 @@ struct MfmaArgs {
   int n_rows;                   // output columns per token (rows of one weight matrix)
   int top_k;
   int tile_rows;                // unrouted: token rows of a tile
+  int parts;                    // k_mfma_parts: parts the contraction is in, each of whole superblocks and as long
+  float* planes;                // the second part's sums, [*][n_rows], the others' `plane` elements apart; the first's: `out`
+  size_t plane;
 };
 
 // SwiGLU's gate in the matrix-core regime: x / (1 + e^-x) from the hardware's exp2 and reciprocal (a few ulp of
@@ -730,8 +733,8 @@ constexpr size_t mfma_rows_lds() {
 template <int MI, int WAVES>
 constexpr int kWgsPerCu = MI > 2 ? 1 : 3;
 
-template <int QUANT, int NM, bool ROUTED, int MI, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_rows(MfmaArgs a) {
+template <int QUANT, int NM, bool ROUTED, int MI, int WAVES, bool kInParts>
+__device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   constexpr int kTM = 32 * MI;                    // token rows of a tile at most
   constexpr int kTR = WAVES * kWRows;             // weight rows of a tile
   constexpr int kSlot = MI * kBlockBytes;         // an activation step in LDS
@@ -739,6 +742,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   using Window = WWindow<QUANT, MI>;
   constexpr int kRun = Window::kRunBytes, kRunInstr = Window::kRunInstr;
   constexpr bool kScaled = ROUTED && NM == 1;
+  constexpr uint32_t kSbBytes = QUANT == kQ6K ? kQ6KBytes : 8 * kQ8Bytes;
   extern __shared__ __attribute__((aligned(16))) uint8_t mfma_smem[];
   uint8_t* const sA = mfma_smem;
   uint8_t* const sW = sA + kRing * kSlot;
@@ -753,8 +757,9 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   const int n_ntiles = a.n_rows / (kTR / NM);
   const int tile_rows = a.tile_rows;
   const int n_mtiles = ROUTED ? a.tile_list[0] : (valid + tile_rows - 1) / tile_rows;
-  const int total = n_mtiles * n_ntiles;
-  const int nsteps = a.K / kSK, nsb = a.K / 256;
+  const int parts = kInParts ? a.parts : 1;
+  const int total = n_mtiles * n_ntiles * parts;
+  const int k_part = a.K / parts, nsteps = k_part / kSK, nsb = k_part / 256;
   const uint32_t row_bytes = QUANT == kQ6K ? (uint32_t)(a.K / 256) * kQ6KBytes : (uint32_t)(a.K / 32) * kQ8Bytes;
 
   // Which items this workgroup takes.  Workgroup ids are dealt round-robin to the eight XCDs, each with its own L2: when
@@ -776,10 +781,10 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
     return lane;
   };
 
-  struct Item { int e, m0, rows, nt; };
+  struct Item { int e, m0, rows, nt, part; };
   auto decode = [&](int item) __attribute__((always_inline)) {
-    const int mt = item / n_ntiles;
-    Item it{0, mt * tile_rows, min(tile_rows, valid - mt * tile_rows), item % n_ntiles};
+    const int row = item / n_ntiles, mt = kInParts ? row / parts : row;
+    Item it{0, mt * tile_rows, min(tile_rows, valid - mt * tile_rows), item % n_ntiles, kInParts ? row % parts : 0};
     if (ROUTED) {
       typedef int int4v __attribute__((ext_vector_type(4)));
       int4v ent;
@@ -802,9 +807,14 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
     w_off[i] = (uint32_t)(pc / Window::kPieces) * row_bytes + (uint32_t)(pc % Window::kPieces) * 16;
   }
   const uint8_t *w_base0, *w_base1;  // the runs' first rows, of the item the weight stream is in
+  // (in parts) how far into its rows an item starts, the weight stream's, and whether it ends them
+  auto start_of = [&](const Item& it) __attribute__((always_inline)) { return kInParts ? (uint32_t)(it.part * nsb) * kSbBytes : 0u; };
+  [[maybe_unused]] uint32_t w_from = 0;
+  [[maybe_unused]] bool w_ends = true;
   uint32_t w_last0, w_last1;         // the last whole piece of the stack from there
   auto set_w = [&](const Item& it) __attribute__((always_inline)) {
     const int r0 = it.nt * (kTR / NM) + wave * (kWRows / NM);
+    if constexpr (kInParts) w_from = start_of(it), w_ends = it.part + 1 == parts;
     const size_t off0 = (size_t)it.e * a.expert_bytes + (size_t)r0 * row_bytes;
     const size_t off1 = NM == 2 ? off0 : off0 + (size_t)16 * row_bytes;
     w_base0 = a.w0 + off0;
@@ -838,13 +848,15 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   const uint32_t my_row = (uint32_t)(col & 15) * row_bytes;
   const bool even_rows = QUANT == kQ6K && (row_bytes & 3) == 0;  // (then a superblock starts on a word in every row or in none)
   const uint8_t* const my_window = slot + (col >> 4) * kRun + (col & 15) * (Window::kPieces * 16);
-  auto read_w = [&](int u, int half, WHalf<QUANT>& r) __attribute__((always_inline)) {  // half `u` of the contraction out of the slot
-    const uint32_t at = (uint32_t)(QUANT == kQ6K ? u >> 1 : u) * Window::kSpan, mis = (my_row + at) & Window::kStart;
+  // half `u` of the contraction, which starts `from` bytes into its rows, out of the slot
+  auto read_w = [&](uint32_t from, int u, int half, WHalf<QUANT>& r) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)(QUANT == kQ6K ? u >> 1 : u) * Window::kSpan + from, mis = (my_row + at) & Window::kStart;
     if constexpr (QUANT == kQ6K) w_read(my_window, mis, even_rows && (at & 2) == 0, half, h, r);
     else w_read(my_window + mis, 0, false, half, h, r);
   };
   // (Q6_K) the window just landed is the last of its rows: what no piece inside the tensor holds, where a row ends it
   auto patch_w = [&]() __attribute__((always_inline)) {
+    if (kInParts && !w_ends) return;
     const size_t run_bytes = (size_t)16 * row_bytes;
     if (w_base0 + run_bytes == a.w0 + a.w_bytes) patch_window<kQ6K>(a.w0, a.w_bytes - kQ6KBytes, slot + 15 * (Window::kPieces * 16));
     if (w_base1 + run_bytes == (NM == 2 ? a.w1 : a.w0) + a.w_bytes)
@@ -866,6 +878,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
       if (ROUTED && NM == 2) arow = sId[tb * kTM + live] / a.top_k;
       a_lanes[i] = __builtin_amdgcn_readfirstlane(WAVES * i < pieces ? ~0u : 0u);
       a_off[i] = ((uint32_t)arow * (uint32_t)a.K + (uint32_t)((lane & 7) ^ pc_swizzle(row)) * 8u) * 2u;
+      if constexpr (kInParts) a_off[i] += (uint32_t)(it.part * k_part) * 2u;
     }
   };
   const uint32_t lds_a = lds_address(sA) + (uint32_t)wave * 1024u;
@@ -911,6 +924,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   }
   set_w(cur);
   set_a(cur, 0);
+  w_at = w_from;
   request_w_all();
 #pragma unroll
   for (a_ks = 0; a_ks < kRing; ++a_ks) {  // (a contraction has at least four steps)
@@ -920,15 +934,15 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   a_ks = kRing - 1;
   all_landed();
   if (QUANT == kQ6K && w_win == n_win) patch_w();
-  read_w(0, 0, raw[0]);
-  if constexpr (QUANT == kQ6K) read_w(1, 1, raw[1]);
+  read_w(start_of(cur), 0, 0, raw[0]);
+  if constexpr (QUANT == kQ6K) read_w(start_of(cur), 1, 1, raw[1]);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   // (the requests that the chunks before the first would have made: the next window's)
   if (w_win == n_win) {
     w_win = 0;
     if (first + stride < hi) set_w(decode(first + stride));
   }
-  w_at = (uint32_t)w_win * Window::kSpan;
+  w_at = (uint32_t)w_win * Window::kSpan + w_from;
   ++w_win;
   request_w_all();
   wait_vm<0>();
@@ -980,18 +994,19 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
           // raw weights out of the slot: the next superblock's (Q6_K), the next half's (Q8_0)
           if constexpr (QUANT == kQ6K) {
             const int u = sb + 1 == nsb ? 0 : 2 * sb + 2;
+            const uint32_t from = kInParts ? start_of(sb + 1 == nsb ? nxt : cur) : 0;
             if constexpr (C == 12 || C == 13) {
               if (early == (C == 12)) {
                 wait_vm<Req::after_w(C)>();
                 if (w_win == n_win) patch_w();
-                read_w(u, 0, next[0]);
+                read_w(from, u, 0, next[0]);
               }
             }
-            if constexpr (C == 14) read_w(u + 1, 1, next[1]);
+            if constexpr (C == 14) read_w(from, u + 1, 1, next[1]);
           } else if constexpr ((C & 7) == 5 || (C & 7) == 6) {
             if (early == ((C & 7) == 5)) {
               wait_vm<Req::after_w(C)>();
-              read_w(C < 8 ? 1 : 0, 0, C < 8 ? second : next[0]);
+              read_w(0, C < 8 ? 1 : 0, 0, C < 8 ? second : next[0]);  // (Q8_0 superblocks are whole pieces)
             }
           }
           if constexpr ((C & 3) == 3) {
@@ -1021,7 +1036,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
                   set_w(nxt);
                 }
               }
-              w_at = (uint32_t)w_win * Window::kSpan;
+              w_at = (uint32_t)w_win * Window::kSpan + w_from;
               ++w_win;
             }
             ring = ring_after(ring);
@@ -1096,6 +1111,7 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
         } else {
           const int c = cur.nt * kTR + 32 * wave + col;
           float* out = static_cast<float*>(a.out) + c;
+          if (kInParts && cur.part > 0) out = a.planes + (size_t)(cur.part - 1) * a.plane + c;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             int orow[4];
@@ -1133,6 +1149,15 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   }
   // (nothing may still be on its way into this workgroup's LDS when it ends)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+template <int QUANT, int NM, bool ROUTED, int MI, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_rows(MfmaArgs a) {
+  mfma_rows_body<QUANT, NM, ROUTED, MI, WAVES, false>(a);
+}
+// An unrouted down contraction in parts (down_parts).
+template <int QUANT, int MI, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_parts(MfmaArgs a) {
+  mfma_rows_body<QUANT, 1, false, MI, WAVES, true>(a);
 }
 
 // fp32 -> fp16 activations for live rows; rows past `valid` are left alone.
@@ -1223,16 +1248,26 @@ static bool pc_form(const xabe_moe_kernels* k, size_t) { return k->mfma_form == 
 static size_t pass_tokens(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
   return b->valid_published > 0 ? std::min<size_t>((size_t)b->valid_published, k->g.max_tokens) : k->g.max_tokens;
 }
-// Whether an unrouted pass takes the wide form: when whole tiles of it give every CU one (dense sibling: 300 tokens 432
-// us against 392 narrow, 450 tokens 471 against 518, 2048 1200 against 1750; the shared expert of the routed model stays
-// narrow up to 8192 tokens, where it leaves room beside it for the launches it runs along with: 1965 against 1980 us for
-// two blocks).
+// Whether the launches of an unrouted pass take the wide form: when whole tiles of it give every CU one, or, as narrow tiles
+// dequantise a row of weights once per 64 tokens, as soon as wide ones occupy half of the CUs.  Gate/up: more than 96 tokens of
+// matrices whose tiles do that in one row; down in parts: more than 192.  (The shared expert of the routed model stays narrow
+// up to 8192 tokens, where it leaves room beside it for the launches it runs along with: 1965 against 1980 us for two blocks.)
+// Dense sibling, us per block, both narrow / gate/up wide / both wide: 96 tokens 152 / 149 / 162, 128: 164 / 162 / 177, 192: 203 / 185 /
+// 199, 224: 250 / 247 / 239, 256: 263 / 252 / 244, 288: 307 / 272 / 258, 383: 362 / 319 / 292, 450: 463 / 379 / 326.
 static bool unrouted_wide(const xabe_moe_kernels* k, size_t tokens) {
   return tokens / kWideRows * (k->g.intermediate / 128) >= (size_t)k->num_cus;
+}
+static bool unrouted_up_wide(const xabe_moe_kernels* k, size_t tokens) {
+  return unrouted_wide(k, tokens) || (tokens > kWideRows / 2 && 2 * (k->g.intermediate / 128) >= (size_t)k->num_cus);
+}
+static bool unrouted_down_wide(const xabe_moe_kernels* k, size_t tokens, int parts) {
+  const size_t items = (tokens + kWideRows - 1) / kWideRows * (k->g.hidden / 256) * parts;
+  return unrouted_wide(k, tokens) || (parts > 1 && tokens > kWideRows && 2 * items >= (size_t)k->num_cus);
 }
 // Token rows of a wide unrouted tile: the height whose items, dealt in rounds to the CUs, end first, an item's time being
 // that of its 32-row blocks and about 3.6 blocks' more (dense sibling, 2048 tokens: a superblock of the contraction
 // takes 2.3 us and 0.64 us per block; down 385 us at 192 rows, one round, and 616 at 160, two).
+// (A part of a contraction is an item like another: `row_tiles` counts it.)
 static int unrouted_tile_rows(const xabe_moe_kernels* k, size_t tokens, size_t row_tiles) {
   int best = 32;
   double best_cost = 1e30;
@@ -1263,6 +1298,12 @@ static int configure_one() {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_rows_lds<kQ8_0, MI, WAVES>()));
   return XABE_OK;
 }
+template <int QUANT, int MI, int WAVES>
+static int configure_parts() {
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mfma_parts<QUANT, MI, WAVES>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)mfma_rows_lds<QUANT, MI, WAVES>()));
+  return XABE_OK;
+}
 template <int NM>
 static int configure_pc() {
   const void* fns[2] = {reinterpret_cast<const void*>(k_mfma_pc<kQ6K, NM>), reinterpret_cast<const void*>(k_mfma_pc<kQ8_0, NM>)};
@@ -1291,6 +1332,10 @@ static int mfma_set_limits() {
   XABE_TRY((configure_one<2, false, 2, 4>()));
   XABE_TRY((configure_one<1, true, 2, 4>()));
   XABE_TRY((configure_one<2, true, 2, 4>()));
+  XABE_TRY((configure_parts<kQ6K, 6, 8>()));
+  XABE_TRY((configure_parts<kQ8_0, 6, 8>()));
+  XABE_TRY((configure_parts<kQ6K, 2, 4>()));
+  XABE_TRY((configure_parts<kQ8_0, 2, 4>()));
   return XABE_OK;
 }
 
@@ -1310,6 +1355,18 @@ static int launch_rows(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, 
     hipLaunchKernelGGL((k_mfma_rows<kQ6K, NM, ROUTED, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ6K, MI, WAVES>()), s, a);
   else
     hipLaunchKernelGGL((k_mfma_rows<kQ8_0, NM, ROUTED, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ8_0, MI, WAVES>()), s, a);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
+template <int MI, int WAVES>
+static int launch_parts(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, size_t mtiles, hipStream_t s) {
+  const size_t items = mtiles * (size_t)(a.n_rows / (WAVES * kWRows)) * a.parts;
+  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(items, (size_t)k->num_cus * kWgsPerCu<MI, WAVES>));
+  if (quant == XABE_QUANT_Q6K)
+    hipLaunchKernelGGL((k_mfma_parts<kQ6K, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ6K, MI, WAVES>()), s, a);
+  else
+    hipLaunchKernelGGL((k_mfma_parts<kQ8_0, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ8_0, MI, WAVES>()), s, a);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
@@ -1379,8 +1436,60 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
   return XABE_OK;
 }
 
+// Parts of an unrouted down contraction.  Its row tiles are few where the contraction is long (5120 rows: 40 narrow tiles, 20
+// wide), and a tile walks its whole contraction alone: 64 tokens took 147 us on 40 workgroups.  Up to 1024 tokens the
+// contraction is in four parts (or as many as divide it), whose sums are added in order by one more launch; by the
+// buffers' size and the geometry alone, so that a token's row is the same bits in every pass and in every pass of buffers up to
+// that size.  Wider passes have tiles enough, and four planes of sums would cost them more than they gain (2048 tokens of
+// the dense sibling: as many rounds of items, and 170 MB each way).  The planes lie in the fp32 intermediate rows, which the
+// matrix-core regime does not use.
+constexpr size_t kPartsMaxTokens = 1024;
+static int down_parts(const xabe_moe_geometry& g) {
+  if (g.max_tokens > kPartsMaxTokens) return 1;
+  const size_t nsb = g.intermediate / 256;
+  for (int parts = 4; parts > 1; --parts)
+    if (nsb % parts == 0 && nsb / parts >= 8 && (size_t)(parts - 1) * g.hidden <= g.intermediate) return parts;
+  return 1;
+}
+
+// The parts' sums of a live row in order, and the residual where there is one.  Bound by memory (hidden is a multiple of 256).
+__global__ void __launch_bounds__(256) k_add_parts(const float* __restrict__ planes, size_t plane, int parts, const int* __restrict__ valid_tokens,
+                                                   int hidden, const float* __restrict__ residual, float* __restrict__ out, float* __restrict__ l_out) {
+  const int t = blockIdx.x, j = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (t >= *valid_tokens || j >= hidden) return;
+  const size_t i = (size_t)t * hidden + j;
+  const bool whole = ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(l_out)) & 15) == 0;
+  float v[4], x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (whole) {
+    const float4 f = *reinterpret_cast<const float4*>(out + i);
+    v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+    if (l_out) {
+      const float4 r = *reinterpret_cast<const float4*>(residual + i);
+      x[0] = r.x, x[1] = r.y, x[2] = r.z, x[3] = r.w;
+    }
+  } else {  // (rows that start on any float)
+    for (int c = 0; c < 4; ++c) v[c] = out[i + c], x[c] = l_out ? residual[i + c] : 0.0f;
+  }
+  float4 p[3];
+#pragma unroll
+  for (int n = 0; n < 3; ++n) p[n] = *reinterpret_cast<const float4*>(planes + (size_t)min(n, parts - 2) * plane + i);
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+    if (n + 1 < parts) v[0] += p[n].x, v[1] += p[n].y, v[2] += p[n].z, v[3] += p[n].w;
+  if (whole) {
+    *reinterpret_cast<float4*>(out + i) = make_float4(v[0], v[1], v[2], v[3]);
+    if (l_out) *reinterpret_cast<float4*>(l_out + i) = make_float4(v[0] + x[0], v[1] + x[1], v[2] + x[2], v[3] + x[3]);
+  } else {
+    for (int c = 0; c < 4; ++c) {
+      out[i + c] = v[c];
+      if (l_out) l_out[i + c] = v[c] + x[c];
+    }
+  }
+}
+
 int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
+                       xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out, const float* residual, float* l_out,
+                       bool* added) {
   const xabe_moe_geometry& g = k->g;
   if (!b->x_h_ready) XABE_TRY(to_f16(k, s, b, x));
   MfmaArgs a;
@@ -1395,7 +1504,7 @@ int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   a.n_rows = (int)g.intermediate;
   a.w_bytes = gate.len;
   const size_t tokens = pass_tokens(k, b);
-  const bool wide = unrouted_wide(k, tokens);
+  bool wide = unrouted_up_wide(k, tokens);
   a.tile_rows = wide ? unrouted_tile_rows(k, tokens, g.intermediate / 128) : kNarrowRows;
   size_t tiles = (g.max_tokens + a.tile_rows - 1) / a.tile_rows;
   if (wide) XABE_TRY((launch_rows<2, false, 6, 8>(k, gate.quant, a, tiles, s)));
@@ -1407,10 +1516,23 @@ int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
   a.out = out;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  a.tile_rows = wide ? unrouted_tile_rows(k, tokens, g.hidden / 256) : kNarrowRows;
+  a.parts = down_parts(g);
+  a.planes = b->shared_inter;
+  a.plane = g.max_tokens * g.hidden;
+  wide = unrouted_down_wide(k, tokens, a.parts);
+  a.tile_rows = wide ? unrouted_tile_rows(k, tokens, g.hidden / 256 * a.parts) : kNarrowRows;
   tiles = (g.max_tokens + a.tile_rows - 1) / a.tile_rows;
-  if (wide) return launch_rows<1, false, 6, 8>(k, down.quant, a, tiles, s);
-  return launch_rows<1, false, 2, 4>(k, down.quant, a, tiles, s);
+  *added = a.parts > 1;
+  if (a.parts == 1) {
+    if (wide) return launch_rows<1, false, 6, 8>(k, down.quant, a, tiles, s);
+    return launch_rows<1, false, 2, 4>(k, down.quant, a, tiles, s);
+  }
+  if (wide) XABE_TRY((launch_parts<6, 8>(k, down.quant, a, tiles, s)));
+  else XABE_TRY((launch_parts<2, 4>(k, down.quant, a, tiles, s)));
+  hipLaunchKernelGGL(k_add_parts, dim3((unsigned)g.max_tokens, (unsigned)((g.hidden + 1023) / 1024)), dim3(256), 0, s, a.planes, a.plane,
+                     a.parts, b->valid_tokens, (int)g.hidden, residual, out, l_out);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
 }
 
 }  // namespace xabe

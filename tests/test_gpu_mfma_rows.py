@@ -86,3 +86,40 @@ def test_unrouted_widths_across_the_rule(X, quant, hidden, inter, widths):
         rows.append(got[0])
     for wider in rows[1:]:   # a token's row does not depend on the batch around it
         assert torch.equal(wider[:widths[0]].view(torch.int32), rows[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("quant", ["q6k", "q8_0"])
+@pytest.mark.parametrize("hidden,inter", [(512, 6912), (768, 8704), (512, 11008), (1280, 4096)])
+def test_long_down_contractions_in_parts(X, quant, hidden, inter):
+    # three, two and one part (27, 34 and 43 superblocks), and none for want of a place for the planes; both tile forms; the block,
+    # whose last launch adds the residual, against the separate calls
+    import torch
+
+    weights = _weights(X, quant, quant, hidden * inter)
+    norm = 1.0 + X.synth_normal_f32(4, hidden, 0.1)
+    rows = []
+    for tokens, live in ((64, 64), (100, 97), (1024, 1000)):
+        x = X.synth_normal_f32(9, tokens * hidden, 1.0).view(tokens, hidden)
+        blk = X.DenseFfnBlock(hidden, inter, tokens)
+        ffn, l_out = torch.full_like(x, -7.0), torch.full_like(x, -7.0)
+        blk.publish_tokens(live)
+        blk.forward(X.DenseFfnLayerWeights(norm, *weights), x, live, ffn, l_out)
+        k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, tokens))
+        got = []
+        for mma in (True, False):
+            if not mma:
+                k.disable_tensor_cores()
+            b = k.shared_only_buffers(True)
+            k.set_valid_tokens(b, live)
+            out = torch.full_like(x, -7.0)
+            (k.shared_expert_mma if mma else k.shared_expert)(b, *weights, blk.normed().view(tokens, hidden), out)
+            got.append(out)
+        torch.cuda.synchronize()
+        _close(got[0][:live], got[1][:live])
+        assert torch.equal(ffn[:live].view(torch.int32), got[0][:live].view(torch.int32))
+        assert torch.equal(l_out[:live], ffn[:live] + x[:live])
+        for t in (ffn, l_out, got[0]):
+            assert (t[live:] == -7.0).all()
+        rows.append(ffn[:64])
+    for wider in rows[1:]:   # a token's row does not depend on the batch around it
+        assert torch.equal(wider.view(torch.int32), rows[0].view(torch.int32))
