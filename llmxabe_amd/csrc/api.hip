@@ -302,6 +302,8 @@ int xabe_moe_kernels_new(const xabe_moe_geometry* geometry, xabe_moe_kernels** o
   // everything one-time happens here, none of it on the launch path (launches are captured into graphs)
   int st = mfma_configure();
   if (st == XABE_OK) st = digit_rows_configure();
+  if (st == XABE_OK) st = digit_columns_configure();
+  if (st == XABE_OK) st = digit_narrow_configure();
   if (st == XABE_OK) st = decode_block_configure();
   if (st != XABE_OK) {
     delete k;
@@ -347,8 +349,20 @@ int xabe_moe_kernels_set_exact_decode_regime(xabe_moe_kernels* k, int on) {
 // so that a token's row is the same bits at every width.  Dense block, Q6_K, us, lanes / digits: hidden 1024, intermediate
 // 4352: one token 15 / 21, eight 30 / 36, thirty-two 87 / 63; 2048, 6144: 20 / 26, 50 / 45, 157 / 87; Q8_0, 2048, 8192:
 // 29 / 29, seven 105 / 48.
+constexpr size_t kSharedPairsMaxElements = (size_t)8 << 20;  // (shared_by_pairs)
 static bool shared_on_digits(const xabe_moe_geometry& g) {
   return g.hidden > 2048 || (g.intermediate > 2048 && g.hidden * g.intermediate >= ((size_t)10 << 20));
+}
+
+// Large Q6_K matrices: the intermediate rows are scaled by whole superblocks, like the activations, after gate/up, and the
+// launches are digit_narrow.hip's and, from five tokens on, digit_columns.hip's.  By the geometry and the formats alone, for the same reason.
+// (Scales by groups of sixteen, which gate/up's workgroups make by themselves, cost down ten instructions per row, group and
+// token, and its sums a rounding per group.)  Dense block, us, scales by group / by superblock: one token 54.8 / 50.3, two 58.7 /
+// 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105, sixteen 183 / 109.
+static bool shared_whole(const xabe_moe_geometry& g, int gate_q, int up_q, int down_q) {
+  return gate_q == XABE_QUANT_Q6K && up_q == XABE_QUANT_Q6K && down_q == XABE_QUANT_Q6K && shared_on_digits(g) &&
+         g.hidden % 256 == 0 && g.intermediate % 256 == 0 && g.hidden >= 2048 && g.intermediate >= 2048 &&
+         g.hidden * g.intermediate > kSharedPairsMaxElements;
 }
 
 constexpr size_t kDigitScratchRows = 8192;  // intermediate rows of the routed experts whose digits the scratch holds
@@ -419,6 +433,9 @@ static int alloc_buffers(const xabe_moe_kernels* k, void* stream, int scope, boo
   A(&b->shared_x_e, shared_rows * nsb_h);
   A(&b->shared_inter_d, shared_rows * nsb_i * kSbDigitBytes);
   A(&b->shared_inter_e, shared_rows * nsb_i * 16);
+  A(&b->shared_parts, shared_rows > 4 && shared_whole(g, XABE_QUANT_Q6K, XABE_QUANT_Q6K, XABE_QUANT_Q6K)
+                          ? kWholeQuarters * shared_rows * g.hidden
+                          : 0);
   // matrix-core staging: only passes wide enough to take that regime pay for it
   A(&b->x_h, (wide && mma) ? g.max_tokens * g.hidden : 0);
   A(&b->inter_h, (wide && mma && routed) ? sorted * g.intermediate : 0);
@@ -454,7 +471,7 @@ void xabe_moe_buffers_free(xabe_moe_buffers* b) {
                   b->num_tokens_post_pad, b->valid_tokens, b->align_hist, b->partial, b->shared_inter, b->x_h, b->inter_h,
                   b->shared_inter_h, b->tile_list, b->router_partial, b->seam_arrivals,
                   b->x_d, b->x_e, b->inter, b->inter_d, b->inter_e, b->shared_x_d, b->shared_x_e,
-                  b->shared_inter_d, b->shared_inter_e};
+                  b->shared_inter_d, b->shared_inter_e, b->shared_parts};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete b;
@@ -793,13 +810,22 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
   return XABE_OK;
 }
 
+// Whether gate/up of n tokens makes its activations' digits itself.
+static bool shared_makes(const xabe_moe_kernels* k, int gate_q, int up_q, int down_q, size_t n) {
+  return shared_whole(k->g, gate_q, up_q, down_q) && digit_up_serves(k, k->g.hidden, n);
+}
 // gate/up and down of a single-expert stack on the digit contraction, for tokens first .. first + n - 1, whose activation
-// digits are in b->shared_x_d (x: the rows of all tokens)
+// digits are in b->shared_x_d unless shared_makes says otherwise (x: the rows of all tokens; with `norm`, shared_makes holds and
+// they are normalised first, and go to `normed`)
 static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                          xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out, size_t first, size_t n,
-                         const float* residual = nullptr, float* l_out = nullptr) {
+                         const float* residual = nullptr, float* l_out = nullptr, const float* norm = nullptr,
+                         float eps = 0.0f, float* normed = nullptr) {
   const xabe_moe_geometry& g = k->g;
   RowsArgs a = rows_args(k, b);
+  a.norm = norm;
+  a.normed = normed ? normed + first * g.hidden : nullptr;
+  a.eps = eps;
   a.unit0 = (int)first;
   a.w0 = static_cast<const uint8_t*>(gate.bytes);
   a.w1 = static_cast<const uint8_t*>(up.bytes);
@@ -808,11 +834,15 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   a.xd = b->shared_x_d;
   a.xe = b->shared_x_e;
   a.out = b->shared_inter + first * g.intermediate;
-  a.out_d = b->shared_inter_d;
+  const bool whole = shared_whole(g, gate.quant, up.quant, down.quant), columns = whole && n > 4 && !k->force_community;
+  a.out_d = whole ? nullptr : b->shared_inter_d;
   a.out_e = b->shared_inter_e;
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
-  XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, n, s));
+  if (columns) XABE_TRY(launch_digit_columns(k, 2, a, n, s));
+  else if (shared_makes(k, gate.quant, up.quant, down.quant, n)) XABE_TRY(launch_digit_up(k, a, n, s));
+  else XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, n, s));
+  if (whole && (columns || !digit_down_makes(k, n))) XABE_TRY(launch_digitize_rows(s, a.out, g.intermediate, n, b->shared_inter_d, b->shared_inter_e));
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.w_bytes = down.len;
@@ -824,14 +854,16 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   a.l_out = l_out ? l_out + first * g.hidden : nullptr;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  return launch_digit_rows(k, kRowsShared, down.quant, 1, a, n, s);
+  a.parts = b->shared_parts;
+  if (columns) return launch_digit_columns(k, 1, a, n, s);
+  return whole ? launch_digit_down(k, a, n, s) : launch_digit_rows(k, kRowsShared, down.quant, 1, a, n, s);
 }
 
 // The same on the pair kernel: a token is a unit of expert 0.  Up to four tokens it saves the launch that makes the digits
 // (hidden 4096, intermediate 1024, Q6_K: one token 18.7 -> 17.9 us, three 22.5 -> 17.9); beyond, and for matrices that do
 // not stay in the caches, rows read and unpacked once per token cost more.
 static bool shared_by_pairs(const xabe_moe_kernels* k) {
-  return k->g.max_tokens <= 4 && k->g.hidden * k->g.intermediate <= ((size_t)8 << 20) && !k->force_community;
+  return k->g.max_tokens <= 4 && k->g.hidden * k->g.intermediate <= kSharedPairsMaxElements && !k->force_community;
 }
 static int shared_pairs(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                         xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {
@@ -868,7 +900,8 @@ static int shared_fp32(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffer
     if (shared_by_pairs(k)) return shared_pairs(k, s, b, gate, up, down, x, out);
     for (size_t first = 0; first < g.max_tokens; first += kSharedDigitTokens) {
       const size_t n = std::min(kSharedDigitTokens, g.max_tokens - first);
-      XABE_TRY(launch_digitize_rows(s, x + first * g.hidden, g.hidden, n, b->shared_x_d, b->shared_x_e));
+      if (!shared_makes(k, gate.quant, up.quant, down.quant, n))
+        XABE_TRY(launch_digitize_rows(s, x + first * g.hidden, g.hidden, n, b->shared_x_d, b->shared_x_e));
       XABE_TRY(shared_digits(k, s, b, gate, up, down, x, out, first, n));
     }
     return XABE_OK;
@@ -894,6 +927,10 @@ int xabe::dense_fp32_fused(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_bu
   for (size_t first = 0; first < g.max_tokens; first += kSharedDigitTokens) {
     const size_t n = std::min(kSharedDigitTokens, g.max_tokens - first), at = first * g.hidden;
     const int nsb = (int)digit_superblocks(g.hidden);
+    if (shared_makes(k, gate.quant, up.quant, down.quant, n)) {
+      XABE_TRY(shared_digits(k, s, b, gate, up, down, residual, ffn_out, first, n, residual, l_out, post_norm, eps, normed));
+      continue;
+    }
     hipLaunchKernelGGL(k_rms_norm_digits, dim3((unsigned)n, (unsigned)((nsb + 3) / 4)), dim3(256), 0, s, residual + at, post_norm,
                        normed + at, (int)g.hidden, eps, nsb, b->shared_x_d, b->shared_x_e);
     XABE_HIP_TRY(hipGetLastError());

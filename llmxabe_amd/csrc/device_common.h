@@ -150,6 +150,15 @@ __device__ __forceinline__ void lds_dma_16(const void* base, uint32_t voff, uint
 #pragma clang diagnostic pop
 }
 
+// One dword per lane from `base` + `voff` into LDS at `dst` + 4 * lane (see lds_dma_16).
+__device__ __forceinline__ void lds_dma_4(const void* base, uint32_t voff, uint32_t dst) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base),
+               "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 // The lane's number, made where it is asked for (__lane_id() is the same value, but the compiler makes it, and whatever is
 // derived from it, once, outside all loops): for what a loop does rarely, in kernels that fill their registers.  Held all
 // along it would be spilled, and what reloads a spilled register waits for every request in flight.

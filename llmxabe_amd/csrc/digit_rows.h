@@ -22,10 +22,13 @@ struct RowsArgs {
   size_t expert_bytes;       // bytes of one expert in a stack (0: a single matrix)
   const float* x;            // the activation rows, [row][K] (what a marked group goes back to)
   const uint8_t* xd;         // digits of the activation rows, [row][superblock][kSbDigitBytes] (pairs' gate/up makes its own)
-  const float* xe;           // their scales: gate/up [row][superblock], down [row][superblock][16] (by group)
+  const float* xe;           // their scales: gate/up [row][superblock], down [row][superblock][16] (by group; or as gate/up)
   float* out;                // [row][n_rows]
   uint8_t* out_d;            // nm = 2: digits of the output rows (null: not written)
   float* out_e;
+  const float* norm;         // launch_digit_up: x is normalised with this weight, and goes to `normed`
+  float* normed;
+  float eps;
   const float* residual;     // with l_out: l_out = out + residual
   float* l_out;
   const int* valid_tokens;
@@ -39,6 +42,8 @@ struct RowsArgs {
   // filled in by launch_digit_rows
   int nsb, out_nsb, classes, tile_rows, n_tiles;
   int units, shares, xcd_units;  // pairs (xcd_units: units of one share side by side, one per XCD; 0: plain order)
+  int tokens;                      // launch_digit_columns: rows of a plane of `parts`
+  float* parts;                    // [quarter][token][n_rows]
   int shared_wgs, shared_rps;      // pairs with the shared expert: its workgroups per chunk of two tokens, rows per step
   uint32_t row_bytes;
 };
@@ -78,6 +83,23 @@ int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, u
 int launch_digitize_groups(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
 // `units`: dispatch blocks, or the tokens of a single matrix
 int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s);
+// What the launches have in common: superblocks, classes and tiles of the matrix.
+void rows_shape(RowsArgs& a, int quant, int nm);
+
+// Down of a large single Q6_K matrix, whose activations are scaled by superblocks (digit_columns.hip): classes are superblock
+// mod 32, class c in quarter c / 8; a quarter adds its classes in order, each half of the superblocks by itself, then the two
+// halves; the quarters are added in pairs.
+constexpr int kWholeQuarters = 4;
+int digit_columns_configure();
+int digit_narrow_configure();
+// Gate and up for one or two tokens, from a.x alone.
+bool digit_up_serves(const xabe_moe_kernels* k, size_t hidden, size_t tokens);
+int launch_digit_up(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipStream_t s);
+// Down for up to four tokens.  One, and each by itself under force_community: from a.x alone; otherwise from its digits.
+bool digit_down_makes(const xabe_moe_kernels* k, size_t tokens);
+int launch_digit_down(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipStream_t s);
+// Any number of tokens, of such a matrix or of gate/up's.  nm = 1 with a.parts, kWholeQuarters * tokens * n_rows floats.
+int launch_digit_columns(const xabe_moe_kernels* k, int nm, RowsArgs a, size_t tokens, hipStream_t s);
 // One (token, k) pair per unit, straight from topk_ids: pairs a.unit0 .. a.unit0 + units - 1.  `shared`: the shared
 // expert's rows of the same shape (whole superblocks, at most 2048 elements) ride along.
 int launch_digit_pairs(const xabe_moe_kernels* k, int quant, int nm, RowsArgs a, size_t units, hipStream_t s,

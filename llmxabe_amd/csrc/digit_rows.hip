@@ -678,7 +678,7 @@ int launch_digitize_groups(hipStream_t s, const float* x, size_t K, size_t rows,
   return XABE_OK;
 }
 
-static void rows_shape(RowsArgs& a, int quant, int nm) {
+void rows_shape(RowsArgs& a, int quant, int nm) {
   const size_t be = xabe_expert_quant_block_elements(quant), bb = xabe_expert_quant_block_bytes(quant);
   a.nsb = (int)digit_superblocks((size_t)a.K);
   a.row_bytes = (uint32_t)((size_t)a.K / be * bb);

@@ -395,17 +395,21 @@ __device__ __forceinline__ float half_fp32_all(const SbRaw<QUANT>& r, const floa
   (half_fp32_eight<QUANT, K>(r, own, out), ...);
   return out;
 }
-template <int QUANT>
-__device__ __forceinline__ float half_fp32(SbRaw<QUANT>& r, const float* __restrict__ x, int half, int lane) {
-  float own[8];
+using HalfOrder = std::integer_sequence<int, 0, 1, 4, 5, 8, 9, 12, 13, 2, 3, 6, 7, 10, 11, 14, 15>;  // (l outermost)
+__device__ __forceinline__ void half_own(const float* __restrict__ x, int half, int lane, float (&own)[8]) {
   const uint8_t* const at = reinterpret_cast<const uint8_t*>(x) + (uint32_t)(half * 512 + (lane & 15) * 32);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const float4 v = reinterpret_cast<const float4*>(at)[i];
     own[4 * i] = v.x, own[4 * i + 1] = v.y, own[4 * i + 2] = v.z, own[4 * i + 3] = v.w;
   }
+}
+template <int QUANT>
+__device__ __forceinline__ float half_fp32(SbRaw<QUANT>& r, const float* __restrict__ x, int half, int lane) {
+  float own[8];
+  half_own(x, half, lane, own);
   opaque(r);
-  return half_fp32_all<QUANT>(r, own, std::integer_sequence<int, 0, 1, 4, 5, 8, 9, 12, 13, 2, 3, 6, 7, 10, 11, 14, 15>{});  // (l outermost)
+  return half_fp32_all<QUANT>(r, own, HalfOrder{});
 }
 
 // The lane's eight group sums of one superblock for NT tokens: out[t] = the half's sum.
@@ -560,6 +564,12 @@ struct LdsDigits {
   template <int E_STRIDE>
   __device__ __forceinline__ float4 scale(int t, int l) const { return *reinterpret_cast<const float4*>(e + t * E_STRIDE + l * 16); }
 };
+
+template <int N>
+__device__ __forceinline__ void wait_but() {  // all but the last N requests of this wavefront are there
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+
 
 // What the pieces of the window that starts at byte `start` of a tensor and ends with it could not hold, two bytes at a time,
 // to the window at `slot`.  SPAN: the bytes wanted from `start` on.

@@ -178,6 +178,7 @@ struct xabe_moe_buffers {
   size_t n_digit_rows;
   uint8_t *x_d, *inter_d, *shared_x_d, *shared_inter_d;
   float *x_e, *inter_e, *shared_x_e, *shared_inter_e;
+  float* shared_parts;  // digit_columns.hip
   float* inter;         // [slot][intermediate]: the routed intermediate rows
   float* partial;       // [flat][hidden]
   float* shared_inter;  // [token][intermediate]

@@ -24,6 +24,7 @@
 #include "digits.h"
 #include "host_common.h"
 #include "lm_head_tiles.h"
+#include "planes.h"
 
 namespace xabe {
 
@@ -31,7 +32,6 @@ typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 typedef __bf16 v8b_t __attribute__((ext_vector_type(8)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
-typedef uint16_t v2s_t __attribute__((ext_vector_type(2)));
 
 constexpr int kTileRows = 32;
 
@@ -238,13 +238,22 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
 using Q8Dma = SliceDma<kQ8_0>;
 constexpr int kQ8Digits = 8192;  // LDS of four tokens' digits of a superblock, as the instruction takes them: [block][lane][16]
 
+// For which of four tokens a lane of quarter g, token g's, holds a NaN.
+__device__ __forceinline__ uint32_t marked_tokens(float v) {
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(v != v);
+  uint32_t m = 0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) m |= (uint32_t)((lanes >> (16 * g) & 0xffff) != 0) << g;
+  return m;
+}
+
 // Token t's superblock by multiply-adds, as a lane of quarter g holds it: eight columns of every block; the four quarters'
 // sums are added in pairs.
 __device__ __forceinline__ float q8_plain(const LmHeadArgs& a, int t, int row, int sb, int g) {
   const uint8_t* w = a.w + (size_t)row * (a.K / 32 * kQ8Bytes) + (size_t)sb * (8 * kQ8Bytes);
   const float* x = a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems + 8 * g;
   float v = 0.0f;
-#pragma unroll 2
+#pragma unroll 4
   for (int b = 0; b < 8; ++b) {
     const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(w + kQ8Bytes * b));
     int8_t c[8];
@@ -345,7 +354,9 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
   request(sh.row_lo, 0);
   request(sh.row_lo, 1);
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) e[q] = 16.0f * q8_digits(a, sh, 4 * q, f[q], rest + (size_t)sh.wave * kQ8Digits, op[q]);  // (2^36 of the digits, 2^32 of the scale)
+  for (int q = 0; q < NQ; ++q) {
+    e[q] = 16.0f * q8_digits(a, sh, 4 * q, f[q], rest + (size_t)sh.wave * kQ8Digits, op[q]);  // (2^36 of the digits, 2^32 of the scale)
+  }
   __syncthreads();
   auto reduce = [&](int n) __attribute__((always_inline)) {
     head_reduce<1, 4 * NQ>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
@@ -416,19 +427,19 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
         out[q] = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(acc[q][3], 0x1p-12f, acc[q][2]), 0x1p-12f, acc[q][1]), 0x1p-12f, acc[q][0]) * e[q];
         nan |= out[q] != out[q];
       }
+      // (a block's scale that is not finite makes NaNs, too)
+      uint32_t m = 0;
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan && row0 + 16 * s + sh.r < sh.row_hi) != 0, 0)) {
-        const int row = min(row0 + 16 * s + sh.r, a.vocab - 1);
-#pragma unroll 1
-        for (int t = 0; t < a.nt; ++t) {
-          bool mine_too = false;
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) mine_too |= t == 4 * q + sh.g && out[q] != out[q];
-          if (!__builtin_amdgcn_ballot_w64(mine_too)) continue;
-          const float plain = q8_plain(a, t, row, sb, sh.g);
+        for (int q = 0; q < NQ; ++q) m |= marked_tokens(out[q]) << (4 * q);
+      }
+      for (; __builtin_expect(m != 0, 0); m &= m - 1) {
+        const int t = __builtin_ctz(m);
+        if (t >= a.nt) break;
+        const float plain = q8_plain(a, t, min(row0 + 16 * s + sh.r, a.vocab - 1), sb, sh.g);
 #pragma unroll
-          for (int q = 0; q < NQ; ++q)
-            if (t == 4 * q + sh.g && out[q] != out[q]) out[q] = plain;
-        }
+        for (int q = 0; q < NQ; ++q)
+          if (t == 4 * q + sh.g && out[q] != out[q]) out[q] = plain;
       }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) mine[(4 * q + sh.g) * kTileRows + 16 * s + sh.r] = out[q];
@@ -451,21 +462,6 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
 using Q6Dma = SliceDma<kQ6K>;
 constexpr int kQ6Digits = 8 * kSbDigitBytes;  // LDS of eight tokens' digits of a superblock
 
-// Both planes of the sixteen codes of a lane: ql and qh words, step 0 low nibbles and 1 high ones; `up`, `down`: how far the
-// two high bits of the lane's group are from bits 4 and 5; `scale`: four times the group's scale, twice; `add`: 128 less
-// 32 times that.
-__device__ __forceinline__ void q6_planes(const v4u_t& ql, const v4u_t& qh, int step, uint32_t shift, v2s_t scale, v2s_t add, v4i_t& hi, v4i_t& lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t t = step == 0 ? (ql[i] & 0x0f0f0f0fu) | ((qh[i] << shift) & 0x30303030u)
-                                 : ((ql[i] >> 4) & 0x0f0f0f0fu) | ((qh[i] >> shift) & 0x30303030u);
-    const v2s_t even = __builtin_bit_cast(v2s_t, t & 0x00ff00ffu), odd = __builtin_bit_cast(v2s_t, (t >> 8) & 0x00ff00ffu);
-    const uint32_t pe = __builtin_bit_cast(uint32_t, (v2s_t)(even * scale + add)), po = __builtin_bit_cast(uint32_t, (v2s_t)(odd * scale + add));
-    hi[i] = (int)__builtin_amdgcn_perm(po, pe, 0x07030501u);
-    lo[i] = (int)(__builtin_amdgcn_perm(po, pe, 0x06020400u) ^ 0x80808080u);
-  }
-}
-
 template <int NO>
 __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_tiles[];
@@ -486,6 +482,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
   };
   v4i_t op[NO][4][3];  // [step of 64 elements: half, step][digits 0..3 of tokens 0..3, of tokens 4..7, digits 4 and 5]
   float e[NO][2];      // scales of tokens g and 4 + g
+  uint32_t marks = 0;  // tokens whose superblock is marked
   float4 f[8 * NO];
 #pragma unroll
   for (int t = 0; t < 8 * NO; ++t)
@@ -506,14 +503,8 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint8_t* group = lds + (4 * (2 * (j & 1) + (g >> 1)) + 2 * (j >> 1) + (g & 1)) * kGroupBytes;
-      const int t = r >> 2, i = r & 3;
-      op[o][j][0] = *reinterpret_cast<const v4i_t*>(group + t * kSbDigitBytes + 16 * i);
-      op[o][j][1] = *reinterpret_cast<const v4i_t*>(group + (4 + t) * kSbDigitBytes + 16 * i);
-      op[o][j][2] = *reinterpret_cast<const v4i_t*>(group + (t + 4 * (i >> 1)) * kSbDigitBytes + 16 * (4 + (i & 1)));
-    }
+    planes_operands(lds, kSbDigitBytes, op[o]);
+    marks |= (marked_tokens(e[o][0]) | marked_tokens(e[o][1]) << 4) << (8 * o);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   __syncthreads();
@@ -536,82 +527,36 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
         const int live = a.vocab - (row0 + 16 * s);
         if (live >= 1 && live <= 16) dma.patch_tail(a.w, run_off(row0, s), live, sb, slot + s * Q6Dma::kRunBytes);
       }
-      v4u_t ql[2], qh[2];
-      int sc[4];
-      // (rows are whole words: every window starts at the same half word)
-      const uint8_t* const b = static_cast<const uint8_t*>(__builtin_assume_aligned(slot + s * Q6Dma::kRunBytes + r * (Q6Dma::kP * 16), 16));
-      const uint32_t mis = (uint32_t)(sb & 1) * 2;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const v4u_t l = *reinterpret_cast<const v4u_t*>(b + 64 * h + 16 * g), m = *reinterpret_cast<const v4u_t*>(b + 128 + 32 * h + 16 * (g & 1));
-        const uint32_t l4 = lds_word(b + 64 * h + 16 * g + 16), m4 = lds_word(b + 128 + 32 * h + 16 * (g & 1) + 16);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          ql[h][i] = __builtin_amdgcn_alignbit(i < 3 ? l[i + 1] : l4, l[i], 8 * mis);
-          qh[h][i] = __builtin_amdgcn_alignbit(i < 3 ? m[i + 1] : m4, m[i], 8 * mis);
-        }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sc[2 * h + j] = *reinterpret_cast<const int8_t*>(b + mis + 192 + 8 * h + 4 * j + g);
-      }
-      const uint32_t d = *reinterpret_cast<const uint16_t*>(b + mis + 208);
+      Q6Quarter w;
+      w.read(slot + s * Q6Dma::kRunBytes + r * (Q6Dma::kP * 16), (uint32_t)(sb & 1) * 2, g);  // (rows are whole words)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (s == 1 && n > 0) reduce(n - 1);
       if (!last) request(row0 + kTileRows, s);
       float out[2][NO][2];
-      bool nan = false;
-      const float quarter = f16_bits_to_f32(d) * 0.25f;
+      const float quarter = f16_bits_to_f32(w.d) * 0.25f;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         v4i_t hi[2], lo[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint16_t four = (uint16_t)(sc[2 * h + j] << 2);
-          const v2s_t scale = {four, four}, add = (v2s_t){128, 128} - (v2s_t)(scale << 5);
-          q6_planes(ql[h], qh[h], j, shift[j], scale, add, hi[j], lo[j]);
-        }
+        w.planes(h, shift, hi, lo);
 #pragma unroll
         for (int o = 0; o < NO; ++o) {
-          v4i_t H[3], L[3];
-#pragma unroll
-          for (int f = 0; f < 3; ++f) {
-            const v4i_t zero = {0, 0, 0, 0};
-            H[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h][f], hi[0], zero, 0, 0, 0);
-            L[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h][f], lo[0], zero, 0, 0, 0);
-          }
-#pragma unroll
-          for (int f = 0; f < 3; ++f) {
-            H[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h + 1][f], hi[1], H[f], 0, 0, 0);
-            L[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[o][2 * h + 1][f], lo[1], L[f], 0, 0, 0);
-          }
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            int sum[6];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) sum[k] = (H[t][k] << 8) + L[t][k];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) sum[4 + k] = (H[2][2 * t + k] << 8) + L[2][2 * t + k];
-            out[h][o][t] = join_sums(sum) * (quarter * e[o][t]);
-            nan |= out[h][o][t] != out[h][o][t];
-          }
+          const float eo[2] = {quarter * e[o][0], quarter * e[o][1]};
+          planes_dot(op[o][2 * h], op[o][2 * h + 1], hi, lo, eo, out[h][o]);
         }
       }
-      if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan && row0 + 16 * s + r < sh.row_hi) != 0, 0)) {
-        // half_fp32 wants a lane per row and half: lane 32 h + r
-        const int row = min(row0 + 16 * s + r, a.vocab - 1);
-        SbRaw<kQ6K> raw;
+      for (uint32_t m = marks; __builtin_expect(m != 0, 0); m &= m - 1) {
+        const int t = __builtin_ctz(m), row = min(row0 + 16 * s + r, a.vocab - 1);
+        SbRaw<kQ6K> raw;  // (a lane per row and half: lane 32 h + r)
         sb_read(a.w + (size_t)row * row_bytes + (size_t)sb * kQ6KBytes, sh.lane >> 5, raw);
-#pragma unroll 1
-        for (int t = 0; t < a.nt; ++t) {
-          const float plain = half_fp32(raw, a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems, sh.lane >> 5, sh.lane);
-          const float half[2] = {__shfl(plain, r, 64), __shfl(plain, 32 + r, 64)};
+        const float plain = half_fp32(raw, a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems, sh.lane >> 5, sh.lane);
+        const float half[2] = {__shfl(plain, r, 64), __shfl(plain, 32 + r, 64)};
 #pragma unroll
-          for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int o = 0; o < NO; ++o)
+          for (int o = 0; o < NO; ++o)
 #pragma unroll
-              for (int u = 0; u < 2; ++u)
-                if (t == 8 * o + 4 * u + g && out[h][o][u] != out[h][o][u]) out[h][o][u] = half[h];
-        }
+            for (int u = 0; u < 2; ++u)
+              if (t == 8 * o + 4 * u + g) out[h][o][u] = half[h];
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h)

@@ -693,15 +693,6 @@ __device__ __forceinline__ void lds_dma_16_lanes(const void* base, uint32_t voff
                "s"(__builtin_amdgcn_readfirstlane(lanes_hi)) : "memory", "m0");
 #pragma clang diagnostic pop
 }
-// One dword per lane from `base` + `voff` into LDS at `dst` + 4 * lane (see lds_dma_16).
-__device__ __forceinline__ void lds_dma_4(const void* base, uint32_t voff, uint32_t dst) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base),
-               "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
-#pragma clang diagnostic pop
-}
-
 template <int MI>
 constexpr int kRing = MI > 2 ? 4 : 3;  // steps of activations in LDS
 // The requests of a superblock's sixteen chunks, in order.  Activations: after the barrier that frees a place in the ring

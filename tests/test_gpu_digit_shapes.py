@@ -93,3 +93,40 @@ def test_single_matrix_rows(fmt, hidden, inter):
         assert np.array_equal(got[:live].view(np.uint32), one.cpu().numpy()[:live].view(np.uint32)), tokens
         alone = got if tokens == 1 else alone
         assert np.array_equal(got[0].view(np.uint32), alone[0].view(np.uint32)), tokens
+
+
+@pytest.mark.parametrize("hidden,inter", [(2048, 4352), (2304, 3840), (8448, 2048)])
+def test_large_q6_k_matrices(hidden, inter):
+    # gate, up and down too large for the caches: passes of one, two, up to four, eight and sixteen tokens, in kernels of their
+    # own.  Odd numbers of superblocks and of sixteen-row sets, several row tiles per compute unit, shares of unequal size; rows
+    # with marked superblocks (elements forty binary orders apart) and an infinity next to ordinary ones.
+    import torch
+    import llmxabe_amd as X
+
+    q = X.ExpertQuant.Q6K
+    st, host = _stacks(X, q, 1, hidden, inter, 9200)
+    x = X.synth_normal_f32(9210, 33 * hidden, 1.0).view(33, hidden)
+    x[1, 1::2] *= 2.0 ** -40
+    x[6, 300] = 2.0 ** 30
+    x[12, 5] = float("inf")
+    finite = [t for t in range(33) if t not in (6, 12)]
+    ref = np.array([_ffn64(host, 0, v) for v in x.double().cpu().numpy()[finite]])
+
+    def run(rows, live):
+        k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, len(rows)))
+        b = k.shared_only_buffers(False)
+        k.set_valid_tokens(b, live)
+        out = torch.full(rows.shape, 7.0, device="cuda")
+        k.shared_expert(b, *st, rows.reshape(-1).contiguous(), out.view(-1))
+        return out.cpu().numpy()
+
+    alone = np.concatenate([run(x[t:t + 1], 1) for t in range(33)])
+    err = np.abs(alone[finite] - ref).max() / np.abs(ref).max()
+    print(hidden, inter, f"{err:.2e}", flush=True)
+    assert err <= TOL, err
+    assert not np.isfinite(alone[12]).all()
+    same = lambda a, b: np.array_equal(a, b, equal_nan=True)
+    for tokens, live in ((2, 2), (3, 3), (4, 3), (5, 5), (8, 7), (9, 9), (16, 16), (17, 16), (33, 33)):
+        got = run(x[:tokens], live)
+        assert same(got[:live], alone[:live]), tokens
+        assert (got[live:] == 7.0).all(), tokens
