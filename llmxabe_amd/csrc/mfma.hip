@@ -52,6 +52,7 @@ struct MfmaArgs {
   int top_k;
   int tile_rows;                // unrouted: token rows of a tile
   int parts;                    // k_mfma_parts: parts the contraction is in, each of whole superblocks and as long
+  int resident;                 // workgroups that fit the chip
   float* planes;                // the second part's sums, [*][n_rows], the others' `plane` elements apart; the first's: `out`
   size_t plane;
 };
@@ -757,11 +758,19 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   // there is work for every workgroup, XCD x takes a contiguous eighth of the items (token tile major) and its workgroups
   // walk that range together, so an activation tile is fetched into one L2 instead of into all eight, and the token tiles
   // of one expert reuse its weights from that L2.
-  const bool by_xcd = (gridDim.x & 7u) == 0 && total >= 2 * (int)gridDim.x;
+  // Routed gate/up, narrow: a third round of items would be two thirds full at most, and it begins late on the CUs that the shared
+  // expert still holds when the launch begins.  There a grid of twice the workgroups that fit (gate_up_twice) deals the
+  // second half to whatever CU is free first, one or two items each; in fewer rounds, or more, the half that fits does as
+  // well or better by itself (the others leave here).
+  constexpr bool kTwice = ROUTED && NM == 2 && MI <= 2;
+  const bool twice = kTwice && total >= 2 * a.resident && total < 3 * a.resident;
+  const int wgs = kTwice && !twice ? min((int)gridDim.x, a.resident) : (int)gridDim.x;
+  const bool by_xcd = (wgs & 7) == 0 && (twice || total >= 2 * wgs);
   const int xcd = blockIdx.x & 7;
   const int lo = by_xcd ? (int)((long long)total * xcd / 8) : 0, hi = by_xcd ? (int)((long long)total * (xcd + 1) / 8) : total;
   const int first = lo + (by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x);
-  const int stride = by_xcd ? (int)(gridDim.x >> 3) : (int)gridDim.x;
+  const int stride = by_xcd ? wgs >> 3 : wgs;
+  if (kTwice && (int)blockIdx.x >= wgs) return;
   if (first >= hi) return;
 
   // The lane's number for what an item does once: its arithmetic belongs there and not in registers all along, which would
@@ -1225,6 +1234,11 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
 static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
   return narrow_tiles(tokens, g.experts_per_token, g.num_experts) ? kNarrowRows : kWideRows;
 }
+// Whether narrow gate/up is launched with twice the workgroups that fit: while an expert's share averages one block of 32 rows.
+// Blocks of the routed model, us, once / twice: 100 tokens 229 / 223, 256: 248 / 239, 512: 259 / 252, 900: 283 / 280; with the
+// published layout 238 / 236, 256 / 247, 268 / 261, 293 / 290; skewed loads, whose items are less than two rounds, alike.  At 1237
+// tokens, where items are one block or two, 327 / 313, but 314 / 317 in the published layout, and skewed 255 / 260.
+static bool gate_up_twice(const xabe_moe_geometry& g, size_t tokens) { return tokens * g.experts_per_token <= 32 * g.num_experts; }
 // The specialised form (k_mfma_pc) serves both routed launches for contractions of whole superblocks and at least
 // eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_rows everywhere; it is the faster at every width
 // measured, see k_mfma_pc).
@@ -1339,9 +1353,11 @@ int mfma_configure() {
 }
 
 template <int NM, bool ROUTED, int MI, int WAVES>
-static int launch_rows(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, size_t max_mtiles, hipStream_t s) {
+static int launch_rows(const xabe_moe_kernels* k, int quant, MfmaArgs a, size_t max_mtiles, hipStream_t s, bool twice = false) {
   const size_t max_items = max_mtiles * (size_t)(a.n_rows / (WAVES * kWRows / NM));
-  const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(max_items, (size_t)k->num_cus * kWgsPerCu<MI, WAVES>));
+  a.resident = k->num_cus * kWgsPerCu<MI, WAVES>;
+  const size_t most = (size_t)a.resident * (twice ? 2 : 1);
+  const unsigned grid = (unsigned)std::max<size_t>(1, std::min(max_items, most));
   if (quant == XABE_QUANT_Q6K)
     hipLaunchKernelGGL((k_mfma_rows<kQ6K, NM, ROUTED, MI, WAVES>), dim3(grid), dim3(64 * WAVES), (mfma_rows_lds<kQ6K, MI, WAVES>()), s, a);
   else
@@ -1410,7 +1426,7 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
   a.n_rows = (int)g.intermediate;
   const bool pc = pc_form(k, pass_tokens(k, b));
   if (pc) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
-  else if (bm == kNarrowRows) XABE_TRY((launch_rows<2, true, 2, 4>(k, gate.quant, a, max_mtiles, s)));
+  else if (bm == kNarrowRows) XABE_TRY((launch_rows<2, true, 2, 4>(k, gate.quant, a, max_mtiles, s, gate_up_twice(g, pass_tokens(k, b)))));
   else XABE_TRY((launch_rows<2, true, 6, 8>(k, gate.quant, a, max_mtiles, s)));
   // down -> partial[flat][H], scaled by the routing weight
   a.w0 = static_cast<const uint8_t*>(down.bytes);

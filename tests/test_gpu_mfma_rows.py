@@ -60,6 +60,34 @@ def test_experts_of_every_size(X, counts, hidden, inter, up, down):
     assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
 
 
+@pytest.mark.parametrize("experts", [191, 192, 193, 287, 288])
+def test_gate_up_items_of_two_to_three_rounds(X, experts):
+    # eight gate/up items per expert: 1528 to 2304, about two and three times the 768 workgroups that a chip of 256 CUs holds
+    import torch
+
+    hidden, inter, tokens = 512, 512, experts + 3
+    g = X.MoeGeometry(experts, 1, hidden, inter, 32, tokens)
+    weights = _weights(X, "q6k", "q8_0", experts * hidden * inter)
+    x = X.synth_normal_f32(9, tokens * hidden, 1.0).view(tokens, hidden)
+    logits = torch.zeros(tokens, experts, device="cuda")
+    logits[torch.arange(tokens), torch.arange(tokens) % experts] = 5.0
+    out = []
+    for form in (1, 2, None):
+        k = X.MoeKernels(g)
+        if form is None:
+            k.disable_tensor_cores()
+        else:
+            k.set_mfma_form(form)
+        b = k.buffers()
+        k.set_valid_tokens(b, tokens)
+        k.route_and_dispatch(b, logits.view(-1))
+        k.grouped_forward_partial(b, *weights, x)
+        torch.cuda.synchronize()
+        out.append(b.partial().clone()[:tokens * hidden].view(tokens, hidden))
+    _close(out[0], out[2])
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
+
+
 @pytest.mark.parametrize("quant", ["q6k", "q8_0"])
 @pytest.mark.parametrize("hidden,inter,widths", [(256, 16384, (383, 384, 385, 1000)), (512, 256, (64, 65, 97, 193)),
                                                  (1280, 11008, (576, 640, 769))])
