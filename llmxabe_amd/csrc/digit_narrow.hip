@@ -123,6 +123,10 @@ __global__ void __launch_bounds__(64 * kUpWaves<NT>, kUpWaves<NT> / 4) k_digit_u
       if (NORM && (at % (int)gridDim.x == (int)blockIdx.x || scale != scale)) {
         // (one workgroup writes it; of a marked superblock every one, to read it below)
         *reinterpret_cast<float4*>(a.normed + (size_t)(slot0 + t) * a.K + at * kSbElems + 4 * lane) = make_float4(v[0], v[1], v[2], v[3]);
+        // A store of sixteen bytes still reads its registers while the next two instructions run.  The compiler keeps them apart
+        // from what writes these registers next, but not across the branch that ends this block: with one instruction in
+        // between a quarter of the lanes stored the next token's LDS address.
+        asm volatile("s_nop 2" ::: "memory");
         if (scale != scale) wait_but<0>();
       }
     }

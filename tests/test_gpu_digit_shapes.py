@@ -130,3 +130,17 @@ def test_large_q6_k_matrices(hidden, inter):
         got = run(x[:tokens], live)
         assert same(got[:live], alone[:live]), tokens
         assert (got[live:] == 7.0).all(), tokens
+    # the dense block: one and two tokens are normalised inside gate/up
+    norm = 1.0 + X.synth_normal_f32(9211, hidden, 0.1)
+    x[12, 5], x[11, 7] = 2.0 ** 60, float("inf")
+    for rows in (x[1:2], x[6:8], x[11:13], x[12:13], x[10:13]):
+        rows = rows.contiguous()
+        blk = X.DenseFfnBlock(hidden, inter, len(rows))
+        ffn, l_out = torch.zeros_like(rows), torch.zeros_like(rows)
+        blk.forward(X.DenseFfnLayerWeights(norm, *st), rows, len(rows), ffn, l_out)
+        normed = torch.zeros_like(rows)
+        X.LayerOpsKernels.rms_norm(rows, norm, normed, len(rows), hidden, 1e-6)
+        got = blk.normed().view(len(rows), hidden)
+        assert same(got.cpu().numpy(), normed.cpu().numpy())
+        assert same(ffn.cpu().numpy(), run(normed, len(rows)))
+        assert same(l_out.cpu().numpy(), (ffn + rows).cpu().numpy())
