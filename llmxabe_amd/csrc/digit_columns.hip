@@ -351,24 +351,41 @@ int digit_columns_configure() {
   return once.run(dev, columns_set_limits);
 }
 
+template <int NM, int NO>
+static int columns_go(const RowsArgs& a, unsigned workgroups, size_t passes, hipStream_t s) {
+  hipLaunchKernelGGL((k_digit_columns<NM, NO>), dim3(workgroups, (unsigned)passes), dim3(512), kColLds, s, a);
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+// Passes of sixteen; for what is left one of eight, or up to four tokens as they go by themselves (launch_digit_rows,
+// launch_digit_down; three and four tokens' gate/up there 36 us, down 29, one and two 30 and 19, a pass of eight 43 and 31, of
+// sixteen 63 and 41).  Dense sibling, us, passes of sixteen only / of eight, too / these: 17 tokens 184 / 172 / 155, 20 188 / 177 /
+// 166, 24 190 / 181 / -, 33 270 / 255 / 239, 49 354 / 338 / 324.
 int launch_digit_columns(const xabe_moe_kernels* k, int nm, RowsArgs a, size_t tokens, hipStream_t s) {
   rows_shape(a, XABE_QUANT_Q6K, nm);
   a.tokens = (int)tokens;
-  const size_t passes = (tokens + 15) / 16, each = (tokens + passes - 1) / passes, wide = each > 8 ? 16 : 8;
   const int quarters = nm == 1 ? kWholeQuarters : 1, sets = a.n_rows * nm / 16;
-  const dim3 grid((unsigned)(std::min(sets, std::max(1, k->num_cus / quarters)) * quarters), (unsigned)((tokens + wide - 1) / wide));
+  const unsigned workgroups = (unsigned)(std::min(sets, std::max(1, k->num_cus / quarters)) * quarters);
+  const size_t wide = (tokens + 7) / 16, done = std::min(tokens, 16 * wide), left = tokens - done;
+  const bool eight = left > 4;
+  RowsArgs rest = a;  // of tokens done, done + 1, ..
+  rest.unit0 += (int)done;
+  rest.x += done * a.K;
+  rest.xd += done * a.nsb * kSbDigitBytes;
+  rest.xe += done * a.nsb;
+  rest.out += done * a.n_rows;
+  if (nm == 1) rest.parts += done * a.n_rows;
+  if (a.l_out) rest.residual += done * a.n_rows, rest.l_out += done * a.n_rows;
   if (nm == 2) {
-    if (wide == 16) hipLaunchKernelGGL((k_digit_columns<2, 2>), grid, dim3(512), kColLds, s, a);
-    else hipLaunchKernelGGL((k_digit_columns<2, 1>), grid, dim3(512), kColLds, s, a);
-    XABE_HIP_TRY(hipGetLastError());
-    return XABE_OK;
+    if (wide) XABE_TRY((columns_go<2, 2>(a, workgroups, wide, s)));
+    if (eight) return columns_go<2, 1>(rest, workgroups, 1, s);
+    return left ? launch_digit_rows(k, kRowsShared, XABE_QUANT_Q6K, 2, rest, left, s) : XABE_OK;
   }
-  if (wide == 16) hipLaunchKernelGGL((k_digit_columns<1, 2>), grid, dim3(512), kColLds, s, a);
-  else hipLaunchKernelGGL((k_digit_columns<1, 1>), grid, dim3(512), kColLds, s, a);
+  if (wide) XABE_TRY((columns_go<1, 2>(a, workgroups, wide, s)));
+  if (eight) XABE_TRY((columns_go<1, 1>(rest, workgroups, 1, s)));
+  hipLaunchKernelGGL(k_columns_out, dim3((unsigned)(eight ? tokens : done), (unsigned)((a.n_rows + 1023) / 1024)), dim3(256), 0, s, a);
   XABE_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_columns_out, dim3((unsigned)tokens, (unsigned)((a.n_rows + 1023) / 1024)), dim3(256), 0, s, a);
-  XABE_HIP_TRY(hipGetLastError());
-  return XABE_OK;
+  return left && !eight ? launch_digit_down(k, rest, left, s) : XABE_OK;
 }
 
 }  // namespace xabe

@@ -105,11 +105,12 @@ def test_large_q6_k_matrices(hidden, inter):
 
     q = X.ExpertQuant.Q6K
     st, host = _stacks(X, q, 1, hidden, inter, 9200)
-    x = X.synth_normal_f32(9210, 33 * hidden, 1.0).view(33, hidden)
+    x = X.synth_normal_f32(9210, 36 * hidden, 1.0).view(36, hidden)
     x[1, 1::2] *= 2.0 ** -40
     x[6, 300] = 2.0 ** 30
     x[12, 5] = float("inf")
-    finite = [t for t in range(33) if t not in (6, 12)]
+    x[17, 2::3] *= 2.0 ** -35
+    finite = [t for t in range(36) if t not in (6, 12)]
     ref = np.array([_ffn64(host, 0, v) for v in x.double().cpu().numpy()[finite]])
 
     def run(rows, live):
@@ -120,13 +121,13 @@ def test_large_q6_k_matrices(hidden, inter):
         k.shared_expert(b, *st, rows.reshape(-1).contiguous(), out.view(-1))
         return out.cpu().numpy()
 
-    alone = np.concatenate([run(x[t:t + 1], 1) for t in range(33)])
+    alone = np.concatenate([run(x[t:t + 1], 1) for t in range(36)])
     err = np.abs(alone[finite] - ref).max() / np.abs(ref).max()
     print(hidden, inter, f"{err:.2e}", flush=True)
     assert err <= TOL, err
     assert not np.isfinite(alone[12]).all()
     same = lambda a, b: np.array_equal(a, b, equal_nan=True)
-    for tokens, live in ((2, 2), (3, 3), (4, 3), (5, 5), (8, 7), (9, 9), (16, 16), (17, 16), (33, 33)):
+    for tokens, live in ((2, 2), (3, 3), (4, 3), (5, 5), (8, 7), (9, 9), (16, 16), (17, 16), (19, 19), (24, 24), (33, 33), (36, 34)):
         got = run(x[:tokens], live)
         assert same(got[:live], alone[:live]), tokens
         assert (got[live:] == 7.0).all(), tokens
