@@ -349,7 +349,6 @@ int xabe_moe_kernels_set_exact_decode_regime(xabe_moe_kernels* k, int on) {
 // so that a token's row is the same bits at every width.  Dense block, Q6_K, us, lanes / digits: hidden 1024, intermediate
 // 4352: one token 15 / 21, eight 30 / 36, thirty-two 87 / 63; 2048, 6144: 20 / 26, 50 / 45, 157 / 87; Q8_0, 2048, 8192:
 // 29 / 29, seven 105 / 48.
-constexpr size_t kSharedPairsMaxElements = (size_t)8 << 20;  // (shared_by_pairs)
 static bool shared_on_digits(const xabe_moe_geometry& g) {
   return g.hidden > 2048 || (g.intermediate > 2048 && g.hidden * g.intermediate >= ((size_t)10 << 20));
 }
@@ -357,12 +356,17 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
 // Large Q6_K matrices: the intermediate rows are scaled by whole superblocks, like the activations, after gate/up, and the
 // launches are digit_narrow.hip's and, from five tokens on, digit_columns.hip's.  By the geometry and the formats alone, for the same reason.
 // (Scales by groups of sixteen, which gate/up's workgroups make by themselves, cost down ten instructions per row, group and
-// token, and its sums a rounding per group.)  Dense block, us, scales by group / by superblock: one token 54.8 / 50.3, two 58.7 /
-// 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105, sixteen 183 / 109.
+// token, and its sums a rounding per group.)  Dense block, us, scales by group / by superblock, hidden 5120, intermediate 17408: one
+// token 54.8 / 50.3, two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105, sixteen 183 / 109.
+// Where no width loses by it.  Intermediate rows of 32 superblocks and more: shorter ones leave classes of down's without any, and the
+// launch that writes their digits is more than down gains (one / four / eight / forty tokens, 3072 x 8192 29.6 / 39.3 / 49.6 / 133 by
+// group, 24.7 / 39.1 / 38.0 / 105 by superblock; 4096 x 4096 23.4 / 30.4 / 38.6 / 107, 20.6 / 31.4 / 36.0 / 101; 4096 x 2304 19.6 /
+// 24.7 / 30.6 / 73, 16.9 / 25.7 / 34.2 / 96).  Hidden sizes of at most 21 superblocks: a tile of down's few-token launch holds 21 rows
+// for each of 256 compute units, and beyond that it is two half-full ones (6144 x 10240 47.5 / 61.2 / 80.1 / 323, 54.8 / 75.3 / 72.3 /
+// 232; 8192 x 28672 at one and four tokens 130 / 160, 145 / 186).
 static bool shared_whole(const xabe_moe_geometry& g, int gate_q, int up_q, int down_q) {
-  return gate_q == XABE_QUANT_Q6K && up_q == XABE_QUANT_Q6K && down_q == XABE_QUANT_Q6K && shared_on_digits(g) &&
-         g.hidden % 256 == 0 && g.intermediate % 256 == 0 && g.hidden >= 2048 && g.intermediate >= 2048 &&
-         g.hidden * g.intermediate > kSharedPairsMaxElements;
+  return gate_q == XABE_QUANT_Q6K && up_q == XABE_QUANT_Q6K && down_q == XABE_QUANT_Q6K && g.hidden % 256 == 0 &&
+         g.intermediate % 256 == 0 && g.hidden >= 2048 && g.hidden <= (size_t)kWholeMaxSb * 256 && g.intermediate >= (size_t)kWholeMinInterSb * 256;
 }
 
 constexpr size_t kDigitScratchRows = 8192;  // intermediate rows of the routed experts whose digits the scratch holds
@@ -812,7 +816,7 @@ int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_wei
 
 // Whether gate/up of n tokens makes its activations' digits itself.
 static bool shared_makes(const xabe_moe_kernels* k, int gate_q, int up_q, int down_q, size_t n) {
-  return shared_whole(k->g, gate_q, up_q, down_q) && digit_up_serves(k, k->g.hidden, n);
+  return shared_whole(k->g, gate_q, up_q, down_q) && (n == 2 || digit_down_makes(k, n));
 }
 // gate/up and down of a single-expert stack on the digit contraction, for tokens first .. first + n - 1, whose activation
 // digits are in b->shared_x_d unless shared_makes says otherwise (x: the rows of all tokens; with `norm`, shared_makes holds and
@@ -863,7 +867,7 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
 // (hidden 4096, intermediate 1024, Q6_K: one token 18.7 -> 17.9 us, three 22.5 -> 17.9); beyond, and for matrices that do
 // not stay in the caches, rows read and unpacked once per token cost more.
 static bool shared_by_pairs(const xabe_moe_kernels* k) {
-  return k->g.max_tokens <= 4 && k->g.hidden * k->g.intermediate <= kSharedPairsMaxElements && !k->force_community;
+  return k->g.max_tokens <= 4 && k->g.hidden * k->g.intermediate <= ((size_t)8 << 20) && !k->force_community;
 }
 static int shared_pairs(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                         xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out) {

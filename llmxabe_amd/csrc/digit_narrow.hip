@@ -37,6 +37,7 @@ constexpr int kUpUnits = NT == 1 ? 7 : 9;  // a wavefront has at most
 template <int NT>
 constexpr int kUpFixed = kZeroBytes + NT * (kUpMaxSb + 1) * 4 + 16 - (NT * (kUpMaxSb + 1) * 4) % 16 + kUpWaves<NT> * kUpSlot;
 constexpr int up_area(int nt) { return nt == 1 ? 2048 : 3072; }  // LDS per superblock: digits, or the rows' elements and the weight's
+static_assert(kUpFixed<1> + kWholeMaxSb * up_area(1) <= kMaxLds && kUpFixed<2> + kWholeMaxSb * up_area(2) <= kMaxLds, "the rows fit beside the slots");
 
 template <int NT, bool NORM>
 __global__ void __launch_bounds__(64 * kUpWaves<NT>, kUpWaves<NT> / 4) k_digit_up(RowsArgs a) {
@@ -392,9 +393,6 @@ int launch_digit_down(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipS
   return tokens == 2 ? down_go<2, 16, 1>(a, k->num_cus, 1, s) : down_go<4, 8, 2>(a, k->num_cus, 1, s);
 }
 
-// Where gate and up are k_digit_up's: rows of at most 23 superblocks (one token; two: 24), whose elements LDS has room for.
-template <int NT>
-static bool up_fits(const RowsArgs& a) { return a.nsb >= 8 && a.nsb <= kUpMaxSb && kUpFixed<NT> + a.nsb * up_area(NT) <= kMaxLds; }
 template <int NT>
 static int up_go(const RowsArgs& a, int cus, unsigned passes, hipStream_t s) {
   int shares = cus;
@@ -406,12 +404,6 @@ static int up_go(const RowsArgs& a, int cus, unsigned passes, hipStream_t s) {
   else hipLaunchKernelGGL((k_digit_up<NT, false>), grid, block, lds, s, a);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
-}
-bool digit_up_serves(const xabe_moe_kernels* k, size_t hidden, size_t tokens) {
-  RowsArgs a = {};
-  a.K = (int)hidden;
-  rows_shape(a, XABE_QUANT_Q6K, 2);
-  return digit_down_makes(k, tokens) ? up_fits<1>(a) : tokens == 2 && up_fits<2>(a);
 }
 int launch_digit_up(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipStream_t s) {
   rows_shape(a, XABE_QUANT_Q6K, 2);

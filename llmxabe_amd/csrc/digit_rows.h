@@ -90,10 +90,10 @@ void rows_shape(RowsArgs& a, int quant, int nm);
 // mod 32, class c in quarter c / 8; a quarter adds its classes in order, each half of the superblocks by itself, then the two
 // halves; the quarters are added in pairs.
 constexpr int kWholeQuarters = 4;
+constexpr int kWholeMaxSb = 21, kWholeMinInterSb = 32;  // superblocks of the hidden size at most, of the intermediate size at least
 int digit_columns_configure();
 int digit_narrow_configure();
 // Gate and up for one or two tokens, from a.x alone.
-bool digit_up_serves(const xabe_moe_kernels* k, size_t hidden, size_t tokens);
 int launch_digit_up(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipStream_t s);
 // Down for up to four tokens.  One, and each by itself under force_community: from a.x alone; otherwise from its digits.
 bool digit_down_makes(const xabe_moe_kernels* k, size_t tokens);

@@ -145,3 +145,65 @@ def test_large_q6_k_matrices(hidden, inter):
         assert same(got.cpu().numpy(), normed.cpu().numpy())
         assert same(ffn.cpu().numpy(), run(normed, len(rows)))
         assert same(l_out.cpu().numpy(), (ffn + rows).cpu().numpy())
+
+
+# (hidden, intermediate) of the kernels that scale the intermediate rows by superblocks: the smallest of both, odd numbers of
+# superblocks (9 and 33, 21 and 35), more sets of sixteen gate/up rows than a wavefront holds sums of (73 superblocks), more
+# shares of gate and up than compute units (81)
+WHOLE = [(2048, 8192), (2304, 8448), (5376, 8960), (2048, 18688), (5376, 20736)]
+
+
+def _ffn64_rows(X, st, x, hidden, inter):
+    q = X.ExpertQuant.Q6K
+    w = lambda i, rows, cols: X.dequantize(q, st[i].bytes).double().view(rows, cols)
+    g, u = x @ w(0, inter, hidden).T, x @ w(1, inter, hidden).T
+    return (g / (1 + (-g).exp()) * u) @ w(2, hidden, inter).T
+
+
+@pytest.mark.parametrize("hidden,inter", WHOLE)
+def test_intermediate_rows_scaled_by_superblocks(hidden, inter):
+    # every pass width, one token's row being the same bits in all of them; rows with marked superblocks of the activations and
+    # an infinity; the dense block, whose one and two tokens are normalised inside gate/up
+    import torch
+    import llmxabe_amd as X
+
+    q = X.ExpertQuant.Q6K
+    st = [X.QuantTensor(X.synth_quant(q, 9300 + i, hidden * inter, 0.02), q) for i in range(3)]
+    x = X.synth_normal_f32(9310, 19 * hidden, 1.0).view(19, hidden)
+    x[1, 1::2] *= 2.0 ** -40
+    x[6, 300] = 2.0 ** 30
+    x[12, 5] = float("inf")
+    x[17, 2::3] *= 2.0 ** -35
+    finite = [t for t in range(19) if t not in (6, 12)]
+    ref = _ffn64_rows(X, st, x[finite].double(), hidden, inter)
+    same = lambda a, b: np.array_equal(a.cpu().numpy(), b.cpu().numpy(), equal_nan=True)
+
+    def run(rows, live):
+        k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, len(rows)))
+        b = k.shared_only_buffers(False)
+        k.set_valid_tokens(b, live)
+        out = torch.full(rows.shape, 7.0, device="cuda")
+        k.shared_expert(b, *st, rows.reshape(-1).contiguous(), out.view(-1))
+        return out
+
+    alone = torch.cat([run(x[t:t + 1], 1) for t in range(19)])
+    err = ((alone[finite] - ref).abs().max() / ref.abs().max()).item()
+    print(hidden, inter, f"{err:.2e}", flush=True)
+    assert err <= TOL, err
+    assert not alone[12].isfinite().all()
+    for tokens, live in ((2, 2), (3, 3), (4, 3), (5, 5), (8, 7), (16, 16), (17, 16), (19, 19)):
+        got = run(x[:tokens], live)
+        assert same(got[:live], alone[:live]), tokens
+        assert (got[live:] == 7.0).all(), tokens
+    norm = 1.0 + X.synth_normal_f32(9311, hidden, 0.1)
+    x[12, 5], x[11, 7] = 2.0 ** 60, float("inf")
+    for rows in (x[1:2], x[6:8], x[11:13], x[12:13], x[10:13]):
+        rows = rows.contiguous()
+        blk = X.DenseFfnBlock(hidden, inter, len(rows))
+        ffn, l_out = torch.zeros_like(rows), torch.zeros_like(rows)
+        blk.forward(X.DenseFfnLayerWeights(norm, *st), rows, len(rows), ffn, l_out)
+        normed = torch.zeros_like(rows)
+        X.LayerOpsKernels.rms_norm(rows, norm, normed, len(rows), hidden, 1e-6)
+        assert same(blk.normed().view(len(rows), hidden), normed)
+        assert same(ffn, run(normed, len(rows)))
+        assert same(l_out, ffn + rows)
