@@ -357,7 +357,9 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
 // launches are digit_narrow.hip's and, from five tokens on, digit_columns.hip's.  By the geometry and the formats alone, for the same reason.
 // (Scales by groups of sixteen, which gate/up's workgroups make by themselves, cost down ten instructions per row, group and
 // token, and its sums a rounding per group.)  Dense block, us, scales by group / by superblock, hidden 5120, intermediate 17408: one
-// token 54.8 / 50.3, two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105, sixteen 183 / 109.
+// token 54.8 / 50.3 (four layers in turn 60.4 / 57.4), two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105,
+// sixteen 183 / 109.  With 0.4 % of the intermediate values a thousand times the others, whose superblocks the digits do not hold
+// (digit_rests): one 54.0 / 49.7, three 70.5 / 68.7, seven 98.9 / 87.3, sixteen 183 / 125, sixty-three 695 / 448.
 // Where no width loses by it.  Intermediate rows of 32 superblocks and more: shorter ones leave classes of down's without any, and the
 // launch that writes their digits is more than down gains (one / four / eight / forty tokens, 3072 x 8192 29.6 / 39.3 / 49.6 / 133 by
 // group, 24.7 / 39.1 / 38.0 / 105 by superblock; 4096 x 4096 23.4 / 30.4 / 38.6 / 107, 20.6 / 31.4 / 36.0 / 101; 4096 x 2304 19.6 /
@@ -846,7 +848,7 @@ static int shared_digits(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buff
   if (columns) XABE_TRY(launch_digit_columns(k, 2, a, n, s));
   else if (shared_makes(k, gate.quant, up.quant, down.quant, n)) XABE_TRY(launch_digit_up(k, a, n, s));
   else XABE_TRY(launch_digit_rows(k, kRowsShared, gate.quant, 2, a, n, s));
-  if (whole && (columns || !digit_down_makes(k, n))) XABE_TRY(launch_digitize_rows(s, a.out, g.intermediate, n, b->shared_inter_d, b->shared_inter_e));
+  if (whole && (columns || !digit_down_makes(k, n))) XABE_TRY(launch_digitize_rows(s, a.out, g.intermediate, n, b->shared_inter_d, b->shared_inter_e, true));
   a.w0 = static_cast<const uint8_t*>(down.bytes);
   a.w1 = nullptr;
   a.w_bytes = down.len;

@@ -159,9 +159,10 @@ __global__ void __launch_bounds__(512, 2) k_digit_columns(RowsArgs a) {
         for (int o = 0; o < NO; ++o)
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
-            e[o][u] = scales[8 * o + 4 * u + g];
-            dead[o][u] = e[o][u] != e[o][u];
-            marked |= dead[o][u];
+            const float scale = scales[8 * o + 4 * u + g];
+            e[o][u] = __builtin_fabsf(scale);
+            dead[o][u] = scale != scale;
+            marked |= !(scale >= 0.0f);
           }
         // Tokens whose superblock is marked: its halves' plain sums into the sums of every set here, and zero for what the
         // matrix instructions make of it.  (Not where a set is multiplied: a branch there cost fifty spilled registers.)
@@ -169,15 +170,44 @@ __global__ void __launch_bounds__(512, 2) k_digit_columns(RowsArgs a) {
 #pragma unroll 1
           for (int t = 0; t < n_tok; ++t) {
             const float scale = scales[t];
-            if (scale == scale) continue;
-            // (a lane per row and half: lane 32 h + r; the next set's rows are on their way while one is summed.  SwiGLU's rows have a
-            // marked superblock in about five hundred, so this is met in most passes of eight tokens: a trip to memory for every
-            // eight elements had made down's launch 55 us long, 33 like this)
+            if (scale >= 0.0f) continue;
+            // A few values' rests, a weight of every row for each.  (Dense block of 7 / 16 / 63 tokens, 0.4 % of SwiGLU's values
+            // a thousand times the others, us: 136 / 178 / 585 where such superblocks were summed again whole, 87 / 125 / 448 like this;
+            // normal rows 80 / 114 / 384, 80 / 110 / 366.)
+            if (NM == 1 && scale < 0.0f) {
+              const float4 f = reinterpret_cast<const float4*>(a.x + (size_t)(slot0 + t) * a.K + sb * kSbElems)[lane];
+              const float q4[4] = {f.x, f.y, f.z, f.w};
+              float rest[4];
+              digit_rests(q4, scale, rest);
+              for_rests(rest, [&](int p, float value) __attribute__((always_inline)) {
+                const uint8_t* at = a.w0 + (size_t)(16 * set0) * row_bytes + (size_t)(sb * kQ6KBytes);
+                uint32_t off = (uint32_t)r * row_bytes;
+                asm volatile("" : "+s"(at), "+v"(off));  // (made here, not ahead of the loops and spilled)
+                float own[2][2 * NO];  // zero but for the token's and the half's sums
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                  for (int u = 0; u < 2 * NO; ++u) own[h][u] = t == 4 * u + g && h == p >> 7 ? value : 0.0f;
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                  const float w = q6k_weight(at, off, p);
+                  const float finite = __builtin_isfinite(w) ? w : 0.0f;
+                  if (i + 1 < sets) at += 16 * row_bytes;
+#pragma unroll
+                  for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int u = 0; u < 2 * NO; ++u) acc[i][h][u] = __builtin_fmaf(finite, own[h][u], acc[i][h][u]);
+                }
+              });
+              continue;
+            }
+            // (a lane per row and half: lane 32 h + r; the next set's rows are on their way while one is summed)
             float own[8];
             half_own(a.x + (size_t)(slot0 + t) * a.K + sb * kSbElems, lane >> 5, lane, own);
             SbRaw<kQ6K> raw[2];
             auto fetch = [&](int i) __attribute__((always_inline)) {
-              const int row = row_of(set0 + min(i, sets - 1), r >> 3) + (r & 7);
+              int row = row_of(set0 + min(i, sets - 1), r >> 3) + (r & 7);
+              asm volatile("" : "+v"(row));  // (the rows' offsets are made here, not ahead of the loops: fifty registers)
               sb_read(rows_of(r >> 3) + (size_t)row * row_bytes + (size_t)sb * kQ6KBytes, lane >> 5, raw[i & 1]);
             };
             fetch(0);

@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
     float e[NT], v[NT];
     if constexpr (MADE) {  // (the same while the rows are on their way, out of a slot of their own: no faster)
       const float q[4] = {f[0].x, f[0].y, f[0].z, f[0].w};
-      e[0] = digitize_quads(q, dig);
+      e[0] = digitize_quads<true>(q, dig);
     }
     if (SLOTS == 2 && sb + WAVES < nsb) wait_but<kInstr>();
     else wait_but<0>();
@@ -301,8 +301,31 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
     }
     uint8_t* const slot = slots + buf * kSlot;
     if (sb == nsb - 1 && row0 + rows == a.n_rows) patch_window<kQ6K>(a.w0, a.w_bytes - kQ6KBytes, slot + (rows - 1) * kRow);
+    const uint8_t* const bytes = slot + row * kRow + (((uint32_t)off + (uint32_t)row * row_bytes + (uint32_t)(sb * kQ6KBytes)) & 3u);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {  // (ahead of the superblock's sum: k_digit_columns' order)
+      if (__builtin_expect(e[t] < 0.0f, 0)) {
+        float4 own;
+        if constexpr (MADE) own = f[t];
+        else own = *reinterpret_cast<const float4*>(a.x + (size_t)(slot0 + min(t, n_tok - 1)) * a.K + sb * kSbElems + lane * 4);
+        const float q4[4] = {own.x, own.y, own.z, own.w};
+        float rest[4], sum = 0.0f;
+        digit_rests(q4, e[t], rest);
+#pragma unroll
+        for (int q = 0; q < kTurns; ++q)
+          if (q == n % kTurns) sum = acc[q][t];
+        for_rests(rest, [&](int p, float value) __attribute__((always_inline)) {
+          const float w = q6k_weight(bytes, 0, p);
+          if (p >> 7 == half && __builtin_isfinite(w)) sum = __builtin_fmaf(w, value, sum);
+        });
+#pragma unroll
+        for (int q = 0; q < kTurns; ++q)
+          if (q == n % kTurns) acc[q][t] = sum;
+        e[t] = -e[t];
+      }
+    }
     SbRaw<kQ6K> raw;
-    sb_read_slot(slot + row * kRow + (((uint32_t)off + (uint32_t)row * row_bytes + (uint32_t)(sb * kQ6KBytes)) & 3u), half, raw);
+    sb_read_slot(bytes, half, raw);
     if constexpr (kHeld) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) ax[j] = x.high(j & 3, j >> 2, 0);

@@ -79,7 +79,8 @@ __device__ __forceinline__ void store_digit_group(float v, int row, uint8_t* xd,
 
 // host side
 int digit_rows_configure();
-int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
+// (`rests`: with negative scales, which down of `shared_whole` matrices takes: digit_rests)
+int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe, bool rests = false);
 int launch_digitize_groups(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe);
 // `units`: dispatch blocks, or the tokens of a single matrix
 int launch_digit_rows(const xabe_moe_kernels* k, int mode, int quant, int nm, RowsArgs a, size_t units, hipStream_t s);
@@ -88,7 +89,8 @@ void rows_shape(RowsArgs& a, int quant, int nm);
 
 // Down of a large single Q6_K matrix, whose activations are scaled by superblocks (digit_columns.hip): classes are superblock
 // mod 32, class c in quarter c / 8; a quarter adds its classes in order, each half of the superblocks by itself, then the two
-// halves; the quarters are added in pairs.
+// halves; the quarters are added in pairs.  Values that the digits of a superblock do not hold exactly, a few of them, are added to
+// the class ahead of the superblock's sum (digit_rests).
 constexpr int kWholeQuarters = 4;
 constexpr int kWholeMaxSb = 21, kWholeMinInterSb = 32;  // superblocks of the hidden size at most, of the intermediate size at least
 int digit_columns_configure();

@@ -23,6 +23,7 @@ namespace xabe {
 
 // Digits of fp32 rows, scaled by superblocks: a wavefront per superblock; elements past the end of the row are zeros.
 // (A thread per group of sixteen took 4.7 us for a single row, this 2.)
+template <bool RESTS>
 __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__ x, int K, int nsb, int rows, uint8_t* __restrict__ xd,
                                                        float* __restrict__ xe) {
   const int i = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)__lane_id();
@@ -31,7 +32,7 @@ __global__ void __launch_bounds__(256) k_digitize_rows(const float* __restrict__
   const float4 f = reinterpret_cast<const float4*>(x + (size_t)row * K)[min(at, K / 4 - 1)];
   const bool in = 4 * at < K;
   const float v[4] = {in ? f.x : 0.0f, in ? f.y : 0.0f, in ? f.z : 0.0f, in ? f.w : 0.0f};
-  const float scale = digitize_quads(v, xd + (size_t)i * kSbDigitBytes);
+  const float scale = digitize_quads<RESTS>(v, xd + (size_t)i * kSbDigitBytes);
   if (lane == 0) xe[i] = scale;
 }
 
@@ -664,9 +665,9 @@ int digit_rows_configure() {
   return once.run(dev, digit_rows_set_limits);
 }
 
-int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe) {
+int launch_digitize_rows(hipStream_t s, const float* x, size_t K, size_t rows, uint8_t* xd, float* xe, bool rests) {
   const size_t nsb = digit_superblocks(K), n = rows * nsb;
-  hipLaunchKernelGGL(k_digitize_rows, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
+  hipLaunchKernelGGL(rests ? k_digitize_rows<true> : k_digitize_rows<false>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, x, (int)K, (int)nsb, (int)rows, xd, xe);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }

@@ -23,6 +23,10 @@
 // round sixteen times: measured against float64, 1e-7 of the outputs' peak, the lanes' fp32 sums 1.7e-7.  (Four digits
 // held values within 2^6 of the largest only: beside an outlier of 3e4 whose codes are zero the rest of the row was off
 // by 7e-6 of its peak.)
+// SwiGLU's rows in whole superblocks have such a value in one superblock of four hundred for normal rows, and in one of
+// twelve where 0.4 % of them are a thousand times the others.  There up to kRests values are held to whole numbers all the same and
+// what is left of them, exactly, is added weight by weight (digit_rests): a multiply-add and a few bytes per row and
+// value instead of 256 multiply-adds per row.  More than that, infinities, NaN and magnitudes near the ends are marked as above.
 //
 // Why this form: one conversion and one multiply-add per weight and token on a 16-lane SIMD (4.9 vector instructions
 // per weight in all) bound every batch wider than a few tokens.  Here a weight costs ~1.3 instructions to unpack
@@ -146,7 +150,10 @@ __device__ __forceinline__ float digitize_superblock(const float (&x)[16], int p
   return digit_scale(mag, e, row16_any(inexact));
 }
 
-// A superblock whose sixty-four quads of elements the wavefront's lanes hold: digits to `base`; returns its scale.
+// A superblock whose sixty-four quads of elements the wavefront's lanes hold: digits to `base`; returns its scale.  RESTS: where
+// at most kRests values are not held exactly, the digits are of whole numbers beside theirs, and the scale is negative (digit_rests).
+constexpr int kRests = 8;
+template <bool RESTS = false>
 __device__ __forceinline__ float digitize_quads(const float (&x)[4], uint8_t* base) {
   const int lane = (int)__lane_id();
   uint32_t mag = 0;
@@ -160,7 +167,47 @@ __device__ __forceinline__ float digitize_quads(const float (&x)[4], uint8_t* ba
   uint8_t* d = base + digit_group_offset(lane >> 2) + 4 * (lane & 3);
 #pragma unroll
   for (int p = 0; p < 6; ++p) *reinterpret_cast<uint32_t*>(d + 16 * p) = plane[p];
-  return digit_scale(mag, e, __builtin_amdgcn_ballot_w64(inexact) != 0);
+  const uint64_t any = __builtin_amdgcn_ballot_w64(inexact);
+  if constexpr (RESTS) {
+    if (any == 0) return digit_scale(mag, e, false);
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = __builtin_ldexpf(x[i], shift);
+      n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(__builtin_rintf(v) != v));
+    }
+    return -digit_scale(mag, e, n > kRests);
+  }
+  return digit_scale(mag, e, any != 0);
+}
+// What the digits of a superblock with a negative scale leave of its values, the lane's quad: exact, and zero but for a few.
+__device__ __forceinline__ void digit_rests(const float (&x)[4], float scale, float (&rest)[4]) {
+  const int shift = 159 - (int)(__builtin_bit_cast(uint32_t, scale) >> 23 & 0xffu);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float v = __builtin_ldexpf(x[i], shift), low = __builtin_fmaf(__builtin_rintf(v * 0x1p-16f), -65536.0f, v);  // (digits_of)
+    rest[i] = __builtin_ldexpf(low - __builtin_truncf(low), -shift);
+  }
+}
+// Calls add(element, rest) for each, in the order that every kernel adds them in.
+template <typename Add>
+__device__ __forceinline__ void for_rests(const float (&rest)[4], Add add) {
+  float v = rest[0], r1 = rest[1], r2 = rest[2], r3 = rest[3];
+#pragma unroll 1
+  for (int i = 0; i < 4; ++i, v = r1, r1 = r2, r2 = r3) {
+#pragma unroll 1
+    for (uint64_t m = __builtin_amdgcn_ballot_w64(v != 0.0f); m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      add(4 * l + i, lane_bcast(v, l));
+    }
+  }
+}
+// Element p's weight out of its superblock's bytes, which lie at sb + off.
+__device__ __forceinline__ float q6k_weight(const uint8_t* sb, uint32_t off, int p) {
+  const int h = p >> 7, k = p >> 5 & 3, l = p & 31;
+  const int low = (sb + (64 * h + 32 * (k & 1) + l))[off] >> (4 * (k >> 1)) & 15, high = (sb + (128 + 32 * h + l))[off] >> (2 * k) & 3;
+  const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(sb + 208 + off));
+  return d * (float)(int8_t)(sb + (192 + 8 * h + 2 * k + (l >> 4)))[off] * (float)((low | high << 4) - 32);
 }
 
 // The same with the scale of every group, sixteen at `scales`.

@@ -207,3 +207,43 @@ def test_intermediate_rows_scaled_by_superblocks(hidden, inter):
         assert same(blk.normed().view(len(rows), hidden), normed)
         assert same(ffn, run(normed, len(rows)))
         assert same(l_out, ffn + rows)
+
+
+@pytest.mark.parametrize("hidden,inter", [(2048, 8192), (5376, 8960)])
+@pytest.mark.parametrize("small", [1, 8, 9, 40])
+def test_values_far_below_their_superblocks_largest(hidden, inter, small):
+    # intermediate rows whose superblocks hold one large value, which down's weights ignore, and `small` ones 2^-32 of it, which
+    # the 48-bit numbers hold to fourteen bits: up to eight are added by themselves, more take the whole superblock along.  float64
+    # within TOL, and the same bits at every width
+    import torch
+    import llmxabe_amd as X
+
+    q = X.ExpertQuant.Q6K
+    st = [X.synth_quant(q, 9400 + i, hidden * inter, 0.02) for i in range(3)]
+    factor = torch.zeros(inter, device="cuda")
+    sbs = (0, 5, inter // 256 - 1)
+    for sb in sbs:
+        factor[256 * sb + 7] = 2.0 ** 16
+        factor[256 * sb + 16 + 5 * torch.arange(small, device="cuda")] = 1.0
+    for i in (0, 1):
+        d = st[i].view(inter, hidden // 256, 210)[:, :, 208:]
+        d.copy_((d.contiguous().view(torch.float16).float() * factor.view(-1, 1, 1)).half().view(torch.uint8))
+    st[2].view(hidden, inter // 256, 210)[:, list(sbs), 192] = 0   # the scale of the large values' group
+    st = [X.QuantTensor(t, q) for t in st]
+    x = X.synth_normal_f32(9410, 19 * hidden, 1.0).view(19, hidden)
+    ref = _ffn64_rows(X, st, x.double(), hidden, inter)
+
+    def run(n):
+        k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, n))
+        b = k.shared_only_buffers(False)
+        k.set_valid_tokens(b, n)
+        out = torch.full((n, hidden), 7.0, device="cuda")
+        k.shared_expert(b, *st, x[:n].reshape(-1).contiguous(), out.view(-1))
+        return out
+
+    rows = run(19)
+    err = ((rows - ref).abs().max(1).values / ref.abs().max(1).values).max().item()
+    print(hidden, inter, small, f"{err:.2e}", flush=True)
+    assert err <= TOL, err
+    for n in (1, 2, 3, 4, 5, 8, 16):
+        assert torch.equal(run(n).view(torch.int32), rows[:n].view(torch.int32)), n
