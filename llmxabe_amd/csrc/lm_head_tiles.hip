@@ -61,9 +61,9 @@ __device__ __forceinline__ void wait_but(bool last) {
 }
 
 // The sums the wavefronts left at red[wave][half][token][32], added and stored.  HALVES 2: one after the other, each half of
-// the superblocks by itself, then the two (k_lm_head_quant's order); otherwise in pairs.  `plain(v, t, row)`: what the logit v is replaced by.
-template <int HALVES, int TOKENS, typename Plain>
-__device__ __forceinline__ void head_reduce(const float* red, const HeadShare& sh, const LmHeadArgs& a, int row0, Plain plain) {
+// the superblocks by itself, then the two (k_lm_head_quant's order); otherwise in pairs.
+template <int HALVES, int TOKENS>
+__device__ __forceinline__ void head_reduce(const float* red, const HeadShare& sh, const LmHeadArgs& a, int row0) {
   constexpr int kStride = HALVES * TOKENS * kTileRows;
 #pragma unroll 1
   for (int i = threadIdx.x; i < a.nt * kTileRows; i += (int)blockDim.x) {
@@ -86,9 +86,36 @@ __device__ __forceinline__ void head_reduce(const float* red, const HeadShare& s
         total[h] = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       }
     }
-    if (row < sh.row_hi) a.out[(size_t)(a.t0 + t) * a.vocab + row] = plain(HALVES == 2 ? total[0] + total[HALVES - 1] : total[0], t, row);
+    if (row < sh.row_hi) a.out[(size_t)(a.t0 + t) * a.vocab + row] = HALVES == 2 ? total[0] + total[HALVES - 1] : total[0];
   }
 }
+
+// Activations of the tokens whose superblock is marked, as they came: the LDS behind the sums holds those of the first PLACES
+// tokens of every wavefront, 1 KB each, for the whole launch.  Fetched per tile they would be waited for behind the requested rows, and
+// every wavefront of the workgroup waits for the one that sums a superblock again, so that it takes its weights, too, from where they
+// are: registers, or the slot.  248 320 x 2048, one marked superblock in the pass, us, weights and activations fetched / this: Q8_0 at 1
+// / 3 / 8 / 16 tokens 238 / 240 / 220 / 217, now 98 / 101 / 130 / 157; Q6_K at 5 / 8 / 16 174 / 175 / 205, now 137 / 137 / 172.
+template <int PLACES>
+struct MarkedRows {
+  const float* at;  // the wavefront's
+  uint32_t marks;
+  // (the wavefronts are done with the digits that lay there)
+  __device__ __forceinline__ void fill(const LmHeadArgs& a, const HeadShare& sh, float* lds, uint32_t marks_) {
+    float* const mine = lds + sh.wave * PLACES * kSbElems;
+    at = mine;
+    marks = marks_;
+    int place = 0;
+#pragma unroll 1
+    for (uint32_t m = marks; m != 0 && place < PLACES; m &= m - 1, ++place)
+      reinterpret_cast<float4*>(mine + place * kSbElems)[sh.lane] =
+          reinterpret_cast<const float4*>(a.x + (size_t)(a.t0 + __builtin_ctz(m)) * a.K + sh.wave * kSbElems)[sh.lane];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  // which place a token has (PLACES or more: none)
+  __device__ __forceinline__ int place(int t) const { return marks >> t & 1 ? __builtin_popcount(marks & ((1u << t) - 1)) : PLACES; }
+};
 
 // ------------------------------------------------------------------------------------------------
 // bf16.  A fp32 activation is the sum of three bf16 numbers, each the leading eight bits of what is left, so every product
@@ -98,20 +125,33 @@ __device__ __forceinline__ void head_reduce(const float* red, const HeadShare& s
 // that of the outputs 0.76e-7, the lanes 1.24e-7).
 // A lane's pieces of an activation reach down to bf16's (fp32's) smallest exponent: columns whose largest is below 2^-30
 // are multiplied by 2^90 first, and those with a value that would lose its last piece all the same are marked by a NaN
-// scale.  A logit that is not finite, by a mark, an infinity or a NaN, is summed again by fp32 multiply-adds, so that it is
-// what those make of it.
+// scale.  A sum of 256 columns that is not finite, by a mark, an infinity or a NaN, is made again by fp32 multiply-adds, so
+// that it is what those make of it (one such token, 1 / 3 / 8 / 16 tokens 195 / 198 / 211 / 226 us; the whole row again by a lane per logit
+// 1350 to 1380).
 // ------------------------------------------------------------------------------------------------
 constexpr int kBf16Slot = kTileRows * 512;
 
-__device__ __forceinline__ float bf16_logit(const LmHeadArgs& a, int t, int row) {
-  const uint16_t* w = reinterpret_cast<const uint16_t*>(a.w) + (size_t)row * a.K;
-  const float* x = a.x + (size_t)(a.t0 + t) * a.K;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 1
-  for (int k = 0; k < a.K; k += 8)
+// 256 columns by multiply-adds out of a lane's weights and its token's activations `x` (uniform); the four quarters' sums are added
+// in pairs.  Scalar loads: vector ones would be waited for behind the rows that are on their way.
+__device__ __forceinline__ float bf16_plain(const float* x, const v8b_t (&w)[8], int g) {
+  typedef const __attribute__((address_space(4))) float* scalars_t;
+  scalars_t at = (scalars_t)(uintptr_t)x;
+  float u[4] = {0, 0, 0, 0};  // by quarter; the lane's own is used
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = __builtin_fmaf(__builtin_bit_cast(float, (uint32_t)w[k + j] << 16), x[k + j], s[j]);
-  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  for (int j = 0; j < 8; ++j) {
+    v4u_t own = __builtin_bit_cast(v4u_t, w[j]);
+    // (step by step: all weights as fp32, and all loads, at once were 140 spilled registers)
+    asm volatile("" : "+s"(at), "+v"(own), "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float f = __builtin_bit_cast(float, i & 1 ? own[i / 2] & 0xffff0000u : own[i / 2] << 16);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) u[q] = __builtin_fmaf(f, at[32 * j + 8 * q + i], u[q]);
+    }
+  }
+  float v = g & 2 ? (g & 1 ? u[3] : u[2]) : (g & 1 ? u[1] : u[0]);
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
 }
 
 __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
@@ -189,8 +229,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) scale[i] = __shfl(down, 4 * sh.g + i, 64);
   auto reduce = [&](int n) __attribute__((always_inline)) {
-    head_reduce<1, 16>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
-                       [&](float v, int t, int row) __attribute__((always_inline)) { return __builtin_isfinite(v) ? v : bf16_logit(a, t, row); });
+    head_reduce<1, 16>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n);
   };
 
 #pragma unroll 1
@@ -216,11 +255,33 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
         hi[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[0][j], w[j], zero, 0, 0, 0);
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[1][j], w[j], lo, 0, 0, 0);
       }
+      float out[4];
+      bool finite = true;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float sum = ((hi[0][i] + hi[1][i]) + (hi[2][i] + hi[3][i])) + ((hi[4][i] + hi[5][i]) + (hi[6][i] + hi[7][i]));
-        mine[(4 * sh.g + i) * kTileRows + 16 * s + sh.r] = (sum + lo[i]) * scale[i];
+        out[i] = (sum + lo[i]) * scale[i];
+        finite = finite && __builtin_isfinite(out[i]);
       }
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!finite && row0 + 16 * s + sh.r < sh.row_hi) != 0, 0)) {
+        uint32_t m = 0;  // tokens with a sum that is not finite
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint64_t lanes = __builtin_amdgcn_ballot_w64(!__builtin_isfinite(out[i]));
+#pragma unroll
+          for (int g = 0; g < 4; ++g) m |= (uint32_t)((lanes >> (16 * g) & 0xffff) != 0) << (4 * g + i);
+        }
+#pragma unroll 1
+        for (m &= (1u << a.nt) - 1; m != 0; m &= m - 1) {
+          const int t = __builtin_ctz(m);
+          const float plain = bf16_plain(a.x + (size_t)(a.t0 + t) * a.K + sh.wave * 256, w, sh.g);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (t == 4 * sh.g + i && !__builtin_isfinite(out[i])) out[i] = plain;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[(4 * sh.g + i) * kTileRows + 16 * s + sh.r] = out[i];
     }
     __syncthreads();
   }
@@ -238,6 +299,11 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
 using Q8Dma = SliceDma<kQ8_0>;
 constexpr int kQ8Digits = 8192;  // LDS of four tokens' digits of a superblock, as the instruction takes them: [block][lane][16]
 
+// Places for marked tokens' activations behind the sums of 4 nq tokens, where the digits were.
+template <int NQ>
+constexpr int kQ8Places = 8 - NQ;
+static_assert(2 * 4 * 4 * kTileRows * 4 + kQ8Places<4> * kSbElems * 4 <= kQ8Digits, "the sums and the places lie where the digits did");
+
 // For which of four tokens a lane of quarter g, token g's, holds a NaN.
 __device__ __forceinline__ uint32_t marked_tokens(float v) {
   const uint64_t lanes = __builtin_amdgcn_ballot_w64(v != v);
@@ -247,19 +313,21 @@ __device__ __forceinline__ uint32_t marked_tokens(float v) {
   return m;
 }
 
-// Token t's superblock by multiply-adds, as a lane of quarter g holds it: eight columns of every block; the four quarters'
-// sums are added in pairs.
-__device__ __forceinline__ float q8_plain(const LmHeadArgs& a, int t, int row, int sb, int g) {
-  const uint8_t* w = a.w + (size_t)row * (a.K / 32 * kQ8Bytes) + (size_t)sb * (8 * kQ8Bytes);
-  const float* x = a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems + 8 * g;
+// A superblock by multiply-adds out of a lane's codes and its token's activations `x` (the superblock's, plus 8 g): eight columns of every
+// block; the four quarters' sums are added in pairs.
+__device__ __forceinline__ float q8_plain(const float* x, const uint32_t (&code)[8][2], const uint32_t (&d)[4]) {
   float v = 0.0f;
-#pragma unroll 4
-  for (int b = 0; b < 8; ++b) {
-    const float d = f16_bits_to_f32(*reinterpret_cast<const uint16_t*>(w + kQ8Bytes * b));
-    int8_t c[8];
-    __builtin_memcpy(c, __builtin_assume_aligned(w + kQ8Bytes * b + 2 + 8 * g, 2), 8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v = __builtin_fmaf(x[32 * b + i], d * (float)c[i], v);
+  for (int b = 0; b < 8; ++b) {
+    const float ws = f16_bits_to_f32(d[b / 2] >> (16 * (b & 1)) & 0xffffu);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float4 f = *reinterpret_cast<const float4*>(x + 32 * b + 4 * i);
+      v = __builtin_fmaf(f.x, ws * (float)(int8_t)code[b][i], v);
+      v = __builtin_fmaf(f.y, ws * (float)(int8_t)(code[b][i] >> 8), v);
+      v = __builtin_fmaf(f.z, ws * (float)(int8_t)(code[b][i] >> 16), v);
+      v = __builtin_fmaf(f.w, ws * (float)(int8_t)(code[b][i] >> 24), v);
+    }
   }
   v += __shfl_xor(v, 16, 64);
   return v + __shfl_xor(v, 32, 64);
@@ -358,9 +426,15 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
     e[q] = 16.0f * q8_digits(a, sh, 4 * q, f[q], rest + (size_t)sh.wave * kQ8Digits, op[q]);  // (2^36 of the digits, 2^32 of the scale)
   }
   __syncthreads();
+  MarkedRows<kQ8Places<NQ>> kept;
+  {
+    uint32_t m = 0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) m |= marked_tokens(e[q]) << (4 * q);
+    kept.fill(a, sh, red + 2 * sh.waves * kRed, m & ((1u << a.nt) - 1));
+  }
   auto reduce = [&](int n) __attribute__((always_inline)) {
-    head_reduce<1, 4 * NQ>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
-                        [](float v, int, int) __attribute__((always_inline)) { return v; });
+    head_reduce<1, 4 * NQ>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n);
   };
 
 #pragma unroll 1
@@ -436,7 +510,9 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
       for (; __builtin_expect(m != 0, 0); m &= m - 1) {
         const int t = __builtin_ctz(m);
         if (t >= a.nt) break;
-        const float plain = q8_plain(a, t, min(row0 + 16 * s + sh.r, a.vocab - 1), sb, sh.g);
+        const int place = kept.place(t);
+        const float plain = place < kQ8Places<NQ> ? q8_plain(kept.at + place * kSbElems + 8 * sh.g, code, d)
+                                                  : q8_plain(a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems + 8 * sh.g, code, d);
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
           if (t == 4 * q + sh.g && out[q] != out[q]) out[q] = plain;
@@ -461,6 +537,9 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
 // ------------------------------------------------------------------------------------------------
 using Q6Dma = SliceDma<kQ6K>;
 constexpr int kQ6Digits = 8 * kSbDigitBytes;  // LDS of eight tokens' digits of a superblock
+template <int NO>
+constexpr int kQ6Places = 12 - 4 * NO;  // (kQ8Places)
+static_assert(2 * 2 * 8 * 2 * kTileRows * 4 + kQ6Places<2> * kSbElems * 4 <= kQ6Digits, "the sums and the places lie where the digits did");
 
 template <int NO>
 __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
@@ -508,9 +587,10 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   __syncthreads();
+  MarkedRows<kQ6Places<NO>> kept;
+  kept.fill(a, sh, red + 2 * sh.waves * kRed, marks);
   auto reduce = [&](int n) __attribute__((always_inline)) {
-    head_reduce<2, 8 * NO>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n,
-                        [](float v, int, int) __attribute__((always_inline)) { return v; });
+    head_reduce<2, 8 * NO>(red + (size_t)(n & 1) * sh.waves * kRed, sh, a, sh.row_lo + kTileRows * n);
   };
   const uint32_t shift[2] = {4u - 2u * (uint32_t)(g >> 1), 2u * (uint32_t)(g >> 1)};
 
@@ -520,6 +600,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
     float* const buf = red + (size_t)(n & 1) * sh.waves * kRed;
     const bool last = n + 1 == sh.tiles;
     float* const mine = buf + sh.wave * kRed;
+    SbRaw<kQ6K> raw;  // of a marked superblock, a lane per row and half: lane 32 h + 16 s + r
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       wait_but<Q6Dma::kInstr>(last);
@@ -529,6 +610,8 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
       }
       Q6Quarter w;
       w.read(slot + s * Q6Dma::kRunBytes + r * (Q6Dma::kP * 16), (uint32_t)(sb & 1) * 2, g);  // (rows are whole words)
+      if (__builtin_expect(marks != 0, 0) && (s == 0 || (sh.lane & 16)))
+        sb_read_slot(slot + s * Q6Dma::kRunBytes + r * (Q6Dma::kP * 16) + (sb & 1) * 2, sh.lane >> 5, raw);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (s == 1 && n > 0) reduce(n - 1);
       if (!last) request(row0 + kTileRows, s);
@@ -544,26 +627,20 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
           planes_dot(op[o][2 * h], op[o][2 * h + 1], hi, lo, eo, out[h][o]);
         }
       }
-      for (uint32_t m = marks; __builtin_expect(m != 0, 0); m &= m - 1) {
-        const int t = __builtin_ctz(m), row = min(row0 + 16 * s + r, a.vocab - 1);
-        SbRaw<kQ6K> raw;  // (a lane per row and half: lane 32 h + r)
-        sb_read(a.w + (size_t)row * row_bytes + (size_t)sb * kQ6KBytes, sh.lane >> 5, raw);
-        const float plain = half_fp32(raw, a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems, sh.lane >> 5, sh.lane);
-        const float half[2] = {__shfl(plain, r, 64), __shfl(plain, 32 + r, 64)};
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int o = 0; o < NO; ++o)
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-              if (t == 8 * o + 4 * u + g) out[h][o][u] = half[h];
-      }
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int o = 0; o < NO; ++o)
 #pragma unroll
           for (int t = 0; t < 2; ++t) mine[(h * 8 * NO + 8 * o + 4 * t + g) * kTileRows + 16 * s + r] = out[h][o][t];
+    }
+    for (uint32_t m = marks; __builtin_expect(m != 0, 0); m &= m - 1) {  // both sets' rows in place of the NaNs
+      const int t = __builtin_ctz(m), place = kept.place(t);
+      float own[8];
+      if (place < kQ6Places<NO>) half_own(kept.at + place * kSbElems, sh.lane >> 5, sh.lane, own);
+      else half_own(a.x + (size_t)(a.t0 + t) * a.K + sb * kSbElems, sh.lane >> 5, sh.lane, own);
+      opaque(raw);
+      mine[((sh.lane >> 5) * 8 * NO + t) * kTileRows + (sh.lane & 31)] = half_fp32_all<kQ6K>(raw, own, HalfOrder{});
     }
     __syncthreads();
   }

@@ -170,6 +170,41 @@ def test_passes_of_up_to_sixteen_tokens(oracle, X, fmt, vocab, hidden, tokens):
     assert np.array_equal(bad[1:tokens - 1].view(np.uint32), got[1:tokens - 1].view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q6K", "Bf16"])
+@pytest.mark.parametrize("vocab,hidden,tokens", [(70, 512, 4), (2049, 2048, 8), (45, 1024, 11), (300, 2048, 16)])
+def test_many_tokens_with_marked_columns(oracle, X, fmt, vocab, hidden, tokens):
+    # more tokens than a wavefront keeps the rows of whose columns neither pieces nor digits hold, in one superblock and in all; a
+    # weight row of infinities.  float64 within 5e-7 of the peak, the same bits alone, and the rest of the rows untouched
+    import torch
+
+    fmt = getattr(X.HeadFormat, fmt)
+    w, host = _weights(X, oracle, fmt, vocab, hidden, 35000 + vocab)
+    x = X.synth_normal_f32(35001, tokens * hidden, 1.0).view(tokens, hidden)
+    x[:, 256:512:3] *= 2.0 ** -110
+    x[tokens - 1, ::5] *= 2.0 ** -110
+    run = lambda rows: _run(X, X.LmHeadKernels(X.LmHeadGeometry(hidden, vocab, len(rows))), w, fmt, rows.contiguous(), len(rows))
+    got = run(x)
+    for t in range(tokens):
+        ref = host.astype(np.float64) @ x[t].cpu().numpy().astype(np.float64)
+        err = np.abs(got[t] - ref).max() / np.abs(ref).max()
+        assert err <= 5e-7, (str(fmt), t, err)
+        assert np.array_equal(run(x[t:t + 1])[0].view(np.uint32), got[t].view(np.uint32)), t
+    row = 33
+    raw = w.bytes if hasattr(w, "bytes") else w
+    per = raw.numel() // vocab
+    if fmt == X.HeadFormat.Bf16:
+        raw.view(torch.bfloat16).view(vocab, hidden)[row] = float("inf")
+    else:   # the first scale of the row
+        at = row * per + (208 if fmt == X.HeadFormat.Q6K else 0)
+        raw.view(torch.uint8)[at:at + 2] = torch.tensor([0x00, 0x7c], dtype=torch.uint8, device="cuda")
+    bad = run(x)
+    assert not np.isfinite(bad[:, row]).any()
+    keep = np.arange(vocab) != row
+    assert np.array_equal(bad[:, keep].view(np.uint32), got[:, keep].view(np.uint32))
+    for t in (0, tokens - 1):
+        assert np.array_equal(run(x[t:t + 1])[0], bad[t], equal_nan=True), t
+
+
 def test_forward_error_paths(oracle, X):
     import torch
 
