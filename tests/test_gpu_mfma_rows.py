@@ -90,7 +90,10 @@ def test_gate_up_items_of_two_to_three_rounds(X, experts):
 
 @pytest.mark.parametrize("quant", ["q6k", "q8_0"])
 @pytest.mark.parametrize("hidden,inter,widths", [(256, 16384, (383, 384, 385, 1000)), (512, 256, (64, 65, 97, 193)),
-                                                 (1280, 11008, (576, 640, 769))])
+                                                 (1280, 11008, (576, 640, 769)),
+                                                 # 128 tiles of gate/up in one row (wide from 97 tokens), 128 parts of down in two (from 193)
+                                                 (256, 16384, (95, 96, 97, 192)), (4096, 12288, (192, 193, 384)),
+                                                 (5120, 17408, (96, 97, 192, 193, 320))])
 def test_unrouted_widths_across_the_rule(X, quant, hidden, inter, widths):
     import torch
 
@@ -150,4 +153,35 @@ def test_long_down_contractions_in_parts(X, quant, hidden, inter):
             assert (t[live:] == -7.0).all()
         rows.append(ffn[:64])
     for wider in rows[1:]:   # a token's row does not depend on the batch around it
+        assert torch.equal(wider.view(torch.int32), rows[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("quant", ["q6k", "q8_0"])
+@pytest.mark.parametrize("hidden,inter", [(512, 6912), (4096, 12288)])
+def test_few_live_tokens_in_buffers_of_more_than_1024(X, quant, hidden, inter):
+    # there the down contraction is one chain at every width: float32 at the tolerance above, a row the same bits in every pass
+    import torch
+
+    weights, tokens = _weights(X, quant, quant, hidden * inter), 1025
+    norm = 1.0 + X.synth_normal_f32(4, hidden, 0.1)
+    x = X.synth_normal_f32(9, tokens * hidden, 1.0).view(tokens, hidden)
+    k = X.MoeKernels(X.MoeGeometry(1, 1, hidden, inter, 32, 257))
+    k.disable_tensor_cores()
+    b = k.shared_only_buffers(True)
+    blk = X.DenseFfnBlock(hidden, inter, tokens)
+    rows = []
+    for live in (65, 257, 1025):
+        ffn, l_out = torch.full_like(x, -7.0), torch.full_like(x, -7.0)
+        blk.publish_tokens(live)
+        blk.forward(X.DenseFfnLayerWeights(norm, *weights), x, live, ffn, l_out)
+        n = min(live, 257)
+        want = torch.zeros(257, hidden, device="cuda")
+        k.set_valid_tokens(b, n)
+        k.shared_expert(b, *weights, blk.normed().view(tokens, hidden)[:257].contiguous(), want)
+        torch.cuda.synchronize()
+        _close(ffn[:n], want[:n])
+        assert torch.equal(l_out[:live], ffn[:live] + x[:live])
+        assert (ffn[live:] == -7.0).all() and (l_out[live:] == -7.0).all()
+        rows.append(ffn[:65].clone())
+    for wider in rows[1:]:
         assert torch.equal(wider.view(torch.int32), rows[0].view(torch.int32))
