@@ -360,12 +360,11 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
 // token 54.8 / 50.3 (four layers in turn 60.4 / 57.4), two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105,
 // sixteen 183 / 109.  With 0.4 % of the intermediate values a thousand times the others, whose superblocks the digits do not hold
 // (digit_rests): one 54.0 / 49.7, three 70.5 / 68.7, seven 98.9 / 87.3, sixteen 183 / 125, sixty-three 695 / 448.
-// Where no width loses by it.  Intermediate rows of 32 superblocks and more: shorter ones leave classes of down's without any, and the
-// launch that writes their digits is more than down gains (one / four / eight / forty tokens, 3072 x 8192 29.6 / 39.3 / 49.6 / 133 by
-// group, 24.7 / 39.1 / 38.0 / 105 by superblock; 4096 x 4096 23.4 / 30.4 / 38.6 / 107, 20.6 / 31.4 / 36.0 / 101; 4096 x 2304 19.6 /
-// 24.7 / 30.6 / 73, 16.9 / 25.7 / 34.2 / 96).  Hidden sizes of at most 21 superblocks: a tile of down's few-token launch holds 21 rows
-// for each of 256 compute units, and beyond that it is two half-full ones (6144 x 10240 47.5 / 61.2 / 80.1 / 323, 54.8 / 75.3 / 72.3 /
-// 232; 8192 x 28672 at one and four tokens 130 / 160, 145 / 186).
+// Intermediate rows of 32 superblocks and more, where no width but two and four tokens loses by it, and these 2 % (one / two / three / four /
+// eight / forty tokens, 2048 x 8192 23.3 / 25.1 / 30.8 / 30.9 / 41.0 / 110 by group, 22.0 / 24.4 / 30.2 / 31.7 / 29.2 / 80 by superblock;
+// 3072 x 8192 26.7 / 28.7 / 34.1 / 34.0 / 45.4 / 133, 24.7 / 29.3 / 33.5 / 34.8 / 34.6 / 97).  Hidden sizes of at most 21 superblocks: a
+// tile of down's few-token launch holds 21 rows for each of 256 compute units, and beyond that it is two half-full ones (one / four / eight
+// / forty tokens, 6144 x 10240 41.5 / 52.6 / 74 / 330 by group, 49.8 / 69.3 / 67 / 224; 8192 x 28672 127 / 156 / 219 / 1002, 142 / 184 / 186 / 676).
 static bool shared_whole(const xabe_moe_geometry& g, int gate_q, int up_q, int down_q) {
   return gate_q == XABE_QUANT_Q6K && up_q == XABE_QUANT_Q6K && down_q == XABE_QUANT_Q6K && g.hidden % 256 == 0 &&
          g.intermediate % 256 == 0 && g.hidden >= 2048 && g.hidden <= (size_t)kWholeMaxSb * 256 && g.intermediate >= (size_t)kWholeMinInterSb * 256;

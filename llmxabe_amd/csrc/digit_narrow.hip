@@ -210,21 +210,23 @@ __global__ void __launch_bounds__(64 * kUpWaves<NT>, kUpWaves<NT> / 4) k_digit_u
 // ------------------------------------------------------------------------------------------------
 // Down for up to four tokens, the sums of the same classes in the same order.  A workgroup is a tile of rows, as many as give
 // every compute unit one (5120 rows: twenty), a wavefront per superblock mod 16, or mod 8 with two superblocks on their way
-// where the digits leave no room for sixteen slots.  Bound by latency and, with two fifths of the lanes without a row, by vector
+// where four tokens' digits leave no room for sixteen slots (tiles of more than sixteen rows).  Bound by latency and, with two fifths of the lanes without a row, by vector
 // instructions.  One token: the wavefront writes the digits of the superblock that it multiplies itself (100 instructions per
 // superblock and workgroup), where a launch for them is 5 us; two tokens: twice as many instructions are more than that.
 // Dense sibling's 73 MB, us, k_digit_rows with scales by group / eight wavefronts / sixteen: one token 20.3 / 22.3 / 19.3, two
-// 20.5 / 21.6 / 19.4 and 5 for the digits, four 33 / 29.2 / - and 5.
+// 20.5 / 21.6 / 19.4 and 5 for the digits, four 33 / 29.2 / - and 5.  Its block of three tokens 67.5 / 69.5 / 63.5.  Blocks of smaller
+// matrices: three tokens, 2048 x 8192 31.1 / 33.5 / 30.6, 3072 x 8192 34.8 / 37.0 / 34.0, 4096 x 11008 47.8 / 48.9 / 44.0; four tokens 30.8 /
+// 32.8 / 31.5, 34.2 / 35.7 / 35.0, 47.3 / 48.8 / 47.9.
 // ------------------------------------------------------------------------------------------------
-template <int NT, int WAVES, int SLOTS>
+constexpr int kDownRows = 21;  // (five instructions bring 320 pieces, a row is 15)
+template <int NT, int WAVES, int SLOTS, int ROWS>  // ROWS: of a tile at most
 struct DigitDown {
-  static constexpr int kInstr = 5, kSlot = kInstr * 1024;  // DMA instructions of a tile's superblock, 64 pieces each
-  static constexpr int kRows = kSlot / (15 * 16);          // at most
+  static constexpr int kInstr = (15 * ROWS + 63) / 64, kSlot = 15 * ROWS * 16;  // DMA instructions of a tile's superblock, 64 pieces each
   static constexpr int kPer = SLOTS * kSlot + NT * kSbDigitBytes, kLds = kZeroBytes + WAVES * kPer;
 };
-template <int NT, int WAVES, int SLOTS>
+template <int NT, int WAVES, int SLOTS, int ROWS>
 __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a) {
-  using L = DigitDown<NT, WAVES, SLOTS>;
+  using L = DigitDown<NT, WAVES, SLOTS, ROWS>;
   constexpr bool MADE = NT == 1;
   constexpr int kTurns = 32 / WAVES, kRow = 15 * 16, kSlot = L::kSlot, kInstr = L::kInstr;
   extern __shared__ __attribute__((aligned(16))) uint8_t s_down[];
@@ -239,17 +241,22 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
   const uint32_t slots_lds = lds_address(slots), dig_lds = lds_address(dig);
   const size_t off = (size_t)row0 * row_bytes, base = off & ~(size_t)15;
   const uint32_t last = (uint32_t)min((a.w_bytes - base - 16) & ~(size_t)3, (size_t)0xfffffff0u);
-  uint32_t w_off[kInstr];
-#pragma unroll
-  for (int i = 0; i < kInstr; ++i) {
+  auto offset = [&](int i, int lane) __attribute__((always_inline)) {
     const int pc = min(64 * i + lane, 15 * rows - 1);
-    w_off[i] = ((uint32_t)off & 15u) + (uint32_t)(pc / 15) * row_bytes + (uint32_t)(pc % 15) * 16;
+    return ((uint32_t)off & 15u) + (uint32_t)(pc / 15) * row_bytes + (uint32_t)(pc % 15) * 16;
+  };
+  constexpr bool kHeldOffsets = NT < 4 || WAVES < 16;  // (no registers for them otherwise)
+  uint32_t w_off[kHeldOffsets ? kInstr : 1];
+  if constexpr (kHeldOffsets) {
+#pragma unroll
+    for (int i = 0; i < kInstr; ++i) w_off[i] = offset(i, lane);
   }
   // (windows start on words; pieces that would reach past the tensor repeat its end)
   auto request_w = [&](int sb, int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kInstr; ++i)
-      lds_dma_16(a.w0 + base, min((w_off[i] + (uint32_t)(sb * kQ6KBytes)) & ~3u, last), slots_lds + buf * kSlot + i * 1024);
+      if (i + 1 < kInstr || lane < 15 * ROWS - 64 * i)
+        lds_dma_16(a.w0 + base, min(((kHeldOffsets ? w_off[kHeldOffsets ? i : 0] : offset(i, fresh_lane())) + (uint32_t)(sb * kQ6KBytes)) & ~3u, last), slots_lds + buf * kSlot + i * 1024);
   };
   float4 f[MADE ? NT : 1];
   float e_next[NT];
@@ -283,7 +290,6 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
   x.point(dig, dig, s_zero);
   constexpr bool kHeld = WAVES == 8 && !MADE;  // the operands leave LDS for registers, and the next digits are requested with the next rows
   v4i_t ax[kHeld ? 8 : 1], az[kHeld ? 4 : 1];
-  const int row = min(lane & 31, rows - 1);
   const uint64_t live = __builtin_amdgcn_ballot_w64((lane & 31) < rows);
 #pragma unroll 1
   for (int sb = wave, n = 0; sb < nsb; sb += WAVES, ++n) {
@@ -300,6 +306,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
       for (int t = 0; t < NT; ++t) e[t] = e_next[t];
     }
     uint8_t* const slot = slots + buf * kSlot;
+    const int row = min((kHeldOffsets ? lane : fresh_lane()) & 31, rows - 1);
     if (sb == nsb - 1 && row0 + rows == a.n_rows) patch_window<kQ6K>(a.w0, a.w_bytes - kQ6KBytes, slot + (rows - 1) * kRow);
     const uint8_t* const bytes = slot + row * kRow + (((uint32_t)off + (uint32_t)row * row_bytes + (uint32_t)(sb * kQ6KBytes)) & 3u);
 #pragma unroll
@@ -339,7 +346,11 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
         raw, [&](int s, int l, int tg) __attribute__((always_inline)) { return kHeld ? ax[kHeld ? 4 * l + s : 0] : x.high(s, l, tg); },
         [&](int s, int l, int tg) __attribute__((always_inline)) { return kHeld ? az[kHeld ? s : 0] : x.low(s, l, tg); },
         [&](int t, int) __attribute__((always_inline)) { return e[t]; },
-        [&](int t) __attribute__((always_inline)) { return a.x + (size_t)(slot0 + min(t, n_tok - 1)) * a.K + sb * kSbElems; }, v, live);
+        [&](int t) __attribute__((always_inline)) {
+          const float* at = a.x + (size_t)(slot0 + min(t, n_tok - 1)) * a.K + sb * kSbElems;
+          asm volatile("" : "+s"(at));  // (made here, not ahead of the loop and spilled)
+          return at;
+        }, v, live);
 #pragma unroll
     for (int q = 0; q < kTurns; ++q) {  // (the sums stay in registers)
       if (q != n % kTurns) continue;
@@ -379,10 +390,10 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES / 4) k_digit_down(RowsArgs a
 }
 
 // ------------------------------------------------------------------ host side
-template <int NT, int WAVES, int SLOTS>
+template <int NT, int WAVES, int SLOTS, int ROWS = kDownRows>
 static int down_limit() {
-  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_down<NT, WAVES, SLOTS>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, DigitDown<NT, WAVES, SLOTS>::kLds));
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_digit_down<NT, WAVES, SLOTS, ROWS>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, DigitDown<NT, WAVES, SLOTS, ROWS>::kLds));
   return XABE_OK;
 }
 template <int NT, bool NORM>
@@ -393,19 +404,21 @@ static int up_limit() {
 static int digit_narrow_set_limits() {
   XABE_TRY((down_limit<1, 16, 1>()));
   XABE_TRY((down_limit<2, 16, 1>()));
+  XABE_TRY((down_limit<3, 16, 1>()));
   XABE_TRY((down_limit<4, 8, 2>()));
+  XABE_TRY((down_limit<4, 16, 1, 16>()));
   XABE_TRY((up_limit<1, false>()));
   XABE_TRY((up_limit<1, true>()));
   XABE_TRY((up_limit<2, false>()));
   return up_limit<2, true>();
 }
-template <int NT, int WAVES, int SLOTS>
+template <int NT, int WAVES, int SLOTS, int ROWS = kDownRows>
 static int down_go(RowsArgs a, int cus, unsigned passes, hipStream_t s) {
-  using L = DigitDown<NT, WAVES, SLOTS>;
-  const int per_cu = (a.n_rows + cus * L::kRows - 1) / (cus * L::kRows);
+  using L = DigitDown<NT, WAVES, SLOTS, ROWS>;
+  const int per_cu = (a.n_rows + cus * ROWS - 1) / (cus * ROWS);
   a.tile_rows = (a.n_rows + cus * per_cu - 1) / (cus * per_cu);
   const unsigned tiles = (unsigned)((a.n_rows + a.tile_rows - 1) / a.tile_rows);
-  hipLaunchKernelGGL((k_digit_down<NT, WAVES, SLOTS>), dim3(tiles, passes), dim3(64 * WAVES), L::kLds, s, a);
+  hipLaunchKernelGGL((k_digit_down<NT, WAVES, SLOTS, ROWS>), dim3(tiles, passes), dim3(64 * WAVES), L::kLds, s, a);
   XABE_HIP_TRY(hipGetLastError());
   return XABE_OK;
 }
@@ -413,7 +426,9 @@ bool digit_down_makes(const xabe_moe_kernels* k, size_t tokens) { return tokens 
 int launch_digit_down(const xabe_moe_kernels* k, RowsArgs a, size_t tokens, hipStream_t s) {
   rows_shape(a, XABE_QUANT_Q6K, 1);
   if (digit_down_makes(k, tokens)) return down_go<1, 16, 1>(a, k->num_cus, (unsigned)tokens, s);
-  return tokens == 2 ? down_go<2, 16, 1>(a, k->num_cus, 1, s) : down_go<4, 8, 2>(a, k->num_cus, 1, s);
+  if (tokens == 2) return down_go<2, 16, 1>(a, k->num_cus, 1, s);
+  if (tokens == 3) return down_go<3, 16, 1>(a, k->num_cus, 1, s);
+  return a.n_rows <= 16 * k->num_cus ? down_go<4, 16, 1, 16>(a, k->num_cus, 1, s) : down_go<4, 8, 2>(a, k->num_cus, 1, s);
 }
 
 template <int NT>
