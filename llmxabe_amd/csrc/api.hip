@@ -360,11 +360,15 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
 // token 54.8 / 50.3 (four layers in turn 60.4 / 57.4), two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105,
 // sixteen 183 / 109.  With 0.4 % of the intermediate values a thousand times the others, whose superblocks the digits do not hold
 // (digit_rests): one 54.0 / 49.7, three 70.5 / 68.7, seven 98.9 / 87.3, sixteen 183 / 125, sixty-three 695 / 448.
-// Intermediate rows of 32 superblocks and more, where no width but two and four tokens loses by it, and these 2 % (one / two / three / four /
-// eight / forty tokens, 2048 x 8192 23.3 / 25.1 / 30.8 / 30.9 / 41.0 / 110 by group, 22.0 / 24.4 / 30.2 / 31.7 / 29.2 / 80 by superblock;
-// 3072 x 8192 26.7 / 28.7 / 34.1 / 34.0 / 45.4 / 133, 24.7 / 29.3 / 33.5 / 34.8 / 34.6 / 97).  Hidden sizes of at most 21 superblocks: a
-// tile of down's few-token launch holds 21 rows for each of 256 compute units, and beyond that it is two half-full ones (one / four / eight
-// / forty tokens, 6144 x 10240 41.5 / 52.6 / 74 / 330 by group, 49.8 / 69.3 / 67 / 224; 8192 x 28672 127 / 156 / 219 / 1002, 142 / 184 / 186 / 676).
+// Intermediate rows of 24 superblocks and more, where every width gains by it but four tokens, whose digits take a launch that down does
+// not make up for (one / two / three / four / eight / forty tokens, 2048 x 6144 20.2 / 21.9 / 26.6 / 26.6 / 35.7 / 99 by group, 17.9 /
+// 21.0 / 26.2 / 27.7 / 27.0 / 73 by superblock; 3072 x 8192 26.7 / 28.7 / 34.1 / 34.0 / 45.4 / 133, 24.7 / 29.3 / 33.5 / 34.8 / 34.6 / 97;
+// 4096 x 6144 27.3 / 29.0 / 36.0 / 36.0 / 47.5 / 156, 24.0 / 27.8 / 34.4 / 35.3 / 40.0 / 110; 5120 x 6144 29.6 / 31.4 / 38.0 / 37.9 / 49.5 /
+// 198, 26.8 / 30.6 / 37.5 / 40.0 / 44.6 / 123).  Shorter rows lose more: 4096 x 4096 21.3 / 22.7 / 27.5 / 27.5 / 33.9 / 105, 19.8 /
+// 22.5 / 28.0 / 28.6 / 33.9 / 92; 5120 x 2560 20.2 / 21.6 / 25.5 / 25.5 / 32.3 / 109, 17.5 / 21.4 / 25.7 / 26.6 / 37.1 / 103.
+// Hidden sizes of at most 21 superblocks: a tile of down's few-token launch holds 21 rows for each of 256 compute units, and beyond that
+// it is two half-full ones (one / four / eight / forty tokens, 6144 x 10240 41.5 / 52.6 / 74 / 330 by group, 49.8 / 69.3 / 67 / 224;
+// 8192 x 28672 127 / 156 / 219 / 1002, 142 / 184 / 186 / 676).
 static bool shared_whole(const xabe_moe_geometry& g, int gate_q, int up_q, int down_q) {
   return gate_q == XABE_QUANT_Q6K && up_q == XABE_QUANT_Q6K && down_q == XABE_QUANT_Q6K && g.hidden % 256 == 0 &&
          g.intermediate % 256 == 0 && g.hidden >= 2048 && g.hidden <= (size_t)kWholeMaxSb * 256 && g.intermediate >= (size_t)kWholeMinInterSb * 256;

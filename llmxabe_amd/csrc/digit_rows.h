@@ -92,7 +92,7 @@ void rows_shape(RowsArgs& a, int quant, int nm);
 // halves; the quarters are added in pairs.  Values that the digits of a superblock do not hold exactly, a few of them, are added to
 // the class ahead of the superblock's sum (digit_rests).
 constexpr int kWholeQuarters = 4;
-constexpr int kWholeMaxSb = 21, kWholeMinInterSb = 32;  // superblocks of the hidden size at most, of the intermediate size at least
+constexpr int kWholeMaxSb = 21, kWholeMinInterSb = 24;  // superblocks of the hidden size at most, of the intermediate size at least
 int digit_columns_configure();
 int digit_narrow_configure();
 // Gate and up for one or two tokens, from a.x alone.

@@ -148,9 +148,9 @@ def test_large_q6_k_matrices(hidden, inter):
 
 
 # (hidden, intermediate) of the kernels that scale the intermediate rows by superblocks: the smallest of both, odd numbers of
-# superblocks (9 and 33, 21 and 35), more sets of sixteen gate/up rows than a wavefront holds sums of (73 superblocks), more
+# superblocks (9 and 25, 9 and 33, 21 and 35: classes of down's without any, with one and two), more sets of sixteen gate/up rows than a wavefront holds sums of (73 superblocks), more
 # shares of gate and up than compute units (81), down's widest tiles for sixteen wavefronts of four tokens (4096 on 256 compute units)
-WHOLE = [(2048, 8192), (4096, 8192), (2304, 8448), (5376, 8960), (2048, 18688), (5376, 20736)]
+WHOLE = [(2048, 6144), (2048, 8192), (4096, 8192), (2304, 6400), (2304, 8448), (5376, 8960), (2048, 18688), (5376, 20736)]
 
 
 def _ffn64_rows(X, st, x, hidden, inter):
