@@ -357,11 +357,11 @@ static bool shared_on_digits(const xabe_moe_geometry& g) {
 // launches are digit_narrow.hip's and, from five tokens on, digit_columns.hip's.  By the geometry and the formats alone, for the same reason.
 // (Scales by groups of sixteen, which gate/up's workgroups make by themselves, cost down ten instructions per row, group and
 // token, and its sums a rounding per group.)  Dense block, us, scales by group / by superblock, hidden 5120, intermediate 17408: one
-// token 54.8 / 50.3 (four layers in turn 60.4 / 57.4), two 58.7 / 55.1, four 70.3 / 70.1, five 100 / 81, eight 102 / 83, nine 182 / 105,
-// sixteen 183 / 109.  With 0.4 % of the intermediate values a thousand times the others, whose superblocks the digits do not hold
-// (digit_rests): one 54.0 / 49.7, three 70.5 / 68.7, seven 98.9 / 87.3, sixteen 183 / 125, sixty-three 695 / 448.
-// Intermediate rows of 24 superblocks and more, where every width gains by it but four tokens, whose digits take a launch that down does
-// not make up for (one / two / three / four / eight / forty tokens, 2048 x 6144 20.2 / 21.9 / 26.6 / 26.6 / 35.7 / 99 by group, 17.9 /
+// token 55.2 / 50.0 (four layers in turn 59.8 / 57.3), two 57.4 / 55.0, three 67.5 / 63.0, four 66.8 / 67.0, five 96 / 74, eight 96 / 76,
+// sixteen 181 / 102.  With 0.4 % of the intermediate values a thousand times the others, whose superblocks the digits do not hold
+// (digit_rests): one 55.9 / 51.7, three 68.5 / 64.1, four 69.2 / 68.9, seven 99 / 82, sixteen 183 / 128, sixty-three 691 / 445.
+// Intermediate rows of 24 superblocks and more, where every width gains by it but two tokens at some sizes and four, whose digits take
+// a launch that down does not make up for, 2 and 5 % (one / two / three / four / eight / forty tokens, 2048 x 6144 20.2 / 21.9 / 26.6 / 26.6 / 35.7 / 99 by group, 17.9 /
 // 21.0 / 26.2 / 27.7 / 27.0 / 73 by superblock; 3072 x 8192 26.7 / 28.7 / 34.1 / 34.0 / 45.4 / 133, 24.7 / 29.3 / 33.5 / 34.8 / 34.6 / 97;
 // 4096 x 6144 27.3 / 29.0 / 36.0 / 36.0 / 47.5 / 156, 24.0 / 27.8 / 34.4 / 35.3 / 40.0 / 110; 5120 x 6144 29.6 / 31.4 / 38.0 / 37.9 / 49.5 /
 // 198, 26.8 / 30.6 / 37.5 / 40.0 / 44.6 / 123).  Shorter rows lose more: 4096 x 4096 21.3 / 22.7 / 27.5 / 27.5 / 33.9 / 105, 19.8 /

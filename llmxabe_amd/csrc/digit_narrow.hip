@@ -22,7 +22,7 @@ constexpr int kMaxLds = 160 * 1024;
 //
 // The first units' rows are on their way (29 MB over the chip, 5 us) while the workgroup normalises the tokens' rows and writes
 // their digits, for itself: every workgroup does that again, but the launch that does it once takes 5 us by itself.  The rows,
-// the norm weight and then the digits take turns in one area of LDS.  Rows come in with each 2048-byte run's pieces permuted
+// the norm weight and then the digits take turns in one area of LDS.  Rows come in with each superblock's 64 pieces permuted
 // (piece q at q ^ (q / 8 mod 8)): the fold's lanes read pieces eight apart.
 // Hidden 5120, intermediate 17408, 146 MB (27 us at the rate of a large copy), us, k_rms_norm_digits and k_digit_rows / this: one
 // token 5 and 30.1 / 30.8, two 5 and 30.7 / 33.5.  (Four tokens' digits would leave no room for the rows.)

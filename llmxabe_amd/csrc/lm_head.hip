@@ -547,8 +547,8 @@ int xabe_lm_head_forward(const xabe_lm_head* h, void* stream, int format, const 
   a.w_bytes = weight_len;
   a.seg_sb = 0;
   const bool quant = format == XABE_HEAD_Q8_0 || format == XABE_HEAD_Q6K;
-  // (Q6_K up to four tokens: forward pass over the model's vocabulary, us, k_lm_head_quant / tiles: four 98 / 115, five
-  // 120 / 115, eight 158 / 119, sixteen 309 / 163; the same bits)
+  // (Q6_K: forward pass over the model's vocabulary, us, k_lm_head_quant / tiles: one token 82 / 112, two 84 / 107, three 90 / 104, four
+  // 94 / 104, five 119 / 108, eight 160 / 106, sixteen 311 / 152; the same bits)
   const bool tiles = xabe::head_tiles_width(g.hidden) &&
                      (format == XABE_HEAD_Q8_0 || format == XABE_HEAD_BF16 || (format == XABE_HEAD_Q6K && tokens > 4));
   // passes of equal width: nine tokens as five and four, not as eight and one

@@ -15,8 +15,8 @@
 //
 // Bound by bytes, but for Q6_K's vector instructions at more than eight tokens.  248 320 x 2048, us for a pass over the
 // matrix, before / with these (1 / 3 / 8 / 16 tokens): Q8_0 99 / 107 / 153 / 294, now 97 / 102 / 111 / 128 (5.6 to
-// 4.2 TB/s); bf16 178 / 189 / 389 / 756, now 173 / 180 / 186 / 197 (5.9 to 5.2 TB/s); Q6_K at 8 / 16 tokens 158 / 309, now
-// 119 / 163.  (One request per tile, and shares that do not start on a line: Q8_0 106 / 108 / 119 / 150.)
+// 4.2 TB/s); bf16 178 / 189 / 389 / 756, now 173 / 180 / 186 / 197 (5.9 to 5.2 TB/s); Q6_K at 5 / 8 / 16 tokens 119 / 160
+// / 311, now 108 / 106 / 152.  (One request per tile, and shares that do not start on a line: Q8_0 106 / 108 / 119 / 150.)
 //
 // Per (row, token) the order of operations is fixed: a token's logits are the same bits at every batch width.
 #include <algorithm>
@@ -55,9 +55,9 @@ struct HeadShare {
 
 // All but the last N of this wavefront's requests are there (stores count, too); the last tile waits for everything.
 template <int N>
-__device__ __forceinline__ void wait_but(bool last) {
-  if (last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+__device__ __forceinline__ void wait_tile(bool last) {
+  if (last) wait_but<0>();
+  else wait_but<N>();
 }
 
 // The sums the wavefronts left at red[wave][half][token][32], added and stored.  HALVES 2: one after the other, each half of
@@ -240,7 +240,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_bf16(LmHeadArgs a) {
     float* const mine = buf + sh.wave * kRed;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      wait_but<8>(last);
+      wait_tile<8>(last);
       v8b_t w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = *reinterpret_cast<const v8b_t*>(slot + (16 * s + sh.r) * 512 + (((4 * j + sh.g) ^ sh.r) * 16));
@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q8(LmHeadArgs a) {
     float* const mine = buf + sh.wave * kRed;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      wait_but<Q8Dma::kInstr>(last);
+      wait_tile<Q8Dma::kInstr>(last);
       // The lane's eight codes of every block: on a word in odd blocks, half a word past one in even ones.
       uint32_t code[8][2], d[4];  // (two blocks' scales to a register)
       const uint8_t* p = slot + s * Q8Dma::kRunBytes + sh.r * SbRaw<kQ8_0>::kBytes;
@@ -603,7 +603,7 @@ __global__ void __launch_bounds__(512, 2) k_head_tiles_q6(LmHeadArgs a) {
     SbRaw<kQ6K> raw;  // of a marked superblock, a lane per row and half: lane 32 h + 16 s + r
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      wait_but<Q6Dma::kInstr>(last);
+      wait_tile<Q6Dma::kInstr>(last);
       if (sb == sh.waves - 1 && row0 + kTileRows >= a.vocab) {  // (the tensor's last bytes, which no whole piece held)
         const int live = a.vocab - (row0 + 16 * s);
         if (live >= 1 && live <= 16) dma.patch_tail(a.w, run_off(row0, s), live, sb, slot + s * Q6Dma::kRunBytes);

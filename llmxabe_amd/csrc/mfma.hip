@@ -1235,9 +1235,11 @@ static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
   return narrow_tiles(tokens, g.experts_per_token, g.num_experts) ? kNarrowRows : kWideRows;
 }
 // Whether narrow gate/up is launched with twice the workgroups that fit: while an expert's share averages one block of 32 rows.
-// Blocks of the routed model, us, once / twice: 100 tokens 229 / 223, 256: 248 / 239, 512: 259 / 252, 900: 283 / 280; with the
-// published layout 238 / 236, 256 / 247, 268 / 261, 293 / 290; skewed loads, whose items are less than two rounds, alike.  At 1237
-// tokens, where items are one block or two, 327 / 313, but 314 / 317 in the published layout, and skewed 255 / 260.
+// Layers of the routed model in a row, us, once / twice: 512 tokens 259.6 / 251.0, 700: 269 / 265, 900: 279.5 / 277.4, 1000: 285.5 / 284.0,
+// 1024: 286.3 / 285.1; with the seam 252 / 245, 263 / 258, 275 / 270, 279.2 / 277.4, 279.6 / 278.4; with the published layout 267 / 260, 279 / 274,
+// 292 / 286, 296 / 293, 297 / 295.5; 100 and 256 tokens gain as 512 do.  Skewed loads: less than two rounds of items up to 900 tokens, and alike;
+// 950: 229 / 220, 1000: 253 / 227, 1024: 229 / 228.  At 1237 tokens, where items are one block or two, 327 / 313, but 314 / 317 in the
+// published layout, and skewed 255 / 260.
 static bool gate_up_twice(const xabe_moe_geometry& g, size_t tokens) { return tokens * g.experts_per_token <= 32 * g.num_experts; }
 // The specialised form (k_mfma_pc) serves both routed launches for contractions of whole superblocks and at least
 // eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_rows everywhere; it is the faster at every width
@@ -1447,9 +1449,9 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
 // wide), and a tile walks its whole contraction alone: 64 tokens took 147 us on 40 workgroups.  Up to 1024 tokens the
 // contraction is in four parts (or as many as divide it), whose sums are added in order by one more launch; by the
 // buffers' size and the geometry alone, so that a token's row is the same bits in every pass and in every pass of buffers up to
-// that size.  Wider passes have tiles enough, and four planes of sums would cost them more than they gain (2048 tokens of
-// the dense sibling: as many rounds of items, and 170 MB each way).  The planes lie in the fp32 intermediate rows, which the
-// matrix-core regime does not use.
+// that size.  (Not in those of larger ones, where few live tokens walk one chain, too.)  Wider passes have tiles enough, and four
+// planes of sums would cost them more than they gain (2048 tokens of the dense sibling: as many rounds of items, and 170 MB each
+// way).  The planes lie in the fp32 intermediate rows, which the matrix-core regime does not use.
 constexpr size_t kPartsMaxTokens = 1024;
 static int down_parts(const xabe_moe_geometry& g) {
   if (g.max_tokens > kPartsMaxTokens) return 1;
