@@ -533,8 +533,10 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 //    (tests/test_spilled_registers.py).  With up to seven in eight of the sixteen forms the routed down launch drained
 //    its queue once per item, right behind the item's stores.  Scalar registers are kept in lanes of vector ones where there
 //    are too many (up to 119): no memory operation, but lane reads in the loop over the superblocks;
-//  - the two wavefronts of a SIMD make their requests and read raw weights at different times (`early`): behind a barrier
-//    both would leave the matrix pipe idle together;
+//  - what lies between the matrix instructions is kept there (w_part pins its results: the compiler moved the making of a
+//    chunk's halfs behind the chunk wherever a branch followed).  Wavefronts of a SIMD that make their requests at different times
+//    measured no better than all behind the matrix instructions, and cost a branch per chunk (both builds in turn, with the
+//    stores below: 1237 tokens 317 -> 309 us, 1400 669 -> 648 for two layers, two blocks of 8192 1860 -> 1820, dense 2048 1132 -> 1096);
 //  - LDS reads on their own width's boundary (any other takes 64 cycles), rows spread over the banks by the windows' odd
 //    count of sixteen bytes, activations by pc_swizzle.
 // A short contraction (down of the routed model: two superblocks) is bound by what an item costs besides: its stores, which
@@ -654,9 +656,13 @@ __device__ __forceinline__ uint32_t w_codes(const WHalf<kQ8_0>& r, int w) {
 template <int C, int PART, int QUANT>
 __device__ __forceinline__ void w_part(const WHalf<QUANT>& r, uint32_t pick, WChunk& k) {
   if constexpr (PART == 0) {
-    if constexpr ((C & 3) == 0) k.scales = w_scales(r, C >> 2, pick);
+    if constexpr ((C & 3) == 0) {
+      k.scales = w_scales(r, C >> 2, pick);
+      asm volatile("" : "+v"(k.scales));
+    }
   } else if constexpr (PART <= 2) {
     k.code[PART - 1] = w_codes<C>(r, PART - 1);
+    asm volatile("" : "+v"(k.code[PART - 1]));
   } else {
     constexpr int w = PART - 3;
     const _Float16 off = QUANT == kQ6K ? (_Float16)-1056.0f : (_Float16)-1152.0f;  // (1024 of the byte's placing, and the codes' centre)
@@ -667,6 +673,7 @@ __device__ __forceinline__ void w_part(const WHalf<QUANT>& r, uint32_t pick, WCh
       v = (v + half2v{off, off}) * half2v{s, s};
       k.out[2 * w + i] = __builtin_bit_cast(uint32_t, v);
     }
+    asm volatile("" : "+v"(k.out[2 * w]), "+v"(k.out[2 * w + 1]));
   }
 }
 template <int C, int PART = 0, int QUANT>
@@ -867,16 +874,16 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   // piece q = wave + WAVES i of a step: token rows 8 q .. 8 q + 7; lane: row 8 q + (lane >> 3), position lane & 7, which
   // holds chunk (lane & 7) ^ pc_swizzle(row)
   constexpr int kPI = 4 * MI / WAVES;
-  uint32_t a_off[kPI], a_lanes[kPI];  // the lane's piece of either instruction; which instructions are for live rows
+  uint32_t a_off[kPI];  // the lane's piece of each instruction
+  int a_pieces = 0;     // pieces of live 32-row blocks
   auto set_a = [&](const Item& it, int tb) __attribute__((always_inline)) {
-    const int pieces = (it.rows + 31) / 32 * 4;
+    a_pieces = (it.rows + 31) / 32 * 4;
     const int lane = item_lane();
 #pragma unroll
     for (int i = 0; i < kPI; ++i) {
       const int row = 8 * (wave + WAVES * i) + (lane >> 3), live = min(row, it.rows - 1);
       int arow = it.m0 + live;
-      if (ROUTED && NM == 2) arow = sId[tb * kTM + live] / a.top_k;
-      a_lanes[i] = __builtin_amdgcn_readfirstlane(WAVES * i < pieces ? ~0u : 0u);
+      if (ROUTED && NM == 2) arow = (int)((uint32_t)sId[tb * kTM + live] / (uint32_t)a.top_k);
       a_off[i] = ((uint32_t)arow * (uint32_t)a.K + (uint32_t)((lane & 7) ^ pc_swizzle(row)) * 8u) * 2u;
       if constexpr (kInParts) a_off[i] += (uint32_t)(it.part * k_part) * 2u;
     }
@@ -886,8 +893,10 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   uint32_t a_to = 0;  // its place in the ring
   auto request_a = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kPI; ++i)
-      lds_dma_16_lanes(a.a, a_off[i] + (uint32_t)a_ks * (kSK * 2u), lds_a + a_to + 1024u * WAVES * i, a_lanes[i], a_lanes[i]);
+    for (int i = 0; i < kPI; ++i) {
+      const uint32_t live = WAVES * i < a_pieces ? ~0u : 0u;
+      lds_dma_16_lanes(a.a, a_off[i] + (uint32_t)a_ks * (kSK * 2u), lds_a + a_to + 1024u * WAVES * i, live, live);
+    }
   };
   auto request_ids = [&](const Item& it, int tb) __attribute__((always_inline)) {
     const int lane = item_lane();
@@ -906,10 +915,6 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   // where the lane finds its row's eight elements of chunk kk of a step: piece 4 (kk >> 1) + 2 h + (kk & 1)
   const uint32_t frag = (uint32_t)col * (kSK * 2) + (uint32_t)(((2 * h) ^ pc_swizzle(col)) * 16);
   const uint32_t pick = w_scale_bytes(h);
-  // The two wavefronts of a SIMD do what is not matrix instructions at different times (before a chunk's and behind them,
-  // one chunk and the next): behind a barrier both would leave the matrix pipe idle together.
-  const bool early = wave < WAVES / 2;
-
   Item cur = decode(first), nxt = cur;
   int tb = 0;              // which of the two tables is this item's
   WHalf<QUANT> raw[QUANT == kQ6K ? 2 : 1];  // the raw weights that an item starts on: a superblock's halves, or its first
@@ -995,19 +1000,15 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
           if constexpr (QUANT == kQ6K) {
             const int u = sb + 1 == nsb ? 0 : 2 * sb + 2;
             const uint32_t from = kInParts ? start_of(sb + 1 == nsb ? nxt : cur) : 0;
-            if constexpr (C == 12 || C == 13) {
-              if (early == (C == 12)) {
-                wait_vm<Req::after_w(C)>();
-                if (w_win == n_win) patch_w();
-                read_w(from, u, 0, next[0]);
-              }
+            if constexpr (C == 13) {
+              wait_vm<Req::after_w(C)>();
+              if (w_win == n_win) patch_w();
+              read_w(from, u, 0, next[0]);
             }
             if constexpr (C == 14) read_w(from, u + 1, 1, next[1]);
-          } else if constexpr ((C & 7) == 5 || (C & 7) == 6) {
-            if (early == ((C & 7) == 5)) {
-              wait_vm<Req::after_w(C)>();
-              read_w(0, C < 8 ? 1 : 0, 0, C < 8 ? second : next[0]);  // (Q8_0 superblocks are whole pieces)
-            }
+          } else if constexpr ((C & 7) == 6) {
+            wait_vm<Req::after_w(C)>();
+            read_w(0, C < 8 ? 1 : 0, 0, C < 8 ? second : next[0]);  // (Q8_0 superblocks are whole pieces)
           }
           if constexpr ((C & 3) == 3) {
             constexpr int S = C >> 2;
@@ -1041,18 +1042,14 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
             }
             ring = ring_after(ring);
           }
-          auto requests = [&]() __attribute__((always_inline)) {
-            if constexpr (Req::a_at(C) != 0) request_a();
-            if constexpr (Req::w_at(C) != 0) request_w(std::integral_constant<int, QUANT == kQ6K ? (C + 1) & 15 : (C + 1) & 7>{});
-          };
-          constexpr bool kRequests = Req::a_at(C) != 0 || Req::w_at(C) != 0;
-          if (kRequests && early) requests();
           order_fence();
           const WHalf<QUANT>& r1 = half_of(std::integral_constant<int, C1>{});
           const uint8_t* pa = sA + ((frag ^ (64u * ((C1 >> 1) & 1) + 16u * (C1 & 1))) + ring);
 #pragma unroll
           for (int i = 0; i < NB; ++i) {
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb, acc[i], 0, 0, 0);
+            // (which operand comes first decides what a lane's sums are: a token's for gate/up, a weight row's for down)
+            acc[i] = NM == 2 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(fb, fa[i], acc[i], 0, 0, 0)
+                             : __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb, acc[i], 0, 0, 0);
             fa[i] = *reinterpret_cast<const half8*>(pa + i * kBlockBytes);
             // the next chunk's weights between the matrix instructions: the two run beside each other (up to four vector
             // instructions cost a matrix instruction nothing)
@@ -1063,7 +1060,8 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
             if (4 * NB / kWParts == i) w_part<C1 & 7, 4>(r1, pick, wc);
             __builtin_amdgcn_sched_barrier(0);
           }
-          if (kRequests && !early) requests();
+          if constexpr (Req::a_at(C) != 0) request_a();
+          if constexpr (Req::w_at(C) != 0) request_w(std::integral_constant<int, QUANT == kQ6K ? (C + 1) & 15 : (C + 1) & 7>{});
           fb = w_halfs(wc);
           if constexpr (C1 == 0) {
             raw[0] = next[0];
@@ -1088,46 +1086,59 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
         chunk(std::integral_constant<int, 15>{});
       }
 
-      // epilogue.  acc[i][v]: tile row 32 i + (v / 4) * 8 + h * 4 + v % 4, column lane % 32 of the wavefront
+      // epilogue.  acc[i][v] of block i: gate/up, token lane % 32 and weight row (v / 4) * 8 + h * 4 + v % 4 of the wavefront's, so that
+      // a token's gate and up columns are in one lane and leave as sixteen bytes; down, the other way round, so that a store
+      // covers 128 bytes of a row (as sixteen bytes per lane, 64 of a row, 1237 tokens took 319 us instead of 309)
       const int lane = item_lane();
       const int h = lane >> 5, col = lane & 31;
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         const int left = cur.rows - 32 * i;  // live rows from this block on
         if constexpr (NM == 2) {
-          // lanes 0-15 hold a gate column's element, lanes 16-31 the matching up column's: an exchange of two registers'
-          // halves leaves gate and up of one row in lanes 0-15, of the next row in lanes 16-31
-          const int odd = (lane >> 4) & 1, c = cur.nt * (kTR / 2) + 16 * wave + (lane & 15);
-          _Float16* out = static_cast<_Float16*>(a.out) + (size_t)(cur.m0 + 32 * i) * a.n_rows + c;
+          // registers 0-7 are gate columns, 8-15 the matching up columns; as halfs, two exchanges between the lane halves give
+          // lane h of a token the columns 8 h .. 8 h + 7
+          uint32_t p[4];
 #pragma unroll
-          for (int v = 0; v < 16; v += 2) {
-            const float even_row = acc[i][v], odd_row = acc[i][v + 1];
-            const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, even_row), __builtin_bit_cast(uint32_t, odd_row), false, false);
-            const uint32_t gb = sw[0], ub = sw[1];
-            const float g = __builtin_bit_cast(float, gb) * kWScaleInv, up = __builtin_bit_cast(float, ub) * kWScaleInv;
-            const int r = (v >> 2) * 8 + h * 4 + (v & 3) + odd;
-            if (r < left) out[(size_t)r * a.n_rows] = (_Float16)(silu_fast(g) * up);
+          for (int v = 0; v < 8; v += 2) {
+            uint16_t o[2];
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+              // (silu_fast(g) * up, both sums' 2^-8 on the gate; halfs one by one: a pair's conversion would round the product twice)
+              const float g = acc[i][v + w], e = __builtin_amdgcn_exp2f(g * (-1.44269504088896340736f * kWScaleInv));
+              o[w] = __builtin_bit_cast(uint16_t, (_Float16)(g * (kWScaleInv * kWScaleInv) * __builtin_amdgcn_rcpf(1.0f + e) * acc[i][v + w + 8]));
+            }
+            p[v / 2] = o[0] | (uint32_t)o[1] << 16;
           }
+          const auto s0 = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+          _Float16* block = static_cast<_Float16*>(a.out) + (size_t)(cur.m0 + 32 * i) * a.n_rows + cur.nt * (kTR / 2) + 16 * wave;
+          if (col < left) *reinterpret_cast<u32x4*>(block + (uint32_t)(col * a.n_rows + 8 * h)) = u32x4{s0[0], s1[0], s0[1], s1[1]};
         } else {
-          const int c = cur.nt * kTR + 32 * wave + col;
-          float* out = static_cast<float*>(a.out) + c;
-          if (kInParts && cur.part > 0) out = a.planes + (size_t)(cur.part - 1) * a.plane + c;
+          float* out = static_cast<float*>(a.out);
+          if (kInParts && cur.part > 0) out = a.planes + (size_t)(cur.part - 1) * a.plane;
+          out += cur.nt * kTR + 32 * wave;
+          if (!ROUTED) out += (size_t)(cur.m0 + 32 * i) * a.n_rows;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            int orow[4];
-            float s[4];
+            if (8 * q >= left) break;
+            int4 id = {0, 0, 0, 0};
+            float4 w4 = {1.0f, 1.0f, 1.0f, 1.0f};
+            if constexpr (ROUTED) {
+              id = *reinterpret_cast<const int4*>(sId + 32 * i + 8 * q + 4 * h);
+              w4 = *reinterpret_cast<const float4*>(sScale + 32 * i + 8 * q + 4 * h);
+            }
+            const int ids[4] = {id.x, id.y, id.z, id.w};
+            const float ws[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-              const int r = 32 * i + 8 * q + 4 * h + w;
-              orow[w] = ROUTED ? sId[r] : cur.m0 + r;
-              s[w] = ROUTED ? sScale[r] : 1.0f;
+              const int r = 8 * q + 4 * h + w;
+              float* to = out + ((size_t)(uint32_t)(ROUTED ? ids[w] : r) * (uint32_t)a.n_rows + (uint32_t)col);
+              if (r < left) *to = ws[w] * kWScaleInv * acc[i][4 * q + w];
             }
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-              if (8 * q + 4 * h + w < left) out[(size_t)orow[w] * a.n_rows] = s[w] * (acc[i][4 * q + w] * kWScaleInv);
           }
         }
       }
+      // (a join of its own for the last store's branch: run into the item loop's, it makes the weights' scalar addresses vector ones)
+      asm volatile("" ::: "memory");
     };
     const int nb = (cur.rows + 31) / 32;
     if constexpr (MI > 2) {
