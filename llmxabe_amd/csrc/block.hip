@@ -27,11 +27,14 @@ static int block_alloc(float** p, size_t n, hipStream_t s) {
   return XABE_OK;
 }
 
-// (default priority, like every stream this library makes)
+// (default priority, like every stream this library makes.  The events order kernels of one device, whose own fences make
+// their writes visible to each other: with the system-wide fence of a plain event between them a fork and a join cost about 3 us
+// more, published layout 1237 tokens 314 / 312 us, skewed 700 399 / 395, one Q6_K block of 512 254 / 251)
 static int block_side_stream(xabe_moe_block* blk) {
+  constexpr unsigned kFlags = hipEventDisableTiming | hipEventDisableSystemFence;
   XABE_HIP_TRY(hipStreamCreateWithFlags(&blk->side, hipStreamNonBlocking));
-  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->forked, hipEventDisableTiming));
-  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->joined, hipEventDisableTiming));
+  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->forked, kFlags));
+  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->joined, kFlags));
   return XABE_OK;
 }
 
