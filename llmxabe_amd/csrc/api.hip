@@ -809,6 +809,10 @@ static int check_shared_stacks(const xabe_moe_kernels* k, xabe_quant_tensor gate
   return XABE_OK;
 }
 
+int xabe::check_shared_expert(const xabe_moe_kernels* k, const xabe_moe_layer_weights* w) {
+  return check_shared_stacks(k, w->shared_gate, w->shared_up, w->shared_down);
+}
+
 int xabe::check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_weights* w) {
   XABE_TRY(check_routed_stacks(k, w->gate_exps, w->up_exps, w->down_exps));
   XABE_TRY(check_shared_stacks(k, w->shared_gate, w->shared_up, w->shared_down));
@@ -981,6 +985,19 @@ int xabe_moe_shared_expert_mma(const xabe_moe_kernels* k, void* stream, xabe_moe
   bool added = false;
   return xabe::shared_expert_mma_residual(k, as_stream(stream), b, gate, up, down, hidden_states, hidden_states_len, out, out_len,
                                           nullptr, nullptr, &added);
+}
+
+bool xabe::grouped_forward_takes_shared(const xabe_moe_kernels* k, const xabe_moe_buffers* b, const xabe_moe_layer_weights* w) {
+  return !flat_regime(k) && mfma_supported(k, b, w->gate_exps.quant, w->up_exps.quant, w->down_exps.quant, true) &&
+         mfma_supported(k, b, w->shared_gate.quant, w->shared_up.quant, w->shared_down.quant, false) && mfma_takes_shared(k, b);
+}
+
+int xabe::grouped_forward_with_shared(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, const xabe_moe_layer_weights* w,
+                                      const float* x, float* shared_out) {
+  XABE_TRY(require_routed(b, "grouped_forward_partial"));
+  XABE_TRY(check_routed_stacks(k, w->gate_exps, w->up_exps, w->down_exps));
+  const MfmaShared shared = {w->shared_gate, w->shared_up, w->shared_down, shared_out};
+  return mfma_grouped_forward_partial(k, s, b, w->gate_exps, w->up_exps, w->down_exps, x, &shared);
 }
 
 int xabe_moe_grouped_forward_partial_with_shared(const xabe_moe_kernels* k, void* stream, xabe_moe_buffers* b,

@@ -70,6 +70,7 @@ bool decode_block_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b
 // the checks the step-by-step entry points make on a layer's six stacks (whole blocks, element counts, formats,
 // 16-byte-aligned device pointers), for the block-level paths that launch without passing through them (api.hip)
 int check_layer_stacks(const xabe_moe_kernels* k, const xabe_moe_layer_weights* w);
+int check_shared_expert(const xabe_moe_kernels* k, const xabe_moe_layer_weights* w);
 // The seam between this block and the next as the decode launches see it: `input_normed`: `normed` holds the pass's
 // rows already; `next_normed` (null: the pass ends at l_out): where the third launch's last workgroup per token
 // writes rms_norm(l_out, next_w, next_eps), `next_normed_h` (may be null) its fp16 copy.
@@ -127,8 +128,19 @@ bool mfma_supported(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int ga
 // token-tile height of the routed launches of the pass as published, and the entries `tile_list` holds; false when
 // these buffers carry no list
 bool mfma_tile_plan(const xabe_moe_kernels* k, const xabe_moe_buffers* b, int* bm, int* capacity);
+// (`shared`: null, or the shared expert of the same pass and its ungated rows, which go along in the same launches where
+// mfma_takes_shared says so)
+struct MfmaShared {
+  xabe_quant_tensor gate, up, down;
+  float* out;
+};
+bool mfma_takes_shared(const xabe_moe_kernels* k, const xabe_moe_buffers* b);
 int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                                 xabe_quant_tensor up, xabe_quant_tensor down, const float* x);
+                                 xabe_quant_tensor up, xabe_quant_tensor down, const float* x, const MfmaShared* shared = nullptr);
+// xabe_moe_grouped_forward_partial with that shared expert (api.hip)
+bool grouped_forward_takes_shared(const xabe_moe_kernels* k, const xabe_moe_buffers* b, const xabe_moe_layer_weights* w);
+int grouped_forward_with_shared(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, const xabe_moe_layer_weights* w,
+                                const float* x, float* shared_out);
 // (`residual`, `l_out`: null, or l_out = out + residual where a launch comes by that can add it: `*added`)
 int mfma_shared_expert(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
                        xabe_quant_tensor up, xabe_quant_tensor down, const float* x, float* out, const float* residual,

@@ -732,8 +732,20 @@ constexpr size_t mfma_rows_lds() {
 template <int MI, int WAVES>
 constexpr int kWgsPerCu = MI > 2 ? 1 : 3;
 
+// The items first, first + stride, ... below hi; none where first is not below hi.
+struct Dealt { int first, hi, stride; };
+
+// Items of a launch: (token tile, row tile) pairs, times the parts of a contraction.
+template <int NM, bool ROUTED, int WAVES>
+__device__ __forceinline__ int count_items(const MfmaArgs& a, int parts) {
+  const int tiles = ROUTED ? a.tile_list[0] : (__builtin_amdgcn_readfirstlane(*a.valid_tokens) + a.tile_rows - 1) / a.tile_rows;
+  return tiles * (a.n_rows / (WAVES * kWRows / NM)) * parts;
+}
+
 template <int QUANT, int NM, bool ROUTED, int MI, int WAVES, bool kInParts>
-__device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
+__device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a, const Dealt& dealt) {
+  const int first = dealt.first, hi = dealt.hi, stride = dealt.stride;
+  if (first >= hi) return;
   constexpr int kTM = 32 * MI;                    // token rows of a tile at most
   constexpr int kTR = WAVES * kWRows;             // weight rows of a tile
   constexpr int kSlot = MI * kBlockBytes;         // an activation step in LDS
@@ -755,30 +767,9 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   const int valid = __builtin_amdgcn_readfirstlane(*a.valid_tokens);
   const int n_ntiles = a.n_rows / (kTR / NM);
   const int tile_rows = a.tile_rows;
-  const int n_mtiles = ROUTED ? a.tile_list[0] : (valid + tile_rows - 1) / tile_rows;
   const int parts = kInParts ? a.parts : 1;
-  const int total = n_mtiles * n_ntiles * parts;
   const int k_part = a.K / parts, nsteps = k_part / kSK, nsb = k_part / 256;
   const uint32_t row_bytes = QUANT == kQ6K ? (uint32_t)(a.K / 256) * kQ6KBytes : (uint32_t)(a.K / 32) * kQ8Bytes;
-
-  // Which items this workgroup takes.  Workgroup ids are dealt round-robin to the eight XCDs, each with its own L2: when
-  // there is work for every workgroup, XCD x takes a contiguous eighth of the items (token tile major) and its workgroups
-  // walk that range together, so an activation tile is fetched into one L2 instead of into all eight, and the token tiles
-  // of one expert reuse its weights from that L2.
-  // Routed gate/up, narrow: a third round of items would be two thirds full at most, and it begins late on the CUs that the shared
-  // expert still holds when the launch begins.  There a grid of twice the workgroups that fit (gate_up_twice) deals the
-  // second half to whatever CU is free first, one or two items each; in fewer rounds, or more, the half that fits does as
-  // well or better by itself (the others leave here).
-  constexpr bool kTwice = ROUTED && NM == 2 && MI <= 2;
-  const bool twice = kTwice && total >= 2 * a.resident && total < 3 * a.resident;
-  const int wgs = kTwice && !twice ? min((int)gridDim.x, a.resident) : (int)gridDim.x;
-  const bool by_xcd = (wgs & 7) == 0 && (twice || total >= 2 * wgs);
-  const int xcd = blockIdx.x & 7;
-  const int lo = by_xcd ? (int)((long long)total * xcd / 8) : 0, hi = by_xcd ? (int)((long long)total * (xcd + 1) / 8) : total;
-  const int first = lo + (by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x);
-  const int stride = by_xcd ? wgs >> 3 : wgs;
-  if (kTwice && (int)blockIdx.x >= wgs) return;
-  if (first >= hi) return;
 
   // The lane's number for what an item does once: its arithmetic belongs there and not in registers all along, which would
   // be spilled, and what reloads a spilled register waits for every request in flight.
@@ -1161,14 +1152,58 @@ __device__ __forceinline__ void mfma_rows_body(const MfmaArgs& a) {
   // (nothing may still be on its way into this workgroup's LDS when it ends)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
+// Which items a workgroup takes.  Workgroup ids are dealt round-robin to the eight XCDs, each with its own L2: when
+// there is work for every workgroup, XCD x takes a contiguous eighth of the items (token tile major) and its workgroups
+// walk that range together, so an activation tile is fetched into one L2 instead of into all eight, and the token tiles
+// of one expert reuse its weights from that L2.
+// Routed gate/up, narrow: a third round of items would be two thirds full at most, and it begins late on the CUs that a
+// launch beside this one still holds when it begins.  There a grid of twice the workgroups that fit (gate_up_twice) deals the
+// second half to whatever CU is free first, one or two items each; in fewer rounds, or more, the half that fits does as
+// well or better by itself (the others get nothing).
+template <bool kTwice>
+__device__ __forceinline__ Dealt deal_items(int total, int resident) {
+  const bool twice = kTwice && total >= 2 * resident && total < 3 * resident;
+  const int wgs = kTwice && !twice ? min((int)gridDim.x, resident) : (int)gridDim.x;
+  const bool by_xcd = (wgs & 7) == 0 && (twice || total >= 2 * wgs);
+  const int xcd = blockIdx.x & 7;
+  const int lo = by_xcd ? (int)((long long)total * xcd / 8) : 0, hi = by_xcd ? (int)((long long)total * (xcd + 1) / 8) : total;
+  const int first = lo + (by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x);
+  return {kTwice && (int)blockIdx.x >= wgs ? hi : first, hi, by_xcd ? wgs >> 3 : wgs};
+}
+
 template <int QUANT, int NM, bool ROUTED, int MI, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_rows(MfmaArgs a) {
-  mfma_rows_body<QUANT, NM, ROUTED, MI, WAVES, false>(a);
+  constexpr bool kTwice = ROUTED && NM == 2 && MI <= 2;
+  mfma_rows_body<QUANT, NM, ROUTED, MI, WAVES, false>(a, deal_items<kTwice>(count_items<NM, ROUTED, WAVES>(a, 1), a.resident));
 }
 // An unrouted down contraction in parts (down_parts).
 template <int QUANT, int MI, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)) k_mfma_parts(MfmaArgs a) {
-  mfma_rows_body<QUANT, 1, false, MI, WAVES, true>(a);
+  mfma_rows_body<QUANT, 1, false, MI, WAVES, true>(a, deal_items<false>(count_items<1, false, WAVES>(a, a.parts), a.resident));
+}
+// The routed experts' items (QUANT, `a`) and the shared expert's (SQUANT, `s`) of one pass in one launch, narrow form.  Alone a launch of
+// the shared expert's is a workgroup per CU or fewer, as long as one item (512 tokens: 28 us and 14); here they fill the last round of
+// the routed items: workgroups that have one routed item fewer come first.  512 tokens, skewed: gate/up 66 -> 70 us, down 43 -> 48,
+// and in front of it routing 13 -> 11 and 14 us less of fork, join and waiting.  Shared items first: 512 tokens 252.9 -> 255.1.
+template <int QUANT, int SQUANT, int NM>
+__global__ void __launch_bounds__(256, 3) k_mfma_with_shared(MfmaArgs a, MfmaArgs s) {
+  const int routed = count_items<NM, true, 4>(a, 1), shared = count_items<NM, false, 4>(s, 1), total = routed + shared;
+  const bool twice = NM == 2 && total >= 2 * a.resident && total < 3 * a.resident;  // (deal_items)
+  const int wgs = twice ? (int)gridDim.x : min((int)gridDim.x, a.resident);
+  if ((int)blockIdx.x >= wgs) return;
+  const bool by_xcd = (wgs & 7) == 0 && (twice || total >= 2 * wgs);
+  const int xcd = blockIdx.x & 7, rank = by_xcd ? (int)blockIdx.x >> 3 : (int)blockIdx.x, stride = by_xcd ? wgs >> 3 : wgs;
+  auto share = [&](int items, int behind) __attribute__((always_inline)) {  // of the XCD, dealt from its workgroup `behind` on
+    const int lo = by_xcd ? (int)((long long)items * xcd / 8) : 0, hi = by_xcd ? (int)((long long)items * (xcd + 1) / 8) : items;
+    const int place = rank - behind % stride;
+    return Dealt{lo + (place < 0 ? place + stride : place), hi, stride};
+  };
+  const Dealt mine = share(routed, 0);
+  const int before = by_xcd ? (int)((long long)routed * (xcd + 1) / 8) - (int)((long long)routed * xcd / 8) : routed;
+  mfma_rows_body<QUANT, NM, true, 2, 4, false>(a, mine);
+  // (the bodies share LDS: each ends with its own requests landed, and all wavefronts are past their last reads here)
+  __syncthreads();
+  mfma_rows_body<SQUANT, NM, false, 2, 4, false>(s, share(shared, before));
 }
 
 // fp32 -> fp16 activations for live rows; rows past `valid` are left alone.
@@ -1339,7 +1374,22 @@ static int launch_pc(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, si
   return XABE_OK;
 }
 
+template <int QUANT, int SQUANT, int NM>
+constexpr size_t with_shared_lds() { return std::max(mfma_rows_lds<QUANT, 2, 4>(), mfma_rows_lds<SQUANT, 2, 4>()); }
+template <int QUANT, int SQUANT>
+static int configure_with_shared() {
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mfma_with_shared<QUANT, SQUANT, 2>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)with_shared_lds<QUANT, SQUANT, 2>()));
+  XABE_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mfma_with_shared<QUANT, SQUANT, 1>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)with_shared_lds<QUANT, SQUANT, 1>()));
+  return XABE_OK;
+}
+
 static int mfma_set_limits() {
+  XABE_TRY((configure_with_shared<kQ6K, kQ6K>()));
+  XABE_TRY((configure_with_shared<kQ6K, kQ8_0>()));
+  XABE_TRY((configure_with_shared<kQ8_0, kQ6K>()));
+  XABE_TRY((configure_with_shared<kQ8_0, kQ8_0>()));
   XABE_TRY((configure_pc<2>()));
   XABE_TRY((configure_pc<1>()));
   XABE_TRY((configure_one<1, false, 6, 8>()));
@@ -1379,6 +1429,26 @@ static int launch_rows(const xabe_moe_kernels* k, int quant, MfmaArgs a, size_t 
   return XABE_OK;
 }
 
+template <int NM>
+static int launch_with_shared(const xabe_moe_kernels* k, int quant, int shared_quant, MfmaArgs a, const MfmaArgs& sh, size_t max_mtiles,
+                              size_t shared_mtiles, hipStream_t s, bool twice) {
+  const size_t max_items = (max_mtiles + shared_mtiles) * (size_t)(a.n_rows / (4 * kWRows / NM));
+  a.resident = k->num_cus * kWgsPerCu<2, 4>;
+  const unsigned grid = (unsigned)std::max<size_t>(1, std::min(max_items, (size_t)a.resident * (twice ? 2 : 1)));
+  auto launch = [&](auto q, auto sq) {
+    constexpr int Q = decltype(q)::value, SQ = decltype(sq)::value;
+    hipLaunchKernelGGL((k_mfma_with_shared<Q, SQ, NM>), dim3(grid), dim3(256), (with_shared_lds<Q, SQ, NM>()), s, a, sh);
+  };
+  auto with = [&](auto q) {
+    if (shared_quant == XABE_QUANT_Q6K) launch(q, std::integral_constant<int, kQ6K>{});
+    else launch(q, std::integral_constant<int, kQ8_0>{});
+  };
+  if (quant == XABE_QUANT_Q6K) with(std::integral_constant<int, kQ6K>{});
+  else with(std::integral_constant<int, kQ8_0>{});
+  XABE_HIP_TRY(hipGetLastError());
+  return XABE_OK;
+}
+
 template <int MI, int WAVES>
 static int launch_parts(const xabe_moe_kernels* k, int quant, const MfmaArgs& a, size_t mtiles, hipStream_t s) {
   const size_t items = mtiles * (size_t)(a.n_rows / (WAVES * kWRows)) * a.parts;
@@ -1403,7 +1473,7 @@ int mfma_convert_activations(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_
 }
 
 int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_moe_buffers* b, xabe_quant_tensor gate,
-                                 xabe_quant_tensor up, xabe_quant_tensor down, const float* x) {
+                                 xabe_quant_tensor up, xabe_quant_tensor down, const float* x, const MfmaShared* shared) {
   const xabe_moe_geometry& g = k->g;
   if (!b->x_h_ready) XABE_TRY(to_f16(k, s, b, x));
   int bm = 0, cap = 0;
@@ -1438,7 +1508,19 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
   a.K = (int)g.hidden;
   a.n_rows = (int)g.intermediate;
   const bool pc = pc_form(k, pass_tokens(k, b));
-  if (pc) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
+  MfmaArgs sh = a;
+  size_t shared_tiles = 0;
+  if (shared) {  // (mfma_takes_shared)
+    sh.top_k = 1;
+    sh.tile_rows = kNarrowRows;
+    sh.w0 = static_cast<const uint8_t*>(shared->gate.bytes);
+    sh.w1 = static_cast<const uint8_t*>(shared->up.bytes);
+    sh.expert_bytes = 0;
+    sh.w_bytes = shared->gate.len;
+    sh.out = b->shared_inter_h;
+    shared_tiles = (g.max_tokens + kNarrowRows - 1) / kNarrowRows;
+    XABE_TRY((launch_with_shared<2>(k, gate.quant, shared->gate.quant, a, sh, max_mtiles, shared_tiles, s, true)));
+  } else if (pc) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
   else if (bm == kNarrowRows) XABE_TRY((launch_rows<2, true, 2, 4>(k, gate.quant, a, max_mtiles, s, gate_up_twice(g, pass_tokens(k, b)))));
   else XABE_TRY((launch_rows<2, true, 6, 8>(k, gate.quant, a, max_mtiles, s)));
   // down -> partial[flat][H], scaled by the routing weight
@@ -1450,7 +1532,16 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
   a.out = b->partial;
   a.K = (int)g.intermediate;
   a.n_rows = (int)g.hidden;
-  if (pc) XABE_TRY((launch_pc<1>(k, down.quant, a, max_mtiles * (g.hidden / kPR), s)));
+  if (shared) {
+    sh.w0 = static_cast<const uint8_t*>(shared->down.bytes);
+    sh.w1 = nullptr;
+    sh.w_bytes = shared->down.len;
+    sh.a = reinterpret_cast<const _Float16*>(b->shared_inter_h);
+    sh.out = shared->out;
+    sh.K = a.K;
+    sh.n_rows = a.n_rows;
+    XABE_TRY((launch_with_shared<1>(k, down.quant, shared->down.quant, a, sh, max_mtiles, shared_tiles, s, false)));
+  } else if (pc) XABE_TRY((launch_pc<1>(k, down.quant, a, max_mtiles * (g.hidden / kPR), s)));
   else if (bm == kNarrowRows) XABE_TRY((launch_rows<1, true, 2, 4>(k, down.quant, a, max_mtiles, s)));
   else XABE_TRY((launch_rows<1, true, 6, 8>(k, down.quant, a, max_mtiles, s)));
   return XABE_OK;
@@ -1470,6 +1561,19 @@ static int down_parts(const xabe_moe_geometry& g) {
   for (int parts = 4; parts > 1; --parts)
     if (nsb % parts == 0 && nsb / parts >= 8 && (size_t)(parts - 1) * g.hidden <= g.intermediate) return parts;
   return 1;
+}
+
+// Whether the shared expert's items go along with the routed ones (k_mfma_with_shared): where both take narrow tiles, the shared
+// down projection is whole and an expert's share is at most one block of 32 rows.  Then both kinds fit in three rounds of gate/up items,
+// the launches in front of them (router, routing, tables) have the chip to themselves, and nothing is forked or joined.
+// One layer, us, beside the router on a stream of its own / along (published layout): 64 tokens 213 / 202, 100: 238 / 226, 256:
+// 246 / 238, 512: 261 / 253, 700: 272 / 268, 1024: 295 / 293; skewed 300: 138 / 130, 512: 169 / 160, 900: 230 / 217; Q6_K 512: 252 / 246.
+// Above: 1237: 308 / 319, skewed 257 / 258, 1500: 343 / 337.
+bool mfma_takes_shared(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
+  const size_t tokens = pass_tokens(k, b);
+  int bm = 0, cap = 0;
+  if (!gate_up_twice(k->g, tokens) || !mfma_tile_plan(k, b, &bm, &cap) || bm != kNarrowRows || pc_form(k, tokens)) return false;
+  return down_parts(k->g) == 1 && !unrouted_up_wide(k, tokens) && !unrouted_down_wide(k, tokens, 1);
 }
 
 // The parts' sums of a live row in order, and the residual where there is one.  Bound by memory (hidden is a multiple of 256).

@@ -50,7 +50,7 @@ def spilled():
 
 
 @pytest.mark.parametrize("kernel,forms", [("k_mfma_rows", 16), ("k_decode_up", 24), ("k_decode_up_shared", 4), ("k_decode_down", 12),
-                                          ("k_mfma_parts", 4), ("k_digit_columns", 4), ("k_digit_down", 5), ("k_digit_up", 4),
+                                          ("k_mfma_parts", 4), ("k_mfma_with_shared", 8), ("k_digit_columns", 4), ("k_digit_down", 5), ("k_digit_up", 4),
                                           ("k_head_tiles_bf16", 1), ("k_head_tiles_q8", 4), ("k_head_tiles_q6", 2)])
 def test_no_vector_register_is_spilled(spilled, kernel, forms):
     got = {name: n for name, n in spilled.items() if name.split("<")[0] == kernel}
