@@ -15,8 +15,8 @@ struct xabe_moe_block {
   float *normed, *logits, *routed, *shexp, *gate;
   size_t n_act, n_logits;
   int fused_decode;  // decode widths: the regrouped three-launch block where the shape allows
-  // matrix-core widths: the shared expert runs beside the router, the routing and the dispatch tables, on a stream
-  // of the block's own that forks from the caller's after the RMSNorm and joins it before the combine
+  // matrix-core widths where the shared expert's tiles do not go along with the routed ones: it runs beside the router, the routing and
+  // the dispatch tables, on a stream of the block's own that forks from the caller's after the RMSNorm and joins it before the combine
   hipStream_t side;
   hipEvent_t forked, joined;
 };
@@ -183,7 +183,7 @@ int xabe_moe_block_forward_seam(xabe_moe_block* blk, void* stream, const xabe_mo
   const bool shared_mma =
       wide && mfma_supported(blk->moe, blk->buffers, w->shared_gate.quant, w->shared_up.quant, w->shared_down.quant, false);
   if (shared_mma && grouped_forward_takes_shared(blk->moe, blk->buffers, w)) {
-    // Narrow tiles on both sides: the shared expert's go along with the routed ones.
+    // Up to 32 rows an expert: the shared expert's tiles go along with the routed ones.
     XABE_TRY(check_shared_expert(blk->moe, w));
     if (!normed_h) XABE_TRY(mfma_convert_activations(blk->moe, as_stream(stream), blk->buffers, blk->normed));
     XABE_TRY(route_rows(blk, stream, w, logit_bias));
@@ -192,7 +192,7 @@ int xabe_moe_block_forward_seam(xabe_moe_block* blk, void* stream, const xabe_mo
     blk->buffers->x_h_ready = false;
     if (st != XABE_OK) return st;
   } else if (shared_mma && blk->side) {
-    // Wide tiles: the shared expert needs the rows only, so it forks off here and runs beside steps 2 and 3,
+    // Above: the shared expert needs the rows only, so it forks off here and runs beside steps 2 and 3,
     // whose first launches (router, routing, dispatch tables, tile lists) leave most of the device idle.
     hipStream_t s = as_stream(stream);
     if (!normed_h) XABE_TRY(mfma_convert_activations(blk->moe, s, blk->buffers, blk->normed));

@@ -1281,7 +1281,8 @@ static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
   return narrow_tiles(tokens, g.experts_per_token, g.num_experts) ? kNarrowRows : kWideRows;
 }
 // Whether narrow gate/up is launched with twice the workgroups that fit: while an expert's share averages one block of 32 rows.
-// Layers of the routed model in a row, us, once / twice: 512 tokens 259.6 / 251.0, 700: 269 / 265, 900: 279.5 / 277.4, 1000: 285.5 / 284.0,
+// With the shared expert's items along (k_mfma_with_shared), one layer, us, once / twice: 80 tokens 217 / 222, 256: 241 / 238, 512: 256 / 254,
+// 700 and 1000 alike; skewed 120 to 700 alike, 1000: 223 / 226.  By itself, the shared expert on a stream beside it, layers of the routed model in a row, us, once / twice: 512 tokens 259.6 / 251.0, 700: 269 / 265, 900: 279.5 / 277.4, 1000: 285.5 / 284.0,
 // 1024: 286.3 / 285.1; with the seam 252 / 245, 263 / 258, 275 / 270, 279.2 / 277.4, 279.6 / 278.4; with the published layout 267 / 260, 279 / 274,
 // 292 / 286, 296 / 293, 297 / 295.5; 100 and 256 tokens gain as 512 do.  Skewed loads: less than two rounds of items up to 900 tokens, and alike;
 // 950: 229 / 220, 1000: 253 / 227, 1024: 229 / 228.  At 1237 tokens, where items are one block or two, 327 / 313, but 314 / 317 in the

@@ -41,3 +41,42 @@ def test_rows_are_those_of_the_separate_calls(oracle, experts, top_k, hidden, in
     assert torch.equal(blk.buffers().topk_ids()[:live * top_k], b.topk_ids()[:live * top_k])
     for got, want in ((blk.buffers().partial()[:n * top_k], b.partial()[:n * top_k]), (blk.shared_ungated()[:n], shared[:n])):
         assert torch.equal(got.view(torch.int32), want.view(torch.int32)) and bool(want.isfinite().all())
+
+
+# along with the routed tiles and, one token on, on a stream beside them: passes back to back on one block, alternating two inputs,
+# eagerly and as a graph replayed with eager passes between the replays
+@pytest.mark.parametrize("tokens", [512, 513])
+def test_passes_back_to_back_on_either_side_of_the_rule(oracle, tokens):
+    import torch
+
+    import llmxabe_amd as X
+
+    g = X.MoeGeometry(128, 8, 512, 256, X.moe_block_size(tokens), tokens)
+    w = make_layer(oracle, g, seed=70).dev
+    xs = [activations(71 + i, tokens, 512) for i in range(2)]
+    blk = X.MoeBlock(g)
+    blk.publish_tokens(tokens)
+    out = lambda: [torch.zeros_like(xs[0]) for _ in range(4)]
+    want, got = out(), out()
+
+    def both(to):
+        for i in range(2):
+            blk.forward(w, xs[i], tokens, to[2 * i], to[2 * i + 1])
+
+    for i in range(2):
+        blk.forward(w, xs[i], tokens, want[2 * i], want[2 * i + 1])
+        torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        both(got)
+        stream.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with torch.cuda.graph(graph, stream=stream):
+            both(got)
+        for _ in range(3):
+            for t in got:
+                t.zero_()
+            graph.replay()
+            blk.forward(w, xs[0], tokens, torch.zeros_like(xs[0]), torch.zeros_like(xs[0]))
+            stream.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
