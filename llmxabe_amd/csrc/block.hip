@@ -27,14 +27,15 @@ static int block_alloc(float** p, size_t n, hipStream_t s) {
   return XABE_OK;
 }
 
-// (default priority, like every stream this library makes.  The events order kernels of one device, whose own fences make
-// their writes visible to each other: with the system-wide fence of a plain event between them a fork and a join cost about 3 us
-// more, published layout 1237 tokens 314 / 312 us, skewed 700 399 / 395, one Q6_K block of 512 254 / 251)
+// (default priority, like every stream this library makes.  The fork stands behind whatever the caller has put on its stream, a copy
+// of the shared expert's weights from the host or another device among it, which no kernel touches before the side stream's: its event
+// makes a plain event's system-wide fence.  The join orders kernels of one device, whose own fences make their writes visible to each
+// other, and goes without.  Both plain / so / both without, one layer, us: 1237 tokens 316 / 311 / 316, 2048: 377 / 371 / 374, skewed 1500
+// 290 / 287 / 288, 8192 965 / 959 / 962)
 static int block_side_stream(xabe_moe_block* blk) {
-  constexpr unsigned kFlags = hipEventDisableTiming | hipEventDisableSystemFence;
   XABE_HIP_TRY(hipStreamCreateWithFlags(&blk->side, hipStreamNonBlocking));
-  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->forked, kFlags));
-  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->joined, kFlags));
+  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->forked, hipEventDisableTiming));
+  XABE_HIP_TRY(hipEventCreateWithFlags(&blk->joined, hipEventDisableTiming | hipEventDisableSystemFence));
   return XABE_OK;
 }
 
