@@ -24,6 +24,7 @@
 #include "device_once.h"
 #include "digits.h"
 #include "host_common.h"
+#include "shared_along.h"
 #include "tile_list.h"
 
 namespace xabe {
@@ -550,7 +551,6 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 // workgroups per CU: a tile's start and end are then beside other tiles' steps).  Where the line lies: narrow_tiles,
 // unrouted_wide.
 constexpr int kSK = 64;                          // contraction elements per activation step
-constexpr int kNarrowRows = 64;                  // token rows of a tile, narrow form
 constexpr int kWideRows = 192;                   // token rows of a tile at most, wide form
 constexpr int kWRows = 32;                       // weight rows of a wavefront
 constexpr int kBlockBytes = 32 * kSK * 2;        // 32 token rows of an activation step in LDS
@@ -1287,7 +1287,7 @@ static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
 // 292 / 286, 296 / 293, 297 / 295.5; 100 and 256 tokens gain as 512 do.  Skewed loads: less than two rounds of items up to 900 tokens, and alike;
 // 950: 229 / 220, 1000: 253 / 227, 1024: 229 / 228.  At 1237 tokens, where items are one block or two, 327 / 313, but 314 / 317 in the
 // published layout, and skewed 255 / 260.
-static bool gate_up_twice(const xabe_moe_geometry& g, size_t tokens) { return tokens * g.experts_per_token <= 32 * g.num_experts; }
+static bool gate_up_twice(const xabe_moe_geometry& g, size_t tokens) { return share_in_one_block(tokens, g.experts_per_token, g.num_experts); }
 // The specialised form (k_mfma_pc) serves both routed launches for contractions of whole superblocks and at least
 // eight steps, when asked for: `mfma_form` 2 (0 and 1: k_mfma_rows everywhere; it is the faster at every width
 // measured, see k_mfma_pc).
@@ -1520,7 +1520,7 @@ int mfma_grouped_forward_partial(const xabe_moe_kernels* k, hipStream_t s, xabe_
     sh.w_bytes = shared->gate.len;
     sh.out = b->shared_inter_h;
     shared_tiles = (g.max_tokens + kNarrowRows - 1) / kNarrowRows;
-    XABE_TRY((launch_with_shared<2>(k, gate.quant, shared->gate.quant, a, sh, max_mtiles, shared_tiles, s, true)));
+    XABE_TRY((launch_with_shared<2>(k, gate.quant, shared->gate.quant, a, sh, max_mtiles, shared_tiles, s, gate_up_twice(g, pass_tokens(k, b)))));
   } else if (pc) XABE_TRY((launch_pc<2>(k, gate.quant, a, max_mtiles * (g.intermediate / (kPR / 2)), s)));
   else if (bm == kNarrowRows) XABE_TRY((launch_rows<2, true, 2, 4>(k, gate.quant, a, max_mtiles, s, gate_up_twice(g, pass_tokens(k, b)))));
   else XABE_TRY((launch_rows<2, true, 6, 8>(k, gate.quant, a, max_mtiles, s)));
@@ -1565,16 +1565,15 @@ static int down_parts(const xabe_moe_geometry& g) {
 }
 
 // Whether the shared expert's items go along with the routed ones (k_mfma_with_shared): where both take narrow tiles, the shared
-// down projection is whole and an expert's share is at most one block of 32 rows.  Then both kinds fit in three rounds of gate/up items,
-// the launches in front of them (router, routing, tables) have the chip to themselves, and nothing is forked or joined.
-// One layer, us, beside the router on a stream of its own / along (published layout): 64 tokens 213 / 202, 100: 238 / 226, 256:
-// 246 / 238, 512: 261 / 253, 700: 272 / 268, 1024: 295 / 293; skewed 300: 138 / 130, 512: 169 / 160, 900: 230 / 217; Q6_K 512: 252 / 246.
-// Above: 1237: 308 / 319, skewed 257 / 258, 1500: 343 / 337.
+// down projection is whole, and shared_along's rule on sizes says so.
+static_assert(kNarrowUpRows == 4 * kWRows / 2 && kNarrowDownRows == 4 * kWRows, "the items that shared_along counts");
 bool mfma_takes_shared(const xabe_moe_kernels* k, const xabe_moe_buffers* b) {
+  const xabe_moe_geometry& g = k->g;
   const size_t tokens = pass_tokens(k, b);
+  if (!shared_along(tokens, g.max_tokens, g.experts_per_token, g.num_experts, g.hidden, g.intermediate, (size_t)k->num_cus * kWgsPerCu<2, 4>)) return false;
   int bm = 0, cap = 0;
-  if (!gate_up_twice(k->g, tokens) || !mfma_tile_plan(k, b, &bm, &cap) || bm != kNarrowRows || pc_form(k, tokens)) return false;
-  return down_parts(k->g) == 1 && !unrouted_up_wide(k, tokens) && !unrouted_down_wide(k, tokens, 1);
+  if (!mfma_tile_plan(k, b, &bm, &cap) || bm != kNarrowRows || pc_form(k, tokens)) return false;
+  return down_parts(g) == 1 && !unrouted_up_wide(k, tokens) && !unrouted_down_wide(k, tokens, 1);
 }
 
 // The parts' sums of a live row in order, and the residual where there is one.  Bound by memory (hidden is a multiple of 256).
