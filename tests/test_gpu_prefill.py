@@ -224,15 +224,16 @@ def test_tall_tiles_give_the_rows_of_the_short_tiles(oracle, X):
     assert rel_to_peak(wide[rows], ref) <= MFMA_REL
 
 
-def test_wide_block_passes_back_to_back_keep_their_own_shared_rows(oracle, X):
-    """At matrix-core widths the shared expert runs on a stream of the block's own, forked from the caller's after the
-    RMSNorm and joined before the combine.  Passes issued back to back on one block, alternating two inputs, must each
-    give the bits of the same pass run alone: a pass's shared rows are not read before they are written, nor
-    overwritten by the next pass before its combine has read them.  Eagerly on a caller's stream, and as a captured
+# 512: the shared expert's tiles go along in the routed launches; 1237 and 2048: on the stream beside them, narrow and wide routed tiles
+@pytest.mark.parametrize("tokens", [512, 1237, 2048])
+def test_wide_block_passes_back_to_back_keep_their_own_shared_rows(oracle, X, tokens):
+    """At matrix-core widths the shared expert's tiles go along in the routed launches, or it runs on a stream of the block's own,
+    forked from the caller's after the RMSNorm and joined before the combine.  Passes issued back to back on one block,
+    alternating two inputs, must each give the bits of the same pass run alone: a pass's shared rows are not read before they are
+    written, nor overwritten by the next pass before its combine has read them.  Eagerly on a caller's stream, and as a captured
     graph replayed with eager passes between the replays."""
     import torch
 
-    tokens = 512
     g = X.MoeGeometry.qwen3_6(X.moe_block_size(tokens), tokens)
     layer = make_layer(oracle, g, seed=710)
     xa, xb = activations(41, tokens, 2048), activations(42, tokens, 2048)

@@ -53,9 +53,9 @@ def _two_layers(X, oracle, max_tokens, small=False, **kw):
     return [make_layer(oracle, g, seed=8100 + 50 * i, **kw) for i in range(2)]
 
 
-# (max_tokens, live tokens, three-launch decode on): every regime the block has
+# (max_tokens, live tokens, three-launch decode on): every regime the block has (from 1100 on with the shared expert on a stream beside)
 WIDTHS = [(1, 1, True), (3, 3, True), (8, 5, True), (32, 32, True), (3, 3, False), (12, 9, False), (48, 40, True), (200, 170, True),
-          (512, 512, True)]
+          (512, 512, True), (1237, 1100, True), (2048, 2048, True)]
 
 
 @pytest.mark.parametrize("max_tokens,tokens,decode_fused", WIDTHS)
