@@ -5,7 +5,9 @@
 // int8 shared-expert path (moe.rs:6389-6476); one reader per format feeds the same
 // MFMA body for gate, up and down, so there is no per-format asymmetry.
 //
-// Two kernels: k_mfma_rows, and k_mfma_pc, an alternative form of the routed launches (same bits) kept for comparison.
+// One body (mfma_rows_body) in three kernels: k_mfma_rows (routed or unrouted rows), k_mfma_parts (an unrouted contraction in parts) and
+// k_mfma_with_shared (routed and shared rows of a narrow pass); and k_mfma_pc, an alternative form of the routed launches (same
+// bits) kept for comparison.
 // Token tiles of the routed launches come from a device-built list with entries for the run of every *active* expert in
 // the dispatch table: experts with no tokens cost nothing, whatever the skew.  Workgroups are persistent and stride over
 // (token tile, row tile) items.
@@ -521,8 +523,8 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 //
 // What bounds it (gate/up of the dense sibling, 2048 x 5120 -> 2 x 17408, 730 GFLOP): the matrix instructions alone take
 // 450 us at the 1620 TFLOP/s that the chip holds on random data (it lowers its clock: power, not issue slots), the
-// kernel 750 (57 % of its cycles are matrix instructions), the kernel that dequantised 128 x 128 tiles through LDS
-// 969.  Added one by one to the matrix instructions: making halfs 75 us, activation reads 48, raw weight reads 93, the
+// kernel 708 (65 % of its cycles are matrix instructions; 750 and 57 % before these were kept apart, see below), the kernel that
+// dequantised 128 x 128 tiles through LDS 969.  Added one by one to the matrix instructions: making halfs 75 us, activation reads 48, raw weight reads 93, the
 // requests 162.  Hence
 //  - vector instructions between the matrix instructions, up to four of which cost one nothing (five parts of a chunk's
 //    weights spread over its NB matrix instructions, w_part);
@@ -533,11 +535,12 @@ __global__ void __launch_bounds__(1024, 4) k_mfma_pc(MfmaArgs a) {
 //    spilled vector register would undo that (its reload waits for everything requested before it): there is none
 //    (tests/test_spilled_registers.py).  With up to seven in eight of the sixteen forms the routed down launch drained
 //    its queue once per item, right behind the item's stores.  Scalar registers are kept in lanes of vector ones where there
-//    are too many (up to 119): no memory operation, but lane reads in the loop over the superblocks;
+//    are too many (up to 120, wide routed down of Q6_K; 37 to 70 in k_mfma_with_shared with a Q6_K side, whose routed body alone has 27 and 34): no memory operation, but lane reads in the loop over the superblocks;
 //  - what lies between the matrix instructions is kept there (w_part pins its results: the compiler moved the making of a
 //    chunk's halfs behind the chunk wherever a branch followed).  Wavefronts of a SIMD that make their requests at different times
 //    measured no better than all behind the matrix instructions, and cost a branch per chunk (both builds in turn, with the
-//    stores below: 1237 tokens 317 -> 309 us, 1400 669 -> 648 for two layers, two blocks of 8192 1860 -> 1820, dense 2048 1132 -> 1096);
+//    stores below: published layout 1237 tokens 322 -> 316 us, 1400 659 -> 638 for two layers, two blocks of 8192 with the seam 1896 -> 1852,
+//    dense 2048 1159 -> 1122; narrow Q8_0 launches with a workgroup or two per CU lose 1 %);
 //  - LDS reads on their own width's boundary (any other takes 64 cycles), rows spread over the banks by the windows' odd
 //    count of sixteen bytes, activations by pc_swizzle.
 // A short contraction (down of the routed model: two superblocks) is bound by what an item costs besides: its stores, which
@@ -1182,9 +1185,10 @@ __global__ void __launch_bounds__(64 * WAVES, (kWgsPerCu<MI, WAVES> * WAVES / 4)
   mfma_rows_body<QUANT, 1, false, MI, WAVES, true>(a, deal_items<false>(count_items<1, false, WAVES>(a, a.parts), a.resident));
 }
 // The routed experts' items (QUANT, `a`) and the shared expert's (SQUANT, `s`) of one pass in one launch, narrow form.  Alone a launch of
-// the shared expert's is a workgroup per CU or fewer, as long as one item (512 tokens: 28 us and 14); here they fill the last round of
-// the routed items: workgroups that have one routed item fewer come first.  512 tokens, skewed: gate/up 66 -> 70 us, down 43 -> 48,
-// and in front of it routing 13 -> 11 and 14 us less of fork, join and waiting.  Shared items first: 512 tokens 252.9 -> 255.1.
+// the shared expert's is a workgroup per CU or fewer, as long as one item (512 tokens: 27 us and 12); here they fill the last round of
+// the routed items: workgroups that have one routed item fewer come first.  By trace, 512 tokens, skewed: gate/up 64 to 70 us without, 70
+// with, down 40 and 46, the routing in front 12 and 10, and no fork, join or waiting: a block 168 to 176 and 161 to 162 us.  Shared items first: 512 tokens
+// 252.9 -> 255.1.  (The items are dealt as in deal_items, in two kinds: a change of one belongs in the other.)
 template <int QUANT, int SQUANT, int NM>
 __global__ void __launch_bounds__(256, 3) k_mfma_with_shared(MfmaArgs a, MfmaArgs s) {
   const int routed = count_items<NM, true, 4>(a, 1), shared = count_items<NM, false, 4>(s, 1), total = routed + shared;
@@ -1281,8 +1285,8 @@ static int routed_tile_rows(const xabe_moe_geometry& g, size_t tokens) {
   return narrow_tiles(tokens, g.experts_per_token, g.num_experts) ? kNarrowRows : kWideRows;
 }
 // Whether narrow gate/up is launched with twice the workgroups that fit: while an expert's share averages one block of 32 rows.
-// With the shared expert's items along (k_mfma_with_shared), one layer, us, once / twice: 80 tokens 217 / 222, 256: 241 / 238, 512: 256 / 254,
-// 700 and 1000 alike; skewed 120 to 700 alike, 1000: 223 / 226.  By itself, the shared expert on a stream beside it, layers of the routed model in a row, us, once / twice: 512 tokens 259.6 / 251.0, 700: 269 / 265, 900: 279.5 / 277.4, 1000: 285.5 / 284.0,
+// With the shared expert's items along (k_mfma_with_shared), one layer, us, once / twice: 80 tokens 217 / 222 (the loss that this line
+// accepts), 256: 241 / 238, 512: 256 / 254, 700 and 1000 alike; skewed 120 to 700 alike, 1000: 223 / 226.  By itself, the shared expert on a stream beside it, layers of the routed model in a row, us, once / twice: 512 tokens 259.6 / 251.0, 700: 269 / 265, 900: 279.5 / 277.4, 1000: 285.5 / 284.0,
 // 1024: 286.3 / 285.1; with the seam 252 / 245, 263 / 258, 275 / 270, 279.2 / 277.4, 279.6 / 278.4; with the published layout 267 / 260, 279 / 274,
 // 292 / 286, 296 / 293, 297 / 295.5; 100 and 256 tokens gain as 512 do.  Skewed loads: less than two rounds of items up to 900 tokens, and alike;
 // 950: 229 / 220, 1000: 253 / 227, 1024: 229 / 228.  At 1237 tokens, where items are one block or two, 327 / 313, but 314 / 317 in the

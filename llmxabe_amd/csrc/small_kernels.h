@@ -422,8 +422,9 @@ struct TileListArgs {
 // A chain of round trips: the ids are requested before the live count is known (ranges cut from the buffers' size), the
 // scan goes through the wavefronts' lanes with two barriers, and rounds past the live count are skipped: 14.6 -> 10.4 us at
 // 512 tokens.  Its wavefronts, like those of the three launches that wider passes take, run ahead of the shared expert's
-// where the two are on one CU (s_setprio: 0.2 to 0.8 % of a block up to 1024 tokens, nothing to see from 2048 on; a workgroup
-// that finds no room on any CU waits for it all the same).
+// where the two are on one CU (s_setprio).  Up to 1024 tokens that is only so in layers whose shared expert keeps a stream of its own
+// (shared_along.h), and there as elsewhere nothing is to be seen of it (without / with, 64 experts of 2048 x 1536, 340 tokens 216 / 214 us, 64 of
+// 2048 x 1024, 256 tokens 164.5 / 164.8); a workgroup that finds no room on any CU waits for it all the same.
 // ---------------------------------------------------------------------------------
 constexpr int kAlignFusedMaxSelections = 8192;
 constexpr int kAlignFusedWaves = 16;
