@@ -31,7 +31,8 @@ static int block_alloc(float** p, size_t n, hipStream_t s) {
 // of the shared expert's weights from the host or another device among it, which no kernel touches before the side stream's: its event
 // makes a plain event's system-wide fence.  The join orders kernels of one device, whose own fences make their writes visible to each
 // other, and goes without.  Both plain / so / both without, one layer, us: 1237 tokens 316 / 311 / 316, 2048: 377 / 371 / 374, skewed 1500
-// 290 / 287 / 288, 8192 965 / 959 / 962)
+// 290 / 287 / 288, 8192 965 / 959 / 962; what the fork's fence costs, so / both without: published layout, 1237 tokens 323 / 320, two blocks
+// of 8192 with the seam 1893 / 1885)
 static int block_side_stream(xabe_moe_block* blk) {
   XABE_HIP_TRY(hipStreamCreateWithFlags(&blk->side, hipStreamNonBlocking));
   XABE_HIP_TRY(hipEventCreateWithFlags(&blk->forked, hipEventDisableTiming));
